@@ -56,7 +56,8 @@ def _time_op(torch, fn, iters=20, warmup=3):
 
 
 class AttnTimer:
-    """Brackets every attention launch of the timed region with HIP events on the launch stream."""
+    """Brackets every attention launch with HIP events on the launch stream, in steps that follow the timed region:
+    inside it a block is one native call, whose kernels are not called one by one from here."""
 
     def __init__(self, torch, kernels):
         self.torch, self.kernels = torch, kernels
@@ -78,11 +79,11 @@ class AttnTimer:
             self.flops.append(4.0 * q.shape[0] * q.shape[2] * q.shape[1] * k.shape[1] * q.shape[3])
             return out
 
-        self.kernels.attn_fwd = timed
+        self.kernels.attn_fwd, self.kernels.NATIVE_BLOCKS = timed, False
         return self
 
     def __exit__(self, *exc):
-        self.kernels.attn_fwd = self.orig
+        self.kernels.attn_fwd, self.kernels.NATIVE_BLOCKS = self.orig, True
 
     def mean_ms(self):
         return sum(s.elapsed_time(e) for s, e in self.pairs) / max(len(self.pairs), 1)
@@ -156,11 +157,13 @@ class StepKernelTimer:
         self.saved = [(k, "adaln_modulate_pair", k.adaln_modulate_pair), (k, "qknorm_rope_pair", k.qknorm_rope_pair),
                       (k, "linear", k.linear), (k, "attn_fwd", k.attn_fwd), (F, "linear", F.linear)]
         k.adaln_modulate_pair, k.qknorm_rope_pair, k.linear, k.attn_fwd, F.linear = adaln_pair, qknorm_pair, linear, attn, f_linear
+        k.NATIVE_BLOCKS = False   # the blocks call the wrappers one by one
         return self
 
     def __exit__(self, *exc):
         for mod, name, fn in self.saved:
             setattr(mod, name, fn)
+        self.kernels.NATIVE_BLOCKS = True
 
     def report(self, steps):
         out = {}
@@ -329,7 +332,7 @@ def run_secondary(torch, kernels, args):
     """Flux / Wan shapes: same timing protocol as the headline line, one JSON line, no CPU leg."""
     make = flux_workload if args.workload == "flux" else wan_workload
     model, step, lat, name, gemm_flop, valid = make(torch, None if args.blocks == LAYERS else args.blocks)
-    with torch.inference_mode(), AttnTimer(torch, kernels) as timer:
+    with torch.inference_mode():
         if args.autotune > 0:
             kernels.set_linear_autotune(args.autotune)
             step(0, lat)
@@ -337,17 +340,21 @@ def run_secondary(torch, kernels, args):
         for i in range(args.warmup):
             lat = step(i, lat)
         torch.cuda.synchronize()
-        timer.active = True
         t0 = time.perf_counter()
         for i in range(args.warmup, args.warmup + args.steps):
             lat = step(i, lat)
         torch.cuda.synchronize()
         elapsed = time.perf_counter() - t0
-        timer.active = False
+        n_attn_steps = 1 if args.workload == "wan" else 2
+        with AttnTimer(torch, kernels) as timer:
+            timer.active = True
+            for i in range(n_attn_steps):
+                lat = step(i, lat)
+            torch.cuda.synchronize()
     assert bool(torch.isfinite(lat.float()).all()), "non-finite latents"
     ms, flop, n = timer.dominant()
     tf = flop / ms / 1e9
-    attn_total = sum(timer.flops) / args.steps
+    attn_total = sum(timer.flops) / n_attn_steps
     in_step = None
     if not args.no_in_step:   # as for the headline workload: extra steps outside the timed region, kernel by kernel
         n_extra = 1 if args.workload == "wan" else 2
@@ -781,7 +788,7 @@ def main():
         noise = combine_cfg_noise(out[0:1], out[1:2], 4.0, True)
         return euler_step(lat, noise, float(sig[i]), float(sig[i + 1]))
 
-    with torch.inference_mode(), AttnTimer(torch, kernels) as timer:
+    with torch.inference_mode():
         lat = latents
         if args.autotune > 0:   # untimed: pick the library kernel for each fused-epilogue GEMM
             kernels.set_linear_autotune(args.autotune)
@@ -790,13 +797,16 @@ def main():
         for i in range(args.warmup):
             lat = step(i, lat)
         torch.cuda.synchronize()
-        timer.active = True
         t0 = time.perf_counter()
         for i in range(args.warmup, total_steps):
             lat = step(i, lat)
         torch.cuda.synchronize()
         elapsed = time.perf_counter() - t0
-        timer.active = False
+        with AttnTimer(torch, kernels) as timer:   # two more steps, attention between events
+            timer.active = True
+            for i in range(2):
+                lat = step(i, lat)
+            torch.cuda.synchronize()
         attn_ms = timer.mean_ms()
         n_attn = len(timer.pairs)
     assert bool(torch.isfinite(lat.float()).all()), "non-finite latents"

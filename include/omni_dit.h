@@ -371,6 +371,12 @@ int odit_linear_rows(const void* x, const void* w, const void* bias, void* out, 
                      int epilogue, int gate_dtype, int dtype, int rows_per_gate, int64_t gate_stride,
                      unsigned flags, void* workspace, size_t workspace_bytes, void* stream);
 
+/* Names the library kernel for plain projections of one problem (ODIT_EPI_BIAS, dense rows) ahead of time by the
+ * library's own solution index, as an offline tuning run found it; process-wide, applies to problems first seen
+ * afterwards. A solution that the loaded library does not have, or that does not take the problem, is ignored. The indices
+ * belong to one library version: the caller compares versions. No counterpart in the reference. */
+int odit_linear_prefer(int M, int N, int K, int dtype, int solution);
+
 /* What odit_linear_rows would do with these arguments, without launching anything: *handwritten = 1 when
  * a hand-written kernel would run, *launches = kernel launches the call would make. */
 int odit_linear_rows_plan(const void* x, const void* w, const void* bias, void* out, const void* residual,

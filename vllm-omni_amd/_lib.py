@@ -92,6 +92,7 @@ _SIGNATURES = {
         [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_int,
          C.c_int64, C.c_int64, C.c_int64, C.c_int64, C.c_int, C.c_int, C.c_int, C.c_void_p, C.c_size_t, C.c_void_p],
     ),
+    "odit_linear_prefer": (C.c_int, [C.c_int, C.c_int, C.c_int, C.c_int, C.c_int]),
     "odit_linear_rows": (
         C.c_int,
         [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_int,
@@ -157,6 +158,28 @@ def load() -> C.CDLL:
         fn.argtypes = argtypes
     _lib = lib
     return lib
+
+
+NATIVE_NAME = "_native.so"
+_native = None
+
+
+def native():
+    """The native host path (csrc/native.cpp), loaded once behind the kernel library it calls; raises loudly when
+    it is not there."""
+    global _native
+    if _native is None:
+        load()
+        path = LIB_PATH.with_name(NATIVE_NAME)
+        if not path.exists():
+            raise OmniDitLibraryError(f"{path} not found: build it with `python {path.parent / 'csrc' / 'build.py'}`. "
+                                      "There is no fallback path.")
+        try:
+            from . import _native as module
+        except ImportError as e:  # built against another torch, unresolved symbols, ...
+            raise OmniDitLibraryError(f"cannot load {path}: {e}") from e
+        _native = module
+    return _native
 
 
 def is_available() -> bool:

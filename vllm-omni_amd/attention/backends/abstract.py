@@ -54,9 +54,8 @@ class AttentionMetadata:
     ``value_tail`` (not in the reference): the ``value`` argument then holds only the rows of the first
     keys and this tensor the rest, so a caller with the values of two streams in two buffers does not
     have to concatenate them.
-    ``attn_mask_checked`` (not in the reference): the caller vouches that ``attn_mask`` is worth applying
-    (it has already dropped an all-true mask, or accepts the masked kernel for one), so the backend skips
-    its own all-true test, which costs a device-to-host synchronisation per call."""
+    ``attn_mask_checked`` (not in the reference): the caller has looked at ``attn_mask`` itself. Kept for callers that
+    set it; the backend tests no mask for being all true any more (that test synchronised, the kernel needs none)."""
 
     attn_mask: torch.Tensor | None = None
     joint_attn_mask: torch.Tensor | None = None

@@ -61,17 +61,14 @@ class HipFlashAttentionImpl(AttentionImpl):
 
     def forward_hip(self, query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
                     attn_metadata: AttentionMetadata | None = None) -> torch.Tensor:
-        """q [B,Sq,H,D], k/v [B,Sk,Hkv,D] -> [B,Sq,H,D]. A [B,Sk] ``attn_mask`` excludes keys; an
-        all-true mask is dropped like the reference does (flash_attn.py:80-84) unless
-        ``attn_metadata.attn_mask_checked`` says the caller has seen to that (the test synchronises). With
+        """q [B,Sq,H,D], k/v [B,Sk,Hkv,D] -> [B,Sq,H,D]. A [B,Sk] ``attn_mask`` excludes keys. (The reference drops an
+        all-true mask, flash_attn.py:80-84. That test synchronises; the kernel gives the same values for one and runs
+        tiles without an excluded key like those of a launch without a mask.) With
         ``attn_metadata.output_split`` = s the result is the pair (out[:, :s], out[:, s:]), both dense;
         with ``attn_metadata.value_tail`` the values are [value; value_tail] along the keys, read in place."""
         mask = attn_metadata.attn_mask if attn_metadata is not None else None
         if not self.kernel_takes_layer or not self.kernel_takes_mask(mask, query.shape[0], key.shape[1]):
             return self.sdpa.forward_hip(query, key, value, attn_metadata)
-        if mask is not None:
-            if not attn_metadata.attn_mask_checked and bool(torch.all(mask != 0)):
-                mask = None
         split = attn_metadata.output_split if attn_metadata is not None else None
         v_tail = attn_metadata.value_tail if attn_metadata is not None else None
         if v_tail is not None:

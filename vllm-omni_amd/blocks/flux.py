@@ -31,6 +31,7 @@ from ..attention.backends.abstract import AttentionMetadata
 from ..attention.layer import Attention
 from ..layers.rmsnorm import RMSNorm
 from ..layers.rope import RotaryEmbedding
+from . import qwen_image
 from .qwen_image import (AdaLayerNormContinuous, FeedForward, QwenTimestepProjEmbeddings, TimestepEmbedding,
                          Transformer2DModelOutput, _require_single_gpu, project_residual)
 
@@ -42,9 +43,17 @@ class FluxRotary:
     def __init__(self, cos: torch.Tensor, sin: torch.Tensor):
         self.cos, self.sin = cos, sin
         self.cos32, self.sin32 = cos.float().contiguous(), sin.float().contiguous()
+        self._split = None
 
     def __iter__(self):
         return iter((self.cos, self.sin))
+
+    def split(self, n_txt: int):
+        """(image cos, image sin, text cos, text sin) rows of the float32 tables; kept for the blocks of a forward."""
+        if self._split is None or self._split[0] != n_txt:
+            c, s = self.cos32, self.sin32
+            self._split = (n_txt, (c[n_txt:], s[n_txt:], c[:n_txt], s[:n_txt]))
+        return self._split[1]
 
 
 def _rotary(image_rotary_emb) -> FluxRotary | None:
@@ -192,6 +201,15 @@ class FluxTransformerBlock(nn.Module):
         all blocks at once; otherwise they are computed here as in the reference. ``gate_rows`` = float32
         (gates, gates * biases), each [B, 2 (hidden, context), 2 (attention, feed-forward), C]."""
         rr = self.ref_rounding
+        rotary = _rotary(image_rotary_emb)
+        if not rr and mod_params is not None and rotary is not None and not joint_attention_kwargs and kernels.native_blocks():
+            g, gb = gate_rows if gate_rows is not None else (None, None)
+            n_c = encoder_hidden_states.shape[1]
+            done = kernels.native().flux_block(
+                self, self.attn.heads, self.attn.head_dim, hidden_states, encoder_hidden_states, *mod_params, g, gb,
+                *rotary.split(n_c), None, qwen_image.FUSE_MIN_ROWS, kernels.linear_engine_flags())
+            if done is not None:
+                return done
         pre = [[None, None], [None, None]]
         if gate_rows is not None:
             pre = [[(gate_rows[0][:, s, j], gate_rows[1][:, s, j]) for j in range(2)] for s in range(2)]
@@ -247,6 +265,13 @@ class FluxSingleTransformerBlock(nn.Module):
                       gate_rows: tuple[torch.Tensor, torch.Tensor] | None = None) -> torch.Tensor:
         """``gate_rows`` = float32 (gate [B,C], gate * proj_out.bias [B,C]) made by the caller."""
         B, S, C = x.shape
+        if not self.ref_rounding and mod is not None and gate_rows is not None and kernels.native_blocks():
+            rot = _rotary(image_rotary_emb)
+            if rot is not None:
+                done = kernels.native().flux_single_block(self, self.attn.heads, self.attn.head_dim, x, mod, *gate_rows, rot.cos32,
+                                                          rot.sin32, in_place, kernels.linear_engine_flags())
+                if done is not None:
+                    return done
         n, gate = self.norm(x, emb=temb, mod=mod)
         fused = not self.ref_rounding and x.dtype != torch.float32
         if fused:
@@ -502,3 +527,6 @@ class FluxTransformer2DModel(nn.Module):
         with torch.no_grad():
             for k, p in own.items():
                 p.copy_(weights[k].to(device=p.device, dtype=p.dtype))
+
+
+kernels.native_classes(FluxAttention=FluxAttention)

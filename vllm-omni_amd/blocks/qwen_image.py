@@ -9,7 +9,8 @@ qit.py:1073-1113). Differences are all below the module interfaces:
     writes straight into the joint [B, S_txt+S_img, H, D] buffers (qit.py:588-606);
   * adaLN LayerNorm+modulate and the gated residual are one pass each (qit.py:770-773, 794-806);
   * GELU(tanh) runs in place on the MLP-up output (qit.py:424);
-  * dense projections are ``torch.nn.functional.linear`` (hipBLASLt MFMA GEMMs).
+  * dense projections are ``torch.nn.functional.linear`` (hipBLASLt MFMA GEMMs);
+  * a block of plain modules runs as ONE native call (``csrc/native.cpp``), which makes the same launches.
 """
 
 from __future__ import annotations
@@ -25,6 +26,7 @@ import torch.nn.functional as F
 from .. import kernels
 from .._lib import ODIT_NORM_HEAD
 from ..attention.backends.abstract import AttentionMetadata
+from ..attention.backends.hip_flash import HipFlashAttentionImpl
 from ..attention.layer import Attention
 from ..layers.adalayernorm import AdaLayerNorm, adaln_pair
 from ..layers.rmsnorm import RMSNorm
@@ -163,6 +165,7 @@ class QwenEmbedRope(nn.Module):
         self.axis_of = torch.repeat_interleave(torch.arange(len(self.axes_dim), device=cpu),
                                                torch.tensor([d // 2 for d in self.axes_dim], device=cpu))
         self._tables = lru_cache(maxsize=16)(self._build)
+        self._float_tables = lru_cache(maxsize=16)(self._split)
 
     def _table(self, positions: torch.Tensor) -> torch.Tensor:
         """positions: int64 [N, 3] -> complex64 [N, sum(d) / 2] unit phasors."""
@@ -206,6 +209,13 @@ class QwenEmbedRope(nn.Module):
     def forward(self, video_fhw, txt_seq_lens, device):
         return self._tables(self._norm_shapes(video_fhw), int(max(txt_seq_lens)), str(device))
 
+    def _split(self, shapes, txt_len: int, device: str) -> "RotaryTables":
+        return RotaryTables(*self._tables(shapes, txt_len, device))
+
+    def tables(self, video_fhw, txt_seq_lens, device) -> "RotaryTables":
+        """``forward``'s tables with the float32 cos/sin the kernels read, cached like them."""
+        return self._float_tables(self._norm_shapes(video_fhw), int(max(txt_seq_lens)), str(device))
+
 
 class QwenEmbedLayer3DRope(QwenEmbedRope):
     """The layered-image variant's tables (qit.py:183-296): as QwenEmbedRope for the layers, the last
@@ -216,7 +226,7 @@ class QwenEmbedLayer3DRope(QwenEmbedRope):
 
 
 class RotaryTables:
-    """Complex tables as the reference passes them between modules, plus float32 cos/sin views."""
+    """Complex tables as the reference passes them between modules, plus float32 cos/sin copies of them."""
 
     def __init__(self, vid_freqs: torch.Tensor, txt_freqs: torch.Tensor):
         self.vid_freqs, self.txt_freqs = vid_freqs, txt_freqs
@@ -228,6 +238,18 @@ class RotaryTables:
 
     def __getitem__(self, i: int):
         return (self.vid_freqs, self.txt_freqs)[i]
+
+
+def joint_key_mask(txt_mask, img_mask, B: int, S_txt: int, S_img: int, device) -> torch.Tensor | None:
+    """[B, S_txt + S_img] boolean key mask of the joint sequence from the two streams' masks (None = all true)."""
+    if txt_mask is None and img_mask is None:
+        return None
+    out = torch.ones((B, S_txt + S_img), dtype=torch.bool, device=device)
+    if txt_mask is not None:
+        out[:, :S_txt] = txt_mask
+    if img_mask is not None:
+        out[:, S_txt:] = img_mask
+    return out
 
 
 class QwenImageCrossAttention(nn.Module):
@@ -257,8 +279,10 @@ class QwenImageCrossAttention(nn.Module):
 
     def forward(self, hidden_states: torch.Tensor, encoder_hidden_states: torch.Tensor, vid_freqs, txt_freqs=None,
                 hidden_states_mask: torch.Tensor | None = None,
-                encoder_hidden_states_mask: torch.Tensor | None = None, residuals=None):
-        """``residuals`` = (img_residual, img_gate, txt_residual, txt_gate[, img_pre, txt_pre]): return
+                encoder_hidden_states_mask: torch.Tensor | None = None, residuals=None,
+                joint_mask: torch.Tensor | None = None):
+        """``joint_mask`` = the caller's [B, S_txt + S_img] key mask (then the two stream masks are not read).
+        ``residuals`` = (img_residual, img_gate, txt_residual, txt_gate[, img_pre, txt_pre]): return
         residual + gate * projection for both streams (new tensors) instead of the bare projections;
         the ``*_pre`` pairs are caller-made float32 (gate, gate * bias) rows (see project_residual)."""
         tables = vid_freqs if isinstance(vid_freqs, RotaryTables) else RotaryTables(vid_freqs, txt_freqs)
@@ -287,14 +311,11 @@ class QwenImageCrossAttention(nn.Module):
         meta = AttentionMetadata(output_split=S_txt)
         if v_in_place:
             jv, meta.value_tail = txt_qkv[:, :, 2], img_qkv[:, :, 2]
-        if hidden_states_mask is not None or encoder_hidden_states_mask is not None:
-            ones = lambda n: torch.ones((B, n), dtype=torch.bool, device=jq.device)  # noqa: E731
-            txt_m = encoder_hidden_states_mask if encoder_hidden_states_mask is not None else ones(S_txt)
-            img_m = hidden_states_mask if hidden_states_mask is not None else ones(S_img)
-            meta.attn_mask = torch.cat([txt_m.bool(), img_m.bool()], dim=1)
-            # the model drops an all-true mask once per forward (run_blocks); for a direct call of a block
-            # with one the masked kernel gives the same values, and testing here would synchronise per block
-            meta.attn_mask_checked = True
+        if joint_mask is None:
+            joint_mask = joint_key_mask(encoder_hidden_states_mask, hidden_states_mask, B, S_txt, S_img, jq.device)
+        if joint_mask is not None:
+            # (an all-true mask gives the values of no mask; testing for one would synchronise)
+            meta.attn_mask, meta.attn_mask_checked = joint_mask, True
         txt_attn, img_attn = self.attn(jq, jk, jv, meta)
         if residuals is not None:
             img_res, img_gate, txt_res, txt_gate = residuals[:4]
@@ -317,7 +338,7 @@ class QwenImageTransformerBlock(nn.Module):
                  fuse_epilogues: bool = True):
         super().__init__()
         self.dim = dim
-        fused = fuse_epilogues and not ref_rounding
+        self.fused = fused = fuse_epilogues and not ref_rounding
         self.num_attention_heads, self.attention_head_dim = num_attention_heads, attention_head_dim
         self.img_mod = nn.Sequential(SiLU(), nn.Linear(dim, 6 * dim, bias=True))
         self.img_norm1 = AdaLayerNorm(dim, elementwise_affine=False, eps=eps, ref_rounding=ref_rounding)
@@ -337,14 +358,11 @@ class QwenImageTransformerBlock(nn.Module):
                 joint_attention_kwargs: dict[str, Any] | None = None, modulate_index: torch.Tensor | None = None,
                 hidden_states_mask: torch.Tensor | None = None,
                 mod_params: tuple[torch.Tensor, torch.Tensor] | None = None,
-                gate_rows: tuple[torch.Tensor, torch.Tensor] | None = None):
+                gate_rows: tuple[torch.Tensor, torch.Tensor] | None = None, joint_mask: torch.Tensor | None = None):
         """``mod_params`` = (img [B,6C], txt [B,6C]) computed by the caller for all blocks at once
         (they depend on ``temb`` only); when absent they are computed here as in the reference.
         ``gate_rows`` = float32 (gates, gates * biases), each [B, 2 (img, txt), 2 (attention, MLP), C],
         likewise made once per step: the fused output projections then need no per-call set-up."""
-        pre = [[None, None], [None, None]]
-        if gate_rows is not None and modulate_index is None:
-            pre = [[(gate_rows[0][:, s, j], gate_rows[1][:, s, j]) for j in range(2)] for s in range(2)]
         rr = self.ref_rounding
         if mod_params is not None:
             img_mod_params, txt_mod_params = mod_params
@@ -353,6 +371,21 @@ class QwenImageTransformerBlock(nn.Module):
             if self.zero_cond_t:
                 temb = torch.chunk(temb, 2, dim=0)[0]
             txt_mod_params = self.txt_mod(temb)
+        tables = image_rotary_emb if isinstance(image_rotary_emb, RotaryTables) else RotaryTables(*image_rotary_emb)
+        if joint_mask is None:
+            joint_mask = joint_key_mask(encoder_hidden_states_mask, hidden_states_mask, hidden_states.shape[0],
+                                        encoder_hidden_states.shape[1], hidden_states.shape[1], hidden_states.device)
+        if self.fused and modulate_index is None and kernels.native_blocks():
+            g, gb = gate_rows if gate_rows is not None else (None, None)
+            done = kernels.native().qwen_block(
+                self, self.num_attention_heads, self.attention_head_dim, hidden_states, encoder_hidden_states, img_mod_params,
+                txt_mod_params, g, gb, tables.img_cos, tables.img_sin, tables.txt_cos, tables.txt_sin, joint_mask, FUSE_MIN_ROWS,
+                kernels.linear_engine_flags())
+            if done is not None:
+                return done
+        pre = [[None, None], [None, None]]
+        if gate_rows is not None and modulate_index is None:
+            pre = [[(gate_rows[0][:, s, j], gate_rows[1][:, s, j]) for j in range(2)] for s in range(2)]
         img_mod1, img_mod2 = img_mod_params.chunk(2, dim=-1)
         txt_mod1, txt_mod2 = txt_mod_params.chunk(2, dim=-1)
 
@@ -363,13 +396,13 @@ class QwenImageTransformerBlock(nn.Module):
         else:
             img_modulated, img_gate1 = self.img_norm1(hidden_states, img_mod1, modulate_index)
             txt_modulated, txt_gate1 = self.txt_norm1(encoder_hidden_states, txt_mod1)
-        tables = image_rotary_emb if isinstance(image_rotary_emb, RotaryTables) else RotaryTables(*image_rotary_emb)
         # the block's inputs are never written (callers such as TeaCache keep them to form residuals):
         # the attention residuals land in new tensors, the MLP residuals then update those in place
         hidden_states, encoder_hidden_states = self.attn(
             img_modulated, txt_modulated, tables, hidden_states_mask=hidden_states_mask,
             encoder_hidden_states_mask=encoder_hidden_states_mask,
-            residuals=(hidden_states, img_gate1, encoder_hidden_states, txt_gate1, pre[0][0], pre[1][0]))
+            residuals=(hidden_states, img_gate1, encoder_hidden_states, txt_gate1, pre[0][0], pre[1][0]),
+            joint_mask=joint_mask)
 
         if modulate_index is None:
             (img_modulated2, img_gate2), (txt_modulated2, txt_gate2) = adaln_pair(
@@ -441,6 +474,13 @@ class AdaLayerNormContinuous(nn.Module):
         return kernels.adaln_modulate(x, shift, scale, eps=self.eps)
 
 
+@lru_cache(maxsize=16)
+def _conditioning_index(samples: tuple, device: str) -> torch.Tensor:
+    """Built on the host once per set of image shapes, like the rotary tables."""
+    rows = [[0] * math.prod(s[0]) + [1] * sum(math.prod(x) for x in s[1:]) for s in samples]
+    return torch.tensor(rows, device=device, dtype=torch.int32)
+
+
 class QwenImageTransformer2DModel(nn.Module):
     """Stem, N dual-stream blocks, head (qit.py:817-1071). ``prepare`` / ``run_blocks`` / ``finish``
     are the three stages TeaCache needs to call separately (cache/teacache/extractors.py:147-279)."""
@@ -503,8 +543,7 @@ class QwenImageTransformer2DModel(nn.Module):
         temb = self.time_text_embed(timestep, img, additional_t_cond)
         if txt_seq_lens is None:
             txt_seq_lens = [encoder_hidden_states.shape[1]]
-        vid_freqs, txt_freqs = self.pos_embed(img_shapes, txt_seq_lens, device=img.device)
-        return img, txt, temb, RotaryTables(vid_freqs, txt_freqs)
+        return img, txt, temb, self.pos_embed.tables(img_shapes, txt_seq_lens, device=img.device)
 
     def modulate_index(self, img_shapes, device) -> torch.Tensor | None:
         """[B, S_img] int32 per-token conditioning choice of the editing variant: 0 (real timestep) for the
@@ -512,9 +551,9 @@ class QwenImageTransformer2DModel(nn.Module):
         per sample a list of (frame, height, width) (qit.py:146-154). None for the plain model."""
         if not self.zero_cond_t:
             return None
-        samples = [[s] if isinstance(s[0], int) else list(s) for s in img_shapes]  # bare (f, h, w) = one image
-        rows = [[0] * math.prod(s[0]) + [1] * sum(math.prod(x) for x in s[1:]) for s in samples]
-        return torch.tensor(rows, device=device, dtype=torch.int32)
+        samples = tuple((tuple(s),) if isinstance(s[0], int) else tuple(tuple(x) for x in s)  # bare (f, h, w) = one image
+                        for s in img_shapes)
+        return _conditioning_index(samples, str(device))
 
     def fuse_modulation(self) -> None:
         """Stack every block's img_mod / txt_mod Linear into one [L, 2, 6C, C] weight so that the
@@ -568,9 +607,10 @@ class QwenImageTransformer2DModel(nn.Module):
 
     def run_blocks(self, img, txt, temb, rotary, encoder_hidden_states_mask=None, attention_kwargs=None,
                    modulate_index=None):
+        # the reference drops an all-true mask (qit.py:1044-1048), which takes a synchronisation; the masked kernel gives
+        # the same values for one and costs nothing on tiles without an excluded key
         mask = encoder_hidden_states_mask
-        if mask is not None and bool(mask.all()):
-            mask = None  # all-true masks are dropped (qit.py:1044-1048)
+        joint = joint_key_mask(mask, None, img.shape[0], txt.shape[1], img.shape[1], img.device)
         mods = self.all_modulations(temb)
         rows = self.all_gate_rows(mods)
         for i, block in enumerate(self.transformer_blocks):
@@ -578,7 +618,7 @@ class QwenImageTransformer2DModel(nn.Module):
             gr = (rows[0][:, i], rows[1][:, i]) if rows is not None else None
             txt, img = block(hidden_states=img, encoder_hidden_states=txt, encoder_hidden_states_mask=mask,
                              temb=temb, image_rotary_emb=rotary, joint_attention_kwargs=attention_kwargs,
-                             modulate_index=modulate_index, mod_params=mp, gate_rows=gr)
+                             modulate_index=modulate_index, mod_params=mp, gate_rows=gr, joint_mask=joint)
         return img, txt
 
     def finish(self, img, temb, return_dict: bool = True):
@@ -620,3 +660,8 @@ class QwenImageTransformer2DModel(nn.Module):
         with torch.no_grad():
             for k, p in own.items():
                 p.copy_(weights[k].to(device=p.device, dtype=p.dtype))
+
+
+kernels.native_classes(Linear=nn.Linear, RMSNorm=RMSNorm, AdaLayerNorm=AdaLayerNorm, Attention=Attention,
+                       AttentionImpl=HipFlashAttentionImpl, FeedForward=FeedForward, ApproxGELU=ApproxGELU,
+                       QwenImageCrossAttention=QwenImageCrossAttention)

@@ -36,6 +36,7 @@ import torch.nn.functional as F
 from .. import kernels
 from .._lib import ODIT_NORM_ROW
 from ..attention.layer import Attention
+from . import qwen_image
 from .qwen_image import (ApproxGELU, QwenTimestepProjEmbeddings, TimestepEmbedding, Transformer2DModelOutput,
                          project_residual)
 
@@ -247,6 +248,7 @@ class WanTransformerBlock(nn.Module):
         self.scale_shift_table = nn.Parameter(torch.randn(1, 6, dim) / dim ** 0.5)
         self._ln2_f32: tuple[int, torch.Tensor, torch.Tensor] | None = None
         self._table_f32: tuple[tuple, torch.Tensor] | None = None
+        self._bias_f32: tuple[tuple, torch.Tensor] | None = None
 
     def _table(self) -> torch.Tensor:
         """float32 [6, C] copy of scale_shift_table, refreshed when the parameter changes."""
@@ -255,6 +257,17 @@ class WanTransformerBlock(nn.Module):
         if self._table_f32 is None or self._table_f32[0] != tag:
             self._table_f32 = (tag, p.detach().float().reshape(6, -1).contiguous())
         return self._table_f32[1]
+
+    def gated_biases(self) -> torch.Tensor:
+        """float32 [6, C]: in rows 2 and 5 the biases of the projections those gates scale (attn1.to_out, ffn.net_2),
+        zero elsewhere: times the modulation rows it gives gate * bias rows that lie where the gate rows do."""
+        ps = (self.attn1.to_out.bias, self.ffn.net_2.bias)
+        tag = tuple((p._version, p.data_ptr(), p.device) for p in ps)
+        if self._bias_f32 is None or self._bias_f32[0] != tag:
+            t = torch.zeros((6, ps[0].shape[0]), dtype=torch.float32, device=ps[0].device)
+            t[2], t[5] = ps[0].detach().float(), ps[1].detach().float()
+            self._bias_f32 = (tag, t)
+        return self._bias_f32[1]
 
     def _norm2_affine(self):
         """float32 copies of norm2's weight/bias, refreshed when the parameters change."""
@@ -270,6 +283,10 @@ class WanTransformerBlock(nn.Module):
         """``mod`` = float32 [B, 6, C] = scale_shift_table + temb when the caller formed it for all
         blocks at once; otherwise it is formed here as in the reference. ``gate_bias`` = float32 [B, 2, C]:
         the two gates times the biases of the projections they scale (attn1.to_out, ffn.net_2)."""
+        if kernels.native_blocks() and hidden_states.dtype != torch.float32:
+            done = self._forward_native(hidden_states, encoder_hidden_states, temb, rotary_emb, mod, gate_bias)
+            if done is not None:
+                return done
         if mod is None and temb.ndim == 4:
             return self._forward_per_token(hidden_states, encoder_hidden_states, temb, rotary_emb)
         if mod is None:
@@ -289,6 +306,23 @@ class WanTransformerBlock(nn.Module):
         n = kernels.adaln_modulate(x, c_shift, c_scale, eps=self.eps, out=n if n is not x else None)
         return project_residual(self.ffn.net_2, self.ffn.net_0(n), x, c_gate, out=x, pre=pre2)
 
+
+    def _forward_native(self, x, ctx, temb, rotary_emb, mod, gate_bias):
+        """The whole block as one native call, or None where the call or a submodule is not of the plain form."""
+        rot = _rotary(rotary_emb)
+        per_token = mod is None and temb.ndim == 4
+        if rot is None:
+            return None
+        if mod is None and not per_token:
+            mod = self.scale_shift_table + temb.float()
+        if gate_bias is None and not per_token:
+            gate_bias = (mod * self.gated_biases())[:, 2::3]
+        lw, lb = (None, None) if isinstance(self.norm2, nn.Identity) else self._norm2_affine()
+        a = self.attn1
+        return kernels.native().wan_block(self, a.num_heads, a.head_dim, x, ctx, None if per_token else mod,
+                                          None if per_token else gate_bias, temb if per_token else None,
+                                          self._table() if per_token else None, lw, lb, rot.cos32, rot.sin32,
+                                          qwen_image.FUSE_MIN_ROWS, kernels.linear_engine_flags())
 
     def _forward_per_token(self, x: torch.Tensor, ctx: torch.Tensor, temb: torch.Tensor, rotary_emb) -> torch.Tensor:
         """temb [B, S, 6, C] (wan.py:641-652): every token has its own six modulation rows. The reference
@@ -492,8 +526,7 @@ class WanTransformer3DModel(nn.Module):
         mods = self.all_modulations(timestep_proj)
         gb = None
         if x.dtype != torch.float32:  # gates (rows 2 and 5) times the biases they scale, [L, B, 2, C]
-            biases = torch.stack([torch.stack([blk.attn1.to_out.bias, blk.ffn.net_2.bias]) for blk in self.blocks])
-            gb = mods[:, :, 2::3] * biases.float().unsqueeze(1)
+            gb = (mods * torch.stack([blk.gated_biases() for blk in self.blocks]).unsqueeze(1))[:, :, 2::3]
         for i, block in enumerate(self.blocks):
             x = block(x, ctx, None, rotary, mod=mods[i], gate_bias=None if gb is None else gb[i])
         return x
@@ -542,3 +575,7 @@ class WanTransformer3DModel(nn.Module):
         with torch.no_grad():
             for k, p in own.items():
                 p.copy_(weights[k].to(device=p.device, dtype=p.dtype))
+
+
+kernels.native_classes(DistributedRMSNorm=DistributedRMSNorm, WanFeedForward=WanFeedForward, WanSelfAttention=WanSelfAttention,
+                       WanCrossAttention=WanCrossAttention)

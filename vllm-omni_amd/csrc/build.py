@@ -3,7 +3,9 @@
 Usage:  python vllm-omni_amd/csrc/build.py [--force] [--jobs N]
 
 Every translation unit is compiled to an object under csrc/build/ and linked into
-``<package>/libomni_dit_hip.so`` next to the Python sources, so the library travels with the tree.
+``<package>/libomni_dit_hip.so`` next to the Python sources, so the library travels with the tree. The native host
+path (``native.cpp``: host code against torch's headers, no device code) becomes ``<package>/_native.so``, a Python
+extension module linked against that library.
 """
 
 from __future__ import annotations
@@ -22,6 +24,8 @@ LIB_NAME = "libomni_dit_hip.so"
 LIB_PATH = PKG / LIB_NAME
 # bench.py's calibration probe (a bare MFMA loop): a library of its own, not part of the product's C ABI
 PROBE_LIB_PATH = PKG / "libomni_dit_probe.so"
+NATIVE_SRC = CSRC / "native.cpp"
+NATIVE_PATH = PKG / "_native.so"
 OBJ_DIR = CSRC / "build"
 HEADERS = [CSRC / "odit_common.h", CSRC / "attn_common.h", CSRC / "attn_tail.h", CSRC / "gemm_bf16.h",
            CSRC / "gemm_epilogue.h", PKG.parent / "include" / "omni_dit.h"]
@@ -81,6 +85,27 @@ def _run(cmd: list[str]) -> None:
         sys.stderr.write(err + "\n")
 
 
+def _native_compile(obj: Path) -> list[str]:
+    """The host compiler's command for native.cpp (torch's and Python's headers; no offload)."""
+    import sysconfig
+
+    import torch
+
+    inc = Path(torch.__file__).resolve().parent / "include"
+    return [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1",
+            "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-isystem{inc}",
+            f"-isystem{inc / 'torch' / 'csrc' / 'api' / 'include'}", "-isystem/opt/rocm/include",
+            f"-isystem{sysconfig.get_paths()['include']}", "-c", str(NATIVE_SRC), "-o", str(obj)]
+
+
+def _native_link(obj: Path, out: Path) -> list[str]:
+    import torch
+
+    lib = Path(torch.__file__).resolve().parent / "lib"
+    return [os.environ.get("CXX", "g++"), "-shared", "-o", str(out), str(obj), f"-L{PKG}", "-l:" + LIB_NAME, f"-L{lib}",
+            "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip", "-Wl,-rpath,$ORIGIN"]
+
+
 def build(force: bool = False, jobs: int | None = None, verbose: bool = True) -> Path:
     hipcc = _hipcc()
     OBJ_DIR.mkdir(exist_ok=True)
@@ -96,10 +121,13 @@ def build(force: bool = False, jobs: int | None = None, verbose: bool = True) ->
             objs[lib].append(obj)
             if force or _stale(obj, [src_path, *HEADERS, Path(__file__)]):
                 work.append([hipcc, *HIPCC_FLAGS, *defines, "-c", str(src_path), "-o", str(obj)])
+    native_obj = OBJ_DIR / "native.o"
+    native_stale = force or _stale(native_obj, [NATIVE_SRC, PKG.parent / "include" / "omni_dit.h", Path(__file__)])
+    host = [_native_compile(native_obj)] if native_stale else []
     if verbose:
-        print(f"[omni_dit build] compiling {len(work)}/{len(UNITS) + len(PROBE_UNITS)} units with {jobs} jobs", flush=True)
+        print(f"[omni_dit build] compiling {len(work) + len(host)}/{len(UNITS) + len(PROBE_UNITS) + 1} units with {jobs} jobs", flush=True)
     with ThreadPoolExecutor(max_workers=jobs) as ex:
-        list(ex.map(_run, work))
+        list(ex.map(_run, host + work))
     for lib, link in ((LIB_PATH, LINK_LIBS), (PROBE_LIB_PATH, [])):
         if work or force or not lib.exists():
             tmp = lib.with_suffix(".so.tmp")
@@ -107,6 +135,12 @@ def build(force: bool = False, jobs: int | None = None, verbose: bool = True) ->
             os.replace(tmp, lib)
         if verbose:
             print(f"[omni_dit build] {lib} ({lib.stat().st_size} bytes)", flush=True)
+    if native_stale or not NATIVE_PATH.exists():
+        tmp = NATIVE_PATH.with_suffix(".so.tmp")
+        _run(_native_link(native_obj, tmp))
+        os.replace(tmp, NATIVE_PATH)
+    if verbose:
+        print(f"[omni_dit build] {NATIVE_PATH} ({NATIVE_PATH.stat().st_size} bytes)", flush=True)
     return LIB_PATH
 
 

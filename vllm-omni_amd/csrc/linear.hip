@@ -79,6 +79,11 @@ static thread_local LinState g_lin;
 static std::mutex g_engine_mu;
 static std::unordered_map<LinKey, bool, LinKeyHash> g_handwritten_wins;
 
+// Library kernels chosen ahead of time for plain projections (odit_linear_prefer): (N, M, K, element type) -> the
+// library's own solution index. Few entries, read when a problem is first seen.
+struct Preferred { int m, n, k, dtype, solution; };
+static std::vector<Preferred> g_preferred;  // guarded by g_engine_mu
+
 #define ODIT_LT(call)                                                                      \
   do {                                                                                     \
     const hipblasStatus_t st__ = (call);                                                   \
@@ -243,6 +248,31 @@ static int lin_prepare(const LinCall& c, hipblasLtHandle_t* h, LinPlan** plan, c
   return ODIT_OK;
 }
 
+// The solution that odit_linear_prefer named for this problem (a plain projection with bias and dense rows), when the
+// library has it and it accepts the problem and the workspace.
+static bool lin_preferred_algo(hipblasLtHandle_t h, LinPlan& p, const LinCall& c, size_t lib_ws_bytes) {
+  if (c.epilogue != ODIT_EPI_BIAS || c.ldx != c.K || c.ldw != c.K || c.ldo != c.N) return false;
+  int solution = -1;
+  {
+    std::lock_guard<std::mutex> lock(g_engine_mu);
+    for (const Preferred& e : g_preferred)
+      if (e.m == c.M && e.n == c.N && e.k == c.K && e.dtype == c.dtype) { solution = e.solution; break; }
+  }
+  if (solution < 0) return false;
+  std::vector<int> index{solution};
+  std::vector<hipblasLtMatmulHeuristicResult_t> found;
+  if (hipblaslt_ext::getAlgosFromIndex(h, index, found) != HIPBLAS_STATUS_SUCCESS || found.empty()) return false;
+  const float one = 1.f, zero = 0.f;
+  size_t need = 0;
+  if (hipblaslt_ext::matmulIsAlgoSupported(h, p.desc, &one, p.a, p.b, &zero, p.c, p.d, found[0].algo, need) != HIPBLAS_STATUS_SUCCESS ||
+      need > lib_ws_bytes)
+    return false;
+  p.algo = found[0].algo;
+  p.algo_ws = need;
+  p.have_algo = true;
+  return true;
+}
+
 static int lin_default_algo(hipblasLtHandle_t h, LinPlan& p, size_t lib_ws_bytes) {
   hipblasLtMatmulPreference_t pref;
   ODIT_LT(hipblasLtMatmulPreferenceCreate(&pref));
@@ -311,7 +341,7 @@ static int lin_run_library(const odit::LinCall& c) {
   size_t lws_bytes;
   int rc = lin_prepare(c, &h, &p, &alpha, &cptr, &lws, &lws_bytes);
   if (rc != ODIT_OK) return rc;
-  if (!p->have_algo || p->algo_ws > lws_bytes) {
+  if ((!p->have_algo || p->algo_ws > lws_bytes) && !lin_preferred_algo(h, *p, c, lws_bytes)) {
     rc = lin_default_algo(h, *p, lws_bytes);
     if (rc != ODIT_OK) return rc;
   }
@@ -366,6 +396,17 @@ static bool lin_prefers_handwritten(int dev, int kind, const odit::LinCall& c, i
   }
   if (kind == 2) return false;
   return c.K >= 2 * c.N;
+}
+
+extern "C" int odit_linear_prefer(int M, int N, int K, int dtype, int solution) {
+  using namespace odit;
+  ODIT_CHECK_ARG(M > 0 && N > 0 && K > 0 && solution >= 0, "odit_linear_prefer: bad problem or solution index");
+  std::lock_guard<std::mutex> lock(g_engine_mu);
+  for (Preferred& e : g_preferred)
+    if (e.m == M && e.n == N && e.k == K && e.dtype == dtype) { e.solution = solution; return ODIT_OK; }
+  if (g_preferred.size() >= 1024) { set_error("odit_linear_prefer: more than 1024 problems"); return ODIT_EINVAL; }
+  g_preferred.push_back({M, N, K, dtype, solution});
+  return ODIT_OK;
 }
 
 extern "C" size_t odit_linear_workspace_bytes(void) {

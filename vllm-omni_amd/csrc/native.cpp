@@ -1,0 +1,1320 @@
+// The host path in native code: a CPython module (vllm_omni_amd._native) between the Python layer and the C ABI
+// of libomni_dit_hip.so.
+//
+// Two kinds of functions:
+//   * one per kernel wrapper of kernels.py: checks the tensors, takes their addresses and strides, allocates the
+//     result and calls the C entry point. A call whose arguments are not of the usual form (or that the C entry
+//     point refuses) returns None and enqueues nothing; the Python wrapper then runs its general path, which
+//     handles the unusual forms and raises the errors;
+//   * one per transformer block: the block's launches one after the other with raw addresses, its intermediate
+//     tensors carved out of ONE allocation, weights looked up in the modules' own parameter dictionaries on every
+//     call (so replaced or reloaded parameters are seen). A module tree that is not the plain one (a replaced
+//     projection, a hook on it) makes the function return None and the Python block runs.
+//
+// What it is for: a block makes about 14 launches. Through ctypes, with the tensor views and checks in Python, each
+// cost 20-35 us of host time, so every problem whose kernels take less than that (up to 512 x 512 pixels, a whole
+// block in 250-500 us) ran at the host's pace.
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+
+#include <ATen/ATen.h>
+#include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <map>
+#include <vector>
+
+#include "../../include/omni_dit.h"
+
+namespace {
+
+using at::Tensor;
+
+// ---------------------------------------------------------------------------------------------- basics
+const Tensor* tensor_of(PyObject* o) { return THPVariable_Check(o) ? &THPVariable_Unpack(o) : nullptr; }
+
+// a tensor or None; false for anything else
+bool optional_tensor(PyObject* o, const Tensor** out) {
+  *out = nullptr;
+  if (o == Py_None) return true;
+  *out = tensor_of(o);
+  return *out != nullptr;
+}
+
+int code_of(const Tensor& t) {
+  switch (t.scalar_type()) {
+    case at::kBFloat16: return ODIT_BF16;
+    case at::kHalf: return ODIT_F16;
+    case at::kFloat: return ODIT_F32;
+    default: return -1;
+  }
+}
+
+void* ptr(const Tensor* t) { return t ? t->data_ptr() : nullptr; }
+bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
+
+// the stream that work of this call goes to, and its device
+struct Where {
+  void* stream = nullptr;
+  int device = -1;
+  Where() {
+    static const bool gpu = c10::hip::device_count() > 0;
+    if (!gpu) return;  // holds nothing: every call takes the Python path, which refuses CPU tensors
+    const auto s = c10::hip::getCurrentHIPStream();
+    stream = s.stream();
+    device = s.device_index();
+  }
+  bool holds(const Tensor& t) const { return t.is_cuda() && t.device().index() == device; }
+  bool holds(const Tensor* t) const { return t == nullptr || holds(*t); }
+};
+
+PyObject* none() { Py_RETURN_NONE; }
+PyObject* wrap(Tensor t) { return THPVariable_Wrap(std::move(t)); }
+PyObject* wrap2(Tensor a, Tensor b) {
+  PyObject* r = PyTuple_New(2);
+  PyTuple_SET_ITEM(r, 0, wrap(std::move(a)));
+  PyTuple_SET_ITEM(r, 1, wrap(std::move(b)));
+  return r;
+}
+
+// C++ exceptions (allocation failures) become Python's
+#define NATIVE_BEGIN try {
+#define NATIVE_END                                        \
+  }                                                       \
+  catch (const c10::OutOfMemoryError& e) {                \
+    PyErr_SetString(PyExc_RuntimeError, e.what_without_backtrace()); \
+    return nullptr;                                       \
+  }                                                       \
+  catch (const std::exception& e) {                       \
+    PyErr_SetString(PyExc_RuntimeError, e.what());        \
+    return nullptr;                                       \
+  }
+
+// ------------------------------------------------------------------------------------------- scratch
+// Scratch belongs to kernels.py (one buffer per device and stream; launches on one stream are ordered, so they can
+// share it). The buffers handed out are remembered here, with a reference that keeps them alive; kernels.py is asked
+// when there is none yet or it is too small. All of this runs under the interpreter lock.
+PyObject* g_linear_scratch_fn = nullptr;  // (device index, stream) -> tensor
+PyObject* g_attn_scratch_fn = nullptr;    // (device index, stream, bytes) -> tensor
+
+struct Scratch { void* p = nullptr; size_t bytes = 0; };
+using ScratchPool = std::map<std::pair<int, void*>, Tensor>;
+constexpr size_t kScratchKept = 64;  // remembered (device, stream) pairs; past that all are forgotten
+
+bool scratch_from(ScratchPool& pool, const Where& w, size_t bytes, Scratch* s, PyObject* (*ask)(const Where&, size_t)) {
+  auto it = pool.find({w.device, w.stream});
+  if (it == pool.end() || static_cast<size_t>(it->second.numel()) < bytes) {
+    PyObject* got = ask(w, bytes);
+    if (got == nullptr) return false;
+    const Tensor* t = tensor_of(got);
+    if (t == nullptr) { Py_DECREF(got); PyErr_SetString(PyExc_TypeError, "scratch must be a tensor"); return false; }
+    if (pool.size() >= kScratchKept) pool.clear();
+    it = pool.insert_or_assign({w.device, w.stream}, *t).first;
+    Py_DECREF(got);
+  }
+  s->p = it->second.data_ptr();
+  s->bytes = static_cast<size_t>(it->second.numel());
+  return true;
+}
+
+bool linear_scratch(const Where& w, Scratch* s) {
+  static auto* pool = new ScratchPool;  // (never destroyed: the allocator may be gone first at process end)
+  return scratch_from(*pool, w, 1, s, [](const Where& w_, size_t) {
+    return PyObject_CallFunction(g_linear_scratch_fn, "in", w_.device, reinterpret_cast<Py_ssize_t>(w_.stream));
+  });
+}
+bool attn_scratch(const Where& w, size_t bytes, Scratch* s) {
+  static auto* pool = new ScratchPool;
+  return scratch_from(*pool, w, bytes, s, [](const Where& w_, size_t n) {
+    return PyObject_CallFunction(g_attn_scratch_fn, "inn", w_.device, reinterpret_cast<Py_ssize_t>(w_.stream),
+                                 static_cast<Py_ssize_t>(n));
+  });
+}
+
+// ---------------------------------------------------------------------------------------- activations
+template <int (*FN)(const void*, void*, int64_t, int, void*)>
+PyObject* py_unary(PyObject*, PyObject* const* a, Py_ssize_t n) {  // (x, out or None)
+  NATIVE_BEGIN
+  const Tensor *x, *o;
+  if (n != 2 || !(x = tensor_of(a[0])) || !optional_tensor(a[1], &o)) return none();
+  const Where w;
+  const int dt = code_of(*x);
+  if (dt < 0 || !w.holds(x) || !w.holds(o) || !x->is_contiguous()) return none();
+  if (o && (o->sizes() != x->sizes() || o->scalar_type() != x->scalar_type() || !o->is_contiguous())) return none();
+  Tensor out = o ? *o : at::empty_like(*x);
+  if (FN(x->data_ptr(), out.data_ptr(), x->numel(), dt, w.stream) != 0) return none();
+  if (o) { Py_INCREF(a[1]); return a[1]; }
+  return wrap(std::move(out));
+  NATIVE_END
+}
+
+// ------------------------------------------------------------------------------------------------ adaLN
+bool f32_row(const Tensor* t, int64_t C) {
+  return t == nullptr || (t->scalar_type() == at::kFloat && t->dim() > 0 && t->numel() == C && t->size(-1) == C && t->stride(-1) == 1);
+}
+
+// (x, shift, scale, eps, index, ln_weight, ln_bias, shift_bias, scale_bias, ref_rounding, out)
+PyObject* py_adaln(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  NATIVE_BEGIN
+  const Tensor *x, *sh, *sc, *index, *lw, *lb, *sb, *cb, *o;
+  if (n != 11 || !(x = tensor_of(a[0])) || !optional_tensor(a[1], &sh) || !optional_tensor(a[2], &sc) ||
+      !optional_tensor(a[4], &index) || !optional_tensor(a[5], &lw) || !optional_tensor(a[6], &lb) ||
+      !optional_tensor(a[7], &sb) || !optional_tensor(a[8], &cb) || !optional_tensor(a[10], &o))
+    return none();
+  const double eps = PyFloat_AsDouble(a[3]);
+  if (eps == -1.0 && PyErr_Occurred()) return nullptr;
+  const int rr = PyObject_IsTrue(a[9]);
+  const Where w;
+  const int dt = code_of(*x);
+  if (dt < 0 || x->dim() != 3 || x->stride(2) != 1) return none();
+  for (const Tensor* t : {x, sh, sc, index, lw, lb, sb, cb, o})
+    if (!w.holds(t)) return none();
+  const int64_t B = x->size(0), S = x->size(1), C = x->size(2);
+  const int64_t need = index ? 2 * B : B;
+  const Tensor* first = sh ? sh : sc;
+  bool per_token = first && first->dim() == 3;
+  if (per_token && index) return none();
+  int mod_dt = dt;
+  for (const Tensor* t : {sh, sc}) {
+    if (!t) continue;
+    if (per_token ? (t->dim() != 3 || t->size(0) != B || t->size(1) != S || t->size(2) != C)
+                  : (t->dim() != 2 || t->size(1) != C || t->size(0) < need))
+      return none();
+    if (t->stride(-1) != 1) return none();
+    mod_dt = code_of(*t);
+  }
+  if (sh && sc) {
+    if (sh->scalar_type() != sc->scalar_type() || sh->stride(0) != sc->stride(0)) return none();
+    if (per_token && sh->stride(1) != sc->stride(1)) return none();
+  }
+  int64_t ms = 0, mss = 0;
+  if (first) {
+    ms = first->size(0) > 1 ? first->stride(0) : 0;
+    if (per_token) mss = S > 1 ? first->stride(1) : C;
+    else if (first->size(0) == 1) ms = first->size(1);
+  }
+  if (index && (index->dim() != 2 || index->size(0) != B || index->size(1) != S || index->scalar_type() != at::kInt || !index->is_contiguous()))
+    return none();
+  if (!f32_row(lw, C) || !f32_row(lb, C) || !f32_row(sb, C) || !f32_row(cb, C)) return none();
+  if (o && (o->sizes() != x->sizes() || o->scalar_type() != x->scalar_type() || o->stride(2) != 1)) return none();
+  Tensor out = o ? *o : at::empty({B, S, C}, x->options());
+  const int64_t xs[2] = {x->stride(0), x->stride(1)}, os[2] = {out.stride(0), out.stride(1)};
+  if (odit_adaln_modulate(x->data_ptr(), out.data_ptr(), ptr(sh), ptr(sc), static_cast<const int32_t*>(ptr(index)),
+                          static_cast<const float*>(ptr(lw)), static_cast<const float*>(ptr(lb)),
+                          static_cast<const float*>(ptr(sb)), static_cast<const float*>(ptr(cb)), B, S, C, xs, os, ms, mss,
+                          static_cast<float>(eps), mod_dt, dt, rr ? ODIT_FLAG_REF_ROUNDING : 0u, w.stream) != 0)
+    return none();
+  if (o) { Py_INCREF(a[10]); return a[10]; }
+  return wrap(std::move(out));
+  NATIVE_END
+}
+
+// AdaLayerNorm.forward_hip without index and affine: (x [B,S,C], mod_params [B,3C] = shift, scale, gate, eps, ref_rounding)
+// -> (out, gate [B,1,C])
+PyObject* py_adaln_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  NATIVE_BEGIN
+  const Tensor *x, *m;
+  if (n != 4 || !(x = tensor_of(a[0])) || !(m = tensor_of(a[1]))) return none();
+  const double eps = PyFloat_AsDouble(a[2]);
+  const int rr = PyObject_IsTrue(a[3]);
+  if (PyErr_Occurred()) return nullptr;
+  const Where w;
+  const int dt = code_of(*x), mdt = code_of(*m);
+  if (dt < 0 || mdt < 0 || x->dim() != 3 || x->stride(2) != 1 || !w.holds(x) || !w.holds(m) || m->dim() != 2 ||
+      m->size(0) != x->size(0) || m->size(1) != 3 * x->size(2) || m->stride(1) != 1)
+    return none();
+  const int64_t B = x->size(0), S = x->size(1), C = x->size(2);
+  Tensor out = at::empty({B, S, C}, x->options());
+  const int64_t xs[2] = {x->stride(0), x->stride(1)}, os[2] = {S * C, C};
+  const char* mp = static_cast<const char*>(m->data_ptr());
+  if (odit_adaln_modulate(x->data_ptr(), out.data_ptr(), mp, mp + C * m->element_size(), nullptr, nullptr, nullptr, nullptr, nullptr,
+                          B, S, C, xs, os, B > 1 ? m->stride(0) : 0, 0, static_cast<float>(eps), mdt, dt,
+                          rr ? ODIT_FLAG_REF_ROUNDING : 0u, w.stream) != 0)
+    return none();
+  return wrap2(std::move(out), m->narrow(1, 2 * C, C).unsqueeze(1));
+  NATIVE_END
+}
+
+// (x0, shift0, scale0, x1, shift1, scale1, eps, ref_rounding)
+PyObject* py_adaln_pair(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  NATIVE_BEGIN
+  if (n != 8) return none();
+  const Tensor* t[6];
+  const Where w;
+  for (int i = 0; i < 6; ++i)
+    if (!(t[i] = tensor_of(a[i])) || !w.holds(t[i])) return none();
+  const double eps = PyFloat_AsDouble(a[6]);
+  if (eps == -1.0 && PyErr_Occurred()) return nullptr;
+  const int rr = PyObject_IsTrue(a[7]);
+  const Tensor &x0 = *t[0], &x1 = *t[3];
+  const int dt = code_of(x0), mdt = code_of(*t[1]);
+  if (dt < 0 || mdt < 0 || x0.dim() != 3 || x1.dim() != 3 || x1.scalar_type() != x0.scalar_type()) return none();
+  const int64_t B = x0.size(0), C = x0.size(2);
+  if (x1.size(0) != B || x1.size(2) != C) return none();
+  int64_t xs[4], os[4], ms[2];
+  int S[2];
+  const void *xp[2], *sp[2], *cp[2];
+  for (int i = 0; i < 2; ++i) {
+    const Tensor &x = *t[3 * i], &sh = *t[3 * i + 1], &sc = *t[3 * i + 2];
+    if (x.stride(2) != 1 || sh.dim() != 2 || sc.dim() != 2 || sh.size(0) != B || sc.size(0) != B || sh.size(1) != C ||
+        sc.size(1) != C || sh.stride(1) != 1 || sc.stride(1) != 1 || sh.stride(0) != sc.stride(0) ||
+        code_of(sh) != mdt || code_of(sc) != mdt)
+      return none();
+    S[i] = static_cast<int>(x.size(1));
+    xs[2 * i] = x.stride(0); xs[2 * i + 1] = x.stride(1);
+    os[2 * i] = x.size(1) * C; os[2 * i + 1] = C;
+    ms[i] = B > 1 ? sh.stride(0) : 0;
+    xp[i] = x.data_ptr(); sp[i] = sh.data_ptr(); cp[i] = sc.data_ptr();
+  }
+  Tensor o0 = at::empty({B, S[0], C}, x0.options()), o1 = at::empty({B, S[1], C}, x0.options());
+  void* op[2] = {o0.data_ptr(), o1.data_ptr()};
+  if (odit_adaln_modulate_pair(xp, op, sp, cp, B, S, C, xs, os, ms, static_cast<float>(eps), mdt, dt,
+                               rr ? ODIT_FLAG_REF_ROUNDING : 0u, w.stream) != 0)
+    return none();
+  return wrap2(std::move(o0), std::move(o1));
+  NATIVE_END
+}
+
+// ------------------------------------------------------------------------------------- QK norm + rotary
+struct QkProblem {
+  const Tensor *q, *k, *v, *wq, *wk, *cos, *sin;
+  int64_t B, S, H, D;
+  int rot, w_dtype;
+};
+
+// the checks of kernels._qk_problem
+bool qk_problem(const Where& w, const Tensor* q, const Tensor* k, const Tensor* v, const Tensor* qo, const Tensor* ko,
+                const Tensor* vo, const Tensor* wq, const Tensor* wk, const Tensor* cos, const Tensor* sin, int mode, QkProblem* p) {
+  for (const Tensor* t : {q, k, v, qo, ko, vo, wq, wk, cos, sin})
+    if (!w.holds(t)) return false;
+  if (q->dim() != 4 || code_of(*q) < 0) return false;
+  const int64_t B = q->size(0), S = q->size(1), H = q->size(2), D = q->size(3);
+  for (const Tensor* t : {q, k, v}) {
+    if (!t) continue;
+    if (t->sizes() != q->sizes() || t->scalar_type() != q->scalar_type() || t->stride(3) != 1 || t->stride(2) != D ||
+        t->stride(0) != q->stride(0) || t->stride(1) != q->stride(1))
+      return false;
+  }
+  const int64_t St = qo->dim() == 4 ? qo->size(1) : -1;
+  const Tensor* outs[3] = {qo, ko, vo};
+  const Tensor* srcs[3] = {q, k, v};
+  for (int i = 0; i < 3; ++i) {
+    const Tensor* t = outs[i];
+    if ((t == nullptr) != (srcs[i] == nullptr)) return false;
+    if (!t) continue;
+    if (t->dim() != 4 || t->size(0) != B || t->size(1) != St || t->size(2) != H || t->size(3) != D ||
+        t->scalar_type() != q->scalar_type() || !t->is_contiguous())
+      return false;
+  }
+  p->rot = 0;
+  if (cos) {
+    if (!sin || cos->dim() != 2 || cos->sizes() != sin->sizes() || cos->size(0) != S || cos->scalar_type() != at::kFloat ||
+        sin->scalar_type() != at::kFloat || !cos->is_contiguous() || !sin->is_contiguous())
+      return false;
+    p->rot = static_cast<int>(2 * cos->size(1));
+  } else if (sin) {
+    return false;
+  }
+  p->w_dtype = code_of(*q);
+  if (mode != ODIT_NORM_NONE) {
+    const int64_t want = mode == ODIT_NORM_HEAD ? D : H * D;
+    const Tensor* seen = nullptr;
+    for (const Tensor* t : {wq, wk}) {
+      if (!t) continue;
+      if (t->numel() != want || !t->is_contiguous() || code_of(*t) < 0) return false;
+      if (seen && seen->scalar_type() != t->scalar_type()) return false;
+      seen = t;
+    }
+    if (seen) p->w_dtype = code_of(*seen);
+  }
+  p->q = q; p->k = k; p->v = v; p->wq = wq; p->wk = wk; p->cos = cos; p->sin = sin;
+  p->B = B; p->S = S; p->H = H; p->D = D;
+  return true;
+}
+
+// (q, k, v, q_out, k_out, v_out, wq, wk, cos, sin, eps, out_seq_offset, norm_mode, flags) -> True or None
+PyObject* py_qknorm_rope(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  NATIVE_BEGIN
+  if (n != 14) return none();
+  const Tensor* t[10];
+  for (int i = 0; i < 10; ++i)
+    if (!optional_tensor(a[i], &t[i])) return none();
+  if (!t[0] || !t[3]) return none();
+  const double eps = PyFloat_AsDouble(a[10]);
+  const long off = PyLong_AsLong(a[11]), mode = PyLong_AsLong(a[12]), flags = PyLong_AsLong(a[13]);
+  if (PyErr_Occurred()) return nullptr;
+  const Where w;
+  QkProblem p;
+  if (!qk_problem(w, t[0], t[1], t[2], t[3], t[4], t[5], t[6], t[7], t[8], t[9], mode, &p)) return none();
+  const int64_t st[2] = {p.q->stride(0), p.q->stride(1)};
+  if (odit_qknorm_rope(ptr(p.q), ptr(p.k), ptr(p.v), t[3]->data_ptr(), ptr(t[4]), ptr(t[5]), ptr(p.wq), ptr(p.wk),
+                       static_cast<const float*>(ptr(p.cos)), static_cast<const float*>(ptr(p.sin)), p.B, p.S, p.H, p.D, p.rot,
+                       st, off, t[3]->size(1), static_cast<float>(eps), mode, p.w_dtype, code_of(*p.q), flags, w.stream) != 0)
+    return none();
+  Py_RETURN_TRUE;
+  NATIVE_END
+}
+
+// (q0, k0, v0, wq0, wk0, cos0, sin0, off0,  q1, ..., off1,  q_out, k_out, v_out, eps, norm_mode, flags) -> True or None
+PyObject* py_qknorm_rope_pair(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  NATIVE_BEGIN
+  if (n != 22) return none();
+  const Tensor *qo, *ko, *vo;
+  if (!(qo = tensor_of(a[16])) || !optional_tensor(a[17], &ko) || !optional_tensor(a[18], &vo)) return none();
+  const double eps = PyFloat_AsDouble(a[19]);
+  const long mode = PyLong_AsLong(a[20]), flags = PyLong_AsLong(a[21]);
+  if (PyErr_Occurred()) return nullptr;
+  const Where w;
+  QkProblem p[2];
+  int off[2], S[2];
+  const void *q[2], *k[2], *v[2], *wq[2], *wk[2];
+  const float *cs[2], *sn[2];
+  int64_t st[4];
+  for (int i = 0; i < 2; ++i) {
+    const Tensor* t[7];
+    for (int j = 0; j < 7; ++j)
+      if (!optional_tensor(a[8 * i + j], &t[j])) return none();
+    if (!t[0]) return none();
+    const long o = PyLong_AsLong(a[8 * i + 7]);
+    if (PyErr_Occurred()) return nullptr;
+    if (!qk_problem(w, t[0], t[1], t[2], qo, t[1] ? ko : nullptr, t[2] ? vo : nullptr, t[3], t[4], t[5], t[6], mode, &p[i])) return none();
+    off[i] = static_cast<int>(o);
+    S[i] = static_cast<int>(p[i].S);
+    q[i] = ptr(t[0]); k[i] = ptr(t[1]); v[i] = ptr(t[2]); wq[i] = ptr(t[3]); wk[i] = ptr(t[4]);
+    cs[i] = static_cast<const float*>(ptr(t[5])); sn[i] = static_cast<const float*>(ptr(t[6]));
+    st[2 * i] = t[0]->stride(0); st[2 * i + 1] = t[0]->stride(1);
+  }
+  if (p[0].B != p[1].B || p[0].H != p[1].H || p[0].D != p[1].D || p[0].rot != p[1].rot || p[0].w_dtype != p[1].w_dtype ||
+      p[0].q->scalar_type() != p[1].q->scalar_type() || (k[0] == nullptr) != (k[1] == nullptr) ||
+      (v[0] == nullptr) != (v[1] == nullptr) || (cs[0] == nullptr) != (cs[1] == nullptr))
+    return none();
+  if (odit_qknorm_rope_pair(q, k, v, qo->data_ptr(), k[0] ? ptr(ko) : nullptr, v[0] ? ptr(vo) : nullptr, wq, wk, cs, sn, p[0].B, S, p[0].H, p[0].D,
+                            p[0].rot, st, off, qo->size(1), static_cast<float>(eps), mode, p[0].w_dtype,
+                            code_of(*p[0].q), flags, w.stream) != 0)
+    return none();
+  Py_RETURN_TRUE;
+  NATIVE_END
+}
+
+// ----------------------------------------------------------------------------------------------- layers
+// RMSNorm.forward_hip: (x, weight, eps): every row of the last axis on its own
+PyObject* py_rmsnorm(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  NATIVE_BEGIN
+  const Tensor *x, *wt;
+  if (n != 3 || !(x = tensor_of(a[0])) || !(wt = tensor_of(a[1]))) return none();
+  const double eps = PyFloat_AsDouble(a[2]);
+  if (PyErr_Occurred()) return nullptr;
+  const Where w;
+  const int dt = code_of(*x);
+  if (dt < 0 || x->dim() < 1 || !w.holds(x) || !w.holds(wt) || !x->is_contiguous() || wt->scalar_type() != x->scalar_type() ||
+      !wt->is_contiguous())
+    return none();
+  const int64_t width = x->size(-1);
+  if (wt->numel() != width || width == 0) return none();
+  const int64_t rows = x->numel() / width;
+  if (rows >= (1ll << 31)) return none();
+  const int epv = dt == ODIT_F32 ? 4 : 8;
+  const int64_t lanes = width / epv;
+  int64_t hd = width;
+  int mode = ODIT_NORM_HEAD;
+  if (width % epv != 0 || lanes > 64 || (lanes & (lanes - 1)) != 0) {
+    mode = ODIT_NORM_ROW;
+    hd = 0;
+    for (int64_t d : {128, 64, 32, 16, 8})
+      if (width % d == 0) { hd = d; break; }
+    if (hd == 0) return none();
+  }
+  Tensor out = at::empty(x->sizes(), x->options());
+  const int64_t st[2] = {rows * width, width};
+  if (odit_qknorm_rope(x->data_ptr(), nullptr, nullptr, out.data_ptr(), nullptr, nullptr, wt->data_ptr(), nullptr, nullptr,
+                       nullptr, 1, static_cast<int>(rows), static_cast<int>(width / hd), static_cast<int>(hd), 0, st, 0,
+                       static_cast<int>(rows), static_cast<float>(eps), mode, dt, dt, 0u, w.stream) != 0)
+    return none();
+  return wrap(std::move(out));
+  NATIVE_END
+}
+
+// RotaryEmbedding.forward_hip: (x [B,S,H,D], cos, sin float32 [S, rot/2], flags)
+PyObject* py_rotary(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  NATIVE_BEGIN
+  const Tensor *x, *cs, *sn;
+  if (n != 4 || !(x = tensor_of(a[0])) || !(cs = tensor_of(a[1])) || !(sn = tensor_of(a[2]))) return none();
+  const long flags = PyLong_AsLong(a[3]);
+  if (PyErr_Occurred()) return nullptr;
+  const Where w;
+  if (x->dim() != 4 || code_of(*x) < 0 || !w.holds(x)) return none();
+  Tensor out = at::empty(x->sizes(), x->options());
+  QkProblem p;
+  if (!qk_problem(w, x, nullptr, nullptr, &out, nullptr, nullptr, nullptr, nullptr, cs, sn, ODIT_NORM_NONE, &p)) return none();
+  const int64_t st[2] = {x->stride(0), x->stride(1)};
+  if (odit_qknorm_rope(x->data_ptr(), nullptr, nullptr, out.data_ptr(), nullptr, nullptr, nullptr, nullptr,
+                       static_cast<const float*>(ptr(cs)), static_cast<const float*>(ptr(sn)), p.B, p.S, p.H, p.D, p.rot, st, 0,
+                       p.S, 1e-6f, ODIT_NORM_NONE, code_of(*x), code_of(*x), flags, w.stream) != 0)
+    return none();
+  return wrap(std::move(out));
+  NATIVE_END
+}
+
+// -------------------------------------------------------------------------------------------- attention
+bool attn_operand(const Tensor& t) {
+  return t.dim() == 4 && t.stride(3) == 1 && t.stride(0) % 8 == 0 && t.stride(1) % 8 == 0 && t.stride(2) % 8 == 0 && aligned16(t.data_ptr());
+}
+
+// (q, k, v, v_tail, scale, key_mask, return_lse, split (-1: none), use_workspace)
+PyObject* py_attn(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  NATIVE_BEGIN
+  const Tensor *q, *k, *v, *vt, *mask;
+  if (n != 9 || !(q = tensor_of(a[0])) || !(k = tensor_of(a[1])) || !(v = tensor_of(a[2])) || !optional_tensor(a[3], &vt) ||
+      !optional_tensor(a[5], &mask))
+    return none();
+  const double scale = PyFloat_AsDouble(a[4]);
+  const int want_lse = PyObject_IsTrue(a[6]), use_ws = PyObject_IsTrue(a[8]);
+  const long split = PyLong_AsLong(a[7]);
+  if (PyErr_Occurred()) return nullptr;
+  const Where w;
+  for (const Tensor* t : {q, k, v, vt, mask})
+    if (!w.holds(t)) return none();
+  if (!attn_operand(*q) || !attn_operand(*k) || !attn_operand(*v) || (vt && !attn_operand(*vt))) return none();
+  const int dt = code_of(*q);
+  if ((dt != ODIT_BF16 && dt != ODIT_F16) || k->scalar_type() != q->scalar_type() || v->scalar_type() != q->scalar_type() ||
+      (vt && vt->scalar_type() != q->scalar_type()))
+    return none();
+  const int64_t B = q->size(0), Sq = q->size(1), H = q->size(2), D = q->size(3), Sk = k->size(1), Hkv = k->size(2);
+  if (k->size(0) != B || k->size(3) != D || v->size(0) != B || v->size(2) != Hkv || v->size(3) != D) return none();
+  int k_split = 0;
+  if (vt) {
+    k_split = static_cast<int>(v->size(1));
+    if (vt->size(0) != B || vt->size(2) != Hkv || vt->size(3) != D || v->size(1) + vt->size(1) != Sk || k_split % 64 != 0 ||
+        k_split == 0 || vt->size(1) == 0 || v->stride(1) != vt->stride(1))
+      return none();
+  } else if (v->size(1) != Sk) {
+    return none();
+  }
+  if (mask && (mask->dim() != 2 || mask->size(0) != B || mask->size(1) != Sk || !mask->is_contiguous() ||
+               (mask->scalar_type() != at::kBool && mask->scalar_type() != at::kByte)))
+    return none();
+  if (split > Sq || B == 0 || Sq == 0 || Sk == 0) return none();
+  Scratch ws;
+  if (use_ws) {
+    const size_t need = odit_attn_fwd_workspace_bytes(B, Sq, Sk, H, D);
+    if (need > 0 && !attn_scratch(w, need, &ws)) return nullptr;
+  }
+  Tensor o = at::empty({B, split < 0 ? Sq : split, H, D}, q->options()), ot, lse;
+  if (split >= 0) ot = at::empty({B, Sq - split, H, D}, q->options());
+  if (want_lse) lse = at::empty({B, H, Sq}, q->options().dtype(at::kFloat));
+  void *head = o.data_ptr(), *tail = nullptr;
+  int64_t n_head = split < 0 ? Sq : split;
+  int cut = 0;
+  if (split == 0) { head = ot.data_ptr(); n_head = Sq; }
+  else if (split > 0 && split < Sq) { tail = ot.data_ptr(); cut = static_cast<int>(split); }
+  const int64_t qs[3] = {q->stride(0), q->stride(1), q->stride(2)}, ks[3] = {k->stride(0), k->stride(1), k->stride(2)},
+                vs[3] = {v->stride(0), v->stride(1), v->stride(2)}, os[3] = {n_head * H * D, H * D, D},
+                ts[3] = {(Sq - cut) * H * D, H * D, D};
+  int64_t vts[3] = {0, 0, 0};
+  if (vt) { vts[0] = vt->stride(0); vts[1] = vt->stride(1); vts[2] = vt->stride(2); }
+  if (odit_attn_fwd_ex(ptr(q), ptr(k), ptr(v), ptr(vt), k_split, head, tail, cut, static_cast<const uint8_t*>(ptr(mask)),
+                       want_lse ? lse.data_ptr<float>() : nullptr, B, Sq, Sk, H, Hkv, D, qs, ks, vs, vt ? vts : nullptr, os,
+                       tail ? ts : nullptr, static_cast<float>(scale), dt, ws.p, ws.bytes, w.stream) != 0)
+    return none();
+  if (split < 0 && !want_lse) return wrap(std::move(o));
+  if (split < 0) return wrap2(std::move(o), std::move(lse));
+  if (!want_lse) return wrap2(std::move(o), std::move(ot));
+  PyObject* r = PyTuple_New(3);
+  PyTuple_SET_ITEM(r, 0, wrap(std::move(o)));
+  PyTuple_SET_ITEM(r, 1, wrap(std::move(ot)));
+  PyTuple_SET_ITEM(r, 2, wrap(std::move(lse)));
+  return r;
+  NATIVE_END
+}
+
+// ----------------------------------------------------------------------------------------------- linear
+// rows of the last axis of t with one row stride (kernels._rows2d); false when they have none
+bool rows_of(const Tensor& t, int64_t* rows, int64_t* ld) {
+  const int64_t w = t.dim() > 0 ? t.size(-1) : 0;
+  if (w == 0 || t.stride(-1) != 1) return false;
+  *rows = t.numel() / w;
+  if (t.is_contiguous()) { *ld = w; return true; }
+  if (t.dim() != 2) return false;
+  *ld = *rows > 1 ? t.stride(0) : w;
+  return true;
+}
+
+// (x, weight, bias, gelu, residual, gate, gate_bias, prescaled, out, engine flags)
+PyObject* py_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  NATIVE_BEGIN
+  const Tensor *x, *wt, *b, *r, *g, *gb, *o;
+  if (n != 10 || !(x = tensor_of(a[0])) || !(wt = tensor_of(a[1])) || !optional_tensor(a[2], &b) || !optional_tensor(a[4], &r) ||
+      !optional_tensor(a[5], &g) || !optional_tensor(a[6], &gb) || !optional_tensor(a[8], &o))
+    return none();
+  const int gelu = PyObject_IsTrue(a[3]), pre = PyObject_IsTrue(a[7]);
+  const long flags = PyLong_AsLong(a[9]);
+  if (PyErr_Occurred()) return nullptr;
+  const Where w;
+  for (const Tensor* t : {x, wt, b, r, g, gb, o})
+    if (!w.holds(t)) return none();
+  const int dt = code_of(*x);
+  if (dt < 0 || x->dim() < 1 || wt->dim() != 2 || wt->stride(1) != 1 || wt->size(1) != x->size(-1) ||
+      wt->scalar_type() != x->scalar_type())
+    return none();
+  const int64_t N = wt->size(0), K = wt->size(1);
+  int64_t M, ldx, ldo, ldr = 0;
+  if (N == 0 || K == 0 || !rows_of(*x, &M, &ldx) || M == 0 || M >= (1ll << 31)) return none();
+  if (b && (b->numel() != N || !b->is_contiguous() || b->scalar_type() != x->scalar_type())) return none();
+  auto same_rows = [&](const Tensor& t, int64_t* ld) {
+    if (t.dim() != x->dim() || t.scalar_type() != x->scalar_type() || t.size(-1) != N) return false;
+    for (int64_t d = 0; d + 1 < x->dim(); ++d)
+      if (t.size(d) != x->size(d)) return false;
+    int64_t rows;
+    return rows_of(t, &rows, ld);
+  };
+  if ((o && !same_rows(*o, &ldo)) || (r && !same_rows(*r, &ldr))) return none();
+  if (g && !r) return none();
+  if (gelu && r) return none();
+  int epi, gate_code = dt, rows_per_gate = 0;
+  int64_t gstride = 0;
+  const void* bias_ptr = ptr(b);
+  if (!r) {
+    epi = gelu ? (b ? ODIT_EPI_BIAS_GELU_TANH : ODIT_EPI_GELU_TANH) : (b ? ODIT_EPI_BIAS : ODIT_EPI_NONE);
+  } else {
+    epi = pre ? ODIT_EPI_GATED_RESIDUAL_PRE : ODIT_EPI_GATED_RESIDUAL;
+    auto row_stride = [&](const Tensor& t, int64_t* st) {  // [N], or [B,N] / [B,1,N] with one row per batch row
+      if (t.stride(-1) != 1 || t.size(-1) != N) return false;
+      if (t.dim() == 1) { *st = -1; return true; }
+      if (x->dim() < 2 || t.size(0) != x->size(0)) return false;
+      if (t.dim() == 3 && t.size(1) != 1) return false;
+      if (t.dim() > 3) return false;
+      *st = t.size(0) > 1 ? t.stride(0) : -1;
+      return true;
+    };
+    if (g) {
+      if (!row_stride(*g, &gstride)) return none();
+      if (g->scalar_type() != x->scalar_type() && g->scalar_type() != at::kFloat) return none();
+      gate_code = code_of(*g);
+      if (gstride >= 0) rows_per_gate = static_cast<int>(M / x->size(0)); else gstride = 0;
+    }
+    if (pre) {
+      if (!g || gate_code != ODIT_F32) return none();
+      bias_ptr = nullptr;
+      if (gb) {
+        int64_t bs;
+        if (gb->dim() != g->dim() || gb->scalar_type() != at::kFloat || !row_stride(*gb, &bs)) return none();
+        if (rows_per_gate > 0 && bs != gstride) return none();
+        bias_ptr = gb->data_ptr();
+      }
+    } else if (gb) {
+      return none();
+    }
+  }
+  Scratch ws;
+  if (!linear_scratch(w, &ws)) return nullptr;
+  Tensor out;
+  if (o) {
+    out = *o;
+  } else {
+    auto sizes = x->sizes().vec();
+    sizes.back() = N;
+    out = at::empty(sizes, x->options());
+    ldo = N;
+  }
+  if (odit_linear_rows(x->data_ptr(), wt->data_ptr(), bias_ptr, out.data_ptr(), ptr(r), ptr(g), M, N, K, ldx,
+                       N > 1 ? wt->stride(0) : K, ldo, ldr, epi, gate_code, dt, rows_per_gate, gstride,
+                       static_cast<unsigned>(flags), ws.p, ws.bytes, w.stream) != 0)
+    return none();
+  if (o) { Py_INCREF(a[8]); return a[8]; }
+  return wrap(std::move(out));
+  NATIVE_END
+}
+
+// ------------------------------------------------------------------------------------------------ blocks
+// Reading a module tree. Everything below works on borrowed references.
+struct Names {
+  PyObject *modules, *parameters, *fwd_hooks, *pre_hooks, *forward, *weight, *bias, *eps, *elementwise_affine, *ref_rounding, *attention,
+      *softmax_scale;
+};
+Names g_name;
+PyTypeObject *g_linear_type, *g_rmsnorm_type, *g_rownorm_type, *g_adaln_type, *g_attention_type, *g_attention_impl_type,
+    *g_feed_forward_type, *g_gelu_type, *g_wan_ffn_type, *g_qwen_attention_type, *g_flux_attention_type, *g_wan_self_type, *g_wan_cross_type;
+
+PyObject* instance_dict(PyObject* m) {
+  PyObject** d = m ? _PyObject_GetDictPtr(m) : nullptr;
+  return d ? *d : nullptr;
+}
+PyObject* item(PyObject* dict, PyObject* name) { return dict && PyDict_Check(dict) ? PyDict_GetItem(dict, name) : nullptr; }
+
+// the instance dict of a module without hooks or a replaced forward; `type`: its exact class (null: any)
+PyObject* plain_module(PyObject* m, PyTypeObject* type) {
+  if (m == nullptr || (type != nullptr && Py_TYPE(m) != type)) return nullptr;
+  PyObject* d = instance_dict(m);
+  if (d == nullptr) return nullptr;
+  for (PyObject* h : {item(d, g_name.fwd_hooks), item(d, g_name.pre_hooks)})
+    if (h == nullptr || !PyDict_Check(h) || PyDict_Size(h) != 0) return nullptr;
+  if (item(d, g_name.forward) != nullptr) return nullptr;
+  return d;
+}
+// child `name` of the module whose instance dict is `d`
+PyObject* child(PyObject* d, const char* name) {
+  PyObject* mods = item(d, g_name.modules);
+  return mods && PyDict_Check(mods) ? PyDict_GetItemString(mods, name) : nullptr;
+}
+const Tensor* parameter(PyObject* d, PyObject* name) {
+  PyObject* p = item(item(d, g_name.parameters), name);
+  return p && p != Py_None ? tensor_of(p) : nullptr;
+}
+
+struct Lin {
+  const void *w = nullptr, *b = nullptr;
+  int64_t n = 0, k = 0, ldw = 0;
+};
+
+// The shared state of one block call: where it runs, its element type, and whether every operand so far was usable.
+struct BlockCall {
+  Where where;
+  Scratch lin_ws;
+  int dtype = -1;
+  at::ScalarType st = at::kBFloat16;
+  unsigned engine = 0;
+  int rc = 0;  // first non-zero status of a C call
+
+  bool operand(const Tensor& t) const { return where.holds(t) && t.scalar_type() == st; }
+
+  bool linear(PyObject* m, Lin* out, bool need_bias = true) const {
+    PyObject* d = plain_module(m, g_linear_type);
+    const Tensor *w = d ? parameter(d, g_name.weight) : nullptr, *b = d ? parameter(d, g_name.bias) : nullptr;
+    if (!w || !operand(*w) || w->dim() != 2 || w->stride(1) != 1 || (need_bias && !b)) return false;
+    if (b && (!operand(*b) || !b->is_contiguous() || b->numel() != w->size(0))) return false;
+    *out = Lin{w->data_ptr(), ptr(b), w->size(0), w->size(1), w->size(0) > 1 ? w->stride(0) : w->size(1)};
+    return true;
+  }
+  bool norm_weight(PyObject* m, PyTypeObject* type, int64_t n, const void** out, int* w_dtype) const {
+    PyObject* d = plain_module(m, type);
+    const Tensor* w = d ? parameter(d, g_name.weight) : nullptr;
+    if (!w || !where.holds(*w) || !w->is_contiguous() || w->numel() != n) return false;
+    const int c = code_of(*w);
+    if (c != dtype && c != ODIT_F32) return false;
+    if (*w_dtype >= 0 && *w_dtype != c) return false;
+    *w_dtype = c;
+    *out = w->data_ptr();
+    return true;
+  }
+  // gelu(tanh) projection and plain down-projection of a feed-forward
+  bool feed_forward(PyObject* ff, Lin* up, Lin* down) const {
+    PyObject* d = plain_module(ff, g_feed_forward_type);
+    PyObject* net = d ? child(d, "net") : nullptr;
+    PyObject* nd = net ? instance_dict(net) : nullptr;
+    PyObject* act = nd ? plain_module(child(nd, "0"), g_gelu_type) : nullptr;
+    return act && linear(child(act, "proj"), up) && linear(child(nd, "2"), down);
+  }
+  bool attention(PyObject* m, double* scale) const {
+    PyObject* d = plain_module(m, g_attention_type);
+    PyObject *impl = d ? item(d, g_name.attention) : nullptr, *s = d ? item(d, g_name.softmax_scale) : nullptr;
+    if (!impl || Py_TYPE(impl) != g_attention_impl_type || !s || !PyFloat_Check(s)) return false;
+    *scale = PyFloat_AS_DOUBLE(s);
+    return true;
+  }
+
+  void check(int status) { if (rc == 0) rc = status; }
+
+  // y[M,N] = x W^T + b with an optional GELU; rows dense
+  void project(const void* x, const Lin& l, void* y, int64_t M, bool gelu) {
+    if (rc != 0) return;
+    const int epi = gelu ? (l.b ? ODIT_EPI_BIAS_GELU_TANH : ODIT_EPI_GELU_TANH) : (l.b ? ODIT_EPI_BIAS : ODIT_EPI_NONE);
+    check(odit_linear_rows(x, l.w, l.b, y, nullptr, nullptr, M, l.n, l.k, l.k, l.ldw, l.n, 0, epi, dtype, dtype, 0, 0, engine,
+                           lin_ws.p, lin_ws.bytes, where.stream));
+  }
+};
+
+// a gate row per batch entry (and, in the pre-scaled form, the gate times the projection's bias), or no gate at all
+struct Gate {
+  const void* gate = nullptr;   // element type `dtype`, or float32 when pre
+  const void* gbias = nullptr;  // float32, pre only
+  int64_t stride = 0;           // elements between batch entries
+  bool pre = false;
+  int code = 0;                 // element type of `gate` where not pre
+};
+
+// out = residual + gate * (x W^T + b), B batch entries of S rows. The hand-written GEMM takes one gate row per
+// entry in one launch; for short entries the library's one launch per entry is slower than one launch over all rows
+// followed by the gated-residual pass (`min_rows`), which needs the `tmp` rows.
+void project_gated(BlockCall& c, const void* x, const Lin& l, const void* residual, void* out, int64_t B, int64_t S, const Gate& g,
+                   int64_t min_rows, void* tmp, const Gate& plain) {
+  if (c.rc != 0) return;
+  const int M = static_cast<int>(B * S);
+  const int epi = g.pre ? ODIT_EPI_GATED_RESIDUAL_PRE : ODIT_EPI_GATED_RESIDUAL;
+  const int rows = g.gate && B > 1 ? static_cast<int>(S) : 0;
+  const void* bias = g.pre ? g.gbias : l.b;
+  const int gcode = g.pre ? ODIT_F32 : (g.gate ? g.code : c.dtype);
+  if (rows > 0 && S < min_rows) {
+    int own = 0, launches = 0;
+    c.check(odit_linear_rows_plan(x, l.w, bias, out, residual, g.gate, M, l.n, l.k, l.k, l.ldw, l.n, l.n, epi, gcode, c.dtype, rows,
+                                  g.stride, c.engine, c.lin_ws.p, c.lin_ws.bytes, &own, &launches));
+    if (c.rc != 0) return;
+    if (!own) {
+      c.project(x, l, tmp, M, false);
+      if (c.rc != 0) return;
+      const int64_t st[2] = {S * l.n, l.n}, gs[2] = {plain.stride, 0};
+      c.check(odit_gated_residual(residual, tmp, plain.gate, nullptr, out, B, S, l.n, st, st, st, gs, plain.code, c.dtype, 0u, c.where.stream));
+      return;
+    }
+  }
+  c.check(odit_linear_rows(x, l.w, bias, out, residual, g.gate, M, l.n, l.k, l.k, l.ldw, l.n, l.n, epi, gcode, c.dtype, rows, g.stride,
+                           c.engine, c.lin_ws.p, c.lin_ws.bytes, c.where.stream));
+}
+
+// one allocation for a block's intermediate tensors
+struct Slab {
+  Tensor t;
+  size_t used = 0, size = 0;
+  int esz;
+  std::vector<std::pair<void**, size_t>> parts;
+  explicit Slab(int esz_) : esz(esz_) {}
+  void want(void** p, int64_t elements) {
+    parts.emplace_back(p, size);
+    size += (static_cast<size_t>(elements) * esz + 255) / 256 * 256;
+  }
+  void allocate(const at::TensorOptions& opts) {
+    t = at::empty({static_cast<int64_t>(size)}, opts.dtype(at::kByte));
+    for (auto& p : parts) *p.first = static_cast<char*>(t.data_ptr()) + p.second;
+  }
+};
+
+// ---- dual-stream block (Qwen-Image, Flux): stream 0 = image, 1 = text; joint rows are [text; image] -------------
+struct DualBlock {
+  Lin qkv[2], out[2], up[2], down[2];
+  const void *nq[2], *nk[2];
+  int w_dtype = -1;
+  double scale = 0, eps_qk = 0, eps[2] = {0, 0};  // eps of the first and the second norm
+  int64_t H = 0, D = 0;
+};
+
+struct ModRow {  // [B, 6C]: shift, scale, gate of the attention, then of the feed-forward
+  const char* p;
+  int64_t stride;
+};
+
+bool mod_row(const BlockCall& c, const Tensor* t, int64_t B, int64_t C, ModRow* m) {
+  if (!t || !c.operand(*t) || t->dim() != 2 || t->size(0) != B || t->size(1) != 6 * C || t->stride(1) != 1) return false;
+  m->p = static_cast<const char*>(t->data_ptr());
+  m->stride = B > 1 ? t->stride(0) : 0;
+  return true;
+}
+
+bool f32_table(const BlockCall& c, const Tensor* t, int64_t rows, int64_t cols) {
+  return t && c.where.holds(*t) && t->scalar_type() == at::kFloat && t->dim() == 2 && t->size(0) == rows && t->size(1) == cols && t->is_contiguous();
+}
+
+// gates / gate * bias rows: float32 [B, 2 (stream), 2 (attention, feed-forward), C]
+bool gate_rows(const BlockCall& c, const Tensor* t, int64_t B, int64_t C) {
+  return t && c.where.holds(*t) && t->scalar_type() == at::kFloat && t->dim() == 4 && t->size(0) == B && t->size(1) == 2 &&
+         t->size(2) == 2 && t->size(3) == C && t->stride(3) == 1;
+}
+
+// x[2]: [B,S,C] dense; tables cos/sin per stream; key_mask [B, S_txt + S_img] or null. Returns false (nothing enqueued)
+// when an operand is unusual; c.rc carries a C error.
+bool run_dual(BlockCall& c, const DualBlock& k, const Tensor& img, const Tensor& txt, const ModRow mod[2], const Tensor* gates,
+              const Tensor* gbias, const Tensor* const cos[2], const Tensor* const sin[2], const Tensor* mask, int64_t min_rows,
+              Tensor result[2]) {
+  const Tensor* x[2] = {&img, &txt};
+  const int64_t B = img.size(0), C = img.size(2), H = k.H, D = k.D, HD = H * D;
+  const int64_t S[2] = {img.size(1), txt.size(1)}, Sj = S[0] + S[1];
+  if (B * Sj >= (1ll << 31) || S[0] == 0 || S[1] == 0 || (D != 64 && D != 128)) return false;
+  int64_t F[2];
+  for (int i = 0; i < 2; ++i) {
+    F[i] = k.up[i].n;
+    if (k.qkv[i].k != C || k.qkv[i].n != 3 * HD || k.out[i].k != HD || k.out[i].n != C || k.up[i].k != C || k.down[i].k != F[i] ||
+        k.down[i].n != C)
+      return false;
+    if (!f32_table(c, cos[i], S[i], cos[0]->size(1)) || !f32_table(c, sin[i], S[i], cos[0]->size(1))) return false;
+  }
+  if (mask && (!c.where.holds(*mask) || mask->dim() != 2 || mask->size(0) != B || mask->size(1) != Sj || !mask->is_contiguous() ||
+               (mask->scalar_type() != at::kBool && mask->scalar_type() != at::kByte)))
+    return false;
+  const bool pre = gates != nullptr;
+  if (pre && (!gate_rows(c, gates, B, C) || !gate_rows(c, gbias, B, C))) return false;
+  for (int d = 0; pre && d < 3; ++d)
+    if (gates->size(d) > 1 && gates->stride(d) != gbias->stride(d)) return false;
+  const int esz = 2;
+  // values are read where the projections left them when the text rows are whole key tiles and 32-bit offsets reach them
+  const bool v_in_place = S[1] % 64 == 0 && (Sj + 64) * 3 * HD * esz < (1ll << 31);
+  const size_t attn_need = odit_attn_fwd_workspace_bytes(B, Sj, Sj, H, D);
+  Scratch attn_ws;
+  if (attn_need > 0 && !attn_scratch(c.where, attn_need, &attn_ws)) { c.rc = -100; return true; }
+
+  void *n[2], *qkv[2], *jq, *jk, *jv = nullptr, *o[2], *u[2], *tmp;
+  Slab slab(esz);
+  for (int i = 0; i < 2; ++i) {
+    slab.want(&n[i], B * S[i] * C);
+    slab.want(&qkv[i], B * S[i] * 3 * HD);
+    slab.want(&o[i], B * S[i] * HD);
+    slab.want(&u[i], B * S[i] * F[i]);
+  }
+  slab.want(&jq, B * Sj * HD);
+  slab.want(&jk, B * Sj * HD);
+  if (!v_in_place) slab.want(&jv, B * Sj * HD);
+  slab.want(&tmp, B * (S[0] > S[1] ? S[0] : S[1]) * C);
+  slab.allocate(img.options());
+  for (int i = 0; i < 2; ++i) result[i] = at::empty({B, S[i], C}, img.options());
+
+  auto norms = [&](const void* const src[2], int which) {
+    const int64_t col = which * 3 * C * esz;
+    const void *sh[2] = {mod[0].p + col, mod[1].p + col}, *sc[2] = {mod[0].p + col + C * esz, mod[1].p + col + C * esz};
+    const int Si[2] = {static_cast<int>(S[0]), static_cast<int>(S[1])};
+    const int64_t st[4] = {S[0] * C, C, S[1] * C, C}, ms[2] = {mod[0].stride, mod[1].stride};
+    void* dst[2] = {n[0], n[1]};
+    c.check(odit_adaln_modulate_pair(src, dst, sh, sc, B, Si, C, st, st, ms, static_cast<float>(k.eps[which]), c.dtype, c.dtype, 0u, c.where.stream));
+  };
+  auto gate_of = [&](int stream, int which, Gate* plain) {
+    Gate g;
+    g.gate = mod[stream].p + (which * 3 + 2) * C * esz;
+    g.stride = mod[stream].stride;
+    g.code = c.dtype;
+    *plain = g;
+    if (pre) {
+      const int64_t off = stream * gates->stride(1) + which * gates->stride(2);
+      g.gate = gates->data_ptr<float>() + off;
+      g.gbias = gbias->data_ptr<float>() + off;
+      g.stride = B > 1 ? gates->stride(0) : 0;
+      g.pre = true;
+    }
+    return g;
+  };
+
+  const void* src[2] = {x[0]->data_ptr(), x[1]->data_ptr()};
+  norms(src, 0);
+  for (int i = 0; i < 2; ++i) c.project(n[i], k.qkv[i], qkv[i], B * S[i], false);
+  if (c.rc == 0) {  // problem 0 = text rows [0, S_txt), problem 1 = image rows
+    auto part = [&](int stream, int which) { return static_cast<char*>(qkv[stream]) + which * HD * esz; };
+    const void *qi[2] = {part(1, 0), part(0, 0)}, *ki[2] = {part(1, 1), part(0, 1)},
+               *vi[2] = {v_in_place ? nullptr : part(1, 2), v_in_place ? nullptr : part(0, 2)}, *wq[2] = {k.nq[1], k.nq[0]},
+               *wk[2] = {k.nk[1], k.nk[0]};
+    const float *cs[2] = {cos[1]->data_ptr<float>(), cos[0]->data_ptr<float>()}, *sn[2] = {sin[1]->data_ptr<float>(), sin[0]->data_ptr<float>()};
+    const int Si[2] = {static_cast<int>(S[1]), static_cast<int>(S[0])}, off[2] = {0, static_cast<int>(S[1])};
+    const int64_t st[4] = {S[1] * 3 * HD, 3 * HD, S[0] * 3 * HD, 3 * HD};
+    c.check(odit_qknorm_rope_pair(qi, ki, vi, jq, jk, v_in_place ? nullptr : jv, wq, wk, cs, sn, B, Si, H, D,
+                                  static_cast<int>(2 * cos[0]->size(1)), st, off, Sj, static_cast<float>(k.eps_qk), ODIT_NORM_HEAD, k.w_dtype,
+                                  c.dtype, 0u, c.where.stream));
+  }
+  if (c.rc == 0) {
+    const int64_t js[3] = {Sj * HD, HD, D}, vt[3] = {S[1] * 3 * HD, 3 * HD, D}, vi[3] = {S[0] * 3 * HD, 3 * HD, D},
+                  ot[3] = {S[1] * HD, HD, D}, oi[3] = {S[0] * HD, HD, D};
+    const void* v0 = v_in_place ? static_cast<char*>(qkv[1]) + 2 * HD * esz : jv;
+    const void* v1 = v_in_place ? static_cast<char*>(qkv[0]) + 2 * HD * esz : nullptr;
+    c.check(odit_attn_fwd_ex(jq, jk, v0, v1, v_in_place ? static_cast<int>(S[1]) : 0, o[1], o[0], static_cast<int>(S[1]),
+                             static_cast<const uint8_t*>(ptr(mask)), nullptr, B, Sj, Sj, H, H, D, js, js, v_in_place ? vt : js,
+                             v_in_place ? vi : nullptr, ot, oi, static_cast<float>(k.scale), c.dtype, attn_ws.p, attn_ws.bytes,
+                             c.where.stream));
+  }
+  void* res[2] = {result[0].data_ptr(), result[1].data_ptr()};
+  Gate plain;
+  for (int i = 0; i < 2; ++i) {
+    const Gate g = gate_of(i, 0, &plain);
+    project_gated(c, o[i], k.out[i], src[i], res[i], B, S[i], g, min_rows, tmp, plain);
+  }
+  const void* mid[2] = {res[0], res[1]};
+  if (c.rc == 0) norms(mid, 1);
+  for (int i = 0; i < 2; ++i) {
+    c.project(n[i], k.up[i], u[i], B * S[i], true);
+    const Gate g = gate_of(i, 1, &plain);
+    project_gated(c, u[i], k.down[i], res[i], res[i], B, S[i], g, min_rows, tmp, plain);
+  }
+  return true;
+}
+
+// the float attribute `name` of a module's instance dict
+bool float_attr(PyObject* d, PyObject* name, double* v) {
+  PyObject* o = item(d, name);
+  if (!o || !PyFloat_Check(o)) return false;
+  *v = PyFloat_AS_DOUBLE(o);
+  return true;
+}
+bool is_false(PyObject* d, PyObject* name) { return item(d, name) == Py_False; }
+
+// an AdaLayerNorm without affine and reference rounding
+bool plain_adaln(PyObject* m, double* eps) {
+  PyObject* d = plain_module(m, g_adaln_type);
+  return d && is_false(d, g_name.elementwise_affine) && is_false(d, g_name.ref_rounding) && float_attr(d, g_name.eps, eps);
+}
+
+// to_qkv, add_kv_proj, the four head norms, the attention layer
+bool dual_attention(const BlockCall& c, PyObject* attn, PyTypeObject* type, DualBlock* k) {
+  PyObject* d = plain_module(attn, type);
+  if (!d || !c.linear(child(d, "to_qkv"), &k->qkv[0]) || !c.linear(child(d, "add_kv_proj"), &k->qkv[1]) ||
+      !c.linear(child(d, "to_add_out"), &k->out[1]) || !c.attention(child(d, "attn"), &k->scale) || !float_attr(d, g_name.eps, &k->eps_qk))
+    return false;
+  const char* names[4] = {"norm_q", "norm_added_q", "norm_k", "norm_added_k"};
+  for (int i = 0; i < 4; ++i) {
+    const void** out = i < 2 ? &k->nq[i] : &k->nk[i - 2];
+    if (!c.norm_weight(child(d, names[i]), g_rmsnorm_type, k->D, out, &k->w_dtype)) return false;
+  }
+  return true;
+}
+
+bool block_input(BlockCall& c, const Tensor* x) {
+  if (!x || x->dim() != 3 || !x->is_contiguous() || !c.where.holds(*x)) return false;
+  const int dt = code_of(*x);
+  if (dt != ODIT_BF16 && dt != ODIT_F16) return false;
+  c.dtype = dt;
+  c.st = x->scalar_type();
+  return linear_scratch(c.where, &c.lin_ws);
+}
+
+PyObject* block_error(int rc) {
+  if (PyErr_Occurred()) return nullptr;
+  return PyErr_Format(PyExc_RuntimeError, "native block: a kernel call failed with status %d: %s", rc, odit_last_error());
+}
+
+// Arguments of the two dual-stream blocks: (block, heads, head_dim, hidden_states, encoder_hidden_states, img mods [B,6C], txt mods [B,6C],
+// gates, gate * bias (float32 [B,2,2,C] or None), img cos, img sin, txt cos, txt sin, key mask or None, min rows, engine flags).
+// -> (encoder_hidden_states, hidden_states) or None
+PyObject* dual_block(PyObject* const* a, Py_ssize_t n, bool flux) {
+  NATIVE_BEGIN
+  if (n != 16) return none();
+  BlockCall c;
+  DualBlock k;
+  const Tensor *img = tensor_of(a[3]), *txt = tensor_of(a[4]), *m0 = tensor_of(a[5]), *m1 = tensor_of(a[6]), *gates, *gbias, *mask;
+  k.H = PyLong_AsLong(a[1]);
+  k.D = PyLong_AsLong(a[2]);
+  const int64_t min_rows = PyLong_AsLong(a[14]);
+  c.engine = static_cast<unsigned>(PyLong_AsLong(a[15]));
+  if (PyErr_Occurred()) return nullptr;
+  if (!optional_tensor(a[7], &gates) || !optional_tensor(a[8], &gbias) || !optional_tensor(a[13], &mask)) return none();
+  const Tensor *cos[2] = {tensor_of(a[9]), tensor_of(a[11])}, *sin[2] = {tensor_of(a[10]), tensor_of(a[12])};
+  if (!cos[0] || !cos[1] || !sin[0] || !sin[1] || cos[0]->dim() != 2) return none();
+  if (!block_input(c, img)) return PyErr_Occurred() ? nullptr : none();
+  if (!txt || txt->dim() != 3 || !txt->is_contiguous() || !c.operand(*txt) || txt->size(0) != img->size(0) || txt->size(2) != img->size(2)) return none();
+  const int64_t B = img->size(0), C = img->size(2);
+  ModRow mod[2];
+  if (!mod_row(c, m0, B, C, &mod[0]) || !mod_row(c, m1, B, C, &mod[1])) return none();
+  PyObject* d = instance_dict(a[0]);
+  PyObject* attn = d ? child(d, "attn") : nullptr;
+  if (!attn || !dual_attention(c, attn, flux ? g_flux_attention_type : g_qwen_attention_type, &k)) return none();
+  PyObject* attn_d = instance_dict(attn);
+  if (!flux) {
+    double e[4];
+    if (!plain_adaln(child(d, "img_norm1"), &e[0]) || !plain_adaln(child(d, "txt_norm1"), &e[1]) ||
+        !plain_adaln(child(d, "img_norm2"), &e[2]) || !plain_adaln(child(d, "txt_norm2"), &e[3]) || e[0] != e[1] || e[2] != e[3])
+      return none();
+    k.eps[0] = e[0];
+    k.eps[1] = e[2];
+    if (!c.linear(child(attn_d, "to_out"), &k.out[0]) || !c.feed_forward(child(d, "img_mlp"), &k.up[0], &k.down[0]) ||
+        !c.feed_forward(child(d, "txt_mlp"), &k.up[1], &k.down[1]))
+      return none();
+  } else {
+    PyObject *n1 = instance_dict(child(d, "norm1")), *n2 = instance_dict(child(d, "norm2")), *outs = instance_dict(child(attn_d, "to_out"));
+    if (!n1 || !n2 || !outs || !float_attr(n1, g_name.eps, &k.eps[0]) || !float_attr(n2, g_name.eps, &k.eps[1])) return none();
+    if (!c.linear(child(outs, "0"), &k.out[0]) || !c.feed_forward(child(d, "ff"), &k.up[0], &k.down[0]) ||
+        !c.feed_forward(child(d, "ff_context"), &k.up[1], &k.down[1]))
+      return none();
+  }
+  Tensor out[2];
+  if (!run_dual(c, k, *img, *txt, mod, gates, gbias, cos, sin, mask, min_rows, out)) return none();
+  if (c.rc != 0) return block_error(c.rc);
+  if (c.dtype == ODIT_F16) {  // the reference clips after every block
+    out[1].clamp_(-65504, 65504);
+    if (!flux) out[0].clamp_(-65504, 65504);
+  }
+  return wrap2(std::move(out[1]), std::move(out[0]));
+  NATIVE_END
+}
+PyObject* py_qwen_block(PyObject*, PyObject* const* a, Py_ssize_t n) { return dual_block(a, n, false); }
+PyObject* py_flux_block(PyObject*, PyObject* const* a, Py_ssize_t n) { return dual_block(a, n, true); }
+
+// ---- Flux single-stream block on a joint sequence ------------------------------------------------------------
+// (block, heads, head_dim, x [B,S,C], mods [B,3C], gate, gate * bias (float32 [B,C]), cos, sin, in_place, engine flags) -> x or None
+PyObject* py_flux_single_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  NATIVE_BEGIN
+  if (n != 11) return none();
+  BlockCall c;
+  const Tensor *x = tensor_of(a[3]), *mod = tensor_of(a[4]), *gate = tensor_of(a[5]), *gbias = tensor_of(a[6]), *cos = tensor_of(a[7]), *sin = tensor_of(a[8]);
+  const int64_t H = PyLong_AsLong(a[1]), D = PyLong_AsLong(a[2]);
+  const int in_place = PyObject_IsTrue(a[9]);
+  c.engine = static_cast<unsigned>(PyLong_AsLong(a[10]));
+  if (PyErr_Occurred()) return nullptr;
+  if (!x || !mod || !gate || !gbias || !cos || !sin || cos->dim() != 2) return none();
+  if (!block_input(c, x)) return PyErr_Occurred() ? nullptr : none();
+  const int64_t B = x->size(0), S = x->size(1), C = x->size(2), HD = H * D;
+  if (B * S >= (1ll << 31) || S == 0 || (D != 64 && D != 128) || !c.operand(*mod) || mod->dim() != 2 || mod->size(0) != B || mod->size(1) != 3 * C || mod->stride(1) != 1) return none();
+  for (const Tensor* t : {gate, gbias})
+    if (!c.where.holds(*t) || t->scalar_type() != at::kFloat || t->dim() != 2 || t->size(0) != B || t->size(1) != C || t->stride(1) != 1) return none();
+  if (B > 1 && gate->stride(0) != gbias->stride(0)) return none();
+  if (!f32_table(c, cos, S, cos->size(1)) || !f32_table(c, sin, S, cos->size(1))) return none();
+  PyObject* d = instance_dict(a[0]);
+  PyObject *norm = d ? instance_dict(child(d, "norm")) : nullptr, *attn = d ? plain_module(child(d, "attn"), g_flux_attention_type) : nullptr;
+  Lin qkv, up, down;
+  double eps, eps_qk, scale;
+  const void *wq, *wk;
+  int w_dtype = -1;
+  if (!norm || !attn || !float_attr(norm, g_name.eps, &eps) || !float_attr(attn, g_name.eps, &eps_qk) || !c.linear(child(attn, "to_qkv"), &qkv) ||
+      !c.attention(child(attn, "attn"), &scale) || !c.norm_weight(child(attn, "norm_q"), g_rmsnorm_type, D, &wq, &w_dtype) ||
+      !c.norm_weight(child(attn, "norm_k"), g_rmsnorm_type, D, &wk, &w_dtype) || !c.linear(child(d, "proj_mlp"), &up) ||
+      !c.linear(child(d, "proj_out"), &down))
+    return none();
+  const int64_t F = up.n;
+  if (HD != C || qkv.k != C || qkv.n != 3 * HD || up.k != C || down.k != C + F || down.n != C) return none();
+  const size_t attn_need = odit_attn_fwd_workspace_bytes(B, S, S, H, D);
+  Scratch attn_ws;
+  if (attn_need > 0 && !attn_scratch(c.where, attn_need, &attn_ws)) return nullptr;
+  const int esz = 2;
+  void *nx, *q3, *q, *k, *o, *u;
+  Slab slab(esz);
+  slab.want(&nx, B * S * C);
+  slab.want(&q3, B * S * 3 * HD);
+  slab.want(&q, B * S * HD);
+  slab.want(&k, B * S * HD);
+  slab.want(&o, B * S * HD);
+  slab.want(&u, B * S * F);
+  slab.allocate(x->options());
+  Tensor out = in_place ? *x : at::empty({B, S, C}, x->options());
+  const int64_t ms = B > 1 ? mod->stride(0) : 0, rs[2] = {S * C, C};
+  const char* mp = static_cast<const char*>(mod->data_ptr());
+  c.check(odit_adaln_modulate(x->data_ptr(), nx, mp, mp + C * esz, nullptr, nullptr, nullptr, nullptr, nullptr, B, S, C, rs, rs, ms, 0,
+                              static_cast<float>(eps), c.dtype, c.dtype, 0u, c.where.stream));
+  c.project(nx, up, u, B * S, true);
+  c.project(nx, qkv, q3, B * S, false);
+  const int64_t st[2] = {S * 3 * HD, 3 * HD};
+  char* qp = static_cast<char*>(q3);
+  if (c.rc == 0)
+    c.check(odit_qknorm_rope(qp, qp + HD * esz, nullptr, q, k, nullptr, wq, wk, cos->data_ptr<float>(), sin->data_ptr<float>(), B, S, H, D,
+                             static_cast<int>(2 * cos->size(1)), st, 0, S, static_cast<float>(eps_qk), ODIT_NORM_HEAD, w_dtype, c.dtype, 0u,
+                             c.where.stream));
+  if (c.rc == 0) {
+    const int64_t ds[3] = {S * HD, HD, D}, vs[3] = {S * 3 * HD, 3 * HD, D};
+    c.check(odit_attn_fwd_ex(q, k, qp + 2 * HD * esz, nullptr, 0, o, nullptr, 0, nullptr, nullptr, B, S, S, H, H, D, ds, ds, vs, nullptr, ds, nullptr,
+                             static_cast<float>(scale), c.dtype, attn_ws.p, attn_ws.bytes, c.where.stream));
+  }
+  // gate * proj_out(cat([attention, mlp])) + x as two accumulating products over the two column ranges of the weight
+  Gate g;
+  g.gate = gate->data_ptr();
+  g.gbias = gbias->data_ptr();
+  g.stride = B > 1 ? gate->stride(0) : 0;
+  g.pre = true;
+  Lin wm = down, wa = down;
+  wm.w = static_cast<const char*>(down.w) + C * esz;
+  wm.k = F;
+  wa.k = C;
+  project_gated(c, u, wm, x->data_ptr(), out.data_ptr(), B, S, g, 0, nullptr, Gate());
+  g.gbias = nullptr;
+  project_gated(c, o, wa, out.data_ptr(), out.data_ptr(), B, S, g, 0, nullptr, Gate());
+  if (c.rc != 0) return block_error(c.rc);
+  if (c.dtype == ODIT_F16) out.clamp_(-65504, 65504);
+  if (in_place) { Py_INCREF(a[3]); return a[3]; }
+  return wrap(std::move(out));
+  NATIVE_END
+}
+
+// ---- Wan block: self-attention, cross-attention to the text, feed-forward ------------------------------------------
+// (block, heads, head_dim, x [B,S,C], context [B,T,C], mod float32 [B,6,C] or None, gate * bias float32 [B,2,C] or None, temb [B,S,6,C] or None,
+//  table float32 [6,C] or None, norm2 weight, norm2 bias (float32 [C] or None), cos, sin, min rows, engine flags) -> x or None
+// (gate * bias rows lie as far apart from batch entry to batch entry as the mod rows)
+PyObject* py_wan_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  NATIVE_BEGIN
+  if (n != 15) return none();
+  BlockCall c;
+  const Tensor *x = tensor_of(a[3]), *ctx = tensor_of(a[4]), *mod, *gb, *temb, *table, *lw, *lb, *cos = tensor_of(a[11]), *sin = tensor_of(a[12]);
+  const int64_t H = PyLong_AsLong(a[1]), D = PyLong_AsLong(a[2]);
+  const int64_t min_rows = PyLong_AsLong(a[13]);
+  c.engine = static_cast<unsigned>(PyLong_AsLong(a[14]));
+  if (PyErr_Occurred()) return nullptr;
+  if (!optional_tensor(a[5], &mod) || !optional_tensor(a[6], &gb) || !optional_tensor(a[7], &temb) || !optional_tensor(a[8], &table) ||
+      !optional_tensor(a[9], &lw) || !optional_tensor(a[10], &lb) || !ctx || !cos || !sin || cos->dim() != 2)
+    return none();
+  if (!block_input(c, x)) return PyErr_Occurred() ? nullptr : none();
+  const int64_t B = x->size(0), S = x->size(1), C = x->size(2), HD = H * D, T = ctx->dim() == 3 ? ctx->size(1) : 0;
+  if (B * S >= (1ll << 31) || S == 0 || T == 0 || (D != 64 && D != 128) || !c.operand(*ctx) || !ctx->is_contiguous() || ctx->size(0) != B || ctx->size(2) != C || HD != C) return none();
+  const bool per_token = temb != nullptr;
+  if (per_token) {
+    if (!table || !c.operand(*temb) || temb->dim() != 4 || temb->size(0) != B || temb->size(1) != S || temb->size(2) != 6 || temb->size(3) != C ||
+        temb->stride(3) != 1 || !c.where.holds(*table) || table->scalar_type() != at::kFloat || !table->is_contiguous() || table->numel() != 6 * C)
+      return none();
+  } else {
+    if (!mod || !gb || !c.where.holds(*mod) || !c.where.holds(*gb) || mod->scalar_type() != at::kFloat || gb->scalar_type() != at::kFloat ||
+        mod->dim() != 3 || mod->size(0) != B || mod->size(1) != 6 || mod->size(2) != C || mod->stride(2) != 1 || gb->dim() != 3 || gb->size(0) != B ||
+        gb->size(1) != 2 || gb->size(2) != C || gb->stride(2) != 1 || (B > 1 && gb->stride(0) != mod->stride(0)))
+      return none();
+  }
+  if ((lw == nullptr) != (lb == nullptr) || !f32_row(lw, C) || !f32_row(lb, C) || !c.where.holds(lw) || !c.where.holds(lb)) return none();
+  if (!f32_table(c, cos, S, cos->size(1)) || !f32_table(c, sin, S, cos->size(1))) return none();
+  PyObject* d = instance_dict(a[0]);
+  PyObject *a1 = d ? plain_module(child(d, "attn1"), g_wan_self_type) : nullptr, *a2 = d ? plain_module(child(d, "attn2"), g_wan_cross_type) : nullptr,
+           *ffn = d ? plain_module(child(d, "ffn"), g_wan_ffn_type) : nullptr;
+  if (!a1 || !a2 || !ffn) return none();
+  PyObject* act = plain_module(child(ffn, "net_0"), g_gelu_type);
+  Lin qkv, out1, q2, k2, v2, out2, up, down;
+  double eps, scale1, scale2, eps_n[4];
+  const void* nw[4];
+  int w_dtype = -1;
+  if (!act || !float_attr(d, g_name.eps, &eps) || !c.linear(child(a1, "to_qkv"), &qkv) || !c.linear(child(a1, "to_out"), &out1) ||
+      !c.linear(child(a2, "to_q"), &q2) || !c.linear(child(a2, "to_k"), &k2) || !c.linear(child(a2, "to_v"), &v2) ||
+      !c.linear(child(a2, "to_out"), &out2) || !c.linear(child(act, "proj"), &up) || !c.linear(child(ffn, "net_2"), &down) ||
+      !c.attention(child(a1, "attn"), &scale1) || !c.attention(child(a2, "attn"), &scale2))
+    return none();
+  if (PyObject* mods2 = item(a2, g_name.modules); mods2 && PyDict_GetItemString(mods2, "add_k_proj") != nullptr &&
+      PyDict_GetItemString(mods2, "add_k_proj") != Py_None)
+    return none();  // image-conditioned cross-attention
+  PyObject* norms[4] = {child(a1, "norm_q"), child(a1, "norm_k"), child(a2, "norm_q"), child(a2, "norm_k")};
+  for (int i = 0; i < 4; ++i) {
+    if (!c.norm_weight(norms[i], g_rownorm_type, HD, &nw[i], &w_dtype) || !float_attr(instance_dict(norms[i]), g_name.eps, &eps_n[i])) return none();
+  }
+  if (eps_n[0] != eps_n[1]) return none();
+  const int64_t F = up.n;
+  if (qkv.k != C || qkv.n != 3 * HD || out1.k != HD || out1.n != C || q2.k != C || q2.n != HD || k2.k != C || k2.n != HD || v2.k != C ||
+      v2.n != HD || out2.k != HD || out2.n != C || up.k != C || down.k != F || down.n != C)
+    return none();
+  const size_t need1 = odit_attn_fwd_workspace_bytes(B, S, S, H, D), need2 = odit_attn_fwd_workspace_bytes(B, S, T, H, D);
+  Scratch ws;
+  const size_t need = need1 > need2 ? need1 : need2;
+  if (need > 0 && !attn_scratch(c.where, need, &ws)) return nullptr;
+  const int esz = 2;
+  void *nx, *q3, *q, *k, *o, *u, *kc, *kn, *vc, *y;
+  Slab slab(esz);
+  slab.want(&nx, B * S * C);
+  slab.want(&q3, B * S * 3 * HD);
+  slab.want(&q, B * S * HD);
+  slab.want(&k, B * S * HD);
+  slab.want(&o, B * S * HD);
+  slab.want(&u, B * S * F);
+  slab.want(&kc, B * T * HD);
+  slab.want(&kn, B * T * HD);
+  slab.want(&vc, B * T * HD);
+  slab.want(&y, B * S * C);
+  slab.allocate(x->options());
+  Tensor out = at::empty({B, S, C}, x->options());
+  const int64_t rs[2] = {S * C, C};
+  const char* tp = per_token ? static_cast<const char*>(temb->data_ptr()) : nullptr;
+  auto modulate = [&](const void* src, int row) {  // rows `row` (shift) and row + 1 (scale)
+    if (per_token) {
+      const float* tab = table->data_ptr<float>();
+      c.check(odit_adaln_modulate(src, nx, tp + row * temb->stride(2) * esz, tp + (row + 1) * temb->stride(2) * esz, nullptr, nullptr, nullptr,
+                                  tab + row * C, tab + (row + 1) * C, B, S, C, rs, rs, B > 1 ? temb->stride(0) : 0, S > 1 ? temb->stride(1) : C,
+                                  static_cast<float>(eps), c.dtype, c.dtype, 0u, c.where.stream));
+    } else {
+      const float* m = mod->data_ptr<float>();
+      c.check(odit_adaln_modulate(src, nx, m + row * mod->stride(1), m + (row + 1) * mod->stride(1), nullptr, nullptr, nullptr, nullptr, nullptr, B, S, C,
+                                  rs, rs, B > 1 ? mod->stride(0) : 0, 0, static_cast<float>(eps), ODIT_F32, c.dtype, 0u, c.where.stream));
+    }
+  };
+  // out = residual + gate row * (src W^T + b)
+  auto gated = [&](const void* src, const Lin& l, const void* residual, int row, int which) {
+    if (c.rc != 0) return;
+    if (per_token) {
+      c.project(src, l, y, B * S, false);
+      const int64_t gs[2] = {B > 1 ? temb->stride(0) : 0, S > 1 ? temb->stride(1) : 0};
+      if (c.rc == 0)
+        c.check(odit_gated_residual(residual, y, tp + row * temb->stride(2) * esz, table->data_ptr<float>() + row * C, out.data_ptr(), B, S, C, rs, rs, rs,
+                                    gs, c.dtype, c.dtype, 0u, c.where.stream));
+      return;
+    }
+    Gate g, plain;
+    plain.gate = g.gate = mod->data_ptr<float>() + row * mod->stride(1);
+    plain.stride = g.stride = B > 1 ? mod->stride(0) : 0;
+    plain.code = ODIT_F32;
+    g.gbias = gb->data_ptr<float>() + which * gb->stride(1);
+    g.pre = true;
+    project_gated(c, src, l, residual, out.data_ptr(), B, S, g, min_rows, y, plain);
+  };
+  modulate(x->data_ptr(), 0);
+  c.project(nx, qkv, q3, B * S, false);
+  char* qp = static_cast<char*>(q3);
+  const int64_t st3[2] = {S * 3 * HD, 3 * HD}, st1[2] = {S * HD, HD}, stc[2] = {T * HD, HD};
+  if (c.rc == 0)
+    c.check(odit_qknorm_rope(qp, qp + HD * esz, nullptr, q, k, nullptr, nw[0], nw[1], cos->data_ptr<float>(), sin->data_ptr<float>(), B, S, H, D,
+                             static_cast<int>(2 * cos->size(1)), st3, 0, S, static_cast<float>(eps_n[0]), ODIT_NORM_ROW, w_dtype, c.dtype, 0u,
+                             c.where.stream));
+  const int64_t ds[3] = {S * HD, HD, D}, vs[3] = {S * 3 * HD, 3 * HD, D}, cs3[3] = {T * HD, HD, D};
+  if (c.rc == 0)
+    c.check(odit_attn_fwd_ex(q, k, qp + 2 * HD * esz, nullptr, 0, o, nullptr, 0, nullptr, nullptr, B, S, S, H, H, D, ds, ds, vs, nullptr, ds, nullptr,
+                             static_cast<float>(scale1), c.dtype, need1 > 0 ? ws.p : nullptr, need1 > 0 ? ws.bytes : 0, c.where.stream));
+  gated(o, out1, x->data_ptr(), 2, 0);
+  const void* n2 = out.data_ptr();
+  if (c.rc == 0 && lw) {
+    c.check(odit_adaln_modulate(out.data_ptr(), nx, nullptr, nullptr, nullptr, lw->data_ptr<float>(), lb->data_ptr<float>(), nullptr, nullptr, B, S, C, rs,
+                                rs, 0, 0, static_cast<float>(eps), c.dtype, c.dtype, 0u, c.where.stream));
+    n2 = nx;
+  }
+  c.project(n2, q2, k, B * S, false);
+  c.project(ctx->data_ptr(), k2, kc, B * T, false);
+  c.project(ctx->data_ptr(), v2, vc, B * T, false);
+  if (c.rc == 0)
+    c.check(odit_qknorm_rope(k, nullptr, nullptr, q, nullptr, nullptr, nw[2], nullptr, nullptr, nullptr, B, S, H, D, 0, st1, 0, S,
+                             static_cast<float>(eps_n[2]), ODIT_NORM_ROW, w_dtype, c.dtype, 0u, c.where.stream));
+  if (c.rc == 0)
+    c.check(odit_qknorm_rope(kc, nullptr, nullptr, kn, nullptr, nullptr, nw[3], nullptr, nullptr, nullptr, B, T, H, D, 0, stc, 0, T,
+                             static_cast<float>(eps_n[3]), ODIT_NORM_ROW, w_dtype, c.dtype, 0u, c.where.stream));
+  if (c.rc == 0)
+    c.check(odit_attn_fwd_ex(q, kn, vc, nullptr, 0, o, nullptr, 0, nullptr, nullptr, B, S, T, H, H, D, ds, cs3, cs3, nullptr, ds, nullptr,
+                             static_cast<float>(scale2), c.dtype, need2 > 0 ? ws.p : nullptr, need2 > 0 ? ws.bytes : 0, c.where.stream));
+  project_gated(c, o, out2, out.data_ptr(), out.data_ptr(), B, S, Gate(), 0, nullptr, Gate());  // no gate on this residual
+  if (c.rc == 0) modulate(out.data_ptr(), 3);
+  c.project(nx, up, u, B * S, true);
+  gated(u, down, out.data_ptr(), 5, 1);
+  if (c.rc != 0) return block_error(c.rc);
+  return wrap(std::move(out));
+  NATIVE_END
+}
+
+// -------------------------------------------------------------------------------------------- module
+// (linear scratch, attention scratch)
+PyObject* py_configure(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  if (n != 2) { PyErr_SetString(PyExc_TypeError, "configure takes two callables"); return nullptr; }
+  Py_INCREF(a[0]); Py_INCREF(a[1]);
+  Py_XSETREF(g_linear_scratch_fn, a[0]);
+  Py_XSETREF(g_attn_scratch_fn, a[1]);
+  Py_RETURN_NONE;
+}
+
+// the classes whose instances the block functions recognise, by name
+PyObject* py_classes(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  if (n != 1 || !PyDict_Check(a[0])) { PyErr_SetString(PyExc_TypeError, "classes takes a dict"); return nullptr; }
+  const struct { const char* name; PyTypeObject** slot; } want[] = {
+      {"Linear", &g_linear_type}, {"RMSNorm", &g_rmsnorm_type}, {"DistributedRMSNorm", &g_rownorm_type}, {"AdaLayerNorm", &g_adaln_type},
+      {"Attention", &g_attention_type}, {"AttentionImpl", &g_attention_impl_type}, {"FeedForward", &g_feed_forward_type},
+      {"ApproxGELU", &g_gelu_type}, {"WanFeedForward", &g_wan_ffn_type}, {"QwenImageCrossAttention", &g_qwen_attention_type},
+      {"FluxAttention", &g_flux_attention_type}, {"WanSelfAttention", &g_wan_self_type}, {"WanCrossAttention", &g_wan_cross_type}};
+  for (const auto& w : want) {
+    PyObject* t = PyDict_GetItemString(a[0], w.name);
+    if (t == nullptr) continue;
+    if (!PyType_Check(t)) { PyErr_SetString(PyExc_TypeError, w.name); return nullptr; }
+    Py_INCREF(t);
+    Py_XSETREF(*w.slot, reinterpret_cast<PyTypeObject*>(t));
+  }
+  Py_RETURN_NONE;
+}
+
+bool intern_names() {
+  const struct { const char* s; PyObject** slot; } want[] = {
+      {"_modules", &g_name.modules}, {"_parameters", &g_name.parameters}, {"_forward_hooks", &g_name.fwd_hooks},
+      {"_forward_pre_hooks", &g_name.pre_hooks}, {"forward", &g_name.forward}, {"weight", &g_name.weight}, {"bias", &g_name.bias},
+      {"eps", &g_name.eps}, {"elementwise_affine", &g_name.elementwise_affine}, {"ref_rounding", &g_name.ref_rounding},
+      {"attention", &g_name.attention}, {"softmax_scale", &g_name.softmax_scale}};
+  for (const auto& w : want)
+    if ((*w.slot = PyUnicode_InternFromString(w.s)) == nullptr) return false;
+  return true;
+}
+
+#define NATIVE_FN(name, fn) {name, reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(fn)), METH_FASTCALL, nullptr}
+PyMethodDef kMethods[] = {
+    NATIVE_FN("configure", &py_configure),
+    NATIVE_FN("silu", &py_unary<odit_silu>),
+    NATIVE_FN("gelu_tanh", &py_unary<odit_gelu_tanh>),
+    NATIVE_FN("adaln", &py_adaln),
+    NATIVE_FN("adaln_layer", &py_adaln_layer),
+    NATIVE_FN("adaln_pair", &py_adaln_pair),
+    NATIVE_FN("qknorm_rope", &py_qknorm_rope),
+    NATIVE_FN("qknorm_rope_pair", &py_qknorm_rope_pair),
+    NATIVE_FN("rmsnorm", &py_rmsnorm),
+    NATIVE_FN("rotary", &py_rotary),
+    NATIVE_FN("attn", &py_attn),
+    NATIVE_FN("linear", &py_linear),
+    NATIVE_FN("classes", &py_classes),
+    NATIVE_FN("qwen_block", &py_qwen_block),
+    NATIVE_FN("flux_block", &py_flux_block),
+    NATIVE_FN("flux_single_block", &py_flux_single_block),
+    NATIVE_FN("wan_block", &py_wan_block),
+    {nullptr, nullptr, 0, nullptr}};
+
+PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_native", "native host path of the kernel wrappers", -1, kMethods,
+                       nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__native(void) { return intern_names() ? PyModule_Create(&kModule) : nullptr; }

@@ -31,7 +31,30 @@ def enable(path: os.PathLike | str = RESULTS) -> bool:
     tunable.tuning_enable(False)
     tunable.enable(True)
     tunable.read_file(os.fspath(path))
+    _prefer_in_library(Path(path), {k: v for k, v in tunable.get_validators()})
     return True
+
+
+def _prefer_in_library(path: Path, versions: dict[str, str]) -> int:
+    """The bf16 bias projections of the table for ``odit_linear`` too (the blocks' projections go there and not through
+    torch): their hipBLASLt solution indices, when the table was made with the library versions of this process.
+    Returns how many."""
+    from . import _lib
+
+    made_with, found = {}, []
+    for line in path.read_text().splitlines():
+        f = line.split(",")
+        if f[0] == "Validator":
+            made_with[f[1]] = f[2]
+        elif f[0] == "GemmAndBiasTunableOp_BFloat16_TN" and f[2].startswith("Gemm_Hipblaslt_"):
+            n, m, k = (int(v) for v in f[1].split("_")[1:4])
+            found.append((m, n, k, int(f[2].rsplit("_", 1)[1])))
+    if any(versions.get(key) != made_with.get(key) for key in ("HIPBLASLT_VERSION", "GCN_ARCH_NAME")):
+        return 0
+    lib = _lib.load()
+    for m, n, k, solution in found:
+        _lib.check(lib.odit_linear_prefer(m, n, k, _lib.ODIT_BF16, solution), "odit_linear_prefer")
+    return len(found)
 
 
 def tune(out: os.PathLike | str = RESULTS, max_seconds_per_gemm: int = 30) -> None:

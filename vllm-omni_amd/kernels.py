@@ -4,11 +4,17 @@ Each function validates on the host what the kernel assumes (device, dtype, cont
 axis, alignment is checked again inside the library), passes raw device pointers, element strides and
 torch's current HIP stream, and raises if the library reports an error. Nothing here computes: a
 missing library or a CPU tensor is an error, never a fallback.
+
+Calls of the usual form are checked and launched by the native module (``csrc/native.cpp``, a few microseconds of
+host time per call instead of 15 to 35 through the code below); it answers None, with nothing enqueued, to
+everything else, and the Python code here then handles it: operands that have to be copied or converted first,
+and the errors.
 """
 
 from __future__ import annotations
 
 import torch
+from torch.nn.modules import module as _global_hooks
 
 from . import _lib
 from ._lib import (
@@ -29,6 +35,48 @@ from ._lib import (
     ODIT_NORM_NONE,
     ODIT_NORM_ROW,
 )
+
+_nat = None
+
+
+def _load_native():
+    """The native module, told where its scratch comes from and which modules its block functions know."""
+    global _nat
+    nat = _lib.native()
+    nat.configure(_linear_scratch, _attn_scratch)
+    nat.classes(_NATIVE_CLASSES)
+    _nat = nat
+    return nat
+
+
+def native():
+    """The native module (loaded and configured on first use)."""
+    return _nat or _load_native()
+
+
+NATIVE_BLOCKS = True  # off: whole blocks go through the per-kernel wrappers below (for timing them one by one)
+
+
+def native_blocks() -> bool:
+    """Whether a transformer block may run as one native call: nothing observes its kernels or submodules."""
+    return (NATIVE_BLOCKS and _LINEAR_AUTOTUNE_ITERS == 0 and not torch.is_grad_enabled()
+            and not _global_hooks._global_forward_hooks and not _global_hooks._global_forward_pre_hooks)
+
+
+def linear_engine_flags() -> int:
+    """The engine bits that ``set_linear_engine`` chose, for the native block functions."""
+    return _LINEAR_ENGINE_FLAGS
+
+
+_NATIVE_CLASSES: dict[str, type] = {}
+
+
+def native_classes(**classes) -> None:
+    """Name the classes (exact types) whose instances the native block functions recognise as plain."""
+    _NATIVE_CLASSES.update(classes)
+    if _nat is not None:
+        _nat.classes(_NATIVE_CLASSES)
+
 
 _DTYPE_CODE = {torch.bfloat16: ODIT_BF16, torch.float16: ODIT_F16, torch.float32: ODIT_F32}
 
@@ -99,6 +147,11 @@ def attn_fwd(
     v_tail = None
     if isinstance(v, (tuple, list)):
         v, v_tail = v
+    out = (_nat or _load_native()).attn(q, k, v, v_tail, scale, key_mask, return_lse,
+                                        -1 if split is None else (split if split >= 0 else 1 << 40), use_workspace)
+    if out is not None:
+        return out
+    if v_tail is not None:
         if v.dim() != 4 or v_tail.dim() != 4 or k.dim() != 4 or v.shape[1] + v_tail.shape[1] != k.shape[1]:
             raise ValueError(f"value pair {tuple(v.shape)} + {tuple(v_tail.shape)} does not cover k {tuple(k.shape)}")
         direct = (v.dim() == 4 and v_tail.dim() == 4 and v.shape[1] % 64 == 0 and 0 < v.shape[1] and v_tail.shape[1] > 0
@@ -192,16 +245,18 @@ _ATTN_SCRATCH: dict[tuple[int, int], torch.Tensor] = {}
 
 
 def _attn_workspace(lib, device: torch.device, B: int, Sq: int, Sk: int, H: int, D: int) -> torch.Tensor | None:
+    need = int(lib.odit_attn_fwd_workspace_bytes(B, Sq, Sk, H, D))
+    return None if need == 0 else _attn_scratch(device.index or 0, _stream(), need)
+
+
+def _attn_scratch(device: int, stream: int, need: int) -> torch.Tensor:
     """Scratch for the key-split tail of the attention launch, one growing buffer per (device, stream):
     launches on one stream are ordered, so they can share it."""
-    need = int(lib.odit_attn_fwd_workspace_bytes(B, Sq, Sk, H, D))
-    if need == 0:
-        return None
-    key = (device.index or 0, _stream())
+    key = (device, stream)
     ws = _ATTN_SCRATCH.get(key)
     if ws is None or ws.numel() < need:
         # zero-filled once: the first kilobyte holds the ticket words the persistent kernel draws its units from
-        ws = torch.zeros(need, dtype=torch.uint8, device=device)
+        ws = torch.zeros(need, dtype=torch.uint8, device=torch.device("cuda", device))
         _ATTN_SCRATCH[key] = ws
     return ws
 
@@ -231,8 +286,11 @@ def qknorm_rope(
     a fused-QKV projection). *_out: dense [B,S_total,H,D]; input row s goes to row out_seq_offset+s.
     cos/sin: float32 [S, rot/2] or None.
     """
-    B, S, H, D, S_total, rot, w_dtype, cos, sin = _qk_problem(q, k, v, q_out, k_out, v_out, wq, wk, cos, sin, norm_mode)
     flags = (ODIT_FLAG_NEOX if neox else 0) | (ODIT_FLAG_REF_ROUNDING if ref_rounding else 0)
+    if (_nat or _load_native()).qknorm_rope(q, k, v, q_out, k_out, v_out, wq, wk, cos, sin, eps, out_seq_offset, norm_mode,
+                                            flags):
+        return
+    B, S, H, D, S_total, rot, w_dtype, cos, sin = _qk_problem(q, k, v, q_out, k_out, v_out, wq, wk, cos, sin, norm_mode)
     lib = _lib.load()
     rc = lib.odit_qknorm_rope(
         q.data_ptr(), _ptr(k), _ptr(v), q_out.data_ptr(), _ptr(k_out), _ptr(v_out),
@@ -297,6 +355,10 @@ def qknorm_rope_pair(first: tuple, second: tuple, q_out: torch.Tensor, k_out: to
     the image rows of a dual-stream block) in ONE launch. Each problem is
     (q, k, v, wq, wk, cos, sin, out_seq_offset) with the meaning of ``qknorm_rope``'s arguments; both take the
     same optional operands, head layout, rotary width and dtypes."""
+    flags = (ODIT_FLAG_NEOX if neox else 0) | (ODIT_FLAG_REF_ROUNDING if ref_rounding else 0)
+    if len(first) == len(second) == 8 and (_nat or _load_native()).qknorm_rope_pair(
+            *first, *second, q_out, k_out, v_out, eps, norm_mode, flags):
+        return
     probs = []
     for (q, k, v, wq, wk, cos, sin, off) in (first, second):
         B, S, H, D, S_total, rot, w_dtype, cos, sin = _qk_problem(
@@ -315,7 +377,6 @@ def qknorm_rope_pair(first: tuple, second: tuple, q_out: torch.Tensor, k_out: to
     def both(name):  # the two problems' device addresses of one operand
         return _lib.ptr_array([_ptr(a[name]), _ptr(b[name])])
 
-    flags = (ODIT_FLAG_NEOX if neox else 0) | (ODIT_FLAG_REF_ROUNDING if ref_rounding else 0)
     lib = _lib.load()
     rc = lib.odit_qknorm_rope_pair(
         both("q"), both("k"), both("v"), q_out.data_ptr(), _ptr(k_out), _ptr(v_out),
@@ -345,6 +406,9 @@ def adaln_modulate(
     """LayerNorm(x) * (1 + scale) + shift for x [B,S,C]; shift/scale [Bm,C] views of one modulation
     tensor (Bm = B, or 2B with a per-token `index` [B,S] choosing row b or b+B), or [B,S,C] views with
     one row per token. ``shift_bias`` / ``scale_bias``: float32 [C] tables added to the rows in fp32."""
+    done = (_nat or _load_native()).adaln(x, shift, scale, eps, index, ln_weight, ln_bias, shift_bias, scale_bias, ref_rounding, out)
+    if done is not None:
+        return done
     _dev(x, shift, scale, index, ln_weight, ln_bias, shift_bias, scale_bias, out)
     if x.dim() != 3:
         raise ValueError("adaln_modulate expects x [B,S,C]")
@@ -407,6 +471,9 @@ def adaln_modulate_pair(first: tuple, second: tuple, *, eps: float = 1e-6,
     """``adaln_modulate`` for two tensors of the same width and batch (the image and the text stream of a
     dual-stream block) in ONE launch. Each problem is (x [B,S,C], shift [B,C], scale [B,C]): one modulation row per
     batch entry; returns the two results."""
+    done = (_nat or _load_native()).adaln_pair(*first, *second, eps, ref_rounding)
+    if done is not None:
+        return done
     probs = []
     for (x, shift, scale) in (first, second):
         _dev(x, shift, scale)
@@ -541,11 +608,13 @@ def _unary(name: str, x: torch.Tensor, out: torch.Tensor | None) -> torch.Tensor
 
 
 def gelu_tanh(x: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
-    return _unary("odit_gelu_tanh", x, out)
+    done = (_nat or _load_native()).gelu_tanh(x, out)
+    return _unary("odit_gelu_tanh", x, out) if done is None else done
 
 
 def silu(x: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
-    return _unary("odit_silu", x, out)
+    done = (_nat or _load_native()).silu(x, out)
+    return _unary("odit_silu", x, out) if done is None else done
 
 
 # --------------------------------------------------------------------------------------------- GEMM
@@ -600,11 +669,15 @@ def linear_tuning_report() -> dict[tuple, float]:
 
 
 def _linear_workspace(lib, device: torch.device) -> torch.Tensor:
-    key = (device.index or 0, _stream())
+    return _linear_scratch(device.index or 0, _stream())
+
+
+def _linear_scratch(device: int, stream: int) -> torch.Tensor:
+    key = (device, stream)
     ws = _LINEAR_SCRATCH.get(key)
     if ws is None:
         # zero-filled once: the stream-K kernel keeps its ticket words at the start
-        ws = torch.zeros(int(lib.odit_linear_workspace_bytes()), dtype=torch.uint8, device=device)
+        ws = torch.zeros(int(_lib.load().odit_linear_workspace_bytes()), dtype=torch.uint8, device=torch.device("cuda", device))
         _LINEAR_SCRATCH[key] = ws
     return ws
 
@@ -639,6 +712,11 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = No
     if engine is not None and engine not in _LINEAR_ENGINES:
         raise ValueError(f"engine must be one of {sorted(_LINEAR_ENGINES)}")
     eflags = _LINEAR_ENGINE_FLAGS if engine is None else _LINEAR_ENGINES[engine]
+    if tune_iters == 0 and not plan_only and _LINEAR_AUTOTUNE_ITERS == 0 and (activation is None or activation == "gelu_tanh"):
+        done = (_nat or _load_native()).linear(x, weight, bias, activation is not None, residual, gate, gate_bias, prescaled, out,
+                                               eflags)
+        if done is not None:
+            return done
     _dev(x, weight, bias, residual, gate, out)
     if weight.dim() != 2 or weight.stride(1) != 1 or x.shape[-1] != weight.shape[1]:
         raise ValueError(f"weight must be [N,K] rows with K = {x.shape[-1]}, got {tuple(weight.shape)}")

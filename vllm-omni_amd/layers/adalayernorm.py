@@ -41,6 +41,10 @@ class AdaLayerNorm(CustomOp):
     def forward_hip(self, x: torch.Tensor, mod_params: torch.Tensor, index: torch.Tensor | None = None):
         if x.shape[-1] != self.hidden_size:
             raise ValueError(f"expected last dim {self.hidden_size}, got {x.shape[-1]}")
+        if index is None and not self.elementwise_affine:
+            done = kernels.native().adaln_layer(x, mod_params, self.eps, self.ref_rounding)
+            if done is not None:
+                return done
         squeeze = x.dim() == 2
         x3 = x.unsqueeze(0) if squeeze else x
         shift, scale, gate = mod_params.chunk(3, dim=-1)

@@ -21,6 +21,10 @@ class RMSNorm(CustomOp):
 
     def forward_hip(self, x: torch.Tensor) -> torch.Tensor:
         n = self.hidden_size
+        if x.shape[-1] == n:
+            out = kernels.native().rmsnorm(x, self.weight, self.variance_epsilon)
+            if out is not None:
+                return out
         if x.shape[-1] != n:
             raise ValueError(f"expected last dim {n}, got {x.shape[-1]}")
         epv = 4 if x.dtype == torch.float32 else 8

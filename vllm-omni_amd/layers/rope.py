@@ -8,7 +8,7 @@ from __future__ import annotations
 import torch
 
 from .. import kernels
-from .._lib import ODIT_NORM_NONE
+from .._lib import ODIT_FLAG_NEOX, ODIT_FLAG_REF_ROUNDING, ODIT_NORM_NONE
 from .custom_op import CustomOp
 
 
@@ -22,6 +22,10 @@ class RotaryEmbedding(CustomOp):
     def forward_hip(self, x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.Tensor:
         if cos.dim() == 3:  # (B,S,rot/2) -> first batch row, as rope.py:117-120
             cos, sin = cos[0], sin[0]
+        out = kernels.native().rotary(x, cos, sin, (ODIT_FLAG_NEOX if self.is_neox_style else 0)
+                                      | (ODIT_FLAG_REF_ROUNDING if self.ref_rounding else 0))
+        if out is not None:
+            return out
         if x.dim() != 4:
             raise ValueError("RotaryEmbedding expects x [B,S,H,D]")
         B, S, H, D = x.shape
