@@ -19,6 +19,7 @@
 
 #include <algorithm>
 #include <mutex>
+#include <string>
 #include <unordered_map>
 #include <vector>
 
@@ -273,21 +274,66 @@ static bool lin_preferred_algo(hipblasLtHandle_t h, LinPlan& p, const LinCall& c
   return true;
 }
 
-static int lin_default_algo(hipblasLtHandle_t h, LinPlan& p, size_t lib_ws_bytes) {
+// Macro tile of a library kernel, from its name ("..._MT256x192x64_..."): features x rows x reduction step. Only the
+// kernels of the usual wave layout (WG32_8, or a hand-scheduled one) with steps of 64 count: the others of the same
+// tile run 10 to 25 % slower, and the time model below was fitted without them.
+static bool lin_macro_tile(const std::string& name, int* features, int* rows) {
+  const size_t at = name.find("_MT");
+  int step = 0;
+  if (at == std::string::npos || sscanf(name.c_str() + at, "_MT%dx%dx%d", features, rows, &step) != 3 || step != 64) return false;
+  return name.rfind("Custom", 0) == 0 || name.find("_WG32_8_", at) != std::string::npos;
+}
+
+// Expected time (us) of a problem on a library kernel of one macro tile: rounds of tiles over the compute units times the
+// time of one tile, fitted to 1600 launches (bf16, 1024 <= M <= 13056, the projections of widths 3072 and 5120, last
+// round over 0.93 full; residual 9 %). The library divides a last round that is not full between the units (stream-K). At
+// K >= 8192 that costs up to a round more than its share of tiles (M=6144, N=3072, K=12288 on 256 x 160 tiles, 1.8
+// rounds: 682 us; on 192 x 192, 2.0 rounds: 340), unless the round is at least 0.88 full: then it is left undivided.
+static double lin_tile_us(int M, int N, int K, int features, int rows, int cus) {
+  const int64_t tiles = static_cast<int64_t>((N + features - 1) / features) * ((M + rows - 1) / rows);
+  const int64_t rounds = (tiles + cus - 1) / cus;
+  const double share = static_cast<double>(tiles) / cus, last = share - static_cast<double>(rounds - 1);
+  const double tile = 2.31 + K * (2.35e-7 * features * rows + 1.26e-5 * (features + rows) + 1.82e-3);
+  if (last >= 0.88 || K < 8192) return static_cast<double>(rounds) * tile;
+  return (share + std::min({1.0, share, 0.3 + last})) * tile;
+}
+
+// Problems with many rows and a long reduction take the candidate with the shortest expected time instead of the first of
+// the library's ranking. Over 58 problems with K of 12288 and 13824 the first is 25 % slower than the best of 32 on average
+// and up to 2 x, the choice made here 4 %: M=9210 (a 16:9 image being edited beside its source, two prompts), N=3072,
+// K=12288 798 -> 493 us; M=6144 682 -> 340. At K = 5120 (116 problems) the first is 7 % off, the choice 3 %. With K of 3072
+// the first is 5 % off, and what the model chose instead ran 5 % slower inside a step of 4608 rows, so it stays; below 1024
+// rows a launch is less than one round of large tiles and the model says nothing.
+constexpr int kLinRankMinRows = 1024, kLinRankMinK = 4096;
+constexpr int kLinCandidates = 32;
+
+static int lin_default_algo(hipblasLtHandle_t h, LinPlan& p, const LinCall& c, size_t lib_ws_bytes) {
   hipblasLtMatmulPreference_t pref;
   ODIT_LT(hipblasLtMatmulPreferenceCreate(&pref));
   const uint64_t maxws = lib_ws_bytes;
   hipblasLtMatmulPreferenceSetAttribute(pref, HIPBLASLT_MATMUL_PREF_MAX_WORKSPACE_BYTES, &maxws, sizeof(maxws));
-  hipblasLtMatmulHeuristicResult_t res[1];
+  const bool rank = c.M >= kLinRankMinRows && c.K >= kLinRankMinK && c.dtype != ODIT_F32;
+  hipblasLtMatmulHeuristicResult_t res[kLinCandidates];
   int n = 0;
-  const hipblasStatus_t st = hipblasLtMatmulAlgoGetHeuristic(h, p.desc, p.a, p.b, p.c, p.d, pref, 1, res, &n);
+  const hipblasStatus_t st = hipblasLtMatmulAlgoGetHeuristic(h, p.desc, p.a, p.b, p.c, p.d, pref, rank ? kLinCandidates : 1, res, &n);
   hipblasLtMatmulPreferenceDestroy(pref);
   if (st != HIPBLAS_STATUS_SUCCESS || n < 1) {
     set_error("odit_linear: hipBLASLt has no kernel for this problem (status %d)", static_cast<int>(st));
     return ODIT_ENOTSUP;
   }
-  p.algo = res[0].algo;
-  p.algo_ws = res[0].workspaceSize;
+  int best = 0;
+  double best_us = 0;
+  const int cus = rank ? device_cus() : 0;
+  for (int i = 0; i < n && cus > 0; ++i) {
+    int features, rows;
+    if (res[i].state != HIPBLAS_STATUS_SUCCESS || res[i].workspaceSize > lib_ws_bytes ||
+        !lin_macro_tile(hipblaslt_ext::getKernelNameFromAlgo(h, res[i].algo), &features, &rows))
+      continue;
+    const double us = lin_tile_us(c.M, c.N, c.K, features, rows, cus);
+    if (best_us == 0 || us < best_us) { best = i; best_us = us; }
+  }
+  p.algo = res[best].algo;
+  p.algo_ws = res[best].workspaceSize;
   p.have_algo = true;
   return ODIT_OK;
 }
@@ -342,7 +388,7 @@ static int lin_run_library(const odit::LinCall& c) {
   int rc = lin_prepare(c, &h, &p, &alpha, &cptr, &lws, &lws_bytes);
   if (rc != ODIT_OK) return rc;
   if ((!p->have_algo || p->algo_ws > lws_bytes) && !lin_preferred_algo(h, *p, c, lws_bytes)) {
-    rc = lin_default_algo(h, *p, lws_bytes);
+    rc = lin_default_algo(h, *p, c, lws_bytes);
     if (rc != ODIT_OK) return rc;
   }
   const float beta = lin_is_residual(c) ? 1.f : 0.f;
