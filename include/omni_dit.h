@@ -228,6 +228,18 @@ int odit_gated_residual(const void* h, const void* y, const void* gate, const fl
                         const int64_t out_strides[2], const int64_t gate_strides[2], int gate_dtype,
                         int dtype, unsigned flags, void* stream);
 
+/* The gated residual and the adaLN that follows it in ONE pass over dense rows [B,S,C]:
+ *     x = h + gate * y (stored, x may alias h),   out = LayerNorm(x) * (1 + scale) + shift
+ * (qwen_image_transformer.py:794-798, wan2_2_transformer.py:661-665). out == NULL: the residual alone. gate / shift / scale rows
+ * of mod_dtype at {batch, token} strides gate_strides / mod_strides; NULL, the float32 [C] tables and index as for
+ * odit_adaln_modulate and odit_gated_residual (index: rows b or b + B of gate, shift and scale alike; needs token strides of 0).
+ * C a multiple of 8 (float32: 4), up to 8192 (4096); everything 16-byte aligned. */
+int odit_gated_residual_adaln(const void* h, const void* y, const void* gate, const float* gate_bias, void* x,
+                              const void* shift, const void* scale, const float* shift_bias,
+                              const float* scale_bias, const float* ln_weight, const float* ln_bias, void* out,
+                              const int32_t* index, int B, int S, int C, const int64_t gate_strides[2],
+                              const int64_t mod_strides[2], float eps, int mod_dtype, int dtype, void* stream);
+
 /* ---------------------------------------------------------------------------------------------
  * K5  TeaCache relative-L1 reduction, per batch row:
  *        sums[b] = ( sum_i |cur[b,i] - prev[b,i]| , sum_i |prev[b,i]| )

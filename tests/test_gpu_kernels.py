@@ -40,6 +40,49 @@ def _cosine(a, b):
 
 
 # ========================================================================================= K3
+@pytest.mark.parametrize("C", [8, 512, 520, 1032, 3072, 4096, 5120, 8192])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_gated_residual_with_adaln(gpu, dtype, C):
+    """One launch against the residual and the LayerNorm written out: an indexed row choice, per-token rows with tables
+    and an affine LayerNorm, and the residual alone, at the edges of the wavefronts-per-row ranges."""
+    from vllm_omni_amd import _lib
+
+    lib, B, S = _lib.load(), 2, 5
+    g = torch.Generator().manual_seed(C)
+    rnd = lambda *s: torch.randn(*s, generator=g)
+    h, y, mod = rnd(B, S, C).to(dtype), rnd(B, S, C).to(dtype), rnd(2 * B, 3 * C).to(dtype)
+    index = torch.tensor([[0, 1, 0, 1, 1], [1, 0, 0, 0, 1]], dtype=torch.int32)
+    tab, lw, lb, temb = rnd(C), rnd(C), rnd(C), rnd(B, S, C).to(dtype)
+    d = {k: v.to(gpu) for k, v in dict(h=h, y=y, mod=mod, index=index, tab=tab, lw=lw, lb=lb, temb=temb).items()}
+    x, n = torch.full_like(d["h"], float("nan")), torch.full_like(d["h"], float("nan"))
+    p, two, code = (lambda t: None if t is None else t.data_ptr()), lambda a, b: _lib.i64_array((a, b)), 0 if dtype == torch.bfloat16 else 1
+    esz = 2
+
+    def call(gate, gate_bias, shift, scale, lw_, lb_, out, index_, gs, ms):
+        _lib.check(lib.odit_gated_residual_adaln(p(d["h"]), p(d["y"]), gate, p(gate_bias), p(x), shift, scale, None, None, p(lw_), p(lb_), p(out),
+                                                 p(index_), B, S, C, gs, ms, 1e-6, code, code, torch.cuda.current_stream().cuda_stream), "call")
+        return x.float().cpu(), n.float().cpu()
+
+    def norm(v):
+        v = v.to(dtype).float()
+        return (v - v.mean(-1, keepdim=True)) * torch.rsqrt(v.var(-1, unbiased=False, keepdim=True) + 1e-6)
+
+    row = torch.arange(B)[:, None] + B * index
+    m = mod.float()[row]                                     # [B,S,3C]: gate, shift, scale
+    want_x = h.float() + m[..., :C] * y.float()
+    want_n = norm(want_x) * (1 + m[..., 2 * C:]) + m[..., C:2 * C]
+    base, st = p(d["mod"]), two(3 * C, 0)
+    got_x, got_n = call(base, None, base + C * esz, base + 2 * C * esz, None, None, n, d["index"], st, st)
+    tol = 3e-2 if dtype == torch.bfloat16 else 4e-3
+    _close(got_x, want_x, atol=tol, rtol=1e-2, what="residual, indexed gate")
+    _close(got_n, want_n, atol=4 * tol, rtol=2e-2, what="norm behind it")
+    assert torch.equal(call(base, None, None, None, None, None, None, d["index"], st, st)[0], got_x)
+    want_x = h.float() + (temb.float() + tab) * y.float()
+    got_x, got_n = call(p(d["temb"]), d["tab"], None, None, d["lw"], d["lb"], n, None, two(S * C, C), two(0, 0))
+    _close(got_x, want_x, atol=tol, rtol=1e-2, what="residual, gate rows and table")
+    _close(got_n, norm(want_x) * lw + lb, atol=4 * tol, rtol=2e-2, what="affine norm behind it")
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("B,S,C", [(2, 33, 3072), (1, 7, 256), (2, 5, 5120), (3, 4, 40), (1, 3, 1000), (2, 3, 37)])
 def test_adaln_modulate(gpu, dtype, B, S, C):

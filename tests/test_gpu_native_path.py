@@ -32,6 +32,19 @@ def _qwen(gpu, dtype, txt, masked):
     return model, lambda: model(lat, enc, mask, t, [(1, 7, 9)], [txt, txt]).sample
 
 
+def _qwen_edit(gpu, dtype, txt, _):
+    """The editing variant: two images, a conditioning choice per token."""
+    from vllm_omni_amd.blocks.qwen_image import QwenImageTransformer2DModel
+
+    model = _init(QwenImageTransformer2DModel(num_layers=2, attention_head_dim=64, num_attention_heads=4, joint_attention_dim=256,
+                                              axes_dims_rope=(8, 28, 28), zero_cond_t=True), gpu, dtype)
+    model.fuse_modulation()
+    g = torch.Generator().manual_seed(4)
+    lat, enc = torch.randn(2, 63 + 20, 64, generator=g).to(dtype).to(gpu), torch.randn(2, txt, 256, generator=g).to(dtype).to(gpu)
+    t = torch.tensor([0.3, 0.3]).to(dtype).to(gpu)
+    return model, lambda: model(lat, enc, None, t, [[(1, 7, 9), (1, 4, 5)]] * 2, [txt, txt]).sample
+
+
 def _flux(gpu, dtype, txt, masked):
     from vllm_omni_amd.blocks.flux import FluxTransformer2DModel
 
@@ -57,7 +70,7 @@ def _wan(gpu, dtype, txt, per_token):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("make,txt,option", [(_qwen, 64, False), (_qwen, 19, True), (_flux, 64, False), (_flux, 7, False),
+@pytest.mark.parametrize("make,txt,option", [(_qwen, 64, False), (_qwen, 19, True), (_qwen_edit, 19, False), (_flux, 64, False), (_flux, 7, False),
                                              (_wan, 13, False), (_wan, 13, True)])
 def test_native_block_equals_the_per_kernel_path(gpu, monkeypatch, dtype, make, txt, option):
     from vllm_omni_amd import kernels

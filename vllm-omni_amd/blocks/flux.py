@@ -207,7 +207,7 @@ class FluxTransformerBlock(nn.Module):
             n_c = encoder_hidden_states.shape[1]
             done = kernels.native().flux_block(
                 self, self.attn.heads, self.attn.head_dim, hidden_states, encoder_hidden_states, *mod_params, g, gb,
-                *rotary.split(n_c), None, qwen_image.FUSE_MIN_ROWS, kernels.linear_engine_flags())
+                *rotary.split(n_c), None, qwen_image.FUSE_MIN_ROWS, kernels.linear_engine_flags(), None)
             if done is not None:
                 return done
         pre = [[None, None], [None, None]]

@@ -375,12 +375,12 @@ class QwenImageTransformerBlock(nn.Module):
         if joint_mask is None:
             joint_mask = joint_key_mask(encoder_hidden_states_mask, hidden_states_mask, hidden_states.shape[0],
                                         encoder_hidden_states.shape[1], hidden_states.shape[1], hidden_states.device)
-        if self.fused and modulate_index is None and kernels.native_blocks():
-            g, gb = gate_rows if gate_rows is not None else (None, None)
+        if self.fused and kernels.native_blocks():
+            g, gb = gate_rows if gate_rows is not None and modulate_index is None else (None, None)
             done = kernels.native().qwen_block(
                 self, self.num_attention_heads, self.attention_head_dim, hidden_states, encoder_hidden_states, img_mod_params,
                 txt_mod_params, g, gb, tables.img_cos, tables.img_sin, tables.txt_cos, tables.txt_sin, joint_mask, FUSE_MIN_ROWS,
-                kernels.linear_engine_flags())
+                kernels.linear_engine_flags(), modulate_index)
             if done is not None:
                 return done
         pre = [[None, None], [None, None]]

@@ -792,10 +792,10 @@ struct ModRow {  // [B, 6C]: shift, scale, gate of the attention, then of the fe
   int64_t stride;
 };
 
-bool mod_row(const BlockCall& c, const Tensor* t, int64_t B, int64_t C, ModRow* m) {
-  if (!t || !c.operand(*t) || t->dim() != 2 || t->size(0) != B || t->size(1) != 6 * C || t->stride(1) != 1) return false;
+bool mod_row(const BlockCall& c, const Tensor* t, int64_t rows, int64_t C, ModRow* m) {
+  if (!t || !c.operand(*t) || t->dim() != 2 || t->size(0) != rows || t->size(1) != 6 * C || t->stride(1) != 1) return false;
   m->p = static_cast<const char*>(t->data_ptr());
-  m->stride = B > 1 ? t->stride(0) : 0;
+  m->stride = rows > 1 ? t->stride(0) : 0;
   return true;
 }
 
@@ -809,11 +809,12 @@ bool gate_rows(const BlockCall& c, const Tensor* t, int64_t B, int64_t C) {
          t->size(2) == 2 && t->size(3) == C && t->stride(3) == 1;
 }
 
-// x[2]: [B,S,C] dense; tables cos/sin per stream; key_mask [B, S_txt + S_img] or null. Returns false (nothing enqueued)
-// when an operand is unusual; c.rc carries a C error.
+// x[2]: [B,S,C] dense; tables cos/sin per stream; key_mask [B, S_txt + S_img] or null; index: int32 [B, S_img] or null, the
+// image stream's choice between modulation rows b and b + B. Returns false (nothing enqueued) when an operand is unusual;
+// c.rc carries a C error.
 bool run_dual(BlockCall& c, const DualBlock& k, const Tensor& img, const Tensor& txt, const ModRow mod[2], const Tensor* gates,
-              const Tensor* gbias, const Tensor* const cos[2], const Tensor* const sin[2], const Tensor* mask, int64_t min_rows,
-              Tensor result[2]) {
+              const Tensor* gbias, const Tensor* const cos[2], const Tensor* const sin[2], const Tensor* mask, const Tensor* index,
+              int64_t min_rows, Tensor result[2]) {
   const Tensor* x[2] = {&img, &txt};
   const int64_t B = img.size(0), C = img.size(2), H = k.H, D = k.D, HD = H * D;
   const int64_t S[2] = {img.size(1), txt.size(1)}, Sj = S[0] + S[1];
@@ -829,6 +830,10 @@ bool run_dual(BlockCall& c, const DualBlock& k, const Tensor& img, const Tensor&
   if (mask && (!c.where.holds(*mask) || mask->dim() != 2 || mask->size(0) != B || mask->size(1) != Sj || !mask->is_contiguous() ||
                (mask->scalar_type() != at::kBool && mask->scalar_type() != at::kByte)))
     return false;
+  if (index && (!c.where.holds(*index) || index->scalar_type() != at::kInt || index->dim() != 2 || index->size(0) != B || index->size(1) != S[0] ||
+                !index->is_contiguous() || C % 8 != 0 || C > 8192))
+    return false;
+  const int32_t* idx = index ? index->data_ptr<int32_t>() : nullptr;
   const bool pre = gates != nullptr;
   if (pre && (!gate_rows(c, gates, B, C) || !gate_rows(c, gbias, B, C))) return false;
   for (int d = 0; pre && d < 3; ++d)
@@ -855,13 +860,29 @@ bool run_dual(BlockCall& c, const DualBlock& k, const Tensor& img, const Tensor&
   slab.allocate(img.options());
   for (int i = 0; i < 2; ++i) result[i] = at::empty({B, S[i], C}, img.options());
 
+  const int64_t rows[2][2] = {{S[0] * C, C}, {S[1] * C, C}};
+  auto mod_at = [&](int stream, int col) { return mod[stream].p + col * C * esz; };
+  auto norm = [&](int stream, const void* src, int which) {
+    if (c.rc != 0) return;
+    c.check(odit_adaln_modulate(src, n[stream], mod_at(stream, 3 * which), mod_at(stream, 3 * which + 1), stream == 0 ? idx : nullptr, nullptr, nullptr,
+                                nullptr, nullptr, B, S[stream], C, rows[stream], rows[stream], mod[stream].stride, 0,
+                                static_cast<float>(k.eps[which]), c.dtype, c.dtype, 0u, c.where.stream));
+  };
   auto norms = [&](const void* const src[2], int which) {
-    const int64_t col = which * 3 * C * esz;
-    const void *sh[2] = {mod[0].p + col, mod[1].p + col}, *sc[2] = {mod[0].p + col + C * esz, mod[1].p + col + C * esz};
+    const void *sh[2] = {mod_at(0, 3 * which), mod_at(1, 3 * which)}, *sc[2] = {mod_at(0, 3 * which + 1), mod_at(1, 3 * which + 1)};
     const int Si[2] = {static_cast<int>(S[0]), static_cast<int>(S[1])};
     const int64_t st[4] = {S[0] * C, C, S[1] * C, C}, ms[2] = {mod[0].stride, mod[1].stride};
     void* dst[2] = {n[0], n[1]};
     c.check(odit_adaln_modulate_pair(src, dst, sh, sc, B, Si, C, st, st, ms, static_cast<float>(k.eps[which]), c.dtype, c.dtype, 0u, c.where.stream));
+  };
+  // image rows with a gate per token: the projection, then residual + gate (and the second norm behind the first of them)
+  auto indexed = [&](const void* a, const Lin& l, const void* residual, void* out, int which) {
+    c.project(a, l, tmp, B * S[0], false);
+    if (c.rc != 0) return;
+    const int64_t st[2] = {mod[0].stride, 0};
+    c.check(odit_gated_residual_adaln(residual, tmp, mod_at(0, 3 * which + 2), nullptr, out, which == 0 ? mod_at(0, 3) : nullptr,
+                                      which == 0 ? mod_at(0, 4) : nullptr, nullptr, nullptr, nullptr, nullptr, which == 0 ? n[0] : nullptr, idx, B,
+                                      S[0], C, st, st, static_cast<float>(k.eps[1]), c.dtype, c.dtype, c.where.stream));
   };
   auto gate_of = [&](int stream, int which, Gate* plain) {
     Gate g;
@@ -880,7 +901,12 @@ bool run_dual(BlockCall& c, const DualBlock& k, const Tensor& img, const Tensor&
   };
 
   const void* src[2] = {x[0]->data_ptr(), x[1]->data_ptr()};
-  norms(src, 0);
+  if (idx) {
+    norm(0, src[0], 0);
+    norm(1, src[1], 0);
+  } else {
+    norms(src, 0);
+  }
   for (int i = 0; i < 2; ++i) c.project(n[i], k.qkv[i], qkv[i], B * S[i], false);
   if (c.rc == 0) {  // problem 0 = text rows [0, S_txt), problem 1 = image rows
     auto part = [&](int stream, int which) { return static_cast<char*>(qkv[stream]) + which * HD * esz; };
@@ -907,13 +933,16 @@ bool run_dual(BlockCall& c, const DualBlock& k, const Tensor& img, const Tensor&
   void* res[2] = {result[0].data_ptr(), result[1].data_ptr()};
   Gate plain;
   for (int i = 0; i < 2; ++i) {
+    if (i == 0 && idx) { indexed(o[0], k.out[0], src[0], res[0], 0); continue; }
     const Gate g = gate_of(i, 0, &plain);
     project_gated(c, o[i], k.out[i], src[i], res[i], B, S[i], g, min_rows, tmp, plain);
   }
   const void* mid[2] = {res[0], res[1]};
-  if (c.rc == 0) norms(mid, 1);
+  if (idx) norm(1, mid[1], 1);
+  else if (c.rc == 0) norms(mid, 1);
   for (int i = 0; i < 2; ++i) {
     c.project(n[i], k.up[i], u[i], B * S[i], true);
+    if (i == 0 && idx) { indexed(u[0], k.down[0], res[0], res[0], 1); continue; }
     const Gate g = gate_of(i, 1, &plain);
     project_gated(c, u[i], k.down[i], res[i], res[i], B, S[i], g, min_rows, tmp, plain);
   }
@@ -964,27 +993,30 @@ PyObject* block_error(int rc) {
 }
 
 // Arguments of the two dual-stream blocks: (block, heads, head_dim, hidden_states, encoder_hidden_states, img mods [B,6C], txt mods [B,6C],
-// gates, gate * bias (float32 [B,2,2,C] or None), img cos, img sin, txt cos, txt sin, key mask or None, min rows, engine flags).
+// gates, gate * bias (float32 [B,2,2,C] or None), img cos, img sin, txt cos, txt sin, key mask or None, min rows, engine flags,
+// modulation index int32 [B,S_img] or None (then the img mods are [2B,6C] and there are no gates)).
 // -> (encoder_hidden_states, hidden_states) or None
 PyObject* dual_block(PyObject* const* a, Py_ssize_t n, bool flux) {
   NATIVE_BEGIN
-  if (n != 16) return none();
+  if (n != 17) return none();
   BlockCall c;
   DualBlock k;
-  const Tensor *img = tensor_of(a[3]), *txt = tensor_of(a[4]), *m0 = tensor_of(a[5]), *m1 = tensor_of(a[6]), *gates, *gbias, *mask;
+  const Tensor *img = tensor_of(a[3]), *txt = tensor_of(a[4]), *m0 = tensor_of(a[5]), *m1 = tensor_of(a[6]), *gates, *gbias, *mask, *index;
   k.H = PyLong_AsLong(a[1]);
   k.D = PyLong_AsLong(a[2]);
   const int64_t min_rows = PyLong_AsLong(a[14]);
   c.engine = static_cast<unsigned>(PyLong_AsLong(a[15]));
   if (PyErr_Occurred()) return nullptr;
-  if (!optional_tensor(a[7], &gates) || !optional_tensor(a[8], &gbias) || !optional_tensor(a[13], &mask)) return none();
+  if (!optional_tensor(a[7], &gates) || !optional_tensor(a[8], &gbias) || !optional_tensor(a[13], &mask) || !optional_tensor(a[16], &index) ||
+      (index && gates))
+    return none();
   const Tensor *cos[2] = {tensor_of(a[9]), tensor_of(a[11])}, *sin[2] = {tensor_of(a[10]), tensor_of(a[12])};
   if (!cos[0] || !cos[1] || !sin[0] || !sin[1] || cos[0]->dim() != 2) return none();
   if (!block_input(c, img)) return PyErr_Occurred() ? nullptr : none();
   if (!txt || txt->dim() != 3 || !txt->is_contiguous() || !c.operand(*txt) || txt->size(0) != img->size(0) || txt->size(2) != img->size(2)) return none();
   const int64_t B = img->size(0), C = img->size(2);
   ModRow mod[2];
-  if (!mod_row(c, m0, B, C, &mod[0]) || !mod_row(c, m1, B, C, &mod[1])) return none();
+  if (!mod_row(c, m0, index ? 2 * B : B, C, &mod[0]) || !mod_row(c, m1, B, C, &mod[1])) return none();
   PyObject* d = instance_dict(a[0]);
   PyObject* attn = d ? child(d, "attn") : nullptr;
   if (!attn || !dual_attention(c, attn, flux ? g_flux_attention_type : g_qwen_attention_type, &k)) return none();
@@ -1007,7 +1039,7 @@ PyObject* dual_block(PyObject* const* a, Py_ssize_t n, bool flux) {
       return none();
   }
   Tensor out[2];
-  if (!run_dual(c, k, *img, *txt, mod, gates, gbias, cos, sin, mask, min_rows, out)) return none();
+  if (!run_dual(c, k, *img, *txt, mod, gates, gbias, cos, sin, mask, index, min_rows, out)) return none();
   if (c.rc != 0) return block_error(c.rc);
   if (c.dtype == ODIT_F16) {  // the reference clips after every block
     out[1].clamp_(-65504, 65504);
@@ -1194,12 +1226,17 @@ PyObject* py_wan_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
     }
   };
   // out = residual + gate row * (src W^T + b)
+  const bool norm2_fused = per_token && lw && C % 8 == 0 && C <= 8192;  // with the residual in front of it
   auto gated = [&](const void* src, const Lin& l, const void* residual, int row, int which) {
     if (c.rc != 0) return;
     if (per_token) {
       c.project(src, l, y, B * S, false);
-      const int64_t gs[2] = {B > 1 ? temb->stride(0) : 0, S > 1 ? temb->stride(1) : 0};
-      if (c.rc == 0)
+      const int64_t gs[2] = {B > 1 ? temb->stride(0) : 0, S > 1 ? temb->stride(1) : 0}, none[2] = {0, 0};
+      if (c.rc == 0 && which == 0 && norm2_fused)
+        c.check(odit_gated_residual_adaln(residual, y, tp + row * temb->stride(2) * esz, table->data_ptr<float>() + row * C, out.data_ptr(), nullptr,
+                                          nullptr, nullptr, nullptr, lw->data_ptr<float>(), lb->data_ptr<float>(), nx, nullptr, B, S, C, gs, none,
+                                          static_cast<float>(eps), c.dtype, c.dtype, c.where.stream));
+      else if (c.rc == 0)
         c.check(odit_gated_residual(residual, y, tp + row * temb->stride(2) * esz, table->data_ptr<float>() + row * C, out.data_ptr(), B, S, C, rs, rs, rs,
                                     gs, c.dtype, c.dtype, 0u, c.where.stream));
       return;
@@ -1226,7 +1263,9 @@ PyObject* py_wan_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
                              static_cast<float>(scale1), c.dtype, need1 > 0 ? ws.p : nullptr, need1 > 0 ? ws.bytes : 0, c.where.stream));
   gated(o, out1, x->data_ptr(), 2, 0);
   const void* n2 = out.data_ptr();
-  if (c.rc == 0 && lw) {
+  if (norm2_fused) {
+    n2 = nx;
+  } else if (c.rc == 0 && lw) {
     c.check(odit_adaln_modulate(out.data_ptr(), nx, nullptr, nullptr, nullptr, lw->data_ptr<float>(), lb->data_ptr<float>(), nullptr, nullptr, B, S, C, rs,
                                 rs, 0, 0, static_cast<float>(eps), c.dtype, c.dtype, 0u, c.where.stream));
     n2 = nx;
