@@ -277,11 +277,12 @@ static bool lin_preferred_algo(hipblasLtHandle_t h, LinPlan& p, const LinCall& c
 // Macro tile of a library kernel, from its name ("..._MT256x192x64_..."): features x rows x reduction step. Only the
 // kernels of the usual wave layout (WG32_8, or a hand-scheduled one) with steps of 64 count: the others of the same
 // tile run 10 to 25 % slower, and the time model below was fitted without them.
-static bool lin_macro_tile(const std::string& name, int* features, int* rows) {
+static bool lin_macro_tile(const std::string& name, int* features, int* rows, bool* usual) {
   const size_t at = name.find("_MT");
   int step = 0;
-  if (at == std::string::npos || sscanf(name.c_str() + at, "_MT%dx%dx%d", features, rows, &step) != 3 || step != 64) return false;
-  return name.rfind("Custom", 0) == 0 || name.find("_WG32_8_", at) != std::string::npos;
+  if (at == std::string::npos || sscanf(name.c_str() + at, "_MT%dx%dx%d", features, rows, &step) != 3) return false;
+  *usual = step == 64 && (name.rfind("Custom", 0) == 0 || name.find("_WG32_8_", at) != std::string::npos);
+  return true;
 }
 
 // Expected time (us) of a problem on a library kernel of one macro tile: rounds of tiles over the compute units times the
@@ -299,12 +300,16 @@ static double lin_tile_us(int M, int N, int K, int features, int rows, int cus) 
 }
 
 // Problems with many rows and a long reduction take the candidate with the shortest expected time instead of the first of
-// the library's ranking. Over 58 problems with K of 12288 and 13824 the first is 25 % slower than the best of 32 on average
-// and up to 2 x, the choice made here 4 %: M=9210 (a 16:9 image being edited beside its source, two prompts), N=3072,
-// K=12288 798 -> 493 us; M=6144 682 -> 340. At K = 5120 (116 problems) the first is 7 % off, the choice 3 %. With K of 3072
-// the first is 5 % off, and what the model chose instead ran 5 % slower inside a step of 4608 rows, so it stays; below 1024
-// rows a launch is less than one round of large tiles and the model says nothing.
+// the library's ranking, where it promises 8 % or more. Over 44 problems with K of 12288 and 13824 the first is 25 % slower
+// than the best of 32 on average and up to 2 x, the choice made here 5 %: M=9210 (a 16:9 image being edited beside its
+// source, two prompts), N=3072, K=12288 798 -> 493 us; M=6144 682 -> 340. At K = 5120 (66 problems) the first is 7 % off,
+// the choice 3 %. Below 8 % the model is as often wrong as right (M=1536, N=3072, K=12288: 4 % promised, 133 -> 141 us
+// inside a step); with the margin one of the 110 gets slower. Of two tiles with the same expected time the one that is
+// wider in features wins: 256 x 224 takes 244 us at M=4608, 224 x 256 251. With K of 3072 the first is 5 % off, and what
+// the model chose instead ran 5 % slower inside a step of 4608 rows, so it stays; below 1024 rows a launch is less than one
+// round of large tiles and the model says nothing.
 constexpr int kLinRankMinRows = 1024, kLinRankMinK = 4096;
+constexpr double kLinRankGain = 0.92, kLinTallTile = 1.01;
 constexpr int kLinCandidates = 32;
 
 static int lin_default_algo(hipblasLtHandle_t h, LinPlan& p, const LinCall& c, size_t lib_ws_bytes) {
@@ -322,15 +327,19 @@ static int lin_default_algo(hipblasLtHandle_t h, LinPlan& p, const LinCall& c, s
     return ODIT_ENOTSUP;
   }
   int best = 0;
-  double best_us = 0;
+  double best_us = 0;  // expected time of the choice, times kLinRankGain for the library's first
   const int cus = rank ? device_cus() : 0;
   for (int i = 0; i < n && cus > 0; ++i) {
     int features, rows;
+    bool usual;
     if (res[i].state != HIPBLAS_STATUS_SUCCESS || res[i].workspaceSize > lib_ws_bytes ||
-        !lin_macro_tile(hipblaslt_ext::getKernelNameFromAlgo(h, res[i].algo), &features, &rows))
+        !lin_macro_tile(hipblaslt_ext::getKernelNameFromAlgo(h, res[i].algo), &features, &rows, &usual)) {
+      if (i == 0) break;
       continue;
-    const double us = lin_tile_us(c.M, c.N, c.K, features, rows, cus);
-    if (best_us == 0 || us < best_us) { best = i; best_us = us; }
+    }
+    const double us = lin_tile_us(c.M, c.N, c.K, features, rows, cus) * (rows > features ? kLinTallTile : 1.);
+    if (i == 0) best_us = us * kLinRankGain;
+    else if (usual && us < best_us) { best = i; best_us = us; }
   }
   p.algo = res[best].algo;
   p.algo_ws = res[best].workspaceSize;
