@@ -317,12 +317,12 @@ int odit_silu(const void* x, void* out, int64_t n, int dtype, void* stream);
  *   RowParallelLinear followed by `h + gate * y`           qwen_image_transformer.py:794-795, 801, 806,
  *                                                          flux_transformer.py:288-309, wan2_2_transformer.py:661, 673
  * Engines. hipBLASLt's MFMA kernels (a plain dense GEMM), set up so that bias, activation, gate and
- * residual ride in that kernel's epilogue, and two hand-written bf16 MFMA kernels (K a multiple of 64, N a
- * multiple of 8, 16-byte aligned rows): a stream-K kernel for 64 <= M <= 1024 rows (csrc/gemm_bf16.hip) that
- * keeps all CUs busy on few output tiles, and a tile kernel for more rows (csrc/gemm_bf16_tile.hip: 256 x 256
+ * residual ride in that kernel's epilogue, and two hand-written MFMA kernels (K a multiple of 64, N a
+ * multiple of 8, 16-byte aligned rows): a stream-K kernel, bf16 or fp16, for M <= 1024 rows (csrc/gemm_bf16.hip) that
+ * keeps all CUs busy on few output tiles, and a bf16 tile kernel for more rows (csrc/gemm_bf16_tile.hip: 256 x 256
  * or 256 x 192 output tiles, one per workgroup). Both take one gate vector per group of rows in a single
  * launch (odit_linear_rows). A hand-written kernel runs where a tuning call found it faster or, untuned,
- * where its default rule says so (stream-K: K >= 2 N); the `flags` of odit_linear_rows can force either side.
+ * where its default rule says so (stream-K: K >= 2 N and M >= 48); the `flags` of odit_linear_rows can force either side.
  *
  * x [M,K] (row stride ldx), W [N,K] (row stride ldw: torch's nn.Linear weight, or a column range of
  * one), bias [N] or NULL, out [M,N] (row stride ldo). Gated form: residual [M,N] (row stride ldr; may be
@@ -381,6 +381,21 @@ int odit_linear_tune(const void* x, const void* w, const void* bias, void* out, 
 int odit_linear_rows(const void* x, const void* w, const void* bias, void* out, const void* residual,
                      const void* gate, int M, int N, int K, int64_t ldx, int64_t ldw, int64_t ldo, int64_t ldr,
                      int epilogue, int gate_dtype, int dtype, int rows_per_gate, int64_t gate_stride,
+                     unsigned flags, void* workspace, size_t workspace_bytes, void* stream);
+
+/* Two projections of the same N, K, epilogue and types in ONE launch of the stream-K kernel: the image and the text rows of a
+ * dual-stream block (to_qkv beside add_kv_proj, qwen_image_transformer.py:566-580, and the output, up and down projections).
+ * Fields as the arguments of odit_linear_rows. Returns ODIT_ENOTSUP, with nothing launched, where two odit_linear_rows calls
+ * are the better way (many rows) or the kernel does not take a problem; the caller then makes them. flags as for
+ * odit_linear_rows (ODIT_LINEAR_LIBRARY: always ODIT_ENOTSUP). */
+typedef struct odit_linear_problem {
+  const void *x, *w, *bias, *residual, *gate;
+  void* out;
+  int M, rows_per_gate;
+  int64_t ldx, ldw, ldo, ldr, gate_stride;
+} odit_linear_problem;
+
+int odit_linear_pair(const odit_linear_problem problems[2], int N, int K, int epilogue, int gate_dtype, int dtype,
                      unsigned flags, void* workspace, size_t workspace_bytes, void* stream);
 
 /* Names the library kernel for plain projections of one problem (ODIT_EPI_BIAS, dense rows) ahead of time by the

@@ -366,3 +366,60 @@ def test_linear_tune_compares_both_engines(gpu):
     assert 0 < us < 1e4
     got = kernels.linear(xg, wg, bg)
     torch.testing.assert_close(got.double().cpu(), _ref(x, w, b), atol=2e-2, rtol=2e-2)
+
+
+# ---------------------------------------------------------------------------- two problems in one stream-K launch
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M0,M1,N,K", [
+    (1, 1, 8, 64),          # 64-row tiles, one step
+    (64, 40, 200, 320),     # 64-row tiles, ragged feature tile, every tile shared
+    (65, 64, 392, 448),     # one row over: 128-row tiles
+    (300, 129, 768, 1024),  # ragged row tiles of both
+    (512, 80, 3072, 3072),  # 128-wide tiles, each reduced over several workgroups
+    (592, 1, 9216, 192),    # 192-wide tiles, whole ones
+    (768, 200, 9216, 3072), # 256-wide tiles or ranges across tiles
+])
+def test_linear_pair(gpu, dtype, M0, M1, N, K):
+    """Both problems against the fp64 product: bias, GELU, and gates per group of rows in both gate forms."""
+    from vllm_omni_amd import _lib, kernels
+
+    lib, code = _lib.load(), 0 if dtype == torch.bfloat16 else 1
+    ws = kernels._linear_scratch(gpu.index or 0, torch.cuda.current_stream().cuda_stream)
+    ops_ = [_mk(m, N, K, dtype, seed=m + N + i) for i, m in enumerate((M0, M1))]
+    dev = [[t.to(gpu) for t in o] for o in ops_]
+    g = torch.Generator().manual_seed(5)
+    res = [torch.randn(m, N, generator=g).to(dtype) for m in (M0, M1)]
+    rows = [max(1, m // 2) for m in (M0, M1)]                       # (a last group of one row where m is odd)
+    gates = [torch.randn(-(-m // r), N, generator=g) for m, r in zip((M0, M1), rows)]
+    dres, dgates = [t.to(gpu) for t in res], [t.to(gpu) for t in gates]
+    out = [torch.full((m, N), float("nan"), dtype=dtype, device=gpu) for m in (M0, M1)]
+
+    def run(epilogue, gate_dtype=code, bias=None, gate=None):
+        q = (_lib.LinearProblem * 2)()
+        for i, m in enumerate((M0, M1)):
+            q[i].x, q[i].w, q[i].out, q[i].M = dev[i][0].data_ptr(), dev[i][1].data_ptr(), out[i].data_ptr(), m
+            q[i].ldx, q[i].ldw, q[i].ldo, q[i].ldr = K, K, N, N
+            q[i].bias = (bias[i] if bias else dev[i][2]).data_ptr()
+            if gate:
+                q[i].residual, q[i].gate, q[i].rows_per_gate, q[i].gate_stride = dres[i].data_ptr(), gate[i].data_ptr(), rows[i], N
+        rc = lib.odit_linear_pair(_lib.C.addressof(q), N, K, epilogue, gate_dtype, code, 2, ws.data_ptr(), ws.numel(),
+                                  torch.cuda.current_stream().cuda_stream)
+        _lib.check(rc, "odit_linear_pair")
+        return [t.double().cpu() for t in out]
+
+    plain = [_ref(*o) for o in ops_]
+    tol = _tol(dtype)
+    got = run(1)
+    for a, b in zip(got, plain):
+        torch.testing.assert_close(a, b, atol=tol, rtol=tol)
+    assert all(torch.equal(a, b) for a, b in zip(got, run(1))), "the order of the partial sums must not depend on arrival order"
+    for a, b in zip(run(3), plain):
+        torch.testing.assert_close(a, ops.gelu_tanh(b), atol=tol, rtol=tol)
+    per_row = [t[torch.arange(m) // r].double() for t, m, r in zip(gates, (M0, M1), rows)]
+    want = [r.double() + p * y for r, p, y in zip(res, per_row, plain)]
+    for a, b in zip(run(4, gate_dtype=2, gate=dgates), want):
+        torch.testing.assert_close(a, b, atol=2 * tol, rtol=tol)
+    scaled = [t * o[2].float() for t, o in zip(dgates, dev)]
+    for a, b in zip(run(5, gate_dtype=2, bias=scaled, gate=dgates), want):
+        torch.testing.assert_close(a, b, atol=2 * tol, rtol=tol)
+    assert _counters_are_zero(kernels)

@@ -109,4 +109,6 @@ def test_native_block_leaves_changed_modules_to_python(gpu, monkeypatch):
     with torch.inference_mode():
         changed = call()
         monkeypatch.setattr(kernels, "NATIVE_BLOCKS", False)
-        assert torch.equal(changed, call()) and not torch.equal(changed, plain)
+        stepwise = call()
+    torch.testing.assert_close(changed.float(), stepwise.float(), atol=2e-2, rtol=2e-2)
+    assert (changed - plain).float().norm() > 2 * (changed - stepwise).float().norm()

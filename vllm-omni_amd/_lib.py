@@ -103,6 +103,8 @@ _SIGNATURES = {
          C.c_int64, C.c_int64, C.c_int64, C.c_int64, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int64, C.c_uint,
          C.c_void_p, C.c_size_t, C.c_void_p],
     ),
+    "odit_linear_pair": (
+        C.c_int, [C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_uint, C.c_void_p, C.c_size_t, C.c_void_p]),
     "odit_linear_rows_plan": (
         C.c_int,
         [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_int,
@@ -126,6 +128,14 @@ _SIGNATURES = {
 }
 
 EXPORTED_SYMBOLS = tuple(_SIGNATURES)
+
+
+class LinearProblem(C.Structure):
+    """``odit_linear_problem``."""
+
+    _fields_ = [(n, C.c_void_p) for n in ("x", "w", "bias", "residual", "gate", "out")] + [("M", C.c_int), ("rows_per_gate", C.c_int)] + [
+        (n, C.c_int64) for n in ("ldx", "ldw", "ldo", "ldr", "gate_stride")]
+
 
 
 class OmniDitLibraryError(RuntimeError):

@@ -1,4 +1,4 @@
-// Hand-written bf16 GEMM for projections with few rows (the text stream of a dual-stream block):
+// Hand-written 16-bit GEMM for projections with few rows (the text stream of a dual-stream block, small images):
 // interface between linear.hip (problem checks, dispatch) and gemm_bf16.hip (the kernel).
 #pragma once
 
@@ -19,7 +19,7 @@ struct GemmCall {
 };
 
 constexpr int kGemmBM = 128;  // rows of x per output tile
-constexpr int kGemmBN = 192;  // rows of W (output features) per output tile
+constexpr int kGemmBN = 256;  // rows of W (output features) per output tile, at most
 constexpr int kGemmBK = 64;   // reduction elements per pipeline step
 
 // scratch of the kernel: one 64-bit ticket word per output tile, then two partial-tile slots per workgroup
@@ -28,17 +28,18 @@ constexpr size_t kGemmSlotBytes = static_cast<size_t>(kGemmBM) * kGemmBN * sizeo
 constexpr int kGemmMaxWorkers = 256;
 constexpr size_t kGemmScratchBytes = kGemmCounterBytes + 2 * kGemmMaxWorkers * kGemmSlotBytes;
 
-// whether the kernel takes this problem (bf16, K a multiple of 64, N of 8, 64 <= M <= 1024, 16-byte
-// aligned rows, operands addressable with 32-bit byte offsets)
+// whether the kernel takes this problem (bf16 or fp16, K a multiple of 64, N of 8, 16-byte aligned rows, operands
+// addressable with 32-bit byte offsets, at most 256 row tiles and 4096 output tiles)
 bool gemm_streamk_takes(const GemmCall& c, int dtype);
 
+// One problem (count 1) or two of the same N, K and epilogue in one launch (count 2).
 // `scratch` (kGemmScratchBytes, 256-byte aligned): its first kGemmCounterBytes must have been zero-filled
 // once; they are zero again when the kernel has finished, and what an unfinished launch left there is
 // overridden by the next launch (its ticket words carry a larger epoch).
-int launch_gemm_streamk(const GemmCall& c, void* scratch, hipStream_t stream);
+int launch_gemm_streamk(const GemmCall* c, int count, int dtype, void* scratch, hipStream_t stream);
 
-// workgroups the launch would use and the reduction steps each of them runs
-void gemm_streamk_shape(int M, int N, int K, int device_cus, int* workers, int* steps_per_worker, int* tiles);
+// expected time (us) of a launch over problems of M0 and M1 rows (M1 = 0: one problem)
+float gemm_streamk_us(int M0, int M1, int N, int K, int device_cus);
 
 // compute units of the current device (0 when it cannot be read)
 int device_cus();

@@ -336,7 +336,7 @@ __global__ __launch_bounds__(WM * 2 * 64) __attribute__((amdgpu_waves_per_eu(WM 
       float y[8];
 #pragma unroll
       for (int u = 0; u < 4; ++u) { y[u] = lo[u]; y[4 + u] = hi[u]; }
-      gemm_epilogue_store8(p.ep, m, n, y);
+      gemm_epilogue_store8<bf16_t>(p.ep, m, n, y);
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   }

@@ -17,14 +17,19 @@ struct GemmEpilogue {
 };
 
 __device__ __forceinline__ float gemm_gelu_tanh(float x) {
-  const float u = 0.7978845608028654f * x * fmaf(0.044715f * x, x, 1.f);
-  return x / (1.f + __expf(-2.f * u));
+  // x sigmoid(2 u), u = sqrt(2/pi) (x + 0.044715 x^3), with e^(-2 u) as a power of two and the hardware reciprocal (1 ulp; a
+  // division costs ten instructions, and 48 elements per lane wait here with nothing to overlap: 4.5 us of a 47 us launch
+  // at M=512, N=12288, K=3072)
+  const float e = __builtin_amdgcn_exp2f(x * fmaf(x * x, -2.f * 0.7978845608028654f * 0.044715f * 1.4426950408889634f,
+                                                  -2.f * 0.7978845608028654f * 1.4426950408889634f));
+  return x * __builtin_amdgcn_rcpf(1.f + e);
 }
 
 // y[0..8) = accumulators of row m, features n .. n + 7 (n a multiple of 8, m < M, n < N): applies the
 // epilogue and stores 16 bytes
+template <typename T>
 __device__ __forceinline__ void gemm_epilogue_store8(const GemmEpilogue& p, int m, int n, float (&y)[8]) {
-  const bf16_t* bias_h = static_cast<const bf16_t*>(p.bias);
+  const T* bias_h = static_cast<const T*>(p.bias);
   const float* bias_f = static_cast<const float*>(p.bias);
   const bool gelu = p.epilogue == ODIT_EPI_GELU_TANH || p.epilogue == ODIT_EPI_BIAS_GELU_TANH;
   const bool gated = p.epilogue == ODIT_EPI_GATED_RESIDUAL || p.epilogue == ODIT_EPI_GATED_RESIDUAL_PRE;
@@ -41,9 +46,9 @@ __device__ __forceinline__ void gemm_epilogue_store8(const GemmEpilogue& p, int 
 #pragma unroll
         for (int u = 0; u < 4; ++u) { gt[u] = g0[u]; gt[4 + u] = g1[u]; }
       } else {
-        const u32x4 gv = load_raw(static_cast<const bf16_t*>(p.gate) + grow + n);
+        const u32x4 gv = load_raw(static_cast<const T*>(p.gate) + grow + n);
 #pragma unroll
-        for (int u = 0; u < 8; ++u) gt[u] = Raw<bf16_t>::get(gv, u);
+        for (int u = 0; u < 8; ++u) gt[u] = Raw<T>::get(gv, u);
       }
     }
     if (p.bias != nullptr) {
@@ -55,17 +60,17 @@ __device__ __forceinline__ void gemm_epilogue_store8(const GemmEpilogue& p, int 
       } else {
         const u32x4 bv = load_raw(bias_h + n);
 #pragma unroll
-        for (int u = 0; u < 8; ++u) bs[u] = gt[u] * Raw<bf16_t>::get(bv, u);
+        for (int u = 0; u < 8; ++u) bs[u] = gt[u] * Raw<T>::get(bv, u);
       }
     }
-    const u32x4 rv = load_raw(static_cast<const bf16_t*>(p.residual) + m * p.ldr + n);
+    const u32x4 rv = load_raw(static_cast<const T*>(p.residual) + m * p.ldr + n);
 #pragma unroll
-    for (int u = 0; u < 8; ++u) y[u] = fmaf(gt[u], y[u], bs[u]) + Raw<bf16_t>::get(rv, u);
+    for (int u = 0; u < 8; ++u) y[u] = fmaf(gt[u], y[u], bs[u]) + Raw<T>::get(rv, u);
   } else {
     if (p.bias != nullptr) {
       const u32x4 bv = load_raw(bias_h + n);
 #pragma unroll
-      for (int u = 0; u < 8; ++u) y[u] += Raw<bf16_t>::get(bv, u);
+      for (int u = 0; u < 8; ++u) y[u] += Raw<T>::get(bv, u);
     }
     if (gelu) {
 #pragma unroll
@@ -74,8 +79,8 @@ __device__ __forceinline__ void gemm_epilogue_store8(const GemmEpilogue& p, int 
   }
   u32x4 o;
 #pragma unroll
-  for (int u = 0; u < 4; ++u) Raw<bf16_t>::set2(o, u, y[2 * u], y[2 * u + 1]);
-  store_raw(static_cast<bf16_t*>(p.out) + m * p.ldo + n, o);
+  for (int u = 0; u < 4; ++u) Raw<T>::set2(o, u, y[2 * u], y[2 * u + 1]);
+  store_raw(static_cast<T*>(p.out) + m * p.ldo + n, o);
 }
 
 inline GemmEpilogue gemm_epilogue_of(const GemmCall& c) {

@@ -432,17 +432,17 @@ static int lin_handwritten_kind(const odit::GemmCall& g, int dtype, const void* 
   return sk != nullptr && odit::gemm_streamk_takes(g, dtype) ? 1 : 0;
 }
 
-static int lin_launch_handwritten(int kind, const odit::GemmCall& g, void* sk, hipStream_t stream) {
-  if (kind == 1) return odit::launch_gemm_streamk(g, sk, stream);
+static int lin_launch_handwritten(int kind, const odit::GemmCall& g, int dtype, void* sk, hipStream_t stream) {
+  if (kind == 1) return odit::launch_gemm_streamk(&g, 1, dtype, sk, stream);
   const int cus = odit::device_cus();
   if (cus <= 0) { odit::set_error("odit_linear: cannot read the device's compute-unit count"); return ODIT_ELAUNCH; }
   return odit::launch_gemm_tile(g, cus, stream);
 }
 
-// Without a tuning record: the stream-K kernel where the reduction is long against the number of output
-// tiles (K >= 2 N: the library's choices split K badly there, measured 58 vs 72 us at M=512, N=3072,
-// K=12288); the tile kernel for the gated form with one gate vector per group of rows, where the library
-// needs a launch per group, and for the other forms where measured faster (ODIT_TILE_DEFAULT_ALL).
+// Without a tuning record: the stream-K kernel where the reduction is long against the number of output features (K >= 2 N:
+// the library's choices split K badly there: M=80, N=3072, K=12288 57 us against 31, M=512 69 against 52, M=1024 110
+// against 85) and there is work for all CUs; with a small product (N K < 2^22, a few MB of weights) its ranges would be
+// shorter than what handing partial tiles over costs (M=256, N=256, K=1024: 19 us against 10).
 static bool lin_prefers_handwritten(int dev, int kind, const odit::LinCall& c, int rows_per_gate) {
   {
     std::lock_guard<std::mutex> lock(odit::g_engine_mu);
@@ -450,7 +450,7 @@ static bool lin_prefers_handwritten(int dev, int kind, const odit::LinCall& c, i
     if (it != odit::g_handwritten_wins.end()) return it->second;
   }
   if (kind == 2) return false;
-  return c.K >= 2 * c.N;
+  return c.K >= 2 * c.N && c.M >= 48 && static_cast<int64_t>(c.N) * c.K >= (1ll << 22);
 }
 
 extern "C" int odit_linear_prefer(int M, int N, int K, int dtype, int solution) {
@@ -498,7 +498,7 @@ extern "C" int odit_linear_rows(const void* x, const void* w, const void* bias, 
   if (kind != 0 && engine != 1) {
     int dev = 0;
     if (engine == 2 || (hipGetDevice(&dev) == hipSuccess && lin_prefers_handwritten(dev, kind, c, g.rows_per_gate)))
-      return lin_launch_handwritten(kind, g, sk, c.stream);
+      return lin_launch_handwritten(kind, g, dtype, sk, c.stream);
   }
   if (!per_rows) return lin_run_library(c);
   // the library's epilogue takes one gate vector per launch: one launch per group of rows
@@ -517,6 +517,41 @@ extern "C" int odit_linear_rows(const void* x, const void* w, const void* bias, 
     if (rc != ODIT_OK) return rc;
   }
   return ODIT_OK;
+}
+
+// Two problems in one launch, or two calls? The launch has one set of overheads for both, the weights of the second stream
+// behind those of the first and no gate per launch; the library has the faster main loop for many rows. Up to kPairTiles
+// tiles of 128 rows together the launch wins (us, launch / two library calls): 4 + 1 tiles QKV 42 / 70, out 24 / 36; 6 + 2
+// tiles QKV 69 / 86, MLP up 88 / 102, out 32 / 44. With gates that differ per batch entry the library needs a call per
+// entry, and for few rows a residual pass: kPairTilesGated.
+constexpr int kPairTiles = 8, kPairTilesGated = 20;
+
+extern "C" int odit_linear_pair(const odit_linear_problem* q, int N, int K, int epilogue, int gate_dtype, int dtype, unsigned flags,
+                                void* workspace, size_t workspace_bytes, void* stream) {
+  using namespace odit;
+  ODIT_CHECK_ARG(q != nullptr, "odit_linear_pair: null problems");
+  const int engine = lin_engine_of(flags);
+  void *sk, *lib;
+  size_t lib_bytes;
+  lin_split_ws(workspace, workspace_bytes, &sk, &lib, &lib_bytes);
+  GemmCall g[2];
+  bool per_rows = false, takes = sk != nullptr && engine != 1;
+  int tiles = 0;
+  for (int i = 0; i < 2; ++i) {
+    const LinCall c{q[i].x, q[i].w, q[i].bias, q[i].residual, q[i].gate, q[i].out, q[i].M, N, K, q[i].ldx, q[i].ldw, q[i].ldo, q[i].ldr,
+                    epilogue, gate_dtype, dtype, workspace, workspace_bytes, static_cast<hipStream_t>(stream)};
+    const int rc = lin_check(c);
+    if (rc != ODIT_OK) return rc;
+    ODIT_CHECK_ARG(q[i].rows_per_gate >= 0 && q[i].gate_stride >= 0, "odit_linear_pair: rows_per_gate and gate_stride must not be negative");
+    const bool rows = lin_is_residual(c) && q[i].gate != nullptr && q[i].rows_per_gate > 0 && q[i].rows_per_gate < q[i].M;
+    g[i] = lin_gemm_call(c, rows ? q[i].rows_per_gate : 0, rows ? q[i].gate_stride : 0);
+    per_rows = per_rows || rows;
+    takes = takes && q[i].M > 0 && gemm_streamk_takes(g[i], dtype);
+    tiles += (q[i].M + kGemmBM - 1) / kGemmBM;
+  }
+  if (!takes || (engine != 2 && (tiles > (per_rows ? kPairTilesGated : kPairTiles) || static_cast<int64_t>(N) * K < (1 << 14))))
+    return ODIT_ENOTSUP;  // (no message: the ordinary answer for large problems)
+  return launch_gemm_streamk(g, 2, dtype, sk, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int odit_linear_rows_plan(const void* x, const void* w, const void* bias, void* out, const void* residual,
@@ -631,7 +666,7 @@ static int lin_tune_library(const odit::LinCall& c, int iters, void* flush, size
   return ODIT_OK;
 }
 
-static int lin_time_handwritten(int kind, const odit::GemmCall& g, void* sk, hipStream_t stream, int iters, void* flush,
+static int lin_time_handwritten(int kind, const odit::GemmCall& g, int dtype, void* sk, hipStream_t stream, int iters, void* flush,
                                 size_t flush_bytes, float* us) {
   using namespace odit;
   hipEvent_t e0, e1;
@@ -639,12 +674,12 @@ static int lin_time_handwritten(int kind, const odit::GemmCall& g, void* sk, hip
     set_error("odit_linear_tune: hipEventCreate failed");
     return ODIT_ELAUNCH;
   }
-  int rc = lin_launch_handwritten(kind, g, sk, stream);
+  int rc = lin_launch_handwritten(kind, g, dtype, sk, stream);
   float total = 0.f;
   for (int i = 0; i < iters && rc == ODIT_OK; ++i) {
     if (flush != nullptr && flush_bytes > 0) (void)hipMemsetAsync(flush, i & 0xff, flush_bytes, stream);
     (void)hipEventRecord(e0, stream);
-    rc = lin_launch_handwritten(kind, g, sk, stream);
+    rc = lin_launch_handwritten(kind, g, dtype, sk, stream);
     (void)hipEventRecord(e1, stream);
     if (hipEventSynchronize(e1) != hipSuccess) { set_error("odit_linear_tune: hipEventSynchronize failed"); rc = ODIT_ELAUNCH; }
     float ms = 0.f;
@@ -699,7 +734,7 @@ extern "C" int odit_linear_rows_tune(const void* x, const void* w, const void* b
   const GemmCall g = lin_gemm_call(c, per_rows ? rows_per_gate : 0, per_rows ? gate_stride : 0);
   if (const int kind = lin_handwritten_kind(g, dtype, sk)) {
     float own_us = 0.f;
-    rc = lin_time_handwritten(kind, g, sk, c.stream, iters, flush, flush_bytes, &own_us);
+    rc = lin_time_handwritten(kind, g, dtype, sk, c.stream, iters, flush, flush_bytes, &own_us);
     if (rc != ODIT_OK) return rc;
     int dev = 0;
     (void)hipGetDevice(&dev);

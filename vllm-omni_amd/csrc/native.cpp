@@ -761,6 +761,36 @@ void project_gated(BlockCall& c, const void* x, const Lin& l, const void* residu
                            c.engine, c.lin_ws.p, c.lin_ws.bytes, c.where.stream));
 }
 
+// y[i] = x[i] W[i]^T + b[i] (GELU) for the two streams: one launch where that is the better way
+void project_pair(BlockCall& c, const void* const x[2], const Lin l[2], void* const y[2], const int64_t M[2], bool gelu) {
+  if (c.rc != 0) return;
+  if (l[0].n == l[1].n && l[0].k == l[1].k && (l[0].b == nullptr) == (l[1].b == nullptr)) {
+    odit_linear_problem q[2];
+    for (int i = 0; i < 2; ++i)
+      q[i] = {x[i], l[i].w, l[i].b, nullptr, nullptr, y[i], static_cast<int>(M[i]), 0, l[i].k, l[i].ldw, l[i].n, 0, 0};
+    const int epi = gelu ? (l[0].b ? ODIT_EPI_BIAS_GELU_TANH : ODIT_EPI_GELU_TANH) : (l[0].b ? ODIT_EPI_BIAS : ODIT_EPI_NONE);
+    const int rc = odit_linear_pair(q, l[0].n, l[0].k, epi, c.dtype, c.dtype, c.engine & ODIT_LINEAR_LIBRARY, c.lin_ws.p, c.lin_ws.bytes, c.where.stream);
+    if (rc != ODIT_ENOTSUP) { c.check(rc); return; }
+  }
+  for (int i = 0; i < 2; ++i) c.project(x[i], l[i], y[i], M[i], gelu);
+}
+
+// out[i] = residual[i] + gate[i] * (x[i] W[i]^T + b[i]) for the two streams in one launch; false when two calls are the better way
+bool project_gated_pair(BlockCall& c, const void* const x[2], const Lin l[2], const void* const residual[2], void* const out[2], int64_t B,
+                        const int64_t S[2], const Gate g[2]) {
+  if (c.rc != 0) return true;
+  if (l[0].n != l[1].n || l[0].k != l[1].k || g[0].pre != g[1].pre || g[0].code != g[1].code) return false;
+  odit_linear_problem q[2];
+  for (int i = 0; i < 2; ++i)
+    q[i] = {x[i], l[i].w, g[i].pre ? g[i].gbias : l[i].b, residual[i], g[i].gate, out[i], static_cast<int>(B * S[i]), B > 1 ? static_cast<int>(S[i]) : 0,
+            l[i].k, l[i].ldw, l[i].n, l[i].n, g[i].stride};
+  const int rc = odit_linear_pair(q, l[0].n, l[0].k, g[0].pre ? ODIT_EPI_GATED_RESIDUAL_PRE : ODIT_EPI_GATED_RESIDUAL, g[0].pre ? ODIT_F32 : g[0].code,
+                                  c.dtype, c.engine & ODIT_LINEAR_LIBRARY, c.lin_ws.p, c.lin_ws.bytes, c.where.stream);
+  if (rc == ODIT_ENOTSUP) return false;
+  c.check(rc);
+  return true;
+}
+
 // one allocation for a block's intermediate tensors
 struct Slab {
   Tensor t;
@@ -907,7 +937,8 @@ bool run_dual(BlockCall& c, const DualBlock& k, const Tensor& img, const Tensor&
   } else {
     norms(src, 0);
   }
-  for (int i = 0; i < 2; ++i) c.project(n[i], k.qkv[i], qkv[i], B * S[i], false);
+  const int64_t M[2] = {B * S[0], B * S[1]};
+  project_pair(c, n, k.qkv, qkv, M, false);
   if (c.rc == 0) {  // problem 0 = text rows [0, S_txt), problem 1 = image rows
     auto part = [&](int stream, int which) { return static_cast<char*>(qkv[stream]) + which * HD * esz; };
     const void *qi[2] = {part(1, 0), part(0, 0)}, *ki[2] = {part(1, 1), part(0, 1)},
@@ -932,20 +963,21 @@ bool run_dual(BlockCall& c, const DualBlock& k, const Tensor& img, const Tensor&
   }
   void* res[2] = {result[0].data_ptr(), result[1].data_ptr()};
   Gate plain;
-  for (int i = 0; i < 2; ++i) {
-    if (i == 0 && idx) { indexed(o[0], k.out[0], src[0], res[0], 0); continue; }
-    const Gate g = gate_of(i, 0, &plain);
-    project_gated(c, o[i], k.out[i], src[i], res[i], B, S[i], g, min_rows, tmp, plain);
-  }
+  auto gated = [&](const void* const a[2], const Lin l[2], const void* const residual[2], int which) {
+    const Gate g[2] = {gate_of(0, which, &plain), gate_of(1, which, &plain)};
+    if (!idx && project_gated_pair(c, a, l, residual, res, B, S, g)) return;
+    for (int i = 0; i < 2; ++i) {
+      if (i == 0 && idx) { indexed(a[0], l[0], residual[0], res[0], which); continue; }
+      gate_of(i, which, &plain);
+      project_gated(c, a[i], l[i], residual[i], res[i], B, S[i], g[i], min_rows, tmp, plain);
+    }
+  };
+  gated(o, k.out, src, 0);
   const void* mid[2] = {res[0], res[1]};
   if (idx) norm(1, mid[1], 1);
   else if (c.rc == 0) norms(mid, 1);
-  for (int i = 0; i < 2; ++i) {
-    c.project(n[i], k.up[i], u[i], B * S[i], true);
-    if (i == 0 && idx) { indexed(u[0], k.down[0], res[0], res[0], 1); continue; }
-    const Gate g = gate_of(i, 1, &plain);
-    project_gated(c, u[i], k.down[i], res[i], res[i], B, S[i], g, min_rows, tmp, plain);
-  }
+  project_pair(c, n, k.up, u, M, true);
+  gated(u, k.down, mid, 1);
   return true;
 }
 
