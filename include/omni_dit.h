@@ -373,10 +373,12 @@ int odit_linear_tune(const void* x, const void* w, const void* bias, void* out, 
  * library launch per group of rows otherwise.
  * flags: 0 = choose as described above; ODIT_LINEAR_LIBRARY = hipBLASLt whatever the record says;
  * ODIT_LINEAR_HANDWRITTEN = the hand-written kernel for this row count (ODIT_ENOTSUP when it does not take
- * the problem). Per call: no process-wide switch exists.
+ * the problem); ODIT_LINEAR_FIRST = where hipBLASLt runs the problem, its own first choice (or the one odit_linear_prefer
+ * named), not the one expected or tuned to be faster. Per call: no process-wide switch exists.
  */
 #define ODIT_LINEAR_LIBRARY 1u
 #define ODIT_LINEAR_HANDWRITTEN 2u
+#define ODIT_LINEAR_FIRST 4u
 
 int odit_linear_rows(const void* x, const void* w, const void* bias, void* out, const void* residual,
                      const void* gate, int M, int N, int K, int64_t ldx, int64_t ldw, int64_t ldo, int64_t ldr,
@@ -397,6 +399,25 @@ typedef struct odit_linear_problem {
 
 int odit_linear_pair(const odit_linear_problem problems[2], int N, int K, int epilogue, int gate_dtype, int dtype,
                      unsigned flags, void* workspace, size_t workspace_bytes, void* stream);
+
+/* out = act(x) W^T + bias for up to 16 rows of x (bias may be NULL; silu_input: act = SiLU rounded to the tensor type, else
+ * none): the timestep embedding, modulation and head-norm projections (qwen_image_transformer.py:159-181, 760-767, 1065), one
+ * pass over the weights. ODIT_BF16 or ODIT_F16, K a multiple of 32, 16-byte aligned rows; ODIT_ENOTSUP for anything else, with
+ * nothing launched. Needs no workspace. */
+int odit_linear_few(const void* x, const void* w, const void* bias, void* out, int M, int N, int K, int64_t ldx, int64_t ldw,
+                    int64_t ldo, int dtype, int silu_input, void* stream);
+
+/* The small work of a denoise step, one launch each, rounded where the torch expressions of the reference round:
+ * odit_time_sinusoid: t [n] (t_dtype) -> out [n, dim] (out_dtype) = cos | sin of scale * (t * exp(neg_log_period j / (dim / 2)))
+ *   (diffusers Timesteps with flip_sin_to_cos, qwen_image_transformer.py:165);
+ * odit_cfg_combine: neg + scale * (pos - neg) over dense [rows, C], 16-bit types; `normalize`: every row brought back to the
+ *   norm of pos (cfg_parallel.py:142-176); then C a multiple of 8 and 16-byte aligned tensors, else ODIT_ENOTSUP;
+ * odit_euler_step: out = x + dt * v in float32 (pipeline schedulers' step). */
+int odit_time_sinusoid(const void* t, void* out, int64_t n, int dim, float neg_log_period, float scale, int t_dtype, int out_dtype,
+                       void* stream);
+int odit_cfg_combine(const void* pos, const void* neg, void* out, int64_t rows, int C, float scale, int normalize, int dtype,
+                     void* stream);
+int odit_euler_step(const void* x, const void* v, void* out, int64_t n, float dt, int dtype, void* stream);
 
 /* Names the library kernel for plain projections of one problem (ODIT_EPI_BIAS, dense rows) ahead of time by the
  * library's own solution index, as an offline tuning run found it; process-wide, applies to problems first seen

@@ -332,7 +332,7 @@ class PixArtAlphaTextProjection(nn.Module):
         self.linear_2 = nn.Linear(hidden_size, hidden_size)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return self.linear_2(kernels.silu(self.linear_1(x)))
+        return kernels.project(self.linear_2, kernels.project(self.linear_1, x), silu_input=True)
 
 
 class CombinedTimestepGuidanceTextProjEmbeddings(nn.Module):
@@ -347,9 +347,9 @@ class CombinedTimestepGuidanceTextProjEmbeddings(nn.Module):
 
     def forward(self, timestep: torch.Tensor, guidance: torch.Tensor | None, pooled_projection: torch.Tensor):
         proj = QwenTimestepProjEmbeddings.time_proj
-        emb = self.timestep_embedder(proj(timestep, scale=1.0).to(pooled_projection.dtype))
+        emb = self.timestep_embedder(proj(timestep, scale=1.0, dtype=pooled_projection.dtype))
         if guidance is not None:
-            emb = emb + self.guidance_embedder(proj(guidance, scale=1.0).to(pooled_projection.dtype))
+            emb = emb + self.guidance_embedder(proj(guidance, scale=1.0, dtype=pooled_projection.dtype))
         return emb + self.text_embedder(pooled_projection)
 
 
@@ -401,12 +401,12 @@ class FluxTransformer2DModel(nn.Module):
 
     def prepare(self, hidden_states, encoder_hidden_states, pooled_projections, timestep, img_ids, txt_ids,
                 guidance=None):
-        img = self.x_embedder(hidden_states)
+        img = kernels.project(self.x_embedder, hidden_states)
         timestep = timestep.to(device=img.device, dtype=img.dtype) * 1000
         if guidance is not None:
             guidance = guidance.to(device=img.device, dtype=img.dtype) * 1000
         temb = self.time_text_embed(timestep, guidance, pooled_projections)
-        txt = self.context_embedder(encoder_hidden_states)
+        txt = kernels.project(self.context_embedder, encoder_hidden_states)
         if txt_ids.ndim == 3:
             txt_ids = txt_ids[0]
         if img_ids.ndim == 3:
@@ -475,7 +475,7 @@ class FluxTransformer2DModel(nn.Module):
         if w is None:
             return None
         C, L, Ls = self.inner_dim, len(self.transformer_blocks), len(self.single_transformer_blocks)
-        out = F.linear(kernels.silu(temb), w, self._mod_bias)
+        out = kernels.linear_few(temb, w, self._mod_bias, silu_input=True)
         B = temb.shape[0]
         return out[:, :L * 12 * C].view(B, L, 2, 6 * C), out[:, L * 12 * C:].view(B, Ls, 3 * C)
 
@@ -498,7 +498,7 @@ class FluxTransformer2DModel(nn.Module):
         return x[:, n_txt:], x[:, :n_txt]
 
     def finish(self, img, temb, return_dict: bool = True):
-        out = self.proj_out(self.norm_out(img, temb))
+        out = kernels.project(self.proj_out, self.norm_out(img, temb))
         return Transformer2DModelOutput(sample=out) if return_dict else (out,)
 
     def forward(self, hidden_states: torch.Tensor, encoder_hidden_states: torch.Tensor = None,

@@ -21,7 +21,6 @@ from typing import Any
 
 import torch
 import torch.nn as nn
-import torch.nn.functional as F
 
 from .. import kernels
 from .._lib import ODIT_NORM_HEAD
@@ -428,7 +427,7 @@ class TimestepEmbedding(nn.Module):
         self.linear_2 = nn.Linear(time_embed_dim, time_embed_dim)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return self.linear_2(kernels.silu(self.linear_1(x)))
+        return kernels.project(self.linear_2, kernels.project(self.linear_1, x), silu_input=True)
 
 
 class QwenTimestepProjEmbeddings(nn.Module):
@@ -443,16 +442,20 @@ class QwenTimestepProjEmbeddings(nn.Module):
             self.addition_t_embedding = nn.Embedding(2, embedding_dim)
 
     @staticmethod
-    def time_proj(t: torch.Tensor, dim: int = 256, max_period: int = 10000, scale: float = 1000.0):
+    def time_proj(t: torch.Tensor, dim: int = 256, max_period: int = 10000, scale: float = 1000.0,
+                  dtype: torch.dtype = torch.float32):
         """diffusers ``Timesteps(dim, flip_sin_to_cos=True, downscale_freq_shift=0, scale)``: fp32
         frequencies times ``t.float()``, cosines first."""
+        done = kernels.time_sinusoid(t, dim, max_period, scale, dtype)
+        if done is not None:
+            return done
         half = dim // 2
         freqs = torch.exp(-math.log(max_period) * torch.arange(half, dtype=torch.float32, device=t.device) / half)
         arg = scale * (t[:, None].float() * freqs[None, :])
-        return torch.cat((torch.cos(arg), torch.sin(arg)), dim=-1)
+        return torch.cat((torch.cos(arg), torch.sin(arg)), dim=-1).to(dtype)
 
     def forward(self, timestep: torch.Tensor, hidden_states: torch.Tensor, addition_t_cond=None):
-        emb = self.timestep_embedder(self.time_proj(timestep).to(hidden_states.dtype))
+        emb = self.timestep_embedder(self.time_proj(timestep, dtype=hidden_states.dtype))
         if self.use_additional_t_cond:
             if addition_t_cond is None:
                 raise ValueError("When additional_t_cond is True, addition_t_cond must be provided.")
@@ -469,7 +472,10 @@ class AdaLayerNormContinuous(nn.Module):
         self.linear = nn.Linear(conditioning_embedding_dim, 2 * embedding_dim, bias=True)
 
     def forward(self, x: torch.Tensor, cond: torch.Tensor) -> torch.Tensor:
-        emb = self.linear(kernels.silu(cond).to(x.dtype))
+        if cond.dtype == x.dtype:
+            emb = kernels.project(self.linear, cond, silu_input=True)
+        else:
+            emb = self.linear(kernels.silu(cond).to(x.dtype))
         scale, shift = emb.chunk(2, dim=1)
         return kernels.adaln_modulate(x, shift, scale, eps=self.eps)
 
@@ -533,11 +539,11 @@ class QwenImageTransformer2DModel(nn.Module):
                 additional_t_cond=None):
         """Stem. With ``zero_cond_t`` (editing checkpoints) the timestep is doubled to [t, 0 * t], so temb
         has 2B rows: real-timestep conditioning, then timestep-zero conditioning (qit.py:141-145)."""
-        img = self.img_in(hidden_states)
+        img = kernels.project(self.img_in, hidden_states)
         timestep = timestep.to(device=img.device, dtype=img.dtype)
         if self.zero_cond_t:
             timestep = torch.cat([timestep, timestep * 0], dim=0)
-        txt = self.txt_in(self.txt_norm(encoder_hidden_states))
+        txt = kernels.project(self.txt_in, self.txt_norm(encoder_hidden_states))
         if additional_t_cond is not None and self.zero_cond_t:
             additional_t_cond = torch.cat([additional_t_cond, additional_t_cond], dim=0)
         temb = self.time_text_embed(timestep, img, additional_t_cond)
@@ -602,7 +608,7 @@ class QwenImageTransformer2DModel(nn.Module):
         if w is None:
             return None
         L, C = w.shape[0], self.inner_dim
-        out = F.linear(kernels.silu(temb), w.view(L * 2 * 6 * C, C), self._mod_bias.view(-1))
+        out = kernels.linear_few(temb, w.view(L * 2 * 6 * C, C), self._mod_bias.view(-1), silu_input=True)
         return out.view(temb.shape[0], L, 2, 6 * C)
 
     def run_blocks(self, img, txt, temb, rotary, encoder_hidden_states_mask=None, attention_kwargs=None,
@@ -624,7 +630,7 @@ class QwenImageTransformer2DModel(nn.Module):
     def finish(self, img, temb, return_dict: bool = True):
         if self.zero_cond_t:
             temb = temb.chunk(2, dim=0)[0]  # the head is conditioned on the real timestep (qit.py:1062-1063)
-        out = self.proj_out(self.norm_out(img, temb))
+        out = kernels.project(self.proj_out, self.norm_out(img, temb))
         return Transformer2DModelOutput(sample=out) if return_dict else (out,)
 
     def forward(self, hidden_states: torch.Tensor, encoder_hidden_states: torch.Tensor = None,

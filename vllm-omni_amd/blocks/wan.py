@@ -416,12 +416,17 @@ class WanTimeTextImageEmbedding(nn.Module):
                 encoder_hidden_states_image: torch.Tensor | None = None, timestep_seq_len: int | None = None):
         """timestep [B] -> temb [B,C], timestep_proj [B,6C]; flattened per-token timesteps [B*S] with
         ``timestep_seq_len`` = S -> temb [B,S,C], timestep_proj [B,S,6C] (wan.py:282-296)."""
-        t = QwenTimestepProjEmbeddings.time_proj(timestep, dim=self.time_freq_dim, scale=1.0)
+        t = QwenTimestepProjEmbeddings.time_proj(timestep, dim=self.time_freq_dim, scale=1.0,
+                                                 dtype=self.time_embedder.linear_1.weight.dtype)
         if timestep_seq_len is not None:
             t = t.unflatten(0, (-1, timestep_seq_len))
-        t = t.to(self.time_embedder.linear_1.weight.dtype)
-        temb = self.time_embedder(t).type_as(encoder_hidden_states)
-        timestep_proj = self.time_proj(kernels.silu(temb))
+        mlp = self.time_embedder
+        if encoder_hidden_states.shape[0] == 1:
+            temb = mlp(t).type_as(encoder_hidden_states)
+            timestep_proj = kernels.project(self.time_proj, temb, silu_input=True)
+        else:  # a CFG pair keeps the library's order of summation: guidance multiplies what another one rounds differently
+            temb = mlp.linear_2(kernels.silu(mlp.linear_1(t))).type_as(encoder_hidden_states)
+            timestep_proj = self.time_proj(kernels.silu(temb))
         image = None
         if encoder_hidden_states_image is not None:
             if self.image_embedder is None:

@@ -42,6 +42,8 @@ UNITS: list[tuple[str, list[str], str]] = [
     ("attn_fwd.hip", [], "attn_fwd"),
     ("attn_fwd_dma.hip", [], "attn_fwd_dma"),
     ("linear.hip", [], "linear"),
+    ("linear_few.hip", [], "linear_few"),
+    ("step.hip", [], "step"),
     ("gemm_bf16.hip", [], "gemm_bf16"),
     ("gemm_bf16_tile.hip", [], "gemm_bf16_tile"),
 ]

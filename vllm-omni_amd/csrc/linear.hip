@@ -120,8 +120,8 @@ static int lin_plan_build(const LinKey& key, LinPlan& p) {
   const int32_t ta = HIPBLAS_OP_T, tb = HIPBLAS_OP_N;
   ODIT_LT(hipblasLtMatmulDescSetAttribute(p.desc, HIPBLASLT_MATMUL_DESC_TRANSA, &ta, sizeof(ta)));
   ODIT_LT(hipblasLtMatmulDescSetAttribute(p.desc, HIPBLASLT_MATMUL_DESC_TRANSB, &tb, sizeof(tb)));
-  // key.epi = epilogue * 4 + (bias vector in the epilogue ? 1 : 0) + (alpha vector ? 2 : 0)
-  const int kind = key.epi >> 2;
+  // key.epi = epilogue * 4 + (bias vector in the epilogue ? 1 : 0) + (alpha vector ? 2 : 0); a first-ranked kernel has a plan of its own (+ 0x100)
+  const int kind = (key.epi & 0xff) >> 2;
   const bool has_bias = key.epi & 1, alpha_vec = key.epi & 2;
   const bool gelu = kind == ODIT_EPI_GELU_TANH || kind == ODIT_EPI_BIAS_GELU_TANH;
   const uint32_t epi = gelu ? (has_bias ? HIPBLASLT_EPILOGUE_GELU_BIAS : HIPBLASLT_EPILOGUE_GELU)
@@ -179,6 +179,7 @@ struct LinCall {
   void* ws;
   size_t ws_bytes;
   hipStream_t stream;
+  bool first = false;  // the library's first-ranked kernel (ODIT_LINEAR_FIRST)
 };
 
 static bool lin_is_residual(const LinCall& c) {
@@ -203,7 +204,7 @@ static int lin_prepare(const LinCall& c, hipblasLtHandle_t* h, LinPlan** plan, c
   const bool prep = lin_needs_prep(c);
   const bool alpha_vec = gated && c.gate != nullptr;
   const bool has_bias = c.bias != nullptr;
-  LinKey key{dev, c.M, c.N, c.K, c.epilogue * 4 + (has_bias ? 1 : 0) + (alpha_vec ? 2 : 0), c.dtype,
+  LinKey key{dev, c.M, c.N, c.K, c.epilogue * 4 + (has_bias ? 1 : 0) + (alpha_vec ? 2 : 0) + (c.first ? 0x100 : 0), c.dtype,
              c.ldw, c.ldx, gated ? c.ldr : c.ldo, c.ldo};
   rc = lin_plan(key, plan);
   if (rc != ODIT_OK) return rc;
@@ -317,7 +318,7 @@ static int lin_default_algo(hipblasLtHandle_t h, LinPlan& p, const LinCall& c, s
   ODIT_LT(hipblasLtMatmulPreferenceCreate(&pref));
   const uint64_t maxws = lib_ws_bytes;
   hipblasLtMatmulPreferenceSetAttribute(pref, HIPBLASLT_MATMUL_PREF_MAX_WORKSPACE_BYTES, &maxws, sizeof(maxws));
-  const bool rank = c.M >= kLinRankMinRows && c.K >= kLinRankMinK && c.dtype != ODIT_F32;
+  const bool rank = c.M >= kLinRankMinRows && c.K >= kLinRankMinK && c.dtype != ODIT_F32 && !c.first;
   hipblasLtMatmulHeuristicResult_t res[kLinCandidates];
   int n = 0;
   const hipblasStatus_t st = hipblasLtMatmulAlgoGetHeuristic(h, p.desc, p.a, p.b, p.c, p.d, pref, rank ? kLinCandidates : 1, res, &n);
@@ -474,14 +475,15 @@ extern "C" int odit_linear_rows(const void* x, const void* w, const void* bias, 
                                 int64_t gate_stride, unsigned flags, void* workspace, size_t workspace_bytes,
                                 void* stream) {
   using namespace odit;
-  ODIT_CHECK_ARG((flags & ~(ODIT_LINEAR_LIBRARY | ODIT_LINEAR_HANDWRITTEN)) == 0 &&
+  ODIT_CHECK_ARG((flags & ~(ODIT_LINEAR_LIBRARY | ODIT_LINEAR_HANDWRITTEN | ODIT_LINEAR_FIRST)) == 0 &&
                      (flags & (ODIT_LINEAR_LIBRARY | ODIT_LINEAR_HANDWRITTEN)) != (ODIT_LINEAR_LIBRARY | ODIT_LINEAR_HANDWRITTEN),
-                 "odit_linear_rows: flags may name one engine (ODIT_LINEAR_LIBRARY or ODIT_LINEAR_HANDWRITTEN), got %#x", flags);
+                 "odit_linear_rows: flags may name one engine (ODIT_LINEAR_LIBRARY or ODIT_LINEAR_HANDWRITTEN) and ODIT_LINEAR_FIRST, got %#x", flags);
   void *sk, *lib;
   size_t lib_bytes;
   lin_split_ws(workspace, workspace_bytes, &sk, &lib, &lib_bytes);
   LinCall c{x, w, bias, residual, gate, out, M, N, K, ldx, ldw, ldo, ldr, epilogue, gate_dtype, dtype,
             lib, lib_bytes, static_cast<hipStream_t>(stream)};
+  c.first = (flags & ODIT_LINEAR_FIRST) != 0;
   int rc = lin_check(c);
   if (rc != ODIT_OK || M == 0) return rc;
   ODIT_CHECK_ARG(rows_per_gate >= 0 && (rows_per_gate == 0 || gate_stride >= 0),

@@ -540,6 +540,89 @@ bool rows_of(const Tensor& t, int64_t* rows, int64_t* ld) {
   return true;
 }
 
+// (t [n], dim, -log(max_period), scale, dtype code of the result) -> [n, dim]
+PyObject* py_time_sinusoid(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  NATIVE_BEGIN
+  const Tensor* t;
+  if (n != 5 || !(t = tensor_of(a[0]))) return none();
+  const long dim = PyLong_AsLong(a[1]), code = PyLong_AsLong(a[4]);
+  const double period = PyFloat_AsDouble(a[2]), scale = PyFloat_AsDouble(a[3]);
+  if (PyErr_Occurred()) return nullptr;
+  const Where w;
+  const int dt = code_of(*t);
+  if (dt < 0 || !w.holds(t) || t->dim() != 1 || !t->is_contiguous() || dim <= 0 || dim % 2 || code < 0 || code > 2) return none();
+  Tensor out = at::empty({t->size(0), dim}, t->options().dtype(code == ODIT_BF16 ? at::kBFloat16 : code == ODIT_F16 ? at::kHalf : at::kFloat));
+  if (odit_time_sinusoid(t->data_ptr(), out.data_ptr(), t->size(0), static_cast<int>(dim), static_cast<float>(period),
+                         static_cast<float>(scale), dt, static_cast<int>(code), w.stream) != 0)
+    return none();
+  return wrap(std::move(out));
+  NATIVE_END
+}
+
+// (positive, negative, scale, normalize)
+PyObject* py_cfg_combine(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  NATIVE_BEGIN
+  const Tensor *p, *q;
+  if (n != 4 || !(p = tensor_of(a[0])) || !(q = tensor_of(a[1]))) return none();
+  const double scale = PyFloat_AsDouble(a[2]);
+  const int norm = PyObject_IsTrue(a[3]);
+  if (PyErr_Occurred()) return nullptr;
+  const Where w;
+  const int dt = code_of(*p);
+  if ((dt != ODIT_BF16 && dt != ODIT_F16) || !w.holds(p) || !w.holds(q) || p->dim() < 1 || p->numel() == 0 || p->sizes() != q->sizes() ||
+      p->scalar_type() != q->scalar_type() || !p->is_contiguous() || !q->is_contiguous() || p->size(-1) >= (1ll << 31))
+    return none();
+  Tensor out = at::empty(p->sizes(), p->options());
+  if (odit_cfg_combine(p->data_ptr(), q->data_ptr(), out.data_ptr(), p->numel() / p->size(-1), static_cast<int>(p->size(-1)),
+                       static_cast<float>(scale), norm, dt, w.stream) != 0)
+    return none();
+  return wrap(std::move(out));
+  NATIVE_END
+}
+
+// (x, v, dt)
+PyObject* py_euler_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  NATIVE_BEGIN
+  const Tensor *x, *v;
+  if (n != 3 || !(x = tensor_of(a[0])) || !(v = tensor_of(a[1]))) return none();
+  const double step = PyFloat_AsDouble(a[2]);
+  if (PyErr_Occurred()) return nullptr;
+  const Where w;
+  const int dt = code_of(*x);
+  if (dt < 0 || !w.holds(x) || !w.holds(v) || x->sizes() != v->sizes() || x->scalar_type() != v->scalar_type() ||
+      !x->is_contiguous() || !v->is_contiguous())
+    return none();
+  Tensor out = at::empty(x->sizes(), x->options());
+  if (odit_euler_step(x->data_ptr(), v->data_ptr(), out.data_ptr(), x->numel(), static_cast<float>(step), dt, w.stream) != 0) return none();
+  return wrap(std::move(out));
+  NATIVE_END
+}
+
+// (x, weight, bias or None, silu of x first)
+PyObject* py_linear_few(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  NATIVE_BEGIN
+  const Tensor *x, *wt, *b;
+  if (n != 4 || !(x = tensor_of(a[0])) || !(wt = tensor_of(a[1])) || !optional_tensor(a[2], &b)) return none();
+  const Where w;
+  if (!w.holds(x) || !w.holds(wt) || !w.holds(b)) return none();
+  const int dt = code_of(*x);
+  if (dt < 0 || x->dim() < 1 || wt->dim() != 2 || wt->stride(1) != 1 || wt->size(1) != x->size(-1) ||
+      wt->scalar_type() != x->scalar_type())
+    return none();
+  const int64_t N = wt->size(0), K = wt->size(1);
+  int64_t M, ldx;
+  if (N == 0 || K == 0 || N >= (1ll << 31) || !rows_of(*x, &M, &ldx) || M == 0 || M > 16) return none();
+  if (b && (b->numel() != N || !b->is_contiguous() || b->scalar_type() != x->scalar_type())) return none();
+  std::vector<int64_t> shape(x->sizes().begin(), x->sizes().end());
+  shape.back() = N;
+  Tensor out = at::empty(shape, x->options());
+  if (odit_linear_few(x->data_ptr(), wt->data_ptr(), ptr(b), out.data_ptr(), static_cast<int>(M), static_cast<int>(N),
+                      static_cast<int>(K), ldx, N > 1 ? wt->stride(0) : K, N, dt, PyObject_IsTrue(a[3]), w.stream) != 0)
+    return none();
+  return wrap(std::move(out));
+  NATIVE_END
+}
+
 // (x, weight, bias, gelu, residual, gate, gate_bias, prescaled, out, engine flags)
 PyObject* py_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   NATIVE_BEGIN
@@ -723,6 +806,39 @@ struct BlockCall {
                            lin_ws.p, lin_ws.bytes, where.stream));
   }
 };
+
+// (Linear module, x, silu of x first, engine flags): the module's projection of x with its own parameters as the module holds them now. None for a module that is not a plain torch Linear.
+PyObject* py_project(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  NATIVE_BEGIN
+  const Tensor* x;
+  if (n != 4 || g_linear_type == nullptr || !(x = tensor_of(a[1]))) return none();
+  const int silu = PyObject_IsTrue(a[2]);
+  const long flags = PyLong_AsLong(a[3]);
+  if (PyErr_Occurred()) return nullptr;
+  BlockCall c;
+  c.dtype = code_of(*x);
+  c.st = x->scalar_type();
+  Lin l;
+  int64_t M, ldx;
+  if ((c.dtype != ODIT_BF16 && c.dtype != ODIT_F16) || !c.operand(*x) || x->dim() < 1 || !c.linear(a[0], &l, false) ||
+      x->size(-1) != l.k || l.n == 0 || l.k == 0 || l.n >= (1ll << 31) || !rows_of(*x, &M, &ldx) || M == 0 || M >= (1ll << 31))
+    return none();
+  auto sizes = x->sizes().vec();
+  sizes.back() = l.n;
+  Tensor out = at::empty(sizes, x->options());
+  if (odit_linear_few(x->data_ptr(), l.w, l.b, out.data_ptr(), static_cast<int>(M), static_cast<int>(l.n), static_cast<int>(l.k), ldx,
+                      l.ldw, l.n, c.dtype, silu, c.where.stream) == 0)
+    return wrap(std::move(out));
+  if (silu) return none();
+  if (!linear_scratch(c.where, &c.lin_ws)) return nullptr;
+  const int epi = l.b ? ODIT_EPI_BIAS : ODIT_EPI_NONE;
+  if (odit_linear_rows(x->data_ptr(), l.w, l.b, out.data_ptr(), nullptr, nullptr, static_cast<int>(M), static_cast<int>(l.n),
+                       static_cast<int>(l.k), ldx, l.ldw, l.n, 0, epi, c.dtype, c.dtype, 0, 0, static_cast<unsigned>(flags),
+                       c.lin_ws.p, c.lin_ws.bytes, c.where.stream) != 0)
+    return none();
+  return wrap(std::move(out));
+  NATIVE_END
+}
 
 // a gate row per batch entry (and, in the pre-scaled form, the gate times the projection's bias), or no gate at all
 struct Gate {
@@ -1184,6 +1300,9 @@ PyObject* py_wan_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return none();
   if (!block_input(c, x)) return PyErr_Occurred() ? nullptr : none();
   const int64_t B = x->size(0), S = x->size(1), C = x->size(2), HD = H * D, T = ctx->dim() == 3 ? ctx->size(1) : 0;
+  // A CFG pair's rows keep the library's own kernels: guidance (scale 5 in the video pipelines) multiplies by about 6 what two
+  // orders of summation make of the same product, 0.3 % of the noise to 2 %, which is more than the choice gains here (0 to 7 %).
+  if (B > 1) c.engine |= ODIT_LINEAR_FIRST;
   if (B * S >= (1ll << 31) || S == 0 || T == 0 || (D != 64 && D != 128) || !c.operand(*ctx) || !ctx->is_contiguous() || ctx->size(0) != B || ctx->size(2) != C || HD != C) return none();
   const bool per_token = temb != nullptr;
   if (per_token) {
@@ -1376,6 +1495,11 @@ PyMethodDef kMethods[] = {
     NATIVE_FN("rotary", &py_rotary),
     NATIVE_FN("attn", &py_attn),
     NATIVE_FN("linear", &py_linear),
+    NATIVE_FN("linear_few", &py_linear_few),
+    NATIVE_FN("project", &py_project),
+    NATIVE_FN("time_sinusoid", &py_time_sinusoid),
+    NATIVE_FN("cfg_combine", &py_cfg_combine),
+    NATIVE_FN("euler_step", &py_euler_step),
     NATIVE_FN("classes", &py_classes),
     NATIVE_FN("qwen_block", &py_qwen_block),
     NATIVE_FN("flux_block", &py_flux_block),

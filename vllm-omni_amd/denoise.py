@@ -15,6 +15,8 @@ from dataclasses import dataclass
 import numpy as np
 import torch
 
+from . import kernels
+
 
 def calculate_shift(image_seq_len: int, base_seq_len: int = 256, max_seq_len: int = 4096,
                     base_shift: float = 0.5, max_shift: float = 1.15) -> float:
@@ -34,6 +36,9 @@ def flow_match_sigmas(num_inference_steps: int, image_seq_len: int) -> np.ndarra
 def combine_cfg_noise(noise_pred: torch.Tensor, neg_noise_pred: torch.Tensor, true_cfg_scale: float,
                       cfg_normalize: bool = False) -> torch.Tensor:
     """neg + s (pos - neg); with cfg_normalize, rescaled per token to the positive prediction's norm."""
+    done = kernels.cfg_combine(noise_pred, neg_noise_pred, true_cfg_scale, cfg_normalize)
+    if done is not None:
+        return done
     comb = neg_noise_pred + true_cfg_scale * (noise_pred - neg_noise_pred)
     if not cfg_normalize:
         return comb
@@ -41,6 +46,9 @@ def combine_cfg_noise(noise_pred: torch.Tensor, neg_noise_pred: torch.Tensor, tr
 
 
 def euler_step(latents: torch.Tensor, noise_pred: torch.Tensor, sigma: float, sigma_next: float) -> torch.Tensor:
+    done = kernels.euler_step(latents, noise_pred, sigma_next - sigma)
+    if done is not None:
+        return done
     return (latents.float() + (sigma_next - sigma) * noise_pred.float()).to(latents.dtype)
 
 
@@ -232,6 +240,8 @@ class CFGParallelMixin:
 
     def combine_cfg_noise(self, noise_pred: torch.Tensor, neg_noise_pred: torch.Tensor, true_cfg_scale: float,
                           cfg_normalize: bool = False) -> torch.Tensor:
+        if type(self).cfg_normalize_function is CFGParallelMixin.cfg_normalize_function:
+            return combine_cfg_noise(noise_pred, neg_noise_pred, true_cfg_scale, cfg_normalize)
         comb_pred = neg_noise_pred + true_cfg_scale * (noise_pred - neg_noise_pred)
         return self.cfg_normalize_function(noise_pred, comb_pred) if cfg_normalize else comb_pred
 

@@ -13,6 +13,8 @@ and the errors.
 
 from __future__ import annotations
 
+import math
+
 import torch
 from torch.nn.modules import module as _global_hooks
 
@@ -690,6 +692,46 @@ def _rows2d(t: torch.Tensor, name: str) -> tuple[torch.Tensor, int]:
     if t2 is None:
         raise ValueError(f"{name}: needs a contiguous tensor or a 2-D view with a row stride")
     return t2, (t2.stride(0) if t2.shape[0] > 1 else t2.shape[1])
+
+
+def linear_few(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None, silu_input: bool = False) -> torch.Tensor:
+    """x W^T (+ bias), or silu(x) W^T (+ bias), for an x of a few rows (conditioning vectors): one pass over the
+    weights. Anything the kernel does not take (more than 16 rows, float32, CPU tensors) goes through torch."""
+    done = (_nat or _load_native()).linear_few(x, weight, bias, silu_input)
+    return torch.nn.functional.linear(silu(x) if silu_input else x, weight, bias) if done is None else done
+
+
+def project(lin: torch.nn.Module, x: torch.Tensor, silu_input: bool = False) -> torch.Tensor:
+    """lin(x) or lin(silu(x)) for a Linear module of a model's stem, conditioning or head. A plain ``nn.Linear`` in inference goes down as one native call; a module with hooks or of another
+    class, and everything the kernels do not take, is called as it is."""
+    if x.is_cuda and native_blocks():
+        done = (_nat or _load_native()).project(lin, x, silu_input, _LINEAR_ENGINE_FLAGS)
+        if done is not None:
+            return done
+    return project(lin, silu(x)) if silu_input else lin(x)
+
+
+def time_sinusoid(t: torch.Tensor, dim: int, max_period: float, scale: float, dtype: torch.dtype) -> torch.Tensor | None:
+    """[n, dim] cosines and sines of the timesteps ``t`` [n] in one launch; None for what the kernel does not take."""
+    code = _DTYPE_CODE.get(dtype)
+    if code is None or not t.is_cuda or torch.is_grad_enabled():
+        return None
+    return (_nat or _load_native()).time_sinusoid(t, dim, -math.log(max_period), float(scale), code)
+
+
+def cfg_combine(pos: torch.Tensor, neg: torch.Tensor, scale: float, normalize: bool) -> torch.Tensor | None:
+    """neg + scale (pos - neg), with ``normalize`` rescaled to the norm of ``pos`` over the last dimension, rounded at every
+    operation as torch does; None for what the kernel does not take."""
+    if not pos.is_cuda or torch.is_grad_enabled() or not isinstance(scale, (float, int)):
+        return None
+    return (_nat or _load_native()).cfg_combine(pos, neg, float(scale), bool(normalize))
+
+
+def euler_step(x: torch.Tensor, v: torch.Tensor, dt: float) -> torch.Tensor | None:
+    """x + dt v in float32; None for what the kernel does not take."""
+    if not x.is_cuda or torch.is_grad_enabled() or not isinstance(dt, float):
+        return None
+    return (_nat or _load_native()).euler_step(x, v, dt)
 
 
 def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None, *, activation: str | None = None,
