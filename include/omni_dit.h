@@ -409,12 +409,17 @@ int odit_linear_few(const void* x, const void* w, const void* bias, void* out, i
 
 /* The small work of a denoise step, one launch each, rounded where the torch expressions of the reference round:
  * odit_time_sinusoid: t [n] (t_dtype) -> out [n, dim] (out_dtype) = cos | sin of scale * (t * exp(neg_log_period j / (dim / 2)))
- *   (diffusers Timesteps with flip_sin_to_cos, qwen_image_transformer.py:165);
+ *   (diffusers Timesteps with flip_sin_to_cos, qwen_image_transformer.py:165); `pre` other than 1: t is first rounded to
+ *   out_dtype, multiplied by it and rounded again (flux.py:462-466);
+ * odit_rope_tables: position ids [n_txt, n_axes] and [n_img, n_axes] (dtype, dense) -> float32 cosines and sines
+ *   [n_txt + n_img, sum(axes_dim) / 2], evaluated in float64 (flux.py:369-396); axes_dim is a host array of at most 4;
  * odit_cfg_combine: neg + scale * (pos - neg) over dense [rows, C], 16-bit types; `normalize`: every row brought back to the
  *   norm of pos (cfg_parallel.py:142-176); then C a multiple of 8 and 16-byte aligned tensors, else ODIT_ENOTSUP;
  * odit_euler_step: out = x + dt * v in float32 (pipeline schedulers' step). */
-int odit_time_sinusoid(const void* t, void* out, int64_t n, int dim, float neg_log_period, float scale, int t_dtype, int out_dtype,
-                       void* stream);
+int odit_time_sinusoid(const void* t, void* out, int64_t n, int dim, float neg_log_period, float scale, float pre, int t_dtype,
+                       int out_dtype, void* stream);
+int odit_rope_tables(const void* txt_ids, int64_t n_txt, const void* img_ids, int64_t n_img, float* cos_out, float* sin_out,
+                     const int* axes_dim, int n_axes, double theta, int dtype, void* stream);
 int odit_cfg_combine(const void* pos, const void* neg, void* out, int64_t rows, int C, float scale, int normalize, int dtype,
                      void* stream);
 int odit_euler_step(const void* x, const void* v, void* out, int64_t n, float dt, int dtype, void* stream);

@@ -39,3 +39,19 @@ def test_time_sinusoid(n, dim, scale, t_dtype):
     out = kernels.time_sinusoid(t, dim, 10000, scale, torch.float32)
     torch.testing.assert_close(out, want, rtol=0, atol=2e-4)
     assert torch.equal(kernels.time_sinusoid(t, dim, 10000, scale, torch.bfloat16), out.to(torch.bfloat16))
+    pre = kernels.time_sinusoid(t, dim, 10000, scale, torch.bfloat16, 1000.0)
+    scaled = (t.to(torch.bfloat16) * 1000).float()
+    assert torch.equal(pre, kernels.time_sinusoid(scaled, dim, 10000, scale, torch.bfloat16))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("axes", [(16, 56, 56), (8, 28, 28), (32, 80, 80)])
+@pytest.mark.parametrize("n_txt,n_img", [(0, 1), (1, 0), (7, 8), (15, 2), (512, 1025)])
+@torch.inference_mode()
+def test_rope_tables(n_txt, n_img, axes, dtype):
+    from vllm_omni_amd.blocks.flux import FluxPosEmbed
+    txt, img = ((torch.rand(n, 3, device="cuda") * 200).round().to(dtype) for n in (n_txt, n_img))
+    cos, sin = kernels.rope_tables(txt, img, axes, 10000)
+    want = FluxPosEmbed(10000, list(axes))(torch.cat((txt, img)).cpu())
+    torch.testing.assert_close(cos.cpu(), want[0].float(), rtol=0, atol=1e-7)
+    torch.testing.assert_close(sin.cpu(), want[1].float(), rtol=0, atol=1e-7)

@@ -41,12 +41,34 @@ class FluxRotary:
     [S, D/2] tables the fused kernel reads."""
 
     def __init__(self, cos: torch.Tensor, sin: torch.Tensor):
-        self.cos, self.sin = cos, sin
+        self._tables = (cos, sin)
         self.cos32, self.sin32 = cos.float().contiguous(), sin.float().contiguous()
         self._split = None
 
+    @classmethod
+    def of_ids(cls, pos_embed: FluxPosEmbed, txt_ids: torch.Tensor, img_ids: torch.Tensor) -> FluxRotary:
+        """From position ids: the float32 tables in one launch, the float64 ones only when somebody asks for them."""
+        done = kernels.rope_tables(txt_ids, img_ids, tuple(pos_embed.axes_dim), pos_embed.theta)
+        if done is None:
+            return cls(*pos_embed(torch.cat((txt_ids, img_ids), dim=0)))
+        r = cls.__new__(cls)
+        r.cos32, r.sin32 = done
+        r._tables, r._ids, r._split = None, (pos_embed, txt_ids, img_ids), None
+        return r
+
     def __iter__(self):
-        return iter((self.cos, self.sin))
+        if self._tables is None:
+            pos_embed, txt_ids, img_ids = self._ids
+            self._tables = pos_embed(torch.cat((txt_ids, img_ids), dim=0))
+        return iter(self._tables)
+
+    @property
+    def cos(self) -> torch.Tensor:
+        return tuple(self)[0]
+
+    @property
+    def sin(self) -> torch.Tensor:
+        return tuple(self)[1]
 
     def split(self, n_txt: int):
         """(image cos, image sin, text cos, text sin) rows of the float32 tables; kept for the blocks of a forward."""
@@ -345,11 +367,12 @@ class CombinedTimestepGuidanceTextProjEmbeddings(nn.Module):
             self.guidance_embedder = TimestepEmbedding(256, embedding_dim)
         self.text_embedder = PixArtAlphaTextProjection(pooled_projection_dim, embedding_dim)
 
-    def forward(self, timestep: torch.Tensor, guidance: torch.Tensor | None, pooled_projection: torch.Tensor):
+    def forward(self, timestep: torch.Tensor, guidance: torch.Tensor | None, pooled_projection: torch.Tensor,
+                pre: float = 1.0):
         proj = QwenTimestepProjEmbeddings.time_proj
-        emb = self.timestep_embedder(proj(timestep, scale=1.0, dtype=pooled_projection.dtype))
+        emb = self.timestep_embedder(proj(timestep, scale=1.0, dtype=pooled_projection.dtype, pre=pre))
         if guidance is not None:
-            emb = emb + self.guidance_embedder(proj(guidance, scale=1.0, dtype=pooled_projection.dtype))
+            emb = emb + self.guidance_embedder(proj(guidance, scale=1.0, dtype=pooled_projection.dtype, pre=pre))
         return emb + self.text_embedder(pooled_projection)
 
 
@@ -402,16 +425,21 @@ class FluxTransformer2DModel(nn.Module):
     def prepare(self, hidden_states, encoder_hidden_states, pooled_projections, timestep, img_ids, txt_ids,
                 guidance=None):
         img = kernels.project(self.x_embedder, hidden_states)
-        timestep = timestep.to(device=img.device, dtype=img.dtype) * 1000
-        if guidance is not None:
-            guidance = guidance.to(device=img.device, dtype=img.dtype) * 1000
-        temb = self.time_text_embed(timestep, guidance, pooled_projections)
+        if type(self.time_text_embed) is CombinedTimestepGuidanceTextProjEmbeddings and pooled_projections.dtype == img.dtype:
+            if guidance is not None:
+                guidance = guidance.to(device=img.device)
+            temb = self.time_text_embed(timestep.to(device=img.device), guidance, pooled_projections, pre=1000.0)
+        else:
+            timestep = timestep.to(device=img.device, dtype=img.dtype) * 1000
+            if guidance is not None:
+                guidance = guidance.to(device=img.device, dtype=img.dtype) * 1000
+            temb = self.time_text_embed(timestep, guidance, pooled_projections)
         txt = kernels.project(self.context_embedder, encoder_hidden_states)
         if txt_ids.ndim == 3:
             txt_ids = txt_ids[0]
         if img_ids.ndim == 3:
             img_ids = img_ids[0]
-        rotary = FluxRotary(*self.pos_embed(torch.cat((txt_ids, img_ids), dim=0)))
+        rotary = FluxRotary.of_ids(self.pos_embed, txt_ids, img_ids)
         return img, txt, temb, rotary
 
     def fuse_modulation(self) -> None:

@@ -443,12 +443,14 @@ class QwenTimestepProjEmbeddings(nn.Module):
 
     @staticmethod
     def time_proj(t: torch.Tensor, dim: int = 256, max_period: int = 10000, scale: float = 1000.0,
-                  dtype: torch.dtype = torch.float32):
+                  dtype: torch.dtype = torch.float32, pre: float = 1.0):
         """diffusers ``Timesteps(dim, flip_sin_to_cos=True, downscale_freq_shift=0, scale)``: fp32
-        frequencies times ``t.float()``, cosines first."""
-        done = kernels.time_sinusoid(t, dim, max_period, scale, dtype)
+        frequencies times ``t.float()``, cosines first; with ``pre``, of ``t.to(dtype) * pre``."""
+        done = kernels.time_sinusoid(t, dim, max_period, scale, dtype, pre)
         if done is not None:
             return done
+        if pre != 1.0:
+            t = t.to(dtype) * pre
         half = dim // 2
         freqs = torch.exp(-math.log(max_period) * torch.arange(half, dtype=torch.float32, device=t.device) / half)
         arg = scale * (t[:, None].float() * freqs[None, :])

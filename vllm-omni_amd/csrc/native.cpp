@@ -540,22 +540,50 @@ bool rows_of(const Tensor& t, int64_t* rows, int64_t* ld) {
   return true;
 }
 
-// (t [n], dim, -log(max_period), scale, dtype code of the result) -> [n, dim]
+// (t [n], dim, -log(max_period), scale, dtype code of the result, factor applied before in that type) -> [n, dim]
 PyObject* py_time_sinusoid(PyObject*, PyObject* const* a, Py_ssize_t n) {
   NATIVE_BEGIN
   const Tensor* t;
-  if (n != 5 || !(t = tensor_of(a[0]))) return none();
+  if (n != 6 || !(t = tensor_of(a[0]))) return none();
   const long dim = PyLong_AsLong(a[1]), code = PyLong_AsLong(a[4]);
-  const double period = PyFloat_AsDouble(a[2]), scale = PyFloat_AsDouble(a[3]);
+  const double period = PyFloat_AsDouble(a[2]), scale = PyFloat_AsDouble(a[3]), pre = PyFloat_AsDouble(a[5]);
   if (PyErr_Occurred()) return nullptr;
   const Where w;
   const int dt = code_of(*t);
   if (dt < 0 || !w.holds(t) || t->dim() != 1 || !t->is_contiguous() || dim <= 0 || dim % 2 || code < 0 || code > 2) return none();
   Tensor out = at::empty({t->size(0), dim}, t->options().dtype(code == ODIT_BF16 ? at::kBFloat16 : code == ODIT_F16 ? at::kHalf : at::kFloat));
   if (odit_time_sinusoid(t->data_ptr(), out.data_ptr(), t->size(0), static_cast<int>(dim), static_cast<float>(period),
-                         static_cast<float>(scale), dt, static_cast<int>(code), w.stream) != 0)
+                         static_cast<float>(scale), static_cast<float>(pre), dt, static_cast<int>(code), w.stream) != 0)
     return none();
   return wrap(std::move(out));
+  NATIVE_END
+}
+
+// (text ids [n, axes], image ids [m, axes], axis widths, theta) -> float32 (cos, sin), each [n + m, half]
+PyObject* py_rope_tables(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  NATIVE_BEGIN
+  const Tensor *t, *i;
+  if (n != 4 || !(t = tensor_of(a[0])) || !(i = tensor_of(a[1])) || !PyTuple_Check(a[2])) return none();
+  int axes[4], half = 0;
+  const Py_ssize_t n_axes = PyTuple_GET_SIZE(a[2]);
+  if (n_axes < 1 || n_axes > 4) return none();
+  for (Py_ssize_t k = 0; k < n_axes; ++k) {
+    axes[k] = static_cast<int>(PyLong_AsLong(PyTuple_GET_ITEM(a[2], k)));
+    half += axes[k] / 2;
+  }
+  const double theta = PyFloat_AsDouble(a[3]);
+  if (PyErr_Occurred()) return nullptr;
+  const Where w;
+  const int dt = code_of(*t);
+  if (dt < 0 || !w.holds(t) || !w.holds(i) || t->scalar_type() != i->scalar_type() || t->dim() != 2 || i->dim() != 2 ||
+      t->size(1) != n_axes || i->size(1) != n_axes || !t->is_contiguous() || !i->is_contiguous())
+    return none();
+  const int64_t rows = t->size(0) + i->size(0);
+  Tensor c = at::empty({rows, half}, t->options().dtype(at::kFloat)), s = at::empty({rows, half}, t->options().dtype(at::kFloat));
+  if (odit_rope_tables(t->data_ptr(), t->size(0), i->data_ptr(), i->size(0), c.data_ptr<float>(), s.data_ptr<float>(), axes,
+                       static_cast<int>(n_axes), theta, dt, w.stream) != 0)
+    return none();
+  return wrap2(std::move(c), std::move(s));
   NATIVE_END
 }
 
@@ -1498,6 +1526,7 @@ PyMethodDef kMethods[] = {
     NATIVE_FN("linear_few", &py_linear_few),
     NATIVE_FN("project", &py_project),
     NATIVE_FN("time_sinusoid", &py_time_sinusoid),
+    NATIVE_FN("rope_tables", &py_rope_tables),
     NATIVE_FN("cfg_combine", &py_cfg_combine),
     NATIVE_FN("euler_step", &py_euler_step),
     NATIVE_FN("classes", &py_classes),

@@ -1,4 +1,5 @@
-// The small work around the transformer in a denoise step: the timestep sinusoid, the CFG combination and the Euler update.
+// The small work around the transformer in a denoise step: the timestep sinusoid, the rotary tables of the position ids, the CFG
+// combination and the Euler update.
 // Every tensor here is a few KB to a few MB, so what bounds it is the number of launches and the host time of each: as torch
 // operations the three were 10, 7 and 5 launches (about 2 us each on the GPU and 4 to 8 us on the host); here each is one.
 // Every intermediate is rounded where the torch expression rounds it, with no contraction of multiply and add.
@@ -12,17 +13,50 @@ namespace {
 constexpr int kBlock = 256;
 constexpr int kMaxBlocks = 4096;
 
-// out[i, :] = cos | sin of scale * (t[i] * exp(-log(max_period) j / half)); the accurate exp, cos and sin, which torch calls
+// out[i, :] = cos | sin of scale * (t[i] * exp(-log(max_period) j / half)); the accurate exp, cos and sin, which torch calls.
+// `pre` other than 1 is a factor that the caller's expression applies in T before it (Flux: timestep.to(T) * 1000).
 template <typename TT, typename T>
 __global__ __launch_bounds__(kBlock) void time_sinusoid_kernel(const TT* __restrict__ t, T* __restrict__ out, int64_t n, int half,
-                                                               float neg_log_period, float scale) {
+                                                               float neg_log_period, float scale, float pre) {
   for (int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x; i < n * half; i += static_cast<int64_t>(gridDim.x) * kBlock) {
     const int64_t row = i / half;
     const int j = static_cast<int>(i - row * half);
     const float freq = expf(neg_log_period * static_cast<float>(j) / static_cast<float>(half));
-    const float arg = scale * (to_float(t[row]) * freq);
+    float tv = to_float(t[row]);
+    if (pre != 1.f) tv = round_to<T>(round_to<T>(tv) * pre);
+    const float arg = scale * (tv * freq);
     out[row * 2 * half + j] = from_float<T>(cosf(arg));
     out[row * 2 * half + half + j] = from_float<T>(sinf(arg));
+  }
+}
+
+// Rotary tables of position ids, text rows before image rows: out[row, j] = cos | sin of id[row, axis] * theta^(-2 k / d), k the
+// column j within its axis, everything in float64 up to the rounding to float32. As torch operations this was 33 launches
+// (4 to 7 us each, 150 us per step, and as much host time again); as one launch it takes about 6 us at 4608 rows of 64 columns,
+// bound by the float64 pow, sin and cos. A thread keeps one column, so the pow is paid once for kRopeRows / 4 rows.
+constexpr int kMaxAxes = 4, kRopeRows = 16;
+struct RopeAxes {
+  int count, half;           // axes, columns in all
+  int start[kMaxAxes + 1];   // first column of every axis
+};
+template <typename T>
+__global__ __launch_bounds__(kBlock) void rope_tables_kernel(const T* __restrict__ txt, int64_t n_txt, const T* __restrict__ img,
+                                                             int64_t n, float* __restrict__ cos_out, float* __restrict__ sin_out,
+                                                             RopeAxes ax, double theta) {
+  const int64_t row_end = min(n, (static_cast<int64_t>(blockIdx.x) + 1) * kRopeRows);
+  for (int j = threadIdx.x % 64; j < ax.half; j += 64) {
+    int a = 0;
+    while (a + 1 < ax.count && j >= ax.start[a + 1]) ++a;
+    const int d = 2 * (ax.start[a + 1] - ax.start[a]);
+    const double inv = 1.0 / pow(theta, static_cast<double>(2 * (j - ax.start[a])) / static_cast<double>(d));
+    for (int64_t row = static_cast<int64_t>(blockIdx.x) * kRopeRows + threadIdx.x / 64; row < row_end; row += kBlock / 64) {
+      const T* id = row < n_txt ? txt + row * ax.count : img + (row - n_txt) * ax.count;
+      const double ang = static_cast<double>(to_float(id[a])) * inv;
+      double c, s;
+      sincos(ang, &s, &c);
+      cos_out[row * ax.half + j] = static_cast<float>(c);
+      sin_out[row * ax.half + j] = static_cast<float>(s);
+    }
   }
 }
 
@@ -87,26 +121,51 @@ int blocks_for(int64_t threads) {
 }
 
 template <typename TT, typename T>
-int launch_sinusoid(const void* t, void* out, int64_t n, int half, float neg_log_period, float scale, hipStream_t s) {
+int launch_sinusoid(const void* t, void* out, int64_t n, int half, float neg_log_period, float scale, float pre, hipStream_t s) {
   time_sinusoid_kernel<TT, T><<<blocks_for(n * half), kBlock, 0, s>>>(static_cast<const TT*>(t), static_cast<T*>(out), n, half,
-                                                                     neg_log_period, scale);
+                                                                     neg_log_period, scale, pre);
   return check_launch("odit_time_sinusoid");
 }
 
 }  // namespace
 }  // namespace odit
 
-extern "C" int odit_time_sinusoid(const void* t, void* out, int64_t n, int dim, float neg_log_period, float scale, int t_dtype,
-                                  int out_dtype, void* stream) {
+extern "C" int odit_time_sinusoid(const void* t, void* out, int64_t n, int dim, float neg_log_period, float scale, float pre,
+                                  int t_dtype, int out_dtype, void* stream) {
   using namespace odit;
   ODIT_CHECK_ARG(t && out && n >= 0 && dim > 0 && dim % 2 == 0, "odit_time_sinusoid: needs t, out and an even dim (n=%lld dim=%d)",
                  static_cast<long long>(n), dim);
   if (n == 0) return ODIT_OK;
   const hipStream_t s = static_cast<hipStream_t>(stream);
   ODIT_DISPATCH_DTYPE(t_dtype, TT, {
-    ODIT_DISPATCH_DTYPE(out_dtype, T, { return launch_sinusoid<TT, T>(t, out, n, dim / 2, neg_log_period, scale, s); });
+    ODIT_DISPATCH_DTYPE(out_dtype, T, { return launch_sinusoid<TT, T>(t, out, n, dim / 2, neg_log_period, scale, pre, s); });
   });
   return ODIT_OK;
+}
+
+extern "C" int odit_rope_tables(const void* txt_ids, int64_t n_txt, const void* img_ids, int64_t n_img, float* cos_out,
+                                float* sin_out, const int* axes_dim, int n_axes, double theta, int dtype, void* stream) {
+  using namespace odit;
+  ODIT_CHECK_ARG(n_txt >= 0 && n_img >= 0 && (txt_ids || n_txt == 0) && (img_ids || n_img == 0) && cos_out && sin_out && axes_dim &&
+                     n_axes >= 1 && n_axes <= kMaxAxes && theta > 0,
+                 "odit_rope_tables: bad arguments (rows %lld + %lld, %d axes)", static_cast<long long>(n_txt),
+                 static_cast<long long>(n_img), n_axes);
+  RopeAxes ax{};
+  ax.count = n_axes;
+  for (int i = 0; i < n_axes; ++i) {
+    ODIT_CHECK_ARG(axes_dim[i] > 0 && axes_dim[i] % 2 == 0, "odit_rope_tables: axis widths must be even, got %d", axes_dim[i]);
+    ax.start[i + 1] = ax.start[i] + axes_dim[i] / 2;
+  }
+  ax.half = ax.start[n_axes];
+  const int64_t n = n_txt + n_img;
+  if (n == 0) return ODIT_OK;
+  const int64_t blocks = (n + kRopeRows - 1) / kRopeRows;
+  ODIT_CHECK_ARG(blocks <= (1 << 24), "odit_rope_tables: too many rows (%lld)", static_cast<long long>(n));
+  ODIT_DISPATCH_DTYPE(dtype, T, {
+    rope_tables_kernel<T><<<static_cast<int>(blocks), kBlock, 0, static_cast<hipStream_t>(stream)>>>(
+        static_cast<const T*>(txt_ids), n_txt, static_cast<const T*>(img_ids), n, cos_out, sin_out, ax, theta);
+  });
+  return check_launch("odit_rope_tables");
 }
 
 extern "C" int odit_cfg_combine(const void* pos, const void* neg, void* out, int64_t rows, int C, float scale, int normalize,

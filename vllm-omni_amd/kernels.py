@@ -711,12 +711,22 @@ def project(lin: torch.nn.Module, x: torch.Tensor, silu_input: bool = False) -> 
     return project(lin, silu(x)) if silu_input else lin(x)
 
 
-def time_sinusoid(t: torch.Tensor, dim: int, max_period: float, scale: float, dtype: torch.dtype) -> torch.Tensor | None:
-    """[n, dim] cosines and sines of the timesteps ``t`` [n] in one launch; None for what the kernel does not take."""
+def time_sinusoid(t: torch.Tensor, dim: int, max_period: float, scale: float, dtype: torch.dtype,
+                  pre: float = 1.0) -> torch.Tensor | None:
+    """[n, dim] cosines and sines of the timesteps ``t`` [n], or of ``t.to(dtype) * pre``, in one launch; None for what the
+    kernel does not take."""
     code = _DTYPE_CODE.get(dtype)
     if code is None or not t.is_cuda or torch.is_grad_enabled():
         return None
-    return (_nat or _load_native()).time_sinusoid(t, dim, -math.log(max_period), float(scale), code)
+    return (_nat or _load_native()).time_sinusoid(t, dim, -math.log(max_period), float(scale), code, float(pre))
+
+
+def rope_tables(txt_ids: torch.Tensor, img_ids: torch.Tensor, axes_dim: tuple[int, ...], theta: float):
+    """float32 (cos, sin) rotary tables of text ids followed by image ids, evaluated in float64, in one launch; None for what
+    the kernel does not take."""
+    if not txt_ids.is_cuda or torch.is_grad_enabled():
+        return None
+    return (_nat or _load_native()).rope_tables(txt_ids, img_ids, axes_dim, float(theta))
 
 
 def cfg_combine(pos: torch.Tensor, neg: torch.Tensor, scale: float, normalize: bool) -> torch.Tensor | None:
