@@ -1,0 +1,74 @@
+"""What the models form from their parameters follows the parameters, however they are written (CPU)."""
+
+import pytest
+import torch
+
+
+def _write(p, value, how):
+    if how == "data":        # the usual form of a weight loader: neither the version counter nor the address changes
+        p.data.copy_(value)
+    else:
+        with torch.no_grad():
+            p.copy_(value)
+
+
+def _random_(model):
+    g = torch.Generator().manual_seed(0)
+    for p in model.parameters():
+        p.data.copy_(torch.randn(p.shape, generator=g) * 0.1)
+    return model
+
+
+@pytest.mark.parametrize("how", ["data", "in place"])
+def test_qwen_gate_rows_follow_the_biases(how):
+    from vllm_omni_amd.blocks.qwen_image import QwenImageTransformer2DModel
+
+    model = _random_(QwenImageTransformer2DModel(num_layers=2, attention_head_dim=64, num_attention_heads=1, joint_attention_dim=64,
+                                                 axes_dims_rope=(8, 28, 28)).to(torch.bfloat16))
+    mods = torch.randn(2, 2, 2, 6 * 64).to(torch.bfloat16)
+    model.all_gate_rows(mods)
+    for i, pick in enumerate((lambda b: b.attn.to_out, lambda b: b.img_mlp.net[2], lambda b: b.attn.to_add_out, lambda b: b.txt_mlp.net[2])):
+        bias = pick(model.transformer_blocks[1]).bias
+        _write(bias, torch.full_like(bias, 0.5 + i), how)
+        gates, gb = model.all_gate_rows(mods)
+        assert gb.dtype == torch.float32
+        assert torch.equal(gb[:, 1, i // 2, i % 2], gates[:, 1, i // 2, i % 2] * (0.5 + i))
+
+
+@pytest.mark.parametrize("how", ["data", "in place"])
+def test_flux_gate_rows_follow_the_biases(how):
+    from vllm_omni_amd.blocks.flux import FluxTransformer2DModel
+
+    model = _random_(FluxTransformer2DModel(num_layers=1, num_single_layers=2, attention_head_dim=64, num_attention_heads=1,
+                                            joint_attention_dim=64, pooled_projection_dim=8, axes_dims_rope=(8, 28, 28)).to(torch.bfloat16))
+    mods = (torch.randn(2, 1, 2, 6 * 64).to(torch.bfloat16), torch.randn(2, 2, 3 * 64).to(torch.bfloat16))
+    model.all_gate_rows(mods)
+    dual, single = model.transformer_blocks[0].ff_context.net[2].bias, model.single_transformer_blocks[1].proj_out.bias
+    _write(dual, torch.full_like(dual, 0.5), how)
+    _write(single, torch.full_like(single, 2.0), how)
+    (dg, dgb), (sg, sgb) = model.all_gate_rows(mods)
+    assert dgb.dtype == sgb.dtype == torch.float32
+    assert torch.equal(dgb[:, 0, 1, 1], dg[:, 0, 1, 1] * 0.5)
+    assert torch.equal(sgb[:, 1], sg[:, 1] * 2.0)
+
+
+@pytest.mark.parametrize("how", ["data", "in place"])
+def test_wan_rows_follow_the_parameters(how):
+    from vllm_omni_amd.blocks.wan import WanTransformer3DModel
+
+    model = _random_(WanTransformer3DModel(num_attention_heads=1, attention_head_dim=64, text_dim=32, ffn_dim=128, num_layers=2).to(torch.bfloat16))
+    mods = torch.randn(2, 3, 6, 64)
+    block = model.blocks[1]
+    for _ in range(2):  # the second time round whatever the first could have kept is there
+        for p in (block.attn1.to_out.bias, block.ffn.net_2.bias, block.norm2.weight, block.norm2.bias, block.scale_shift_table):
+            _write(p, torch.randn(p.shape).to(p.dtype), how)
+        gb = model.gate_bias_rows(mods)
+        # (rows of the gates and of gate * bias have to lie equally far apart from batch entry to batch entry)
+        assert gb.shape == (2, 3, 2, 64) and gb.dtype == torch.float32 and gb[1].stride(0) == mods[1].stride(0)
+        assert torch.equal(gb[1, :, 0], mods[1, :, 2] * block.attn1.to_out.bias.float())
+        assert torch.equal(gb[1, :, 1], mods[1, :, 5] * block.ffn.net_2.bias.float())
+        one = (mods[1] * block.gated_biases())[:, 2::3]
+        assert torch.equal(one, gb[1])
+        for w, b in (model.norm2_affines()[1], block._norm2_affine()):
+            assert torch.equal(w, block.norm2.weight.float()) and torch.equal(b, block.norm2.bias.float())
+        assert torch.equal(block._table(), block.scale_shift_table[0].float())

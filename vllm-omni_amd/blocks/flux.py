@@ -415,7 +415,6 @@ class FluxTransformer2DModel(nn.Module):
         self.proj_out = nn.Linear(self.inner_dim, patch_size * patch_size * self.out_channels, bias=True)
         self.parallel_config = None
         self.do_true_cfg = False
-        self._res_bias = None
 
     # -- stages ---------------------------------------------------------------------------------
     @property
@@ -463,25 +462,18 @@ class FluxTransformer2DModel(nn.Module):
                 l.weight.data, l.bias.data = w_all[r:r + n], b_all[r:r + n]
                 r += n
         self._mod_weight, self._mod_bias = w_all, b_all
-        self._res_bias = None
 
     def _gated_biases(self):
-        """float32 biases of the gated output projections, dual [L, 2 (hidden, context), 2, C] and single
-        [Ls, C] (None where there are no such blocks); rebuilt when any of them has been written since."""
+        """Biases of the gated output projections, dual [L, 2 (hidden, context), 2, C] and single [Ls, C] (None where
+        there are no such blocks), read on every call: a kept copy would miss ``p.data.copy_``."""
         dual = [p for blk in self.transformer_blocks
                 for p in (blk.attn.to_out[0].bias, blk.ff.net[2].bias, blk.attn.to_add_out.bias, blk.ff_context.net[2].bias)]
         single = [blk.proj_out.bias for blk in self.single_transformer_blocks]
-        ps = dual + single
-        tag = (sum(p._version for p in ps), ps[0].device, ps[0].dtype)
-        if self._res_bias is None or self._res_bias[0] != tag:
-            C = self.inner_dim
-            d = torch.stack(dual).detach().float().view(len(self.transformer_blocks), 2, 2, C) if dual else None
-            sgl = torch.stack(single).detach().float() if single else None
-            self._res_bias = (tag, d, sgl)
-        return self._res_bias[1], self._res_bias[2]
+        d = torch.stack(dual).detach().view(len(self.transformer_blocks), 2, 2, self.inner_dim) if dual else None
+        return d, torch.stack(single).detach() if single else None
 
     def all_gate_rows(self, mods):
-        """float32 (gates, gates * biases) of every gated projection, two small elementwise ops per step:
+        """float32 (gates, gates * biases) of every gated projection, three small ops per step and kind of block:
         dual [B, L, 2, 2, C] pairs and single [B, Ls, C] pairs (None where there are no such blocks)."""
         if mods is None or mods[0].dtype == torch.float32:
             return None, None

@@ -246,49 +246,44 @@ class WanTransformerBlock(nn.Module):
         self.ffn = WanFeedForward(dim=dim, inner_dim=ffn_dim, dim_out=dim)
         self.norm3 = FP32LayerNorm(dim, eps, elementwise_affine=False)
         self.scale_shift_table = nn.Parameter(torch.randn(1, 6, dim) / dim ** 0.5)
-        self._ln2_f32: tuple[int, torch.Tensor, torch.Tensor] | None = None
-        self._table_f32: tuple[tuple, torch.Tensor] | None = None
-        self._bias_f32: tuple[tuple, torch.Tensor] | None = None
 
+    # What follows is formed from the parameters on every call, here or by the model for all blocks at once. (No copy is
+    # kept: ``p.data.copy_`` changes neither a parameter's version counter nor its address, and a copy made on one
+    # stream may not be ready on another.)
     def _table(self) -> torch.Tensor:
-        """float32 [6, C] copy of scale_shift_table, refreshed when the parameter changes."""
-        p = self.scale_shift_table
-        tag = (p._version, p.data_ptr(), p.device)
-        if self._table_f32 is None or self._table_f32[0] != tag:
-            self._table_f32 = (tag, p.detach().float().reshape(6, -1).contiguous())
-        return self._table_f32[1]
+        """float32 [6, C] form of scale_shift_table."""
+        return self.scale_shift_table.detach().float().reshape(6, -1)
 
     def gated_biases(self) -> torch.Tensor:
-        """float32 [6, C]: in rows 2 and 5 the biases of the projections those gates scale (attn1.to_out, ffn.net_2),
-        zero elsewhere: times the modulation rows it gives gate * bias rows that lie where the gate rows do."""
-        ps = (self.attn1.to_out.bias, self.ffn.net_2.bias)
-        tag = tuple((p._version, p.data_ptr(), p.device) for p in ps)
-        if self._bias_f32 is None or self._bias_f32[0] != tag:
-            t = torch.zeros((6, ps[0].shape[0]), dtype=torch.float32, device=ps[0].device)
-            t[2], t[5] = ps[0].detach().float(), ps[1].detach().float()
-            self._bias_f32 = (tag, t)
-        return self._bias_f32[1]
+        """[6, C]: in row 2 the bias of attn1.to_out, in row 5 that of ffn.net_2, the projections those gates scale (the
+        other rows repeat them): times the modulation rows it gives gate * bias rows that lie where the gate rows do."""
+        return torch.stack(self.gated_bias_rows()).detach()
 
-    def _norm2_affine(self):
-        """float32 copies of norm2's weight/bias, refreshed when the parameters change."""
-        w, b = self.norm2.weight, self.norm2.bias
-        tag = (w._version, b._version, w.data_ptr(), w.device)
-        if self._ln2_f32 is None or self._ln2_f32[0] != tag:
-            self._ln2_f32 = (tag, w.detach().float().contiguous(), b.detach().float().contiguous())
-        return self._ln2_f32[1], self._ln2_f32[2]
+    def gated_bias_rows(self) -> tuple[torch.Tensor, ...]:
+        return (self.attn1.to_out.bias,) * 3 + (self.ffn.net_2.bias,) * 3
+
+    def _norm2_affine(self) -> tuple[torch.Tensor, torch.Tensor]:
+        """float32 forms of norm2's weight and bias."""
+        return self.norm2.weight.detach().float().contiguous(), self.norm2.bias.detach().float().contiguous()
 
     def forward(self, hidden_states: torch.Tensor, encoder_hidden_states: torch.Tensor, temb: torch.Tensor,
-                rotary_emb=None, mod: torch.Tensor | None = None,
-                gate_bias: torch.Tensor | None = None) -> torch.Tensor:
+                rotary_emb=None, mod: torch.Tensor | None = None, gate_bias: torch.Tensor | None = None,
+                table: torch.Tensor | None = None,
+                norm2_affine: tuple[torch.Tensor, torch.Tensor] | None = None) -> torch.Tensor:
         """``mod`` = float32 [B, 6, C] = scale_shift_table + temb when the caller formed it for all
         blocks at once; otherwise it is formed here as in the reference. ``gate_bias`` = float32 [B, 2, C]:
-        the two gates times the biases of the projections they scale (attn1.to_out, ffn.net_2)."""
+        the two gates times the biases of the projections they scale (attn1.to_out, ffn.net_2). ``table`` = float32 [6, C],
+        ``norm2_affine`` = float32 weight and bias [C], likewise formed by the caller for all blocks."""
+        if norm2_affine is None and not isinstance(self.norm2, nn.Identity):
+            norm2_affine = self._norm2_affine()
+        if mod is None and temb.ndim == 4 and table is None:
+            table = self._table()
         if kernels.native_blocks() and hidden_states.dtype != torch.float32:
-            done = self._forward_native(hidden_states, encoder_hidden_states, temb, rotary_emb, mod, gate_bias)
+            done = self._forward_native(hidden_states, encoder_hidden_states, temb, rotary_emb, mod, gate_bias, table, norm2_affine)
             if done is not None:
                 return done
         if mod is None and temb.ndim == 4:
-            return self._forward_per_token(hidden_states, encoder_hidden_states, temb, rotary_emb)
+            return self._forward_per_token(hidden_states, encoder_hidden_states, temb, rotary_emb, table, norm2_affine)
         if mod is None:
             mod = self.scale_shift_table + temb.float()
         shift_msa, scale_msa, gate_msa, c_shift, c_scale, c_gate = (mod[:, i] for i in range(6))
@@ -300,14 +295,13 @@ class WanTransformerBlock(nn.Module):
         if isinstance(self.norm2, nn.Identity):
             n = x
         else:
-            lw, lb = self._norm2_affine()
+            lw, lb = norm2_affine
             n = kernels.adaln_modulate(x, None, None, eps=self.eps, ln_weight=lw, ln_bias=lb, out=n)
         x = self.attn2(n, encoder_hidden_states, residual=x, out=x)
         n = kernels.adaln_modulate(x, c_shift, c_scale, eps=self.eps, out=n if n is not x else None)
         return project_residual(self.ffn.net_2, self.ffn.net_0(n), x, c_gate, out=x, pre=pre2)
 
-
-    def _forward_native(self, x, ctx, temb, rotary_emb, mod, gate_bias):
+    def _forward_native(self, x, ctx, temb, rotary_emb, mod, gate_bias, table, norm2_affine):
         """The whole block as one native call, or None where the call or a submodule is not of the plain form."""
         rot = _rotary(rotary_emb)
         per_token = mod is None and temb.ndim == 4
@@ -317,20 +311,20 @@ class WanTransformerBlock(nn.Module):
             mod = self.scale_shift_table + temb.float()
         if gate_bias is None and not per_token:
             gate_bias = (mod * self.gated_biases())[:, 2::3]
-        lw, lb = (None, None) if isinstance(self.norm2, nn.Identity) else self._norm2_affine()
+        lw, lb = norm2_affine if norm2_affine is not None else (None, None)
         a = self.attn1
         return kernels.native().wan_block(self, a.num_heads, a.head_dim, x, ctx, None if per_token else mod,
                                           None if per_token else gate_bias, temb if per_token else None,
-                                          self._table() if per_token else None, lw, lb, rot.cos32, rot.sin32,
+                                          table if per_token else None, lw, lb, rot.cos32, rot.sin32,
                                           qwen_image.FUSE_MIN_ROWS, kernels.linear_engine_flags())
 
-    def _forward_per_token(self, x: torch.Tensor, ctx: torch.Tensor, temb: torch.Tensor, rotary_emb) -> torch.Tensor:
+    def _forward_per_token(self, x: torch.Tensor, ctx: torch.Tensor, temb: torch.Tensor, rotary_emb, tab: torch.Tensor,
+                           norm2_affine: tuple[torch.Tensor, torch.Tensor] | None) -> torch.Tensor:
         """temb [B, S, 6, C] (wan.py:641-652): every token has its own six modulation rows. The reference
         forms table + temb.float() as six float32 [B,S,C] tensors per block; here the kernels read the
         rows of ``temb`` as they are and add the float32 table row in registers — the same fp32 sum."""
         if temb.shape[:2] != x.shape[:2] or temb.shape[2] != 6 or temb.stride(-1) != 1:
             raise ValueError(f"per-token temb must be [B,S,6,C] matching x, got {tuple(temb.shape)}")
-        tab = self._table()
         row = lambda i: temb[:, :, i]  # noqa: E731  ([B,S,C] view, token stride 6C)
         n = kernels.adaln_modulate(x, row(0), row(1), eps=self.eps, shift_bias=tab[0], scale_bias=tab[1])
         a = self.attn1(n, rotary_emb)
@@ -338,7 +332,7 @@ class WanTransformerBlock(nn.Module):
         if isinstance(self.norm2, nn.Identity):
             n = x
         else:
-            lw, lb = self._norm2_affine()
+            lw, lb = norm2_affine
             n = kernels.adaln_modulate(x, None, None, eps=self.eps, ln_weight=lw, ln_bias=lb, out=n)
         x = self.attn2(n, ctx, residual=x, out=x)
         n = kernels.adaln_modulate(x, row(3), row(4), eps=self.eps, shift_bias=tab[3], scale_bias=tab[4],
@@ -523,17 +517,30 @@ class WanTransformer3DModel(nn.Module):
         tables = torch.cat([blk.scale_shift_table for blk in self.blocks], dim=0)  # [L, 6, C]
         return tables.unsqueeze(1) + timestep_proj.float().unsqueeze(0)
 
+    def gate_bias_rows(self, mods: torch.Tensor) -> torch.Tensor:
+        """float32 [L, B, 2, C]: every block's two gates (rows 2 and 5 of ``mods``) times the biases they scale."""
+        biases = torch.stack([b for blk in self.blocks for b in blk.gated_bias_rows()]).detach()
+        return (mods * biases.view(len(self.blocks), 1, 6, -1))[:, :, 2::3]
+
+    def norm2_affines(self) -> list:
+        """Every block's norm2 weight and bias as float32 rows, two small ops per step (None: the block looks itself)."""
+        norms = [blk.norm2 for blk in self.blocks]
+        if any(type(n) is not FP32LayerNorm for n in norms):
+            return [None] * len(norms)
+        rows = torch.stack([t for n in norms for t in (n.weight, n.bias)]).detach().float()
+        return [(rows[2 * i], rows[2 * i + 1]) for i in range(len(norms))]
+
     def run_blocks(self, x, ctx, timestep_proj, rotary):
+        affines = self.norm2_affines()
         if timestep_proj.ndim == 4:  # per-token timesteps: the blocks read the rows of timestep_proj directly
-            for block in self.blocks:
-                x = block(x, ctx, timestep_proj, rotary)
+            tables = torch.cat([blk.scale_shift_table for blk in self.blocks], dim=0).detach().float() if len(self.blocks) else ()
+            for block, table, affine in zip(self.blocks, tables, affines):
+                x = block(x, ctx, timestep_proj, rotary, table=table, norm2_affine=affine)
             return x
         mods = self.all_modulations(timestep_proj)
-        gb = None
-        if x.dtype != torch.float32:  # gates (rows 2 and 5) times the biases they scale, [L, B, 2, C]
-            gb = (mods * torch.stack([blk.gated_biases() for blk in self.blocks]).unsqueeze(1))[:, :, 2::3]
+        gb = self.gate_bias_rows(mods) if x.dtype != torch.float32 else None
         for i, block in enumerate(self.blocks):
-            x = block(x, ctx, None, rotary, mod=mods[i], gate_bias=None if gb is None else gb[i])
+            x = block(x, ctx, None, rotary, mod=mods[i], gate_bias=None if gb is None else gb[i], norm2_affine=affines[i])
         return x
 
     def finish(self, x: torch.Tensor, temb: torch.Tensor, grid: tuple[int, int, int], return_dict: bool = True):
