@@ -16,7 +16,6 @@ qit.py:1073-1113). Differences are all below the module interfaces:
 from __future__ import annotations
 
 import math
-from functools import lru_cache
 from typing import Any
 
 import torch
@@ -30,6 +29,7 @@ from ..attention.layer import Attention
 from ..layers.adalayernorm import AdaLayerNorm, adaln_pair
 from ..layers.rmsnorm import RMSNorm
 from ..layers.rope import RotaryEmbedding
+from .tables import TableCache
 
 
 def _require_single_gpu(od_config: Any | None) -> None:
@@ -163,8 +163,8 @@ class QwenEmbedRope(nn.Module):
             1.0 / torch.pow(theta, torch.arange(0, d, 2, device=cpu).to(torch.float32).div(d)) for d in self.axes_dim])
         self.axis_of = torch.repeat_interleave(torch.arange(len(self.axes_dim), device=cpu),
                                                torch.tensor([d // 2 for d in self.axes_dim], device=cpu))
-        self._tables = lru_cache(maxsize=16)(self._build)
-        self._float_tables = lru_cache(maxsize=16)(self._split)
+        self._tables = TableCache(self._build, 16)
+        self._float_tables = TableCache(self._split, 16)
 
     def _table(self, positions: torch.Tensor) -> torch.Tensor:
         """positions: int64 [N, 3] -> complex64 [N, sum(d) / 2] unit phasors."""
@@ -231,6 +231,9 @@ class RotaryTables:
         self.vid_freqs, self.txt_freqs = vid_freqs, txt_freqs
         self.img_cos, self.img_sin = vid_freqs.real.contiguous(), vid_freqs.imag.contiguous()
         self.txt_cos, self.txt_sin = txt_freqs.real.contiguous(), txt_freqs.imag.contiguous()
+
+    def tensors(self) -> tuple[torch.Tensor, ...]:
+        return self.vid_freqs, self.txt_freqs, self.img_cos, self.img_sin, self.txt_cos, self.txt_sin
 
     def __iter__(self):  # unpacks like the reference's (vid_freqs, txt_freqs) tuple
         return iter((self.vid_freqs, self.txt_freqs))
@@ -482,11 +485,12 @@ class AdaLayerNormContinuous(nn.Module):
         return kernels.adaln_modulate(x, shift, scale, eps=self.eps)
 
 
-@lru_cache(maxsize=16)
-def _conditioning_index(samples: tuple, device: str) -> torch.Tensor:
-    """Built on the host once per set of image shapes, like the rotary tables."""
+def _build_conditioning_index(samples: tuple, device: str) -> torch.Tensor:
     rows = [[0] * math.prod(s[0]) + [1] * sum(math.prod(x) for x in s[1:]) for s in samples]
     return torch.tensor(rows, device=device, dtype=torch.int32)
+
+
+_conditioning_index = TableCache(_build_conditioning_index, 16)  # once per set of image shapes, like the rotary tables
 
 
 class QwenImageTransformer2DModel(nn.Module):

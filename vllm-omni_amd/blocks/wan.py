@@ -26,7 +26,6 @@ to the text attention before the output projection.
 from __future__ import annotations
 
 import math
-from functools import lru_cache
 from typing import Any
 
 import torch
@@ -39,6 +38,7 @@ from ..attention.layer import Attention
 from . import qwen_image
 from .qwen_image import (ApproxGELU, QwenTimestepProjEmbeddings, TimestepEmbedding, Transformer2DModelOutput,
                          project_residual)
+from .tables import TableCache
 
 
 class DistributedRMSNorm(nn.Module):
@@ -72,6 +72,9 @@ class WanRotary:
     def __iter__(self):
         return iter((self.freqs_cos, self.freqs_sin))
 
+    def tensors(self) -> tuple[torch.Tensor, ...]:
+        return self.freqs_cos, self.freqs_sin, self.cos32, self.sin32
+
 
 def _rotary(rotary_emb) -> WanRotary | None:
     if rotary_emb is None or isinstance(rotary_emb, WanRotary):
@@ -96,7 +99,7 @@ class WanRotaryPosEmbed(nn.Module):
             sin.append(ang.sin().float().repeat_interleave(2, dim=-1))
         self.register_buffer("freqs_cos", torch.cat(cos, dim=1), persistent=False)
         self.register_buffer("freqs_sin", torch.cat(sin, dim=1), persistent=False)
-        self._tables = lru_cache(maxsize=8)(self._build)
+        self._tables = TableCache(self._build, 8)
 
     def _build(self, ppf: int, pph: int, ppw: int, device: str) -> WanRotary:
         D = self.attention_head_dim
