@@ -1,0 +1,90 @@
+"""What a user changes in a module tree takes effect: hooks run, replaced submodules and switches are used, although a
+plain tree runs through native calls that never call the modules."""
+
+import pytest
+import torch
+
+from test_gpu_native_path import _flux, _qwen
+from vllm_omni_amd.hooks.base import HookRegistry, ModelHook
+
+pytestmark = pytest.mark.gpu
+
+
+def _both(monkeypatch, call):
+    """(result of the default path, result of the per-kernel path)"""
+    from vllm_omni_amd import kernels
+
+    with torch.inference_mode():
+        native = call()
+        with monkeypatch.context() as m:
+            m.setattr(kernels, "NATIVE_BLOCKS", False)
+            stepwise = call()
+    return native.float(), stepwise.float()
+
+
+def _single_norm(model):
+    return model.single_transformer_blocks[0].norm
+
+
+def test_hook_and_replaced_norm_of_a_flux_single_block(gpu, monkeypatch):
+    from vllm_omni_amd.blocks.flux import AdaLayerNormZeroSingle
+
+    class Scaled(AdaLayerNormZeroSingle):
+        def forward(self, x, emb=None, mod=None):
+            n, gate = super().forward(x, emb, mod)
+            return 3 * n, gate
+
+    model, call = _flux(gpu, torch.bfloat16, 64, False)
+    plain, _ = _both(monkeypatch, call)
+    seen = []
+    handle = _single_norm(model).register_forward_hook(lambda *a: seen.append(1))
+    with torch.inference_mode():
+        call()
+        handle.remove()
+
+        class Count(ModelHook):
+            def pre_forward(self, module, *args, **kwargs):
+                seen.append(2)
+                return args, kwargs
+
+        HookRegistry.get_or_create(_single_norm(model)).register_hook("count", Count())
+        call()
+    assert seen == [1, 2]
+    new = Scaled(256).to(gpu).to(torch.bfloat16)
+    new.load_state_dict({k: v for k, v in _single_norm(model).state_dict().items()})
+    model.single_transformer_blocks[0].norm = new
+    native, stepwise = _both(monkeypatch, call)
+    torch.testing.assert_close(native, stepwise, atol=2e-2, rtol=2e-2)
+    assert (native - plain).norm() > 2 * (native - stepwise).norm()
+
+
+def _attention_scale(model, block):
+    block.attn.attn.attention.softmax_scale *= 4
+
+
+def _qk_ref_rounding(model, block):
+    block.attn.ref_rounding = True
+
+
+def _unfused_mlp(model, block):
+    (block.img_mlp if hasattr(block, "img_mlp") else block.ff).net[0].fused = False
+
+
+@pytest.mark.parametrize("change", [_attention_scale, _qk_ref_rounding, _unfused_mlp])
+@pytest.mark.parametrize("make", [_qwen, _flux])
+def test_switches_on_submodules_are_read(gpu, monkeypatch, make, change):
+    """A switch set on one submodule sends its block to Python (the same bits as without the native path); a scale set on
+    the attention's backend object is the one that the native block uses."""
+    model, call = make(gpu, torch.bfloat16, 64, False)
+    out = []
+    model.transformer_blocks[-1].register_forward_hook(lambda m, a, result: out.append(torch.cat(result, dim=1).float()))
+    _both(monkeypatch, call)
+    for block in model.transformer_blocks:
+        change(model, block)
+    _both(monkeypatch, call)
+    plain, _, native, stepwise = out
+    if change is _attention_scale:
+        torch.testing.assert_close(native, stepwise, atol=2e-2, rtol=2e-2)
+        assert (native - plain).norm() > 2 * (native - stepwise).norm()
+    else:
+        assert torch.equal(native, stepwise)

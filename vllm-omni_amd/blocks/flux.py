@@ -549,4 +549,4 @@ class FluxTransformer2DModel(nn.Module):
                 p.copy_(weights[k].to(device=p.device, dtype=p.dtype))
 
 
-kernels.native_classes(FluxAttention=FluxAttention)
+kernels.native_classes(FluxAttention=FluxAttention, AdaLayerNormZeroSingle=AdaLayerNormZeroSingle)

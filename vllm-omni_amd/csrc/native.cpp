@@ -9,7 +9,8 @@
 //   * one per transformer block: the block's launches one after the other with raw addresses, its intermediate
 //     tensors carved out of ONE allocation, weights looked up in the modules' own parameter dictionaries on every
 //     call (so replaced or reloaded parameters are seen). A module tree that is not the plain one (a replaced
-//     projection, a hook on it) makes the function return None and the Python block runs.
+//     submodule, a hook on one that the Python block would call, a switch set on one) makes the function return None
+//     and the Python block runs.
 //
 // What it is for: a block makes about 14 launches. Through ctypes, with the tensor views and checks in Python, each
 // cost 20-35 us of host time, so every problem whose kernels take less than that (up to 512 x 512 pixels, a whole
@@ -741,11 +742,12 @@ PyObject* py_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
 // Reading a module tree. Everything below works on borrowed references.
 struct Names {
   PyObject *modules, *parameters, *fwd_hooks, *pre_hooks, *forward, *weight, *bias, *eps, *elementwise_affine, *ref_rounding, *attention,
-      *softmax_scale;
+      *softmax_scale, *fused, *forward_hip, *kernel_takes_layer;
 };
 Names g_name;
 PyTypeObject *g_linear_type, *g_rmsnorm_type, *g_rownorm_type, *g_adaln_type, *g_attention_type, *g_attention_impl_type,
-    *g_feed_forward_type, *g_gelu_type, *g_wan_ffn_type, *g_qwen_attention_type, *g_flux_attention_type, *g_wan_self_type, *g_wan_cross_type;
+    *g_feed_forward_type, *g_gelu_type, *g_wan_ffn_type, *g_qwen_attention_type, *g_flux_attention_type, *g_flux_single_norm_type,
+    *g_wan_self_type, *g_wan_cross_type;
 
 PyObject* instance_dict(PyObject* m) {
   PyObject** d = m ? _PyObject_GetDictPtr(m) : nullptr;
@@ -767,6 +769,15 @@ PyObject* plain_module(PyObject* m, PyTypeObject* type) {
 PyObject* child(PyObject* d, const char* name) {
   PyObject* mods = item(d, g_name.modules);
   return mods && PyDict_Check(mods) ? PyDict_GetItemString(mods, name) : nullptr;
+}
+bool is_true(PyObject* d, PyObject* name) { return item(d, name) == Py_True; }
+bool is_false(PyObject* d, PyObject* name) { return item(d, name) == Py_False; }
+// the float attribute `name` of a module's instance dict
+bool float_attr(PyObject* d, PyObject* name, double* v) {
+  PyObject* o = item(d, name);
+  if (!o || !PyFloat_Check(o)) return false;
+  *v = PyFloat_AS_DOUBLE(o);
+  return true;
 }
 const Tensor* parameter(PyObject* d, PyObject* name) {
   PyObject* p = item(item(d, g_name.parameters), name);
@@ -808,20 +819,26 @@ struct BlockCall {
     *out = w->data_ptr();
     return true;
   }
+  // projection with GELU(tanh) in its epilogue
+  bool gelu_projection(PyObject* m, Lin* up) const {
+    PyObject* d = plain_module(m, g_gelu_type);
+    return d && is_true(d, g_name.fused) && linear(child(d, "proj"), up);
+  }
   // gelu(tanh) projection and plain down-projection of a feed-forward
   bool feed_forward(PyObject* ff, Lin* up, Lin* down) const {
     PyObject* d = plain_module(ff, g_feed_forward_type);
-    PyObject* net = d ? child(d, "net") : nullptr;
+    PyObject* net = d && is_true(d, g_name.fused) ? child(d, "net") : nullptr;
     PyObject* nd = net ? instance_dict(net) : nullptr;
-    PyObject* act = nd ? plain_module(child(nd, "0"), g_gelu_type) : nullptr;
-    return act && linear(child(act, "proj"), up) && linear(child(nd, "2"), down);
+    return nd && gelu_projection(child(nd, "0"), up) && linear(child(nd, "2"), down);
   }
+  // an Attention layer whose backend object runs the kernel with its own scale
   bool attention(PyObject* m, double* scale) const {
     PyObject* d = plain_module(m, g_attention_type);
-    PyObject *impl = d ? item(d, g_name.attention) : nullptr, *s = d ? item(d, g_name.softmax_scale) : nullptr;
-    if (!impl || Py_TYPE(impl) != g_attention_impl_type || !s || !PyFloat_Check(s)) return false;
-    *scale = PyFloat_AS_DOUBLE(s);
-    return true;
+    PyObject* impl = d ? item(d, g_name.attention) : nullptr;
+    if (!impl || Py_TYPE(impl) != g_attention_impl_type) return false;
+    PyObject* id = instance_dict(impl);
+    return id && item(id, g_name.forward) == nullptr && item(id, g_name.forward_hip) == nullptr && is_true(id, g_name.kernel_takes_layer) &&
+           float_attr(id, g_name.softmax_scale, scale);
   }
 
   void check(int status) { if (rc == 0) rc = status; }
@@ -1125,15 +1142,6 @@ bool run_dual(BlockCall& c, const DualBlock& k, const Tensor& img, const Tensor&
   return true;
 }
 
-// the float attribute `name` of a module's instance dict
-bool float_attr(PyObject* d, PyObject* name, double* v) {
-  PyObject* o = item(d, name);
-  if (!o || !PyFloat_Check(o)) return false;
-  *v = PyFloat_AS_DOUBLE(o);
-  return true;
-}
-bool is_false(PyObject* d, PyObject* name) { return item(d, name) == Py_False; }
-
 // an AdaLayerNorm without affine and reference rounding
 bool plain_adaln(PyObject* m, double* eps) {
   PyObject* d = plain_module(m, g_adaln_type);
@@ -1143,7 +1151,7 @@ bool plain_adaln(PyObject* m, double* eps) {
 // to_qkv, add_kv_proj, the four head norms, the attention layer
 bool dual_attention(const BlockCall& c, PyObject* attn, PyTypeObject* type, DualBlock* k) {
   PyObject* d = plain_module(attn, type);
-  if (!d || !c.linear(child(d, "to_qkv"), &k->qkv[0]) || !c.linear(child(d, "add_kv_proj"), &k->qkv[1]) ||
+  if (!d || !is_false(d, g_name.ref_rounding) || (type == g_qwen_attention_type && !is_true(d, g_name.fused)) || !c.linear(child(d, "to_qkv"), &k->qkv[0]) || !c.linear(child(d, "add_kv_proj"), &k->qkv[1]) ||
       !c.linear(child(d, "to_add_out"), &k->out[1]) || !c.attention(child(d, "attn"), &k->scale) || !float_attr(d, g_name.eps, &k->eps_qk))
     return false;
   const char* names[4] = {"norm_q", "norm_added_q", "norm_k", "norm_added_k"};
@@ -1247,12 +1255,12 @@ PyObject* py_flux_single_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (B > 1 && gate->stride(0) != gbias->stride(0)) return none();
   if (!f32_table(c, cos, S, cos->size(1)) || !f32_table(c, sin, S, cos->size(1))) return none();
   PyObject* d = instance_dict(a[0]);
-  PyObject *norm = d ? instance_dict(child(d, "norm")) : nullptr, *attn = d ? plain_module(child(d, "attn"), g_flux_attention_type) : nullptr;
+  PyObject *norm = d ? plain_module(child(d, "norm"), g_flux_single_norm_type) : nullptr, *attn = d ? plain_module(child(d, "attn"), g_flux_attention_type) : nullptr;
   Lin qkv, up, down;
   double eps, eps_qk, scale;
   const void *wq, *wk;
   int w_dtype = -1;
-  if (!norm || !attn || !float_attr(norm, g_name.eps, &eps) || !float_attr(attn, g_name.eps, &eps_qk) || !c.linear(child(attn, "to_qkv"), &qkv) ||
+  if (!norm || !is_false(norm, g_name.ref_rounding) || !attn || !is_false(attn, g_name.ref_rounding) || !float_attr(norm, g_name.eps, &eps) || !float_attr(attn, g_name.eps, &eps_qk) || !c.linear(child(attn, "to_qkv"), &qkv) ||
       !c.attention(child(attn, "attn"), &scale) || !c.norm_weight(child(attn, "norm_q"), g_rmsnorm_type, D, &wq, &w_dtype) ||
       !c.norm_weight(child(attn, "norm_k"), g_rmsnorm_type, D, &wk, &w_dtype) || !c.linear(child(d, "proj_mlp"), &up) ||
       !c.linear(child(d, "proj_out"), &down))
@@ -1349,14 +1357,13 @@ PyObject* py_wan_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
   PyObject *a1 = d ? plain_module(child(d, "attn1"), g_wan_self_type) : nullptr, *a2 = d ? plain_module(child(d, "attn2"), g_wan_cross_type) : nullptr,
            *ffn = d ? plain_module(child(d, "ffn"), g_wan_ffn_type) : nullptr;
   if (!a1 || !a2 || !ffn) return none();
-  PyObject* act = plain_module(child(ffn, "net_0"), g_gelu_type);
   Lin qkv, out1, q2, k2, v2, out2, up, down;
   double eps, scale1, scale2, eps_n[4];
   const void* nw[4];
   int w_dtype = -1;
-  if (!act || !float_attr(d, g_name.eps, &eps) || !c.linear(child(a1, "to_qkv"), &qkv) || !c.linear(child(a1, "to_out"), &out1) ||
+  if (!float_attr(d, g_name.eps, &eps) || !c.linear(child(a1, "to_qkv"), &qkv) || !c.linear(child(a1, "to_out"), &out1) ||
       !c.linear(child(a2, "to_q"), &q2) || !c.linear(child(a2, "to_k"), &k2) || !c.linear(child(a2, "to_v"), &v2) ||
-      !c.linear(child(a2, "to_out"), &out2) || !c.linear(child(act, "proj"), &up) || !c.linear(child(ffn, "net_2"), &down) ||
+      !c.linear(child(a2, "to_out"), &out2) || !c.gelu_projection(child(ffn, "net_0"), &up) || !c.linear(child(ffn, "net_2"), &down) ||
       !c.attention(child(a1, "attn"), &scale1) || !c.attention(child(a2, "attn"), &scale2))
     return none();
   if (PyObject* mods2 = item(a2, g_name.modules); mods2 && PyDict_GetItemString(mods2, "add_k_proj") != nullptr &&
@@ -1487,7 +1494,8 @@ PyObject* py_classes(PyObject*, PyObject* const* a, Py_ssize_t n) {
       {"Linear", &g_linear_type}, {"RMSNorm", &g_rmsnorm_type}, {"DistributedRMSNorm", &g_rownorm_type}, {"AdaLayerNorm", &g_adaln_type},
       {"Attention", &g_attention_type}, {"AttentionImpl", &g_attention_impl_type}, {"FeedForward", &g_feed_forward_type},
       {"ApproxGELU", &g_gelu_type}, {"WanFeedForward", &g_wan_ffn_type}, {"QwenImageCrossAttention", &g_qwen_attention_type},
-      {"FluxAttention", &g_flux_attention_type}, {"WanSelfAttention", &g_wan_self_type}, {"WanCrossAttention", &g_wan_cross_type}};
+      {"FluxAttention", &g_flux_attention_type},
+      {"AdaLayerNormZeroSingle", &g_flux_single_norm_type}, {"WanSelfAttention", &g_wan_self_type}, {"WanCrossAttention", &g_wan_cross_type}};
   for (const auto& w : want) {
     PyObject* t = PyDict_GetItemString(a[0], w.name);
     if (t == nullptr) continue;
@@ -1503,7 +1511,8 @@ bool intern_names() {
       {"_modules", &g_name.modules}, {"_parameters", &g_name.parameters}, {"_forward_hooks", &g_name.fwd_hooks},
       {"_forward_pre_hooks", &g_name.pre_hooks}, {"forward", &g_name.forward}, {"weight", &g_name.weight}, {"bias", &g_name.bias},
       {"eps", &g_name.eps}, {"elementwise_affine", &g_name.elementwise_affine}, {"ref_rounding", &g_name.ref_rounding},
-      {"attention", &g_name.attention}, {"softmax_scale", &g_name.softmax_scale}};
+      {"attention", &g_name.attention}, {"softmax_scale", &g_name.softmax_scale}, {"fused", &g_name.fused},
+      {"forward_hip", &g_name.forward_hip}, {"kernel_takes_layer", &g_name.kernel_takes_layer}};
   for (const auto& w : want)
     if ((*w.slot = PyUnicode_InternFromString(w.s)) == nullptr) return false;
   return true;
