@@ -88,3 +88,61 @@ def test_switches_on_submodules_are_read(gpu, monkeypatch, make, change):
         assert (native - plain).norm() > 2 * (native - stepwise).norm()
     else:
         assert torch.equal(native, stepwise)
+
+
+def test_position_embedders_are_called_unless_plain(gpu):
+    """A subclass with its own positions is used, hooks run, and a module with nothing but ``forward`` is enough."""
+    from vllm_omni_amd.blocks.flux import FluxPosEmbed
+    from vllm_omni_amd.blocks.qwen_image import QwenEmbedRope
+
+    class HalfFlux(FluxPosEmbed):
+        def forward(self, ids):
+            return super().forward(ids * 0.5)
+
+    class OnlyForward(torch.nn.Module):
+        def __init__(self, inner):
+            super().__init__()
+            self.inner = inner
+
+        def forward(self, *args, **kwargs):
+            return tuple(self.inner(*args, **kwargs))
+
+    class NearerText(QwenEmbedRope):
+        def forward(self, video_fhw, txt_seq_lens, device):
+            vid, txt = super().forward(video_fhw, txt_seq_lens, device)
+            return vid, txt * txt
+
+    for make, cls, own in ((_flux, HalfFlux, lambda: HalfFlux(10000, [8, 28, 28])),
+                           (_qwen, NearerText, lambda: NearerText(10000, [8, 28, 28]))):
+        model, call = make(gpu, torch.bfloat16, 64, False)
+        seen = []
+        with torch.inference_mode():
+            plain = call()
+            handle = model.pos_embed.register_forward_hook(lambda *a: seen.append(1))
+            hooked = call()
+            handle.remove()
+            model.pos_embed = OnlyForward(model.pos_embed)
+            wrapped = call()
+            model.pos_embed = own()
+            changed = call()
+        assert seen == [1]
+        # (the float32 tables are made another way: from float64 or from complex ones)
+        torch.testing.assert_close(hooked.float(), plain.float(), atol=2e-2, rtol=2e-2)
+        assert torch.equal(wrapped, hooked)
+        assert (changed - plain).float().norm() > 2 * (hooked - plain).float().norm() and not torch.equal(changed, plain)
+
+
+def test_wrapped_time_embedding_gets_the_scaled_timestep(gpu):
+    model, call = _flux(gpu, torch.bfloat16, 64, False)
+    inner, seen = model.time_text_embed.forward, []
+
+    def forward(timestep, guidance, pooled):   # an offloading wrapper of the documented signature
+        seen.append(timestep.item())
+        return inner(timestep, guidance, pooled)
+
+    with torch.inference_mode():
+        plain = call()
+        model.time_text_embed.forward = forward
+        wrapped = call()
+    assert seen == [torch.tensor(0.3).bfloat16().mul(1000).item()]
+    assert torch.equal(plain, wrapped)

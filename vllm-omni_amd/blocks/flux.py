@@ -47,8 +47,11 @@ class FluxRotary:
 
     @classmethod
     def of_ids(cls, pos_embed: FluxPosEmbed, txt_ids: torch.Tensor, img_ids: torch.Tensor) -> FluxRotary:
-        """From position ids: the float32 tables in one launch, the float64 ones only when somebody asks for them."""
-        done = kernels.rope_tables(txt_ids, img_ids, tuple(pos_embed.axes_dim), pos_embed.theta)
+        """From position ids: the float32 tables in one launch, the float64 ones only when somebody asks for them. A
+        ``pos_embed`` of another class, or with hooks, is called."""
+        done = None
+        if kernels.plain_module(pos_embed, FluxPosEmbed):
+            done = kernels.rope_tables(txt_ids, img_ids, tuple(pos_embed.axes_dim), pos_embed.theta)
         if done is None:
             return cls(*pos_embed(torch.cat((txt_ids, img_ids), dim=0)))
         r = cls.__new__(cls)
@@ -424,7 +427,7 @@ class FluxTransformer2DModel(nn.Module):
     def prepare(self, hidden_states, encoder_hidden_states, pooled_projections, timestep, img_ids, txt_ids,
                 guidance=None):
         img = kernels.project(self.x_embedder, hidden_states)
-        if type(self.time_text_embed) is CombinedTimestepGuidanceTextProjEmbeddings and pooled_projections.dtype == img.dtype:
+        if kernels.plain_module(self.time_text_embed, CombinedTimestepGuidanceTextProjEmbeddings) and pooled_projections.dtype == img.dtype:
             if guidance is not None:
                 guidance = guidance.to(device=img.device)
             temb = self.time_text_embed(timestep.to(device=img.device), guidance, pooled_projections, pre=1000.0)

@@ -554,7 +554,9 @@ class QwenImageTransformer2DModel(nn.Module):
         temb = self.time_text_embed(timestep, img, additional_t_cond)
         if txt_seq_lens is None:
             txt_seq_lens = [encoder_hidden_states.shape[1]]
-        return img, txt, temb, self.pos_embed.tables(img_shapes, txt_seq_lens, device=img.device)
+        if kernels.plain_module(self.pos_embed, QwenEmbedRope, QwenEmbedLayer3DRope):
+            return img, txt, temb, self.pos_embed.tables(img_shapes, txt_seq_lens, device=img.device)
+        return img, txt, temb, RotaryTables(*self.pos_embed(img_shapes, txt_seq_lens, device=img.device))
 
     def modulate_index(self, img_shapes, device) -> torch.Tensor | None:
         """[B, S_img] int32 per-token conditioning choice of the editing variant: 0 (real timestep) for the

@@ -65,6 +65,13 @@ def native_blocks() -> bool:
             and not _global_hooks._global_forward_hooks and not _global_hooks._global_forward_pre_hooks)
 
 
+def plain_module(m: torch.nn.Module, *classes: type) -> bool:
+    """Whether what a call of ``m`` does is known from its class alone: exactly one of ``classes``, with no hook on it or on
+    all modules, and no ``forward`` of its own (offloading wrappers and this package's hook registry put one there)."""
+    return (type(m) in classes and not m._forward_hooks and not m._forward_pre_hooks and "forward" not in m.__dict__
+            and not _global_hooks._global_forward_hooks and not _global_hooks._global_forward_pre_hooks)
+
+
 def linear_engine_flags() -> int:
     """The engine bits that ``set_linear_engine`` chose, for the native block functions."""
     return _LINEAR_ENGINE_FLAGS
