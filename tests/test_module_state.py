@@ -72,3 +72,66 @@ def test_wan_rows_follow_the_parameters(how):
         for w, b in (model.norm2_affines()[1], block._norm2_affine()):
             assert torch.equal(w, block.norm2.weight.float()) and torch.equal(b, block.norm2.bias.float())
         assert torch.equal(block._table(), block.scale_shift_table[0].float())
+
+
+def _qwen_stem():
+    from vllm_omni_amd.blocks.qwen_image import QwenImageTransformer2DModel
+
+    model = QwenImageTransformer2DModel(num_layers=1, attention_head_dim=64, num_attention_heads=1, joint_attention_dim=64,
+                                        axes_dims_rope=(8, 28, 28))
+    return model, model.transformer_blocks[0].img_mod[1], (None, None, None, None, None, None)
+
+
+def _flux_stem():
+    from vllm_omni_amd.blocks.flux import FluxTransformer2DModel
+
+    model = FluxTransformer2DModel(num_layers=1, num_single_layers=0, attention_head_dim=64, num_attention_heads=1,
+                                   joint_attention_dim=64, pooled_projection_dim=8, axes_dims_rope=(8, 28, 28))
+    return model, model.transformer_blocks[0].norm1.linear, (None,) * 6
+
+
+def _decision_rows(monkeypatch, model, args):
+    """The shift and scale that the cache decision is made with, on a given stem output."""
+    from vllm_omni_amd import kernels
+    from vllm_omni_amd.cache.teacache.extractors import get_extractor
+
+    img, temb = torch.zeros(2, 3, 64), torch.linspace(-1, 1, 128).view(2, 64)
+    monkeypatch.setattr(model, "prepare", lambda *a, **k: (img, None, temb, None), raising=False)
+    monkeypatch.setattr(kernels, "silu", torch.nn.functional.silu)
+    rows = []
+    monkeypatch.setattr(kernels, "adaln_modulate", lambda x, shift, scale, **k: rows.extend((shift, scale)) or x)
+    with torch.no_grad():
+        get_extractor(type(model).__name__)(model, *args)
+    return torch.cat(rows, dim=-1)
+
+
+@pytest.mark.parametrize("make,how", [(m, h) for m in (_qwen_stem, _flux_stem) for h in ("plain", "hook", "global hook", "own forward")]
+                         + [(_qwen_stem, "activation hook")])
+def test_cache_decision_projection_is_called_unless_plain(monkeypatch, make, how):
+    model, lin, args = make()
+    _random_(model)
+    want = lin(torch.nn.functional.silu(torch.linspace(-1, 1, 128).view(2, 64)))[:, :128].detach()
+    seen, handle = [], None
+    if how == "hook":
+        lin.register_forward_hook(lambda *a: seen.append(1))
+    elif how == "global hook":
+        handle = torch.nn.modules.module.register_module_forward_hook(lambda m, *a: seen.append(1) if m is lin else None)
+    elif how == "own forward":   # as an offloading wrapper puts it there: the weight is elsewhere between calls
+        weight, inner = lin.weight.data, lin.forward
+
+        def forward(x):
+            seen.append(1)
+            lin.weight.data = weight
+            return inner(x)
+
+        lin.forward = forward
+        lin.weight.data = torch.empty(0, 64)
+    elif how == "activation hook":
+        model.transformer_blocks[0].img_mod[0].register_forward_hook(lambda *a: seen.append(1))
+    try:
+        got = _decision_rows(monkeypatch, model, args)
+    finally:
+        if handle is not None:
+            handle.remove()
+    assert seen == ([] if how == "plain" else [1])
+    torch.testing.assert_close(got, want)

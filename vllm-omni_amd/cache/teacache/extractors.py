@@ -11,6 +11,7 @@ import torch
 import torch.nn as nn
 
 from ... import kernels
+from ...blocks.qwen_image import SiLU
 
 
 @dataclass
@@ -53,13 +54,13 @@ class CacheContext:
                              f"hidden_states on {self.hidden_states.device}")
 
 
-def _first_rows(lin: nn.Module, temb: torch.Tensor, n: int) -> torch.Tensor:
+def _first_rows(lin: nn.Module, temb: torch.Tensor, n: int) -> torch.Tensor | None:
     """The first ``n`` outputs of ``lin(silu(temb))``: the decision needs one shift and one scale of the six parameters, so a
-    plain Linear's other weight rows are not read here (61 us for all of Flux's through the library). A Linear with hooks or of
-    another class is called whole."""
-    if type(lin) is nn.Linear and not lin._forward_hooks and not lin._forward_pre_hooks and not torch.is_grad_enabled():
-        return kernels.linear_few(temb, lin.weight[:n], lin.bias[:n] if lin.bias is not None else None, silu_input=True)
-    return lin(kernels.silu(temb))[..., :n]
+    plain Linear's other weight rows are not read here (61 us for all of Flux's through the library). None for a Linear with
+    hooks, with a forward of its own or of another class: the caller calls it whole."""
+    if not kernels.plain_module(lin, nn.Linear) or torch.is_grad_enabled():
+        return None
+    return kernels.linear_few(temb, lin.weight[:n], lin.bias[:n] if lin.bias is not None else None, silu_input=True)
 
 
 def extract_qwen_context(module: nn.Module, hidden_states: torch.Tensor,
@@ -80,7 +81,10 @@ def extract_qwen_context(module: nn.Module, hidden_states: torch.Tensor,
     img, txt, temb, rotary = module.prepare(hidden_states, encoder_hidden_states, timestep, img_shapes, txt_seq_lens,
                                             additional_t_cond)
     block0 = module.transformer_blocks[0]
-    shift, scale = _first_rows(block0.img_mod[1], temb, 2 * img.shape[-1]).chunk(2, dim=-1)
+    mod, n, rows = block0.img_mod, 2 * img.shape[-1], None
+    if kernels.plain_module(mod, nn.Sequential) and len(mod) == 2 and kernels.plain_module(mod[0], SiLU):
+        rows = _first_rows(mod[1], temb, n)
+    shift, scale = (mod(temb)[..., :n] if rows is None else rows).chunk(2, dim=-1)
     # The decision tensor is always rounded where the reference's torch ops round (one 50 MB elementwise pass
     # per step), whatever rounding the block stack itself runs with: skip/compute decisions then do not depend
     # on whether the model was built with fused GEMM epilogues.
@@ -123,7 +127,9 @@ def extract_flux_context(module: nn.Module, hidden_states: torch.Tensor,
     img, txt, temb, rotary = module.prepare(hidden_states, encoder_hidden_states, pooled_projections, timestep,
                                             img_ids, txt_ids, guidance)
     norm1 = module.transformer_blocks[0].norm1
-    shift, scale = _first_rows(norm1.linear, temb, 2 * img.shape[-1]).chunk(2, dim=-1)
+    n = 2 * img.shape[-1]
+    rows = _first_rows(norm1.linear, temb, n)
+    shift, scale = (norm1.linear(kernels.silu(temb))[..., :n] if rows is None else rows).chunk(2, dim=-1)
     # reference rounding for the decision tensor, whatever the blocks run with (see extract_qwen_context)
     modulated = kernels.adaln_modulate(img, shift, scale, eps=norm1.eps, ref_rounding=True)
     return_dict = kwargs.get("return_dict", True)
