@@ -135,3 +135,37 @@ def test_cache_decision_projection_is_called_unless_plain(monkeypatch, make, how
             handle.remove()
     assert seen == ([] if how == "plain" else [1])
     torch.testing.assert_close(got, want)
+
+
+@pytest.mark.parametrize("batch", [1, 2])
+@pytest.mark.parametrize("how", ["hook", "own forward", "replaced"])
+def test_wan_time_embedder_is_called(monkeypatch, how, batch):
+    from vllm_omni_amd import kernels
+    from vllm_omni_amd.blocks.wan import WanTimeTextImageEmbedding
+
+    monkeypatch.setattr(kernels, "silu", torch.nn.functional.silu)
+    monkeypatch.setattr(kernels, "gelu_tanh", lambda x, out=None: torch.nn.functional.gelu(x, approximate="tanh"))
+    emb = _random_(WanTimeTextImageEmbedding(64, 16, 6 * 64, 32))
+    t, text = torch.full((batch,), 500.0), torch.randn(batch, 3, 32)
+    seen = []
+    with torch.no_grad():
+        plain = emb(t, text)
+        if how == "hook":
+            emb.time_embedder.register_forward_hook(lambda m, a, out: seen.append(1) or 2 * out)
+        elif how == "own forward":
+            inner = emb.time_embedder.forward
+            emb.time_embedder.forward = lambda x: seen.append(1) or 2 * inner(x)
+        else:
+            class Twice(torch.nn.Module):
+                def __init__(self, mlp):
+                    super().__init__()
+                    self.linear_1, self.linear_2 = mlp.linear_1, mlp.linear_2
+
+                def forward(self, x):
+                    seen.append(1)
+                    return 2 * self.linear_2(torch.nn.functional.silu(self.linear_1(x)))
+
+            emb.time_embedder = Twice(emb.time_embedder)
+        changed = emb(t, text)
+    assert seen == [1]
+    torch.testing.assert_close(changed[0], 2 * plain[0])

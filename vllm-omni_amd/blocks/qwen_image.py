@@ -429,7 +429,10 @@ class TimestepEmbedding(nn.Module):
         self.linear_1 = nn.Linear(in_channels, time_embed_dim)
         self.linear_2 = nn.Linear(time_embed_dim, time_embed_dim)
 
-    def forward(self, x: torch.Tensor) -> torch.Tensor:
+    def forward(self, x: torch.Tensor, library: bool = False) -> torch.Tensor:
+        """``library``: both projections as torch's linear, whatever kernel would take them."""
+        if library:
+            return self.linear_2(kernels.silu(self.linear_1(x)))
         return kernels.project(self.linear_2, kernels.project(self.linear_1, x), silu_input=True)
 
 

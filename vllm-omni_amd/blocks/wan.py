@@ -422,7 +422,8 @@ class WanTimeTextImageEmbedding(nn.Module):
             temb = mlp(t).type_as(encoder_hidden_states)
             timestep_proj = kernels.project(self.time_proj, temb, silu_input=True)
         else:  # a CFG pair keeps the library's order of summation: guidance multiplies what another one rounds differently
-            temb = mlp.linear_2(kernels.silu(mlp.linear_1(t))).type_as(encoder_hidden_states)
+            known = type(mlp) is TimestepEmbedding and "forward" not in mlp.__dict__   # (hooks run either way)
+            temb = (mlp(t, library=True) if known else mlp(t)).type_as(encoder_hidden_states)
             timestep_proj = self.time_proj(kernels.silu(temb))
         image = None
         if encoder_hidden_states_image is not None:
