@@ -169,3 +169,20 @@ def test_wan_time_embedder_is_called(monkeypatch, how, batch):
         changed = emb(t, text)
     assert seen == [1]
     torch.testing.assert_close(changed[0], 2 * plain[0])
+
+
+@pytest.mark.parametrize("where", ["class", "instance"])
+def test_a_pipelines_own_cfg_normalisation_is_used(where):
+    from vllm_omni_amd.denoise import CFGParallelMixin
+
+    class Pipe(CFGParallelMixin):
+        pass
+
+    pipe = Pipe()
+    if where == "class":
+        Pipe.cfg_normalize_function = lambda self, pred, comb: comb * 0 + 7
+    else:
+        pipe.cfg_normalize_function = lambda pred, comb: comb * 0 + 7
+    pos, neg = torch.randn(1, 3, 8), torch.randn(1, 3, 8)
+    assert torch.equal(pipe.combine_cfg_noise(pos, neg, 4.0, True), torch.full((1, 3, 8), 7.0))
+    torch.testing.assert_close(pipe.combine_cfg_noise(pos, neg, 4.0, False), neg + 4.0 * (pos - neg))

@@ -240,7 +240,8 @@ class CFGParallelMixin:
 
     def combine_cfg_noise(self, noise_pred: torch.Tensor, neg_noise_pred: torch.Tensor, true_cfg_scale: float,
                           cfg_normalize: bool = False) -> torch.Tensor:
-        if type(self).cfg_normalize_function is CFGParallelMixin.cfg_normalize_function:
+        own = type(self).cfg_normalize_function is not CFGParallelMixin.cfg_normalize_function or "cfg_normalize_function" in vars(self)
+        if not own:
             return combine_cfg_noise(noise_pred, neg_noise_pred, true_cfg_scale, cfg_normalize)
         comb_pred = neg_noise_pred + true_cfg_scale * (noise_pred - neg_noise_pred)
         return self.cfg_normalize_function(noise_pred, comb_pred) if cfg_normalize else comb_pred
