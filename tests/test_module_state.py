@@ -186,17 +186,3 @@ def test_a_pipelines_own_cfg_normalisation_is_used(where):
     pos, neg = torch.randn(1, 3, 8), torch.randn(1, 3, 8)
     assert torch.equal(pipe.combine_cfg_noise(pos, neg, 4.0, True), torch.full((1, 3, 8), 7.0))
     torch.testing.assert_close(pipe.combine_cfg_noise(pos, neg, 4.0, False), neg + 4.0 * (pos - neg))
-
-
-def test_joint_key_mask_takes_masks_of_the_streams_shapes_only():
-    from vllm_omni_amd.blocks.qwen_image import joint_key_mask
-
-    cpu = torch.device("cpu")
-    txt = torch.tensor([[2, 0, 1], [0, 1, 1]])
-    got = joint_key_mask(txt, None, 2, 3, 2, cpu)
-    assert torch.equal(got, torch.tensor([[True, False, True, True, True], [False, True, True, True, True]]))
-    assert torch.equal(joint_key_mask(None, txt.bool(), 2, 1, 3, cpu)[:, 1:], txt.bool())
-    assert joint_key_mask(None, None, 2, 3, 2, cpu) is None
-    for bad in (txt[:1], txt[:, :1], txt[0], txt[:, :, None]):   # what would broadcast is refused
-        with pytest.raises(ValueError):
-            joint_key_mask(bad, None, 2, 3, 2, cpu)

@@ -246,11 +246,12 @@ def joint_key_mask(txt_mask, img_mask, B: int, S_txt: int, S_img: int, device) -
     """[B, S_txt + S_img] boolean key mask of the joint sequence from the two streams' masks (None = all true)."""
     if txt_mask is None and img_mask is None:
         return None
-    parts = [m.bool() if m is not None else torch.ones((B, n), dtype=torch.bool, device=device)
-             for m, n in ((txt_mask, S_txt), (img_mask, S_img))]
-    if any(tuple(m.shape) != (B, n) for m, n in zip(parts, (S_txt, S_img))):
-        raise ValueError(f"masks must be {(B, S_txt)} and {(B, S_img)}, got {[tuple(m.shape) for m in parts]}")
-    return torch.cat(parts, dim=1)
+    out = torch.ones((B, S_txt + S_img), dtype=torch.bool, device=device)
+    if txt_mask is not None:
+        out[:, :S_txt] = txt_mask
+    if img_mask is not None:
+        out[:, S_txt:] = img_mask
+    return out
 
 
 class QwenImageCrossAttention(nn.Module):
