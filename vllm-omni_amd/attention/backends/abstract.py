@@ -54,8 +54,8 @@ class AttentionMetadata:
     ``value_tail`` (not in the reference): the ``value`` argument then holds only the rows of the first
     keys and this tensor the rest, so a caller with the values of two streams in two buffers does not
     have to concatenate them.
-    ``attn_mask_checked`` (not in the reference): the caller has looked at ``attn_mask`` itself. Kept for callers that
-    set it; the backend tests no mask for being all true any more (that test synchronised, the kernel needs none)."""
+    ``attn_mask_checked`` (not in the reference): accepted and not read. It once told the backend to skip a test for an
+    all-true mask, which synchronised; there is no such test any more."""
 
     attn_mask: torch.Tensor | None = None
     joint_attn_mask: torch.Tensor | None = None

@@ -62,8 +62,8 @@ class HipFlashAttentionImpl(AttentionImpl):
     def forward_hip(self, query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
                     attn_metadata: AttentionMetadata | None = None) -> torch.Tensor:
         """q [B,Sq,H,D], k/v [B,Sk,Hkv,D] -> [B,Sq,H,D]. A [B,Sk] ``attn_mask`` excludes keys. (The reference drops an
-        all-true mask, flash_attn.py:80-84. That test synchronises; the kernel gives the same values for one and runs
-        tiles without an excluded key like those of a launch without a mask.) With
+        all-true mask, flash_attn.py:80-84. That test synchronises; the kernel gives the same bits for one, and runs tiles
+        without an excluded key like those of a launch without a mask.) With
         ``attn_metadata.output_split`` = s the result is the pair (out[:, :s], out[:, s:]), both dense;
         with ``attn_metadata.value_tail`` the values are [value; value_tail] along the keys, read in place."""
         mask = attn_metadata.attn_mask if attn_metadata is not None else None

@@ -20,6 +20,16 @@
 // barrier per tile - two in the anti-phase form of 8 wavefronts, see NW below -, XCD-aware workgroup order)
 // is as in attn_fwd_pipe_kernel.
 //
+// Key mask. Before the first scores each wavefront turns its share of the mask row into one 64-bit word per key tile (a
+// ballot over the tile's 64 bytes; keys past Sk are zero bits) in LDS. A tile whose word is all ones then runs like a tile of
+// a launch without a mask, any other one selects its scores by the word's bits, wave-uniform both. Read as bytes from
+// global memory at every tile, 32 loads, clamps and selects per lane, a mask cost 33 to 84 % whatever was in it. us, bf16,
+// no mask / all-true mask, bytes / all-true mask, words:
+//   B=2 S=4352 H=24 D=128  450 / 735 / 461      B=1 S=4608 H=24 D=128  256 / 471 / 263
+//   B=2 S=592 H=24 D=128   18.8 / 26.8 / 18.9   B=2 S=4352 H=24 D=64   284 / 505 / 292
+// (and 499 / 293 / 20.6 / 336 with a random mask, where every tile is mixed).
+// Past kMaskWords tiles, and in the persistent form, whose units change the batch row, the mask is read as bytes.
+//
 // Persistent form (MODE 2), a measurement aid that no default launch uses (ODIT_ATTN_PERSISTENT=1 in the
 // environment turns it on for launches of 4-wavefront workgroups, i.e. with ODIT_ATTN_WAVES=4 at head size 128). With more units than workgroup slots the launch has as many workgroups as run at
 // once, and each runs unit after unit as ONE stream of key tiles: the tile pipeline runs across the unit
@@ -85,11 +95,16 @@ typedef __attribute__((address_space(3))) void* lds_void_p;
 //         tiles [jt0, n_tiles) of unit n_full + i / key_chunks and leaves an unnormalised partial
 //         result in scratch for attn_merge_kernel.
 // MODE 2: persistent, see above.
-// Separate instantiations, so the extra bookkeeping of one cannot disturb the register allocation of another.
+// MODE 3, 4: 0 and 1 for a key mask held as words.
+// Separate instantiations, so the extra bookkeeping of one cannot disturb the register allocation of another (that of the
+// words in the launches without a mask: 452 -> 460 us at B=2 S=4352 H=24 D=128, 252 -> 262 at B=1 S=4608).
+constexpr int kMaskWords = 1024;  // 8 KB of LDS: two workgroups of D = 128 still fit a compute unit (144 of 160 KB)
+
 template <typename T, int D, int NW, int MODE>
 __global__ __launch_bounds__(NW * 64, 8 / NW) void attn_fwd_dma_kernel(const AttnParams p) {
-  constexpr bool TAIL = MODE == 1;
+  constexpr bool TAIL = MODE == 1 || MODE == 4;
   constexpr bool PERSIST = MODE == 2;
+  constexpr bool WORDS = MODE == 3 || MODE == 4;
   using M = Mma<T>;
   using frag = typename M::frag;
   constexpr int BN = 64;
@@ -122,7 +137,8 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void attn_fwd_dma_kernel(const Att
   // persistent form: the unit after the current one (-1: none, or not drawn yet)
   int next_pid = -1;
   __shared__ int next_unit_box;  // thread 0's draw, handed to the workgroup across a tile's barrier
-  if constexpr (MODE == 0) {
+  __shared__ uint64_t mask_words[WORDS ? kMaskWords : 1];  // of key tiles jt0, jt0 + 1, ...
+  if constexpr (MODE == 0 || MODE == 3) {
     pid = xcd_remap(blockIdx.x, p.n_full);
   } else if constexpr (TAIL) {  // this workgroup covers key tiles [jt0, n_tiles) of unit pid (jt0 is even)
     pid = p.n_full + part / p.key_chunks;
@@ -329,9 +345,22 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void attn_fwd_dma_kernel(const Att
       }
   };
 
-  auto mask_and_max = [&](int j, const uint8_t* mrow, f32x16_v(&s)[2]) -> float {
-    // branch-free selects: every lane rewrites all its scores, excluded ones with -inf
-    if (mrow != nullptr) {
+  // excluded scores of tile j become -inf (branch-free selects: every lane rewrites all its scores); returns the lane's maximum.
+  // w: the tile's mask word (WORDS)
+  auto mask_and_max = [&](int j, const uint8_t* mrow, uint64_t w, f32x16_v(&s)[2]) -> float {
+    if constexpr (WORDS) {
+      // (this lane's keys are 8 g + 4 hh + t of each half of the tile)
+      const uint32_t half[2] = {static_cast<uint32_t>(w) >> (4 * hh), static_cast<uint32_t>(w >> 32) >> (4 * hh)};
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+#pragma unroll
+          for (int t = 0; t < 4; ++t) {
+            const float x = s[kt][g * 4 + t];
+            s[kt][g * 4 + t] = (half[kt] & (1u << (g * 8 + t))) ? x : -INFINITY;
+          }
+    } else if (mrow != nullptr) {
 #pragma unroll
       for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
@@ -544,7 +573,9 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void attn_fwd_dma_kernel(const Att
       vlo[step % (PF + 1)] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_p)(vp));
       vhi[step % (PF + 1)] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_p)(vp + 8 * ROWB));
     };
-    const bool plain_next = has_next && mrow_n == nullptr && (jn + 1) * BN <= p.Sk;  // no exclusions in the next scores
+    bool plain_next = has_next && mrow_n == nullptr && (jn + 1) * BN <= p.Sk;  // no exclusions in the next scores
+    uint64_t word = 0;  // (the same in every lane)
+    if (WORDS && has_next) word = mask_words[WORDS ? jn - jt0 : 0];
     float mx = -INFINITY;
 #pragma unroll
     for (int st = 0; st < PF; ++st) v_fetch(st);
@@ -556,6 +587,11 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void attn_fwd_dma_kernel(const Att
       u32x4_v pb;
       pb.x = pf[kt][g2][0]; pb.y = pf[kt][g2][1]; pb.z = pf[kt][g2][2]; pb.w = pf[kt][g2][3];
       o[dt] = M::run(__builtin_bit_cast(frag, av), __builtin_bit_cast(frag, pb), o[dt]);
+      if (WORDS && st == 1) {
+        const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(word));
+        const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(word >> 32));
+        plain_next = has_next && (lo & hi) == ~0u;
+      }
       if (st == 1 && plain_next) {  // wave-uniform
         float t = s_next[0][0];
 #pragma unroll
@@ -567,7 +603,7 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void attn_fwd_dma_kernel(const Att
       __builtin_amdgcn_sched_barrier(0);  // keep the reads of step st+PF ahead of this MFMA
     }
     if (has_next && !plain_next) {
-      const float t = mask_and_max(jn, mrow_n, s_next);
+      const float t = mask_and_max(jn, mrow_n, word, s_next);
       mx = fmaxf(t, __shfl_xor(t, 32, 64));
     }
     __builtin_amdgcn_s_waitcnt(0);  // this wave's tile loads have landed in LDS
@@ -601,12 +637,31 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void attn_fwd_dma_kernel(const Att
   if (!PP || !grp1) dma_tile(krsrc, true, static_cast<uint32_t>(jt0) * k_tile_step, kKoff);
   if (!PP || grp1) dma_v(jt0, kVoff);
   if ((!PP || !grp1) && jt0 + 1 < n_tiles) dma_tile(krsrc, true, static_cast<uint32_t>(jt0 + 1) * k_tile_step, kKoff + TILEB);
+  if constexpr (WORDS) {  // behind the first tile loads; up to MB independent loads per memory round trip
+    constexpr int MB = 8;
+    for (int j0 = jt0 + __builtin_amdgcn_readfirstlane(wave); j0 < n_tiles; j0 += MB * NW) {
+      uint8_t m[MB];
+#pragma unroll
+      for (int i = 0; i < MB; ++i) {
+        const int key = (j0 + i * NW) * BN + lane;
+        if (j0 + i * NW < n_tiles) m[i] = mrow[key < p.Sk ? key : p.Sk - 1];
+      }
+#pragma unroll
+      for (int i = 0; i < MB; ++i) {
+        const int j = j0 + i * NW;
+        if (j < n_tiles) {  // (wave-uniform)
+          const uint64_t w = __ballot((j * BN + lane < p.Sk) & (m[i] != 0));
+          if (lane == 0) mask_words[j - jt0] = w;
+        }
+      }
+    }
+  }
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
   f32x16_v sa[2], sb[2];
   qk_plain(Kb, sa);
   {
-    const float t = mask_and_max(jt0, mrow, sa);
+    const float t = mask_and_max(jt0, mrow, mask_words[0], sa);
     settle_max(fmaxf(t, __shfl_xor(t, 32, 64)));
   }
   // every wavefront has read the first K tile: the loop's first tile load overwrites it
@@ -720,6 +775,7 @@ static int launch_dma(AttnParams& p, hipStream_t stream, void* ws, size_t ws_byt
     }
   }
   const int n_parts = t.rem * t.key_chunks;
+  const bool words = p.mask != nullptr && n_tiles <= kMaskWords;
   int rc = ODIT_OK;
   if (p.n_full > 0) {
     // the persistent form draws its units from ticket words at the head of the workspace
@@ -732,13 +788,15 @@ static int launch_dma(AttnParams& p, hipStream_t stream, void* ws, size_t ws_byt
       }
     }
     if (W == 0) {
-      hipLaunchKernelGGL((attn_fwd_dma_kernel<T, D, NW, 0>), dim3(p.n_full), dim3(NW * 64), 0, stream, p);
+      if (words) hipLaunchKernelGGL((attn_fwd_dma_kernel<T, D, NW, 3>), dim3(p.n_full), dim3(NW * 64), 0, stream, p);
+      else hipLaunchKernelGGL((attn_fwd_dma_kernel<T, D, NW, 0>), dim3(p.n_full), dim3(NW * 64), 0, stream, p);
     }
     rc = check_launch("odit_attn_fwd");
   }
   if (rc != ODIT_OK || n_parts == 0) return rc;
   // stream order puts these after the full rounds, when every slot is free again
-  hipLaunchKernelGGL((attn_fwd_dma_kernel<T, D, NW, 1>), dim3(n_parts), dim3(NW * 64), 0, stream, p);
+  if (words) hipLaunchKernelGGL((attn_fwd_dma_kernel<T, D, NW, 4>), dim3(n_parts), dim3(NW * 64), 0, stream, p);
+  else hipLaunchKernelGGL((attn_fwd_dma_kernel<T, D, NW, 1>), dim3(n_parts), dim3(NW * 64), 0, stream, p);
   rc = check_launch("odit_attn_fwd (key-split tail)");
   if (rc != ODIT_OK) return rc;
   const int64_t rows = static_cast<int64_t>(t.rem) * BM;
