@@ -467,16 +467,16 @@ class FluxTransformer2DModel(nn.Module):
         self._mod_weight, self._mod_bias = w_all, b_all
 
     def _gated_biases(self):
-        """Biases of the gated output projections, dual [L, 2 (hidden, context), 2, C] and single [Ls, C] (None where
+        """float32 biases of the gated output projections, dual [L, 2 (hidden, context), 2, C] and single [Ls, C] (None where
         there are no such blocks), read on every call: a kept copy would miss ``p.data.copy_``."""
         dual = [p for blk in self.transformer_blocks
                 for p in (blk.attn.to_out[0].bias, blk.ff.net[2].bias, blk.attn.to_add_out.bias, blk.ff_context.net[2].bias)]
         single = [blk.proj_out.bias for blk in self.single_transformer_blocks]
-        d = torch.stack(dual).detach().view(len(self.transformer_blocks), 2, 2, self.inner_dim) if dual else None
-        return d, torch.stack(single).detach() if single else None
+        d = torch.stack(dual).detach().float().view(len(self.transformer_blocks), 2, 2, self.inner_dim) if dual else None
+        return d, torch.stack(single).detach().float() if single else None
 
     def all_gate_rows(self, mods):
-        """float32 (gates, gates * biases) of every gated projection, three small ops per step and kind of block:
+        """float32 (gates, gates * biases) of every gated projection, four small ops per step and kind of block:
         dual [B, L, 2, 2, C] pairs and single [B, Ls, C] pairs (None where there are no such blocks)."""
         if mods is None or mods[0].dtype == torch.float32:
             return None, None

@@ -589,16 +589,16 @@ class QwenImageTransformer2DModel(nn.Module):
         self._mod_weight, self._mod_bias = w_all, b_all
 
     def _gated_biases(self) -> torch.Tensor:
-        """[L, 2 (img, txt), 2 (attention, MLP), C]: biases of the four gated output projections of every block, read
+        """float32 [L, 2 (img, txt), 2 (attention, MLP), C]: biases of the four gated output projections of every block, read
         on every call: nothing a copy could be tagged with sees every way of writing a parameter (``p.data.copy_``
         changes neither its version counter nor its address)."""
         ps = [p for blk in self.transformer_blocks
               for p in (blk.attn.to_out.bias, blk.img_mlp.net[2].bias, blk.attn.to_add_out.bias, blk.txt_mlp.net[2].bias)]
-        return torch.stack(ps).detach().view(len(self.transformer_blocks), 2, 2, self.inner_dim)
+        return torch.stack(ps).detach().float().view(len(self.transformer_blocks), 2, 2, self.inner_dim)
 
     def all_gate_rows(self, mods: torch.Tensor | None):
         """float32 (gates, gates * biases) [B, L, 2, 2, C] of the four gated projections of every block,
-        from the stacked modulation parameters: three small ops per step."""
+        from the stacked modulation parameters: four small ops per step."""
         if mods is None or mods.dtype == torch.float32 or self.zero_cond_t:
             return None  # per-token gates of the editing variant do not fit one row per batch entry
         B, L, C = mods.shape[0], mods.shape[1], self.inner_dim

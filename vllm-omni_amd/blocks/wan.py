@@ -258,9 +258,9 @@ class WanTransformerBlock(nn.Module):
         return self.scale_shift_table.detach().float().reshape(6, -1)
 
     def gated_biases(self) -> torch.Tensor:
-        """[6, C]: in row 2 the bias of attn1.to_out, in row 5 that of ffn.net_2, the projections those gates scale (the
+        """float32 [6, C]: in row 2 the bias of attn1.to_out, in row 5 that of ffn.net_2, the projections those gates scale (the
         other rows repeat them): times the modulation rows it gives gate * bias rows that lie where the gate rows do."""
-        return torch.stack(self.gated_bias_rows()).detach()
+        return torch.stack(self.gated_bias_rows()).detach().float()
 
     def gated_bias_rows(self) -> tuple[torch.Tensor, ...]:
         return (self.attn1.to_out.bias,) * 3 + (self.ffn.net_2.bias,) * 3
@@ -523,7 +523,7 @@ class WanTransformer3DModel(nn.Module):
 
     def gate_bias_rows(self, mods: torch.Tensor) -> torch.Tensor:
         """float32 [L, B, 2, C]: every block's two gates (rows 2 and 5 of ``mods``) times the biases they scale."""
-        biases = torch.stack([b for blk in self.blocks for b in blk.gated_bias_rows()]).detach()
+        biases = torch.stack([b for blk in self.blocks for b in blk.gated_bias_rows()]).detach().float()
         return (mods * biases.view(len(self.blocks), 1, 6, -1))[:, :, 2::3]
 
     def norm2_affines(self) -> list:
