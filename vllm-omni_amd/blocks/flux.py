@@ -34,6 +34,7 @@ from ..layers.rope import RotaryEmbedding
 from . import qwen_image
 from .qwen_image import (AdaLayerNormContinuous, FeedForward, QwenTimestepProjEmbeddings, TimestepEmbedding,
                          Transformer2DModelOutput, _require_single_gpu, project_residual)
+from .weights import parameter_at
 
 
 class FluxRotary:
@@ -469,9 +470,10 @@ class FluxTransformer2DModel(nn.Module):
     def _gated_biases(self):
         """float32 biases of the gated output projections, dual [L, 2 (hidden, context), 2, C] and single [Ls, C] (None where
         there are no such blocks), read on every call: a kept copy would miss ``p.data.copy_``."""
-        dual = [p for blk in self.transformer_blocks
-                for p in (blk.attn.to_out[0].bias, blk.ff.net[2].bias, blk.attn.to_add_out.bias, blk.ff_context.net[2].bias)]
-        single = [blk.proj_out.bias for blk in self.single_transformer_blocks]
+        dual = [parameter_at(blk, *path) for blk in self.transformer_blocks
+                for path in (("attn", "to_out", "0", "bias"), ("ff", "net", "2", "bias"), ("attn", "to_add_out", "bias"),
+                             ("ff_context", "net", "2", "bias"))]
+        single = [parameter_at(blk, "proj_out", "bias") for blk in self.single_transformer_blocks]
         d = torch.stack(dual).detach().float().view(len(self.transformer_blocks), 2, 2, self.inner_dim) if dual else None
         return d, torch.stack(single).detach().float() if single else None
 

@@ -30,6 +30,7 @@ from ..layers.adalayernorm import AdaLayerNorm, adaln_pair
 from ..layers.rmsnorm import RMSNorm
 from ..layers.rope import RotaryEmbedding
 from .tables import TableCache
+from .weights import parameter_at
 
 
 def _require_single_gpu(od_config: Any | None) -> None:
@@ -592,8 +593,9 @@ class QwenImageTransformer2DModel(nn.Module):
         """float32 [L, 2 (img, txt), 2 (attention, MLP), C]: biases of the four gated output projections of every block, read
         on every call: nothing a copy could be tagged with sees every way of writing a parameter (``p.data.copy_``
         changes neither its version counter nor its address)."""
-        ps = [p for blk in self.transformer_blocks
-              for p in (blk.attn.to_out.bias, blk.img_mlp.net[2].bias, blk.attn.to_add_out.bias, blk.txt_mlp.net[2].bias)]
+        ps = [parameter_at(blk, *path) for blk in self.transformer_blocks
+              for path in (("attn", "to_out", "bias"), ("img_mlp", "net", "2", "bias"), ("attn", "to_add_out", "bias"),
+                           ("txt_mlp", "net", "2", "bias"))]
         return torch.stack(ps).detach().float().view(len(self.transformer_blocks), 2, 2, self.inner_dim)
 
     def all_gate_rows(self, mods: torch.Tensor | None):

@@ -28,7 +28,8 @@ class TableCache:
 
     def __init__(self, build: Callable[..., Any], maxsize: int):
         self._build, self._maxsize = build, maxsize
-        self._entries: OrderedDict[tuple, tuple[Any, int | None]] = OrderedDict()  # key -> value, the stream it was made on
+        # key -> value, the GPU it is on (None: host memory) and the stream it was made on
+        self._entries: OrderedDict[tuple, tuple[Any, torch.device | None, int]] = OrderedDict()
         self._lock = threading.Lock()
 
     def __reduce__(self):  # a copy of a module starts with an empty cache around its own ``build``
@@ -41,29 +42,28 @@ class TableCache:
                 self._entries.move_to_end(key)
         if entry is None:
             entry = self._make(key)
-        value, made_on = entry
-        if made_on is not None:
-            tensors = _tensors(value)
-            stream = torch.cuda.current_stream(tensors[0].device)
+        value, device, made_on = entry
+        if device is not None:
+            stream = torch.cuda.current_stream(device)
             if stream.cuda_stream != made_on:
-                for t in tensors:
+                for t in _tensors(value):
                     t.record_stream(stream)
         return value
 
-    def _make(self, key: tuple) -> tuple[Any, int | None]:
+    def _make(self, key: tuple) -> tuple[Any, torch.device | None, int]:
         value = self._build(*key)
-        made_on = None
+        entry = (value, None, 0)
         device = _tensors(value)[0].device
         if device.type == "cuda":
             if torch.cuda.is_current_stream_capturing():
-                return value, None
+                return entry
             stream = torch.cuda.current_stream(device)
             done = torch.cuda.Event()
             done.record(stream)
             done.synchronize()
-            made_on = stream.cuda_stream
+            entry = (value, device, stream.cuda_stream)
         with self._lock:
-            self._entries[key] = (value, made_on)
+            self._entries[key] = entry
             while len(self._entries) > self._maxsize:
                 self._entries.popitem(last=False)
-        return value, made_on
+        return entry

@@ -39,6 +39,7 @@ from . import qwen_image
 from .qwen_image import (ApproxGELU, QwenTimestepProjEmbeddings, TimestepEmbedding, Transformer2DModelOutput,
                          project_residual)
 from .tables import TableCache
+from .weights import parameter_at
 
 
 class DistributedRMSNorm(nn.Module):
@@ -263,7 +264,7 @@ class WanTransformerBlock(nn.Module):
         return torch.stack(self.gated_bias_rows()).detach().float()
 
     def gated_bias_rows(self) -> tuple[torch.Tensor, ...]:
-        return (self.attn1.to_out.bias,) * 3 + (self.ffn.net_2.bias,) * 3
+        return (parameter_at(self, "attn1", "to_out", "bias"),) * 3 + (parameter_at(self, "ffn", "net_2", "bias"),) * 3
 
     def _norm2_affine(self) -> tuple[torch.Tensor, torch.Tensor]:
         """float32 forms of norm2's weight and bias."""
