@@ -373,8 +373,9 @@ int odit_linear_tune(const void* x, const void* w, const void* bias, void* out, 
  * library launch per group of rows otherwise.
  * flags: 0 = choose as described above; ODIT_LINEAR_LIBRARY = hipBLASLt whatever the record says;
  * ODIT_LINEAR_HANDWRITTEN = the hand-written kernel for this row count (ODIT_ENOTSUP when it does not take
- * the problem); ODIT_LINEAR_FIRST = where hipBLASLt runs the problem, its own first choice (or the one odit_linear_prefer
- * named), not the one expected or tuned to be faster. Per call: no process-wide switch exists.
+ * the problem); ODIT_LINEAR_FIRST = where hipBLASLt runs the problem and no tuning call of this thread chose a kernel for it,
+ * its own first choice (or the one odit_linear_prefer named), not the one expected to be faster. Per call: no process-wide
+ * switch exists.
  */
 #define ODIT_LINEAR_LIBRARY 1u
 #define ODIT_LINEAR_HANDWRITTEN 2u

@@ -422,7 +422,7 @@ class WanTimeTextImageEmbedding(nn.Module):
         if encoder_hidden_states.shape[0] == 1:
             temb = mlp(t).type_as(encoder_hidden_states)
             timestep_proj = kernels.project(self.time_proj, temb, silu_input=True)
-        else:  # a CFG pair keeps the library's order of summation: guidance multiplies what another one rounds differently
+        else:  # a batch keeps the library's order of summation, as its blocks do (csrc/native.cpp, the Wan block)
             known = type(mlp) is TimestepEmbedding and "forward" not in mlp.__dict__   # (hooks run either way)
             temb = (mlp(t, library=True) if known else mlp(t)).type_as(encoder_hidden_states)
             timestep_proj = self.time_proj(kernels.silu(temb))

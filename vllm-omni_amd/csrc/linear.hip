@@ -179,7 +179,7 @@ struct LinCall {
   void* ws;
   size_t ws_bytes;
   hipStream_t stream;
-  bool first = false;  // the library's first-ranked kernel (ODIT_LINEAR_FIRST)
+  bool first = false;  // the library's first-ranked kernel, unless one was tuned (ODIT_LINEAR_FIRST)
 };
 
 static bool lin_is_residual(const LinCall& c) {
@@ -204,8 +204,12 @@ static int lin_prepare(const LinCall& c, hipblasLtHandle_t* h, LinPlan** plan, c
   const bool prep = lin_needs_prep(c);
   const bool alpha_vec = gated && c.gate != nullptr;
   const bool has_bias = c.bias != nullptr;
-  LinKey key{dev, c.M, c.N, c.K, c.epilogue * 4 + (has_bias ? 1 : 0) + (alpha_vec ? 2 : 0) + (c.first ? 0x100 : 0), c.dtype,
-             c.ldw, c.ldx, gated ? c.ldr : c.ldo, c.ldo};
+  LinKey key{dev, c.M, c.N, c.K, c.epilogue * 4 + (has_bias ? 1 : 0) + (alpha_vec ? 2 : 0), c.dtype, c.ldw, c.ldx,
+             gated ? c.ldr : c.ldo, c.ldo};
+  if (c.first) {  // unless a tuning call has found this problem's fastest kernel: what it chose runs
+    const auto it = g_lin.plans.find(key);
+    if (it == g_lin.plans.end() || !it->second.tuned) key.epi |= 0x100;
+  }
   rc = lin_plan(key, plan);
   if (rc != ODIT_OK) return rc;
   const size_t gb = lin_gate_bytes(c);
