@@ -20,10 +20,13 @@
 
 #include <ATen/ATen.h>
 #include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <map>
+#include <optional>
+#include <utility>
 #include <vector>
 
 #include "../../include/omni_dit.h"
@@ -92,42 +95,74 @@ PyObject* wrap2(Tensor a, Tensor b) {
     return nullptr;                                       \
   }
 
+// Other Python threads run while one of these exists. What allocates, ranks a library's kernels for a new problem or waits
+// for room in a full queue (all of it inside the C calls and at::empty) happens under one; nothing under it may touch a
+// Python object, and the tensors it works on are held by the caller's arguments or by BlockCall.
+class Unlocked {
+ public:
+  Unlocked() : state_(PyEval_SaveThread()) {}
+  ~Unlocked() { PyEval_RestoreThread(state_); }
+  Unlocked(const Unlocked&) = delete;
+  Unlocked& operator=(const Unlocked&) = delete;
+
+ private:
+  PyThreadState* state_;
+};
+template <typename F> auto unlocked(F f) {
+  const Unlocked u;
+  return f();
+}
+Tensor fresh(at::IntArrayRef sizes, const at::TensorOptions& opts) {
+  return unlocked([&] { return at::empty(sizes, opts); });
+}
+
 // ------------------------------------------------------------------------------------------- scratch
-// Scratch belongs to kernels.py (one buffer per device and stream; launches on one stream are ordered, so they can
-// share it). The buffers handed out are remembered here, with a reference that keeps them alive; kernels.py is asked
-// when there is none yet or it is too small. All of this runs under the interpreter lock.
+// Scratch belongs to kernels.py: one buffer per thread, device and stream. (Launches on one stream are ordered, so those of
+// one thread can share it. Those of two threads may alternate, and some calls make several launches that hand results to
+// each other in it.) What a thread was given is remembered here without a reference of its own and without the interpreter
+// lock's help, as the memory is the thread's; kernels.py is asked when there is none, it is gone or too small, and in a
+// graph capture, where kernels.py has to keep what the graph will use.
 PyObject* g_linear_scratch_fn = nullptr;  // (device index, stream) -> tensor
 PyObject* g_attn_scratch_fn = nullptr;    // (device index, stream, bytes) -> tensor
 
 struct Scratch { void* p = nullptr; size_t bytes = 0; };
-using ScratchPool = std::map<std::pair<int, void*>, Tensor>;
+using ScratchRef = c10::weak_intrusive_ptr<c10::TensorImpl>;
+using ScratchPool = std::map<std::pair<int, void*>, ScratchRef>;
 constexpr size_t kScratchKept = 64;  // remembered (device, stream) pairs; past that all are forgotten
 
 bool scratch_from(ScratchPool& pool, const Where& w, size_t bytes, Scratch* s, PyObject* (*ask)(const Where&, size_t)) {
-  auto it = pool.find({w.device, w.stream});
-  if (it == pool.end() || static_cast<size_t>(it->second.numel()) < bytes) {
-    PyObject* got = ask(w, bytes);
-    if (got == nullptr) return false;
-    const Tensor* t = tensor_of(got);
-    if (t == nullptr) { Py_DECREF(got); PyErr_SetString(PyExc_TypeError, "scratch must be a tensor"); return false; }
-    if (pool.size() >= kScratchKept) pool.clear();
-    it = pool.insert_or_assign({w.device, w.stream}, *t).first;
-    Py_DECREF(got);
+  const auto it = pool.find({w.device, w.stream});
+  const bool recording = c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None;
+  if (it != pool.end() && !recording) {
+    if (const auto t = it->second.lock(); t.defined() && static_cast<size_t>(t->numel()) >= bytes) {
+      s->p = t->mutable_data();
+      s->bytes = static_cast<size_t>(t->numel());
+      return true;
+    }
   }
-  s->p = it->second.data_ptr();
-  s->bytes = static_cast<size_t>(it->second.numel());
+  PyObject* got = ask(w, bytes);
+  if (got == nullptr) return false;
+  const Tensor* t = tensor_of(got);
+  if (t == nullptr) { Py_DECREF(got); PyErr_SetString(PyExc_TypeError, "scratch must be a tensor"); return false; }
+  if (!recording) {
+    if (pool.size() >= kScratchKept) pool.clear();
+    pool.insert_or_assign({w.device, w.stream}, ScratchRef(t->getIntrusivePtr()));
+  }
+  s->p = t->data_ptr();
+  s->bytes = static_cast<size_t>(t->numel());
+  Py_DECREF(got);  // (kernels.py keeps it)
   return true;
 }
 
 bool linear_scratch(const Where& w, Scratch* s) {
-  static auto* pool = new ScratchPool;  // (never destroyed: the allocator may be gone first at process end)
-  return scratch_from(*pool, w, 1, s, [](const Where& w_, size_t) {
+  static thread_local ScratchPool pool;
+  return scratch_from(pool, w, 1, s, [](const Where& w_, size_t) {
     return PyObject_CallFunction(g_linear_scratch_fn, "in", w_.device, reinterpret_cast<Py_ssize_t>(w_.stream));
   });
 }
 bool attn_scratch(const Where& w, size_t bytes, Scratch* s) {
-  static auto* pool = new ScratchPool;
-  return scratch_from(*pool, w, bytes, s, [](const Where& w_, size_t n) {
+  static thread_local ScratchPool pool;
+  return scratch_from(pool, w, bytes, s, [](const Where& w_, size_t n) {
     return PyObject_CallFunction(g_attn_scratch_fn, "inn", w_.device, reinterpret_cast<Py_ssize_t>(w_.stream),
                                  static_cast<Py_ssize_t>(n));
   });
@@ -143,8 +178,8 @@ PyObject* py_unary(PyObject*, PyObject* const* a, Py_ssize_t n) {  // (x, out or
   const int dt = code_of(*x);
   if (dt < 0 || !w.holds(x) || !w.holds(o) || !x->is_contiguous()) return none();
   if (o && (o->sizes() != x->sizes() || o->scalar_type() != x->scalar_type() || !o->is_contiguous())) return none();
-  Tensor out = o ? *o : at::empty_like(*x);
-  if (FN(x->data_ptr(), out.data_ptr(), x->numel(), dt, w.stream) != 0) return none();
+  Tensor out = o ? *o : fresh(x->sizes(), x->options());
+  if (unlocked([&] { return FN(x->data_ptr(), out.data_ptr(), x->numel(), dt, w.stream); }) != 0) return none();
   if (o) { Py_INCREF(a[1]); return a[1]; }
   return wrap(std::move(out));
   NATIVE_END
@@ -199,12 +234,12 @@ PyObject* py_adaln(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return none();
   if (!f32_row(lw, C) || !f32_row(lb, C) || !f32_row(sb, C) || !f32_row(cb, C)) return none();
   if (o && (o->sizes() != x->sizes() || o->scalar_type() != x->scalar_type() || o->stride(2) != 1)) return none();
-  Tensor out = o ? *o : at::empty({B, S, C}, x->options());
+  Tensor out = o ? *o : fresh({B, S, C}, x->options());
   const int64_t xs[2] = {x->stride(0), x->stride(1)}, os[2] = {out.stride(0), out.stride(1)};
-  if (odit_adaln_modulate(x->data_ptr(), out.data_ptr(), ptr(sh), ptr(sc), static_cast<const int32_t*>(ptr(index)),
+  if (unlocked([&] { return odit_adaln_modulate(x->data_ptr(), out.data_ptr(), ptr(sh), ptr(sc), static_cast<const int32_t*>(ptr(index)),
                           static_cast<const float*>(ptr(lw)), static_cast<const float*>(ptr(lb)),
                           static_cast<const float*>(ptr(sb)), static_cast<const float*>(ptr(cb)), B, S, C, xs, os, ms, mss,
-                          static_cast<float>(eps), mod_dt, dt, rr ? ODIT_FLAG_REF_ROUNDING : 0u, w.stream) != 0)
+                          static_cast<float>(eps), mod_dt, dt, rr ? ODIT_FLAG_REF_ROUNDING : 0u, w.stream); }) != 0)
     return none();
   if (o) { Py_INCREF(a[10]); return a[10]; }
   return wrap(std::move(out));
@@ -226,12 +261,12 @@ PyObject* py_adaln_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
       m->size(0) != x->size(0) || m->size(1) != 3 * x->size(2) || m->stride(1) != 1)
     return none();
   const int64_t B = x->size(0), S = x->size(1), C = x->size(2);
-  Tensor out = at::empty({B, S, C}, x->options());
+  Tensor out = fresh({B, S, C}, x->options());
   const int64_t xs[2] = {x->stride(0), x->stride(1)}, os[2] = {S * C, C};
   const char* mp = static_cast<const char*>(m->data_ptr());
-  if (odit_adaln_modulate(x->data_ptr(), out.data_ptr(), mp, mp + C * m->element_size(), nullptr, nullptr, nullptr, nullptr, nullptr,
+  if (unlocked([&] { return odit_adaln_modulate(x->data_ptr(), out.data_ptr(), mp, mp + C * m->element_size(), nullptr, nullptr, nullptr, nullptr, nullptr,
                           B, S, C, xs, os, B > 1 ? m->stride(0) : 0, 0, static_cast<float>(eps), mdt, dt,
-                          rr ? ODIT_FLAG_REF_ROUNDING : 0u, w.stream) != 0)
+                          rr ? ODIT_FLAG_REF_ROUNDING : 0u, w.stream); }) != 0)
     return none();
   return wrap2(std::move(out), m->narrow(1, 2 * C, C).unsqueeze(1));
   NATIVE_END
@@ -268,10 +303,10 @@ PyObject* py_adaln_pair(PyObject*, PyObject* const* a, Py_ssize_t n) {
     ms[i] = B > 1 ? sh.stride(0) : 0;
     xp[i] = x.data_ptr(); sp[i] = sh.data_ptr(); cp[i] = sc.data_ptr();
   }
-  Tensor o0 = at::empty({B, S[0], C}, x0.options()), o1 = at::empty({B, S[1], C}, x0.options());
+  Tensor o0 = fresh({B, S[0], C}, x0.options()), o1 = fresh({B, S[1], C}, x0.options());
   void* op[2] = {o0.data_ptr(), o1.data_ptr()};
-  if (odit_adaln_modulate_pair(xp, op, sp, cp, B, S, C, xs, os, ms, static_cast<float>(eps), mdt, dt,
-                               rr ? ODIT_FLAG_REF_ROUNDING : 0u, w.stream) != 0)
+  if (unlocked([&] { return odit_adaln_modulate_pair(xp, op, sp, cp, B, S, C, xs, os, ms, static_cast<float>(eps), mdt, dt,
+                               rr ? ODIT_FLAG_REF_ROUNDING : 0u, w.stream); }) != 0)
     return none();
   return wrap2(std::move(o0), std::move(o1));
   NATIVE_END
@@ -349,9 +384,9 @@ PyObject* py_qknorm_rope(PyObject*, PyObject* const* a, Py_ssize_t n) {
   QkProblem p;
   if (!qk_problem(w, t[0], t[1], t[2], t[3], t[4], t[5], t[6], t[7], t[8], t[9], mode, &p)) return none();
   const int64_t st[2] = {p.q->stride(0), p.q->stride(1)};
-  if (odit_qknorm_rope(ptr(p.q), ptr(p.k), ptr(p.v), t[3]->data_ptr(), ptr(t[4]), ptr(t[5]), ptr(p.wq), ptr(p.wk),
+  if (unlocked([&] { return odit_qknorm_rope(ptr(p.q), ptr(p.k), ptr(p.v), t[3]->data_ptr(), ptr(t[4]), ptr(t[5]), ptr(p.wq), ptr(p.wk),
                        static_cast<const float*>(ptr(p.cos)), static_cast<const float*>(ptr(p.sin)), p.B, p.S, p.H, p.D, p.rot,
-                       st, off, t[3]->size(1), static_cast<float>(eps), mode, p.w_dtype, code_of(*p.q), flags, w.stream) != 0)
+                       st, off, t[3]->size(1), static_cast<float>(eps), mode, p.w_dtype, code_of(*p.q), flags, w.stream); }) != 0)
     return none();
   Py_RETURN_TRUE;
   NATIVE_END
@@ -390,9 +425,9 @@ PyObject* py_qknorm_rope_pair(PyObject*, PyObject* const* a, Py_ssize_t n) {
       p[0].q->scalar_type() != p[1].q->scalar_type() || (k[0] == nullptr) != (k[1] == nullptr) ||
       (v[0] == nullptr) != (v[1] == nullptr) || (cs[0] == nullptr) != (cs[1] == nullptr))
     return none();
-  if (odit_qknorm_rope_pair(q, k, v, qo->data_ptr(), k[0] ? ptr(ko) : nullptr, v[0] ? ptr(vo) : nullptr, wq, wk, cs, sn, p[0].B, S, p[0].H, p[0].D,
+  if (unlocked([&] { return odit_qknorm_rope_pair(q, k, v, qo->data_ptr(), k[0] ? ptr(ko) : nullptr, v[0] ? ptr(vo) : nullptr, wq, wk, cs, sn, p[0].B, S, p[0].H, p[0].D,
                             p[0].rot, st, off, qo->size(1), static_cast<float>(eps), mode, p[0].w_dtype,
-                            code_of(*p[0].q), flags, w.stream) != 0)
+                            code_of(*p[0].q), flags, w.stream); }) != 0)
     return none();
   Py_RETURN_TRUE;
   NATIVE_END
@@ -426,11 +461,11 @@ PyObject* py_rmsnorm(PyObject*, PyObject* const* a, Py_ssize_t n) {
       if (width % d == 0) { hd = d; break; }
     if (hd == 0) return none();
   }
-  Tensor out = at::empty(x->sizes(), x->options());
+  Tensor out = fresh(x->sizes(), x->options());
   const int64_t st[2] = {rows * width, width};
-  if (odit_qknorm_rope(x->data_ptr(), nullptr, nullptr, out.data_ptr(), nullptr, nullptr, wt->data_ptr(), nullptr, nullptr,
+  if (unlocked([&] { return odit_qknorm_rope(x->data_ptr(), nullptr, nullptr, out.data_ptr(), nullptr, nullptr, wt->data_ptr(), nullptr, nullptr,
                        nullptr, 1, static_cast<int>(rows), static_cast<int>(width / hd), static_cast<int>(hd), 0, st, 0,
-                       static_cast<int>(rows), static_cast<float>(eps), mode, dt, dt, 0u, w.stream) != 0)
+                       static_cast<int>(rows), static_cast<float>(eps), mode, dt, dt, 0u, w.stream); }) != 0)
     return none();
   return wrap(std::move(out));
   NATIVE_END
@@ -445,13 +480,13 @@ PyObject* py_rotary(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (PyErr_Occurred()) return nullptr;
   const Where w;
   if (x->dim() != 4 || code_of(*x) < 0 || !w.holds(x)) return none();
-  Tensor out = at::empty(x->sizes(), x->options());
+  Tensor out = fresh(x->sizes(), x->options());
   QkProblem p;
   if (!qk_problem(w, x, nullptr, nullptr, &out, nullptr, nullptr, nullptr, nullptr, cs, sn, ODIT_NORM_NONE, &p)) return none();
   const int64_t st[2] = {x->stride(0), x->stride(1)};
-  if (odit_qknorm_rope(x->data_ptr(), nullptr, nullptr, out.data_ptr(), nullptr, nullptr, nullptr, nullptr,
+  if (unlocked([&] { return odit_qknorm_rope(x->data_ptr(), nullptr, nullptr, out.data_ptr(), nullptr, nullptr, nullptr, nullptr,
                        static_cast<const float*>(ptr(cs)), static_cast<const float*>(ptr(sn)), p.B, p.S, p.H, p.D, p.rot, st, 0,
-                       p.S, 1e-6f, ODIT_NORM_NONE, code_of(*x), code_of(*x), flags, w.stream) != 0)
+                       p.S, 1e-6f, ODIT_NORM_NONE, code_of(*x), code_of(*x), flags, w.stream); }) != 0)
     return none();
   return wrap(std::move(out));
   NATIVE_END
@@ -501,9 +536,9 @@ PyObject* py_attn(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const size_t need = odit_attn_fwd_workspace_bytes(B, Sq, Sk, H, D);
     if (need > 0 && !attn_scratch(w, need, &ws)) return nullptr;
   }
-  Tensor o = at::empty({B, split < 0 ? Sq : split, H, D}, q->options()), ot, lse;
-  if (split >= 0) ot = at::empty({B, Sq - split, H, D}, q->options());
-  if (want_lse) lse = at::empty({B, H, Sq}, q->options().dtype(at::kFloat));
+  Tensor o = fresh({B, split < 0 ? Sq : split, H, D}, q->options()), ot, lse;
+  if (split >= 0) ot = fresh({B, Sq - split, H, D}, q->options());
+  if (want_lse) lse = fresh({B, H, Sq}, q->options().dtype(at::kFloat));
   void *head = o.data_ptr(), *tail = nullptr;
   int64_t n_head = split < 0 ? Sq : split;
   int cut = 0;
@@ -514,9 +549,9 @@ PyObject* py_attn(PyObject*, PyObject* const* a, Py_ssize_t n) {
                 ts[3] = {(Sq - cut) * H * D, H * D, D};
   int64_t vts[3] = {0, 0, 0};
   if (vt) { vts[0] = vt->stride(0); vts[1] = vt->stride(1); vts[2] = vt->stride(2); }
-  if (odit_attn_fwd_ex(ptr(q), ptr(k), ptr(v), ptr(vt), k_split, head, tail, cut, static_cast<const uint8_t*>(ptr(mask)),
+  if (unlocked([&] { return odit_attn_fwd_ex(ptr(q), ptr(k), ptr(v), ptr(vt), k_split, head, tail, cut, static_cast<const uint8_t*>(ptr(mask)),
                        want_lse ? lse.data_ptr<float>() : nullptr, B, Sq, Sk, H, Hkv, D, qs, ks, vs, vt ? vts : nullptr, os,
-                       tail ? ts : nullptr, static_cast<float>(scale), dt, ws.p, ws.bytes, w.stream) != 0)
+                       tail ? ts : nullptr, static_cast<float>(scale), dt, ws.p, ws.bytes, w.stream); }) != 0)
     return none();
   if (split < 0 && !want_lse) return wrap(std::move(o));
   if (split < 0) return wrap2(std::move(o), std::move(lse));
@@ -552,9 +587,9 @@ PyObject* py_time_sinusoid(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const Where w;
   const int dt = code_of(*t);
   if (dt < 0 || !w.holds(t) || t->dim() != 1 || !t->is_contiguous() || dim <= 0 || dim % 2 || code < 0 || code > 2) return none();
-  Tensor out = at::empty({t->size(0), dim}, t->options().dtype(code == ODIT_BF16 ? at::kBFloat16 : code == ODIT_F16 ? at::kHalf : at::kFloat));
-  if (odit_time_sinusoid(t->data_ptr(), out.data_ptr(), t->size(0), static_cast<int>(dim), static_cast<float>(period),
-                         static_cast<float>(scale), static_cast<float>(pre), dt, static_cast<int>(code), w.stream) != 0)
+  Tensor out = fresh({t->size(0), dim}, t->options().dtype(code == ODIT_BF16 ? at::kBFloat16 : code == ODIT_F16 ? at::kHalf : at::kFloat));
+  if (unlocked([&] { return odit_time_sinusoid(t->data_ptr(), out.data_ptr(), t->size(0), static_cast<int>(dim), static_cast<float>(period),
+                         static_cast<float>(scale), static_cast<float>(pre), dt, static_cast<int>(code), w.stream); }) != 0)
     return none();
   return wrap(std::move(out));
   NATIVE_END
@@ -580,9 +615,9 @@ PyObject* py_rope_tables(PyObject*, PyObject* const* a, Py_ssize_t n) {
       t->size(1) != n_axes || i->size(1) != n_axes || !t->is_contiguous() || !i->is_contiguous())
     return none();
   const int64_t rows = t->size(0) + i->size(0);
-  Tensor c = at::empty({rows, half}, t->options().dtype(at::kFloat)), s = at::empty({rows, half}, t->options().dtype(at::kFloat));
-  if (odit_rope_tables(t->data_ptr(), t->size(0), i->data_ptr(), i->size(0), c.data_ptr<float>(), s.data_ptr<float>(), axes,
-                       static_cast<int>(n_axes), theta, dt, w.stream) != 0)
+  Tensor c = fresh({rows, half}, t->options().dtype(at::kFloat)), s = fresh({rows, half}, t->options().dtype(at::kFloat));
+  if (unlocked([&] { return odit_rope_tables(t->data_ptr(), t->size(0), i->data_ptr(), i->size(0), c.data_ptr<float>(), s.data_ptr<float>(), axes,
+                       static_cast<int>(n_axes), theta, dt, w.stream); }) != 0)
     return none();
   return wrap2(std::move(c), std::move(s));
   NATIVE_END
@@ -601,9 +636,9 @@ PyObject* py_cfg_combine(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if ((dt != ODIT_BF16 && dt != ODIT_F16) || !w.holds(p) || !w.holds(q) || p->dim() < 1 || p->numel() == 0 || p->sizes() != q->sizes() ||
       p->scalar_type() != q->scalar_type() || !p->is_contiguous() || !q->is_contiguous() || p->size(-1) >= (1ll << 31))
     return none();
-  Tensor out = at::empty(p->sizes(), p->options());
-  if (odit_cfg_combine(p->data_ptr(), q->data_ptr(), out.data_ptr(), p->numel() / p->size(-1), static_cast<int>(p->size(-1)),
-                       static_cast<float>(scale), norm, dt, w.stream) != 0)
+  Tensor out = fresh(p->sizes(), p->options());
+  if (unlocked([&] { return odit_cfg_combine(p->data_ptr(), q->data_ptr(), out.data_ptr(), p->numel() / p->size(-1), static_cast<int>(p->size(-1)),
+                       static_cast<float>(scale), norm, dt, w.stream); }) != 0)
     return none();
   return wrap(std::move(out));
   NATIVE_END
@@ -621,8 +656,8 @@ PyObject* py_euler_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (dt < 0 || !w.holds(x) || !w.holds(v) || x->sizes() != v->sizes() || x->scalar_type() != v->scalar_type() ||
       !x->is_contiguous() || !v->is_contiguous())
     return none();
-  Tensor out = at::empty(x->sizes(), x->options());
-  if (odit_euler_step(x->data_ptr(), v->data_ptr(), out.data_ptr(), x->numel(), static_cast<float>(step), dt, w.stream) != 0) return none();
+  Tensor out = fresh(x->sizes(), x->options());
+  if (unlocked([&] { return odit_euler_step(x->data_ptr(), v->data_ptr(), out.data_ptr(), x->numel(), static_cast<float>(step), dt, w.stream); }) != 0) return none();
   return wrap(std::move(out));
   NATIVE_END
 }
@@ -644,9 +679,9 @@ PyObject* py_linear_few(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (b && (b->numel() != N || !b->is_contiguous() || b->scalar_type() != x->scalar_type())) return none();
   std::vector<int64_t> shape(x->sizes().begin(), x->sizes().end());
   shape.back() = N;
-  Tensor out = at::empty(shape, x->options());
-  if (odit_linear_few(x->data_ptr(), wt->data_ptr(), ptr(b), out.data_ptr(), static_cast<int>(M), static_cast<int>(N),
-                      static_cast<int>(K), ldx, N > 1 ? wt->stride(0) : K, N, dt, PyObject_IsTrue(a[3]), w.stream) != 0)
+  Tensor out = fresh(shape, x->options());
+  if (unlocked([&] { return odit_linear_few(x->data_ptr(), wt->data_ptr(), ptr(b), out.data_ptr(), static_cast<int>(M), static_cast<int>(N),
+                      static_cast<int>(K), ldx, N > 1 ? wt->stride(0) : K, N, dt, PyObject_IsTrue(a[3]), w.stream); }) != 0)
     return none();
   return wrap(std::move(out));
   NATIVE_END
@@ -726,12 +761,12 @@ PyObject* py_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   } else {
     auto sizes = x->sizes().vec();
     sizes.back() = N;
-    out = at::empty(sizes, x->options());
+    out = fresh(sizes, x->options());
     ldo = N;
   }
-  if (odit_linear_rows(x->data_ptr(), wt->data_ptr(), bias_ptr, out.data_ptr(), ptr(r), ptr(g), M, N, K, ldx,
+  if (unlocked([&] { return odit_linear_rows(x->data_ptr(), wt->data_ptr(), bias_ptr, out.data_ptr(), ptr(r), ptr(g), M, N, K, ldx,
                        N > 1 ? wt->stride(0) : K, ldo, ldr, epi, gate_code, dt, rows_per_gate, gstride,
-                       static_cast<unsigned>(flags), ws.p, ws.bytes, w.stream) != 0)
+                       static_cast<unsigned>(flags), ws.p, ws.bytes, w.stream); }) != 0)
     return none();
   if (o) { Py_INCREF(a[8]); return a[8]; }
   return wrap(std::move(out));
@@ -797,6 +832,9 @@ struct BlockCall {
   at::ScalarType st = at::kBFloat16;
   unsigned engine = 0;
   int rc = 0;  // first non-zero status of a C call
+  mutable std::vector<Tensor> held;  // the parameters whose addresses were taken: another thread may replace them meanwhile
+
+  BlockCall() { held.reserve(32); }
 
   bool operand(const Tensor& t) const { return where.holds(t) && t.scalar_type() == st; }
 
@@ -805,6 +843,8 @@ struct BlockCall {
     const Tensor *w = d ? parameter(d, g_name.weight) : nullptr, *b = d ? parameter(d, g_name.bias) : nullptr;
     if (!w || !operand(*w) || w->dim() != 2 || w->stride(1) != 1 || (need_bias && !b)) return false;
     if (b && (!operand(*b) || !b->is_contiguous() || b->numel() != w->size(0))) return false;
+    held.push_back(*w);
+    if (b) held.push_back(*b);
     *out = Lin{w->data_ptr(), ptr(b), w->size(0), w->size(1), w->size(0) > 1 ? w->stride(0) : w->size(1)};
     return true;
   }
@@ -816,6 +856,7 @@ struct BlockCall {
     if (c != dtype && c != ODIT_F32) return false;
     if (*w_dtype >= 0 && *w_dtype != c) return false;
     *w_dtype = c;
+    held.push_back(*w);
     *out = w->data_ptr();
     return true;
   }
@@ -870,17 +911,21 @@ PyObject* py_project(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return none();
   auto sizes = x->sizes().vec();
   sizes.back() = l.n;
-  Tensor out = at::empty(sizes, x->options());
-  if (odit_linear_few(x->data_ptr(), l.w, l.b, out.data_ptr(), static_cast<int>(M), static_cast<int>(l.n), static_cast<int>(l.k), ldx,
-                      l.ldw, l.n, c.dtype, silu, c.where.stream) == 0)
-    return wrap(std::move(out));
+  Tensor out = fresh(sizes, x->options());
+  const int few = unlocked([&] {
+    return odit_linear_few(x->data_ptr(), l.w, l.b, out.data_ptr(), static_cast<int>(M), static_cast<int>(l.n), static_cast<int>(l.k), ldx,
+                           l.ldw, l.n, c.dtype, silu, c.where.stream);
+  });
+  if (few == 0) return wrap(std::move(out));
   if (silu) return none();
   if (!linear_scratch(c.where, &c.lin_ws)) return nullptr;
   const int epi = l.b ? ODIT_EPI_BIAS : ODIT_EPI_NONE;
-  if (odit_linear_rows(x->data_ptr(), l.w, l.b, out.data_ptr(), nullptr, nullptr, static_cast<int>(M), static_cast<int>(l.n),
-                       static_cast<int>(l.k), ldx, l.ldw, l.n, 0, epi, c.dtype, c.dtype, 0, 0, static_cast<unsigned>(flags),
-                       c.lin_ws.p, c.lin_ws.bytes, c.where.stream) != 0)
-    return none();
+  const int rc = unlocked([&] {
+    return odit_linear_rows(x->data_ptr(), l.w, l.b, out.data_ptr(), nullptr, nullptr, static_cast<int>(M), static_cast<int>(l.n),
+                            static_cast<int>(l.k), ldx, l.ldw, l.n, 0, epi, c.dtype, c.dtype, 0, 0, static_cast<unsigned>(flags),
+                            c.lin_ws.p, c.lin_ws.bytes, c.where.stream);
+  });
+  if (rc != 0) return none();
   return wrap(std::move(out));
   NATIVE_END
 }
@@ -1035,6 +1080,7 @@ bool run_dual(BlockCall& c, const DualBlock& k, const Tensor& img, const Tensor&
   const size_t attn_need = odit_attn_fwd_workspace_bytes(B, Sj, Sj, H, D);
   Scratch attn_ws;
   if (attn_need > 0 && !attn_scratch(c.where, attn_need, &attn_ws)) { c.rc = -100; return true; }
+  const Unlocked others_run;  // to the end
 
   void *n[2], *qkv[2], *jq, *jk, *jv = nullptr, *o[2], *u[2], *tmp;
   Slab slab(esz);
@@ -1226,6 +1272,7 @@ PyObject* dual_block(PyObject* const* a, Py_ssize_t n, bool flux) {
   if (!run_dual(c, k, *img, *txt, mod, gates, gbias, cos, sin, mask, index, min_rows, out)) return none();
   if (c.rc != 0) return block_error(c.rc);
   if (c.dtype == ODIT_F16) {  // the reference clips after every block
+    const Unlocked others_run;
     out[1].clamp_(-65504, 65504);
     if (!flux) out[0].clamp_(-65504, 65504);
   }
@@ -1270,6 +1317,7 @@ PyObject* py_flux_single_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const size_t attn_need = odit_attn_fwd_workspace_bytes(B, S, S, H, D);
   Scratch attn_ws;
   if (attn_need > 0 && !attn_scratch(c.where, attn_need, &attn_ws)) return nullptr;
+  std::optional<Unlocked> others_run(std::in_place);
   const int esz = 2;
   void *nx, *q3, *q, *k, *o, *u;
   Slab slab(esz);
@@ -1311,8 +1359,9 @@ PyObject* py_flux_single_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
   project_gated(c, u, wm, x->data_ptr(), out.data_ptr(), B, S, g, 0, nullptr, Gate());
   g.gbias = nullptr;
   project_gated(c, o, wa, out.data_ptr(), out.data_ptr(), B, S, g, 0, nullptr, Gate());
+  if (c.rc == 0 && c.dtype == ODIT_F16) out.clamp_(-65504, 65504);
+  others_run.reset();
   if (c.rc != 0) return block_error(c.rc);
-  if (c.dtype == ODIT_F16) out.clamp_(-65504, 65504);
   if (in_place) { Py_INCREF(a[3]); return a[3]; }
   return wrap(std::move(out));
   NATIVE_END
@@ -1385,6 +1434,7 @@ PyObject* py_wan_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
   Scratch ws;
   const size_t need = need1 > need2 ? need1 : need2;
   if (need > 0 && !attn_scratch(c.where, need, &ws)) return nullptr;
+  std::optional<Unlocked> others_run(std::in_place);
   const int esz = 2;
   void *nx, *q3, *q, *k, *o, *u, *kc, *kn, *vc, *y;
   Slab slab(esz);
@@ -1475,6 +1525,7 @@ PyObject* py_wan_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (c.rc == 0) modulate(out.data_ptr(), 3);
   c.project(nx, up, u, B * S, true);
   gated(u, down, out.data_ptr(), 5, 1);
+  others_run.reset();
   if (c.rc != 0) return block_error(c.rc);
   return wrap(std::move(out));
   NATIVE_END

@@ -14,6 +14,8 @@ and the errors.
 from __future__ import annotations
 
 import math
+import threading
+from collections import OrderedDict
 
 import torch
 from torch.nn.modules import module as _global_hooks
@@ -129,6 +131,44 @@ def _last_contig(t: torch.Tensor, name: str) -> None:
 # Copies this module makes on the caller's behalf where a kernel could not take the operands as given
 # (a path whose point is having none): counted so that a model run can assert it made none.
 HIDDEN_COPIES: dict[str, int] = {"attn_value_pair_concatenated": 0, "made_contiguous": 0}
+
+
+class _Scratch(threading.local):
+    """One kind of scratch of the calling thread, a tensor per (device, stream). Launches on one stream are ordered, so those
+    of one thread can share a buffer; those of two threads may alternate on a stream, also between the launches of one call
+    that hand results to each other in it. A thread's buffers are given back when it ends (or to make room past ``KEPT``),
+    to the stream that they were made and used on."""
+
+    KEPT = 16
+
+    def __init__(self):
+        self._by: OrderedDict[tuple[int, int], tuple[torch.Tensor, bool]] = OrderedDict()  # buffer, made in a capture
+
+    def get(self, device: int, stream: int, need: int) -> torch.Tensor:
+        """At least ``need`` bytes; zero-filled when new (kernels keep ticket words at the start and hand them back at zero).
+        A buffer made in a graph capture is zero only once the graph runs: eager calls get another."""
+        key, recording = (device, stream), torch.cuda.is_current_stream_capturing()
+        ws, made_in_capture = self._by.get(key, (None, False))
+        if ws is None or ws.numel() < need or (made_in_capture and not recording):
+            ws = torch.zeros(need, dtype=torch.uint8, device=torch.device("cuda", device))
+            self._by[key] = (ws, recording)
+            while len(self._by) > self.KEPT:
+                self._by.popitem(last=False)
+        if recording:
+            _IN_GRAPHS[ws.data_ptr()] = ws
+        return ws
+
+    def __getitem__(self, key: tuple[int, int]) -> torch.Tensor:
+        return self._by[key][0]
+
+    def values(self):
+        return [ws for ws, _ in self._by.values()]
+
+    def clear(self) -> None:
+        self._by.clear()
+
+
+_IN_GRAPHS: dict[int, torch.Tensor] = {}  # scratch whose address a recorded graph may hold: kept for the process
 
 
 # --------------------------------------------------------------------------------------------- K1
@@ -250,7 +290,7 @@ def attn_plan(B: int, Sq: int, Sk: int, H: int, D: int, k_seq_stride: int | None
     return buf.value.decode()
 
 
-_ATTN_SCRATCH: dict[tuple[int, int], torch.Tensor] = {}
+_ATTN_SCRATCH = _Scratch()
 
 
 def _attn_workspace(lib, device: torch.device, B: int, Sq: int, Sk: int, H: int, D: int) -> torch.Tensor | None:
@@ -259,15 +299,8 @@ def _attn_workspace(lib, device: torch.device, B: int, Sq: int, Sk: int, H: int,
 
 
 def _attn_scratch(device: int, stream: int, need: int) -> torch.Tensor:
-    """Scratch for the key-split tail of the attention launch, one growing buffer per (device, stream):
-    launches on one stream are ordered, so they can share it."""
-    key = (device, stream)
-    ws = _ATTN_SCRATCH.get(key)
-    if ws is None or ws.numel() < need:
-        # zero-filled once: the first kilobyte holds the ticket words the persistent kernel draws its units from
-        ws = torch.zeros(need, dtype=torch.uint8, device=torch.device("cuda", device))
-        _ATTN_SCRATCH[key] = ws
-    return ws
+    """Scratch for the key-split tail of the attention launch (and the ticket words of its persistent form)."""
+    return _ATTN_SCRATCH.get(device, stream, need)
 
 
 # --------------------------------------------------------------------------------------------- K2
@@ -627,7 +660,7 @@ def silu(x: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
 
 
 # --------------------------------------------------------------------------------------------- GEMM
-_LINEAR_SCRATCH: dict[tuple[int, int], torch.Tensor] = {}
+_LINEAR_SCRATCH = _Scratch()
 _LINEAR_AUTOTUNE_ITERS = 0
 _LINEAR_TUNED: dict[tuple, float] = {}
 
@@ -682,13 +715,8 @@ def _linear_workspace(lib, device: torch.device) -> torch.Tensor:
 
 
 def _linear_scratch(device: int, stream: int) -> torch.Tensor:
-    key = (device, stream)
-    ws = _LINEAR_SCRATCH.get(key)
-    if ws is None:
-        # zero-filled once: the stream-K kernel keeps its ticket words at the start
-        ws = torch.zeros(int(_lib.load().odit_linear_workspace_bytes()), dtype=torch.uint8, device=torch.device("cuda", device))
-        _LINEAR_SCRATCH[key] = ws
-    return ws
+    """The library's workspace and the stream-K kernel's ticket words and partial tiles."""
+    return _LINEAR_SCRATCH.get(device, stream, int(_lib.load().odit_linear_workspace_bytes()))
 
 
 def _rows2d(t: torch.Tensor, name: str) -> tuple[torch.Tensor, int]:
