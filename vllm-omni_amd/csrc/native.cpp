@@ -843,6 +843,8 @@ struct BlockCall {
     const Tensor *w = d ? parameter(d, g_name.weight) : nullptr, *b = d ? parameter(d, g_name.bias) : nullptr;
     if (!w || !operand(*w) || w->dim() != 2 || w->stride(1) != 1 || (need_bias && !b)) return false;
     if (b && (!operand(*b) || !b->is_contiguous() || b->numel() != w->size(0))) return false;
+    // (the library's kernels are chosen by sizes and strides and take the address for aligned; torch looks at it)
+    if (!aligned16(w->data_ptr()) || (b && !aligned16(b->data_ptr()))) return false;
     held.push_back(*w);
     if (b) held.push_back(*b);
     *out = Lin{w->data_ptr(), ptr(b), w->size(0), w->size(1), w->size(0) > 1 ? w->stride(0) : w->size(1)};
@@ -906,7 +908,7 @@ PyObject* py_project(PyObject*, PyObject* const* a, Py_ssize_t n) {
   c.st = x->scalar_type();
   Lin l;
   int64_t M, ldx;
-  if ((c.dtype != ODIT_BF16 && c.dtype != ODIT_F16) || !c.operand(*x) || x->dim() < 1 || !c.linear(a[0], &l, false) ||
+  if ((c.dtype != ODIT_BF16 && c.dtype != ODIT_F16) || !c.operand(*x) || !aligned16(x->data_ptr()) || x->dim() < 1 || !c.linear(a[0], &l, false) ||
       x->size(-1) != l.k || l.n == 0 || l.k == 0 || l.n >= (1ll << 31) || !rows_of(*x, &M, &ldx) || M == 0 || M >= (1ll << 31))
     return none();
   auto sizes = x->sizes().vec();
@@ -1216,7 +1218,7 @@ bool dual_attention(const BlockCall& c, PyObject* attn, PyTypeObject* type, Dual
 }
 
 bool block_input(BlockCall& c, const Tensor* x) {
-  if (!x || x->dim() != 3 || !x->is_contiguous() || !c.where.holds(*x)) return false;
+  if (!x || x->dim() != 3 || !x->is_contiguous() || !c.where.holds(*x) || !aligned16(x->data_ptr())) return false;
   const int dt = code_of(*x);
   if (dt != ODIT_BF16 && dt != ODIT_F16) return false;
   c.dtype = dt;
@@ -1224,8 +1226,12 @@ bool block_input(BlockCall& c, const Tensor* x) {
   return linear_scratch(c.where, &c.lin_ws);
 }
 
-PyObject* block_error(int rc) {
+// The answer of a block function after a C call that did not succeed. A refusal (an operand, a workspace or a problem that a
+// kernel does not take) leaves the block to Python, which has other ways for some of them and raises for the rest: what has
+// been launched wrote this call's own tensors only. Anything else, and a refusal behind a write to the caller's tensor, raises.
+PyObject* block_failed(int rc, bool caller_written = false) {
   if (PyErr_Occurred()) return nullptr;
+  if (!caller_written && (rc == ODIT_EINVAL || rc == ODIT_ENOTSUP || rc == ODIT_EWORKSPACE)) return none();
   return PyErr_Format(PyExc_RuntimeError, "native block: a kernel call failed with status %d: %s", rc, odit_last_error());
 }
 
@@ -1277,7 +1283,7 @@ PyObject* dual_block(PyObject* const* a, Py_ssize_t n, bool flux) {
   }
   Tensor out[2];
   if (!run_dual(c, k, *img, *txt, mod, gates, gbias, cos, sin, mask, index, min_rows, out)) return none();
-  if (c.rc != 0) return block_error(c.rc);
+  if (c.rc != 0) return block_failed(c.rc);
   if (c.dtype == ODIT_F16) {  // the reference clips after every block
     const Unlocked others_run;
     out[1].clamp_(-65504, 65504);
@@ -1364,11 +1370,12 @@ PyObject* py_flux_single_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
   wm.k = F;
   wa.k = C;
   project_gated(c, u, wm, x->data_ptr(), out.data_ptr(), B, S, g, 0, nullptr, Gate());
+  const bool written = in_place && c.rc == 0;
   g.gbias = nullptr;
   project_gated(c, o, wa, out.data_ptr(), out.data_ptr(), B, S, g, 0, nullptr, Gate());
   if (c.rc == 0 && c.dtype == ODIT_F16) out.clamp_(-65504, 65504);
   others_run.reset();
-  if (c.rc != 0) return block_error(c.rc);
+  if (c.rc != 0) return block_failed(c.rc, written);
   if (in_place) { Py_INCREF(a[3]); return a[3]; }
   return wrap(std::move(out));
   NATIVE_END
@@ -1536,7 +1543,7 @@ PyObject* py_wan_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
   c.project(nx, up, u, B * S, true);
   gated(u, down, out.data_ptr(), 5, 1);
   others_run.reset();
-  if (c.rc != 0) return block_error(c.rc);
+  if (c.rc != 0) return block_failed(c.rc);
   return wrap(std::move(out));
   NATIVE_END
 }
