@@ -17,12 +17,17 @@ struct GemmEpilogue {
 };
 
 __device__ __forceinline__ float gemm_gelu_tanh(float x) {
-  // x sigmoid(2 u), u = sqrt(2/pi) (x + 0.044715 x^3), with e^(-2 u) as a power of two and the hardware reciprocal (1 ulp; a
-  // division costs ten instructions, and 48 elements per lane wait here with nothing to overlap: 4.5 us of a 47 us launch
-  // at M=512, N=12288, K=3072)
+  // x sigmoid(2 u), u = sqrt(2/pi) (x + 0.044715 x^3), with e^(-2 u) as a power of two. 48 elements per lane wait here with
+  // nothing to overlap, so the quotient is the hardware reciprocal (1 ulp) with one correction by the remainder, six
+  // instructions where the compiler's division takes ten. Error against float64 (2-norm, relative; reciprocal alone / corrected /
+  // x / (1 + exp) in float32): N(0,1) 4.71e-8 / 4.21e-8 / 4.32e-8, N(0,0.01) 5.18e-8 / 4.37e-8 / 4.37e-8, N(0,3) 3.50e-8 /
+  // 3.34e-8 / 3.35e-8. Time at N=12288, K=3072 (M = 80 / 256 / 512 / 1024), reciprocal alone 30.3 / 36.4 / 47.3 / 90.4 us,
+  // corrected 31.1 / 37.2 / 48.0 / 91.9.
   const float e = __builtin_amdgcn_exp2f(x * fmaf(x * x, -2.f * 0.7978845608028654f * 0.044715f * 1.4426950408889634f,
                                                   -2.f * 0.7978845608028654f * 1.4426950408889634f));
-  return x * __builtin_amdgcn_rcpf(1.f + e);
+  const float d = 1.f + e, r = __builtin_amdgcn_rcpf(d), q = x * r, rem = fmaf(-q, d, x);
+  // (a zero remainder: q is exact; an infinite or NaN one: x or d is infinite and q is the limit)
+  return __builtin_amdgcn_classf(rem, 0x198) ? fmaf(rem, r, q) : q;
 }
 
 // y[0..8) = accumulators of row m, features n .. n + 7 (n a multiple of 8, m < M, n < N): applies the
