@@ -38,9 +38,6 @@ bool gemm_streamk_takes(const GemmCall& c, int dtype);
 // overridden by the next launch (its ticket words carry a larger epoch).
 int launch_gemm_streamk(const GemmCall* c, int count, int dtype, void* scratch, hipStream_t stream);
 
-// expected time (us) of a launch over problems of M0 and M1 rows (M1 = 0: one problem)
-float gemm_streamk_us(int M0, int M1, int N, int K, int device_cus);
-
 // compute units of the current device (0 when it cannot be read)
 int device_cus();
 

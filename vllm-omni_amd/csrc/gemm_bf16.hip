@@ -537,8 +537,6 @@ static StreamkPlan plan_streamk(int M0, int M1, int N, int K, int cus) {
   return best;
 }
 
-float gemm_streamk_us(int M0, int M1, int N, int K, int cus) { return plan_streamk(M0, M1, N, K, cus).us; }
-
 int launch_gemm_streamk(const GemmCall* c, int count, int dtype, void* scratch, hipStream_t stream) {
   const int cus = device_cus();
   if (cus <= 0) { set_error("odit_linear: cannot read the device's compute-unit count"); return ODIT_ELAUNCH; }

@@ -529,7 +529,10 @@ extern "C" int odit_linear_rows(const void* x, const void* w, const void* bias, 
 // behind those of the first and no gate per launch; the library has the faster main loop for many rows. Up to kPairTiles
 // tiles of 128 rows together the launch wins (us, launch / two library calls): 4 + 1 tiles QKV 42 / 70, out 24 / 36; 6 + 2
 // tiles QKV 69 / 86, MLP up 88 / 102, out 32 / 44. With gates that differ per batch entry the library needs a call per
-// entry, and for few rows a residual pass: kPairTilesGated.
+// entry, and for few rows a residual pass: kPairTilesGated. Those are at width 3072, where the lines were drawn. At other
+// widths C (QKV N = 3 C, MLP up 4 C, 6 + 1 tiles; gated MLP down, 16 + 4 tiles in two batch entries): 1024 19 / 23, 25 / 24,
+// 39 / 60; 2048 33 / 42, 42 / 48, 96 / 146; 4096 107 / 106, 151 / 126, 367 / 403; 5120 174 / 145, 232 / 206, 524 / 863: past
+// 3072 the QKV and MLP-up launches should end at 3 to 4 tiles. No dual-stream model here is that wide.
 constexpr int kPairTiles = 8, kPairTilesGated = 20;
 
 extern "C" int odit_linear_pair(const odit_linear_problem* q, int N, int K, int epilogue, int gate_dtype, int dtype, unsigned flags,
