@@ -29,7 +29,7 @@ PEAK_HBM_GBS = 8000.0            # MI355X HBM3E, vendor figure
 # summaries under profiles/ (vllm_omni_amd.profiling.attention_figures), which name the launches they were
 # measured on: a build that dispatches other launches for the headline shape makes bench.py stop.
 
-# Qwen-Image shape at 1024x1024
+# Qwen-Image shape at 1024x1024, the headline workload
 LAYERS, HEADS, HEAD_DIM, MLP_RATIO = 60, 24, 128, 4
 C = HEADS * HEAD_DIM
 S_IMG, S_TXT, TEXT_DIM, IN_CH = 4096, 256, 3584, 64
@@ -241,7 +241,7 @@ def _init_synthetic(torch, model, seed=0):
 
 
 def flux_workload(torch, layers=None):
-    """BASELINE.json configs[4]: Flux shape, 19 dual + 38 single blocks, B=1, 512 text + 4096 image tokens."""
+    """Flux shape, 19 dual + 38 single blocks, B=1, 512 text + 4096 image tokens."""
     from vllm_omni_amd.blocks.flux import FluxTransformer2DModel
     from vllm_omni_amd.denoise import euler_step, flow_match_sigmas
 
@@ -296,7 +296,7 @@ def flux_workload(torch, layers=None):
 
 
 def wan_workload(torch, layers=None):
-    """BASELINE.json configs[3]: Wan2.1-14B shape, 40 blocks, B=2, 21x30x52 = 32760 video tokens, 512 text tokens."""
+    """Wan2.1-14B shape, 40 blocks, B=2, 21x30x52 = 32760 video tokens, 512 text tokens."""
     from vllm_omni_amd.blocks.wan import WanTransformer3DModel
     from vllm_omni_amd.denoise import combine_cfg_noise, euler_step
 
@@ -366,7 +366,7 @@ def run_secondary(torch, kernels, args):
     teacache = None
     if args.teacache is not None:
         if args.workload != "flux":
-            sys.exit("bench.py: --teacache is measured at the Flux shape (BASELINE.json configs[4]): use --workload flux")
+            sys.exit("bench.py: --teacache is measured at the Flux shape: use --workload flux")
         teacache = teacache_trajectory(torch, model, step, args.teacache, args.steps / elapsed)
     print(json.dumps({
         "metric": f"DiT denoise steps/s, {args.workload} shape (1 GPU)", "value": args.steps / elapsed,
@@ -386,7 +386,7 @@ def run_secondary(torch, kernels, args):
 
 
 def teacache_trajectory(torch, model, step, thresh, plain_steps_per_s, steps=28, first_trajectory_decisions=None):
-    """the 28-step trajectory with the TeaCache hook on (relative-L1 threshold `thresh`
+    """The 28-step trajectory with the TeaCache hook on (relative-L1 threshold `thresh`
     on the modulated first-block input, the reference's 4th-order polynomial for this model): one untimed
     trajectory, then the same trajectory timed. Steps/s counts every denoise step, skipped or computed."""
     from vllm_omni_amd.cache.teacache import TeaCacheBackend
@@ -420,7 +420,7 @@ def teacache_trajectory(torch, model, step, thresh, plain_steps_per_s, steps=28,
 
 
 def teacache_flux(torch, kernels):
-    """BASELINE.json configs[4] inside the default run: the Flux-shape model (19 dual + 38 single blocks, 512 text +
+    """The 28-step TeaCache trajectory inside the default run: the Flux-shape model (19 dual + 38 single blocks, 512 text +
     4096 image tokens, bf16), 28 Euler steps under the TeaCache hook at threshold 0.25, next to the uncached rate.
     During the untimed first trajectory the operands of the first three relative-L1 reductions are copied to the
     host, and the scalar the hook thresholded is checked, bit for bit, against the reference's own expression
@@ -736,7 +736,7 @@ def main():
     ap.add_argument("--no-in-step", action="store_true",
                     help="skip the two extra, untimed steps whose kernels are bracketed one by one (kernels_in_step)")
     ap.add_argument("--no-teacache", action="store_true",
-                    help="skip the Flux-shape TeaCache trajectory (BASELINE.json configs[4]) that follows the headline measurement")
+                    help="skip the Flux-shape TeaCache trajectory that follows the headline measurement")
     args = ap.parse_args()
     if args.gpus != 1 or int(os.environ.get("WORLD_SIZE", "1")) != 1:
         sys.exit("bench.py: this build runs the DiT step on ONE GPU (CFG branches are batched on it; "
@@ -848,11 +848,14 @@ def main():
         "config": {"workload": f"Qwen-Image-shape MMDiT denoise step: {args.blocks} dual-stream blocks, hidden {C}, "
                                f"{HEADS} heads x {HEAD_DIM}, MLP {MLP_RATIO * C}, {S_IMG} image + {S_TXT} text tokens, "
                                "CFG batch 2, random weights N(0,0.02)",
-                   "valid": args.blocks == LAYERS, "gemm": "hipBLASLt via torch" + (" (tuned solution table)" if tuned else "") +
-                           ("" if args.linear_engine == "library" else "; text-stream MLP down-projection on the hand-written "
-                            "stream-K MFMA kernel") +
+                   "valid": args.blocks == LAYERS, "gemm": ("plain torch linears" if args.unfused_epilogues else
+                                                                "whole blocks as native calls, projections through odit_linear_rows: "
+                                                                "hipBLASLt's kernels") +
+                           (" (tuned solution table)" if tuned else "") +
+                           ("" if args.linear_engine == "library" or args.unfused_epilogues else
+                            ", the text stream's MLP down-projection on the hand-written stream-K MFMA kernel") +
                            ("; GELU and gated residuals as separate kernels" if args.unfused_epilogues else
-                            "; GELU and gated residuals in the GEMM epilogues (odit_linear)")},
+                            "; GELU and gated residuals in the GEMM epilogues")},
         "roofline": {"kernel": f"joint attention, B=2, 24x128, S=4352; one call = {plan} (timed together)", "bound": "mfma",
                      "achieved": attn_tflops, "peak": PEAK_MFMA_BF16_TFLOPS, "unit": "TFLOP/s",
                      "frac": attn_tflops / PEAK_MFMA_BF16_TFLOPS,

@@ -4,7 +4,7 @@ plain tree runs through native calls that never call the modules."""
 import pytest
 import torch
 
-from test_gpu_native_path import _flux, _qwen
+from test_gpu_native_path import _flux, _qwen, _wan
 from vllm_omni_amd.hooks.base import HookRegistry, ModelHook
 
 pytestmark = pytest.mark.gpu
@@ -146,3 +146,19 @@ def test_wrapped_time_embedding_gets_the_scaled_timestep(gpu):
         wrapped = call()
     assert seen == [torch.tensor(0.3).bfloat16().mul(1000).item()]
     assert torch.equal(plain, wrapped)
+
+
+@pytest.mark.parametrize("make,option", [(_qwen, False), (_flux, False), (_wan, False), (_wan, True)])
+def test_parameters_written_through_data_are_used(gpu, monkeypatch, make, option):
+    """As a weight loader writes them, without a trace in version counters or addresses: the second forward is that of the
+    new values, on both paths."""
+    model, call = make(gpu, torch.bfloat16, 64, option)
+    before, _ = _both(monkeypatch, call)
+    g = torch.Generator(device=gpu).manual_seed(7)
+    for name, p in model.named_parameters():
+        if name.endswith("bias") or "norm" in name or "scale_shift_table" in name:
+            p.data.copy_(p + 0.3 * torch.randn(p.shape, device=gpu, generator=g).to(p.dtype))
+    native, stepwise = _both(monkeypatch, call)
+    bound = 2.0 ** -5   # both paths round at every operation (2^-9); the new values move the result by far more
+    assert (native - stepwise).norm() <= bound * stepwise.norm()
+    assert (native - before).norm() > 4 * bound * before.norm()

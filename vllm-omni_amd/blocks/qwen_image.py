@@ -8,9 +8,11 @@ qit.py:1073-1113). Differences are all below the module interfaces:
   * QK-RMSNorm + rotary + the three ``torch.cat([txt, img])`` copies are one fused pass per stream that
     writes straight into the joint [B, S_txt+S_img, H, D] buffers (qit.py:588-606);
   * adaLN LayerNorm+modulate and the gated residual are one pass each (qit.py:770-773, 794-806);
-  * GELU(tanh) runs in place on the MLP-up output (qit.py:424);
-  * dense projections are ``torch.nn.functional.linear`` (hipBLASLt MFMA GEMMs);
-  * a block of plain modules runs as ONE native call (``csrc/native.cpp``), which makes the same launches.
+  * GELU(tanh) and the gated residuals sit in the epilogues of the MLP-up and the output projections (qit.py:424, 794-806);
+  * dense projections go through ``odit_linear_rows`` / ``odit_linear_pair``: hipBLASLt's MFMA GEMMs for many rows, hand-written
+    ones for few (both streams' in one launch where that is faster);
+  * a block of plain modules runs as ONE native call (``csrc/native.cpp``). Through Python, kernel by kernel, it makes the
+    same launches but for the projections: plain ones are torch's linear, and each stream's are launches of their own.
 """
 
 from __future__ import annotations
@@ -103,8 +105,8 @@ class FeedForward(nn.Module):
 
 
 def project(lin: nn.Linear, x: torch.Tensor) -> torch.Tensor:
-    """lin(x). A bf16 projection that a hand-written GEMM kernel would run (the engine asked for, or the one
-    a tuning call found faster for this problem) goes through ``kernels.linear``; everything else through
+    """lin(x) outside a native block. A bf16 projection that a hand-written GEMM kernel would run (the engine asked for, or
+    the one a tuning call found faster for this problem) goes through ``kernels.linear``; everything else through
     torch's linear (hipBLASLt with the solution table tuned offline)."""
     if (x.dtype == torch.bfloat16 and x.is_cuda and x.is_contiguous()
             and kernels.linear(x, lin.weight, lin.bias, plan_only=True)[0]):
@@ -115,7 +117,7 @@ def project(lin: nn.Linear, x: torch.Tensor) -> torch.Tensor:
 # The gate differs per batch entry. The hand-written GEMM takes one gate vector per batch entry in one
 # launch; the library needs one GEMM per entry, and below this many rows per entry (the 256-token text
 # stream of a CFG batch: two GEMMs of 256 rows) one library GEMM over all entries plus the
-# gated-residual kernel is faster than that (measured: 1.2 ms of a 135 ms step).
+# gated-residual kernel is faster than that (measured: 1.2 ms of a 135 ms step). Native blocks go by it too.
 FUSE_MIN_ROWS = 1024
 
 

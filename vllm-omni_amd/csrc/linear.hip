@@ -2,11 +2,12 @@
 //   * GELU(tanh)                              (MLP up-projection: no separate activation pass)
 //   * out = residual + gate * (x W^T + bias)  (attention / MLP output projections: no separate
 //                                              gated-residual pass)
-// The contraction itself is a genuine dense GEMM and runs on hipBLASLt's MFMA kernels; what this file
-// adds is the problem set-up that lets the library's epilogue do the elementwise work (bias vector,
-// activation, a per-output-feature alpha vector for the gate, beta = 1 on the residual), a per-thread
-// cache of problem descriptors, and an explicit tuning call that times the library's candidate kernels
-// for one problem and remembers the fastest.
+// Which kernel runs is decided here per call. Few rows: the hand-written stream-K kernel (gemm_bf16.hip) where the reduction is
+// long, and for the two streams of a dual-stream block in one launch (odit_linear_pair). Many rows: hipBLASLt's MFMA kernels (or
+// the hand-written tile kernel, gemm_bf16_tile.hip, where asked for or tuned). For the library this file sets the problem up so
+// that its epilogue does the elementwise work (bias vector, activation, a per-output-feature alpha vector for the gate, beta = 1
+// on the residual), keeps problem descriptors per thread, chooses among the library's candidates for long reductions by expected
+// time, and has an explicit tuning call that times all engines for one problem and remembers the fastest.
 //
 // Row-major y[M,N] = x[M,K] W[N,K]^T is the column-major product D(N x M) = op(A) B with A = W stored
 // K x N (ld = ldw, transposed), B = x stored K x M (ld = ldx): the bias and the alpha vector run along

@@ -132,7 +132,7 @@ def summarise_counters(dir_a: str, dir_b: str, probe_stdout: str) -> str:
     _check_plan_in_trace(plan, list(a), "counter pass a")
     L = ["# rocprofv3 hardware-counter summary (SQ block): every hand-written kernel of the path and the two large library GEMMs at the",
          "# Qwen-Image shape (B=2, 4096 image + 256 text tokens, 24 heads x 128, hidden 3072, MLP 12288), bf16, N(0,1) data, MI355X.",
-         "# commands (from the repo root, on the GPU box; one counter set per run):",
+         "# commands (from the repo root; one counter set per run):",
          "#   export TMPDIR=/tmp OUT=<a scratch directory>",
          f"#   rocprofv3 --pmc {PASS_A} --output-format csv -d $OUT/pmc_sq_a -o a -- python3 bench.py --counter-probe > $OUT/pmc_sq_probe.log",
          f"#   rocprofv3 --pmc {PASS_B} --output-format csv -d $OUT/pmc_sq_b -o b -- python3 bench.py --counter-probe",
@@ -245,7 +245,7 @@ def summarise_traffic(dir_fetch: str, dir_write: str, probe_stdout: str) -> str:
 _STEP_NOTES = {
     "qwen_image": ("Qwen-Image-shape denoise step (60 blocks, B=2, 4096+256 tokens)", "",
                    ["# GELU and the image stream's gated residuals run inside the GEMM epilogues (odit_linear -> the Cijk_* kernels); the",
-                    "# text stream's MLP down-projection with its gated residual is gemm_bf16_streamk_kernel, its other gated residual the",
+                    "# text stream's MLP down-projection with its gated residual is gemm_streamk_kernel, its other gated residual the",
                     "# gated_residual_kernel rows."]),
     "flux": ("FLUX.1-shape denoise step (19 dual-stream + 38 single-stream blocks, B=1, 4096+512 tokens)", " --workload flux", []),
     "wan": ("Wan2.2-shape denoise step (40 blocks, B=2, 32760 video tokens, 512 text tokens)", " --workload wan", []),
@@ -257,13 +257,15 @@ def summarise_step(directory: str, bench_stdout: str, workload: str) -> str:
     rows = list(csv.DictReader(open(_one(os.path.join(directory, "**", "*kernel_stats.csv")))))
     d = _probe_json(bench_stdout)
     r = d["roofline"]
-    steps = d["steps"] + d["warmup"]
+    after = 1 if workload == "wan" else 2   # steps behind the timed ones, kernel by kernel, with events around the attention
+    steps = d["steps"] + d["warmup"] + after
     out = [f"# rocprofv3 kernel-trace summary: bench.py, {title}, MI355X",
-           "# commands (from the repo root, on the GPU box):",
+           "# commands (from the repo root):",
            f"#   export TMPDIR=/tmp OUT=<a scratch directory>; rocprofv3 --kernel-trace --stats --output-format csv -d $OUT/prof_{workload} -o bench -- "
            f"python3 bench.py{flag} --steps {d['steps']} --warmup {d['warmup']} --no-cpu --no-kernels --no-in-step --no-teacache > $OUT/prof_{workload}.log",
            f"#   python3 -m vllm_omni_amd.profiling step $OUT/prof_{workload} $OUT/prof_{workload}.log {workload}",
-           f"# {steps} steps recorded ({d['warmup']} warm-up + {d['steps']} timed) => per-step time = total / {steps}. Weight-initialisation kernels of the",
+           f"# {steps} steps recorded ({d['warmup']} warm-up + {d['steps']} timed, blocks as native calls; {after} kernel by kernel with the attention",
+           f"# between events) => per-step time = total / {steps}. Weight-initialisation kernels of the",
            "# synthetic model (at::native::distribution_* = normal_ init, FillFunctor = zero_ init, __amd_rocclr_copyBuffer = stacking the",
            "# modulation weights) are part of the run but not of a step."] + notes + [
            f"# bench.py line of this run (under the profiler): {d['value']:.3f} steps/s, {d['ms_per_step']:.1f} ms/step; attention avg "
