@@ -186,3 +186,22 @@ def test_a_pipelines_own_cfg_normalisation_is_used(where):
     pos, neg = torch.randn(1, 3, 8), torch.randn(1, 3, 8)
     assert torch.equal(pipe.combine_cfg_noise(pos, neg, 4.0, True), torch.full((1, 3, 8), 7.0))
     torch.testing.assert_close(pipe.combine_cfg_noise(pos, neg, 4.0, False), neg + 4.0 * (pos - neg))
+
+
+def test_a_replaced_wan_block_gets_the_arguments_it_knows(monkeypatch):
+    from vllm_omni_amd.blocks.wan import WanTransformer3DModel
+
+    model = _random_(WanTransformer3DModel(num_attention_heads=1, attention_head_dim=64, text_dim=32, ffn_dim=128, num_layers=2))
+    block = model.blocks[0]
+    got = []
+
+    def forward(x, ctx, temb, rotary=None, mod=None, gate_bias=None):
+        got.append((temb is None, mod is None, gate_bias is None))
+        return x + 1
+
+    for b in model.blocks:
+        b.forward = forward
+    x, ctx = torch.zeros(1, 3, 64), torch.zeros(1, 4, 64)
+    assert torch.equal(model.run_blocks(x, ctx, torch.zeros(1, 6, 64), None), x + 2)
+    assert torch.equal(model.run_blocks(x, ctx, torch.zeros(1, 3, 6, 64), None), x + 2)
+    assert got == [(True, False, True)] * 2 + [(False, True, True)] * 2

@@ -536,16 +536,21 @@ class WanTransformer3DModel(nn.Module):
         return [(rows[2 * i], rows[2 * i + 1]) for i in range(len(norms))]
 
     def run_blocks(self, x, ctx, timestep_proj, rotary):
+        per_token = timestep_proj.ndim == 4  # the blocks read the rows of timestep_proj directly
+        mods = gb = tables = None
+        if per_token:
+            tables = torch.cat([blk.scale_shift_table for blk in self.blocks], dim=0).detach().float() if len(self.blocks) else None
+        else:
+            mods = self.all_modulations(timestep_proj)
+            gb = self.gate_bias_rows(mods) if x.dtype != torch.float32 else None
         affines = self.norm2_affines()
-        if timestep_proj.ndim == 4:  # per-token timesteps: the blocks read the rows of timestep_proj directly
-            tables = torch.cat([blk.scale_shift_table for blk in self.blocks], dim=0).detach().float() if len(self.blocks) else ()
-            for block, table, affine in zip(self.blocks, tables, affines):
-                x = block(x, ctx, timestep_proj, rotary, table=table, norm2_affine=affine)
-            return x
-        mods = self.all_modulations(timestep_proj)
-        gb = self.gate_bias_rows(mods) if x.dtype != torch.float32 else None
         for i, block in enumerate(self.blocks):
-            x = block(x, ctx, None, rotary, mod=mods[i], gate_bias=None if gb is None else gb[i], norm2_affine=affines[i])
+            kw = {} if per_token else dict(mod=mods[i], gate_bias=None if gb is None else gb[i])
+            if type(block).forward is WanTransformerBlock.forward and "forward" not in block.__dict__:  # (others may not take them)
+                kw["norm2_affine"] = affines[i]
+                if per_token:
+                    kw["table"] = tables[i]
+            x = block(x, ctx, timestep_proj if per_token else None, rotary, **kw)
         return x
 
     def finish(self, x: torch.Tensor, temb: torch.Tensor, grid: tuple[int, int, int], return_dict: bool = True):

@@ -279,7 +279,8 @@ def attn_fwd(
 def attn_plan(B: int, Sq: int, Sk: int, H: int, D: int, k_seq_stride: int | None = None,
               v_seq_stride: int | None = None, use_workspace: bool = True) -> str:
     """The launches ``attn_fwd`` makes for a problem, as "<kernel> units=<n>" joined by "; " (kernel names as
-    a profiler reports them). Strides default to those of dense [B,S,H,D] tensors."""
+    a profiler reports them). Strides default to those of dense [B,S,H,D] tensors. (With a key mask of up to 65536 keys the
+    kernels are the same but for their last template argument, 3 in the place of 0 and 4 in that of 1.)"""
     lib = _lib.load()
     buf = _lib.C.create_string_buffer(512)
     dense = H * D
