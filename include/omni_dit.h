@@ -66,7 +66,7 @@ const char* odit_last_error(void);
  * multiple of 8 elements and every base pointer 16-byte aligned. H % Hkv == 0 (grouped KV).
  * key_mask: NULL, or uint8 [B,Sk] (row stride Sk); keys with mask == 0 are excluded, matching the
  *   [B,Sk] boolean key-padding mask of flash_attn.py:80-102. A row whose keys are all excluded
- *   returns zeros. A mask without an excluded key gives the bits of no mask, in 1 to 3 % more time.
+ *   returns zeros. A mask without an excluded key gives the bits of no mask, in 1 to 4 % more time.
  * lse: NULL, or float [B,H,Sq] receiving log(sum exp(scale*q.k)) per row (natural log).
  * dtype: ODIT_BF16 or ODIT_F16 (fp32 never reaches a backend: attention/layer.py:134-140).
  * D in {64, 128}.

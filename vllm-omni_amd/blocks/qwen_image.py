@@ -623,7 +623,7 @@ class QwenImageTransformer2DModel(nn.Module):
     def run_blocks(self, img, txt, temb, rotary, encoder_hidden_states_mask=None, attention_kwargs=None,
                    modulate_index=None):
         # the reference drops an all-true mask (qit.py:1044-1048), which takes a synchronisation; the masked kernel gives
-        # the same values for one at 1 to 3 % of its time, as a tile without an excluded key runs without selects
+        # the same values for one at 1 to 4 % of its time, as a tile without an excluded key runs without selects
         mask = encoder_hidden_states_mask
         joint = joint_key_mask(mask, None, img.shape[0], txt.shape[1], img.shape[1], img.device)
         mods = self.all_modulations(temb)

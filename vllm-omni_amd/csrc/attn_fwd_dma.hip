@@ -23,11 +23,11 @@
 // Key mask. Before the first scores each wavefront turns its share of the mask row into one 64-bit word per key tile (a
 // ballot over the tile's 64 bytes; keys past Sk are zero bits) in LDS. A tile whose word is all ones then runs like a tile of
 // a launch without a mask, any other one selects its scores by the word's bits, wave-uniform both. Read as bytes from
-// global memory at every tile, 32 loads, clamps and selects per lane, a mask cost 33 to 84 % whatever was in it. us, bf16,
+// global memory at every tile, 32 loads, clamps and selects per lane, a mask cost 34 to 88 % whatever was in it. us, bf16,
 // no mask / all-true mask, bytes / all-true mask, words:
-//   B=2 S=4352 H=24 D=128  450 / 735 / 461      B=1 S=4608 H=24 D=128  256 / 471 / 263
-//   B=2 S=592 H=24 D=128   18.8 / 26.8 / 18.9   B=2 S=4352 H=24 D=64   284 / 505 / 292
-// (and 499 / 293 / 20.6 / 336 with a random mask, where every tile is mixed).
+//   B=2 S=4352 H=24 D=128  439 / 737 / 451      B=1 S=4608 H=24 D=128  249 / 469 / 258
+//   B=2 S=592 H=24 D=128   18.4 / 26.8 / 18.8   B=2 S=4352 H=24 D=64   279 / 505 / 289
+// (and 490 / 290 / 20.6 / 333 with a random mask, where every tile is mixed).
 // Past kMaskWords tiles, and in the persistent form, whose units change the batch row, the mask is read as bytes.
 //
 // Persistent form (MODE 2), a measurement aid that no default launch uses (ODIT_ATTN_PERSISTENT=1 in the
@@ -575,7 +575,9 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void attn_fwd_dma_kernel(const Att
     };
     bool plain_next = has_next && mrow_n == nullptr && (jn + 1) * BN <= p.Sk;  // no exclusions in the next scores
     uint64_t word = 0;  // (the same in every lane)
-    if (WORDS && has_next) word = mask_words[WORDS ? jn - jt0 : 0];
+    if constexpr (WORDS) {
+      if (has_next) word = mask_words[jn - jt0];
+    }
     float mx = -INFINITY;
 #pragma unroll
     for (int st = 0; st < PF; ++st) v_fetch(st);
@@ -587,10 +589,12 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void attn_fwd_dma_kernel(const Att
       u32x4_v pb;
       pb.x = pf[kt][g2][0]; pb.y = pf[kt][g2][1]; pb.z = pf[kt][g2][2]; pb.w = pf[kt][g2][3];
       o[dt] = M::run(__builtin_bit_cast(frag, av), __builtin_bit_cast(frag, pb), o[dt]);
-      if (WORDS && st == 1) {
-        const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(word));
-        const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(word >> 32));
-        plain_next = has_next && (lo & hi) == ~0u;
+      if constexpr (WORDS) {
+        if (st == 1) {
+          const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(word));
+          const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(word >> 32));
+          plain_next = has_next && (lo & hi) == ~0u;
+        }
       }
       if (st == 1 && plain_next) {  // wave-uniform
         float t = s_next[0][0];
@@ -661,7 +665,9 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void attn_fwd_dma_kernel(const Att
   f32x16_v sa[2], sb[2];
   qk_plain(Kb, sa);
   {
-    const float t = mask_and_max(jt0, mrow, mask_words[0], sa);
+    uint64_t word = 0;
+    if constexpr (WORDS) word = mask_words[0];
+    const float t = mask_and_max(jt0, mrow, word, sa);
     settle_max(fmaxf(t, __shfl_xor(t, 32, 64)));
   }
   // every wavefront has read the first K tile: the loop's first tile load overwrites it
