@@ -318,22 +318,22 @@ int odit_silu(const void* x, void* out, int64_t n, int dtype, void* stream);
  *   RowParallelLinear followed by `h + gate * y`           qwen_image_transformer.py:794-795, 801, 806,
  *                                                          flux_transformer.py:288-309, wan2_2_transformer.py:661, 673
  * Engines. hipBLASLt's MFMA kernels (a plain dense GEMM), set up so that bias, activation, gate and
- * residual ride in that kernel's epilogue, and two hand-written MFMA kernels (K a multiple of 64, N a
- * multiple of 8, 16-byte aligned rows): a stream-K kernel, bf16 or fp16, for M <= 1024 rows (csrc/gemm_bf16.hip) that
- * keeps all CUs busy on few output tiles, and a bf16 tile kernel for more rows (csrc/gemm_bf16_tile.hip: 256 x 256
- * or 256 x 192 output tiles, one per workgroup). Both take one gate vector per group of rows in a single
- * launch (odit_linear_rows). A hand-written kernel runs where a tuning call found it faster or, untuned,
- * where its default rule says so (stream-K: K >= 2 N and M >= 48); the `flags` of odit_linear_rows can force either side.
+ * residual ride in that kernel's epilogue, and two hand-written MFMA kernels, bf16 or fp16 (K a multiple of 64, N a
+ * multiple of 8, 16-byte aligned rows): a stream-K kernel for few rows (csrc/gemm_bf16.hip) and a tile kernel for many
+ * (csrc/gemm_bf16_tile.hip: 256 x 256 or 128 x 256 output tiles, the last round's cut along the reduction where they are
+ * few). Both take one gate vector per group of rows in a single launch (odit_linear_rows). Which runs: what a tuning call
+ * found, else the stream-K kernel for 48 to 1024 rows and K >= 2 N, else the tile kernel (256 rows or more) or the library by
+ * expected time; the `flags` of odit_linear_rows can force either side.
  *
  * x [M,K] (row stride ldx), W [N,K] (row stride ldw: torch's nn.Linear weight, or a column range of
  * one), bias [N] or NULL, out [M,N] (row stride ldo). Gated form: residual [M,N] (row stride ldr; may be
  * `out` itself), gate [N] of `dtype` or float32 (gate_dtype), NULL = ones: one call per batch row when
  * the gate differs per batch row. dtype: ODIT_BF16, ODIT_F16 or ODIT_F32 (fp32 accumulation always).
  * workspace: device scratch, 256-byte aligned, for the library's split-K kernels, in the gated form two
- * float[N] vectors, and the hand-written kernel's tile counters and partial tiles;
+ * float[N] vectors, and the hand-written kernels' ticket words and partial tiles;
  * odit_linear_workspace_bytes() is a size that suits every kernel. A workspace of that size must be
  * ZERO-FILLED ONCE before its first use and not written by the caller afterwards (the first 32 KB hold
- * the stream-K kernel's ticket words, stamped with the launch number like those of odit_rel_l1: every call
+ * the hand-written kernels' ticket words, stamped with the launch number like those of odit_rel_l1: every call
  * leaves them at zero, and what a launch that did not finish left there is overridden by the next one);
  * calls that share a workspace must not overlap in time (one workspace per stream). A smaller workspace goes to the library alone and rules the
  * hand-written kernel out; NULL restricts the choice to library kernels that need none (not allowed
@@ -375,23 +375,25 @@ int odit_linear_tune(const void* x, const void* w, const void* bias, void* out, 
  * flags: 0 = choose as described above; ODIT_LINEAR_LIBRARY = hipBLASLt whatever the record says;
  * ODIT_LINEAR_HANDWRITTEN = the hand-written kernel for this row count (ODIT_ENOTSUP when it does not take
  * the problem); ODIT_LINEAR_FIRST = where hipBLASLt runs the problem and no tuning call of this thread chose a kernel for it,
- * its own first choice (or the one odit_linear_prefer named), not the one expected to be faster. Per call: no process-wide
- * switch exists.
+ * its own first choice (or the one odit_linear_prefer named), not the one expected to be faster, and what ODIT_LINEAR_NO_TILE
+ * says; ODIT_LINEAR_NO_TILE = not the tile kernel, unless a tuning call found it faster (a caller whose results another order of
+ * summation may not move). Per call: no process-wide switch exists.
  */
 #define ODIT_LINEAR_LIBRARY 1u
 #define ODIT_LINEAR_HANDWRITTEN 2u
 #define ODIT_LINEAR_FIRST 4u
+#define ODIT_LINEAR_NO_TILE 8u
 
 int odit_linear_rows(const void* x, const void* w, const void* bias, void* out, const void* residual,
                      const void* gate, int M, int N, int K, int64_t ldx, int64_t ldw, int64_t ldo, int64_t ldr,
                      int epilogue, int gate_dtype, int dtype, int rows_per_gate, int64_t gate_stride,
                      unsigned flags, void* workspace, size_t workspace_bytes, void* stream);
 
-/* Two projections of the same N, K, epilogue and types in ONE launch of the stream-K kernel: the image and the text rows of a
+/* Two projections of the same N, K, epilogue and types in ONE launch of a hand-written kernel (stream-K or tile): the image and the text rows of a
  * dual-stream block (to_qkv beside add_kv_proj, qwen_image_transformer.py:566-580, and the output, up and down projections).
  * Fields as the arguments of odit_linear_rows. Returns ODIT_ENOTSUP, with nothing launched, where two odit_linear_rows calls
- * are the better way (many rows) or the kernel does not take a problem; the caller then makes them. flags as for
- * odit_linear_rows (ODIT_LINEAR_LIBRARY: always ODIT_ENOTSUP). */
+ * are the better way or the kernels do not take a problem; the caller then makes them. flags as for
+ * odit_linear_rows (ODIT_LINEAR_LIBRARY: always ODIT_ENOTSUP; ODIT_LINEAR_HANDWRITTEN: the stream-K kernel). */
 typedef struct odit_linear_problem {
   const void *x, *w, *bias, *residual, *gate;
   void* out;

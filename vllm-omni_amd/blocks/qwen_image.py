@@ -73,9 +73,9 @@ class ApproxGELU(nn.Module):
         self.proj = nn.Linear(dim_in, dim_out, bias=bias)
         self.fused = fused
 
-    def forward(self, x: torch.Tensor) -> torch.Tensor:
+    def forward(self, x: torch.Tensor, engine: str | None = None) -> torch.Tensor:
         if self.fused and x.dtype != torch.float32 and x.is_contiguous():
-            return kernels.linear(x, self.proj.weight, self.proj.bias, activation="gelu_tanh")
+            return kernels.linear(x, self.proj.weight, self.proj.bias, activation="gelu_tanh", engine=engine)
         y = self.proj(x)
         return kernels.gelu_tanh(y, out=y)
 
@@ -123,19 +123,20 @@ FUSE_MIN_ROWS = 1024
 
 def project_residual(lin: nn.Linear, x: torch.Tensor, residual: torch.Tensor, gate: torch.Tensor | None,
                      out: torch.Tensor | None = None, fused: bool = True, ref_rounding: bool = False,
-                     pre: tuple[torch.Tensor, torch.Tensor | None] | None = None) -> torch.Tensor:
+                     pre: tuple[torch.Tensor, torch.Tensor | None] | None = None, engine: str | None = None) -> torch.Tensor:
     """residual + gate * lin(x) (gate [B,N] or [B,1,N], None = plain add) in one GEMM, or, unfused, as
     projection + gated-residual kernel (qit.py:794-806). ``pre`` = (float32 gate [B,N], float32
-    gate * bias [B,N] or None) made by the caller for all blocks at once replaces ``gate`` on the fused path."""
+    gate * bias [B,N] or None) made by the caller for all blocks at once replaces ``gate`` on the fused path. ``engine``: as for
+    ``kernels.linear``."""
     per_token_gate = gate is not None and gate.dim() == 3 and gate.shape[1] != 1
     few_rows = gate is not None and x.dim() == 3 and x.shape[0] > 1 and x.shape[1] < FUSE_MIN_ROWS
     if (fused and not ref_rounding and not per_token_gate and x.dtype != torch.float32
             and x.is_contiguous() and residual.is_contiguous()):
         if pre is not None:
-            args = dict(residual=residual, gate=pre[0], gate_bias=pre[1], prescaled=True)
+            args = dict(residual=residual, gate=pre[0], gate_bias=pre[1], prescaled=True, engine=engine)
             bias = None
         else:
-            args = dict(residual=residual, gate=gate)
+            args = dict(residual=residual, gate=gate, engine=engine)
             bias = lin.bias
         if not few_rows or kernels.linear(x, lin.weight, bias, plan_only=True, **args)[0]:
             return kernels.linear(x, lin.weight, bias, out=out, **args)

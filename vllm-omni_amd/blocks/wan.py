@@ -123,6 +123,17 @@ class WanRotaryPosEmbed(nn.Module):
         return self._tables(nf // p_t, hh // p_h, ww // p_w, str(hidden_states.device))
 
 
+def _batch_engine(x: torch.Tensor) -> str | None:
+    """As in the native block, a batch (a CFG pair) keeps the kernels that earlier versions ran: guidance multiplies the
+    difference of its rows, and results of another order of summation would be as far apart as either is from float32."""
+    return "no_tile" if x.shape[0] > 1 and kernels.linear_engine_flags() == 0 else None
+
+
+def _feed_up(net_0: nn.Module, x: torch.Tensor) -> torch.Tensor:
+    engine = _batch_engine(x)
+    return net_0(x, engine=engine) if engine and kernels.plain_module(net_0, ApproxGELU) else net_0(x)
+
+
 class WanFeedForward(nn.Module):
     """net_0 = Linear + GELU(tanh), net_2 = Linear (wan.py:112-144)."""
 
@@ -133,7 +144,7 @@ class WanFeedForward(nn.Module):
         self.net_2 = nn.Linear(inner_dim, dim_out or dim, bias=bias)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return self.net_2(self.net_0(x))
+        return self.net_2(_feed_up(self.net_0, x))
 
 
 class WanSelfAttention(nn.Module):
@@ -165,7 +176,7 @@ class WanSelfAttention(nn.Module):
                             cos, sin, eps=self.norm_q.eps, norm_mode=ODIT_NORM_ROW)
         o = self.attn(q, k, qkv[:, :, 2]).flatten(2, 3)
         if residual is not None:
-            return project_residual(self.to_out, o, residual, gate, pre=pre)
+            return project_residual(self.to_out, o, residual, gate, pre=pre, engine=_batch_engine(o))
         return self.to_out(o)
 
 
@@ -225,7 +236,7 @@ class WanCrossAttention(nn.Module):
             o_img = self.attn(q, k_img, v_img).flatten(2, 3)
             o = kernels.gated_residual(o, o_img, None, out=o)  # two separate softmaxes, summed (wan.py:577-579)
         if residual is not None:
-            return project_residual(self.to_out, o, residual, None, out=out)
+            return project_residual(self.to_out, o, residual, None, out=out, engine=_batch_engine(o))
         return self.to_out(o)
 
 
@@ -303,7 +314,7 @@ class WanTransformerBlock(nn.Module):
             n = kernels.adaln_modulate(x, None, None, eps=self.eps, ln_weight=lw, ln_bias=lb, out=n)
         x = self.attn2(n, encoder_hidden_states, residual=x, out=x)
         n = kernels.adaln_modulate(x, c_shift, c_scale, eps=self.eps, out=n if n is not x else None)
-        return project_residual(self.ffn.net_2, self.ffn.net_0(n), x, c_gate, out=x, pre=pre2)
+        return project_residual(self.ffn.net_2, _feed_up(self.ffn.net_0, n), x, c_gate, out=x, pre=pre2, engine=_batch_engine(n))
 
     def _forward_native(self, x, ctx, temb, rotary_emb, mod, gate_bias, table, norm2_affine):
         """The whole block as one native call, or None where the call or a submodule is not of the plain form."""

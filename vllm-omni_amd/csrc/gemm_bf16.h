@@ -41,12 +41,33 @@ int launch_gemm_streamk(const GemmCall* c, int count, int dtype, void* scratch, 
 // compute units of the current device (0 when it cannot be read)
 int device_cus();
 
-// ---- gemm_bf16_tile.hip: one 256 x 256 (or 256 x 192) output tile per workgroup, for many rows -------
-// whether the kernel takes this problem (bf16, K a multiple of 64, N of 8, 16-byte aligned rows,
-// operands addressable with 32-bit byte offsets); it needs no scratch
+// expected time of the launch (us), 0 where the kernel has no plan for it
+float gemm_streamk_us(int M0, int M1, int N, int K, int cus);
+
+// ---- gemm_bf16_tile.hip: output tiles of 256 x 256 or 128 x 256, for many rows -------
+// whether the kernel takes this problem (bf16 or fp16, K a multiple of 64, N of 8, 8 rows or more, 16-byte aligned rows,
+// operands addressable with 32-bit byte offsets)
 bool gemm_tile_takes(const GemmCall& c, int dtype);
-int launch_gemm_tile(const GemmCall& c, int device_cus, hipStream_t stream);
-// features per tile (256 or 192: whichever fills the last round of workgroups better) and tiles of a launch
-int gemm_tile_plan(int M, int N, int device_cus, int* tile_n, int* tiles);
+
+// the last K - k_split elements of every row of x come from here (k_split a multiple of 64)
+struct TileX2 {
+  const void* x;
+  int64_t ldx;
+  int k_split;
+};
+
+struct TilePlan {
+  int bm = 0;             // rows per tile (0: no plan)
+  int tiles0, tiles;      // tiles of the first problem, of all
+  int whole, parts;       // tiles that are not cut along the reduction; parts of each of the others
+  int grid;
+  float us;               // expected time
+};
+// One problem or two of the same K; `scratch`: whether tiles may be cut.
+TilePlan plan_gemm_tile(const GemmCall* c, int count, int cus, bool scratch);
+
+// One problem, or two of the same K in one launch. `scratch` as for launch_gemm_streamk, or null (no tile is cut). `x2`: with
+// one problem only.
+int launch_gemm_tile(const GemmCall* c, int count, const TileX2* x2, int dtype, void* scratch, hipStream_t stream);
 
 }  // namespace odit

@@ -81,10 +81,11 @@ __device__ __forceinline__ const char* uniform(const char* p) {
 // 16 bytes per lane past the XCD's L2, where the workgroups of all XCDs see them (what an agent-scope atomic store and
 // load of a word do, four words at a time); `base` is wave-uniform, `off` the lane's byte offset. The address may come
 // out of a v_readfirstlane right in front: a memory instruction may read a scalar register 5 wait states after a vector
-// instruction has written it and no sooner, and the compiler does not look into these statements, so they wait themselves.
+// instruction has written it and no sooner, and the compiler does not look into these statements, so they wait themselves; and a
+// vector instruction may write a 16-byte store's data registers 2 wait states behind it and no sooner.
 __device__ __forceinline__ void store_through(const char* base, uint32_t off, f32x4_v v) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("s_nop 4\n\tglobal_store_dwordx4 %0, %1, %2 sc1" ::"v"(off), "v"(v), "s"(base) : "memory");
+  asm volatile("s_nop 4\n\tglobal_store_dwordx4 %0, %1, %2 sc1\n\ts_nop 1" ::"v"(off), "v"(v), "s"(base) : "memory");
 #endif
 }
 // N vectors 1 KB apart in one round trip (loads and wait in one statement: nothing can touch the registers before the
@@ -535,6 +536,11 @@ static StreamkPlan plan_streamk(int M0, int M1, int N, int K, int cus) {
     offer(groups, 8.f + steps * k.step + k.range + static_cast<float>(steps / k_steps) * 6.f);
   }
   return best;
+}
+
+float gemm_streamk_us(int M0, int M1, int N, int K, int cus) {
+  const StreamkPlan p = plan_streamk(M0, M1, N, K, cus);
+  return p.groups > 0 ? p.us : 0.f;
 }
 
 int launch_gemm_streamk(const GemmCall* c, int count, int dtype, void* scratch, hipStream_t stream) {

@@ -1,416 +1,683 @@
-// bf16 GEMM y = x W^T for projections with many rows (the image stream: M of several thousand), one
-// 256 x 256 (or 256 x 192) output tile per workgroup.
+// 16-bit GEMM y = x W^T for projections with many rows, for one problem or two of the same reduction length in one launch.
 //
-// Workgroup: 8 wavefronts, two per SIMD, laid out 4 (rows) x 2 (features); a wave owns 64 rows x 128 (96)
-// features = 2 x 4 (2 x 3) accumulators of v_mfma_f32_32x32x16_bf16 with W rows as the A operand, so a lane
-// ends up with one output row and 4 x 4 consecutive features per accumulator. Per reduction step of 64 a
-// wave reads 6 (5) fragments of 1 KB from LDS for every 8 (6) matrix instructions. (The kernel is a template
-// over the wave layout; a 2 x 2 layout of four waves with 128 x 128 corners would read a third less, but its
-// 256 accumulator registers fill the accumulation file exactly and the compiler's register allocation then
-// falls apart, so only the eight-wave layout is instantiated.)
+// Workgroup: 8 wavefronts, two per SIMD, on an output tile of BM x BN = 256 x 256 (or 128 x 256). The tile's rows are two
+// halves X0, X1 and its features two halves W0, W1; a wavefront (2 along the rows x 4 along the features) owns a quarter of
+// each of the four quadrants, as v_mfma_f32_16x16x32 accumulators with W rows as the A operand.
 //
-// Tile movement: a step is a 256 x 64 piece of x and a 256 (192) x 64 piece of W, 128-byte rows, moved from
-// global memory straight into LDS by `buffer_load_dwordx4 ... lds` (one wave instruction fills 1 KB = 8
-// rows; the lane chooses WHAT it fetches: 16-byte chunk (l % 8) ^ ((row >> 1) & 7) of its row, which makes
-// the 16-byte fragment reads of 16 consecutive rows cover all 64 banks). Rows past the end of x or W read
-// as zeros through the buffer descriptor. Two LDS stages of 64 (56) KB.
+// Anti-phase. Wavefronts w and w + 4 share a SIMD. A reduction step of 64 is two phases, rows X0 and rows X1, and each phase
+// is a slot of LDS reads and tile loads followed by a slot of 32 matrix instructions. A barrier ends every slot and the second
+// four wavefronts run one slot behind the first four, so on every SIMD one wavefront multiplies while the other one reads: the
+// fragment reads (192 KB per step through an LDS that moves 128 bytes per cycle: 1536 cycles) and the tile loads (64 KB)
+// proceed beside the 2048 cycles of matrix work. The predecessor of this kernel ran its 8 wavefronts in one phase and took
+// one after the other: 1.08 to 1.14 PFLOP/s.
 //
-// Pipeline: ONE barrier per step, placed so that no wave ever waits for LDS behind it. Fragments are read
-// one k16 slice ahead of the matrix instructions that consume them, spread over those instructions. When a
-// wave has issued the reads of step i's last slice it waits for them (and for its own tile loads of step
-// i + 1), then meets the others at the barrier: behind it stage i is free and stage i + 1 is complete, so
-// the wave issues the first half of its loads of step i + 2 into stage i, the reads of step i + 1's first
-// slice, and only then the matrix instructions of step i's last slice, which cover the latency of both; the
-// second half of the loads goes out during the next slice.
+// Tile movement. A step is four units X0, X1, W0, W1 of 128 rows x 128 bytes, moved from global memory straight into LDS by
+// `buffer_load_dwordx4 ... lds` (one wave instruction fills 1 KB = 8 rows; the lane chooses WHAT it fetches, a 16-byte chunk
+// whose number is XORed with bits of the row, so that the 16-byte fragment reads of 16 rows cover all 64 banks). A unit is
+// read in one phase only and both groups of wavefronts have waited for their reads when that phase's slots end, so it is
+// refilled from the next phase on, with the data of two steps later: every load has three phases (about 3000 cycles) to
+// arrive, and a wavefront never waits for its last loads. The loads go out one by one between the fragment reads: in one
+// burst they queue up in front of the texture addresser (16 cycles per instruction) and hold the reads behind them up (N=8192,
+// K=8192, M=8192: 1.48 PFLOP/s in one burst, 1.55 between the reads; among the matrix instructions 1.43: they come too late).
 //
-// Workgroup order: ids are remapped so that the 32 workgroups resident on one XCD at a time form a block of
-// 8 row tiles x 4 feature tiles, i.e. fetch 8 pieces of x and 4 of W per step into that XCD's L2 instead of
-// 32 of each.
+// The workgroup is persistent and the stream of steps does not stop at a tile's end: the next tile's first units are on their
+// way while this tile's epilogue runs. Tiles are dealt out round by round. The tiles of a last round that would leave half or
+// more of the compute units without work are cut along the reduction instead, into 2 to 4 equal parts, and those run first.
+// Each part leaves its fp32 partial tile in scratch (write-through) and takes a ticket; behind the whole tiles the parts of a
+// tile share its four quadrants out between them and each adds up all partial tiles of its quadrants, in the order of the parts
+// (the sum does not depend on who arrives when), and runs their epilogue. A part that does not find the others arrived after a
+// bounded number of looks leaves, and the last to arrive takes what is left: nobody waits for anybody without a bound. (One
+// workgroup adding everything up took 8 us for each further part, 256 KB at a time; so does it 16 for all.) Ticket words carry the
+// launch's epoch (see gemm_bf16.hip).
 //
-// Epilogue: accumulators go through LDS (fp32, 64 features at a time, 68 floats per row: the 16-byte writes
-// of 16 rows cover all banks) and leave as 16-byte pieces of 8 features, whole 128-byte lines per row; bias,
-// activation, gate and residual are applied on the way out (gemm_epilogue.h).
+// Epilogue: W rows are assigned to accumulators so that a lane ends up with 8 consecutive features of one output row, stored
+// as 16 bytes from registers; bias, GELU(tanh), gate and residual are applied on the way.
 //
-// What bounds it: LDS. A step of a 256 x 256 tile reads 192 KB of fragments and takes 64 KB of tile loads,
-// 256 KB through an LDS that moves 128 bytes per cycle, against 2048 cycles of matrix work per SIMD at the
-// nominal rate: 125 bytes per cycle, nothing left. Measured at M = 8192, cold weights (us, this kernel /
-// hipBLASLt's best): N = 12288, K = 3072 with GELU 574 / 449; N = 9216, K = 3072 431 / 434; N = 3072,
-// K = 3072 gated 142 / 118; N = 3072, K = 12288 gated 637 / 427. Timing-only builds on the first problem
-// (ODIT_TILE_ABLATE): matrix instructions alone 390, plus fragment reads 483, plus tile loads instead 517,
-// tile loads and barrier without any matrix instruction 495 - the two kinds of LDS traffic add up instead of
-// hiding behind the matrix pipe. The library's kernel for the same tile runs four waves with 128 x 128 corners
-// (128 KB of fragment reads per step) at 76 % matrix-pipe busy against 56 % here. That layout was also built with
-// the 256 accumulators at fixed accumulation registers named in one-instruction inline assembly (no register
-// allocation problem left: 102 vector registers, no scratch, same results): 560 us with the tile loads going
-// through registers, 610 direct to LDS, and 405 us = 1.53 PFLOP/s with no tile traffic at all - the fetches from
-// L2, not LDS and not the matrix pipe, are what separates both layouts from the library.
+// What bounds it: the matrix pipe and the clock that the part holds under it. 8192 x 8192 x 8192 on random operands takes 1.35
+// us per step of 256 x 256 x 64 (1.59 PFLOP/s; hipBLASLt 1.60 on that card), 1.23 where one round runs. Measured with cold
+// weights, us, this kernel / its predecessor (256 x 256 or 256 x 192 tiles, 8 wavefronts in one phase) / the library's choice:
+// M=8192, N=12288, K=3072 with GELU 440 / 543 / 447; M=8192, N=9216, K=3072 349 / 402 / 437; M=2706, N=5120, K=5120 107 / 135 /
+// 117; M=2706, N=13824, K=5120 with GELU 297 / 399 / 319; M=1536, N=9216, K=3072 70 / 89 / 72. Around the loop a launch costs 6 us,
+// a tile's end 4 (7 with GELU: its arithmetic has no matrix work to hide behind).
 #include <type_traits>
 
 #include "gemm_epilogue.h"
-
-// Timing-only builds (wrong results): bit 0 = no tile loads in the main loop, 1 = no matrix instructions,
-// 2 = no barrier, 3 = tile loads never waited for, 4 = no fragment reads in the main loop.
-#ifndef ODIT_TILE_ABLATE
-#define ODIT_TILE_ABLATE 0
-#endif
-
 
 namespace odit {
 
 namespace {
 
-constexpr int kTileM = 256;                       // rows of x per tile
-constexpr int kTileK = 64;                        // reduction elements per step
-constexpr int kTileXBytes = kTileM * kTileK * 2;  // 32 KB per stage
-constexpr int kEpiPitch = 68;                     // floats per staged row of 64 features
-constexpr int kEpiBytes = kTileM * 2 * kEpiPitch * 4;  // 256 rows x two halves of the features, 64 at a time
+template <typename T> struct Mma16;
+template <> struct Mma16<bf16_t> {
+  using frag = bf16x8_v;
+  static __device__ __forceinline__ f32x4_v run(frag a, frag b, f32x4_v c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+  }
+};
+template <> struct Mma16<f16_t> {
+  using frag = f16x8_v;
+  static __device__ __forceinline__ f32x4_v run(frag a, frag b, f32x4_v c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+  }
+};
+
+constexpr int kTileN = 256;                      // features per tile
+constexpr int kTileK = 64;                       // reduction elements per step
+constexpr int kTileSlot = 256 * kTileN * 4;      // bytes of a partial tile
+static_assert(static_cast<size_t>(kTileSlot) * kGemmMaxWorkers + kGemmCounterBytes <= kGemmScratchBytes, "one slot per workgroup");
+
+struct TileProblem {
+  const void *x, *w;
+  // reduction steps from `k_split` on take their x from x2
+  const void* x2;
+  int M, N, k_split;
+  uint32_t ldx, ldx2, ldw;  // bytes
+  uint32_t x_bytes, x2_bytes, w_bytes;
+  int m_tiles, n_tiles;
+  GemmEpilogue ep;
+};
 
 struct TileParams {
-  const void *x, *w;
-  int M, N, K;
-  int64_t ldx, ldw;
-  GemmEpilogue ep;
-  uint32_t x_bytes, w_bytes;
-  int m_tiles, n_tiles, k_steps, group_m;
+  TileProblem q[2];
+  int tiles0, tiles;  // tiles of the first problem, of both
+  int whole;          // tiles that are not cut; the others are cut into `parts` along the reduction
+  int parts;
+  int k_steps;
+  unsigned long long* counters;  // one ticket word per cut tile, zero between launches
+  unsigned long long epoch;      // larger than that of any earlier launch of the process
+  char* slots;
 };
 
 typedef __attribute__((address_space(3))) void* lds_void_p;
 
-// NT: 32-feature accumulators per wave along the features (the tile is 64 NT features wide: two waves side by
-// side); WM: waves along the rows (4: eight waves of 64 rows, two per SIMD; 2: four waves of 128 rows, one per
-// SIMD with twice the accumulators, which reads a third less from LDS per matrix instruction).
-template <int NT, int WM>
-__global__ __launch_bounds__(WM * 2 * 64) __attribute__((amdgpu_waves_per_eu(WM / 2, WM / 2))) void gemm_bf16_tile_kernel(const TileParams p) {
-  using M = Mma<bf16_t>;
+// A wave-uniform number in a scalar register, where the compiler would not keep it by itself.
+__device__ __forceinline__ int scalar(int a) {
+  int s = __builtin_amdgcn_readfirstlane(a);
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm("" : "+s"(s));
+#endif
+  return s;
+}
+// a / b of wave-uniform numbers (the division runs on the vector unit, and what follows from its result would stay there, buffer
+// descriptors included)
+__device__ __forceinline__ int quotient(int a, int b) { return scalar(static_cast<int>(static_cast<unsigned>(a) / static_cast<unsigned>(b))); }
+
+constexpr int kThrough = 16;  // sc1 of a buffer access: past the XCD's L2, as an agent-scope store or load of a word goes
+// Ticket word of a cut tile: arrivals in bits 0 to 3, claimed quadrants 4 to 7, departures 8 to 11, the launch's epoch from 16 on
+constexpr unsigned long long kArrival = 1, kDeparture = 1 << 8;
+constexpr int kLooks = 64;    // looks for the other parts of a tile, about a microsecond each
+constexpr int kMaxParts = 4;
+
+// What the epilogue of a problem is to a tile with rows m0 .. m0 + BM - 1: 0 bias, 1 bias and GELU, 2 gate and residual, 3 the
+// same where gate vectors change inside the tile
+__device__ __forceinline__ int epilogue_kind(const GemmEpilogue& e, int m0, int bm) {
+  if (e.epilogue == ODIT_EPI_GATED_RESIDUAL || e.epilogue == ODIT_EPI_GATED_RESIDUAL_PRE) {
+    const int last = m0 + bm < e.M ? m0 + bm - 1 : e.M - 1;
+    return e.rows_per_gate > 0 && quotient(m0, e.rows_per_gate) != quotient(last, e.rows_per_gate) ? 3 : 2;
+  }
+  return e.epilogue == ODIT_EPI_GELU_TANH || e.epilogue == ODIT_EPI_BIAS_GELU_TANH ? 1 : 0;
+}
+
+// All loads have arrived, on every path: without it the compiler, which sees paths around the use of a loaded value, waits for
+// it where the register is written next, inside the main loop, and there for the tile loads in flight too (+25 % on a step).
+__device__ __forceinline__ void loads_arrived() { __builtin_amdgcn_s_waitcnt(0x0f70); }  // vmcnt(0)
+
+// This lane's part of a quadrant of a tile: 8 features from n on of the rows m, m + 16, ...
+template <typename T, int MH, int K>
+__device__ __forceinline__ void finish_quadrant(const GemmEpilogue& e, int m0, int m, int n, const f32x4_v (&v)[MH][2]) {
+  const bool in = n < e.N;
+  float gt[8], bs[8];
+  if constexpr (K != 3) gemm_epilogue_vectors8<T>(e, m0, in ? n : 0, gt, bs);
+  u32x4 res[MH];
+  if constexpr (K == 2) {
+#pragma unroll
+    for (int i = 0; i < MH; ++i) {
+      const int row = m + i * 16 < e.M ? m + i * 16 : e.M - 1;
+      res[i] = load_raw(static_cast<const T*>(e.residual) + row * e.ldr + (in ? n : 0));
+    }
+  }
+  loads_arrived();
+#pragma unroll
+  for (int i = 0; i < MH; ++i) {
+    float y[8];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      y[u] = v[i][0][u];
+      y[4 + u] = v[i][1][u];
+    }
+    const bool store = in && m + i * 16 < e.M;
+    if constexpr (K == 3) {
+      if (store) gemm_epilogue_store8<T>(e, m + i * 16, n, y);
+    } else {
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        if constexpr (K == 2) y[u] = fmaf(gt[u], y[u], bs[u]) + Raw<T>::get(res[i], u);
+        else y[u] += bs[u];
+        if constexpr (K == 1) y[u] = gemm_gelu_tanh(y[u]);
+      }
+      u32x4 o;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) Raw<T>::set2(o, u, y[2 * u], y[2 * u + 1]);
+      if (store) store_raw(static_cast<T*>(e.out) + (m + i * 16) * e.ldo + n, o);
+    }
+  }
+  if constexpr (K == 3) loads_arrived();
+}
+template <typename T, int MH>
+__device__ __forceinline__ void finish_quadrant(int kind, const GemmEpilogue& e, int m0, int m, int n, const f32x4_v (&v)[MH][2]) {
+  if (kind == 0) finish_quadrant<T, MH, 0>(e, m0, m, n, v);
+  else if (kind == 1) finish_quadrant<T, MH, 1>(e, m0, m, n, v);
+  else if (kind == 2) finish_quadrant<T, MH, 2>(e, m0, m, n, v);
+  else finish_quadrant<T, MH, 3>(e, m0, m, n, v);
+}
+
+// MH: 16-row accumulators of a wavefront in each half of the rows (4: 256-row tiles, 2: 128)
+template <typename T, int MH>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_tile_kernel(const TileParams p) {
+  using M = Mma16<T>;
   using frag = typename M::frag;
-  constexpr int kTileWaves = WM * 2;
-  constexpr int TM = 8 / WM;                  // 32-row accumulators per wave along the rows
-  constexpr int BN = 64 * NT;                 // features per tile
-  constexpr int WBytes = BN * kTileK * 2;
-  constexpr int Stage = kTileXBytes + WBytes;
-  constexpr int NInst = Stage / 1024;         // wave instructions per step (64 or 56)
-  constexpr int IPW = NInst / kTileWaves;     // per wavefront (8 or 7)
-  constexpr int XInst = kTileXBytes / 1024;   // the first 32 fill the x piece
-  constexpr int LdsBytes = 2 * Stage > kEpiBytes ? 2 * Stage : kEpiBytes;
-  static_assert(NInst % kTileWaves == 0, "tile loads must divide evenly over the wavefronts");
-  __shared__ __attribute__((aligned(1024))) char lds[LdsBytes];
+  constexpr int BM = 64 * MH, HM = 32 * MH;           // rows of a tile, of a half
+  constexpr int kXUnit = HM * 128, kWUnit = 128 * 128;
+  constexpr int kStage = 2 * (kXUnit + kWUnit);
+  constexpr int XJ = MH / 2, WJ = 2, PJ = XJ + WJ;    // tile-load instructions of a wavefront per unit, per phase
+  constexpr int NR = 2 * MH + 4;                      // fragment reads per phase
+  __shared__ __attribute__((aligned(1024))) char lds[2 * kStage + 64];
+  int* const flag = reinterpret_cast<int*>(lds + 2 * kStage);
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int l32 = lane & 31, hh = lane >> 5;
-  const int wm = wave % WM, wn = wave / WM;
-  const int lrow = lane >> 3, lpc = lane & 7;
+  const int wm = wave >> 2, wn = wave & 3;  // (wm is also the group: the second four wavefronts run a slot behind)
+  const int l16 = lane & 15, lq = lane >> 4;
+  const int G = gridDim.x;
+  const int v = xcd_remap(blockIdx.x, G);
+  const int nk = p.k_steps;
 
-  // tile of this workgroup: groups of group_m row tiles, feature tiles outer inside a group
-  int mt, nt;
-  {
-    const int L = xcd_remap(blockIdx.x, gridDim.x);
-    const int per_group = p.group_m * p.n_tiles;
-    const int g = L / per_group;
-    const int first_m = g * p.group_m;
-    const int gm = p.m_tiles - first_m < p.group_m ? p.m_tiles - first_m : p.group_m;
-    const int r = L - g * per_group;
-    nt = r / gm;
-    mt = first_m + (r - nt * gm);
-  }
-  const int m0 = mt * kTileM, n0 = nt * BN;
-
-  auto make_rsrc = [](const void* base, uint32_t bytes) {
+  auto make_rsrc = [](const void* base, uint32_t bytes) __attribute__((always_inline)) {
     const uint64_t a = reinterpret_cast<uint64_t>(base);
     u32x4_v r;
-    r.x = static_cast<uint32_t>(a); r.y = static_cast<uint32_t>(a >> 32) & 0xffffu; r.z = bytes; r.w = 0x00020000u;
+    r.x = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(a));
+    r.y = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(a >> 32) & 0xffffu);
+    r.z = __builtin_amdgcn_readfirstlane(bytes);
+    r.w = 0x00020000u;
     return r;
   };
-  const u32x4_v xrsrc = make_rsrc(p.x, p.x_bytes);
-  const u32x4_v wrsrc = make_rsrc(p.w, p.w_bytes);
 
-  // Instruction q = wave * IPW + i of a step fills LDS bytes [q KB, q KB + 1 KB) of the stage: rows
-  // 8 q' .. 8 q' + 7 of the x piece (q' = q < 32) or of the W piece (q' = q - 32). Lane l lands in row
-  // 8 q' + l / 8, physical chunk l % 8, and fetches logical chunk (l % 8) ^ ((row >> 1) & 7) with
-  // (row >> 1) & 7 = 4 (q' & 1) | (l / 8 >> 1): a per-lane row offset per operand plus a chunk offset whose
-  // bit 6 follows the parity of q'; the rest of the address (first row of the instruction, reduction step)
-  // is scalar.
-  const uint32_t ldx2 = static_cast<uint32_t>(p.ldx * 2), ldw2 = static_cast<uint32_t>(p.ldw * 2);
-  const uint32_t rowx = static_cast<uint32_t>(lrow) * ldx2, roww = static_cast<uint32_t>(lrow) * ldw2;
-  const uint32_t chunk0 = static_cast<uint32_t>((lpc ^ (lrow >> 1)) << 4);  // q' even; odd flips bit 6 (chunk ^ 4)
-  uint32_t srow[IPW];  // byte offset of each instruction's first row
+  // problem, first row and first feature of a tile: groups of 8 row tiles, feature tiles outer inside a group, so that the 32
+  // tiles an XCD runs at a time share 8 pieces of x and 4 of W
+  auto locate = [&](int tile, int& which, int& m0, int& n0) __attribute__((always_inline)) {
+    which = tile >= p.tiles0 ? 1 : 0;
+    const int t = which ? tile - p.tiles0 : tile;
+    const int mt = p.q[which].m_tiles, per = 8 * p.q[which].n_tiles;
+    const int g = quotient(t, per), first = g * 8, gm = mt - first < 8 ? mt - first : 8;
+    const int r = t - g * per, nt = quotient(r, gm);
+    m0 = (first + r - nt * gm) * BM;
+    n0 = nt * kTileN;
+  };
+  // The segments of this workgroup: its part of a cut tile, then whole tiles. A cursor is (part still to do, next whole tile).
+  const int cut = p.tiles - p.whole;
+  const bool has_part = v < cut * p.parts;
+  struct Cursor { bool part; int next; };
+  auto next_segment = [&](Cursor& c, int& tile, int& k0, int& k1) __attribute__((always_inline)) -> bool {
+    if (c.part) {
+      c.part = false;
+      const int part = quotient(v, cut);
+      tile = p.whole + v - part * cut;
+      k0 = quotient(part * nk, p.parts);
+      k1 = quotient((part + 1) * nk, p.parts);
+      return true;
+    }
+    if (c.next >= p.whole) return false;
+    tile = c.next;
+    c.next += G;
+    k0 = 0;
+    k1 = nk;
+    return true;
+  };
+
+  // ---- tile loads ----
+  // Instruction j of this wavefront's share of a unit fills rows (wave * J + j) * 8 .. + 7; lane l lands in row + l / 8, chunk
+  // l % 8, and fetches chunk (l % 8) ^ swizzle(row). Rows past the end re-read the last row: their products land in output
+  // rows and features that are never stored.
+  // (the lane's number is hidden from the compiler wherever a segment begins or ends: it would form what follows from it once in
+  // front of everything and keep it in registers that the main loop needs)
+  auto hidden_lane = [&]() __attribute__((always_inline)) {
+    int l = lane;
+    asm volatile("" : "+v"(l));
+    return l;
+  };
+  u32x4_v xr, wr;
+  uint32_t vx[2][XJ], vw[2][WJ];  // byte offsets of the lane's chunks (X0, X1; W0, W1)
+  constexpr int advance = kTileK * 2;
+  int kx = 0, kw = 0;             // byte offset of the step along x and W rows
+  int left = 0, rest = 0, pq = 0, pm0 = 0;  // steps until x changes its source or the segment ends; behind that
+  Cursor pc{has_part, v};
+  auto x_rows = [&](const void* x, uint32_t bytes, uint32_t ld, int last) __attribute__((always_inline)) {
+    xr = make_rsrc(x, bytes);
+    const int ln = hidden_lane(), lrow = ln >> 3, lch = ln & 7;
 #pragma unroll
-  for (int i = 0; i < IPW; ++i) {
-    const int q = wave * IPW + i;
-    const bool isx = q < XInst;
-    const int qq = isx ? q : q - XInst;
-    srow[i] = isx ? static_cast<uint32_t>(m0 + 8 * qq) * ldx2 : static_cast<uint32_t>(n0 + 8 * qq) * ldw2;
-  }
-  const int q0 = wave * IPW;
-
-  // instructions [i0, i1) of this wave's share of step kk's tile loads, into stage `stage`
-  auto issue = [&](int kk, int stage, int i0, int i1) {
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int j = 0; j < XJ; ++j) {
+        const int r = (wave * XJ + j) * 8 + lrow;
+        int row = pm0 + h * HM + r;
+        row = row < last ? row : last;
+        vx[h][j] = static_cast<uint32_t>(row) * ld + static_cast<uint32_t>((lch ^ ((r >> 1) & 7)) << 4);
+      }
+  };
+  auto fetch_from = [&]() __attribute__((always_inline)) {  // the next segment, or nowhere
+    int tile = 0, k0 = 0, k1 = 1 << 29, n0;
+    // (behind the last segment two more steps are fetched, which nobody uses: from the first row of x and of W, a few steps
+    // into which are in range whatever the row's length, as there are 8 rows or more)
+    const bool any = next_segment(pc, tile, k0, k1);
+    locate(tile, pq, pm0, n0);
+    const TileProblem& q = p.q[pq];
+    wr = make_rsrc(q.w, q.w_bytes);
+    const int ln = hidden_lane(), lrow = ln >> 3, lch = ln & 7;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int j = 0; j < WJ; ++j) {
+        const int r = (wave * WJ + j) * 8 + lrow, last = any ? q.N - 1 : 0;
+        int row = n0 + h * 128 + r;
+        row = row < last ? row : last;
+        vw[h][j] = static_cast<uint32_t>(row) * q.ldw + static_cast<uint32_t>((lch ^ (((r >> 1) & 1) | (((r >> 3) & 3) << 1))) << 4);
+      }
+    pq = scalar(pq);
+    pm0 = scalar(pm0);
+    kw = scalar(k0 * (kTileK * 2));
+    const bool far = k0 >= q.k_split;
+    x_rows(far ? q.x2 : q.x, far ? q.x2_bytes : q.x_bytes, far ? q.ldx2 : q.ldx, any ? q.M - 1 : 0);
+    kx = scalar((far ? k0 - q.k_split : k0) * (kTileK * 2));
+    rest = scalar(any && !far && k1 > q.k_split ? k1 - q.k_split : 0);
+    left = scalar(k1 - k0 - rest);
+  };
+  // the step behind the last one of the segment, or of a source of x
+  auto next_source = [&]() __attribute__((always_inline)) {
+    if (rest > 0) {
+      const TileProblem& q = p.q[pq];
+      x_rows(q.x2, q.x2_bytes, q.ldx2, q.M - 1);
+      kx = scalar(0);
+      kw = scalar(kw + advance);
+      left = scalar(rest);
+      rest = scalar(0);
+    } else {
+      fetch_from();
+    }
+  };
+  const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void_p)lds));
+  auto load = [&](uint32_t dst, uint32_t off, u32x4_v rs, int soff) __attribute__((always_inline)) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    const uint32_t kb = static_cast<uint32_t>(kk) * (kTileK * 2);
-    const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void_p)(lds + stage * Stage + q0 * 1024)));
-#pragma unroll
-    for (int i = 0; i < IPW; ++i) {
-      if (i < i0 || i >= i1) continue;
-      const int q = q0 + i;
-      const bool isx = q < XInst;  // wave-uniform
-      const int par = (isx ? q : q - XInst) & 1;
-      const uint32_t m0v = __builtin_amdgcn_readfirstlane(lds0 + i * 1024);
-      const uint32_t soff = __builtin_amdgcn_readfirstlane(srow[i] + kb);
-      const u32x4_v rs = isx ? xrsrc : wrsrc;
-      const uint32_t vo = (isx ? rowx : roww) + (chunk0 ^ static_cast<uint32_t>(par << 6));
-      // m0 (the LDS destination of the load) is a reserved register: naming it as clobbered draws a
-      // warning per expansion, and leaving it out would hide the write from the compiler
+    const uint32_t m0v = __builtin_amdgcn_readfirstlane(dst);
+    const int s = scalar(soff);
+    // m0 (the LDS destination of the load) is a reserved register: naming it as clobbered draws a
+    // warning per expansion, and leaving it out would hide the write from the compiler
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
-      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                   :
-                   : "s"(m0v), "v"(vo), "s"(rs), "s"(soff)
-                   : "memory", "m0");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                 :
+                 : "s"(m0v), "v"(off), "s"(rs), "s"(s)
+                 : "memory", "m0");
 #pragma clang diagnostic pop
-    }
 #endif
   };
+  auto load_x = [&](int stage, int h, int j) __attribute__((always_inline)) { load(lds0 + stage * kStage + h * kXUnit + (wave * XJ + j) * 1024, vx[h][j], xr, kx); };
+  auto load_w = [&](int stage, int h, int j) __attribute__((always_inline)) { load(lds0 + stage * kStage + 2 * kXUnit + h * kWUnit + (wave * WJ + j) * 1024, vw[h][j], wr, kw); };
 
-  f32x16_v acc[NT][TM];
-#pragma unroll
-  for (int tn = 0; tn < NT; ++tn)
-#pragma unroll
-    for (int tm = 0; tm < TM; ++tm)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[tn][tm][e] = 0.f;
-
-  // fragment (sub-tile t, k16 slice ks) of a piece: row 32 t + l32, logical chunk 2 ks + hh
-  const int frag_lane = l32 * 128 + ((hh ^ ((l32 >> 1) & 7)) << 4);
-  const int x_off = wm * (32 * TM * 128) + frag_lane;
-  const int w_off = kTileXBytes + wn * (32 * NT * 128) + frag_lane;
-
-  frag xf[2][TM], wf[2][NT];
-  auto fetch = [&](int stage, int ks, int set) {
-    if ((ODIT_TILE_ABLATE & 16) && (ks != 0 || stage != 0)) return;
-    const char* xb = lds + stage * Stage;
-#pragma unroll
-    for (int tm = 0; tm < TM; ++tm)
-      xf[set][tm] = __builtin_bit_cast(frag, *reinterpret_cast<const u32x4_v*>(xb + tm * (32 * 128) + (x_off ^ (ks * 32))));
-#pragma unroll
-    for (int tn = 0; tn < NT; ++tn)
-      wf[set][tn] = __builtin_bit_cast(frag, *reinterpret_cast<const u32x4_v*>(xb + tn * (32 * 128) + (w_off ^ (ks * 32))));
+  // ---- fragments ----
+  // x: rows (wave's first row of the half) + 16 m + l16, chunk 4 ks + lq. W: accumulator n of a half takes the features whose
+  // bit 2 is n out of the wavefront's 32, so that n = 0 and 1 together give a lane 8 consecutive ones.
+  const int xrow = wm * (16 * MH) + l16;
+  const int xa = xrow * 128 + ((lq ^ ((xrow >> 1) & 7)) << 4);
+  const int wrow = wn * 32 + ((l16 >> 2) << 3) + (l16 & 3);
+  const int wa = 2 * kXUnit + wrow * 128 + ((lq ^ (((wrow >> 1) & 1) | (((wrow >> 3) & 3) << 1))) << 4);
+  f32x4_v acc[2][2][MH][2];  // half of the rows, half of the features
+  frag xf[2][MH], w0[2][2], w0b[2][2], w1[2][2];
+  auto read_w = [&](int stage, int h, frag (&w)[2][2], int ks, int n) {
+    w[ks][n] = __builtin_bit_cast(frag, *reinterpret_cast<const u32x4_v*>(lds + stage * kStage + (wa ^ (ks * 64)) + h * kWUnit + n * 512));
   };
-  auto multiply = [&](int set) {
-    if (ODIT_TILE_ABLATE & 2) return;
-#pragma unroll
-    for (int tn = 0; tn < NT; ++tn)
-#pragma unroll
-      for (int tm = 0; tm < TM; ++tm) acc[tn][tm] = M::run(wf[set][tn], xf[set][tm], acc[tn][tm]);
+  auto read_x = [&](int stage, int h, int ks, int m) __attribute__((always_inline)) {
+    xf[ks][m] = __builtin_bit_cast(frag, *reinterpret_cast<const u32x4_v*>(lds + stage * kStage + (xa ^ (ks * 64)) + h * kXUnit + m * 2048));
   };
-
-  const int nk = p.k_steps;
-  // The reduction starts at a different step in every row tile and wraps around: the rows of x and W are a
-  // multiple of 4 KB apart for the usual reduction lengths, so at one reduction offset every row of a tile sits in
-  // the same memory channel, and workgroups that all stand at the same offset queue up in front of it. Row tiles
-  // 256 bytes (two steps) apart spread over the channels; the feature tiles of one row tile keep the same offset,
-  // so they still find each other's x pieces in L2. Worth 0 to 5 % (M = 8192, us without / with: N=9216 K=3072
-  // 430 / 406, N=3072 K=12288 630 / 613, N=12288 K=3072 567 / 568); what such strides really cost shows when the
-  // rows are padded by 128 bytes instead: 628 -> 509 us at K=12288, 536 -> 506 at K=3072 (hipBLASLt's kernels are
-  // indifferent to it). Sums are formed in the rotated order.
-  constexpr int kStagger = 32;
-  const int stagger = ((mt % kStagger) * 2) % nk;
-  auto wrapk = [&](int j) {   // reduction step of the j-th step this workgroup runs (j < nk + 3)
-    int t = j + stagger;
-    t = t >= nk ? t - nk : t;
-    return t >= nk ? t - nk : t;
-  };
-  // A step's tile loads go out in two halves, each spread over the matrix instructions of one k16 slice (the
-  // texture addresser takes a wave instruction every 16 cycles: issued faster, the loads fill its queue and the
-  // wave, which issues in order, stalls in front of its next matrix instruction): the first half of step i + 2
-  // right after the barrier that frees its stage (slice 3 of step i), the second half in slice 0 of step i + 1.
-  constexpr int H0 = (IPW + 1) / 2;  // instructions of the first half
-  auto issue_spread = [&](int kk, int stage, int i0, int i1, int part, int parts) {
-    const int n = i1 - i0, a = i0 + n * part / parts, b = i0 + n * (part + 1) / parts;
-    issue(kk, stage, a, b);
-  };
-  issue(wrapk(0), 0, 0, IPW);
-  if (nk > 1) {
-    issue(wrapk(1), 1, 0, H0);
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(H0) : "memory");
-  } else {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  }
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-  fetch(0, 0, 0);
-
-  // one reduction step on stage `stage` (compile-time): slices 0..2, the barrier, then slice 3 in the shadow of
-  // which the first fragment reads of step i + 1 are issued.
-  auto step = [&](int i, auto stage_c) {
-    constexpr int stage = decltype(stage_c)::value;
-    const bool next = i + 1 < nk, more = i + 2 < nk;
+  // A phase's reads (half h of the rows from `stage`, half wh of the features from `w_stage`) with its tile loads in between
+  auto reads = [&](int stage, int h, int w_stage, int wh, frag (&w)[2][2], auto&& load_number) {
 #pragma unroll
-    for (int ks = 0; ks < 3; ++ks) {
-      fetch(stage, ks + 1, (ks + 1) & 1);
-      if (ks == 0 && !(ODIT_TILE_ABLATE & 1)) {
-        // slice 0 carries the second half of step i + 1's tile loads, a few per group of matrix instructions
-#pragma unroll
-        for (int tn = 0; tn < NT; ++tn) {
-          if (next) issue_spread(wrapk(i + 1), stage ^ 1, H0, IPW, tn, NT);
-          if (!(ODIT_TILE_ABLATE & 2))
-#pragma unroll
-            for (int tm = 0; tm < TM; ++tm) acc[tn][tm] = M::run(wf[0][tn], xf[0][tm], acc[tn][tm]);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-        continue;
+    for (int r = 0; r < NR; ++r) {
+      const int ks = r / (NR / 2), i = r % (NR / 2);
+      // one W fragment, MH / 2 of x, and again
+      const int g = i / (1 + MH / 2), o = i % (1 + MH / 2);
+      if (o == 0) read_w(w_stage, wh, w, ks, g);
+      else read_x(stage, h, ks, g * (MH / 2) + o - 1);
+      if ((r + 1) * PJ / NR > r * PJ / NR) {
+        __builtin_amdgcn_sched_barrier(0);
+        load_number(r * PJ / NR);
+        __builtin_amdgcn_sched_barrier(0);
       }
-      multiply(ks & 1);
-      // the reads of the next slice are spread over the matrix instructions of this one: every wave of the
-      // workgroup is at the same point of its step, and a burst of reads from all of them queues up in LDS
-      constexpr int R = TM + NT, Q = TM * NT, per_read = Q / R;
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x008, per_read, 0);
-      }
-      __builtin_amdgcn_sched_group_barrier(0x008, Q - R * per_read, 0);
-      __builtin_amdgcn_sched_barrier(0);
     }
-    // the fragments of slice 3 are in registers, and this wave's loads of step i + 1 have landed ...
-    if (ODIT_TILE_ABLATE & 8) __builtin_amdgcn_s_waitcnt(0xc07f); else  // lgkmcnt(0) only
-    __builtin_amdgcn_s_waitcnt(0);
-    // ... in every wave: stage `stage` is free, stage `stage ^ 1` is complete
-    if (!(ODIT_TILE_ABLATE & 4)) __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    // (after the last step this reads a stage nobody has filled: the values are never used)
-    fetch(stage ^ 1, 0, 0);
+  };
+  auto barrier = [&]() __attribute__((always_inline)) {
     __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int tn = 0; tn < NT; ++tn) {
-      if (more && !(ODIT_TILE_ABLATE & 1)) issue_spread(wrapk(i + 2), stage, 0, H0, tn, NT);
-      if (!(ODIT_TILE_ABLATE & 2))
-#pragma unroll
-      for (int tm = 0; tm < TM; ++tm) acc[tn][tm] = M::run(wf[1][tn], xf[1][tm], acc[tn][tm]);
-      __builtin_amdgcn_sched_barrier(0);
-    }
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
   };
-  {
-    const std::integral_constant<int, 0> s0;
-    const std::integral_constant<int, 1> s1;
-    for (int i = 0; i < nk; i += 2) {
-      step(i, s0);
-      if (i + 1 < nk) step(i + 1, s1);
-    }
-  }
+  // this wavefront's reads are in registers, and its loads of all but the last two phases have landed
+  auto slot_wait = [&]() __attribute__((always_inline)) {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(2 * PJ) : "memory");
+  };
+  auto multiply = [&](int h, frag (&w0)[2][2]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int m = 0; m < MH; ++m)
+#pragma unroll
+          for (int n = 0; n < 2; ++n) acc[h][b][m][n] = M::run(b ? w1[ks][n] : w0[ks][n], xf[ks][m], acc[h][b][m][n]);
+  };
 
-  // ---- epilogue: 64 features of the wave's 64 x (32 NT) corner at a time through its own LDS region ----
-  // (every wave is past the last barrier, so no wave reads a stage any more)
-  constexpr int WR = 32 * TM;  // rows of the wave's corner
-  float* stg = reinterpret_cast<float*>(lds) + wave * (WR * kEpiPitch);
-  const int mw = m0 + wm * WR, nw = n0 + wn * (32 * NT);
+  // step 0 and all of step 1 that its first phases do not load, in the order of the main loop
+  fetch_from();
 #pragma unroll
-  for (int pass = 0; pass < (NT + 1) / 2; ++pass) {
-    constexpr int kFull = 2;
-    const int tn0 = pass * kFull;
-    const int ntn = NT - tn0 < kFull ? NT - tn0 : kFull;  // 32-feature accumulators in this pass
+  for (int j = 0; j < WJ; ++j) load_w(0, 0, j);
 #pragma unroll
-    for (int tn = 0; tn < NT; ++tn) {
-      if (tn / kFull != pass) continue;  // resolved at compile time: both loops are unrolled
-      const int t = tn % kFull;
+  for (int j = 0; j < XJ; ++j) load_x(0, 0, j);
 #pragma unroll
-      for (int tm = 0; tm < TM; ++tm)
+  for (int j = 0; j < WJ; ++j) load_w(0, 1, j);
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          f32x4_v q;
+  for (int j = 0; j < XJ; ++j) load_x(0, 1, j);
+  if (left > 1) {
+    left = scalar(left - 1);
+    kx = scalar(kx + advance);
+    kw = scalar(kw + advance);
+  } else {
+    next_source();
+  }
 #pragma unroll
-          for (int u = 0; u < 4; ++u) q[u] = acc[tn][tm][g * 4 + u];
-          *reinterpret_cast<f32x4_v*>(stg + (tm * 32 + l32) * kEpiPitch + t * 32 + g * 8 + hh * 4) = q;
+  for (int j = 0; j < WJ; ++j) load_w(1, 0, j);
+#pragma unroll
+  for (int j = 0; j < XJ; ++j) load_x(1, 0, j);
+#pragma unroll
+  for (int j = 0; j < WJ; ++j) load_w(1, 1, j);
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PJ) : "memory");
+  barrier();
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+    for (int n = 0; n < 2; ++n) read_w(0, 0, w0, ks, n);
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  barrier();  // W0 of step 0 is read: the first phase refills it
+
+  Cursor cc{has_part, v};
+  int tile, k0, k1;
+  bool more = next_segment(cc, tile, k0, k1);
+  int st = 0;  // stage of the step
+  while (more) {
+    if (wm == 1) barrier();  // a slot behind
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int m = 0; m < MH; ++m)
+#pragma unroll
+          for (int n = 0; n < 2; ++n) acc[h][b][m][n] = f32x4_v{0.f, 0.f, 0.f, 0.f};
+    // One step; `turn`: the loads leave their segment (or x its source) in the middle of it. Most steps do not, and their loop
+    // holds nothing but additions beside the reads, loads and matrix instructions.
+    auto step = [&](int stage, frag (&w0)[2][2], frag (&w0_next)[2][2], auto turn) __attribute__((always_inline)) {
+      // rows X0 of this step; loads: X1 of the next step, W0 of the one after
+      reads(stage, 0, stage, 1, w1, [&](int d) __attribute__((always_inline)) {
+        if (d < XJ) {
+          load_x(stage ^ 1, 1, d);
+        } else {
+          if (d == XJ) {
+            if constexpr (decltype(turn)::value) {
+              next_source();
+            } else {
+              kx = scalar(kx + advance);
+              kw = scalar(kw + advance);
+            }
+          }
+          load_w(stage, 0, d - XJ);
         }
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    const int cpr = 4 * ntn;  // 16-byte output pieces per row
-#pragma unroll 4
-    for (int it = 0; it < cpr * (WR / 64); ++it) {
-      const int idx = it * 64 + lane;
-      const int row = idx / cpr, ch = idx - row * cpr;
-      const int m = mw + row;
-      const int n = nw + tn0 * 32 + ch * 8;
-      const f32x4_v lo = *reinterpret_cast<const f32x4_v*>(stg + row * kEpiPitch + ch * 8);
-      const f32x4_v hi = *reinterpret_cast<const f32x4_v*>(stg + row * kEpiPitch + ch * 8 + 4);
-      if (m >= p.M || n >= p.N) continue;
-      float y[8];
+      });
+      slot_wait();
+      barrier();
+      multiply(0, w0);
+      barrier();
+      // rows X1 of this step and W0 of the next; loads: X0 and W1 of the one after
+      reads(stage, 1, stage ^ 1, 0, w0_next, [&](int d) __attribute__((always_inline)) {
+        if (d < XJ) load_x(stage, 0, d);
+        else load_w(stage, 1, d - XJ);
+      });
+      slot_wait();
+      barrier();
+      multiply(1, w0);
+      barrier();
+    };
+    auto one = [&](auto turn) __attribute__((always_inline)) {
+      step(st, w0, w0b, turn);
 #pragma unroll
-      for (int u = 0; u < 4; ++u) { y[u] = lo[u]; y[4 + u] = hi[u]; }
-      gemm_epilogue_store8<bf16_t>(p.ep, m, n, y);
+      for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+        for (int n = 0; n < 2; ++n) w0[ks][n] = w0b[ks][n];
+      st ^= 1;
+    };
+    for (int todo = k1 - k0; todo > 0;) {
+      int plain = scalar(todo < left - 1 ? todo : left - 1);
+      todo -= plain;
+      left = scalar(left - plain);
+      for (; plain > 1; plain -= 2) {  // W0 in two sets of registers by turns
+        step(st, w0, w0b, std::false_type{});
+        step(st ^ 1, w0b, w0, std::false_type{});
+      }
+      if (plain > 0) one(std::false_type{});
+      if (todo > 0) {
+        one(std::true_type{});
+        --todo;
+      }
     }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (wm == 0) barrier();  // both groups are here
+
+    if (k0 > 0 || k1 < nk) {
+      // A part of a cut tile: to its slot, and a ticket (the sums are formed behind the whole tiles). The address moves on in
+      // the scalar offset: a vector instruction right behind a 16-byte store must not write the store's data registers, the
+      // compiler takes a buffer store with a scalar offset for safe from that and put the next vector offset there, and
+      // accumulators of the last lanes went to memory with it now and then.
+      const auto slots = __builtin_amdgcn_make_buffer_rsrc(p.slots, 0, G * kTileSlot, 0x00020000);
+      const uint32_t off = static_cast<uint32_t>((wave * 64 + hidden_lane()) * 16);
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int i = 0; i < 2 * MH; ++i)
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_v, acc[h][b][i / 2][i % 2]), slots, off,
+                                                   scalar(v * kTileSlot + ((2 * h + b) * 2 * MH + i) * 8192), kThrough);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the partial tile has reached memory before the ticket is taken
+      __syncthreads();
+      if (tid == 0) {
+        unsigned long long* word = p.counters + (tile - p.whole);
+        // two atomics of one thread on one address: applied in program order
+        __hip_atomic_fetch_max(word, p.epoch << 16, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_fetch_add(word, kArrival, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+    } else {
+      int which, m0, n0;
+      locate(tile, which, m0, n0);
+      const GemmEpilogue& e = p.q[which].ep;
+      const int ln = hidden_lane(), kind = epilogue_kind(e, m0, BM);
+      const int m = m0 + wm * (16 * MH) + (ln & 15), n = n0 + wn * 32 + (ln >> 4) * 8;
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) finish_quadrant<T, MH>(kind, e, m0, m + h * HM, n + b * 128, acc[h][b]);
+    }
+    more = next_segment(cc, tile, k0, k1);
   }
+  if (has_part) {
+    // The parts of a tile share its four quadrants out between them: part i adds up and finishes quadrants i, i + parts, ... It
+    // looks for the others to have arrived, a bounded number of times; whoever arrived last certainly finds them all and takes
+    // what is left besides. A quadrant belongs to the one who claims it first.
+    const int part = quotient(v, cut), t = v - part * cut, parts = p.parts;
+    unsigned long long* word = p.counters + t;
+    const unsigned all = static_cast<unsigned>(parts);
+    int which, m0, n0;
+    locate(p.whole + t, which, m0, n0);
+    const GemmEpilogue& e = p.q[which].ep;
+    const int kind = epilogue_kind(e, m0, BM);
+    const auto slots = __builtin_amdgcn_make_buffer_rsrc(p.slots, 0, G * kTileSlot, 0x00020000);
+    unsigned mine = 0;
+    for (int i = part; i < 4; i += parts) mine |= 1u << i;
+    for (int round = 0; round < 2; ++round) {
+      // round 0: this part's own quadrants; round 1: those that nobody has claimed
+      if (tid == 0) {
+        unsigned got = 0;
+        for (int look = 0; look < (round == 0 ? kLooks : 1); ++look) {
+          const unsigned long long w = __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          if ((w & 15u) == all) {
+            const unsigned want = (round == 0 ? mine : 15u) & ~(static_cast<unsigned>(w >> 4) & 15u);
+            if (want != 0)
+              got = want & ~(static_cast<unsigned>(__hip_atomic_fetch_or(word, static_cast<unsigned long long>(want) << 4, __ATOMIC_RELAXED,
+                                                                         __HIP_MEMORY_SCOPE_AGENT) >> 4) & 15u);
+            break;
+          }
+          __builtin_amdgcn_s_sleep(8);
+        }
+        *reinterpret_cast<volatile unsigned*>(flag) = got;
+      }
+      __syncthreads();
+      unsigned got = __builtin_amdgcn_readfirstlane(*reinterpret_cast<volatile unsigned*>(flag));
+      __syncthreads();  // the flag is read before it is written again
+      for (; got != 0; got &= got - 1) {
+        const int quad = __builtin_ctz(got);
+        const int ln = hidden_lane();
+        const uint32_t off = static_cast<uint32_t>((wave * 64 + ln) * 16 + quad * (2 * MH * 8192));
+        f32x4_v sum[MH][2];
+        // all parts of the quadrant in one round trip, added in the order of the parts
+        auto add_up = [&](auto pc) __attribute__((always_inline)) {
+          constexpr int P = decltype(pc)::value;
+          f32x4_v r[P][2 * MH];
+#pragma unroll
+          for (int j = 0; j < P; ++j)
+#pragma unroll
+            for (int i = 0; i < 2 * MH; ++i)
+              r[j][i] = __builtin_bit_cast(f32x4_v, __builtin_amdgcn_raw_buffer_load_b128(slots, off + i * 8192, (t + j * cut) * kTileSlot, kThrough));
+#pragma unroll
+          for (int i = 0; i < 2 * MH; ++i) {
+            sum[i / 2][i % 2] = r[0][i];
+#pragma unroll
+            for (int j = 1; j < P; ++j) sum[i / 2][i % 2] += r[j][i];
+          }
+        };
+        if (parts == 2) add_up(std::integral_constant<int, 2>{});
+        else if (parts == 3) add_up(std::integral_constant<int, 3>{});
+        else add_up(std::integral_constant<int, 4>{});
+        finish_quadrant<T, MH>(kind, e, m0, m0 + (quad >> 1) * HM + wm * (16 * MH) + (ln & 15), n0 + (quad & 1) * 128 + wn * 32 + (ln >> 4) * 8, sum);
+      }
+    }
+    // the last to leave hands the word back at zero
+    if (tid == 0 && ((__hip_atomic_fetch_add(word, kDeparture, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >> 8) & 15u) + 1 == all)
+      __hip_atomic_store(word, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no load into LDS outlives the workgroup
 }
 
-#ifndef ODIT_TILE_WM
-#define ODIT_TILE_WM 4
-#endif
-#ifndef ODIT_TILE_NT
-#define ODIT_TILE_NT (ODIT_TILE_WM == 2 ? 3 : 0)
-#endif
-
-// 192-wide tiles when they fill the last round of workgroups better (N = 9216 or 3072 on 256 CUs)
-int tile_nt_for(int M, int N, int cus) {
-  if (ODIT_TILE_NT != 0) return ODIT_TILE_NT;
-  const int64_t mt = (M + kTileM - 1) / kTileM;
-  int best = 4;
-  int64_t best_cost = -1;
-  for (int nt : {4, 3}) {
-    const int64_t tiles = mt * ((N + 64 * nt - 1) / (64 * nt));
-    const int64_t cost = ((tiles + cus - 1) / cus) * nt;  // rounds x time of one tile
-    if (best_cost < 0 || cost < best_cost) { best_cost = cost; best = nt; }
-  }
-  return best;
-}
+int row_tiles(int M, int bm) { return (M + bm - 1) / bm; }
 
 }  // namespace
 
 bool gemm_tile_takes(const GemmCall& c, int dtype) {
-  if (dtype != ODIT_BF16) return false;
-  if (c.M < 1 || c.K % kTileK != 0 || c.N % 8 != 0) return false;
+  if (dtype != ODIT_BF16 && dtype != ODIT_F16) return false;
+  // (8 rows: what is fetched behind the last segment stays inside the operands)
+  if (c.M < 8 || c.K < kTileK || c.K % kTileK != 0 || c.N < 8 || c.N % 8 != 0) return false;
   if (c.ldx % 8 != 0 || c.ldw % 8 != 0 || c.ldo % 8 != 0) return false;
   if (!aligned16(c.x) || !aligned16(c.w) || !aligned16(c.out)) return false;
-  if (c.bias != nullptr && (reinterpret_cast<uintptr_t>(c.bias) & 15u) != 0) return false;
+  if (c.bias != nullptr && !aligned16(c.bias)) return false;
   const bool gated = c.epilogue == ODIT_EPI_GATED_RESIDUAL || c.epilogue == ODIT_EPI_GATED_RESIDUAL_PRE;
   if (gated) {
     if (c.residual == nullptr || c.ldr % 8 != 0 || !aligned16(c.residual)) return false;
     if (c.gate != nullptr && (!aligned16(c.gate) || c.ldg % 8 != 0)) return false;
     if (c.epilogue == ODIT_EPI_GATED_RESIDUAL_PRE && !c.gate_f32) return false;
   }
-  // 32-bit byte offsets, with room for the rows of a last, partly filled tile
-  const uint64_t xb = (static_cast<uint64_t>(c.M) + kTileM) * c.ldx * 2, wb = (static_cast<uint64_t>(c.N) + 256) * c.ldw * 2;
+  // 32-bit byte offsets
+  const uint64_t xb = (static_cast<uint64_t>(c.M - 1) * c.ldx + c.K) * 2, wb = (static_cast<uint64_t>(c.N - 1) * c.ldw + c.K) * 2;
   if (xb >= (1ull << 32) || wb >= (1ull << 32)) return false;
-  const int64_t tiles = static_cast<int64_t>((c.M + kTileM - 1) / kTileM) * ((c.N + 191) / 192);
-  return tiles < (1ll << 30);
+  return static_cast<int64_t>(row_tiles(c.M, 128)) * row_tiles(c.N, kTileN) < (1 << 28);
 }
 
-int gemm_tile_plan(int M, int N, int cus, int* tile_n, int* tiles) {
-  const int nt = tile_nt_for(M, N, cus > 0 ? cus : 256);
-  *tile_n = 64 * nt;
-  *tiles = ((M + kTileM - 1) / kTileM) * ((N + 64 * nt - 1) / (64 * nt));
-  return nt;
-}
-
-int launch_gemm_tile(const GemmCall& c, int cus, hipStream_t stream) {
-  TileParams p;
-  p.x = c.x; p.w = c.w;
-  p.M = c.M; p.N = c.N; p.K = c.K;
-  p.ldx = c.ldx; p.ldw = c.ldw;
-  p.ep = gemm_epilogue_of(c);
-  p.x_bytes = static_cast<uint32_t>((static_cast<uint64_t>(c.M - 1) * c.ldx + c.K) * 2);
-  p.w_bytes = static_cast<uint32_t>((static_cast<uint64_t>(c.N - 1) * c.ldw + c.K) * 2);
-  int tile_n = 0, tiles = 0;
-  const int nt = gemm_tile_plan(c.M, c.N, cus, &tile_n, &tiles);
-  p.m_tiles = (c.M + kTileM - 1) / kTileM;
-  p.n_tiles = (c.N + tile_n - 1) / tile_n;
-  p.k_steps = c.K / kTileK;
-  p.group_m = 8;
-  constexpr int WM = ODIT_TILE_WM;
-  if (nt == 4) {
-    hipLaunchKernelGGL((gemm_bf16_tile_kernel<4, WM>), dim3(tiles), dim3(WM * 2 * 64), 0, stream, p);
-  } else {
-    hipLaunchKernelGGL((gemm_bf16_tile_kernel<3, WM>), dim3(tiles), dim3(WM * 2 * 64), 0, stream, p);
+// Tile height, and whether and into how many parts the tiles of the last round are cut: by expected time, fitted to 170
+// launches of 256 to 9500 rows of the projections of widths 3072 and 5120 (5.6 %). A step takes 1.23 us on 256-row tiles in a
+// launch's first round, 1.45 in later ones (the clock falls), 1.31 where a round is cut, 0.80 on 128-row tiles; a launch 5.7, a
+// tile's end 3.9, 3 (2) more with GELU; parts 9 and 0.054 for each workgroup that leaves one (half of that for 128 rows), 11 more
+// behind whole tiles. M=1024, N=3072, K=12288: 256 rows in 4 parts 83 us, 2 parts 136, whole 236, 128 rows 99; M=512, N=3072,
+// K=3072: 36, 47, 70 and 29 (4 parts); M=2706, N=13824, K=5120: 3 parts 297, whole 341.
+TilePlan plan_gemm_tile(const GemmCall* c, int count, int cus, bool scratch) {
+  TilePlan best;
+  const int most = cus < kGemmMaxWorkers ? cus : kGemmMaxWorkers, nk = c[0].K / kTileK;
+  for (int bm = 256; bm >= 128; bm /= 2) {
+    const bool tall = bm == 256;
+    TilePlan p;
+    p.bm = bm;
+    p.tiles0 = row_tiles(c[0].M, bm) * row_tiles(c[0].N, kTileN);
+    p.tiles = p.tiles0 + (count > 1 ? row_tiles(c[1].M, bm) * row_tiles(c[1].N, kTileN) : 0);
+    const int rounds = p.tiles / most, rest = p.tiles - rounds * most;
+    float end = 3.9f;
+    for (int i = 0; i < count; ++i)
+      if (c[i].epilogue == ODIT_EPI_GELU_TANH || c[i].epilogue == ODIT_EPI_BIAS_GELU_TANH) end = tall ? 6.9f : 5.9f;
+    auto whole_rounds = [&](int n) { return n == 0 ? 0.f : n * (nk * (tall ? 1.45f : .8f) + end) - nk * (tall ? .22f : 0.f); };
+    for (int parts = 1; parts <= kMaxParts; ++parts) {
+      if (parts > 1 && (!scratch || rest == 0 || rest * parts > most || parts > nk)) break;
+      p.parts = parts;
+      p.whole = parts > 1 ? p.tiles - rest : p.tiles;
+      p.grid = rounds > 0 ? most : rest * parts;
+      if (parts == 1) {
+        p.us = 5.7f + whole_rounds(rounds + (rest > 0 ? 1 : 0));
+      } else {
+        p.us = 5.7f + whole_rounds(rounds) + (nk + parts - 1) / parts * (tall ? 1.31f : .8f) + 9.f + rest * parts * (tall ? .054f : .027f) +
+               (rounds > 0 ? 11.f : 0.f);
+      }
+      if (best.bm == 0 || p.us < best.us) best = p;
+    }
   }
+  return best;
+}
+
+int launch_gemm_tile(const GemmCall* c, int count, const TileX2* x2, int dtype, void* scratch, hipStream_t stream) {
+  const int cus = device_cus();
+  if (cus <= 0) { set_error("odit_linear: cannot read the device's compute-unit count"); return ODIT_ELAUNCH; }
+  const TilePlan plan = plan_gemm_tile(c, count, cus, scratch != nullptr);
+  TileParams p;
+  for (int i = 0; i < 2; ++i) {
+    const GemmCall& g = c[i < count ? i : 0];
+    TileProblem& q = p.q[i];
+    q.x = g.x; q.w = g.w; q.M = g.M; q.N = g.N;
+    q.ldx = static_cast<uint32_t>(g.ldx * 2); q.ldw = static_cast<uint32_t>(g.ldw * 2);
+    const int k1 = x2 ? x2->k_split : g.K;
+    q.x2 = x2 ? x2->x : g.x;
+    q.ldx2 = x2 ? static_cast<uint32_t>(x2->ldx * 2) : q.ldx;
+    q.k_split = k1 / kTileK;
+    q.x_bytes = static_cast<uint32_t>((static_cast<uint64_t>(g.M - 1) * g.ldx + k1) * 2);
+    q.x2_bytes = x2 ? static_cast<uint32_t>((static_cast<uint64_t>(g.M - 1) * x2->ldx + g.K - k1) * 2) : q.x_bytes;
+    q.w_bytes = static_cast<uint32_t>((static_cast<uint64_t>(g.N - 1) * g.ldw + g.K) * 2);
+    q.m_tiles = (g.M + plan.bm - 1) / plan.bm;
+    q.n_tiles = (g.N + kTileN - 1) / kTileN;
+    q.ep = gemm_epilogue_of(g);
+  }
+  p.tiles0 = plan.tiles0; p.tiles = plan.tiles; p.whole = plan.whole; p.parts = plan.parts;
+  p.k_steps = c[0].K / kTileK;
+  p.counters = static_cast<unsigned long long*>(scratch);
+  p.epoch = plan.parts > 1 ? next_ticket_epoch() : 0;
+  p.slots = scratch ? static_cast<char*>(scratch) + kGemmCounterBytes : nullptr;
+  const dim3 grid(plan.grid), block(512);
+#define ODIT_TILE(T)                                                                          \
+  do {                                                                                        \
+    if (plan.bm == 256) hipLaunchKernelGGL((gemm_tile_kernel<T, 4>), grid, block, 0, stream, p); \
+    else hipLaunchKernelGGL((gemm_tile_kernel<T, 2>), grid, block, 0, stream, p);              \
+  } while (0)
+  if (dtype == ODIT_BF16) ODIT_TILE(bf16_t);
+  else ODIT_TILE(f16_t);
+#undef ODIT_TILE
   return check_launch("odit_linear (tile kernel)");
 }
 

@@ -30,6 +30,43 @@ __device__ __forceinline__ float gemm_gelu_tanh(float x) {
   return __builtin_amdgcn_classf(rem, 0x198) ? fmaf(rem, r, q) : q;
 }
 
+// Features n .. n + 7 (n a multiple of 8, n < N) of what row m's accumulators y are combined with: y * gt + bs (+ the residual)
+// for the gated epilogues, y + bs for the others.
+template <typename T>
+__device__ __forceinline__ void gemm_epilogue_vectors8(const GemmEpilogue& p, int m, int n, float (&gt)[8], float (&bs)[8]) {
+  const T* bias_h = static_cast<const T*>(p.bias);
+  const float* bias_f = static_cast<const float*>(p.bias);
+  const bool gated = p.epilogue == ODIT_EPI_GATED_RESIDUAL || p.epilogue == ODIT_EPI_GATED_RESIDUAL_PRE;
+  const bool pre = p.epilogue == ODIT_EPI_GATED_RESIDUAL_PRE;
+#pragma unroll
+  for (int u = 0; u < 8; ++u) { gt[u] = 1.f; bs[u] = 0.f; }
+  const int64_t grow = gated && p.rows_per_gate > 0 ? static_cast<int64_t>(m / p.rows_per_gate) * p.ldg : 0;
+  if (gated && p.gate != nullptr) {
+    if (p.gate_f32) {
+      const float* gp = static_cast<const float*>(p.gate) + grow + n;
+      const f32x4_v g0 = *reinterpret_cast<const f32x4_v*>(gp), g1 = *reinterpret_cast<const f32x4_v*>(gp + 4);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) { gt[u] = g0[u]; gt[4 + u] = g1[u]; }
+    } else {
+      const u32x4 gv = load_raw(static_cast<const T*>(p.gate) + grow + n);
+#pragma unroll
+      for (int u = 0; u < 8; ++u) gt[u] = Raw<T>::get(gv, u);
+    }
+  }
+  if (p.bias != nullptr) {
+    if (pre) {  // float32, already multiplied by the gate, one vector per gate vector
+      const float* bp = bias_f + grow + n;
+      const f32x4_v b0 = *reinterpret_cast<const f32x4_v*>(bp), b1 = *reinterpret_cast<const f32x4_v*>(bp + 4);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) { bs[u] = b0[u]; bs[4 + u] = b1[u]; }
+    } else {
+      const u32x4 bv = load_raw(bias_h + n);
+#pragma unroll
+      for (int u = 0; u < 8; ++u) bs[u] = gated ? gt[u] * Raw<T>::get(bv, u) : Raw<T>::get(bv, u);
+    }
+  }
+}
+
 // y[0..8) = accumulators of row m, features n .. n + 7 (n a multiple of 8, m < M, n < N): applies the
 // epilogue and stores 16 bytes
 template <typename T>

@@ -3,8 +3,9 @@
 //   * out = residual + gate * (x W^T + bias)  (attention / MLP output projections: no separate
 //                                              gated-residual pass)
 // Which kernel runs is decided here per call. Few rows: the hand-written stream-K kernel (gemm_bf16.hip) where the reduction is
-// long, and for the two streams of a dual-stream block in one launch (odit_linear_pair). Many rows: hipBLASLt's MFMA kernels (or
-// the hand-written tile kernel, gemm_bf16_tile.hip, where asked for or tuned). For the library this file sets the problem up so
+// long. Many rows: the hand-written tile kernel (gemm_bf16_tile.hip) or hipBLASLt's MFMA kernels, by expected time. The two
+// streams of a dual-stream block: one launch of either hand-written kernel, or two calls, by expected time
+// (odit_linear_pair). For the library this file sets the problem up so
 // that its epilogue does the elementwise work (bias vector, activation, a per-output-feature alpha vector for the gate, beta = 1
 // on the residual), keeps problem descriptors per thread, chooses among the library's candidates for long reductions by expected
 // time, and has an explicit tuning call that times all engines for one problem and remembers the fastest.
@@ -64,6 +65,7 @@ struct LinPlan {
   size_t algo_ws = 0;
   bool have_algo = false;
   bool tuned = false;
+  float us = 0;  // expected time of a kernel that was ranked, 0: not known
 };
 
 // One hipBLASLt handle and one plan cache per host thread: plans are mutated per call (bias and
@@ -180,7 +182,8 @@ struct LinCall {
   void* ws;
   size_t ws_bytes;
   hipStream_t stream;
-  bool first = false;  // the library's first-ranked kernel, unless one was tuned (ODIT_LINEAR_FIRST)
+  bool first = false;    // the library's first-ranked kernel, unless one was tuned (ODIT_LINEAR_FIRST)
+  bool no_tile = false;  // untuned, not the tile kernel (ODIT_LINEAR_NO_TILE)
 };
 
 static bool lin_is_residual(const LinCall& c) {
@@ -195,24 +198,30 @@ static size_t lin_gate_bytes(const LinCall& c) {
   return lin_needs_prep(c) ? ((static_cast<size_t>(c.N) * 8 + 255) / 256) * 256 : 0;
 }
 
-static int lin_prepare(const LinCall& c, hipblasLtHandle_t* h, LinPlan** plan, const void** alpha_ptr,
-                       const void** c_ptr, void** lib_ws, size_t* lib_ws_bytes) {
+// the handle, and the plan of the problem (as many launches as there are groups of rows share it)
+static int lin_find_plan(const LinCall& c, hipblasLtHandle_t* h, LinPlan** plan) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) { set_error("odit_linear: hipGetDevice failed"); return ODIT_ELAUNCH; }
-  int rc = lin_handle(dev, h);
+  const int rc = lin_handle(dev, h);
   if (rc != ODIT_OK) return rc;
   const bool gated = lin_is_residual(c);
-  const bool prep = lin_needs_prep(c);
-  const bool alpha_vec = gated && c.gate != nullptr;
-  const bool has_bias = c.bias != nullptr;
-  LinKey key{dev, c.M, c.N, c.K, c.epilogue * 4 + (has_bias ? 1 : 0) + (alpha_vec ? 2 : 0), c.dtype, c.ldw, c.ldx,
+  LinKey key{dev, c.M, c.N, c.K, c.epilogue * 4 + (c.bias != nullptr ? 1 : 0) + (gated && c.gate != nullptr ? 2 : 0), c.dtype, c.ldw, c.ldx,
              gated ? c.ldr : c.ldo, c.ldo};
   if (c.first) {  // unless a tuning call has found this problem's fastest kernel: what it chose runs
     const auto it = g_lin.plans.find(key);
     if (it == g_lin.plans.end() || !it->second.tuned) key.epi |= 0x100;
   }
-  rc = lin_plan(key, plan);
+  return lin_plan(key, plan);
+}
+
+static int lin_prepare(const LinCall& c, hipblasLtHandle_t* h, LinPlan** plan, const void** alpha_ptr,
+                       const void** c_ptr, void** lib_ws, size_t* lib_ws_bytes) {
+  int rc = lin_find_plan(c, h, plan);
   if (rc != ODIT_OK) return rc;
+  const bool gated = lin_is_residual(c);
+  const bool prep = lin_needs_prep(c);
+  const bool alpha_vec = gated && c.gate != nullptr;
+  const bool has_bias = c.bias != nullptr;
   const size_t gb = lin_gate_bytes(c);
   if (gb > c.ws_bytes) {
     set_error("odit_linear: workspace of %zu bytes cannot hold the %zu bytes of gate vectors", c.ws_bytes, gb);
@@ -350,7 +359,14 @@ static int lin_default_algo(hipblasLtHandle_t h, LinPlan& p, const LinCall& c, s
   p.algo = res[best].algo;
   p.algo_ws = res[best].workspaceSize;
   p.have_algo = true;
+  p.us = static_cast<float>(best == 0 ? best_us / kLinRankGain : best_us);
   return ODIT_OK;
+}
+
+// the library's kernel for a plan that has none yet
+static int lin_choose_algo(hipblasLtHandle_t h, LinPlan& p, const LinCall& c, size_t lib_ws_bytes) {
+  if ((p.have_algo && p.algo_ws <= lib_ws_bytes) || lin_preferred_algo(h, p, c, lib_ws_bytes)) return ODIT_OK;
+  return lin_default_algo(h, p, c, lib_ws_bytes);
 }
 
 static int lin_check(const LinCall& c) {
@@ -402,10 +418,8 @@ static int lin_run_library(const odit::LinCall& c) {
   size_t lws_bytes;
   int rc = lin_prepare(c, &h, &p, &alpha, &cptr, &lws, &lws_bytes);
   if (rc != ODIT_OK) return rc;
-  if ((!p->have_algo || p->algo_ws > lws_bytes) && !lin_preferred_algo(h, *p, c, lws_bytes)) {
-    rc = lin_default_algo(h, *p, c, lws_bytes);
-    if (rc != ODIT_OK) return rc;
-  }
+  rc = lin_choose_algo(h, *p, c, lws_bytes);
+  if (rc != ODIT_OK) return rc;
   const float beta = lin_is_residual(c) ? 1.f : 0.f;
   ODIT_LT(hipblasLtMatmul(h, p->desc, alpha, c.w, p->a, c.x, p->b, &beta, cptr, p->c, c.out, p->d, &p->algo, lws,
                           lws_bytes, c.stream));
@@ -430,8 +444,8 @@ static odit::LinKey lin_engine_key(int dev, const odit::LinCall& c, int rows_per
                       c.dtype, rows_per_gate, c.ldx, c.ldw, c.ldo};
 }
 
-// Which hand-written kernel takes a problem: 1 = the stream-K kernel (few rows; needs its scratch), 2 = the
-// tile kernel (many rows), 0 = neither.
+// Which hand-written kernel takes a problem where one is asked for: 1 = the stream-K kernel (few rows; needs its scratch), 2 =
+// the tile kernel (many rows), 0 = neither.
 constexpr int kTileMinRows = 1025;
 static int lin_handwritten_kind(const odit::GemmCall& g, int dtype, const void* sk) {
   if (g.M >= kTileMinRows) return odit::gemm_tile_takes(g, dtype) ? 2 : 0;
@@ -440,23 +454,58 @@ static int lin_handwritten_kind(const odit::GemmCall& g, int dtype, const void* 
 
 static int lin_launch_handwritten(int kind, const odit::GemmCall& g, int dtype, void* sk, hipStream_t stream) {
   if (kind == 1) return odit::launch_gemm_streamk(&g, 1, dtype, sk, stream);
-  const int cus = odit::device_cus();
-  if (cus <= 0) { odit::set_error("odit_linear: cannot read the device's compute-unit count"); return ODIT_ELAUNCH; }
-  return odit::launch_gemm_tile(g, cus, stream);
+  return odit::launch_gemm_tile(&g, 1, nullptr, dtype, sk, stream);
 }
 
-// Without a tuning record: the stream-K kernel where the reduction is long against the number of output features (K >= 2 N:
-// the library's choices split K badly there: M=80, N=3072, K=12288 57 us against 31, M=512 69 against 52, M=1024 110
-// against 85) and there is work for all CUs; with a small product (N K < 2^22, a few MB of weights) its ranges would be
-// shorter than what handing partial tiles over costs (M=256, N=256, K=1024: 19 us against 10).
-static bool lin_prefers_handwritten(int dev, int kind, const odit::LinCall& c, int rows_per_gate) {
-  {
-    std::lock_guard<std::mutex> lock(odit::g_engine_mu);
-    const auto it = odit::g_handwritten_wins.find(lin_engine_key(dev, c, rows_per_gate));
-    if (it != odit::g_handwritten_wins.end()) return it->second;
+// What a tuning call found for a problem: 1 the hand-written kernel, 0 the library, -1 nothing was tuned.
+static int lin_tuned(int dev, const odit::LinCall& c, int rows_per_gate) {
+  std::lock_guard<std::mutex> lock(odit::g_engine_mu);
+  const auto it = odit::g_handwritten_wins.find(lin_engine_key(dev, c, rows_per_gate));
+  return it == odit::g_handwritten_wins.end() ? -1 : (it->second ? 1 : 0);
+}
+
+// Expected time (us) of one of the library's launches: that of its ranked kernel where it ranks them (long reductions), else 1.29
+// PFLOP/s behind 17 us; a long reduction takes 22 us more where it is split over few output tiles. Fitted to the launches that
+// the tile kernel's time is fitted to (11 %). Choosing by the two expected times takes 1 % longer over them than the better of
+// both would, the library alone 5 %.
+static float lin_library_us(const odit::LinCall& c, int M) {
+  using namespace odit;
+  if (M >= kLinRankMinRows && c.K >= kLinRankMinK && c.dtype != ODIT_F32) {
+    LinCall one = c;
+    one.M = M;
+    hipblasLtHandle_t h;
+    LinPlan* p;
+    const size_t gb = lin_gate_bytes(one);
+    if (gb <= one.ws_bytes && lin_find_plan(one, &h, &p) == ODIT_OK && lin_choose_algo(h, *p, one, one.ws ? one.ws_bytes - gb : 0) == ODIT_OK && p->us > 0)
+      return p->us;
   }
-  if (kind == 2) return false;
-  return c.K >= 2 * c.N && c.M >= 48 && static_cast<int64_t>(c.N) * c.K >= (1ll << 22);
+  const float us = 16.6f + 2e-9f * M * c.N * c.K / 1.286f;
+  return c.K >= 2 * c.N && static_cast<int64_t>(M) * c.N < 128 * 65536 ? us + 22.f : us;
+}
+static float lin_library_us(const odit::LinCall& c, const odit::GemmCall& g) {  // (a launch for each group of rows with a gate vector of its own)
+  if (g.rows_per_gate <= 0) return lin_library_us(c, g.M);
+  const int full = g.M / g.rows_per_gate, last = g.M % g.rows_per_gate;
+  return full * lin_library_us(c, g.rows_per_gate) + (last > 0 ? lin_library_us(c, last) : 0.f);
+}
+
+// The stream-K kernel for one problem: where the reduction is long against the number of output features (K >= 2 N: the
+// library's choices split K badly there: M=80, N=3072, K=12288 57 us against 31, M=512 69 against 52, M=1024 110 against 85) and
+// there is work for all CUs; with a small product (N K < 2^22, a few MB of weights) its ranges would be shorter than what
+// handing partial tiles over costs (M=256, N=256, K=1024: 19 us against 10).
+static bool lin_streamk_rule(const odit::GemmCall& g) {
+  return g.K >= 2 * g.N && g.M >= 48 && g.M < kTileMinRows && static_cast<int64_t>(g.N) * g.K >= (1ll << 22);
+}
+
+// The kernel of a problem that names no engine: what a tuning call found, else the stream-K kernel by its rule, else the tile
+// kernel where its expected time is below the library's (kTileMinAuto rows or more), else the library (0).
+constexpr int kTileMinAuto = 256;
+static int lin_auto_kind(int dev, const odit::LinCall& c, const odit::GemmCall& g, const void* sk) {
+  const int tuned = lin_tuned(dev, c, g.rows_per_gate);
+  if (tuned >= 0) return tuned == 1 ? lin_handwritten_kind(g, c.dtype, sk) : 0;
+  if (sk != nullptr && lin_streamk_rule(g) && odit::gemm_streamk_takes(g, c.dtype)) return 1;
+  if (c.no_tile || g.M < kTileMinAuto || !odit::gemm_tile_takes(g, c.dtype)) return 0;
+  const odit::TilePlan plan = odit::plan_gemm_tile(&g, 1, odit::device_cus(), sk != nullptr);
+  return plan.bm > 0 && plan.us < lin_library_us(c, g) ? 2 : 0;
 }
 
 extern "C" int odit_linear_prefer(int M, int N, int K, int dtype, int solution) {
@@ -480,15 +529,16 @@ extern "C" int odit_linear_rows(const void* x, const void* w, const void* bias, 
                                 int64_t gate_stride, unsigned flags, void* workspace, size_t workspace_bytes,
                                 void* stream) {
   using namespace odit;
-  ODIT_CHECK_ARG((flags & ~(ODIT_LINEAR_LIBRARY | ODIT_LINEAR_HANDWRITTEN | ODIT_LINEAR_FIRST)) == 0 &&
+  ODIT_CHECK_ARG((flags & ~(ODIT_LINEAR_LIBRARY | ODIT_LINEAR_HANDWRITTEN | ODIT_LINEAR_FIRST | ODIT_LINEAR_NO_TILE)) == 0 &&
                      (flags & (ODIT_LINEAR_LIBRARY | ODIT_LINEAR_HANDWRITTEN)) != (ODIT_LINEAR_LIBRARY | ODIT_LINEAR_HANDWRITTEN),
-                 "odit_linear_rows: flags may name one engine (ODIT_LINEAR_LIBRARY or ODIT_LINEAR_HANDWRITTEN) and ODIT_LINEAR_FIRST, got %#x", flags);
+                 "odit_linear_rows: flags may name one engine (ODIT_LINEAR_LIBRARY or ODIT_LINEAR_HANDWRITTEN), ODIT_LINEAR_FIRST and ODIT_LINEAR_NO_TILE, got %#x", flags);
   void *sk, *lib;
   size_t lib_bytes;
   lin_split_ws(workspace, workspace_bytes, &sk, &lib, &lib_bytes);
   LinCall c{x, w, bias, residual, gate, out, M, N, K, ldx, ldw, ldo, ldr, epilogue, gate_dtype, dtype,
             lib, lib_bytes, static_cast<hipStream_t>(stream)};
   c.first = (flags & ODIT_LINEAR_FIRST) != 0;
+  c.no_tile = c.first || (flags & ODIT_LINEAR_NO_TILE) != 0;
   int rc = lin_check(c);
   if (rc != ODIT_OK || M == 0) return rc;
   ODIT_CHECK_ARG(rows_per_gate >= 0 && (rows_per_gate == 0 || gate_stride >= 0),
@@ -496,17 +546,18 @@ extern "C" int odit_linear_rows(const void* x, const void* w, const void* bias, 
   const bool per_rows = lin_is_residual(c) && gate != nullptr && rows_per_gate > 0 && rows_per_gate < M;
   const int engine = lin_engine_of(flags);
   const GemmCall g = lin_gemm_call(c, per_rows ? rows_per_gate : 0, per_rows ? gate_stride : 0);
-  const int kind = lin_handwritten_kind(g, dtype, sk);
-  if (engine == 2 && kind == 0) {
-    set_error("odit_linear: no hand-written kernel takes this problem (M=%d N=%d K=%d, workspace %zu bytes)",
-              M, N, K, workspace_bytes);
-    return ODIT_ENOTSUP;
+  int dev = 0, kind = 0;
+  if (engine == 2) {
+    kind = lin_handwritten_kind(g, dtype, sk);
+    if (kind == 0) {
+      set_error("odit_linear: no hand-written kernel takes this problem (M=%d N=%d K=%d, workspace %zu bytes)",
+                M, N, K, workspace_bytes);
+      return ODIT_ENOTSUP;
+    }
+  } else if (engine == 0 && hipGetDevice(&dev) == hipSuccess) {
+    kind = lin_auto_kind(dev, c, g, sk);
   }
-  if (kind != 0 && engine != 1) {
-    int dev = 0;
-    if (engine == 2 || (hipGetDevice(&dev) == hipSuccess && lin_prefers_handwritten(dev, kind, c, g.rows_per_gate)))
-      return lin_launch_handwritten(kind, g, dtype, sk, c.stream);
-  }
+  if (kind != 0) return lin_launch_handwritten(kind, g, dtype, sk, c.stream);
   if (!per_rows) return lin_run_library(c);
   // the library's epilogue takes one gate vector per launch: one launch per group of rows
   const size_t esz = dtype == ODIT_F32 ? 4 : 2, gsz = gate_dtype == ODIT_F32 ? 4 : esz;
@@ -526,15 +577,16 @@ extern "C" int odit_linear_rows(const void* x, const void* w, const void* bias, 
   return ODIT_OK;
 }
 
-// Two problems in one launch, or two calls? The launch has one set of overheads for both, the weights of the second stream
-// behind those of the first and no gate per launch; the library has the faster main loop for many rows. Up to kPairTiles
-// tiles of 128 rows together the launch wins (us, launch / two library calls): 4 + 1 tiles QKV 42 / 70, out 24 / 36; 6 + 2
-// tiles QKV 69 / 86, MLP up 88 / 102, out 32 / 44. With gates that differ per batch entry the library needs a call per
-// entry, and for few rows a residual pass: kPairTilesGated. Those are at width 3072, where the lines were drawn. At other
-// widths C (QKV N = 3 C, MLP up 4 C, 6 + 1 tiles; gated MLP down, 16 + 4 tiles in two batch entries): 1024 19 / 23, 25 / 24,
-// 39 / 60; 2048 33 / 42, 42 / 48, 96 / 146; 4096 107 / 106, 151 / 126, 367 / 403; 5120 174 / 145, 232 / 206, 524 / 863: past
-// 3072 the QKV and MLP-up launches should end at 3 to 4 tiles. No dual-stream model here is that wide.
+// Two problems in one launch, or two calls? By expected time. One launch has one set of overheads for both, shares the tiles of
+// the last round out over all CUs and takes gates that differ per batch entry, for which the library needs a call per entry.
+// Measured at width 3072 (us, stream-K pair / tile kernel pair / two library calls): 512 + 80 rows QKV 48 / 53 / 68, MLP down 66
+// / 68 / 125; 1024 + 512 QKV 109 / 75 / 98, out 45 / 50 / 50, MLP up 150 / 118 / 117, down 129 / 112 / 169; 2048 + 342 QKV 163 /
+// 130 / 150, out 56 / 50 / 62, up 221 / 153 / 181, down 176 / 154 / 206; 9210 + 406 QKV - / 394 / 462, up - / 538 / 648. The
+// stream-K kernel's fit ends at kPairTiles tiles of 128 rows together, kPairTilesGated where the library would need a call
+// per entry: past them only the tile kernel is compared.
+// The tile kernel has to promise 6 %: the two estimates are off by that much.
 constexpr int kPairTiles = 8, kPairTilesGated = 20;
+constexpr float kPairGain = .94f;
 
 extern "C" int odit_linear_pair(const odit_linear_problem* q, int N, int K, int epilogue, int gate_dtype, int dtype, unsigned flags,
                                 void* workspace, size_t workspace_bytes, void* stream) {
@@ -545,23 +597,39 @@ extern "C" int odit_linear_pair(const odit_linear_problem* q, int N, int K, int 
   size_t lib_bytes;
   lin_split_ws(workspace, workspace_bytes, &sk, &lib, &lib_bytes);
   GemmCall g[2];
-  bool per_rows = false, takes = sk != nullptr && engine != 1;
-  int tiles = 0;
+  bool per_rows = false, streamk = sk != nullptr && engine != 1, tile = engine != 1, tuned = false;
+  int tiles = 0, dev = 0;
+  float two = 0;
+  if (hipGetDevice(&dev) != hipSuccess) { set_error("odit_linear_pair: hipGetDevice failed"); return ODIT_ELAUNCH; }
   for (int i = 0; i < 2; ++i) {
     const LinCall c{q[i].x, q[i].w, q[i].bias, q[i].residual, q[i].gate, q[i].out, q[i].M, N, K, q[i].ldx, q[i].ldw, q[i].ldo, q[i].ldr,
-                    epilogue, gate_dtype, dtype, workspace, workspace_bytes, static_cast<hipStream_t>(stream)};
+                    epilogue, gate_dtype, dtype, lib, lib_bytes, static_cast<hipStream_t>(stream)};
     const int rc = lin_check(c);
     if (rc != ODIT_OK) return rc;
     ODIT_CHECK_ARG(q[i].rows_per_gate >= 0 && q[i].gate_stride >= 0, "odit_linear_pair: rows_per_gate and gate_stride must not be negative");
     const bool rows = lin_is_residual(c) && q[i].gate != nullptr && q[i].rows_per_gate > 0 && q[i].rows_per_gate < q[i].M;
     g[i] = lin_gemm_call(c, rows ? q[i].rows_per_gate : 0, rows ? q[i].gate_stride : 0);
     per_rows = per_rows || rows;
-    takes = takes && q[i].M > 0 && gemm_streamk_takes(g[i], dtype);
+    streamk = streamk && q[i].M > 0 && gemm_streamk_takes(g[i], dtype);
+    tile = tile && q[i].M > 0 && gemm_tile_takes(g[i], dtype);
+    if (!streamk && !tile) return ODIT_ENOTSUP;
     tiles += (q[i].M + kGemmBM - 1) / kGemmBM;
+    tuned = tuned || lin_tuned(dev, c, g[i].rows_per_gate) >= 0;
+    const float own = lin_streamk_rule(g[i]) && sk != nullptr ? gemm_streamk_us(g[i].M, 0, N, K, device_cus()) : 0.f;
+    const float library = lin_library_us(c, g[i]);
+    two += own > 0.f && own < library ? own : library;
   }
-  if (!takes || (engine != 2 && (tiles > (per_rows ? kPairTilesGated : kPairTiles) || static_cast<int64_t>(N) * K < (1 << 14))))
-    return ODIT_ENOTSUP;  // (no message: the ordinary answer for large problems)
-  return launch_gemm_streamk(g, 2, dtype, sk, static_cast<hipStream_t>(stream));
+  const int cus = device_cus();
+  if (engine == 2) return streamk ? launch_gemm_streamk(g, 2, dtype, sk, static_cast<hipStream_t>(stream)) : ODIT_ENOTSUP;
+  if (static_cast<int64_t>(N) * K < (1 << 14)) return ODIT_ENOTSUP;
+  // (no message where the answer is ODIT_ENOTSUP: two calls are an ordinary answer; problems that were tuned go to what was found)
+  const bool small = streamk && tiles <= (per_rows ? kPairTilesGated : kPairTiles);
+  const TilePlan plan = tile && !tuned ? plan_gemm_tile(g, 2, cus, sk != nullptr) : TilePlan{};
+  const bool wide = plan.bm > 0 && plan.us < kPairGain * two;
+  if (small && !(wide && plan.us < gemm_streamk_us(g[0].M, g[1].M, N, K, cus)))
+    return launch_gemm_streamk(g, 2, dtype, sk, static_cast<hipStream_t>(stream));
+  if (!wide) return ODIT_ENOTSUP;
+  return launch_gemm_tile(g, 2, nullptr, dtype, sk, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int odit_linear_rows_plan(const void* x, const void* w, const void* bias, void* out, const void* residual,
@@ -583,8 +651,9 @@ extern "C" int odit_linear_rows_plan(const void* x, const void* w, const void* b
   const GemmCall g = lin_gemm_call(c, per_rows ? rows_per_gate : 0, per_rows ? gate_stride : 0);
   int dev = 0;
   (void)hipGetDevice(&dev);
-  const int kind = M > 0 ? lin_handwritten_kind(g, dtype, sk) : 0;
-  const bool own = kind != 0 && engine != 1 && (engine == 2 || lin_prefers_handwritten(dev, kind, c, g.rows_per_gate));
+  c.first = (flags & ODIT_LINEAR_FIRST) != 0;
+  c.no_tile = c.first || (flags & ODIT_LINEAR_NO_TILE) != 0;
+  const bool own = M > 0 && engine != 1 && (engine == 2 ? lin_handwritten_kind(g, dtype, sk) : lin_auto_kind(dev, c, g, sk)) != 0;
   *handwritten = own ? 1 : 0;
   *launches = M == 0 ? 0 : (own || !per_rows ? 1 : (M + rows_per_gate - 1) / rows_per_gate);
   if (!own && lin_needs_prep(c)) *launches *= 2;  // plus the [N]-sized gate-vector launch of the library form

@@ -35,6 +35,7 @@ from ._lib import (
     ODIT_FLAG_REF_ROUNDING,
     ODIT_LINEAR_HANDWRITTEN,
     ODIT_LINEAR_LIBRARY,
+    ODIT_LINEAR_NO_TILE,
     ODIT_NORM_HEAD,
     ODIT_NORM_NONE,
     ODIT_NORM_ROW,
@@ -690,14 +691,14 @@ def set_linear_autotune(iters: int) -> None:
         _FLUSH.clear()
 
 
-_LINEAR_ENGINES = {"auto": 0, "library": ODIT_LINEAR_LIBRARY, "handwritten": ODIT_LINEAR_HANDWRITTEN}
+_LINEAR_ENGINES = {"auto": 0, "library": ODIT_LINEAR_LIBRARY, "handwritten": ODIT_LINEAR_HANDWRITTEN, "no_tile": ODIT_LINEAR_NO_TILE}
 _LINEAR_ENGINE_FLAGS = 0
 
 
 def set_linear_engine(engine: str) -> None:
     """Which kernel later ``linear`` calls of this process ask for when they name none themselves: "auto" (a
     hand-written kernel where a tuning run found it faster or its default rule says so, the library
-    elsewhere), "library" (hipBLASLt always) or "handwritten" (the hand-written kernel for the row count
+    elsewhere), "no_tile" (the same without the tile kernel's rule), "library" (hipBLASLt always) or "handwritten" (the hand-written kernel for the row count
     always; problems it does not take raise). The choice travels with every call as a flag of
     ``odit_linear_rows``; the library keeps no switch. For measurements and tests."""
     global _LINEAR_ENGINE_FLAGS
@@ -794,8 +795,8 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = No
     ``tune_iters`` > 0 first times the library's kernels and the hand-written kernel for this problem
     (overwrites ``out``), keeps the faster for later calls and returns its time in microseconds instead
     of the result. ``plan_only`` launches nothing and returns (the hand-written kernel would run, number of
-    kernel launches the call would make). ``engine``: "auto", "library" or "handwritten" for this call
-    (default: what ``set_linear_engine`` chose).
+    kernel launches the call would make). ``engine``: "auto", "library", "handwritten" or "no_tile" (auto without the tile
+    kernel) for this call (default: what ``set_linear_engine`` chose).
     """
     if engine is not None and engine not in _LINEAR_ENGINES:
         raise ValueError(f"engine must be one of {sorted(_LINEAR_ENGINES)}")
