@@ -404,6 +404,21 @@ typedef struct odit_linear_problem {
 int odit_linear_pair(const odit_linear_problem problems[2], int N, int K, int epilogue, int gate_dtype, int dtype,
                      unsigned flags, void* workspace, size_t workspace_bytes, void* stream);
 
+/* Two projections that read the same rows, of widths N[0], N[1] and epilogues of their own (no residual), in one launch of the
+ * tile kernel: to_qkv beside proj_mlp of a single-stream block (flux_transformer.py:288-309), to_k beside to_v of a
+ * cross-attention (wan2_2_transformer.py:520-530). Fields as for odit_linear_pair; problems[0].x and problems[1].x may also
+ * differ. ODIT_ENOTSUP, with nothing launched, where two odit_linear_rows calls are the better way. */
+int odit_linear_fork(const odit_linear_problem problems[2], const int N[2], int K, const int epilogue[2], int dtype, unsigned flags,
+                     void* workspace, size_t workspace_bytes, void* stream);
+
+/* odit_linear_rows of rows that lie in two tensors, x [M,K] beside x2 [M,K2] (W is [N, K + K2]), as one reduction in one launch
+ * of the tile kernel: proj_out of a single-stream block without the concatenation (flux_transformer.py:303-309).
+ * ODIT_ENOTSUP, with nothing launched, where two calls that add up are the better way. */
+int odit_linear_join(const void* x, const void* x2, const void* w, const void* bias, void* out, const void* residual,
+                     const void* gate, int M, int N, int K, int K2, int64_t ldx, int64_t ldx2, int64_t ldw, int64_t ldo,
+                     int64_t ldr, int epilogue, int gate_dtype, int dtype, int rows_per_gate, int64_t gate_stride,
+                     unsigned flags, void* workspace, size_t workspace_bytes, void* stream);
+
 /* out = act(x) W^T + bias for up to 16 rows of x (bias may be NULL; silu_input: act = SiLU rounded to the tensor type, else
  * none): the timestep embedding, modulation and head-norm projections (qwen_image_transformer.py:159-181, 760-767, 1065), one
  * pass over the weights. ODIT_BF16 or ODIT_F16, K a multiple of 32, 16-byte aligned rows; ODIT_ENOTSUP for anything else, with

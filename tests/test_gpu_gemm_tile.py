@@ -178,3 +178,74 @@ def test_pair_of_tuned_problems_goes_to_what_was_found(kernels, gpu):
     assert _pair(lib, ws, q, N, K, 1, 0) == 0
     kernels.linear(ops[0][0], ops[0][1], ops[0][2], out=out[0], tune_iters=2)
     assert _pair(lib, ws, q, N, K, 1, 0) == -2  # ODIT_ENOTSUP
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N0,N1,K", [
+    (1536, 12288, 9216, 3072),  # two rounds of whole 256-row tiles
+    (1111, 5000, 4104, 1024),   # ragged rows and features of both
+    (512, 5120, 5120, 5120),    # tiles in parts, those of either problem
+])
+def test_tile_gemm_fork(kernels, gpu, dtype, M, N0, N1, K):
+    """One x, two weights of different widths, GELU on the first."""
+    from vllm_omni_amd import _lib
+
+    lib, code, C = _lib.load(), 0 if dtype == torch.bfloat16 else 1, _lib.C
+    ws = kernels._linear_scratch(gpu.index or 0, torch.cuda.current_stream().cuda_stream)
+    x, w0, b0, y0 = _mk(gpu, M, N0, K, dtype, 21)
+    _, w1, b1, _ = _mk(gpu, 8, N1, K, dtype, 22)
+    y1 = x.double() @ w1.double().t()
+    out = [torch.full((M, n), float("nan"), dtype=dtype, device=gpu) for n in (N0, N1)]
+    q = (_lib.LinearProblem * 2)()
+    for i, (w, b, n) in enumerate(((w0, b0, N0), (w1, b1, N1))):
+        q[i].x, q[i].w, q[i].bias, q[i].out, q[i].M = x.data_ptr(), w.data_ptr(), b.data_ptr(), out[i].data_ptr(), M
+        q[i].ldx, q[i].ldw, q[i].ldo = K, K, n
+
+    def run(flags):
+        return lib.odit_linear_fork(C.addressof(q), (C.c_int * 2)(N0, N1), K, (C.c_int * 2)(3, 1), code, flags, ws.data_ptr(), ws.numel(),
+                                    torch.cuda.current_stream().cuda_stream)
+
+    assert run(_lib.ODIT_LINEAR_LIBRARY) == run(_lib.ODIT_LINEAR_NO_TILE) == -2  # ODIT_ENOTSUP
+    _lib.check(run(0), "odit_linear_fork")
+    assert _rel(out[0], _gelu(y0 + b0.double())) < _BOUND[dtype] and _rel(out[1], y1 + b1.double()) < _BOUND[dtype]
+    first = [t.clone() for t in out]
+    for _ in range(3):
+        _lib.check(run(0), "odit_linear_fork")
+        assert all(torch.equal(a, b) for a, b in zip(first, out))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,S,N,K,K2", [
+    (1, 1536, 3072, 3072, 12288),  # 3 parts: the sources change inside a part
+    (2, 700, 3072, 3072, 12288),   # gate vectors change inside a tile
+    (1, 4608, 3072, 3072, 12288),  # a round of whole tiles
+    (1, 1100, 1032, 64, 8192),     # one step of the first source, ragged
+    (2, 640, 2048, 8192, 64),      # one step of the second
+])
+def test_tile_gemm_join(kernels, gpu, dtype, B, S, N, K, K2):
+    """Rows in two tensors as one reduction, gated, in place and not."""
+    from vllm_omni_amd import _lib
+
+    lib, code, M = _lib.load(), 0 if dtype == torch.bfloat16 else 1, B * S
+    ws = kernels._linear_scratch(gpu.index or 0, torch.cuda.current_stream().cuda_stream)
+    x, w, b, _ = _mk(gpu, M, N, K + K2, dtype, 31)
+    xa, xb = x[:, :K].contiguous(), x[:, K:].contiguous()
+    g = torch.Generator(device=gpu).manual_seed(32)
+    h, gate = torch.randn(M, N, device=gpu, generator=g).to(dtype), torch.randn(B, N, device=gpu, generator=g)
+    gb = gate * b.float()
+    rows = torch.arange(M, device=gpu) // S
+    want = h.double() + gate.double()[rows] * (x.double() @ w.double().t()) + gb.double()[rows]
+
+    def run(res, out, flags=0):
+        return lib.odit_linear_join(xa.data_ptr(), xb.data_ptr(), w.data_ptr(), gb.data_ptr(), out.data_ptr(), res.data_ptr(), gate.data_ptr(),
+                                    M, N, K, K2, K, K2, K + K2, N, N, 5, 2, code, S if B > 1 else 0, N, flags, ws.data_ptr(), ws.numel(),
+                                    torch.cuda.current_stream().cuda_stream)
+
+    out = torch.full_like(h, float("nan"))
+    assert run(h, out, _lib.ODIT_LINEAR_LIBRARY) == -2  # ODIT_ENOTSUP
+    _lib.check(run(h, out), "odit_linear_join")
+    assert _rel(out, want) < _BOUND[dtype]
+    for _ in range(3):
+        again = h.clone()
+        _lib.check(run(again, again), "odit_linear_join")
+        assert torch.equal(again, out)

@@ -105,6 +105,12 @@ _SIGNATURES = {
     ),
     "odit_linear_pair": (
         C.c_int, [C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_uint, C.c_void_p, C.c_size_t, C.c_void_p]),
+    "odit_linear_fork": (
+        C.c_int, [C.c_void_p, C.POINTER(C.c_int), C.c_int, C.POINTER(C.c_int), C.c_int, C.c_uint, C.c_void_p, C.c_size_t, C.c_void_p]),
+    "odit_linear_join": (
+        C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_int,
+                  C.c_int64, C.c_int64, C.c_int64, C.c_int64, C.c_int64, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int64, C.c_uint,
+                  C.c_void_p, C.c_size_t, C.c_void_p]),
     "odit_linear_few": (
         C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_int64, C.c_int64, C.c_int64,
                   C.c_int, C.c_int, C.c_void_p]),

@@ -499,6 +499,21 @@ static bool lin_streamk_rule(const odit::GemmCall& g) {
 // The kernel of a problem that names no engine: what a tuning call found, else the stream-K kernel by its rule, else the tile
 // kernel where its expected time is below the library's (kTileMinAuto rows or more), else the library (0).
 constexpr int kTileMinAuto = 256;
+
+// expected time of a problem's own call: the better of what it may run on
+static float lin_call_us(const odit::LinCall& c, const odit::GemmCall& g, bool scratch) {
+  float us = lin_library_us(c, g);
+  const int cus = odit::device_cus();
+  if (scratch && lin_streamk_rule(g) && odit::gemm_streamk_takes(g, c.dtype)) {
+    const float own = odit::gemm_streamk_us(g.M, 0, g.N, g.K, cus);
+    if (own > 0.f && own < us) us = own;
+  }
+  if (g.M >= kTileMinAuto && odit::gemm_tile_takes(g, c.dtype)) {
+    const odit::TilePlan plan = odit::plan_gemm_tile(&g, 1, cus, scratch);
+    if (plan.bm > 0 && plan.us < us) us = plan.us;
+  }
+  return us;
+}
 static int lin_auto_kind(int dev, const odit::LinCall& c, const odit::GemmCall& g, const void* sk) {
   const int tuned = lin_tuned(dev, c, g.rows_per_gate);
   if (tuned >= 0) return tuned == 1 ? lin_handwritten_kind(g, c.dtype, sk) : 0;
@@ -597,7 +612,8 @@ extern "C" int odit_linear_pair(const odit_linear_problem* q, int N, int K, int 
   size_t lib_bytes;
   lin_split_ws(workspace, workspace_bytes, &sk, &lib, &lib_bytes);
   GemmCall g[2];
-  bool per_rows = false, streamk = sk != nullptr && engine != 1, tile = engine != 1, tuned = false;
+  bool per_rows = false, streamk = sk != nullptr && engine != 1, tuned = false;
+  bool tile = engine != 1 && (flags & (ODIT_LINEAR_FIRST | ODIT_LINEAR_NO_TILE)) == 0;
   int tiles = 0, dev = 0;
   float two = 0;
   if (hipGetDevice(&dev) != hipSuccess) { set_error("odit_linear_pair: hipGetDevice failed"); return ODIT_ELAUNCH; }
@@ -615,9 +631,7 @@ extern "C" int odit_linear_pair(const odit_linear_problem* q, int N, int K, int 
     if (!streamk && !tile) return ODIT_ENOTSUP;
     tiles += (q[i].M + kGemmBM - 1) / kGemmBM;
     tuned = tuned || lin_tuned(dev, c, g[i].rows_per_gate) >= 0;
-    const float own = lin_streamk_rule(g[i]) && sk != nullptr ? gemm_streamk_us(g[i].M, 0, N, K, device_cus()) : 0.f;
-    const float library = lin_library_us(c, g[i]);
-    two += own > 0.f && own < library ? own : library;
+    two += lin_call_us(c, g[i], sk != nullptr);
   }
   const int cus = device_cus();
   if (engine == 2) return streamk ? launch_gemm_streamk(g, 2, dtype, sk, static_cast<hipStream_t>(stream)) : ODIT_ENOTSUP;
@@ -630,6 +644,73 @@ extern "C" int odit_linear_pair(const odit_linear_problem* q, int N, int K, int 
     return launch_gemm_streamk(g, 2, dtype, sk, static_cast<hipStream_t>(stream));
   if (!wide) return ODIT_ENOTSUP;
   return launch_gemm_tile(g, 2, nullptr, dtype, sk, static_cast<hipStream_t>(stream));
+}
+
+// Two projections that read the same rows, in one launch of the tile kernel or two calls, by expected time (2 % have to be
+// promised: where two calls would run this kernel too, its estimate is off by the same for both). What one launch
+// gains is full rounds (M=1536, N=9216 and 12288, K=3072: 504 tiles, 1.97 rounds, 150 us; 216 and 288 in two calls 194) and the
+// rows' pieces in L2 for both.
+constexpr float kOneLaunchGain = .98f;
+
+extern "C" int odit_linear_fork(const odit_linear_problem* q, const int* N, int K, const int* epilogue, int dtype, unsigned flags, void* workspace,
+                                size_t workspace_bytes, void* stream) {
+  using namespace odit;
+  ODIT_CHECK_ARG(q != nullptr && N != nullptr && epilogue != nullptr, "odit_linear_fork: null arguments");
+  void *sk, *lib;
+  size_t lib_bytes;
+  lin_split_ws(workspace, workspace_bytes, &sk, &lib, &lib_bytes);
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) { set_error("odit_linear_fork: hipGetDevice failed"); return ODIT_ELAUNCH; }
+  GemmCall g[2];
+  bool tile = lin_engine_of(flags) == 0 && (flags & (ODIT_LINEAR_FIRST | ODIT_LINEAR_NO_TILE)) == 0;
+  float two = 0;
+  for (int i = 0; i < 2; ++i) {
+    const LinCall c{q[i].x, q[i].w, q[i].bias, nullptr, nullptr, q[i].out, q[i].M, N[i], K, q[i].ldx, q[i].ldw, q[i].ldo, 0,
+                    epilogue[i], dtype, dtype, lib, lib_bytes, static_cast<hipStream_t>(stream)};
+    const int rc = lin_check(c);
+    if (rc != ODIT_OK) return rc;
+    ODIT_CHECK_ARG(!lin_is_residual(c), "odit_linear_fork: no residual");
+    g[i] = lin_gemm_call(c, 0, 0);
+    if (!tile || q[i].M < kTileMinAuto || !gemm_tile_takes(g[i], dtype) || lin_tuned(dev, c, 0) >= 0) return ODIT_ENOTSUP;
+    two += lin_call_us(c, g[i], sk != nullptr);
+  }
+  const TilePlan plan = plan_gemm_tile(g, 2, device_cus(), sk != nullptr);
+  if (plan.bm == 0 || plan.us >= kOneLaunchGain * two) return ODIT_ENOTSUP;
+  return launch_gemm_tile(g, 2, nullptr, dtype, sk, static_cast<hipStream_t>(stream));
+}
+
+// One projection of rows that lie in two tensors, in one reduction or as two products that add up, by expected time. One
+// reduction rounds once, and reads and writes the output once (M=1536, N=3072, K=12288 and 3072: 128 us, two calls 166).
+extern "C" int odit_linear_join(const void* x, const void* x2, const void* w, const void* bias, void* out, const void* residual, const void* gate,
+                                int M, int N, int K, int K2, int64_t ldx, int64_t ldx2, int64_t ldw, int64_t ldo, int64_t ldr, int epilogue,
+                                int gate_dtype, int dtype, int rows_per_gate, int64_t gate_stride, unsigned flags, void* workspace,
+                                size_t workspace_bytes, void* stream) {
+  using namespace odit;
+  void *sk, *lib;
+  size_t lib_bytes;
+  lin_split_ws(workspace, workspace_bytes, &sk, &lib, &lib_bytes);
+  const LinCall c{x, w, bias, residual, gate, out, M, N, K, ldx, ldw, ldo, ldr, epilogue, gate_dtype, dtype, lib, lib_bytes, static_cast<hipStream_t>(stream)};
+  const int rc = lin_check(c);
+  if (rc != ODIT_OK) return rc;
+  ODIT_CHECK_ARG(x2 != nullptr && K2 > 0 && ldx2 >= K2 && ldw >= K + K2, "odit_linear_join: bad second operand");
+  ODIT_CHECK_ARG(rows_per_gate >= 0 && gate_stride >= 0, "odit_linear_join: rows_per_gate and gate_stride must not be negative");
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) { set_error("odit_linear_join: hipGetDevice failed"); return ODIT_ELAUNCH; }
+  const bool rows = lin_is_residual(c) && gate != nullptr && rows_per_gate > 0 && rows_per_gate < M;
+  LinCall second = c, whole = c;
+  second.K = K2;
+  second.ldx = ldx2;
+  whole.K = K + K2;
+  const GemmCall g1 = lin_gemm_call(c, rows ? rows_per_gate : 0, rows ? gate_stride : 0), g2 = lin_gemm_call(second, g1.rows_per_gate, g1.ldg);
+  GemmCall g = lin_gemm_call(whole, g1.rows_per_gate, g1.ldg);
+  if (lin_engine_of(flags) != 0 || (flags & (ODIT_LINEAR_FIRST | ODIT_LINEAR_NO_TILE)) != 0 || M < kTileMinAuto || K % 64 != 0 || K2 % 64 != 0 ||
+      ldx2 % 8 != 0 || !aligned16(x2) || !gemm_tile_takes(g1, dtype) || !gemm_tile_takes(g2, dtype) || !gemm_tile_takes(g, dtype) ||
+      lin_tuned(dev, c, g1.rows_per_gate) >= 0 || lin_tuned(dev, second, g1.rows_per_gate) >= 0)
+    return ODIT_ENOTSUP;
+  const TilePlan plan = plan_gemm_tile(&g, 1, device_cus(), sk != nullptr);
+  if (plan.bm == 0 || plan.us >= kOneLaunchGain * (lin_call_us(c, g1, sk != nullptr) + lin_call_us(second, g2, sk != nullptr))) return ODIT_ENOTSUP;
+  const TileX2 other{x2, ldx2, K};
+  return launch_gemm_tile(&g, 1, &other, dtype, sk, c.stream);
 }
 
 extern "C" int odit_linear_rows_plan(const void* x, const void* w, const void* bias, void* out, const void* residual,

@@ -977,7 +977,7 @@ void project_pair(BlockCall& c, const void* const x[2], const Lin l[2], void* co
     for (int i = 0; i < 2; ++i)
       q[i] = {x[i], l[i].w, l[i].b, nullptr, nullptr, y[i], static_cast<int>(M[i]), 0, l[i].k, l[i].ldw, l[i].n, 0, 0};
     const int epi = gelu ? (l[0].b ? ODIT_EPI_BIAS_GELU_TANH : ODIT_EPI_GELU_TANH) : (l[0].b ? ODIT_EPI_BIAS : ODIT_EPI_NONE);
-    const int rc = odit_linear_pair(q, l[0].n, l[0].k, epi, c.dtype, c.dtype, c.engine & ODIT_LINEAR_LIBRARY, c.lin_ws.p, c.lin_ws.bytes, c.where.stream);
+    const int rc = odit_linear_pair(q, l[0].n, l[0].k, epi, c.dtype, c.dtype, c.engine & ~static_cast<unsigned>(ODIT_LINEAR_HANDWRITTEN), c.lin_ws.p, c.lin_ws.bytes, c.where.stream);
     if (rc != ODIT_ENOTSUP) { c.check(rc); return; }
   }
   for (int i = 0; i < 2; ++i) c.project(x[i], l[i], y[i], M[i], gelu);
@@ -993,7 +993,7 @@ bool project_gated_pair(BlockCall& c, const void* const x[2], const Lin l[2], co
     q[i] = {x[i], l[i].w, g[i].pre ? g[i].gbias : l[i].b, residual[i], g[i].gate, out[i], static_cast<int>(B * S[i]), B > 1 ? static_cast<int>(S[i]) : 0,
             l[i].k, l[i].ldw, l[i].n, l[i].n, g[i].stride};
   const int rc = odit_linear_pair(q, l[0].n, l[0].k, g[0].pre ? ODIT_EPI_GATED_RESIDUAL_PRE : ODIT_EPI_GATED_RESIDUAL, g[0].pre ? ODIT_F32 : g[0].code,
-                                  c.dtype, c.engine & ODIT_LINEAR_LIBRARY, c.lin_ws.p, c.lin_ws.bytes, c.where.stream);
+                                  c.dtype, c.engine & ~static_cast<unsigned>(ODIT_LINEAR_HANDWRITTEN), c.lin_ws.p, c.lin_ws.bytes, c.where.stream);
   if (rc == ODIT_ENOTSUP) return false;
   c.check(rc);
   return true;
@@ -1002,6 +1002,23 @@ bool project_gated_pair(BlockCall& c, const void* const x[2], const Lin l[2], co
 // One allocation for a block's intermediate tensors. What is dead before another part begins shares its memory: after
 // `mark`, every `rewind` starts laying out from there again, over what came since (all launches are on one stream). A Wan
 // block of 2 x 32760 rows and width 5120 takes 4.7 GB this way; with every part apart it took 7.2.
+// y[i] = x W[i]^T + b[i] for two projections of the same rows (GELU on the first where `gelu`): one launch where that is the better way
+void project_fork(BlockCall& c, const void* x, const Lin l[2], void* const y[2], int64_t M, bool gelu) {
+  if (c.rc != 0) return;
+  if (l[0].k == l[1].k) {
+    odit_linear_problem q[2];
+    int n[2], epi[2];
+    for (int i = 0; i < 2; ++i) {
+      q[i] = {x, l[i].w, l[i].b, nullptr, nullptr, y[i], static_cast<int>(M), 0, l[i].k, l[i].ldw, l[i].n, 0, 0};
+      n[i] = static_cast<int>(l[i].n);
+      epi[i] = gelu && i == 0 ? (l[i].b ? ODIT_EPI_BIAS_GELU_TANH : ODIT_EPI_GELU_TANH) : (l[i].b ? ODIT_EPI_BIAS : ODIT_EPI_NONE);
+    }
+    const int rc = odit_linear_fork(q, n, static_cast<int>(l[0].k), epi, c.dtype, c.engine, c.lin_ws.p, c.lin_ws.bytes, c.where.stream);
+    if (rc != ODIT_ENOTSUP) { c.check(rc); return; }
+  }
+  for (int i = 0; i < 2; ++i) c.project(x, l[i], y[i], M, gelu && i == 0);
+}
+
 struct Slab {
   Tensor t;
   size_t at = 0, marked = 0, size = 0;
@@ -1346,8 +1363,9 @@ PyObject* py_flux_single_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const char* mp = static_cast<const char*>(mod->data_ptr());
   c.check(odit_adaln_modulate(x->data_ptr(), nx, mp, mp + C * esz, nullptr, nullptr, nullptr, nullptr, nullptr, B, S, C, rs, rs, ms, 0,
                               static_cast<float>(eps), c.dtype, c.dtype, 0u, c.where.stream));
-  c.project(nx, up, u, B * S, true);
-  c.project(nx, qkv, q3, B * S, false);
+  const Lin both[2] = {up, qkv};
+  void* const into[2] = {u, q3};
+  project_fork(c, nx, both, into, B * S, true);
   const int64_t st[2] = {S * 3 * HD, 3 * HD};
   char* qp = static_cast<char*>(q3);
   if (c.rc == 0)
@@ -1359,7 +1377,8 @@ PyObject* py_flux_single_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
     c.check(odit_attn_fwd_ex(q, k, qp + 2 * HD * esz, nullptr, 0, o, nullptr, 0, nullptr, nullptr, B, S, S, H, H, D, ds, ds, vs, nullptr, ds, nullptr,
                              static_cast<float>(scale), c.dtype, attn_ws.p, attn_ws.bytes, c.where.stream));
   }
-  // gate * proj_out(cat([attention, mlp])) + x as two accumulating products over the two column ranges of the weight
+  // gate * proj_out(cat([attention, mlp])) + x: one reduction over both, or two accumulating products over the two column
+  // ranges of the weight
   Gate g;
   g.gate = gate->data_ptr();
   g.gbias = gbias->data_ptr();
@@ -1369,10 +1388,19 @@ PyObject* py_flux_single_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
   wm.w = static_cast<const char*>(down.w) + C * esz;
   wm.k = F;
   wa.k = C;
-  project_gated(c, u, wm, x->data_ptr(), out.data_ptr(), B, S, g, 0, nullptr, Gate());
-  const bool written = in_place && c.rc == 0;
-  g.gbias = nullptr;
-  project_gated(c, o, wa, out.data_ptr(), out.data_ptr(), B, S, g, 0, nullptr, Gate());
+  bool written = false;
+  const int joined = c.rc != 0 ? c.rc : odit_linear_join(o, u, down.w, g.gbias, out.data_ptr(), x->data_ptr(), g.gate, static_cast<int>(B * S),
+                                                         static_cast<int>(C), static_cast<int>(C), static_cast<int>(F), C, F, down.ldw, C, C,
+                                                         ODIT_EPI_GATED_RESIDUAL_PRE, ODIT_F32, c.dtype, B > 1 ? static_cast<int>(S) : 0, g.stride,
+                                                         c.engine, c.lin_ws.p, c.lin_ws.bytes, c.where.stream);
+  if (joined != ODIT_ENOTSUP) {
+    c.check(joined);
+  } else {
+    project_gated(c, u, wm, x->data_ptr(), out.data_ptr(), B, S, g, 0, nullptr, Gate());
+    written = in_place && c.rc == 0;
+    g.gbias = nullptr;
+    project_gated(c, o, wa, out.data_ptr(), out.data_ptr(), B, S, g, 0, nullptr, Gate());
+  }
   if (c.rc == 0 && c.dtype == ODIT_F16) out.clamp_(-65504, 65504);
   others_run.reset();
   if (c.rc != 0) return block_failed(c.rc, written);
@@ -1527,8 +1555,9 @@ PyObject* py_wan_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
     n2 = nx;
   }
   c.project(n2, q2, k, B * S, false);
-  c.project(ctx->data_ptr(), k2, kc, B * T, false);
-  c.project(ctx->data_ptr(), v2, vc, B * T, false);
+  const Lin kv[2] = {k2, v2};
+  void* const kv_out[2] = {kc, vc};
+  project_fork(c, ctx->data_ptr(), kv, kv_out, B * T, false);
   if (c.rc == 0)
     c.check(odit_qknorm_rope(k, nullptr, nullptr, q, nullptr, nullptr, nw[2], nullptr, nullptr, nullptr, B, S, H, D, 0, st1, 0, S,
                              static_cast<float>(eps_n[2]), ODIT_NORM_ROW, w_dtype, c.dtype, 0u, c.where.stream));
