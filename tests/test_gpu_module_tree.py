@@ -162,3 +162,29 @@ def test_parameters_written_through_data_are_used(gpu, monkeypatch, make, option
     bound = 2.0 ** -5   # both paths round at every operation (2^-9); the new values move the result by far more
     assert (native - stepwise).norm() <= bound * stepwise.norm()
     assert (native - before).norm() > 4 * bound * before.norm()
+
+
+def test_projection_with_a_hook_or_of_another_class_at_sizes_of_the_hand_written_kernels(gpu):
+    """What ``project`` hands to a hand-written GEMM is the projection of a plain Linear only (1536 x 9216 x 3072 goes to the tile kernel)."""
+    from vllm_omni_amd import kernels
+    from vllm_omni_amd.blocks.qwen_image import project
+
+    class Doubled(torch.nn.Linear):
+        def forward(self, x):
+            return 2 * super().forward(x)
+
+    M, N, K = 1536, 9216, 3072
+    g = torch.Generator(device=gpu).manual_seed(0)
+    x = torch.randn(M, K, device=gpu, generator=g).bfloat16()
+    lin, other = (cls(K, N, device=gpu, dtype=torch.bfloat16) for cls in (torch.nn.Linear, Doubled))
+    other.load_state_dict(lin.state_dict())
+    with torch.inference_mode():
+        assert kernels.linear(x, lin.weight, lin.bias, plan_only=True)[0]
+        plain = project(lin, x)
+        seen = []
+        handle = lin.register_forward_hook(lambda *a: seen.append(1))
+        hooked = project(lin, x)
+        handle.remove()
+        assert seen == [1]
+        assert ((hooked - plain).float().norm() / plain.float().norm()).item() < 2.0 ** -8
+        assert ((project(other, x) - 2 * plain).float().norm() / plain.float().norm()).item() < 2.0 ** -7

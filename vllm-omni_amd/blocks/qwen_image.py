@@ -105,10 +105,10 @@ class FeedForward(nn.Module):
 
 
 def project(lin: nn.Linear, x: torch.Tensor) -> torch.Tensor:
-    """lin(x) outside a native block. A bf16 projection that a hand-written GEMM kernel would run (the engine asked for, or
-    the one a tuning call found faster for this problem) goes through ``kernels.linear``; everything else through
-    torch's linear (hipBLASLt with the solution table tuned offline)."""
-    if (x.dtype == torch.bfloat16 and x.is_cuda and x.is_contiguous()
+    """lin(x) outside a native block. A bf16 projection that a hand-written GEMM kernel would run goes through
+    ``kernels.linear`` where ``lin`` is plain; everything else is called as it is (torch's linear: hipBLASLt with the solution
+    table tuned offline)."""
+    if (x.dtype == torch.bfloat16 and x.is_cuda and x.is_contiguous() and kernels.plain_module(lin, nn.Linear)
             and kernels.linear(x, lin.weight, lin.bias, plan_only=True)[0]):
         return kernels.linear(x, lin.weight, lin.bias)
     return lin(x)
