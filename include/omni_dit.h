@@ -318,12 +318,13 @@ int odit_silu(const void* x, void* out, int64_t n, int dtype, void* stream);
  *   RowParallelLinear followed by `h + gate * y`           qwen_image_transformer.py:794-795, 801, 806,
  *                                                          flux_transformer.py:288-309, wan2_2_transformer.py:661, 673
  * Engines. hipBLASLt's MFMA kernels (a plain dense GEMM), set up so that bias, activation, gate and
- * residual ride in that kernel's epilogue, and two hand-written MFMA kernels, bf16 or fp16 (K a multiple of 64, N a
+ * residual ride in that kernel's epilogue, and three hand-written MFMA kernels, bf16 or fp16 (K a multiple of 64, N a
  * multiple of 8, 16-byte aligned rows): a stream-K kernel for few rows (csrc/gemm_bf16.hip) and a tile kernel for many
  * (csrc/gemm_bf16_tile.hip: 256 x 256 or 128 x 256 output tiles, the last round's cut along the reduction where they are
- * few). Both take one gate vector per group of rows in a single launch (odit_linear_rows). Which runs: what a tuning call
- * found, else the stream-K kernel for 48 to 1024 rows and K >= 2 N, else the tile kernel (256 rows or more) or the library by
- * expected time; the `flags` of odit_linear_rows can force either side.
+ * few), and one for products that are small altogether (csrc/gemm_small.hip: 64 x 64 tiles). All take one gate vector per
+ * group of rows in a single launch (odit_linear_rows). Which runs: what a tuning call found, else the stream-K kernel for 48 to
+ * 1024 rows and K >= 2 N, else the small kernel where all its tiles have a place at once and K <= 1024, else the tile kernel (256
+ * rows or more) or the library by expected time; the `flags` of odit_linear_rows can force either side.
  *
  * x [M,K] (row stride ldx), W [N,K] (row stride ldw: torch's nn.Linear weight, or a column range of
  * one), bias [N] or NULL, out [M,N] (row stride ldo). Gated form: residual [M,N] (row stride ldr; may be

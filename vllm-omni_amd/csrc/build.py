@@ -46,6 +46,7 @@ UNITS: list[tuple[str, list[str], str]] = [
     ("step.hip", [], "step"),
     ("gemm_bf16.hip", [], "gemm_bf16"),
     ("gemm_bf16_tile.hip", [], "gemm_bf16_tile"),
+    ("gemm_small.hip", [], "gemm_small"),
 ]
 PROBE_UNITS: list[tuple[str, list[str], str]] = [("probe.hip", [], "probe")]
 

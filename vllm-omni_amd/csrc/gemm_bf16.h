@@ -70,4 +70,9 @@ TilePlan plan_gemm_tile(const GemmCall* c, int count, int cus, bool scratch);
 // one problem only.
 int launch_gemm_tile(const GemmCall* c, int count, const TileX2* x2, int dtype, void* scratch, hipStream_t stream);
 
+// ---- gemm_small.hip: 64 x 64 output tiles, for products that are small altogether -------
+// One problem, or two of the same N and K in one launch, which gemm_streamk_takes takes. No scratch.
+bool gemm_small_rule(const GemmCall* c, int count, int cus, int max_k);
+int launch_gemm_small(const GemmCall* c, int count, int dtype, hipStream_t stream);
+
 }  // namespace odit

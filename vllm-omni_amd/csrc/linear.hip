@@ -3,7 +3,7 @@
 //   * out = residual + gate * (x W^T + bias)  (attention / MLP output projections: no separate
 //                                              gated-residual pass)
 // Which kernel runs is decided here per call. Few rows: the hand-written stream-K kernel (gemm_bf16.hip) where the reduction is
-// long. Many rows: the hand-written tile kernel (gemm_bf16_tile.hip) or hipBLASLt's MFMA kernels, by expected time. The two
+// long, and a kernel for products that are small altogether (gemm_small.hip). Many rows: the hand-written tile kernel (gemm_bf16_tile.hip) or hipBLASLt's MFMA kernels, by expected time. The two
 // streams of a dual-stream block: one launch of either hand-written kernel, or two calls, by expected time
 // (odit_linear_pair). For the library this file sets the problem up so
 // that its epilogue does the elementwise work (bias vector, activation, a per-output-feature alpha vector for the gate, beta = 1
@@ -454,6 +454,7 @@ static int lin_handwritten_kind(const odit::GemmCall& g, int dtype, const void* 
 
 static int lin_launch_handwritten(int kind, const odit::GemmCall& g, int dtype, void* sk, hipStream_t stream) {
   if (kind == 1) return odit::launch_gemm_streamk(&g, 1, dtype, sk, stream);
+  if (kind == 3) return odit::launch_gemm_small(&g, 1, dtype, stream);
   return odit::launch_gemm_tile(&g, 1, nullptr, dtype, sk, stream);
 }
 
@@ -496,8 +497,11 @@ static bool lin_streamk_rule(const odit::GemmCall& g) {
   return g.K >= 2 * g.N && g.M >= 48 && g.M < kTileMinRows && static_cast<int64_t>(g.N) * g.K >= (1ll << 22);
 }
 
-// The kernel of a problem that names no engine: what a tuning call found, else the stream-K kernel by its rule, else the tile
-// kernel where its expected time is below the library's (kTileMinAuto rows or more), else the library (0).
+// The kernel of a problem that names no engine: what a tuning call found, else the stream-K kernel by its rule, else the kernel
+// for small products (3) by its rule, else the tile kernel where its expected time is below the library's (kTileMinAuto rows or
+// more), else the library (0). One launch of the library takes 8 to 10 us for any small product, the small kernel 4 to 7 up to
+// K = kSmallK; beside a second problem, whose launch it saves, up to kSmallPairK.
+constexpr int kSmallK = 1024, kSmallPairK = 2048;
 constexpr int kTileMinAuto = 256;
 
 // expected time of a problem's own call: the better of what it may run on
@@ -518,6 +522,7 @@ static int lin_auto_kind(int dev, const odit::LinCall& c, const odit::GemmCall& 
   const int tuned = lin_tuned(dev, c, g.rows_per_gate);
   if (tuned >= 0) return tuned == 1 ? lin_handwritten_kind(g, c.dtype, sk) : 0;
   if (sk != nullptr && lin_streamk_rule(g) && odit::gemm_streamk_takes(g, c.dtype)) return 1;
+  if (!c.no_tile && odit::gemm_streamk_takes(g, c.dtype) && odit::gemm_small_rule(&g, 1, odit::device_cus(), kSmallK)) return 3;
   if (c.no_tile || g.M < kTileMinAuto || !odit::gemm_tile_takes(g, c.dtype)) return 0;
   const odit::TilePlan plan = odit::plan_gemm_tile(&g, 1, odit::device_cus(), sk != nullptr);
   return plan.bm > 0 && plan.us < lin_library_us(c, g) ? 2 : 0;
@@ -612,13 +617,13 @@ extern "C" int odit_linear_pair(const odit_linear_problem* q, int N, int K, int 
   size_t lib_bytes;
   lin_split_ws(workspace, workspace_bytes, &sk, &lib, &lib_bytes);
   GemmCall g[2];
-  bool per_rows = false, streamk = sk != nullptr && engine != 1, tuned = false;
+  bool per_rows = false, takes = true, streamk = sk != nullptr && engine != 1, tuned = false;
   bool tile = engine != 1 && (flags & (ODIT_LINEAR_FIRST | ODIT_LINEAR_NO_TILE)) == 0;
   int tiles = 0, dev = 0;
-  float two = 0;
   if (hipGetDevice(&dev) != hipSuccess) { set_error("odit_linear_pair: hipGetDevice failed"); return ODIT_ELAUNCH; }
+  LinCall calls[2];
   for (int i = 0; i < 2; ++i) {
-    const LinCall c{q[i].x, q[i].w, q[i].bias, q[i].residual, q[i].gate, q[i].out, q[i].M, N, K, q[i].ldx, q[i].ldw, q[i].ldo, q[i].ldr,
+    const LinCall& c = calls[i] = LinCall{q[i].x, q[i].w, q[i].bias, q[i].residual, q[i].gate, q[i].out, q[i].M, N, K, q[i].ldx, q[i].ldw, q[i].ldo, q[i].ldr,
                     epilogue, gate_dtype, dtype, lib, lib_bytes, static_cast<hipStream_t>(stream)};
     const int rc = lin_check(c);
     if (rc != ODIT_OK) return rc;
@@ -626,20 +631,22 @@ extern "C" int odit_linear_pair(const odit_linear_problem* q, int N, int K, int 
     const bool rows = lin_is_residual(c) && q[i].gate != nullptr && q[i].rows_per_gate > 0 && q[i].rows_per_gate < q[i].M;
     g[i] = lin_gemm_call(c, rows ? q[i].rows_per_gate : 0, rows ? q[i].gate_stride : 0);
     per_rows = per_rows || rows;
-    streamk = streamk && q[i].M > 0 && gemm_streamk_takes(g[i], dtype);
+    takes = takes && q[i].M > 0 && gemm_streamk_takes(g[i], dtype);
+    streamk = streamk && takes;
     tile = tile && q[i].M > 0 && gemm_tile_takes(g[i], dtype);
-    if (!streamk && !tile) return ODIT_ENOTSUP;
+    if (engine == 1 || (!takes && !tile)) return ODIT_ENOTSUP;
     tiles += (q[i].M + kGemmBM - 1) / kGemmBM;
     tuned = tuned || lin_tuned(dev, c, g[i].rows_per_gate) >= 0;
-    two += lin_call_us(c, g[i], sk != nullptr);
   }
   const int cus = device_cus();
   if (engine == 2) return streamk ? launch_gemm_streamk(g, 2, dtype, sk, static_cast<hipStream_t>(stream)) : ODIT_ENOTSUP;
   if (static_cast<int64_t>(N) * K < (1 << 14)) return ODIT_ENOTSUP;
+  if (takes && !tuned && (flags & (ODIT_LINEAR_FIRST | ODIT_LINEAR_NO_TILE)) == 0 && engine == 0 && gemm_small_rule(g, 2, cus, kSmallPairK))
+    return launch_gemm_small(g, 2, dtype, static_cast<hipStream_t>(stream));
   // (no message where the answer is ODIT_ENOTSUP: two calls are an ordinary answer; problems that were tuned go to what was found)
   const bool small = streamk && tiles <= (per_rows ? kPairTilesGated : kPairTiles);
   const TilePlan plan = tile && !tuned ? plan_gemm_tile(g, 2, cus, sk != nullptr) : TilePlan{};
-  const bool wide = plan.bm > 0 && plan.us < kPairGain * two;
+  const bool wide = plan.bm > 0 && plan.us < kPairGain * (lin_call_us(calls[0], g[0], sk != nullptr) + lin_call_us(calls[1], g[1], sk != nullptr));
   if (small && !(wide && plan.us < gemm_streamk_us(g[0].M, g[1].M, N, K, cus)))
     return launch_gemm_streamk(g, 2, dtype, sk, static_cast<hipStream_t>(stream));
   if (!wide) return ODIT_ENOTSUP;
