@@ -604,9 +604,12 @@ extern "C" int odit_linear_rows(const void* x, const void* w, const void* bias, 
 // 130 / 150, out 56 / 50 / 62, up 221 / 153 / 181, down 176 / 154 / 206; 9210 + 406 QKV - / 394 / 462, up - / 538 / 648. The
 // stream-K kernel's fit ends at kPairTiles tiles of 128 rows together, kPairTilesGated where the library would need a call
 // per entry: past them only the tile kernel is compared.
-// The tile kernel has to promise 6 %: the two estimates are off by that much.
+// Two calls are put 3 % above the sum of their estimates (the second one's rows and weights are cold when it starts). Over 104
+// pairs of 267 to 8759 and 40 to 885 rows, all four products of a dual-stream block (ms): 15.95 by this rule, 15.86 by the better of
+// the three each time, 16.38 where the tile kernel had to promise 6 % (3 % of that between 3 and 6 %: 3024 + 642 MLP down 250 / 227,
+// 8652 + 217 553 / 507, 2048 + 342 QKV 150 / 130).
 constexpr int kPairTiles = 8, kPairTilesGated = 20;
-constexpr float kPairGain = .94f;
+constexpr float kPairGain = 1.03f;
 
 extern "C" int odit_linear_pair(const odit_linear_problem* q, int N, int K, int epilogue, int gate_dtype, int dtype, unsigned flags,
                                 void* workspace, size_t workspace_bytes, void* stream) {
