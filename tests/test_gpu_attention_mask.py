@@ -73,3 +73,30 @@ def test_padding_equals_shorter_keys_at_the_longest_word_table_and_past_it(gpu, 
     want = kernels.attn_fwd(q, k[:, :live].contiguous(), v[:, :live].contiguous(), 0.125)
     # the tiles behind the last key add exact zeros; the key-split of the launch may differ: one step of the type
     torch.testing.assert_close(o.float(), want.float(), rtol=2.0 ** -7, atol=2.0 ** -9)
+
+
+# A unit ends with its last tile that has a live key. 130 and 71 key tiles: the search for it goes over several windows of 64
+# tiles, empty ones among them; 8 heads x 700 queries: batch rows shared out over the XCDs; 16640 queries: a last round cut along the keys, whose
+# ranges may hold no live key; heads of 128 over 2048 keys and more: workgroups of eight wavefronts.
+@pytest.mark.parametrize("B,Sq,Sk,H,Hkv,D", [(6, 40, 8257, 2, 1, 64), (6, 300, 4500, 1, 1, 128), (6, 700, 1024, 8, 2, 64),
+                                             (1, 16640, 1100, 4, 4, 64), (6, 700, 2049, 8, 8, 128)])
+def test_units_end_with_their_last_live_tile(gpu, B, Sq, Sk, H, Hkv, D):
+    g = torch.Generator().manual_seed(Sk)
+    q = torch.randn(B, Sq, H, D, generator=g).bfloat16().cuda()
+    k, v = (torch.randn(B, Sk, Hkv, D, generator=g).bfloat16().cuda() for _ in range(2))
+    a = torch.arange(Sk)
+    n = (Sk + 63) // 64
+    some = torch.rand(n, generator=g) < 0.1
+    some[n // 2] = True
+    rows = [a >= Sk - 70, (a >= 64) & (a < 128 + 5), some[a // 64] & (a % 3 == 0), a == Sk // 2, a < 0, a // 64 != 1]
+    mask = torch.stack([rows[(Sk + i) % 6] for i in range(B)])
+    rep = H // Hkv
+    want, want_lse = _reference(q, k.repeat_interleave(rep, 2), v.repeat_interleave(rep, 2), mask, D ** -0.5)
+    tol = (2 * 0.5 * 2.0 ** -7 + 1e-3) * v.abs().max().item()  # as above
+    for ws in (True, False):
+        o, lse = kernels.attn_fwd(q, k, v, D ** -0.5, key_mask=mask.cuda(), return_lse=True, use_workspace=ws)
+        assert (o.double().cpu() - want).abs().max().item() <= tol
+        dead = ~mask.any(dim=1)
+        assert (o[dead.cuda()] == 0).all() and (lse[dead.cuda()] == float("-inf")).all()
+        if not dead.all():
+            assert (lse.double().cpu() - want_lse)[~dead].abs().max().item() <= 1e-3

@@ -29,6 +29,13 @@
 //   B=2 S=592 H=24 D=128   18.4 / 26.8 / 18.8   B=2 S=4352 H=24 D=64   279 / 505 / 289
 // (and 490 / 290 / 20.6 / 333 with a random mask, where every tile is mixed).
 // Past kMaskWords tiles, and in the persistent form, whose units change the batch row, the mask is read as bytes.
+// With the words a unit ends with the last tile that has a live key: the tiles behind it would add zero probabilities (and are not
+// read: a NaN among their values does not reach the rows). Together with spread_batch below, one batch row padded to 40 % of
+// the other's keys, us, f16, before / now, and the same with an all-true mask:
+//   B=2 S=1357 H=32 (8 of keys) D=64  60.1 / 43.0, 56.0 / 56.2    B=2 S=1195 H=24 D=128  45.8 / 36.4, 46.1 / 45.4
+//   B=2 S=4352 H=24 D=64              320 / 296, 298 / 299        B=2 S=4352 H=24 D=128  485 / 468, 473 / 474
+// Passing over the dead tiles between live ones too, by a list of the live ones, cost 1 to 2 % of every masked launch in the tile
+// loop, and skipping those ahead of the first live one 0.3 us of a second copy of the first scores.
 //
 // Persistent form (MODE 2), a measurement aid that no default launch uses (ODIT_ATTN_PERSISTENT=1 in the
 // environment turns it on for launches of 4-wavefront workgroups, i.e. with ODIT_ATTN_WAVES=4 at head size 128). With more units than workgroup slots the launch has as many workgroups as run at
@@ -95,7 +102,7 @@ typedef __attribute__((address_space(3))) void* lds_void_p;
 //         tiles [jt0, n_tiles) of unit n_full + i / key_chunks and leaves an unnormalised partial
 //         result in scratch for attn_merge_kernel.
 // MODE 2: persistent, see above.
-// MODE 3, 4: 0 and 1 for a key mask held as words.
+// MODE 3, 4: 0 and 1 for a key mask held as words. MODE 5: 3 with the batch rows spread over the XCDs (spread_batch).
 // Separate instantiations, so the extra bookkeeping of one cannot disturb the register allocation of another (that of the
 // words in the launches without a mask: 452 -> 460 us at B=2 S=4352 H=24 D=128, 252 -> 262 at B=1 S=4608).
 constexpr int kMaskWords = 1024;  // 8 KB of LDS: two workgroups of D = 128 still fit a compute unit (144 of 160 KB)
@@ -104,7 +111,7 @@ template <typename T, int D, int NW, int MODE>
 __global__ __launch_bounds__(NW * 64, 8 / NW) void attn_fwd_dma_kernel(const AttnParams p) {
   constexpr bool TAIL = MODE == 1 || MODE == 4;
   constexpr bool PERSIST = MODE == 2;
-  constexpr bool WORDS = MODE == 3 || MODE == 4;
+  constexpr bool WORDS = MODE >= 3;
   using M = Mma<T>;
   using frag = typename M::frag;
   constexpr int BN = 64;
@@ -138,7 +145,7 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void attn_fwd_dma_kernel(const Att
   int next_pid = -1;
   __shared__ int next_unit_box;  // thread 0's draw, handed to the workgroup across a tile's barrier
   __shared__ uint64_t mask_words[WORDS ? kMaskWords : 1];  // of key tiles jt0, jt0 + 1, ...
-  if constexpr (MODE == 0 || MODE == 3) {
+  if constexpr (MODE == 0 || MODE == 3 || MODE == 5) {
     pid = xcd_remap(blockIdx.x, p.n_full);
   } else if constexpr (TAIL) {  // this workgroup covers key tiles [jt0, n_tiles) of unit pid (jt0 is even)
     pid = p.n_full + part / p.key_chunks;
@@ -162,6 +169,11 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void attn_fwd_dma_kernel(const Att
   int h = (pid / p.n_qblocks) % p.H;
   int b = (pid / p.n_qblocks) / p.H;
   int q0 = (pid % p.n_qblocks) * BM + wave * 32;
+  if constexpr (MODE == 5) {
+    h = blockIdx.x % kNumXcd * (p.H / kNumXcd) + blockIdx.y;
+    b = blockIdx.z;
+    q0 = blockIdx.x / kNumXcd * BM + wave * 32;
+  }
 
   // buffer descriptors end right after the last valid key row: later rows read as zeros
   const uint32_t k_bytes = static_cast<uint32_t>(((p.Sk - 1) * p.ks_s + D) * 2);
@@ -663,12 +675,26 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void attn_fwd_dma_kernel(const Att
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
   f32x16_v sa[2], sb[2];
+  uint64_t w = 0;
+  if constexpr (WORDS) w = jt0 + lane < n_tiles ? mask_words[lane] : 0;
   qk_plain(Kb, sa);
   {
     uint64_t word = 0;
     if constexpr (WORDS) word = mask_words[0];
     const float t = mask_and_max(jt0, mrow, word, sa);
     settle_max(fmaxf(t, __shfl_xor(t, 32, 64)));
+  }
+  if (WORDS && n_tiles - jt0 > 1) {
+    // the unit ends with its last tile that has a live key (the same in every wavefront); where none has, with the first
+    int end = jt0 + 1;
+    for (int base = jt0;;) {
+      const uint64_t live = __ballot(w != 0);
+      if (live != 0) end = base + 64 - __builtin_clzll(live);
+      base += 64;
+      if (base >= n_tiles) break;
+      w = base + lane < n_tiles ? mask_words[base + lane - jt0] : 0;
+    }
+    n_tiles = end;
   }
   // every wavefront has read the first K tile: the loop's first tile load overwrites it
   __syncthreads();
@@ -750,6 +776,14 @@ static int persistent_workgroups(int units, int n_tiles, int slots, int nw) {
   return W;
 }
 
+// Batch rows of a masked launch differ in their live tiles, and xcd_remap gives whole batch rows to some of the XCDs: those with
+// the longest row finish last (B=2, one row of 22 tiles and one of 9, 704 units: the XCDs 0 to 3 had 88 units of 22 tiles each). Where the heads divide evenly every XCD gets its share of each row's heads instead, as many in all (keys
+// and values are shared in its L2 as before), by a grid whose linear index runs over the XCDs first.
+// (With units for less than half the slots each has a compute unit, or nearly, to itself either way.)
+static bool spread_batch(const AttnParams& p, int slots) {
+  return p.B > 1 && p.B < 65536 && p.H % kNumXcd == 0 && p.n_full == p.total_blocks && 2 * p.total_blocks > slots;
+}
+
 template <typename T, int D, int NW>
 static int launch_dma(AttnParams& p, hipStream_t stream, void* ws, size_t ws_bytes) {
   constexpr int BM = NW * 32;
@@ -794,7 +828,9 @@ static int launch_dma(AttnParams& p, hipStream_t stream, void* ws, size_t ws_byt
       }
     }
     if (W == 0) {
-      if (words) hipLaunchKernelGGL((attn_fwd_dma_kernel<T, D, NW, 3>), dim3(p.n_full), dim3(NW * 64), 0, stream, p);
+      if (words && spread_batch(p, slots))
+        hipLaunchKernelGGL((attn_fwd_dma_kernel<T, D, NW, 5>), dim3(p.n_qblocks * kNumXcd, p.H / kNumXcd, p.B), dim3(NW * 64), 0, stream, p);
+      else if (words) hipLaunchKernelGGL((attn_fwd_dma_kernel<T, D, NW, 3>), dim3(p.n_full), dim3(NW * 64), 0, stream, p);
       else hipLaunchKernelGGL((attn_fwd_dma_kernel<T, D, NW, 0>), dim3(p.n_full), dim3(NW * 64), 0, stream, p);
     }
     rc = check_launch("odit_attn_fwd");
