@@ -338,9 +338,20 @@ int qknorm_rope_bf16(const QkArgs& a);
 int qknorm_rope_f16(const QkArgs& a);
 int qknorm_rope_f32(const QkArgs& a);
 
-template <typename T, typename TW, int NORM_MODE, bool GENERAL> static int qk_flat(const QkArgs& a) {
+template <typename T, typename TW, int NORM_MODE, bool GENERAL> static int qk_flat(const QkArgs& args) {
   constexpr int EPV = Vec16<T>::N;
-  const int vpr = a.HD / EPV;
+  QkArgs a = args;
+  int vpr = a.HD / EPV;
+  // One tensor only: its second half of heads takes the place of k. A lane then has two loads in flight behind one index computation
+  // and one fetch of cos and sin: rotary alone, f16, B=2 S=6032 H=24 D=128 30.0 -> 27.9 us (5.3 TB/s, a copy's rate), bf16 B=1
+  // S=16384 H=40 66.0 -> 58.1; without the tables the same time.
+  if (a.k_in == nullptr && a.v_in == nullptr && a.HD / a.D % 2 == 0) {
+    a.k_in = static_cast<const T*>(a.q_in) + a.HD / 2;
+    a.k_out = static_cast<T*>(a.q_out) + a.HD / 2;
+    a.wk = a.wq;
+    if (a.pair) { a.k_in2 = static_cast<const T*>(a.q_in2) + a.HD / 2; a.wk2 = a.wq2; }
+    vpr /= 2;
+  }
   QkFlatProblem<T, TW> p0, p1;
   p0.q_in = static_cast<const T*>(a.q_in); p0.k_in = static_cast<const T*>(a.k_in); p0.v_in = static_cast<const T*>(a.v_in);
   p0.wq = static_cast<const TW*>(a.wq); p0.wk = static_cast<const TW*>(a.wk);
