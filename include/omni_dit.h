@@ -435,7 +435,10 @@ int odit_linear_few(const void* x, const void* w, const void* bias, void* out, i
  *   [n_txt + n_img, sum(axes_dim) / 2], evaluated in float64 (flux.py:369-396); axes_dim is a host array of at most 4;
  * odit_cfg_combine: neg + scale * (pos - neg) over dense [rows, C], 16-bit types; `normalize`: every row brought back to the
  *   norm of pos (cfg_parallel.py:142-176); then C a multiple of 8 and 16-byte aligned tensors, else ODIT_ENOTSUP;
- * odit_euler_step: out = x + dt * v in float32 (pipeline schedulers' step). */
+ * odit_euler_step: out = x + dt * v in float32 (pipeline schedulers' step);
+ * odit_gate_rows: for the n gated output projections of a model's blocks, from stacked modulation parameters mods [B, n, 3C]
+ *   (dtype, 16-bit; rows dense, batch rows mods_batch_stride apart) and the projections' biases (n pointers on the host, [C] each):
+ *   float32 gates [B, n, C] = the last third of every triple and gated = gates * bias. */
 int odit_time_sinusoid(const void* t, void* out, int64_t n, int dim, float neg_log_period, float scale, float pre, int t_dtype,
                        int out_dtype, void* stream);
 int odit_rope_tables(const void* txt_ids, int64_t n_txt, const void* img_ids, int64_t n_img, float* cos_out, float* sin_out,
@@ -443,6 +446,8 @@ int odit_rope_tables(const void* txt_ids, int64_t n_txt, const void* img_ids, in
 int odit_cfg_combine(const void* pos, const void* neg, void* out, int64_t rows, int C, float scale, int normalize, int dtype,
                      void* stream);
 int odit_euler_step(const void* x, const void* v, void* out, int64_t n, float dt, int dtype, void* stream);
+int odit_gate_rows(const void* const* bias, int n, const void* mods, int64_t mods_batch_stride, int B, int C, float* gates,
+                   float* gated, int dtype, void* stream);
 
 /* Names the library kernel for plain projections of one problem (ODIT_EPI_BIAS, dense rows) ahead of time by the
  * library's own solution index, as an offline tuning run found it; process-wide, applies to problems first seen

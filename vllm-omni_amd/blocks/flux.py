@@ -468,31 +468,32 @@ class FluxTransformer2DModel(nn.Module):
         self._mod_weight, self._mod_bias = w_all, b_all
 
     def _gated_biases(self):
-        """float32 biases of the gated output projections, dual [L, 2 (hidden, context), 2, C] and single [Ls, C] (None where
-        there are no such blocks), read on every call: a kept copy would miss ``p.data.copy_``."""
+        """Biases of the gated output projections, of the dual-stream blocks (image attention and MLP, text attention and MLP) and of
+        the single-stream ones, read on every call: a kept copy would miss ``p.data.copy_``."""
         dual = [parameter_at(blk, *path) for blk in self.transformer_blocks
                 for path in (("attn", "to_out", "0", "bias"), ("ff", "net", "2", "bias"), ("attn", "to_add_out", "bias"),
                              ("ff_context", "net", "2", "bias"))]
-        single = [parameter_at(blk, "proj_out", "bias") for blk in self.single_transformer_blocks]
-        d = torch.stack(dual).detach().float().view(len(self.transformer_blocks), 2, 2, self.inner_dim) if dual else None
-        return d, torch.stack(single).detach().float() if single else None
+        return dual, [parameter_at(blk, "proj_out", "bias") for blk in self.single_transformer_blocks]
 
     def all_gate_rows(self, mods):
-        """float32 (gates, gates * biases) of every gated projection, four small ops per step and kind of block:
+        """float32 (gates, gates * biases) of every gated projection, one launch (or four small ops) per step and kind of block:
         dual [B, L, 2, 2, C] pairs and single [B, Ls, C] pairs (None where there are no such blocks)."""
         if mods is None or mods[0].dtype == torch.float32:
             return None, None
-        C = self.inner_dim
-        bias_dual, bias_single = self._gated_biases()
-        dual = single = None
-        if bias_dual is not None:
-            B, L = mods[0].shape[:2]
-            g = mods[0].view(B, L, 2, 2, 3 * C)[..., 2 * C:].float()
-            dual = (g, g * bias_dual)
-        if bias_single is not None:
-            g = mods[1][..., 2 * C:].float()
-            single = (g, g * bias_single)
-        return dual, single
+        C, B = self.inner_dim, mods[0].shape[0]
+
+        def pair(m, biases, shape):
+            if not biases:
+                return None
+            rows = kernels.gate_rows(m, biases)
+            if rows is not None:
+                return tuple(t.view(B, *shape) for t in rows)
+            g = m.view(B, *shape[:-1], 3 * C)[..., 2 * C:].float()
+            return g, g * torch.stack(biases).detach().float().view(shape)
+
+        dual, single = self._gated_biases()
+        return (pair(mods[0], dual, (len(self.transformer_blocks), 2, 2, C)),
+                pair(mods[1], single, (len(self.single_transformer_blocks), C)))
 
     def all_modulations(self, temb: torch.Tensor):
         """(dual [B, L, 2, 6C], single [B, Ls, 3C]) or None when not fused."""

@@ -592,23 +592,26 @@ class QwenImageTransformer2DModel(nn.Module):
                     lin.bias.data = b_all[i, j]
         self._mod_weight, self._mod_bias = w_all, b_all
 
-    def _gated_biases(self) -> torch.Tensor:
-        """float32 [L, 2 (img, txt), 2 (attention, MLP), C]: biases of the four gated output projections of every block, read
-        on every call: nothing a copy could be tagged with sees every way of writing a parameter (``p.data.copy_``
-        changes neither its version counter nor its address)."""
-        ps = [parameter_at(blk, *path) for blk in self.transformer_blocks
-              for path in (("attn", "to_out", "bias"), ("img_mlp", "net", "2", "bias"), ("attn", "to_add_out", "bias"),
-                           ("txt_mlp", "net", "2", "bias"))]
-        return torch.stack(ps).detach().float().view(len(self.transformer_blocks), 2, 2, self.inner_dim)
+    def _gated_biases(self) -> list:
+        """Biases of the four gated output projections of every block (image attention and MLP, text attention and MLP), read on
+        every call: nothing a copy could be tagged with sees every way of writing a parameter (``p.data.copy_`` changes
+        neither its version counter nor its address)."""
+        return [parameter_at(blk, *path) for blk in self.transformer_blocks
+                for path in (("attn", "to_out", "bias"), ("img_mlp", "net", "2", "bias"), ("attn", "to_add_out", "bias"),
+                             ("txt_mlp", "net", "2", "bias"))]
 
     def all_gate_rows(self, mods: torch.Tensor | None):
         """float32 (gates, gates * biases) [B, L, 2, 2, C] of the four gated projections of every block,
-        from the stacked modulation parameters: four small ops per step."""
+        from the stacked modulation parameters: one launch per step, or four small ops."""
         if mods is None or mods.dtype == torch.float32 or self.zero_cond_t:
             return None  # per-token gates of the editing variant do not fit one row per batch entry
         B, L, C = mods.shape[0], mods.shape[1], self.inner_dim
+        biases = self._gated_biases()
+        rows = kernels.gate_rows(mods, biases)
+        if rows is not None:
+            return tuple(t.view(B, L, 2, 2, C) for t in rows)
         gates = mods.view(B, L, 2, 2, 3 * C)[..., 2 * C:].float()
-        return gates, gates * self._gated_biases()
+        return gates, gates * torch.stack(biases).detach().float().view(L, 2, 2, C)
 
     def all_modulations(self, temb: torch.Tensor) -> torch.Tensor | None:
         """[B, L, 2, 6C] modulation parameters of every block, or None when not fused. For the editing

@@ -662,6 +662,38 @@ PyObject* py_euler_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
   NATIVE_END
 }
 
+// (modulation parameters [B, ...] with 3 C per gated projection, list of the projections' biases [C]) -> float32 (gates, gates *
+// biases), each [B, projections, C]
+PyObject* py_gate_rows(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  NATIVE_BEGIN
+  const Tensor *m, *first;
+  if (n != 2 || !(m = tensor_of(a[0])) || !PyList_Check(a[1])) return none();
+  const Py_ssize_t rows = PyList_GET_SIZE(a[1]);
+  if (rows == 0 || rows > 65535 || !(first = tensor_of(PyList_GET_ITEM(a[1], 0)))) return none();
+  const Where w;
+  const int dt = code_of(*m);
+  const int64_t C = first->numel(), B = m->dim() > 1 ? m->size(0) : 0;
+  if ((dt != ODIT_BF16 && dt != ODIT_F16) || !w.holds(m) || B <= 0 || B >= 65536 || C <= 0 || C >= (1 << 30) || m->numel() != B * rows * 3 * C)
+    return none();
+  int64_t dense = 1;  // every batch row is dense
+  for (int64_t d = m->dim() - 1; d > 0; --d) {
+    if (m->size(d) != 1 && m->stride(d) != dense) return none();
+    dense *= m->size(d);
+  }
+  std::vector<const void*> bias(static_cast<size_t>(rows));
+  for (Py_ssize_t i = 0; i < rows; ++i) {
+    const Tensor* t = tensor_of(PyList_GET_ITEM(a[1], i));
+    if (!t || !w.holds(t) || t->dim() != 1 || t->size(0) != C || t->scalar_type() != m->scalar_type() || !t->is_contiguous()) return none();
+    bias[static_cast<size_t>(i)] = t->data_ptr();
+  }
+  Tensor g = fresh({B, rows, C}, m->options().dtype(at::kFloat)), gb = fresh({B, rows, C}, m->options().dtype(at::kFloat));
+  if (unlocked([&] { return odit_gate_rows(bias.data(), static_cast<int>(rows), m->data_ptr(), m->stride(0), static_cast<int>(B), static_cast<int>(C),
+                       g.data_ptr<float>(), gb.data_ptr<float>(), dt, w.stream); }) != 0)
+    return none();
+  return wrap2(std::move(g), std::move(gb));
+  NATIVE_END
+}
+
 // (x, weight, bias or None, silu of x first)
 PyObject* py_linear_few(PyObject*, PyObject* const* a, Py_ssize_t n) {
   NATIVE_BEGIN
@@ -1638,6 +1670,7 @@ PyMethodDef kMethods[] = {
     NATIVE_FN("rope_tables", &py_rope_tables),
     NATIVE_FN("cfg_combine", &py_cfg_combine),
     NATIVE_FN("euler_step", &py_euler_step),
+    NATIVE_FN("gate_rows", &py_gate_rows),
     NATIVE_FN("classes", &py_classes),
     NATIVE_FN("qwen_block", &py_qwen_block),
     NATIVE_FN("flux_block", &py_flux_block),

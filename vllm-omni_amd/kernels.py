@@ -781,6 +781,14 @@ def euler_step(x: torch.Tensor, v: torch.Tensor, dt: float) -> torch.Tensor | No
     return (_nat or _load_native()).euler_step(x, v, dt)
 
 
+def gate_rows(mods: torch.Tensor, biases: list):
+    """float32 (gates, gates * biases) [B, n, C] of n gated projections, ``mods`` [B, ...] holding 3 C parameters for each with its
+    gate last; None for what the kernel does not take."""
+    if not mods.is_cuda or torch.is_grad_enabled():
+        return None
+    return (_nat or _load_native()).gate_rows(mods, biases)
+
+
 def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None, *, activation: str | None = None,
            residual: torch.Tensor | None = None, gate: torch.Tensor | None = None, out: torch.Tensor | None = None,
            gate_bias: torch.Tensor | None = None, prescaled: bool = False, tune_iters: int = 0,
