@@ -129,7 +129,7 @@ def test_tile_gemm_pair(kernels, gpu, dtype, M0, M1, N, K):
 
 
 def test_tile_gemm_overrides_stale_ticket_words(kernels, gpu):
-    """Words as a launch that never finished would leave them (arrivals, claims and departures of an old epoch)."""
+    """Words as a launch that never finished would leave them (arrivals, given-up quadrants and departures of an old epoch)."""
     M, N, K = 1100, 1000, 2048
     x, w, b, _ = _mk(gpu, M, N, K, torch.bfloat16, 1)
     want = kernels.linear(x, w, b, engine="handwritten")
@@ -138,6 +138,28 @@ def test_tile_gemm_overrides_stale_ticket_words(kernels, gpu):
         ws[:32768].view(torch.int64).fill_((1 << 16) | 0x3F3)
         assert torch.equal(kernels.linear(x, w, b, engine="handwritten"), want)
         ws[:32768].zero_()  # words of tiles that this problem does not have
+
+
+@pytest.mark.parametrize("M,N,K", [(1100, 1000, 2048), (1100, 2056, 2048), (1100, 5128, 8192), (4200, 4104, 4096)])
+def test_parts_that_do_not_run_at_once(kernels, gpu, M, N, K):
+    """Cut tiles while two other streams keep the compute units busy: parts start long after each other, so some give their
+    quadrants up to the last one. The sums are formed in one order whoever forms them: the same bits as alone."""
+    x, w, b, _ = _mk(gpu, M, N, K, torch.bfloat16, 3)
+    want = kernels.linear(x, w, b, engine="handwritten")
+    here, others = torch.cuda.current_stream(), [torch.cuda.Stream() for _ in range(2)]
+    busy = [torch.randn(4096, 4096, device=gpu).bfloat16() for _ in range(2)]
+    torch.cuda.synchronize()
+    outs = []
+    for s, t in zip(others, busy):
+        with torch.cuda.stream(s):
+            for _ in range(12):
+                kernels.linear(t, t, None, engine="handwritten")
+    for _ in range(12):
+        outs.append(kernels.linear(x, w, b, engine="handwritten"))
+    for s in others:
+        here.wait_stream(s)
+    torch.cuda.synchronize()
+    assert all(torch.equal(o, want) for o in outs)
 
 
 def test_tile_gemm_in_a_graph(kernels, gpu):

@@ -22,13 +22,16 @@
 //
 // The workgroup is persistent and the stream of steps does not stop at a tile's end: the next tile's first units are on their
 // way while this tile's epilogue runs. Tiles are dealt out round by round. The tiles of a last round that would leave half or
-// more of the compute units without work are cut along the reduction instead, into 2 to 4 equal parts, and those run first.
-// Each part leaves its fp32 partial tile in scratch (write-through) and takes a ticket; behind the whole tiles the parts of a
-// tile share its four quadrants out between them and each adds up all partial tiles of its quadrants, in the order of the parts
-// (the sum does not depend on who arrives when), and runs their epilogue. A part that does not find the others arrived after a
-// bounded number of looks leaves, and the last to arrive takes what is left: nobody waits for anybody without a bound. (One
-// workgroup adding everything up took 8 us for each further part, 256 KB at a time; so does it 16 for all.) Ticket words carry the
-// launch's epoch (see gemm_bf16.hip).
+// more of the compute units without work are cut along the reduction instead, into 2 to 4 equal parts, behind the whole tiles.
+// The parts of a tile share its four quadrants out between them: each leaves its fp32 sums for the others' quadrants in scratch
+// (write-through), keeps its own ones' in LDS and takes a ticket; when all have arrived it adds up all sums of its quadrants,
+// in the order of the parts (the result does not depend on who arrives when), and runs their epilogue. A part that does not find
+// the others arrived after a bounded number of looks leaves its own sums in scratch too and goes, and the last to arrive takes
+// what is left: nobody waits for anybody without a bound. Ticket words carry the launch's epoch (see gemm_bf16.hip). What the
+// parts cost is the traffic of their sums (2 x 256 KB for each of them if all go through memory). us, one workgroup adding all up /
+// each its quadrants, all through memory and parts ahead of the whole tiles / as described: M=512, N=3072, K=12288 in 4 parts
+// 77 / 60 / 55; M=512, N=9216, K=3072 in 3 - / 48.5 / 41.5; M=8192, N=9216, K=3072, half a round in 2 parts - / 338 / 323. (With the
+// parts of a tile on one XCD and its L2 in the place of memory: the same time or 2 us more.)
 //
 // Epilogue: W rows are assigned to accumulators so that a lane ends up with 8 consecutive features of one output row, stored
 // as 16 bytes from registers; bias, GELU(tanh), gate and residual are applied on the way.
@@ -36,9 +39,9 @@
 // What bounds it: the matrix pipe and the clock that the part holds under it. 8192 x 8192 x 8192 on random operands takes 1.35
 // us per step of 256 x 256 x 64 (1.59 PFLOP/s; hipBLASLt 1.60 on that card), 1.23 where one round runs. Measured with cold
 // weights, us, this kernel / its predecessor (256 x 256 or 256 x 192 tiles, 8 wavefronts in one phase) / the library's choice:
-// M=8192, N=12288, K=3072 with GELU 440 / 543 / 447; M=8192, N=9216, K=3072 349 / 402 / 437; M=2706, N=5120, K=5120 107 / 135 /
-// 117; M=2706, N=13824, K=5120 with GELU 297 / 399 / 319; M=1536, N=9216, K=3072 70 / 89 / 72. Around the loop a launch costs 6 us,
-// a tile's end 4 (7 with GELU: its arithmetic has no matrix work to hide behind).
+// M=8192, N=12288, K=3072 with GELU 440 / 543 / 447; M=8192, N=9216, K=3072 323 / 402 / 437; M=2706, N=5120, K=5120 107 / 135 /
+// 117; M=2706, N=13824, K=5120 with GELU 289 / 399 / 319; M=1536, N=9216, K=3072 68 / 89 / 72. Around the loop a launch costs 3 us,
+// a tile's end 6 (9 with GELU: its arithmetic has no matrix work to hide behind).
 #include <type_traits>
 
 #include "gemm_epilogue.h"
@@ -89,7 +92,7 @@ __device__ __forceinline__ int scalar(int a) {
 __device__ __forceinline__ int quotient(int a, int b) { return scalar(static_cast<int>(static_cast<unsigned>(a) / static_cast<unsigned>(b))); }
 
 constexpr int kThrough = 16;  // sc1 of a buffer access: past the XCD's L2, as an agent-scope store or load of a word goes
-// Ticket word of a cut tile: arrivals in bits 0 to 3, claimed quadrants 4 to 7, departures 8 to 11, the launch's epoch from 16 on
+// Ticket word of a cut tile: arrivals in bits 0 to 3, quadrants given up 4 to 7, departures 8 to 11, the launch's epoch from 16 on
 constexpr unsigned long long kArrival = 1, kDeparture = 1 << 8;
 constexpr int kLooks = 64;    // looks for the other parts of a tile, about a microsecond each
 constexpr int kMaxParts = 4;
@@ -199,24 +202,30 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     m0 = (first + r - nt * gm) * BM;
     n0 = nt * kTileN;
   };
-  // The segments of this workgroup: its part of a cut tile, then whole tiles. A cursor is (part still to do, next whole tile).
+  // The segments of this workgroup: whole tiles, then its part of a cut tile. A cursor is (part still to do, next whole tile).
   const int cut = p.tiles - p.whole;
   const bool has_part = v < cut * p.parts;
+  // quadrants that this part of a cut tile finishes: its number's, and the one `parts` further
+  auto quadrants = [&]() __attribute__((always_inline)) -> int {
+    const int part = quotient(v, cut);
+    return scalar(1 << part | (part + p.parts < 4 ? 1 << (part + p.parts) : 0));
+  };
+  constexpr int kQuad = 2 * MH * 8192;  // bytes of a quadrant's accumulators
   struct Cursor { bool part; int next; };
   auto next_segment = [&](Cursor& c, int& tile, int& k0, int& k1) __attribute__((always_inline)) -> bool {
-    if (c.part) {
-      c.part = false;
-      const int part = quotient(v, cut);
-      tile = p.whole + v - part * cut;
-      k0 = quotient(part * nk, p.parts);
-      k1 = quotient((part + 1) * nk, p.parts);
+    if (c.next < p.whole) {
+      tile = c.next;
+      c.next += G;
+      k0 = 0;
+      k1 = nk;
       return true;
     }
-    if (c.next >= p.whole) return false;
-    tile = c.next;
-    c.next += G;
-    k0 = 0;
-    k1 = nk;
+    if (!c.part) return false;
+    c.part = false;
+    const int part = quotient(v, cut);
+    tile = p.whole + v - part * cut;
+    k0 = quotient(part * nk, p.parts);
+    k1 = quotient((part + 1) * nk, p.parts);
     return true;
   };
 
@@ -465,30 +474,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
     if (wm == 0) barrier();  // both groups are here
 
-    if (k0 > 0 || k1 < nk) {
-      // A part of a cut tile: to its slot, and a ticket (the sums are formed behind the whole tiles). The address moves on in
-      // the scalar offset: a vector instruction right behind a 16-byte store must not write the store's data registers, the
-      // compiler takes a buffer store with a scalar offset for safe from that and put the next vector offset there, and
-      // accumulators of the last lanes went to memory with it now and then.
-      const auto slots = __builtin_amdgcn_make_buffer_rsrc(p.slots, 0, G * kTileSlot, 0x00020000);
-      const uint32_t off = static_cast<uint32_t>((wave * 64 + hidden_lane()) * 16);
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-#pragma unroll
-          for (int i = 0; i < 2 * MH; ++i)
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_v, acc[h][b][i / 2][i % 2]), slots, off,
-                                                   scalar(v * kTileSlot + ((2 * h + b) * 2 * MH + i) * 8192), kThrough);
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the partial tile has reached memory before the ticket is taken
-      __syncthreads();
-      if (tid == 0) {
-        unsigned long long* word = p.counters + (tile - p.whole);
-        // two atomics of one thread on one address: applied in program order
-        __hip_atomic_fetch_max(word, p.epoch << 16, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_fetch_add(word, kArrival, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
-    } else {
+    if (k0 == 0 && k1 == nk) {
       int which, m0, n0;
       locate(tile, which, m0, n0);
       const GemmEpilogue& e = p.q[which].ep;
@@ -498,69 +484,120 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       for (int b = 0; b < 2; ++b)
 #pragma unroll
         for (int h = 0; h < 2; ++h) finish_quadrant<T, MH>(kind, e, m0, m + h * HM, n + b * 128, acc[h][b]);
+    } else {
+      // A part of a cut tile. The parts share the tile's four quadrants out between them: part i adds up and finishes quadrants i,
+      // i + parts, ..., which it keeps in LDS (each thread its own accumulators; no tile load is in flight any more), and
+      // leaves the others in its slot.
+      // (the slot's address moves on in the scalar offset: a vector instruction right behind a 16-byte store must not write the
+      // store's data registers, the compiler takes a buffer store with a scalar offset for safe from that and put the next vector
+      // offset there, and accumulators of the last lanes went to memory with it now and then)
+      const auto slots = __builtin_amdgcn_make_buffer_rsrc(p.slots, 0, G * kTileSlot, 0x00020000);
+      const uint32_t own = static_cast<uint32_t>((wave * 64 + hidden_lane()) * 16);
+      const int mine = quadrants();
+#pragma unroll
+      for (int quad = 0; quad < 4; ++quad) {
+        if (mine >> quad & 1) continue;
+#pragma unroll
+        for (int i = 0; i < 2 * MH; ++i)
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_v, acc[quad >> 1][quad & 1][i / 2][i % 2]), slots, own,
+                                                 scalar(v * kTileSlot + quad * kQuad + i * 8192), kThrough);
+      }
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the pieces have reached memory before the ticket is taken
+      __syncthreads();
+      if (tid == 0) {
+        unsigned long long* word = p.counters + (tile - p.whole);
+        // two atomics of one thread on one address: applied in program order
+        __hip_atomic_fetch_max(word, p.epoch << 16, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const unsigned old = static_cast<unsigned>(__hip_atomic_fetch_add(word, kArrival, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        flag[1] = (old & 15u) + 1 == static_cast<unsigned>(p.parts) ? old >> 4 & 15u : 0;  // the last to arrive: what was given up
+      }
+      int at = 0;
+#pragma unroll
+      for (int quad = 0; quad < 4; ++quad) {
+        if (!(mine >> quad & 1)) continue;
+#pragma unroll
+        for (int i = 0; i < 2 * MH; ++i) *reinterpret_cast<f32x4_v*>(lds + at + own + i * 8192) = acc[quad >> 1][quad & 1][i / 2][i % 2];
+        at = scalar(at + kQuad);
+      }
     }
     more = next_segment(cc, tile, k0, k1);
   }
   if (has_part) {
-    // The parts of a tile share its four quadrants out between them: part i adds up and finishes quadrants i, i + parts, ... It
-    // looks for the others to have arrived, a bounded number of times; whoever arrived last certainly finds them all and takes
-    // what is left besides. A quadrant belongs to the one who claims it first.
-    const int part = quotient(v, cut), t = v - part * cut, parts = p.parts;
+    // A part looks for all parts of its tile to have arrived, a bounded number of times; then it gives its quadrants up (which fails
+    // if the last one has arrived by now) and leaves them to the last to arrive.
+    const int part = quotient(v, cut), t = v - part * cut, parts = p.parts, mine = quadrants();
     unsigned long long* word = p.counters + t;
     const unsigned all = static_cast<unsigned>(parts);
+    const auto slots = __builtin_amdgcn_make_buffer_rsrc(p.slots, 0, G * kTileSlot, 0x00020000);
+    if (tid == 0) {
+      int got = 0;
+      for (int look = 0; look < kLooks && got == 0; ++look) {
+        const unsigned w = static_cast<unsigned>(__hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        if ((w & 15u) == all) got = mine;
+        else __builtin_amdgcn_s_sleep(8);
+      }
+      flag[0] = got;
+    }
+    __syncthreads();
+    int got = scalar(flag[0]);
+    if (got == 0) {
+      const uint32_t own = static_cast<uint32_t>((wave * 64 + hidden_lane()) * 16);
+      int at = 0;
+      for (int left = mine; left != 0; left &= left - 1) {
+        const int quad = __builtin_ctz(left);
+#pragma unroll
+        for (int i = 0; i < 2 * MH; ++i)
+          __builtin_amdgcn_raw_buffer_store_b128(*reinterpret_cast<const u32x4_v*>(lds + at + own + i * 8192), slots, own,
+                                                 scalar(v * kTileSlot + quad * kQuad + i * 8192), kThrough);
+        at = scalar(at + kQuad);
+      }
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();  // (and the flag has been read)
+      if (tid == 0) {
+        const unsigned old = static_cast<unsigned>(__hip_atomic_fetch_or(word, static_cast<unsigned long long>(mine) << 4, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        flag[0] = (old & 15u) == all ? mine : 0;
+      }
+      __syncthreads();
+      got = scalar(flag[0]);
+    }
+    got = scalar(got | flag[1]);
     int which, m0, n0;
     locate(p.whole + t, which, m0, n0);
     const GemmEpilogue& e = p.q[which].ep;
     const int kind = epilogue_kind(e, m0, BM);
-    const auto slots = __builtin_amdgcn_make_buffer_rsrc(p.slots, 0, G * kTileSlot, 0x00020000);
-    unsigned mine = 0;
-    for (int i = part; i < 4; i += parts) mine |= 1u << i;
-    for (int round = 0; round < 2; ++round) {
-      // round 0: this part's own quadrants; round 1: those that nobody has claimed
-      if (tid == 0) {
-        unsigned got = 0;
-        for (int look = 0; look < (round == 0 ? kLooks : 1); ++look) {
-          const unsigned long long w = __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          if ((w & 15u) == all) {
-            const unsigned want = (round == 0 ? mine : 15u) & ~(static_cast<unsigned>(w >> 4) & 15u);
-            if (want != 0)
-              got = want & ~(static_cast<unsigned>(__hip_atomic_fetch_or(word, static_cast<unsigned long long>(want) << 4, __ATOMIC_RELAXED,
-                                                                         __HIP_MEMORY_SCOPE_AGENT) >> 4) & 15u);
-            break;
-          }
-          __builtin_amdgcn_s_sleep(8);
-        }
-        *reinterpret_cast<volatile unsigned*>(flag) = got;
-      }
-      __syncthreads();
-      unsigned got = __builtin_amdgcn_readfirstlane(*reinterpret_cast<volatile unsigned*>(flag));
-      __syncthreads();  // the flag is read before it is written again
-      for (; got != 0; got &= got - 1) {
-        const int quad = __builtin_ctz(got);
-        const int ln = hidden_lane();
-        const uint32_t off = static_cast<uint32_t>((wave * 64 + ln) * 16 + quad * (2 * MH * 8192));
-        f32x4_v sum[MH][2];
-        // all parts of the quadrant in one round trip, added in the order of the parts
-        auto add_up = [&](auto pc) __attribute__((always_inline)) {
-          constexpr int P = decltype(pc)::value;
-          f32x4_v r[P][2 * MH];
+    for (; got != 0; got &= got - 1) {
+      const int quad = __builtin_ctz(got);
+      const bool kept = mine >> quad & 1;
+      const int ln = hidden_lane();
+      const uint32_t off = static_cast<uint32_t>((wave * 64 + ln) * 16 + quad * kQuad);
+      const uint32_t kept_at = static_cast<uint32_t>((wave * 64 + ln) * 16) + ((mine & ((1 << quad) - 1)) != 0 ? kQuad : 0);
+      f32x4_v sum[MH][2];
+      // all parts of the quadrant in one round trip, added in the order of the parts
+      auto add_up = [&](auto pc) __attribute__((always_inline)) {
+        constexpr int P = decltype(pc)::value;
+        f32x4_v r[P][2 * MH];
 #pragma unroll
-          for (int j = 0; j < P; ++j)
+        for (int j = 0; j < P; ++j) {
+          if (kept && j == part) {
+#pragma unroll
+            for (int i = 0; i < 2 * MH; ++i) r[j][i] = *reinterpret_cast<const f32x4_v*>(lds + kept_at + i * 8192);
+          } else {
 #pragma unroll
             for (int i = 0; i < 2 * MH; ++i)
               r[j][i] = __builtin_bit_cast(f32x4_v, __builtin_amdgcn_raw_buffer_load_b128(slots, off + i * 8192, (t + j * cut) * kTileSlot, kThrough));
-#pragma unroll
-          for (int i = 0; i < 2 * MH; ++i) {
-            sum[i / 2][i % 2] = r[0][i];
-#pragma unroll
-            for (int j = 1; j < P; ++j) sum[i / 2][i % 2] += r[j][i];
           }
-        };
-        if (parts == 2) add_up(std::integral_constant<int, 2>{});
-        else if (parts == 3) add_up(std::integral_constant<int, 3>{});
-        else add_up(std::integral_constant<int, 4>{});
-        finish_quadrant<T, MH>(kind, e, m0, m0 + (quad >> 1) * HM + wm * (16 * MH) + (ln & 15), n0 + (quad & 1) * 128 + wn * 32 + (ln >> 4) * 8, sum);
-      }
+        }
+#pragma unroll
+        for (int i = 0; i < 2 * MH; ++i) {
+          sum[i / 2][i % 2] = r[0][i];
+#pragma unroll
+          for (int j = 1; j < P; ++j) sum[i / 2][i % 2] += r[j][i];
+        }
+      };
+      if (parts == 2) add_up(std::integral_constant<int, 2>{});
+      else if (parts == 3) add_up(std::integral_constant<int, 3>{});
+      else add_up(std::integral_constant<int, 4>{});
+      finish_quadrant<T, MH>(kind, e, m0, m0 + (quad >> 1) * HM + wm * (16 * MH) + (ln & 15), n0 + (quad & 1) * 128 + wn * 32 + (ln >> 4) * 8, sum);
     }
     // the last to leave hands the word back at zero
     if (tid == 0 && ((__hip_atomic_fetch_add(word, kDeparture, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >> 8) & 15u) + 1 == all)
@@ -592,12 +629,13 @@ bool gemm_tile_takes(const GemmCall& c, int dtype) {
   return static_cast<int64_t>(row_tiles(c.M, 128)) * row_tiles(c.N, kTileN) < (1 << 28);
 }
 
-// Tile height, and whether and into how many parts the tiles of the last round are cut: by expected time, fitted to 170
-// launches of 256 to 9500 rows of the projections of widths 3072 and 5120 (5.6 %). A step takes 1.23 us on 256-row tiles in a
-// launch's first round, 1.45 in later ones (the clock falls), 1.31 where a round is cut, 0.80 on 128-row tiles; a launch 5.7, a
-// tile's end 3.9, 3 (2) more with GELU; parts 9 and 0.054 for each workgroup that leaves one (half of that for 128 rows), 11 more
-// behind whole tiles. M=1024, N=3072, K=12288: 256 rows in 4 parts 83 us, 2 parts 136, whole 236, 128 rows 99; M=512, N=3072,
-// K=3072: 36, 47, 70 and 29 (4 parts); M=2706, N=13824, K=5120: 3 parts 297, whole 341.
+// Tile height, and whether and into how many parts the tiles of the last round are cut: by expected time, fitted to 268
+// launches of 256 to 9500 rows of the projections of widths 3072 and 5120, those within a quarter of a problem's best (6.3 %;
+// choosing by it takes 0.2 % longer than the best of all plans). A step takes 1.22 us on 256-row tiles in a launch's first
+// round, 1.32 in later ones (the clock falls), 1.13 where a round is cut, 0.78 on 128-row tiles; a launch 3.1, a tile's end 5.7,
+// 3 (2) more with GELU; a cut 0.088 for each part (0.057 with 128 rows), 5.7 more behind whole tiles. M=459, N=5120, K=13824: 256
+// rows in 4 parts 80 us, 3 parts 98, 2 parts 131, whole 238, 128 rows in 3 parts 77, 2 parts 100; M=504, N=9216, K=3072: 256
+// rows in 3 parts 41, whole 64, 128 rows 48; M=2998, N=12288, K=3072 with GELU: 256 rows in 4 parts 184, whole 215.
 TilePlan plan_gemm_tile(const GemmCall* c, int count, int cus, bool scratch) {
   TilePlan best;
   const int most = cus < kGemmMaxWorkers ? cus : kGemmMaxWorkers, nk = c[0].K / kTileK;
@@ -608,20 +646,20 @@ TilePlan plan_gemm_tile(const GemmCall* c, int count, int cus, bool scratch) {
     p.tiles0 = row_tiles(c[0].M, bm) * row_tiles(c[0].N, kTileN);
     p.tiles = p.tiles0 + (count > 1 ? row_tiles(c[1].M, bm) * row_tiles(c[1].N, kTileN) : 0);
     const int rounds = p.tiles / most, rest = p.tiles - rounds * most;
-    float end = 3.9f;
+    float end = 5.7f;
     for (int i = 0; i < count; ++i)
-      if (c[i].epilogue == ODIT_EPI_GELU_TANH || c[i].epilogue == ODIT_EPI_BIAS_GELU_TANH) end = tall ? 6.9f : 5.9f;
-    auto whole_rounds = [&](int n) { return n == 0 ? 0.f : n * (nk * (tall ? 1.45f : .8f) + end) - nk * (tall ? .22f : 0.f); };
+      if (c[i].epilogue == ODIT_EPI_GELU_TANH || c[i].epilogue == ODIT_EPI_BIAS_GELU_TANH) end = tall ? 8.7f : 7.7f;
+    auto whole_rounds = [&](int n) { return n == 0 ? 0.f : n * (nk * (tall ? 1.32f : .78f) + end) - nk * (tall ? .1f : 0.f); };
     for (int parts = 1; parts <= kMaxParts; ++parts) {
       if (parts > 1 && (!scratch || rest == 0 || rest * parts > most || parts > nk)) break;
       p.parts = parts;
       p.whole = parts > 1 ? p.tiles - rest : p.tiles;
       p.grid = rounds > 0 ? most : rest * parts;
       if (parts == 1) {
-        p.us = 5.7f + whole_rounds(rounds + (rest > 0 ? 1 : 0));
+        p.us = 3.1f + whole_rounds(rounds + (rest > 0 ? 1 : 0));
       } else {
-        p.us = 5.7f + whole_rounds(rounds) + (nk + parts - 1) / parts * (tall ? 1.31f : .8f) + 9.f + rest * parts * (tall ? .054f : .027f) +
-               (rounds > 0 ? 11.f : 0.f);
+        p.us = 3.1f + whole_rounds(rounds) + (nk + parts - 1) / parts * (tall ? 1.13f : .78f) + rest * parts * (tall ? .088f : .057f) +
+               (rounds > 0 ? 5.7f : 0.f);
       }
       if (best.bm == 0 || p.us < best.us) best = p;
     }

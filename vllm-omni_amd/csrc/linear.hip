@@ -497,8 +497,9 @@ static bool lin_streamk_rule(const odit::GemmCall& g) {
   return g.K >= 2 * g.N && g.M >= 48 && g.M < kTileMinRows && static_cast<int64_t>(g.N) * g.K >= (1ll << 22);
 }
 
-// The kernel of a problem that names no engine: what a tuning call found, else the stream-K kernel by its rule, else the kernel
-// for small products (3) by its rule, else the tile kernel where its expected time is below the library's (kTileMinAuto rows or
+// The kernel of a problem that names no engine: what a tuning call found, else the stream-K kernel by its rule or the tile kernel,
+// whose expected time is shorter (N=3072, K=12288, us, stream-K / tile: 300 rows 43 / 49, 400 48 / 49, 512 52 / 56, 592 61 / 55, 1024
+// 84 / 75; N=5120, K=13824: 200 62 / 60, 300 65 / 60, 592 101 / 86, 1024 144 / 112), else the kernel for small products (3) by its rule, else the tile kernel where its expected time is below the library's (kTileMinAuto rows or
 // more), else the library (0). One launch of the library takes 8 to 10 us for any small product, the small kernel 4 to 7 up to
 // K = kSmallK; beside a second problem, whose launch it saves, up to kSmallPairK.
 constexpr int kSmallK = 1024, kSmallPairK = 2048;
@@ -521,9 +522,14 @@ static float lin_call_us(const odit::LinCall& c, const odit::GemmCall& g, bool s
 static int lin_auto_kind(int dev, const odit::LinCall& c, const odit::GemmCall& g, const void* sk) {
   const int tuned = lin_tuned(dev, c, g.rows_per_gate);
   if (tuned >= 0) return tuned == 1 ? lin_handwritten_kind(g, c.dtype, sk) : 0;
-  if (sk != nullptr && lin_streamk_rule(g) && odit::gemm_streamk_takes(g, c.dtype)) return 1;
+  const bool tile = !c.no_tile && g.M >= kTileMinAuto && odit::gemm_tile_takes(g, c.dtype);
+  if (sk != nullptr && lin_streamk_rule(g) && odit::gemm_streamk_takes(g, c.dtype)) {
+    const int cus = odit::device_cus();
+    const odit::TilePlan plan = tile ? odit::plan_gemm_tile(&g, 1, cus, true) : odit::TilePlan{};
+    return plan.bm > 0 && plan.us < odit::gemm_streamk_us(g.M, 0, g.N, g.K, cus) ? 2 : 1;
+  }
   if (!c.no_tile && odit::gemm_streamk_takes(g, c.dtype) && odit::gemm_small_rule(&g, 1, odit::device_cus(), kSmallK)) return 3;
-  if (c.no_tile || g.M < kTileMinAuto || !odit::gemm_tile_takes(g, c.dtype)) return 0;
+  if (!tile) return 0;
   const odit::TilePlan plan = odit::plan_gemm_tile(&g, 1, odit::device_cus(), sk != nullptr);
   return plan.bm > 0 && plan.us < lin_library_us(c, g) ? 2 : 0;
 }
@@ -599,15 +605,13 @@ extern "C" int odit_linear_rows(const void* x, const void* w, const void* bias, 
 
 // Two problems in one launch, or two calls? By expected time. One launch has one set of overheads for both, shares the tiles of
 // the last round out over all CUs and takes gates that differ per batch entry, for which the library needs a call per entry.
-// Measured at width 3072 (us, stream-K pair / tile kernel pair / two library calls): 512 + 80 rows QKV 48 / 53 / 68, MLP down 66
-// / 68 / 125; 1024 + 512 QKV 109 / 75 / 98, out 45 / 50 / 50, MLP up 150 / 118 / 117, down 129 / 112 / 169; 2048 + 342 QKV 163 /
-// 130 / 150, out 56 / 50 / 62, up 221 / 153 / 181, down 176 / 154 / 206; 9210 + 406 QKV - / 394 / 462, up - / 538 / 648. The
-// stream-K kernel's fit ends at kPairTiles tiles of 128 rows together, kPairTilesGated where the library would need a call
-// per entry: past them only the tile kernel is compared.
+// Measured at width 3072 (us, stream-K pair / tile kernel pair / two calls): 512 + 80 QKV 47 / 55 / 71, MLP up 61 / 58 / 70, out 29 /
+// 28 / 37, MLP down 67 / 61 / 90; 810 + 466 QKV 97 / 69 / 84, out 45 / 40 / 44, up 131 / 103 / 107, down 116 / 101 / 126; 3024 + 642 QKV -
+// / 169 / 183, out - / 65 / 83, up - / 219 / 241, down - / 231 / 246. The stream-K kernel's fit ends at kPairTiles tiles of 128 rows
+// together, kPairTilesGated where the library would need a call per entry: past them only the tile kernel is compared.
 // Two calls are put 3 % above the sum of their estimates (the second one's rows and weights are cold when it starts). Over 104
-// pairs of 267 to 8759 and 40 to 885 rows, all four products of a dual-stream block (ms): 15.95 by this rule, 15.86 by the better of
-// the three each time, 16.38 where the tile kernel had to promise 6 % (3 % of that between 3 and 6 %: 3024 + 642 MLP down 250 / 227,
-// 8652 + 217 553 / 507, 2048 + 342 QKV 150 / 130).
+// pairs of 267 to 8759 and 40 to 885 rows, all four products of a dual-stream block (ms): 15.30 by this rule, 15.27 by the better of
+// the three each time, 15.33 with 0 or 6 % in the place of the 3, 15.70 where the tile kernel had to promise 6 %.
 constexpr int kPairTiles = 8, kPairTilesGated = 20;
 constexpr float kPairGain = 1.03f;
 
