@@ -726,8 +726,8 @@ def main():
     ap.add_argument("--autotune", type=int, default=0,
                     help="time the library's kernels for each fused-epilogue GEMM in an untimed first step")
     ap.add_argument("--linear-engine", choices=("auto", "library", "handwritten"), default="auto",
-                    help="A/B switch for the fused-epilogue projections: auto = the hand-written stream-K kernel where "
-                         "it is expected (or was tuned) to win and the library elsewhere; library = hipBLASLt always")
+                    help="A/B switch for the fused-epilogue projections: auto = the hand-written kernels or the "
+                         "library, by expected time or tuning; library = hipBLASLt always")
     ap.add_argument("--teacache", type=float, default=None, metavar="THRESH",
                     help="with --workload flux: also run the 28-step trajectory under the TeaCache hook with this "
                          "relative-L1 threshold and report skip rate and steps/s")
@@ -849,11 +849,11 @@ def main():
                                f"{HEADS} heads x {HEAD_DIM}, MLP {MLP_RATIO * C}, {S_IMG} image + {S_TXT} text tokens, "
                                "CFG batch 2, random weights N(0,0.02)",
                    "valid": args.blocks == LAYERS, "gemm": ("plain torch linears" if args.unfused_epilogues else
-                                                                "whole blocks as native calls, projections through odit_linear_rows: "
-                                                                "hipBLASLt's kernels") +
+                                                                "whole blocks as native calls, projections through odit_linear_pair and "
+                                                                "odit_linear_rows on " +
+                                                                ("hipBLASLt's kernels" if args.linear_engine == "library" else
+                                                                 "the hand-written MFMA kernels or hipBLASLt's, by expected time")) +
                            (" (tuned solution table)" if tuned else "") +
-                           ("" if args.linear_engine == "library" or args.unfused_epilogues else
-                            ", the text stream's MLP down-projection on the hand-written stream-K MFMA kernel") +
                            ("; GELU and gated residuals as separate kernels" if args.unfused_epilogues else
                             "; GELU and gated residuals in the GEMM epilogues")},
         "roofline": {"kernel": f"joint attention, B=2, 24x128, S=4352; one call = {plan} (timed together)", "bound": "mfma",
