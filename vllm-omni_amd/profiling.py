@@ -244,9 +244,9 @@ def summarise_traffic(dir_fetch: str, dir_write: str, probe_stdout: str) -> str:
 # ------------------------------------------------------------------------------------------ step trace
 _STEP_NOTES = {
     "qwen_image": ("Qwen-Image-shape denoise step (60 blocks, B=2, 4096+256 tokens)", "",
-                   ["# GELU and the image stream's gated residuals run inside the GEMM epilogues (odit_linear -> the Cijk_* kernels); the",
-                    "# text stream's MLP down-projection with its gated residual is gemm_streamk_kernel, its other gated residual the",
-                    "# gated_residual_kernel rows."]),
+                   ["# GELU and the gated residuals run inside the GEMM epilogues (gemm_tile_kernel: image and text rows of a block in one launch;",
+                    "# gemm_streamk_kernel: the text stream's MLP down-projection; Cijk_*: the library's). In the two steps that run kernel by kernel",
+                    "# some of them are separate launches."]),
     "flux": ("FLUX.1-shape denoise step (19 dual-stream + 38 single-stream blocks, B=1, 4096+512 tokens)", " --workload flux", []),
     "wan": ("Wan2.2-shape denoise step (40 blocks, B=2, 32760 video tokens, 512 text tokens)", " --workload wan", []),
 }
