@@ -509,7 +509,12 @@ class WanTransformer3DModel(nn.Module):
         p_t, p_h, p_w = self.patch_size
         x = video.view(B, Cin, nf // p_t, p_t, hh // p_h, p_h, ww // p_w, p_w)
         x = x.permute(0, 2, 4, 6, 1, 3, 5, 7).reshape(B, -1, Cin * p_t * p_h * p_w)
-        return F.linear(x, self.patch_embedding.weight.view(self.inner_dim, -1), self.patch_embedding.bias)
+        weight, bias = self.patch_embedding.weight.view(self.inner_dim, -1), self.patch_embedding.bias
+        # one step of 64 per output tile: 2706 rows of width 5120 take the tile kernel 20 us, the library's choice 30. (A batch
+        # keeps the library, as its blocks do.)
+        if B == 1 and x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and weight.dtype == x.dtype and kernels.native_blocks():
+            return kernels.linear(x, weight, bias)
+        return F.linear(x, weight, bias)
 
     def prepare(self, hidden_states: torch.Tensor, timestep: torch.Tensor, encoder_hidden_states: torch.Tensor,
                 encoder_hidden_states_image: torch.Tensor | None = None):
@@ -565,10 +570,18 @@ class WanTransformer3DModel(nn.Module):
         return x
 
     def finish(self, x: torch.Tensor, temb: torch.Tensor, grid: tuple[int, int, int], return_dict: bool = True):
-        shift, scale = self.output_scale_shift_prepare(temb)
-        if shift.ndim == 2:
-            shift, scale = shift.contiguous(), scale.contiguous()
-        x = kernels.adaln_modulate(x, shift, scale, eps=self.eps)
+        prep = self.output_scale_shift_prepare
+        if (temb.shape == x.shape and temb.dtype == x.dtype and x.shape[0] == 1 and not torch.is_grad_enabled()
+                and kernels.plain_module(prep, OutputScaleShiftPrepare)):
+            # a timestep per token: the norm adds the table's rows to the token's own in float32, where the module writes and
+            # reads back two [B,S,C] sums (2706 rows of width 5120: 36 us)
+            table = prep.scale_shift_table.detach().float()[0]
+            x = kernels.adaln_modulate(x, temb, temb, eps=self.eps, shift_bias=table[0], scale_bias=table[1])
+        else:
+            shift, scale = prep(temb)
+            if shift.ndim == 2:
+                shift, scale = shift.contiguous(), scale.contiguous()
+            x = kernels.adaln_modulate(x, shift, scale, eps=self.eps)
         x = self.proj_out(x)
         p_t, p_h, p_w = self.patch_size
         x = x.reshape(x.shape[0], *grid, p_t, p_h, p_w, -1).permute(0, 7, 1, 4, 2, 5, 3, 6)
