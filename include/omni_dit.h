@@ -340,13 +340,15 @@ int odit_silu(const void* x, void* out, int64_t n, int dtype, void* stream);
  * hand-written kernel out; NULL restricts the choice to library kernels that need none (not allowed
  * for the gated form).
  *
- * odit_linear_tune launches every kernel the library offers for the problem, and the hand-written
- * kernel where it takes the problem, on the given buffers
- * (`out` is overwritten; this call synchronises with the stream), keeps the fastest library kernel for later
- * odit_linear calls with the same shape, strides, epilogue and dtype FROM THE SAME HOST THREAD, records
- * for the whole process whether the hand-written kernel beat it, and reports the winner's time. `flush` (optional device buffer, ideally larger than the last-level cache) is
- * overwritten before every timed launch so that each one starts from cold caches, as a projection
- * with its own weights does inside a model. Without tuning the library's own first choice is used.
+ * odit_linear_tune launches every kernel the library offers for the problem, and the hand-written kernels
+ * that may be chosen for it, on the given buffers (`out` is overwritten; this call synchronises with the stream),
+ * keeps the fastest library kernel for later odit_linear calls with the same shape, strides, epilogue and dtype
+ * FROM THE SAME HOST THREAD, records for the whole process which kernel was the fastest, and reports its time. The
+ * record replaces the choice described above, by 3 % or more, and holds where the workspace has room for the hand-written
+ * kernels' scratch as it had (or had not) when it was made; where the library won, in the thread that holds its
+ * kernel. `flush` (optional device buffer, ideally larger than the last-level cache) is overwritten before every timed
+ * launch so that each one starts from cold caches, as a projection with its own weights does inside a model; products
+ * with N K < 2^22 are timed one after the other instead, as in a small model, whose weights stay in the cache.
  */
 enum odit_epilogue {
   ODIT_EPI_NONE = 0,
@@ -393,7 +395,8 @@ int odit_linear_rows(const void* x, const void* w, const void* bias, void* out, 
 /* Two projections of the same N, K, epilogue and types in ONE launch of a hand-written kernel (stream-K or tile): the image and the text rows of a
  * dual-stream block (to_qkv beside add_kv_proj, qwen_image_transformer.py:566-580, and the output, up and down projections).
  * Fields as the arguments of odit_linear_rows. Returns ODIT_ENOTSUP, with nothing launched, where two odit_linear_rows calls
- * are the better way or the kernels do not take a problem; the caller then makes them. flags as for
+ * are the better way (by expected time, or by the time that a tuning call measured for one of the problems) or the kernels do
+ * not take a problem; the caller then makes them. flags as for
  * odit_linear_rows (ODIT_LINEAR_LIBRARY: always ODIT_ENOTSUP; ODIT_LINEAR_HANDWRITTEN: the stream-K kernel). */
 typedef struct odit_linear_problem {
   const void *x, *w, *bias, *residual, *gate;
@@ -462,7 +465,7 @@ int odit_linear_rows_plan(const void* x, const void* w, const void* bias, void* 
                           int epilogue, int gate_dtype, int dtype, int rows_per_gate, int64_t gate_stride,
                           unsigned flags, void* workspace, size_t workspace_bytes, int* handwritten, int* launches);
 
-/* odit_linear_tune for the per-row-group form; *handwritten (may be NULL) = 1 when the hand-written kernel won. */
+/* odit_linear_tune for the per-row-group form; *handwritten (may be NULL) = 1 when a hand-written kernel won. */
 int odit_linear_rows_tune(const void* x, const void* w, const void* bias, void* out, const void* residual,
                           const void* gate, int M, int N, int K, int64_t ldx, int64_t ldw, int64_t ldo, int64_t ldr,
                           int epilogue, int gate_dtype, int dtype, int rows_per_gate, int64_t gate_stride,

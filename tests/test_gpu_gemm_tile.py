@@ -184,8 +184,9 @@ def test_tile_gemm_in_a_graph(kernels, gpu):
     del graph
 
 
-def test_pair_of_tuned_problems_goes_to_what_was_found(kernels, gpu):
-    """A tuning record for one of the two problems: the tile kernel's pair launch is not taken in its place."""
+def test_pair_of_tuned_problems_is_one_launch_where_that_is_faster(kernels, gpu):
+    """Tuning records for one and for both problems: one launch (30 us) stays the choice against two calls, of 26 and 17 us as
+    tuned and of 28 and 20 as expected."""
     from vllm_omni_amd import _lib
 
     M0, M1, N, K = 1216, 448, 6144, 1024  # (sizes that no other test tunes)
@@ -198,8 +199,9 @@ def test_pair_of_tuned_problems_goes_to_what_was_found(kernels, gpu):
         q[i].x, q[i].w, q[i].bias, q[i].out, q[i].M = ops[i][0].data_ptr(), ops[i][1].data_ptr(), ops[i][2].data_ptr(), out[i].data_ptr(), m
         q[i].ldx, q[i].ldw, q[i].ldo, q[i].ldr = K, K, N, N
     assert _pair(lib, ws, q, N, K, 1, 0) == 0
-    kernels.linear(ops[0][0], ops[0][1], ops[0][2], out=out[0], tune_iters=2)
-    assert _pair(lib, ws, q, N, K, 1, 0) == -2  # ODIT_ENOTSUP
+    for (x, w, b, _), o in zip(ops, out):
+        kernels.linear(x, w, b, out=o, tune_iters=2)
+        assert _pair(lib, ws, q, N, K, 1, 0) == 0
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])

@@ -76,12 +76,13 @@ struct LinState {
 };
 static thread_local LinState g_lin;
 
-// Problems for which a tuning call has compared the hand-written kernel with the library: true = the
-// hand-written kernel won (key: the whole problem, rows_per_gate in the lda field). Process-wide and kept
-// for the life of the process: every host thread sees what any thread has measured, and the record
-// outlives the per-thread descriptor cache.
+// What a tuning call found for a problem: the fastest kernel (0 the library's, which is in the plan of the thread that tuned; else
+// a hand-written one, see lin_candidate) and its time. Key: the whole problem, rows_per_gate in the lda field, and whether there
+// was scratch. Process-wide and kept for the life of the process: every host thread sees what any thread has measured, and the
+// record outlives the per-thread descriptor cache.
+struct Tuned { int kind; float us; };
 static std::mutex g_engine_mu;
-static std::unordered_map<LinKey, bool, LinKeyHash> g_handwritten_wins;
+static std::unordered_map<LinKey, Tuned, LinKeyHash> g_tuned;
 
 // Library kernels chosen ahead of time for plain projections (odit_linear_prefer): (N, M, K, element type) -> the
 // library's own solution index. Few entries, read when a problem is first seen.
@@ -198,15 +199,19 @@ static size_t lin_gate_bytes(const LinCall& c) {
   return lin_needs_prep(c) ? ((static_cast<size_t>(c.N) * 8 + 255) / 256) * 256 : 0;
 }
 
+static LinKey lin_plan_key(int dev, const LinCall& c) {
+  const bool gated = lin_is_residual(c);
+  return LinKey{dev, c.M, c.N, c.K, c.epilogue * 4 + (c.bias != nullptr ? 1 : 0) + (gated && c.gate != nullptr ? 2 : 0), c.dtype, c.ldw, c.ldx,
+                gated ? c.ldr : c.ldo, c.ldo};
+}
+
 // the handle, and the plan of the problem (as many launches as there are groups of rows share it)
 static int lin_find_plan(const LinCall& c, hipblasLtHandle_t* h, LinPlan** plan) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) { set_error("odit_linear: hipGetDevice failed"); return ODIT_ELAUNCH; }
   const int rc = lin_handle(dev, h);
   if (rc != ODIT_OK) return rc;
-  const bool gated = lin_is_residual(c);
-  LinKey key{dev, c.M, c.N, c.K, c.epilogue * 4 + (c.bias != nullptr ? 1 : 0) + (gated && c.gate != nullptr ? 2 : 0), c.dtype, c.ldw, c.ldx,
-             gated ? c.ldr : c.ldo, c.ldo};
+  LinKey key = lin_plan_key(dev, c);
   if (c.first) {  // unless a tuning call has found this problem's fastest kernel: what it chose runs
     const auto it = g_lin.plans.find(key);
     if (it == g_lin.plans.end() || !it->second.tuned) key.epi |= 0x100;
@@ -365,7 +370,9 @@ static int lin_default_algo(hipblasLtHandle_t h, LinPlan& p, const LinCall& c, s
 
 // the library's kernel for a plan that has none yet
 static int lin_choose_algo(hipblasLtHandle_t h, LinPlan& p, const LinCall& c, size_t lib_ws_bytes) {
-  if ((p.have_algo && p.algo_ws <= lib_ws_bytes) || lin_preferred_algo(h, p, c, lib_ws_bytes)) return ODIT_OK;
+  if (p.have_algo && p.algo_ws <= lib_ws_bytes) return ODIT_OK;
+  p.tuned = false;  // (what was tuned does not fit into this workspace)
+  if (lin_preferred_algo(h, p, c, lib_ws_bytes)) return ODIT_OK;
   return lin_default_algo(h, p, c, lib_ws_bytes);
 }
 
@@ -438,9 +445,9 @@ static odit::GemmCall lin_gemm_call(const odit::LinCall& c, int rows_per_gate, i
   return g;
 }
 
-// key of the whole problem for the record of which engine won a tuning run
-static odit::LinKey lin_engine_key(int dev, const odit::LinCall& c, int rows_per_gate) {
-  return odit::LinKey{dev, c.M, c.N, c.K, c.epilogue * 4 + (c.bias != nullptr ? 1 : 0) + (c.gate != nullptr ? 2 : 0),
+// key of the whole problem for the record of what a tuning run found
+static odit::LinKey lin_tuned_key(int dev, const odit::LinCall& c, int rows_per_gate, const void* sk) {
+  return odit::LinKey{dev, c.M, c.N, c.K, c.epilogue * 4 + (c.bias != nullptr ? 1 : 0) + (c.gate != nullptr ? 2 : 0) + (sk != nullptr ? 0x100 : 0),
                       c.dtype, rows_per_gate, c.ldx, c.ldw, c.ldo};
 }
 
@@ -458,11 +465,36 @@ static int lin_launch_handwritten(int kind, const odit::GemmCall& g, int dtype, 
   return odit::launch_gemm_tile(&g, 1, nullptr, dtype, sk, stream);
 }
 
-// What a tuning call found for a problem: 1 the hand-written kernel, 0 the library, -1 nothing was tuned.
-static int lin_tuned(int dev, const odit::LinCall& c, int rows_per_gate) {
-  std::lock_guard<std::mutex> lock(odit::g_engine_mu);
-  const auto it = odit::g_handwritten_wins.find(lin_engine_key(dev, c, rows_per_gate));
-  return it == odit::g_handwritten_wins.end() ? -1 : (it->second ? 1 : 0);
+// Whether a hand-written kernel (1 stream-K, 2 tile, 3 small) takes a problem, with this scratch or none.
+static bool lin_kind_takes(int kind, const odit::GemmCall& g, int dtype, const void* sk) {
+  if (kind == 2) return odit::gemm_tile_takes(g, dtype);
+  return (kind == 3 || sk != nullptr) && odit::gemm_streamk_takes(g, dtype);
+}
+
+// Whether this thread's plans of the launches that the library makes for a problem hold the kernels that a tuning call chose.
+static bool lin_library_tuned(int dev, const odit::LinCall& c, const odit::GemmCall& g) {
+  using namespace odit;
+  auto tuned = [&](int M) {
+    LinCall one = c;
+    one.M = M;
+    const auto it = g_lin.plans.find(lin_plan_key(dev, one));
+    return it != g_lin.plans.end() && it->second.tuned;
+  };
+  if (g.rows_per_gate <= 0) return tuned(g.M);
+  return tuned(g.rows_per_gate) && (g.M % g.rows_per_gate == 0 || tuned(g.M % g.rows_per_gate));
+}
+
+// What a tuning call found for a problem, where it holds here: a hand-written kernel has to take these operands (their alignment
+// is not in the key), and what the library won with has to be in this thread's plans; the library's own choice, which is what another
+// thread would get, may be slower than the kernel that the library's best was measured against.
+static bool lin_tuned(int dev, const odit::LinCall& c, const odit::GemmCall& g, const void* sk, odit::Tuned* found) {
+  {
+    std::lock_guard<std::mutex> lock(odit::g_engine_mu);
+    const auto it = odit::g_tuned.find(lin_tuned_key(dev, c, g.rows_per_gate, sk));
+    if (it == odit::g_tuned.end()) return false;
+    *found = it->second;
+  }
+  return found->kind == 0 ? lin_library_tuned(dev, c, g) : lin_kind_takes(found->kind, g, c.dtype, sk);
 }
 
 // Expected time (us) of one of the library's launches: that of its ranked kernel where it ranks them (long reductions), else 1.29
@@ -491,10 +523,11 @@ static float lin_library_us(const odit::LinCall& c, const odit::GemmCall& g) {  
 
 // The stream-K kernel for one problem: where the reduction is long against the number of output features (K >= 2 N: the
 // library's choices split K badly there: M=80, N=3072, K=12288 57 us against 31, M=512 69 against 52, M=1024 110 against 85) and
-// there is work for all CUs; with a small product (N K < 2^22, a few MB of weights) its ranges would be shorter than what
+// there is work for all CUs; with a small product (kSmallWeights: a few MB of weights) its ranges would be shorter than what
 // handing partial tiles over costs (M=256, N=256, K=1024: 19 us against 10).
+constexpr int64_t kSmallWeights = 1ll << 22;  // N K
 static bool lin_streamk_rule(const odit::GemmCall& g) {
-  return g.K >= 2 * g.N && g.M >= 48 && g.M < kTileMinRows && static_cast<int64_t>(g.N) * g.K >= (1ll << 22);
+  return g.K >= 2 * g.N && g.M >= 48 && g.M < kTileMinRows && static_cast<int64_t>(g.N) * g.K >= kSmallWeights;
 }
 
 // The kernel of a problem that names no engine: what a tuning call found, else the stream-K kernel by its rule or the tile kernel,
@@ -505,8 +538,19 @@ static bool lin_streamk_rule(const odit::GemmCall& g) {
 constexpr int kSmallK = 1024, kSmallPairK = 2048;
 constexpr int kTileMinAuto = 256;
 
-// expected time of a problem's own call: the better of what it may run on
-static float lin_call_us(const odit::LinCall& c, const odit::GemmCall& g, bool scratch) {
+// What a tuning call times against the library: every kernel that the rules may choose for the problem (one problem alone or half
+// of a pair, so that no tuned problem is left with less than it had), and the tile kernel for few rows too.
+static bool lin_candidate(int kind, const odit::GemmCall& g, int dtype, const void* sk) {
+  if (!lin_kind_takes(kind, g, dtype, sk)) return false;
+  if (kind == 1) return g.M < kTileMinRows;
+  return kind == 2 || odit::gemm_small_rule(&g, 1, odit::device_cus(), kSmallPairK);
+}
+
+// time of a problem's own call: what a tuning call measured, else the better of what it may run on, by expectation
+static float lin_call_us(int dev, const odit::LinCall& c, const odit::GemmCall& g, const void* sk) {
+  odit::Tuned found;
+  if (lin_tuned(dev, c, g, sk, &found)) return found.us;
+  const bool scratch = sk != nullptr;
   float us = lin_library_us(c, g);
   const int cus = odit::device_cus();
   if (scratch && lin_streamk_rule(g) && odit::gemm_streamk_takes(g, c.dtype)) {
@@ -519,9 +563,7 @@ static float lin_call_us(const odit::LinCall& c, const odit::GemmCall& g, bool s
   }
   return us;
 }
-static int lin_auto_kind(int dev, const odit::LinCall& c, const odit::GemmCall& g, const void* sk) {
-  const int tuned = lin_tuned(dev, c, g.rows_per_gate);
-  if (tuned >= 0) return tuned == 1 ? lin_handwritten_kind(g, c.dtype, sk) : 0;
+static int lin_rule_kind(const odit::LinCall& c, const odit::GemmCall& g, const void* sk) {
   const bool tile = !c.no_tile && g.M >= kTileMinAuto && odit::gemm_tile_takes(g, c.dtype);
   if (sk != nullptr && lin_streamk_rule(g) && odit::gemm_streamk_takes(g, c.dtype)) {
     const int cus = odit::device_cus();
@@ -532,6 +574,10 @@ static int lin_auto_kind(int dev, const odit::LinCall& c, const odit::GemmCall& 
   if (!tile) return 0;
   const odit::TilePlan plan = odit::plan_gemm_tile(&g, 1, odit::device_cus(), sk != nullptr);
   return plan.bm > 0 && plan.us < lin_library_us(c, g) ? 2 : 0;
+}
+static int lin_auto_kind(int dev, const odit::LinCall& c, const odit::GemmCall& g, const void* sk) {
+  odit::Tuned found;
+  return lin_tuned(dev, c, g, sk, &found) ? found.kind : lin_rule_kind(c, g, sk);
 }
 
 extern "C" int odit_linear_prefer(int M, int N, int K, int dtype, int solution) {
@@ -603,8 +649,10 @@ extern "C" int odit_linear_rows(const void* x, const void* w, const void* bias, 
   return ODIT_OK;
 }
 
-// Two problems in one launch, or two calls? By expected time. One launch has one set of overheads for both, shares the tiles of
-// the last round out over all CUs and takes gates that differ per batch entry, for which the library needs a call per entry.
+// Two problems in one launch, or two calls? By expected time; for the call of a problem that was tuned, by what was measured (811
+// + 466 rows, N=9216, K=3072: 73 us in one launch, 93 in two tuned calls; 1216 + 448, N=6144, K=1024: 30 and 36). One launch has
+// one set of overheads for both, shares the tiles of the last round out over all CUs and takes gates that differ per batch
+// entry, for which the library needs a call per entry.
 // Measured at width 3072 (us, stream-K pair / tile kernel pair / two calls): 512 + 80 QKV 47 / 55 / 71, MLP up 61 / 58 / 70, out 29 /
 // 28 / 37, MLP down 67 / 61 / 90; 810 + 466 QKV 97 / 69 / 84, out 45 / 40 / 44, up 131 / 103 / 107, down 116 / 101 / 126; 3024 + 642 QKV -
 // / 169 / 183, out - / 65 / 83, up - / 219 / 241, down - / 231 / 246. The stream-K kernel's fit ends at kPairTiles tiles of 128 rows
@@ -624,7 +672,7 @@ extern "C" int odit_linear_pair(const odit_linear_problem* q, int N, int K, int 
   size_t lib_bytes;
   lin_split_ws(workspace, workspace_bytes, &sk, &lib, &lib_bytes);
   GemmCall g[2];
-  bool per_rows = false, takes = true, streamk = sk != nullptr && engine != 1, tuned = false;
+  bool per_rows = false, takes = true, streamk = sk != nullptr && engine != 1;
   bool tile = engine != 1 && (flags & (ODIT_LINEAR_FIRST | ODIT_LINEAR_NO_TILE)) == 0;
   int tiles = 0, dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) { set_error("odit_linear_pair: hipGetDevice failed"); return ODIT_ELAUNCH; }
@@ -643,17 +691,16 @@ extern "C" int odit_linear_pair(const odit_linear_problem* q, int N, int K, int 
     tile = tile && q[i].M > 0 && gemm_tile_takes(g[i], dtype);
     if (engine == 1 || (!takes && !tile)) return ODIT_ENOTSUP;
     tiles += (q[i].M + kGemmBM - 1) / kGemmBM;
-    tuned = tuned || lin_tuned(dev, c, g[i].rows_per_gate) >= 0;
   }
   const int cus = device_cus();
   if (engine == 2) return streamk ? launch_gemm_streamk(g, 2, dtype, sk, static_cast<hipStream_t>(stream)) : ODIT_ENOTSUP;
   if (static_cast<int64_t>(N) * K < (1 << 14)) return ODIT_ENOTSUP;
-  if (takes && !tuned && (flags & (ODIT_LINEAR_FIRST | ODIT_LINEAR_NO_TILE)) == 0 && engine == 0 && gemm_small_rule(g, 2, cus, kSmallPairK))
+  if (takes && (flags & (ODIT_LINEAR_FIRST | ODIT_LINEAR_NO_TILE)) == 0 && engine == 0 && gemm_small_rule(g, 2, cus, kSmallPairK))
     return launch_gemm_small(g, 2, dtype, static_cast<hipStream_t>(stream));
-  // (no message where the answer is ODIT_ENOTSUP: two calls are an ordinary answer; problems that were tuned go to what was found)
+  // (no message where the answer is ODIT_ENOTSUP: two calls are an ordinary answer)
   const bool small = streamk && tiles <= (per_rows ? kPairTilesGated : kPairTiles);
-  const TilePlan plan = tile && !tuned ? plan_gemm_tile(g, 2, cus, sk != nullptr) : TilePlan{};
-  const bool wide = plan.bm > 0 && plan.us < kPairGain * (lin_call_us(calls[0], g[0], sk != nullptr) + lin_call_us(calls[1], g[1], sk != nullptr));
+  const TilePlan plan = tile ? plan_gemm_tile(g, 2, cus, sk != nullptr) : TilePlan{};
+  const bool wide = plan.bm > 0 && plan.us < kPairGain * (lin_call_us(dev, calls[0], g[0], sk) + lin_call_us(dev, calls[1], g[1], sk));
   if (small && !(wide && plan.us < gemm_streamk_us(g[0].M, g[1].M, N, K, cus)))
     return launch_gemm_streamk(g, 2, dtype, sk, static_cast<hipStream_t>(stream));
   if (!wide) return ODIT_ENOTSUP;
@@ -685,8 +732,8 @@ extern "C" int odit_linear_fork(const odit_linear_problem* q, const int* N, int 
     if (rc != ODIT_OK) return rc;
     ODIT_CHECK_ARG(!lin_is_residual(c), "odit_linear_fork: no residual");
     g[i] = lin_gemm_call(c, 0, 0);
-    if (!tile || q[i].M < kTileMinAuto || !gemm_tile_takes(g[i], dtype) || lin_tuned(dev, c, 0) >= 0) return ODIT_ENOTSUP;
-    two += lin_call_us(c, g[i], sk != nullptr);
+    if (!tile || q[i].M < kTileMinAuto || !gemm_tile_takes(g[i], dtype)) return ODIT_ENOTSUP;
+    two += lin_call_us(dev, c, g[i], sk);
   }
   const TilePlan plan = plan_gemm_tile(g, 2, device_cus(), sk != nullptr);
   if (plan.bm == 0 || plan.us >= kOneLaunchGain * two) return ODIT_ENOTSUP;
@@ -711,18 +758,18 @@ extern "C" int odit_linear_join(const void* x, const void* x2, const void* w, co
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) { set_error("odit_linear_join: hipGetDevice failed"); return ODIT_ELAUNCH; }
   const bool rows = lin_is_residual(c) && gate != nullptr && rows_per_gate > 0 && rows_per_gate < M;
-  LinCall second = c, whole = c;
+  LinCall first = c, second = c, whole = c;  // in two calls the second one's product comes first and has the bias with it
+  first.bias = nullptr;
   second.K = K2;
   second.ldx = ldx2;
   whole.K = K + K2;
-  const GemmCall g1 = lin_gemm_call(c, rows ? rows_per_gate : 0, rows ? gate_stride : 0), g2 = lin_gemm_call(second, g1.rows_per_gate, g1.ldg);
+  const GemmCall g1 = lin_gemm_call(first, rows ? rows_per_gate : 0, rows ? gate_stride : 0), g2 = lin_gemm_call(second, g1.rows_per_gate, g1.ldg);
   GemmCall g = lin_gemm_call(whole, g1.rows_per_gate, g1.ldg);
   if (lin_engine_of(flags) != 0 || (flags & (ODIT_LINEAR_FIRST | ODIT_LINEAR_NO_TILE)) != 0 || M < kTileMinAuto || K % 64 != 0 || K2 % 64 != 0 ||
-      ldx2 % 8 != 0 || !aligned16(x2) || !gemm_tile_takes(g1, dtype) || !gemm_tile_takes(g2, dtype) || !gemm_tile_takes(g, dtype) ||
-      lin_tuned(dev, c, g1.rows_per_gate) >= 0 || lin_tuned(dev, second, g1.rows_per_gate) >= 0)
+      ldx2 % 8 != 0 || !aligned16(x2) || !gemm_tile_takes(g1, dtype) || !gemm_tile_takes(g2, dtype) || !gemm_tile_takes(g, dtype))
     return ODIT_ENOTSUP;
   const TilePlan plan = plan_gemm_tile(&g, 1, device_cus(), sk != nullptr);
-  if (plan.bm == 0 || plan.us >= kOneLaunchGain * (lin_call_us(c, g1, sk != nullptr) + lin_call_us(second, g2, sk != nullptr))) return ODIT_ENOTSUP;
+  if (plan.bm == 0 || plan.us >= kOneLaunchGain * (lin_call_us(dev, first, g1, sk) + lin_call_us(dev, second, g2, sk))) return ODIT_ENOTSUP;
   const TileX2 other{x2, ldx2, K};
   return launch_gemm_tile(&g, 1, &other, dtype, sk, c.stream);
 }
@@ -763,6 +810,39 @@ extern "C" int odit_linear(const void* x, const void* w, const void* bias, void*
                           0, 0u, workspace, workspace_bytes, stream);
 }
 
+// Time of one launch as a tuning call compares it. A projection of a large model starts from cold caches: a flush (where a buffer is
+// given) before every launch. One with a few MB of weights (kSmallWeights) belongs to a small model, whose weights stay in the
+// last-level cache and whose time is often the host's: launches one after the other, as they come there (M=256, N=1024, K=1024, the
+// library / the small kernel: 11.5 us / 7.6 in a row, where a library call occupies the host for longer than the GPU; 9.0 / 12.0
+// behind a flush).
+template <typename Launch>
+static int lin_time(Launch&& launch, const odit::LinCall& c, int reps, void* flush, size_t flush_bytes, float* us) {
+  const bool row = static_cast<int64_t>(c.N) * c.K < kSmallWeights;
+  const int times = row ? 1 : reps, each = row ? 8 * reps : 1;
+  hipEvent_t e0, e1;
+  if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) {
+    odit::set_error("odit_linear_tune: hipEventCreate failed");
+    return ODIT_ELAUNCH;
+  }
+  int rc = launch();
+  float total = 0.f;
+  for (int i = 0; i < times && rc == ODIT_OK; ++i) {
+    if (!row && flush != nullptr && flush_bytes > 0) (void)hipMemsetAsync(flush, i & 0xff, flush_bytes, c.stream);
+    if (row) (void)hipStreamSynchronize(c.stream);
+    (void)hipEventRecord(e0, c.stream);
+    for (int j = 0; j < each && rc == ODIT_OK; ++j) rc = launch();
+    (void)hipEventRecord(e1, c.stream);
+    if (hipEventSynchronize(e1) != hipSuccess) { odit::set_error("odit_linear_tune: hipEventSynchronize failed"); rc = ODIT_ELAUNCH; }
+    float ms = 0.f;
+    (void)hipEventElapsedTime(&ms, e0, e1);
+    total += ms;
+  }
+  (void)hipEventDestroy(e0);
+  (void)hipEventDestroy(e1);
+  *us = total * 1e3f / (times * each);
+  return rc;
+}
+
 // Times the library's kernels for problem c (cold caches before every timed launch when a flush buffer
 // is given: in a model every projection has its own weights, which are never cache-resident, so
 // back-to-back launches on one weight would rank the kernels wrongly) and keeps the fastest in the plan.
@@ -780,30 +860,15 @@ static int lin_tune_library(const odit::LinCall& c, int iters, void* flush, size
   ODIT_LT(hipblaslt_ext::getAllAlgos(h, hipblaslt_ext::GemmType::HIPBLASLT_GEMM, HIPBLAS_OP_T, HIPBLAS_OP_N, t, t, t, t,
                                      HIPBLAS_COMPUTE_32F, all));
   const float beta = lin_is_residual(c) ? 1.f : 0.f;
-  hipEvent_t e0, e1;
-  if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) {
-    set_error("odit_linear_tune: hipEventCreate failed");
-    return ODIT_ELAUNCH;
-  }
   float best = 1e30f;
   int n_ok = 0;
   auto time_algo = [&](hipblasLtMatmulAlgo_t& algo, int reps) -> float {
-    if (hipblasLtMatmul(h, p->desc, alpha, c.w, p->a, c.x, p->b, &beta, cptr, p->c, c.out, p->d, &algo, lws, lws_bytes,
-                        c.stream) != HIPBLAS_STATUS_SUCCESS)
-      return -1.f;
-    float total = 0.f;
-    for (int i = 0; i < reps; ++i) {
-      if (flush != nullptr && flush_bytes > 0) (void)hipMemsetAsync(flush, i & 0xff, flush_bytes, c.stream);
-      (void)hipEventRecord(e0, c.stream);
-      hipblasLtMatmul(h, p->desc, alpha, c.w, p->a, c.x, p->b, &beta, cptr, p->c, c.out, p->d, &algo, lws, lws_bytes,
-                      c.stream);
-      (void)hipEventRecord(e1, c.stream);
-      if (hipEventSynchronize(e1) != hipSuccess) return -1.f;
-      float ms = 0.f;
-      (void)hipEventElapsedTime(&ms, e0, e1);
-      total += ms;
-    }
-    return total * 1e3f / reps;
+    float us = 0.f;
+    auto launch = [&]() -> int {
+      return hipblasLtMatmul(h, p->desc, alpha, c.w, p->a, c.x, p->b, &beta, cptr, p->c, c.out, p->d, &algo, lws, lws_bytes, c.stream) ==
+                     HIPBLAS_STATUS_SUCCESS ? ODIT_OK : ODIT_ELAUNCH;
+    };
+    return lin_time(launch, c, reps, flush, flush_bytes, &us) == ODIT_OK ? us : -1.f;
   };
   // first pass: one timed launch of every kernel the library has for these types that accepts the
   // problem; second pass: the best few again with `iters` launches each
@@ -830,40 +895,12 @@ static int lin_tune_library(const odit::LinCall& c, int iters, void* flush, size
       p->tuned = true;
     }
   }
-  (void)hipEventDestroy(e0);
-  (void)hipEventDestroy(e1);
   if (n_ok == 0) {
     set_error("odit_linear_tune: none of the library's %zu kernels accepts this problem", all.size());
     return ODIT_ENOTSUP;
   }
   *best_us = best;
   return ODIT_OK;
-}
-
-static int lin_time_handwritten(int kind, const odit::GemmCall& g, int dtype, void* sk, hipStream_t stream, int iters, void* flush,
-                                size_t flush_bytes, float* us) {
-  using namespace odit;
-  hipEvent_t e0, e1;
-  if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) {
-    set_error("odit_linear_tune: hipEventCreate failed");
-    return ODIT_ELAUNCH;
-  }
-  int rc = lin_launch_handwritten(kind, g, dtype, sk, stream);
-  float total = 0.f;
-  for (int i = 0; i < iters && rc == ODIT_OK; ++i) {
-    if (flush != nullptr && flush_bytes > 0) (void)hipMemsetAsync(flush, i & 0xff, flush_bytes, stream);
-    (void)hipEventRecord(e0, stream);
-    rc = lin_launch_handwritten(kind, g, dtype, sk, stream);
-    (void)hipEventRecord(e1, stream);
-    if (hipEventSynchronize(e1) != hipSuccess) { set_error("odit_linear_tune: hipEventSynchronize failed"); rc = ODIT_ELAUNCH; }
-    float ms = 0.f;
-    (void)hipEventElapsedTime(&ms, e0, e1);
-    total += ms;
-  }
-  (void)hipEventDestroy(e0);
-  (void)hipEventDestroy(e1);
-  *us = total * 1e3f / iters;
-  return rc;
 }
 
 extern "C" int odit_linear_rows_tune(const void* x, const void* w, const void* bias, void* out, const void* residual,
@@ -883,6 +920,8 @@ extern "C" int odit_linear_rows_tune(const void* x, const void* w, const void* b
   ODIT_CHECK_ARG(M > 0 && iters > 0, "odit_linear_tune: needs M > 0 and iters > 0");
   ODIT_CHECK_ARG(rows_per_gate >= 0 && gate_stride >= 0, "odit_linear_tune: rows_per_gate and gate_stride must not be negative");
   const bool per_rows = lin_is_residual(c) && gate != nullptr && rows_per_gate > 0 && rows_per_gate < M;
+  const GemmCall g = lin_gemm_call(c, per_rows ? rows_per_gate : 0, per_rows ? gate_stride : 0);
+  const int rule = lin_rule_kind(c, g, sk);  // (before the library's plans hold what is tuned)
   // the library runs one launch per group of rows: tune that launch (on the first group), and the shorter
   // launch of a last group that is not full, which is a problem of its own to the library
   LinCall cl = c;
@@ -904,22 +943,31 @@ extern "C" int odit_linear_rows_tune(const void* x, const void* w, const void* b
     if (rc != ODIT_OK) return rc;
     lib_us += last_us;
   }
-  float best = lib_us;
-  const GemmCall g = lin_gemm_call(c, per_rows ? rows_per_gate : 0, per_rows ? gate_stride : 0);
-  if (const int kind = lin_handwritten_kind(g, dtype, sk)) {
+  // two kernels' times less than 3 % apart say nothing about their times in a model: the rule's choice stays
+  constexpr float kSame = .97f;
+  Tuned best{0, lib_us};
+  float best_at = rule == 0 ? kSame * lib_us : lib_us;
+  bool compared = false;
+  for (int kind = 1; kind <= 3; ++kind) {
+    if (!lin_candidate(kind, g, dtype, sk)) continue;
     float own_us = 0.f;
-    rc = lin_time_handwritten(kind, g, dtype, sk, c.stream, iters, flush, flush_bytes, &own_us);
+    rc = lin_time([&]() -> int { return lin_launch_handwritten(kind, g, dtype, sk, c.stream); }, c, iters, flush, flush_bytes, &own_us);
     if (rc != ODIT_OK) return rc;
+    compared = true;
+    const float at = kind == rule ? kSame * own_us : own_us;
+    if (at < best_at) {
+      best = Tuned{kind, own_us};
+      best_at = at;
+    }
+  }
+  if (compared) {
     int dev = 0;
     (void)hipGetDevice(&dev);
-    {
-      std::lock_guard<std::mutex> lock(g_engine_mu);
-      g_handwritten_wins[lin_engine_key(dev, c, per_rows ? rows_per_gate : 0)] = own_us < lib_us;
-    }
-    if (handwritten) *handwritten = own_us < lib_us ? 1 : 0;
-    if (own_us < best) best = own_us;
+    std::lock_guard<std::mutex> lock(g_engine_mu);
+    g_tuned[lin_tuned_key(dev, c, g.rows_per_gate, sk)] = best;
   }
-  if (best_us) *best_us = best;
+  if (handwritten) *handwritten = best.kind != 0 ? 1 : 0;
+  if (best_us) *best_us = best.us;
   return ODIT_OK;
 }
 
