@@ -488,10 +488,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       // A part of a cut tile. The parts share the tile's four quadrants out between them: part i adds up and finishes quadrants i,
       // i + parts, ..., which it keeps in LDS (each thread its own accumulators; no tile load is in flight any more), and
       // leaves the others in its slot.
-      // (the slot's address moves on in the scalar offset: a vector instruction right behind a 16-byte store must not write the
-      // store's data registers, the compiler takes a buffer store with a scalar offset for safe from that and put the next vector
-      // offset there, and accumulators of the last lanes went to memory with it now and then)
-      const auto slots = __builtin_amdgcn_make_buffer_rsrc(p.slots, 0, G * kTileSlot, 0x00020000);
+      // (a vector instruction right behind a 16-byte store must not write the store's data registers. The compiler puts the wait
+      // there, but takes a store with an offset in a scalar register for safe, and accumulators of the last lanes went to memory
+      // overwritten now and then. So the slot is in the descriptor, the rest in the vector offset, and no store has a scalar one.)
+      const auto slot = __builtin_amdgcn_make_buffer_rsrc(p.slots + static_cast<int64_t>(v) * kTileSlot, 0, kTileSlot, 0x00020000);
       const uint32_t own = static_cast<uint32_t>((wave * 64 + hidden_lane()) * 16);
       const int mine = quadrants();
 #pragma unroll
@@ -499,8 +499,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         if (mine >> quad & 1) continue;
 #pragma unroll
         for (int i = 0; i < 2 * MH; ++i)
-          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_v, acc[quad >> 1][quad & 1][i / 2][i % 2]), slots, own,
-                                                 scalar(v * kTileSlot + quad * kQuad + i * 8192), kThrough);
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_v, acc[quad >> 1][quad & 1][i / 2][i % 2]), slot,
+                                                 own + (quad * kQuad + i * 8192), 0, kThrough);
       }
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the pieces have reached memory before the ticket is taken
       __syncthreads();
@@ -541,14 +541,15 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     __syncthreads();
     int got = scalar(flag[0]);
     if (got == 0) {
+      const auto slot = __builtin_amdgcn_make_buffer_rsrc(p.slots + static_cast<int64_t>(v) * kTileSlot, 0, kTileSlot, 0x00020000);
       const uint32_t own = static_cast<uint32_t>((wave * 64 + hidden_lane()) * 16);
       int at = 0;
       for (int left = mine; left != 0; left &= left - 1) {
         const int quad = __builtin_ctz(left);
 #pragma unroll
         for (int i = 0; i < 2 * MH; ++i)
-          __builtin_amdgcn_raw_buffer_store_b128(*reinterpret_cast<const u32x4_v*>(lds + at + own + i * 8192), slots, own,
-                                                 scalar(v * kTileSlot + quad * kQuad + i * 8192), kThrough);
+          __builtin_amdgcn_raw_buffer_store_b128(*reinterpret_cast<const u32x4_v*>(lds + at + own + i * 8192), slot,
+                                                 own + (quad * kQuad + i * 8192), 0, kThrough);
         at = scalar(at + kQuad);
       }
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
