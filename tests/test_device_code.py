@@ -43,3 +43,16 @@ def test_partial_tiles_are_stored_without_a_scalar_offset():
         stores = [i for i in code if i.startswith("buffer_store_dwordx4")]
         assert len(stores) >= 16, name  # 4 quadrants of 4 or 8, and those of a part that gives up
         assert [i for i in stores if not re.search(r"\], 0 offen", i)] == [], name
+
+
+def test_small_kernel_waits_for_its_reads_at_every_barrier():
+    """Behind a step's barrier the stage that was read in the step before is refilled: the wait in front of the barrier names the
+    reads too, wherever the matrix instructions that use them end up."""
+    kernels = _functions("gemm_small.hip")
+    assert len(kernels) == 8
+    for name, code in kernels.items():
+        barriers = [i for i, text in enumerate(code) if text.startswith("s_barrier")]
+        assert barriers, name
+        for at in barriers:
+            wait = next(text for text in reversed(code[:at]) if text.startswith("s_waitcnt"))
+            assert "lgkmcnt(0)" in wait and "vmcnt" in wait, (name, code[at - 6:at + 1])

@@ -122,9 +122,10 @@ __global__ __launch_bounds__(256) void gemm_small_kernel(const SmallParams p) {
 #pragma unroll
     for (int b = 0; b < 2; ++b) acc[a][b] = f32x4_v{0.f, 0.f, 0.f, 0.f};
   for (int i = 0; i < nk; ++i) {
-    // this wavefront's loads of step i have landed, in every wavefront behind the barrier, which has also read step i - 1
-    if (S == kSmallStages && i + S - 2 < nk) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kSmallStages - 2) * 4) : "memory");
-    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    // this wavefront's loads of step i have landed and its reads of step i - 1 are in registers; behind the barrier that holds for
+    // every wavefront, and the stage of step i - 1 is free
+    if (S == kSmallStages && i + S - 2 < nk) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((kSmallStages - 2) * 4) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     if (S == kSmallStages && i > 0 && i - 1 + S < nk) issue(i - 1 + S, (i - 1) % S);
