@@ -10,6 +10,27 @@ typedef __attribute__((__vector_size__(8 * sizeof(_Float16)))) _Float16 f16x8_v;
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16_v;
 typedef __attribute__((__vector_size__(2 * sizeof(float)))) float f32x2_v;
 typedef uint32_t u32x4_v __attribute__((ext_vector_type(4)));
+
+// 16 bytes per lane from global memory straight into LDS: lane l of the wavefront fills bytes 16 l .. of the 1 KB at LDS address
+// `lds` with what lies `off` (its own) + `soff` bytes into the buffer. A memory instruction may read a scalar register 5 wait states
+// after a vector instruction (v_readfirstlane) has written it and no sooner, and the compiler does not look into the statement, so
+// it waits itself (the move to m0 and 4 more). SETTLED: the caller forms descriptor and offset with scalar instructions only, and
+// 1 more is enough, for m0 (attention, B=2, S=1357, 32 heads of 64 with a mask: 52.4 us, with 4 more 52.9; the tile GEMM at 8192 x
+// 8192 x 8192 takes 710 us with 1, 716 with 4). tests/test_device_code.py looks through what the compiler makes of it.
+template <bool SETTLED = false>
+__device__ __forceinline__ void load_lds16(uint32_t lds, uint32_t off, u32x4_v rsrc, uint32_t soff) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  // m0 (the LDS destination of the load) is a reserved register: naming it as clobbered draws a
+  // warning per expansion, and leaving it out would hide the write from the compiler
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop %4\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+               :
+               : "s"(lds), "v"(off), "s"(rsrc), "s"(soff), "n"(SETTLED ? 0 : 3)
+               : "memory", "m0");
+#pragma clang diagnostic pop
+#endif
+}
 typedef uint32_t u32x2_v __attribute__((ext_vector_type(2)));
 typedef float f32x4_v __attribute__((ext_vector_type(4)));
 typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 bf16x2_v;

@@ -273,15 +273,7 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void attn_fwd_dma_kernel(const Att
       const uint32_t m0v = __builtin_amdgcn_readfirstlane(lds0 + i * 1024);
       const uint32_t voff_i = is_k ? (voff0 ^ static_cast<uint32_t>((((RPI * i) % 16) % CPR) * 16)) : voff0;
       const uint32_t soff_i = soff + static_cast<uint32_t>(i) * (is_k ? k_inst_step : v_inst_step);
-      // m0 (the LDS destination of the load) is a reserved register: naming it as clobbered draws a
-      // warning per expansion, and leaving it out would hide the write from the compiler
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                   :
-                   : "s"(m0v), "v"(voff_i), "s"(rsrc), "s"(soff_i)
-                   : "memory", "m0");
-#pragma clang diagnostic pop
+      load_lds16<true>(m0v, voff_i, rsrc, soff_i);
     }
 #endif
   };

@@ -211,15 +211,7 @@ __global__ __launch_bounds__(kWaves * 64, 1) void gemm_streamk_kernel(const Gemm
       const uint32_t dst = __builtin_amdgcn_readfirstlane(
           static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void_p)(lds + stage * kStage + (q0 + i) * 1024))));
       const u32x4_v rs = q0 + i < kXInst ? xrsrc : wrsrc;  // wave-uniform
-      // m0 (the LDS destination of the load) is a reserved register: naming it as clobbered draws a
-      // warning per expansion, and leaving it out would hide the write from the compiler
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                   :
-                   : "s"(dst), "v"(voff[i]), "s"(rs), "s"(soff)
-                   : "memory", "m0");
-#pragma clang diagnostic pop
+      load_lds16(dst, voff[i], rs, soff);
 #endif
     };
 

@@ -301,19 +301,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   };
   const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void_p)lds));
   auto load = [&](uint32_t dst, uint32_t off, u32x4_v rs, int soff) __attribute__((always_inline)) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    const uint32_t m0v = __builtin_amdgcn_readfirstlane(dst);
-    const int s = scalar(soff);
-    // m0 (the LDS destination of the load) is a reserved register: naming it as clobbered draws a
-    // warning per expansion, and leaving it out would hide the write from the compiler
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                 :
-                 : "s"(m0v), "v"(off), "s"(rs), "s"(s)
-                 : "memory", "m0");
-#pragma clang diagnostic pop
-#endif
+    load_lds16(__builtin_amdgcn_readfirstlane(dst), off, rs, scalar(soff));
   };
   auto load_x = [&](int stage, int h, int j) __attribute__((always_inline)) { load(lds0 + stage * kStage + h * kXUnit + (wave * XJ + j) * 1024, vx[h][j], xr, kx); };
   auto load_w = [&](int stage, int h, int j) __attribute__((always_inline)) { load(lds0 + stage * kStage + 2 * kXUnit + h * kWUnit + (wave * WJ + j) * 1024, vw[h][j], wr, kw); };
