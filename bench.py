@@ -724,7 +724,7 @@ def main():
     ap.add_argument("--unfused-epilogues", action="store_true",
                     help="A/B switch: GELU and gated residuals as separate kernels after plain GEMMs")
     ap.add_argument("--autotune", type=int, default=0,
-                    help="time the library's kernels for each fused-epilogue GEMM in an untimed first step")
+                    help="time the library's kernels and the hand-written ones for each fused-epilogue GEMM in an untimed first step")
     ap.add_argument("--linear-engine", choices=("auto", "library", "handwritten"), default="auto",
                     help="A/B switch for the fused-epilogue projections: auto = the hand-written kernels or the "
                          "library, by expected time or tuning; library = hipBLASLt always")
@@ -790,7 +790,7 @@ def main():
 
     with torch.inference_mode():
         lat = latents
-        if args.autotune > 0:   # untimed: pick the library kernel for each fused-epilogue GEMM
+        if args.autotune > 0:   # untimed: pick the kernel for each fused-epilogue GEMM
             kernels.set_linear_autotune(args.autotune)
             step(0, lat)
             kernels.set_linear_autotune(0)

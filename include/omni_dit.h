@@ -277,8 +277,9 @@ int odit_rel_l1(const void* cur, const void* prev, double* sums, void* workspace
  * device image, 2560 bytes per GPU the library is used on, held until the process ends. It calls no
  * allocating routine. Limit: B <= 64 rows (any n); more returns ODIT_EWORKSPACE and enqueues nothing.
  * Two launches: a fill kernel puts the ticket words to zero (a kernel, not a memset, so the call can be
- * captured; whatever an earlier call left in the array, also one that never finished, is gone), then the reduction. Every call on a GPU shares that GPU's array: calls that may overlap on one GPU
- * (different streams without ordering, or several host threads) race and must be serialised by the caller.
+ * captured; whatever an earlier call left in the array, also one that never finished, is gone), then the
+ * reduction. Every call on a GPU shares that GPU's array: calls that may overlap on one GPU (different streams
+ * without ordering, or several host threads) race and must be serialised by the caller.
  * The first call on each device looks the array's address up (hipGetSymbolAddress); make that call outside
  * graph capture.
  */
@@ -322,9 +323,10 @@ int odit_silu(const void* x, void* out, int64_t n, int dtype, void* stream);
  * multiple of 8, 16-byte aligned rows): a stream-K kernel for few rows (csrc/gemm_bf16.hip) and a tile kernel for many
  * (csrc/gemm_bf16_tile.hip: 256 x 256 or 128 x 256 output tiles, the last round's cut along the reduction where they are
  * few), and one for products that are small altogether (csrc/gemm_small.hip: 64 x 64 tiles). All take one gate vector per
- * group of rows in a single launch (odit_linear_rows). Which runs: what a tuning call found, else the stream-K kernel for 48 to
- * 1024 rows and K >= 2 N, else the small kernel where all its tiles have a place at once and K <= 1024, else the tile kernel (256
- * rows or more) or the library by expected time; the `flags` of odit_linear_rows can force either side.
+ * group of rows in a single launch (odit_linear_rows). Which runs: what a tuning call found, else for 48 to 1024 rows and K >= 2 N
+ * (and N K >= 2^22) the stream-K kernel or, from 256 rows on, the tile kernel, by expected time, else the small kernel where
+ * all its tiles have a place at once and K <= 1024, else the tile kernel (256 rows or more) or the library by expected time; the
+ * `flags` of odit_linear_rows can force either side.
  *
  * x [M,K] (row stride ldx), W [N,K] (row stride ldw: torch's nn.Linear weight, or a column range of
  * one), bias [N] or NULL, out [M,N] (row stride ldo). Gated form: residual [M,N] (row stride ldr; may be
@@ -336,9 +338,9 @@ int odit_silu(const void* x, void* out, int64_t n, int dtype, void* stream);
  * ZERO-FILLED ONCE before its first use and not written by the caller afterwards (the first 32 KB hold
  * the hand-written kernels' ticket words, stamped with the launch number like those of odit_rel_l1: every call
  * leaves them at zero, and what a launch that did not finish left there is overridden by the next one);
- * calls that share a workspace must not overlap in time (one workspace per stream). A smaller workspace goes to the library alone and rules the
- * hand-written kernel out; NULL restricts the choice to library kernels that need none (not allowed
- * for the gated form).
+ * calls that share a workspace must not overlap in time (one workspace per stream). A smaller workspace goes to the library
+ * alone: the stream-K kernel is ruled out and the tile kernel cuts no tiles; the small kernel needs none. NULL restricts the
+ * library to kernels that need none as well (not allowed for ODIT_EPI_GATED_RESIDUAL with a gate).
  *
  * odit_linear_tune launches every kernel the library offers for the problem, and the hand-written kernels
  * that may be chosen for it, on the given buffers (`out` is overwritten; this call synchronises with the stream),
@@ -376,11 +378,11 @@ int odit_linear_tune(const void* x, const void* w, const void* bias, void* out, 
  * rows_per_gate = 0 is odit_linear. One launch when a hand-written kernel takes the problem, one
  * library launch per group of rows otherwise.
  * flags: 0 = choose as described above; ODIT_LINEAR_LIBRARY = hipBLASLt whatever the record says;
- * ODIT_LINEAR_HANDWRITTEN = the hand-written kernel for this row count (ODIT_ENOTSUP when it does not take
- * the problem); ODIT_LINEAR_FIRST = where hipBLASLt runs the problem and no tuning call of this thread chose a kernel for it,
- * its own first choice (or the one odit_linear_prefer named), not the one expected to be faster, and what ODIT_LINEAR_NO_TILE
- * says; ODIT_LINEAR_NO_TILE = not the tile kernel, unless a tuning call found it faster (a caller whose results another order of
- * summation may not move). Per call: no process-wide switch exists.
+ * ODIT_LINEAR_HANDWRITTEN = the hand-written kernel for this row count, stream-K up to 1024 rows, tile from 1025 on
+ * (ODIT_ENOTSUP when it does not take the problem); ODIT_LINEAR_FIRST = where hipBLASLt runs the problem and no tuning call of
+ * this thread chose a kernel for it, its own first choice (or the one odit_linear_prefer named), not the one expected to be
+ * faster, and what ODIT_LINEAR_NO_TILE says; ODIT_LINEAR_NO_TILE = neither the tile nor the small kernel, unless a tuning call
+ * found it faster (a caller whose results another order of summation may not move). Per call: no process-wide switch exists.
  */
 #define ODIT_LINEAR_LIBRARY 1u
 #define ODIT_LINEAR_HANDWRITTEN 2u
@@ -392,12 +394,14 @@ int odit_linear_rows(const void* x, const void* w, const void* bias, void* out, 
                      int epilogue, int gate_dtype, int dtype, int rows_per_gate, int64_t gate_stride,
                      unsigned flags, void* workspace, size_t workspace_bytes, void* stream);
 
-/* Two projections of the same N, K, epilogue and types in ONE launch of a hand-written kernel (stream-K or tile): the image and the text rows of a
- * dual-stream block (to_qkv beside add_kv_proj, qwen_image_transformer.py:566-580, and the output, up and down projections).
+/* Two projections of the same N, K, epilogue and types in ONE launch of a hand-written kernel (stream-K, tile or small): the
+ * image and the text rows of a dual-stream block (to_qkv beside add_kv_proj, qwen_image_transformer.py:566-580, and the output, up
+ * and down projections).
  * Fields as the arguments of odit_linear_rows. Returns ODIT_ENOTSUP, with nothing launched, where two odit_linear_rows calls
  * are the better way (by expected time, or by the time that a tuning call measured for one of the problems) or the kernels do
  * not take a problem; the caller then makes them. flags as for
- * odit_linear_rows (ODIT_LINEAR_LIBRARY: always ODIT_ENOTSUP; ODIT_LINEAR_HANDWRITTEN: the stream-K kernel). */
+ * odit_linear_rows (ODIT_LINEAR_LIBRARY: always ODIT_ENOTSUP; ODIT_LINEAR_HANDWRITTEN: the stream-K kernel;
+ * ODIT_LINEAR_NO_TILE and ODIT_LINEAR_FIRST: the stream-K kernel by its rule or ODIT_ENOTSUP). */
 typedef struct odit_linear_problem {
   const void *x, *w, *bias, *residual, *gate;
   void* out;

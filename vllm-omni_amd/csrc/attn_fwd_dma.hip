@@ -31,15 +31,16 @@
 // Past kMaskWords tiles, and in the persistent form, whose units change the batch row, the mask is read as bytes.
 // With the words a unit ends with the last tile that has a live key: the tiles behind it would add zero probabilities (and are not
 // read: a NaN among their values does not reach the rows). Together with spread_batch below, one batch row padded to 40 % of
-// the other's keys, us, f16, before / now, and the same with an all-true mask:
+// the other's keys, us, f16, before / now, and the same with an all-true mask (what a launch gains depends on the padding: with
+// three drawn lengths of the second row the first shape takes 46 to 53):
 //   B=2 S=1357 H=32 (8 of keys) D=64  60.1 / 43.0, 56.0 / 56.2    B=2 S=1195 H=24 D=128  45.8 / 36.4, 46.1 / 45.4
 //   B=2 S=4352 H=24 D=64              320 / 296, 298 / 299        B=2 S=4352 H=24 D=128  485 / 468, 473 / 474
 // Passing over the dead tiles between live ones too, by a list of the live ones, cost 1 to 2 % of every masked launch in the tile
 // loop, and skipping those ahead of the first live one 0.3 us of a second copy of the first scores.
 //
 // Persistent form (MODE 2), a measurement aid that no default launch uses (ODIT_ATTN_PERSISTENT=1 in the
-// environment turns it on for launches of 4-wavefront workgroups, i.e. with ODIT_ATTN_WAVES=4 at head size 128). With more units than workgroup slots the launch has as many workgroups as run at
-// once, and each runs unit after unit as ONE stream of key tiles: the tile pipeline runs across the unit
+// environment turns it on for launches of 4-wavefront workgroups, i.e. with ODIT_ATTN_WAVES=4 at head size 128). With
+// more units than workgroup slots the launch has as many workgroups as run at once, and each runs unit after unit as ONE stream of key tiles: the tile pipeline runs across the unit
 // boundary. Units are handed out dynamically: every XCD owns a contiguous eighth of the units (neighbours in
 // (q block, head) order share keys and values in its L2), its workgroups start on the first ones and draw the
 // next from the XCD's ticket word in scratch whenever they begin a unit, one unit ahead of need, so the draw's
@@ -769,8 +770,9 @@ static int persistent_workgroups(int units, int n_tiles, int slots, int nw) {
 }
 
 // Batch rows of a masked launch differ in their live tiles, and xcd_remap gives whole batch rows to some of the XCDs: those with
-// the longest row finish last (B=2, one row of 22 tiles and one of 9, 704 units: the XCDs 0 to 3 had 88 units of 22 tiles each). Where the heads divide evenly every XCD gets its share of each row's heads instead, as many in all (keys
-// and values are shared in its L2 as before), by a grid whose linear index runs over the XCDs first.
+// the longest row finish last (B=2, one row of 22 tiles and one of 9, 704 units: the XCDs 0 to 3 had 88 units of 22 tiles each).
+// Where the heads divide evenly every XCD gets its share of each row's heads instead, as many in all (keys and values are shared
+// in its L2 as before), by a grid whose linear index runs over the XCDs first.
 // (With units for less than half the slots each has a compute unit, or nearly, to itself either way.)
 static bool spread_batch(const AttnParams& p, int slots) {
   return p.B > 1 && p.B < 65536 && p.H % kNumXcd == 0 && p.n_full == p.total_blocks && 2 * p.total_blocks > slots;

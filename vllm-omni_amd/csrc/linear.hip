@@ -3,12 +3,12 @@
 //   * out = residual + gate * (x W^T + bias)  (attention / MLP output projections: no separate
 //                                              gated-residual pass)
 // Which kernel runs is decided here per call. Few rows: the hand-written stream-K kernel (gemm_bf16.hip) where the reduction is
-// long, and a kernel for products that are small altogether (gemm_small.hip). Many rows: the hand-written tile kernel (gemm_bf16_tile.hip) or hipBLASLt's MFMA kernels, by expected time. The two
-// streams of a dual-stream block: one launch of either hand-written kernel, or two calls, by expected time
-// (odit_linear_pair). For the library this file sets the problem up so
-// that its epilogue does the elementwise work (bias vector, activation, a per-output-feature alpha vector for the gate, beta = 1
-// on the residual), keeps problem descriptors per thread, chooses among the library's candidates for long reductions by expected
-// time, and has an explicit tuning call that times all engines for one problem and remembers the fastest.
+// long, and a kernel for products that are small altogether (gemm_small.hip). Many rows: the hand-written tile kernel
+// (gemm_bf16_tile.hip) or hipBLASLt's MFMA kernels, by expected time. The two streams of a dual-stream block: one launch of a
+// hand-written kernel, or two calls, by expected time (odit_linear_pair). For the library this file sets the problem up so that
+// its epilogue does the elementwise work (bias vector, activation, a per-output-feature alpha vector for the gate, beta = 1 on the
+// residual), keeps problem descriptors per thread, chooses among the library's candidates for long reductions by expected time, and
+// has an explicit tuning call that times the library's kernels and the hand-written ones for one problem and remembers the fastest.
 //
 // Row-major y[M,N] = x[M,K] W[N,K]^T is the column-major product D(N x M) = op(A) B with A = W stored
 // K x N (ld = ldw, transposed), B = x stored K x M (ld = ldx): the bias and the alpha vector run along
@@ -184,7 +184,7 @@ struct LinCall {
   size_t ws_bytes;
   hipStream_t stream;
   bool first = false;    // the library's first-ranked kernel, unless one was tuned (ODIT_LINEAR_FIRST)
-  bool no_tile = false;  // untuned, not the tile kernel (ODIT_LINEAR_NO_TILE)
+  bool no_tile = false;  // untuned, neither the tile nor the small kernel (ODIT_LINEAR_NO_TILE)
 };
 
 static bool lin_is_residual(const LinCall& c) {
@@ -532,9 +532,10 @@ static bool lin_streamk_rule(const odit::GemmCall& g) {
 
 // The kernel of a problem that names no engine: what a tuning call found, else the stream-K kernel by its rule or the tile kernel,
 // whose expected time is shorter (N=3072, K=12288, us, stream-K / tile: 300 rows 43 / 49, 400 48 / 49, 512 52 / 56, 592 61 / 55, 1024
-// 84 / 75; N=5120, K=13824: 200 62 / 60, 300 65 / 60, 592 101 / 86, 1024 144 / 112), else the kernel for small products (3) by its rule, else the tile kernel where its expected time is below the library's (kTileMinAuto rows or
-// more), else the library (0). One launch of the library takes 8 to 10 us for any small product, the small kernel 4 to 7 up to
-// K = kSmallK; beside a second problem, whose launch it saves, up to kSmallPairK.
+// 84 / 75; N=5120, K=13824: 200 62 / 60, 300 65 / 60, 592 101 / 86, 1024 144 / 112), else the kernel for small products (3) by its
+// rule, else the tile kernel where its expected time is below the library's (kTileMinAuto rows or more), else the library (0). One
+// launch of the library takes 8 to 10 us for any small product, the small kernel 4 to 7 up to K = kSmallK; beside a second
+// problem, whose launch it saves, up to kSmallPairK.
 constexpr int kSmallK = 1024, kSmallPairK = 2048;
 constexpr int kTileMinAuto = 256;
 

@@ -1031,9 +1031,6 @@ bool project_gated_pair(BlockCall& c, const void* const x[2], const Lin l[2], co
   return true;
 }
 
-// One allocation for a block's intermediate tensors. What is dead before another part begins shares its memory: after
-// `mark`, every `rewind` starts laying out from there again, over what came since (all launches are on one stream). A Wan
-// block of 2 x 32760 rows and width 5120 takes 4.7 GB this way; with every part apart it took 7.2.
 // y[i] = x W[i]^T + b[i] for two projections of the same rows (GELU on the first where `gelu`): one launch where that is the better way
 void project_fork(BlockCall& c, const void* x, const Lin l[2], void* const y[2], int64_t M, bool gelu) {
   if (c.rc != 0) return;
@@ -1051,6 +1048,9 @@ void project_fork(BlockCall& c, const void* x, const Lin l[2], void* const y[2],
   for (int i = 0; i < 2; ++i) c.project(x, l[i], y[i], M, gelu && i == 0);
 }
 
+// One allocation for a block's intermediate tensors. What is dead before another part begins shares its memory: after
+// `mark`, every `rewind` starts laying out from there again, over what came since (all launches are on one stream). A Wan
+// block of 2 x 32760 rows and width 5120 takes 4.7 GB this way; with every part apart it took 7.2.
 struct Slab {
   Tensor t;
   size_t at = 0, marked = 0, size = 0;

@@ -681,10 +681,10 @@ def _flush_buffer(device: torch.device) -> int:
 
 def set_linear_autotune(iters: int) -> None:
     """With iters > 0, the first ``linear`` call of every new problem (shape, strides, epilogue, dtype)
-    first times the library's kernels for it on scratch copies of the output operands (a blocking,
-    one-off cost of some tenths of a second) and keeps the fastest for the rest of the process. Meant to
-    be switched on around a warm-up pass and off again; 0 = use the library's own first choice for
-    problems not tuned yet."""
+    first times the library's kernels and the hand-written ones for it on scratch copies of the output
+    operands (a blocking, one-off cost of some tenths of a second) and keeps the fastest for the rest of the
+    process (a kernel of the library's for the calls of this thread). Meant to be switched on around a
+    warm-up pass and off again; 0 = problems not tuned yet take the kernel that the rules choose."""
     global _LINEAR_AUTOTUNE_ITERS
     _LINEAR_AUTOTUNE_ITERS = int(iters)
     if _LINEAR_AUTOTUNE_ITERS <= 0:
@@ -698,8 +698,9 @@ _LINEAR_ENGINE_FLAGS = 0
 def set_linear_engine(engine: str) -> None:
     """Which kernel later ``linear`` calls of this process ask for when they name none themselves: "auto" (a
     hand-written kernel where a tuning run found it faster or its default rule says so, the library
-    elsewhere), "no_tile" (the same without the tile kernel's rule), "library" (hipBLASLt always) or "handwritten" (the hand-written kernel for the row count
-    always; problems it does not take raise). The choice travels with every call as a flag of
+    elsewhere), "no_tile" (the same without the rules of the tile and the small kernel), "library" (hipBLASLt
+    always) or "handwritten" (the hand-written kernel for the row count always: stream-K up to 1024 rows, tile
+    above; problems it does not take raise). The choice travels with every call as a flag of
     ``odit_linear_rows``; the library keeps no switch. For measurements and tests."""
     global _LINEAR_ENGINE_FLAGS
     if engine not in _LINEAR_ENGINES:
@@ -717,7 +718,7 @@ def _linear_workspace(lib, device: torch.device) -> torch.Tensor:
 
 
 def _linear_scratch(device: int, stream: int) -> torch.Tensor:
-    """The library's workspace and the stream-K kernel's ticket words and partial tiles."""
+    """The library's workspace and the stream-K and tile kernels' ticket words and partial tiles."""
     return _LINEAR_SCRATCH.get(device, stream, int(_lib.load().odit_linear_workspace_bytes()))
 
 
@@ -739,8 +740,9 @@ def linear_few(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None 
 
 
 def project(lin: torch.nn.Module, x: torch.Tensor, silu_input: bool = False) -> torch.Tensor:
-    """lin(x) or lin(silu(x)) for a Linear module of a model's stem, conditioning or head. A plain ``nn.Linear`` in inference goes down as one native call; a module with hooks or of another
-    class, and everything the kernels do not take, is called as it is."""
+    """lin(x) or lin(silu(x)) for a Linear module of a model's stem, conditioning or head. A plain ``nn.Linear`` in inference
+    goes down as one native call; a module with hooks or of another class, and everything the kernels do not take, is called
+    as it is."""
     if x.is_cuda and native_blocks():
         done = (_nat or _load_native()).project(lin, x, silu_input, _LINEAR_ENGINE_FLAGS)
         if done is not None:
@@ -797,14 +799,15 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = No
 
     activation="gelu_tanh": GELU(tanh) of the result. residual (same shape as the result) with optional
     gate [B,N] / [B,1,N] / [N]: ``residual + gate * (x W^T + bias)``; gates that differ per batch row go
-    down as one call (one launch of the hand-written kernel, or one library launch per batch row). ``prescaled=True``: ``gate`` is float32 and ``gate_bias`` (float32, same shape, or
-    None) already holds gate * bias — nothing is derived per call (``bias`` is then ignored).
+    down as one call (one launch of a hand-written kernel, or one library launch per batch row). ``prescaled=True``:
+    ``gate`` is float32 and ``gate_bias`` (float32, same shape, or None) already holds gate * bias — nothing is
+    derived per call (``bias`` is then ignored).
     ``weight`` may be a column range of a Linear weight (row stride > K).
-    ``tune_iters`` > 0 first times the library's kernels and the hand-written kernel for this problem
-    (overwrites ``out``), keeps the faster for later calls and returns its time in microseconds instead
-    of the result. ``plan_only`` launches nothing and returns (the hand-written kernel would run, number of
+    ``tune_iters`` > 0 first times the library's kernels and the hand-written ones for this problem
+    (overwrites ``out``), keeps the fastest for later calls and returns its time in microseconds instead
+    of the result. ``plan_only`` launches nothing and returns (a hand-written kernel would run, number of
     kernel launches the call would make). ``engine``: "auto", "library", "handwritten" or "no_tile" (auto without the tile
-    kernel) for this call (default: what ``set_linear_engine`` chose).
+    and the small kernel) for this call (default: what ``set_linear_engine`` chose).
     """
     if engine is not None and engine not in _LINEAR_ENGINES:
         raise ValueError(f"engine must be one of {sorted(_LINEAR_ENGINES)}")
