@@ -398,7 +398,7 @@ int odit_linear_rows(const void* x, const void* w, const void* bias, void* out, 
  * image and the text rows of a dual-stream block (to_qkv beside add_kv_proj, qwen_image_transformer.py:566-580, and the output, up
  * and down projections).
  * Fields as the arguments of odit_linear_rows. Returns ODIT_ENOTSUP, with nothing launched, where two odit_linear_rows calls
- * are the better way (by expected time, or by the time that a tuning call measured for one of the problems) or the kernels do
+ * are the better way (by expected time, or the time that a tuning call measured for a problem if that is shorter) or the kernels do
  * not take a problem; the caller then makes them. flags as for
  * odit_linear_rows (ODIT_LINEAR_LIBRARY: always ODIT_ENOTSUP; ODIT_LINEAR_HANDWRITTEN: the stream-K kernel;
  * ODIT_LINEAR_NO_TILE and ODIT_LINEAR_FIRST: the stream-K kernel by its rule or ODIT_ENOTSUP). */

@@ -204,6 +204,26 @@ def test_pair_of_tuned_problems_is_one_launch_where_that_is_faster(kernels, gpu)
         assert _pair(lib, ws, q, N, K, 1, 0) == 0
 
 
+def test_pair_that_is_two_calls_stays_two_calls_when_tuned(kernels, gpu):
+    """Two calls take 103 us, one launch 106. What a tuning call measures behind its cache flush is longer than a call in a model."""
+    from vllm_omni_amd import _lib
+
+    M0, M1, N, K = 1122, 185, 12288, 3072
+    lib = _lib.load()
+    ws = kernels._linear_scratch(gpu.index or 0, torch.cuda.current_stream().cuda_stream)
+    q, ops = (_lib.LinearProblem * 2)(), []
+    for i, m in enumerate((M0, M1)):
+        x, w, b, _ = _mk(gpu, m, N, K, torch.bfloat16, m)
+        out = torch.empty(m, N, dtype=torch.bfloat16, device=gpu)
+        q[i].x, q[i].w, q[i].bias, q[i].out, q[i].M = x.data_ptr(), w.data_ptr(), b.data_ptr(), out.data_ptr(), m
+        q[i].ldx, q[i].ldw, q[i].ldo, q[i].ldr = K, K, N, N
+        ops.append((x, w, b, out))
+    assert _pair(lib, ws, q, N, K, 1, 0) == -2  # ODIT_ENOTSUP
+    for x, w, b, out in ops:
+        kernels.linear(x, w, b, out=out, tune_iters=3)
+        assert _pair(lib, ws, q, N, K, 1, 0) == -2
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("M,N0,N1,K", [
     (1536, 12288, 9216, 3072),  # two rounds of whole 256-row tiles

@@ -547,10 +547,10 @@ static bool lin_candidate(int kind, const odit::GemmCall& g, int dtype, const vo
   return kind == 2 || odit::gemm_small_rule(&g, 1, odit::device_cus(), kSmallPairK);
 }
 
-// time of a problem's own call: what a tuning call measured, else the better of what it may run on, by expectation
+// Time of a problem's own call: the better of what it may run on, by expectation, or what a tuning call measured where that is
+// shorter. (It is behind a flush often 5 to 10 us longer than in a model: taken for itself it made two calls look slower than they
+// are, and 1122 + 185 rows, N=12288, K=3072, 103 us in two calls, went to one launch of 106.)
 static float lin_call_us(int dev, const odit::LinCall& c, const odit::GemmCall& g, const void* sk) {
-  odit::Tuned found;
-  if (lin_tuned(dev, c, g, sk, &found)) return found.us;
   const bool scratch = sk != nullptr;
   float us = lin_library_us(c, g);
   const int cus = odit::device_cus();
@@ -562,6 +562,8 @@ static float lin_call_us(int dev, const odit::LinCall& c, const odit::GemmCall& 
     const odit::TilePlan plan = odit::plan_gemm_tile(&g, 1, cus, scratch);
     if (plan.bm > 0 && plan.us < us) us = plan.us;
   }
+  odit::Tuned found;
+  if (lin_tuned(dev, c, g, sk, &found) && found.us < us) us = found.us;
   return us;
 }
 static int lin_rule_kind(const odit::LinCall& c, const odit::GemmCall& g, const void* sk) {
@@ -650,7 +652,7 @@ extern "C" int odit_linear_rows(const void* x, const void* w, const void* bias, 
   return ODIT_OK;
 }
 
-// Two problems in one launch, or two calls? By expected time; for the call of a problem that was tuned, by what was measured (811
+// Two problems in one launch, or two calls? By expected time, or what was measured for a tuned problem if that is shorter (811
 // + 466 rows, N=9216, K=3072: 73 us in one launch, 93 in two tuned calls; 1216 + 448, N=6144, K=1024: 30 and 36). One launch has
 // one set of overheads for both, shares the tiles of the last round out over all CUs and takes gates that differ per batch
 // entry, for which the library needs a call per entry.
