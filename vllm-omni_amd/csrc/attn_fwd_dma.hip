@@ -104,15 +104,17 @@ typedef __attribute__((address_space(3))) void* lds_void_p;
 //         result in scratch for attn_merge_kernel.
 // MODE 2: persistent, see above.
 // MODE 3, 4: 0 and 1 for a key mask held as words. MODE 5: 3 with the batch rows spread over the XCDs (spread_batch).
+// MODE 6, 7, 8: 0, 3 and 5 of head size 64 with three workgroups per compute unit (fills_three).
 // Separate instantiations, so the extra bookkeeping of one cannot disturb the register allocation of another (that of the
 // words in the launches without a mask: 452 -> 460 us at B=2 S=4352 H=24 D=128, 252 -> 262 at B=1 S=4608).
 constexpr int kMaskWords = 1024;  // 8 KB of LDS: two workgroups of D = 128 still fit a compute unit (144 of 160 KB)
 
 template <typename T, int D, int NW, int MODE>
-__global__ __launch_bounds__(NW * 64, 8 / NW) void attn_fwd_dma_kernel(const AttnParams p) {
+__global__ __launch_bounds__(NW * 64, MODE >= 6 ? 3 : 8 / NW) void attn_fwd_dma_kernel(const AttnParams p) {
   constexpr bool TAIL = MODE == 1 || MODE == 4;
   constexpr bool PERSIST = MODE == 2;
-  constexpr bool WORDS = MODE >= 3;
+  constexpr bool WORDS = MODE >= 3 && MODE != 6;
+  constexpr bool THREE = MODE >= 6, SPREAD = MODE == 5 || MODE == 8;
   using M = Mma<T>;
   using frag = typename M::frag;
   constexpr int BN = 64;
@@ -144,9 +146,13 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void attn_fwd_dma_kernel(const Att
   const int part = blockIdx.x;
   // persistent form: the unit after the current one (-1: none, or not drawn yet)
   int next_pid = -1;
+  // three wavefronts per SIMD: 168 registers, so most of the query fragments stay in LDS and fewer reads run ahead
+  static_assert(!THREE || (D == 64 && NW == 4), "three workgroups per compute unit: head size 64");
+  constexpr int QL = THREE ? (WORDS ? 3 : 4) : 0;
+  __shared__ u32x4_v q_lds[QL > 0 ? NW * QL * 64 : 1];
   __shared__ int next_unit_box;  // thread 0's draw, handed to the workgroup across a tile's barrier
   __shared__ uint64_t mask_words[WORDS ? kMaskWords : 1];  // of key tiles jt0, jt0 + 1, ...
-  if constexpr (MODE == 0 || MODE == 3 || MODE == 5) {
+  if constexpr (!TAIL && !PERSIST) {
     pid = xcd_remap(blockIdx.x, p.n_full);
   } else if constexpr (TAIL) {  // this workgroup covers key tiles [jt0, n_tiles) of unit pid (jt0 is even)
     pid = p.n_full + part / p.key_chunks;
@@ -170,7 +176,7 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void attn_fwd_dma_kernel(const Att
   int h = (pid / p.n_qblocks) % p.H;
   int b = (pid / p.n_qblocks) / p.H;
   int q0 = (pid % p.n_qblocks) * BM + wave * 32;
-  if constexpr (MODE == 5) {
+  if constexpr (SPREAD) {
     h = blockIdx.x % kNumXcd * (p.H / kNumXcd) + blockIdx.y;
     b = blockIdx.z;
     q0 = blockIdx.x / kNumXcd * BM + wave * 32;
@@ -316,6 +322,9 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void attn_fwd_dma_kernel(const Att
       qf[ks] = __builtin_bit_cast(frag, *reinterpret_cast<const u32x4_v*>(qp + ks * 16));
   };
   load_q(b, h, q0);
+  auto q_kept = [&](int ks) { return __builtin_bit_cast(frag, q_lds[(wave * QL + ks - (KS - QL)) * 64 + lane]); };  // (each lane its own)
+#pragma unroll
+  for (int i = 0; i < QL; ++i) q_lds[(wave * QL + i) * 64 + lane] = __builtin_bit_cast(u32x4_v, qf[KS - QL + i]);
 
   f32x16_v o[DT];
 #pragma unroll
@@ -346,7 +355,7 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void attn_fwd_dma_kernel(const Att
       for (int kt = 0; kt < 2; ++kt) {
         const frag a = __builtin_bit_cast(
             frag, *reinterpret_cast<const u32x4_v*>(kt_base + kt * 32 * ROWB + (k_lane ^ (ks * 32))));
-        s[kt] = M::run(a, qf[ks], s[kt]);
+        s[kt] = M::run(a, ks < KS - QL ? qf[ks] : q_kept(ks), s[kt]);
       }
   };
 
@@ -502,19 +511,22 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void attn_fwd_dma_kernel(const Att
       for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
         for (int e = 0; e < 16; ++e) s_next[kt][e] = 0.f;
-      constexpr int KPF = ODIT_ATTN_KPF;  // K fragments in flight ahead of the MFMA that consumes them
+      constexpr int KPF = THREE ? 2 : ODIT_ATTN_KPF;  // K fragments in flight ahead of the MFMA that consumes them
       u32x4_v kfr[KPF + 1];
       auto k_fetch = [&](int i) {
         const int ks = i >> 1, kt = i & 1;
         kfr[i % (KPF + 1)] = *reinterpret_cast<const u32x4_v*>(kt_base + kt * 32 * ROWB + (k_lane_t ^ (ks * 32)));
       };
+      frag qt[2];
+      if constexpr (QL == KS) qt[0] = q_kept(0);
 #pragma unroll
       for (int i = 0; i < KPF; ++i) k_fetch(i);
 #pragma unroll
       for (int i = 0; i < 2 * KS; ++i) {
         if (i + KPF < 2 * KS) k_fetch(i + KPF);
         const int ks = i >> 1, kt = i & 1;
-        s_next[kt] = M::run(__builtin_bit_cast(frag, kfr[i % (KPF + 1)]), qf[ks], s_next[kt]);
+        if (kt == 0 && ks + 1 < KS && ks + 1 >= KS - QL) qt[(ks + 1) & 1] = q_kept(ks + 1);
+        s_next[kt] = M::run(__builtin_bit_cast(frag, kfr[i % (KPF + 1)]), ks < KS - QL ? qf[ks] : qt[ks & 1], s_next[kt]);
         constexpr int PAIRS = 16 / (2 * KS) > 0 ? 16 / (2 * KS) : 1;
 #pragma unroll
         for (int q = 0; q < PAIRS; ++q) {
@@ -570,7 +582,7 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void attn_fwd_dma_kernel(const Att
     int v_lane_t = v_lane;  // (opaque copy, as for the key fragments)
     if constexpr (PERSIST) asm volatile("" : "+v"(v_lane_t));
     constexpr int NSTEP = 4 * DT;
-    constexpr int PF = ODIT_ATTN_VPF;
+    constexpr int PF = THREE ? 2 : ODIT_ATTN_VPF;
     s16x4_d vlo[PF + 1], vhi[PF + 1];
     auto v_fetch = [&](int step) {
       const int dt = step % DT, kt = (step / DT) >> 1, g2 = (step / DT) & 1;
@@ -778,6 +790,16 @@ static bool spread_batch(const AttnParams& p, int slots) {
   return p.B > 1 && p.B < 65536 && p.H % kNumXcd == 0 && p.n_full == p.total_blocks && 2 * p.total_blocks > slots;
 }
 
+// Head size 64 in three workgroups per compute unit instead of two, where they take all units in one round and two would need a
+// second one that the key split does not take. Three wavefronts on a SIMD multiply no faster than two (the vector work of the
+// softmax fills either: B=2 S=4352 H=24 283 us, three everywhere 297; 1024 units of 128 key tiles 315 and 380), so it is a
+// matter of the rounds alone: up to 1.5 rounds of two are one round of three, in which a unit takes 1.5 times as long, and a second
+// round of two takes 0.6 of a first one, its workgroups having a compute unit each. us, two / three, 688 to 752 units:
+//   B=2 S=1357 H=32 f16 54.8 / 48.6, with a padded row 44.5 / 40.7    B=1 S=5500 H=16 174.5 / 151.4, 500 keys 24.2 / 20.8,
+//   64 keys 11.2 / 10.3    B=1 S=12000 H=8 397 / 336    B=3 S=700 H=40 30.8 / 27.1
+// 544 units whose keys are too few to be split (B=1 S=2060, 300 keys, H=32): 18.4 / 14.8.
+static bool fills_three(const TailPlan& t, int units, int slots) { return t.rem == 0 && units > slots && 2 * units <= 3 * slots; }
+
 template <typename T, int D, int NW>
 static int launch_dma(AttnParams& p, hipStream_t stream, void* ws, size_t ws_bytes) {
   constexpr int BM = NW * 32;
@@ -821,7 +843,14 @@ static int launch_dma(AttnParams& p, hipStream_t stream, void* ws, size_t ws_byt
         hipLaunchKernelGGL((attn_fwd_dma_kernel<T, D, NW, 2>), dim3(W), dim3(NW * 64), 0, stream, p);
       }
     }
-    if (W == 0) {
+    const bool three = D == 64 && NW == 4 && W == 0 && fills_three(t, p.total_blocks, slots);
+    if constexpr (D == 64 && NW == 4) {
+      if (three && words && spread_batch(p, slots))
+        hipLaunchKernelGGL((attn_fwd_dma_kernel<T, D, NW, 8>), dim3(p.n_qblocks * kNumXcd, p.H / kNumXcd, p.B), dim3(NW * 64), 0, stream, p);
+      else if (three && words) hipLaunchKernelGGL((attn_fwd_dma_kernel<T, D, NW, 7>), dim3(p.n_full), dim3(NW * 64), 0, stream, p);
+      else if (three) hipLaunchKernelGGL((attn_fwd_dma_kernel<T, D, NW, 6>), dim3(p.n_full), dim3(NW * 64), 0, stream, p);
+    }
+    if (W == 0 && !three) {
       if (words && spread_batch(p, slots))
         hipLaunchKernelGGL((attn_fwd_dma_kernel<T, D, NW, 5>), dim3(p.n_qblocks * kNumXcd, p.H / kNumXcd, p.B), dim3(NW * 64), 0, stream, p);
       else if (words) hipLaunchKernelGGL((attn_fwd_dma_kernel<T, D, NW, 3>), dim3(p.n_full), dim3(NW * 64), 0, stream, p);
@@ -902,7 +931,8 @@ int attn_dma_plan(int B, int Sq, int Sk, int H, int D, bool with_workspace, char
     snprintf(main_text, sizeof(main_text), "attn_fwd_dma_kernel<T, %d, %d, 2> units=%lld on %d persistent workgroups", D,
              nw, static_cast<long long>(main_units), W);
   } else {
-    snprintf(main_text, sizeof(main_text), "attn_fwd_dma_kernel<T, %d, %d, 0> units=%lld", D, nw,
+    const bool three = D == 64 && nw == 4 && main_units <= 0x3fffffff && fills_three(t, static_cast<int>(main_units), slots);
+    snprintf(main_text, sizeof(main_text), "attn_fwd_dma_kernel<T, %d, %d, %d> units=%lld", D, nw, three ? 6 : 0,
              static_cast<long long>(main_units));
   }
   if (t.rem == 0) {
