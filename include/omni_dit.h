@@ -419,6 +419,29 @@ int odit_linear_pair(const odit_linear_problem problems[2], int N, int K, int ep
 int odit_linear_fork(const odit_linear_problem problems[2], const int N[2], int K, const int epilogue[2], int dtype, unsigned flags,
                      void* workspace, size_t workspace_bytes, void* stream);
 
+/* Two projections of the same K in one launch of the tile kernel, of which one or both are projections to query, key and value heads
+ * (heads[i] not NULL): N[i] = 3 H D features (bias or none), S rows of each batch entry (M = B S), whose queries and keys are normed
+ * over each head (mean of squares + eps), weighted and rotated in pairs (2 i, 2 i + 1) at the tile's end and stored with the values in
+ * rows offset .. offset + S - 1 of joint tensors [B, S_total, H D]: to_qkv and add_kv_proj with norm_q, norm_k, norm_added_q,
+ * norm_added_k and the rotary embedding of a dual-stream block (qwen_image_transformer.py:566-620), to_qkv beside proj_mlp of a
+ * single-stream block (flux_transformer.py:288-309). What odit_qknorm_rope makes of the projection's output (the same operations in the same
+ * order; of the two products of an odd feature's rotation the compiler may round the other one) without that output
+ * (problems[i].out is not used). The other problem as for odit_linear_fork. wq, wk [D] of `dtype`; cos, sin float32
+ * [S, D / 2]; D = 64 or 128; everything 16-byte aligned. launch = 0: nothing is launched, only the answer given. ODIT_ENOTSUP,
+ * with nothing launched, where the projections and the pass behind them are expected to be faster apart (ODIT_LINEAR_HANDWRITTEN: in
+ * one launch whatever is expected). */
+typedef struct odit_head_output {
+  void *q, *k, *v;
+  const void *wq, *wk;
+  const float *cos, *sin;
+  int S, offset, S_total, H, D;
+  float eps;
+} odit_head_output;
+
+int odit_linear_heads(const odit_linear_problem problems[2], const int N[2], int K, const int epilogue[2],
+                      const odit_head_output* const heads[2], int dtype, unsigned flags, int launch, void* workspace,
+                      size_t workspace_bytes, void* stream);
+
 /* odit_linear_rows of rows that lie in two tensors, x [M,K] beside x2 [M,K2] (W is [N, K + K2]), as one reduction in one launch
  * of the tile kernel: proj_out of a single-stream block without the concatenation (flux_transformer.py:303-309).
  * ODIT_ENOTSUP, with nothing launched, where two calls that add up are the better way. */

@@ -107,6 +107,9 @@ _SIGNATURES = {
         C.c_int, [C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_uint, C.c_void_p, C.c_size_t, C.c_void_p]),
     "odit_linear_fork": (
         C.c_int, [C.c_void_p, C.POINTER(C.c_int), C.c_int, C.POINTER(C.c_int), C.c_int, C.c_uint, C.c_void_p, C.c_size_t, C.c_void_p]),
+    "odit_linear_heads": (
+        C.c_int, [C.c_void_p, C.POINTER(C.c_int), C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_void_p), C.c_int, C.c_uint, C.c_int, C.c_void_p,
+                  C.c_size_t, C.c_void_p]),
     "odit_linear_join": (
         C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_int,
                   C.c_int64, C.c_int64, C.c_int64, C.c_int64, C.c_int64, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int64, C.c_uint,
@@ -155,6 +158,11 @@ class LinearProblem(C.Structure):
     _fields_ = [(n, C.c_void_p) for n in ("x", "w", "bias", "residual", "gate", "out")] + [("M", C.c_int), ("rows_per_gate", C.c_int)] + [
         (n, C.c_int64) for n in ("ldx", "ldw", "ldo", "ldr", "gate_stride")]
 
+class HeadOutput(C.Structure):
+    """``odit_head_output``."""
+
+    _fields_ = [(n, C.c_void_p) for n in ("q", "k", "v", "wq", "wk", "cos", "sin")] + [
+        (n, C.c_int) for n in ("S", "offset", "S_total", "H", "D")] + [("eps", C.c_float)]
 
 
 class OmniDitLibraryError(RuntimeError):

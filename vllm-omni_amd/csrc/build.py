@@ -28,7 +28,7 @@ NATIVE_SRC = CSRC / "native.cpp"
 NATIVE_PATH = PKG / "_native.so"
 OBJ_DIR = CSRC / "build"
 HEADERS = [CSRC / "odit_common.h", CSRC / "attn_common.h", CSRC / "attn_tail.h", CSRC / "gemm_bf16.h",
-           CSRC / "gemm_epilogue.h", PKG.parent / "include" / "omni_dit.h"]
+           CSRC / "gemm_epilogue.h", CSRC / "gemm_tile.h", PKG.parent / "include" / "omni_dit.h"]
 
 # (source file, extra defines, object stem)
 UNITS: list[tuple[str, list[str], str]] = [
@@ -46,6 +46,7 @@ UNITS: list[tuple[str, list[str], str]] = [
     ("step.hip", [], "step"),
     ("gemm_bf16.hip", [], "gemm_bf16"),
     ("gemm_bf16_tile.hip", [], "gemm_bf16_tile"),
+    ("gemm_tile_heads.hip", [], "gemm_tile_heads"),
     ("gemm_small.hip", [], "gemm_small"),
 ]
 PROBE_UNITS: list[tuple[str, list[str], str]] = [("probe.hip", [], "probe")]

@@ -70,6 +70,22 @@ TilePlan plan_gemm_tile(const GemmCall* c, int count, int cus, bool scratch);
 // one problem only.
 int launch_gemm_tile(const GemmCall* c, int count, const TileX2* x2, int dtype, void* scratch, hipStream_t stream);
 
+// ---- gemm_tile_heads.hip: the tile kernel with query, key and value heads at its end -------
+// Output of a projection to 3 HD features: per batch entry S rows of queries, keys and values of HD / D heads, the first two normed
+// over each head (mean of squares + eps), weighted and rotated in pairs (2 i, 2 i + 1), into rows offset .. of joint tensors [B, S_total, HD].
+struct HeadsOut {
+  void *q, *k, *v;
+  const void *wq, *wk;      // [D], of the tensors' type
+  const float *cos, *sin;   // [S, D / 2]
+  int S, offset, S_total, HD, D;
+  uint32_t div_mul, div_shift;  // (filled in by the launch)
+  float eps;
+};
+// beside gemm_tile_takes, of a call whose `out` is not used
+bool gemm_tile_heads_takes(const GemmCall& c, const HeadsOut& h);
+// One problem, or two of the same K; heads[i].q null: an ordinary output without a gate. `scratch` as for launch_gemm_tile.
+int launch_gemm_tile_heads(const GemmCall* c, int count, const HeadsOut* heads, int dtype, void* scratch, hipStream_t stream);
+
 // ---- gemm_small.hip: 64 x 64 output tiles, for products that are small altogether -------
 // One problem, or two of the same N and K in one launch, which gemm_streamk_takes takes. No scratch.
 bool gemm_small_rule(const GemmCall* c, int count, int cus, int max_k);

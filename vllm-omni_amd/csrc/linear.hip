@@ -743,6 +743,76 @@ extern "C" int odit_linear_fork(const odit_linear_problem* q, const int* N, int 
   return launch_gemm_tile(g, 2, nullptr, dtype, sk, static_cast<hipStream_t>(stream));
 }
 
+// Projections to query, key and value heads with the heads' norm and rotation at the tile's end, or the projections and a pass over
+// their output, by expected time. The pass takes 6 us and 8 bytes for every feature of q at 5 TB/s; the tile's end 4.5 us more a round
+// on 256-row tiles and 1.3 on 128-row ones (its arithmetic has no matrix work to hide behind; beside GELU tiles, whose end is
+// as long, nothing): what would be one launch of the tile kernel anyway nearly always takes the pass with it. Kernel time in a
+// model, us, projections + pass / one launch: 2048 + 342 rows, N=9216, K=3072 119 + 17 / 130; 1024 + 512 rows 73 + 11 / 79; 8192 + 512
+// rows 340 + 45 / 365; 1536 rows, N=12288 with GELU beside N=9216 153 + 10 / 157; 4608 rows 435 + 25 / 438. Few rows, where the
+// stream-K kernel takes the pair, stay there unless the tile kernel wins with its time of cold weights (kColdTile times the
+// expected one, which is of a round in which others fetch the same): 512 + 80 rows 48 + 6 / 56, in the model 0.5 % slower.
+constexpr float kColdTile = 1.18f;
+
+extern "C" int odit_linear_heads(const odit_linear_problem* q, const int* N, int K, const int* epilogue, const odit_head_output* const* heads, int dtype,
+                                 unsigned flags, int launch, void* workspace, size_t workspace_bytes, void* stream) {
+  using namespace odit;
+  ODIT_CHECK_ARG(q != nullptr && N != nullptr && epilogue != nullptr && heads != nullptr && (heads[0] != nullptr || heads[1] != nullptr),
+                 "odit_linear_heads: null arguments");
+  void *sk, *lib;
+  size_t lib_bytes;
+  lin_split_ws(workspace, workspace_bytes, &sk, &lib, &lib_bytes);
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) { set_error("odit_linear_heads: hipGetDevice failed"); return ODIT_ELAUNCH; }
+  const int engine = lin_engine_of(flags);
+  if (engine == 1 || (flags & (ODIT_LINEAR_FIRST | ODIT_LINEAR_NO_TILE)) != 0) return ODIT_ENOTSUP;
+  GemmCall g[2];
+  HeadsOut h[2];
+  LinCall calls[2];
+  float apart = 0.f, pass = 6.f;
+  bool both = true;
+  for (int i = 0; i < 2; ++i) {
+    h[i] = HeadsOut{};
+    LinCall& c = calls[i] = LinCall{q[i].x, q[i].w, q[i].bias, nullptr, nullptr, q[i].out, q[i].M, N[i], K, q[i].ldx, q[i].ldw, q[i].ldo, 0,
+                                    epilogue[i], dtype, dtype, lib, lib_bytes, static_cast<hipStream_t>(stream)};
+    if (heads[i] != nullptr) {
+      const odit_head_output& o = *heads[i];
+      ODIT_CHECK_ARG(o.S > 0 && o.H > 0 && o.D > 0 && o.offset >= 0 && o.offset + static_cast<int64_t>(o.S) <= o.S_total && q[i].M % o.S == 0 &&
+                         static_cast<int64_t>(o.H) * o.D * 3 == N[i] && static_cast<int64_t>(q[i].M / o.S) * o.S_total < (1ll << 31),
+                     "odit_linear_heads: rows or features do not fit the heads");
+      h[i] = HeadsOut{o.q, o.k, o.v, o.wq, o.wk, o.cos, o.sin, o.S, o.offset, o.S_total, o.H * o.D, o.D, 0, 0, o.eps};
+      c.out = o.q;
+      c.ldo = N[i];
+      pass += 8.f / 15e6f * q[i].M * N[i];
+    }
+    both = both && heads[i] != nullptr;
+    const int rc = lin_check(c);
+    if (rc != ODIT_OK) return rc;
+    ODIT_CHECK_ARG(!lin_is_residual(c), "odit_linear_heads: no residual");
+    g[i] = lin_gemm_call(c, 0, 0);
+    if (!gemm_tile_takes(g[i], dtype) || (heads[i] != nullptr && !gemm_tile_heads_takes(g[i], h[i]))) return ODIT_ENOTSUP;
+  }
+  if (engine == 2) return launch == 0 ? ODIT_OK : launch_gemm_tile_heads(g, 2, h, dtype, sk, static_cast<hipStream_t>(stream));
+  const int cus = device_cus();
+  const bool pair = both && N[0] == N[1], streamk_takes = pair && gemm_streamk_takes(g[0], dtype) && gemm_streamk_takes(g[1], dtype);
+  if (streamk_takes && gemm_small_rule(g, 2, cus, kSmallPairK)) return ODIT_ENOTSUP;
+  for (int i = 0; i < 2; ++i) apart += lin_call_us(dev, calls[i], g[i], sk);
+  const TilePlan plan = plan_gemm_tile(g, 2, cus, sk != nullptr);
+  if (plan.bm == 0) return ODIT_ENOTSUP;
+  const int rounds = (plan.tiles + cus - 1) / cus;
+  const float end = both ? (plan.bm == 256 ? 4.5f : 1.3f) * rounds : 0.f;
+  if (pair) {  // what odit_linear_pair would choose
+    apart *= kPairGain;
+    const int tiles = (g[0].M + kGemmBM - 1) / kGemmBM + (g[1].M + kGemmBM - 1) / kGemmBM;
+    const float streamk = sk != nullptr && streamk_takes && tiles <= kPairTiles ? gemm_streamk_us(g[0].M, g[1].M, N[0], K, cus) : 0.f;
+    if (streamk > 0.f && !(plan.us < apart && plan.us < streamk)) apart = streamk - (kColdTile - 1.f) * plan.us;
+  } else {
+    apart *= kOneLaunchGain;
+  }
+  if (plan.us + end >= (plan.us < apart ? plan.us : apart) + pass) return ODIT_ENOTSUP;
+  if (launch == 0) return ODIT_OK;
+  return launch_gemm_tile_heads(g, 2, h, dtype, sk, static_cast<hipStream_t>(stream));
+}
+
 // One projection of rows that lie in two tensors, in one reduction or as two products that add up, by expected time. One
 // reduction rounds once, and reads and writes the output once (M=1536, N=3072, K=12288 and 3072: 128 us, two calls 166).
 extern "C" int odit_linear_join(const void* x, const void* x2, const void* w, const void* bias, void* out, const void* residual, const void* gate,

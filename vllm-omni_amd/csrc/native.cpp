@@ -1048,6 +1048,28 @@ void project_fork(BlockCall& c, const void* x, const Lin l[2], void* const y[2],
   for (int i = 0; i < 2; ++i) c.project(x, l[i], y[i], M, gelu && i == 0);
 }
 
+// Two projections of which one or both go to query, key and value heads, in one launch: heads[i].q null is an ordinary output y[i]
+// (GELU where `gelu`). launch false: whether they would. False, with nothing launched, where the projections and the pass behind
+// them are the better way.
+bool project_heads(BlockCall& c, const void* const x[2], const Lin l[2], void* const y[2], const int64_t M[2], const odit_head_output heads[2],
+                   bool gelu, bool launch) {
+  if (c.rc != 0) return true;
+  if (l[0].k != l[1].k || (c.engine & ODIT_LINEAR_HANDWRITTEN)) return false;
+  odit_linear_problem q[2];
+  const odit_head_output* h[2];
+  int n[2], epi[2];
+  for (int i = 0; i < 2; ++i) {
+    q[i] = {x[i], l[i].w, l[i].b, nullptr, nullptr, y[i], static_cast<int>(M[i]), 0, l[i].k, l[i].ldw, l[i].n, 0, 0};
+    h[i] = heads[i].q ? &heads[i] : nullptr;
+    n[i] = static_cast<int>(l[i].n);
+    epi[i] = !h[i] && gelu ? (l[i].b ? ODIT_EPI_BIAS_GELU_TANH : ODIT_EPI_GELU_TANH) : (l[i].b ? ODIT_EPI_BIAS : ODIT_EPI_NONE);
+  }
+  const int rc = odit_linear_heads(q, n, static_cast<int>(l[0].k), epi, h, c.dtype, c.engine, launch, c.lin_ws.p, c.lin_ws.bytes, c.where.stream);
+  if (rc == ODIT_ENOTSUP && !launch) return false;
+  c.check(rc);
+  return true;
+}
+
 // One allocation for a block's intermediate tensors. What is dead before another part begins shares its memory: after
 // `mark`, every `rewind` starts laying out from there again, over what came since (all launches are on one stream). A Wan
 // block of 2 x 32760 rows and width 5120 takes 4.7 GB this way; with every part apart it took 7.2.
@@ -1131,21 +1153,34 @@ bool run_dual(BlockCall& c, const DualBlock& k, const Tensor& img, const Tensor&
   for (int d = 0; pre && d < 3; ++d)
     if (gates->size(d) > 1 && gates->stride(d) != gbias->stride(d)) return false;
   const int esz = 2;
-  // values are read where the projections left them when the text rows are whole key tiles and 32-bit offsets reach them
-  const bool v_in_place = S[1] % 64 == 0 && (Sj + 64) * 3 * HD * esz < (1ll << 31);
   const size_t attn_need = odit_attn_fwd_workspace_bytes(B, Sj, Sj, H, D);
   Scratch attn_ws;
   if (attn_need > 0 && !attn_scratch(c.where, attn_need, &attn_ws)) { c.rc = -100; return true; }
   const Unlocked others_run;  // to the end
 
-  void *n[2], *qkv[2], *jq, *jk, *jv = nullptr, *o[2], *u[2], *tmp;
+  void *n[2], *qkv[2] = {nullptr, nullptr}, *jq, *jk, *jv = nullptr, *o[2], *u[2], *tmp;
+  const int64_t M[2] = {B * S[0], B * S[1]};
+  // the heads of both streams (image, text) as the projections may leave them: `at` is any aligned address while nothing is launched
+  odit_head_output heads[2];
+  auto heads_at = [&](void* q, void* kk, void* v) {
+    for (int i = 0; i < 2; ++i)
+      heads[i] = {q, kk, v, k.nq[i], k.nk[i], cos[i]->data_ptr<float>(), sin[i]->data_ptr<float>(), static_cast<int>(S[i]),
+                  i == 0 ? static_cast<int>(S[1]) : 0, static_cast<int>(Sj), static_cast<int>(H), static_cast<int>(D), static_cast<float>(k.eps_qk)};
+  };
+  void* const at = img.data_ptr();
+  heads_at(at, at, at);
+  const void* const any[2] = {at, at};
+  const bool fused = k.w_dtype == c.dtype && 2 * cos[0]->size(1) == D && project_heads(c, any, k.qkv, qkv, M, heads, false, false);
+  if (c.rc != 0) return true;
+  // values are read where the projections left them when the text rows are whole key tiles and 32-bit offsets reach them
+  const bool v_in_place = !fused && S[1] % 64 == 0 && (Sj + 64) * 3 * HD * esz < (1ll << 31);
   Slab slab(esz);
   for (int i = 0; i < 2; ++i) {
     slab.want(&n[i], B * S[i] * C);
     slab.want(&o[i], B * S[i] * HD);
   }
   slab.mark();  // up to the attention
-  for (int i = 0; i < 2; ++i) slab.want(&qkv[i], B * S[i] * 3 * HD);
+  for (int i = 0; i < 2 && !fused; ++i) slab.want(&qkv[i], B * S[i] * 3 * HD);
   slab.want(&jq, B * Sj * HD);
   slab.want(&jk, B * Sj * HD);
   if (!v_in_place) slab.want(&jv, B * Sj * HD);
@@ -1202,9 +1237,13 @@ bool run_dual(BlockCall& c, const DualBlock& k, const Tensor& img, const Tensor&
   } else {
     norms(src, 0);
   }
-  const int64_t M[2] = {B * S[0], B * S[1]};
-  project_pair(c, n, k.qkv, qkv, M, false);
-  if (c.rc == 0) {  // problem 0 = text rows [0, S_txt), problem 1 = image rows
+  if (fused) {
+    heads_at(jq, jk, jv);
+    project_heads(c, n, k.qkv, qkv, M, heads, false, true);
+  } else {
+    project_pair(c, n, k.qkv, qkv, M, false);
+  }
+  if (c.rc == 0 && !fused) {  // problem 0 = text rows [0, S_txt), problem 1 = image rows
     auto part = [&](int stream, int which) { return static_cast<char*>(qkv[stream]) + which * HD * esz; };
     const void *qi[2] = {part(1, 0), part(0, 0)}, *ki[2] = {part(1, 1), part(0, 1)},
                *vi[2] = {v_in_place ? nullptr : part(1, 2), v_in_place ? nullptr : part(0, 2)}, *wq[2] = {k.nq[1], k.nq[0]},
@@ -1381,10 +1420,23 @@ PyObject* py_flux_single_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (attn_need > 0 && !attn_scratch(c.where, attn_need, &attn_ws)) return nullptr;
   std::optional<Unlocked> others_run(std::in_place);
   const int esz = 2;
-  void *nx, *q3, *q, *k, *o, *u;
+  void *nx, *q3 = nullptr, *q, *k, *v = nullptr, *o, *u;
   Slab slab(esz);
+  const Lin both[2] = {up, qkv};
+  const int64_t M[2] = {B * S, B * S};
+  odit_head_output heads[2] = {};
+  auto heads_at = [&](void* q_, void* k_, void* v_) {
+    heads[1] = {q_, k_, v_, wq, wk, cos->data_ptr<float>(), sin->data_ptr<float>(), static_cast<int>(S), 0, static_cast<int>(S), static_cast<int>(H),
+                static_cast<int>(D), static_cast<float>(eps_qk)};
+  };
+  void* const at = x->data_ptr();
+  heads_at(at, at, at);
+  const void* const any[2] = {at, at};
+  void* const any_out[2] = {at, at};
+  const bool fused = w_dtype == c.dtype && 2 * cos->size(1) == D && project_heads(c, any, both, any_out, M, heads, true, false);
   slab.want(&nx, B * S * C);
-  slab.want(&q3, B * S * 3 * HD);
+  if (fused) slab.want(&v, B * S * HD);
+  else slab.want(&q3, B * S * 3 * HD);
   slab.want(&q, B * S * HD);
   slab.want(&k, B * S * HD);
   slab.want(&o, B * S * HD);
@@ -1395,19 +1447,24 @@ PyObject* py_flux_single_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const char* mp = static_cast<const char*>(mod->data_ptr());
   c.check(odit_adaln_modulate(x->data_ptr(), nx, mp, mp + C * esz, nullptr, nullptr, nullptr, nullptr, nullptr, B, S, C, rs, rs, ms, 0,
                               static_cast<float>(eps), c.dtype, c.dtype, 0u, c.where.stream));
-  const Lin both[2] = {up, qkv};
   void* const into[2] = {u, q3};
-  project_fork(c, nx, both, into, B * S, true);
+  if (fused) {
+    heads_at(q, k, v);
+    const void* const rows[2] = {nx, nx};
+    project_heads(c, rows, both, into, M, heads, true, true);
+  } else {
+    project_fork(c, nx, both, into, B * S, true);
+  }
   const int64_t st[2] = {S * 3 * HD, 3 * HD};
   char* qp = static_cast<char*>(q3);
-  if (c.rc == 0)
+  if (c.rc == 0 && !fused)
     c.check(odit_qknorm_rope(qp, qp + HD * esz, nullptr, q, k, nullptr, wq, wk, cos->data_ptr<float>(), sin->data_ptr<float>(), B, S, H, D,
                              static_cast<int>(2 * cos->size(1)), st, 0, S, static_cast<float>(eps_qk), ODIT_NORM_HEAD, w_dtype, c.dtype, 0u,
                              c.where.stream));
   if (c.rc == 0) {
     const int64_t ds[3] = {S * HD, HD, D}, vs[3] = {S * 3 * HD, 3 * HD, D};
-    c.check(odit_attn_fwd_ex(q, k, qp + 2 * HD * esz, nullptr, 0, o, nullptr, 0, nullptr, nullptr, B, S, S, H, H, D, ds, ds, vs, nullptr, ds, nullptr,
-                             static_cast<float>(scale), c.dtype, attn_ws.p, attn_ws.bytes, c.where.stream));
+    c.check(odit_attn_fwd_ex(q, k, fused ? v : qp + 2 * HD * esz, nullptr, 0, o, nullptr, 0, nullptr, nullptr, B, S, S, H, H, D, ds, ds, fused ? ds : vs,
+                             nullptr, ds, nullptr, static_cast<float>(scale), c.dtype, attn_ws.p, attn_ws.bytes, c.where.stream));
   }
   // gate * proj_out(cat([attention, mlp])) + x: one reduction over both, or two accumulating products over the two column
   // ranges of the weight
