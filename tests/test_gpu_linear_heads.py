@@ -155,3 +155,34 @@ def test_heads_in_one_launch_where_that_is_expected_to_be_faster(scratch, gpu):
         ps = [_Problem(gpu, torch.bfloat16, 2, S, 3072, 24, 128, seed=S) for S in (S0, S1)]
         joint = [torch.empty(2, S0 + S1, 24, 128, dtype=torch.bfloat16, device=gpu) for _ in range(3)]
         assert _run(ps, (S1, 0), joint, 3072, torch.bfloat16, scratch, launch=0) == want
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,S0,S1,H,K", [
+    (1, 256, 64, 4, 256),   # whole tiles
+    (2, 75, 9, 4, 64),      # one step, batch entries that end inside a tile
+    (3, 100, 5, 3, 128),    # an odd number of heads
+    (1, 8, 65, 5, 512),     # fewer rows than a tile, one row more
+    (33, 1, 2, 2, 1024),    # batch entries of one and two rows, more steps than stages
+])
+def test_heads_of_small_products(scratch, gpu, dtype, B, S0, S1, H, K):
+    """The small kernel, whose tile is a head of 64: the bits of its pair launch and the pass behind it."""
+    print(f"small heads {dtype} B={B} {S0}+{S1} rows, {H} x 64, K={K}", flush=True)
+    ps = [_Problem(gpu, dtype, B, S0, K, H, 64, seed=7), _Problem(gpu, dtype, B, S1, K, H, 64, seed=8)]
+    joint = [torch.full((B, S0 + S1, H, 64), float("nan"), dtype=dtype, device=gpu) for _ in range(3)]
+    _lib.check(_run(ps, (S1, 0), joint, K, dtype, scratch), "odit_linear_heads")
+    _check(ps, (S1, 0), joint, dtype)
+    lib, code = _lib.load(), 0 if dtype == torch.bfloat16 else 1
+    q = (_lib.LinearProblem * 2)(*(p.linear() for p in ps))
+    N = 3 * H * 64
+    _lib.check(lib.odit_linear_pair(C.addressof(q), N, K, 1, code, code, 0, scratch.data_ptr(), scratch.numel(), _stream()), "odit_linear_pair")
+    want = [torch.full_like(t, float("nan")) for t in joint]
+    for p, o in zip(ps, (S1, 0)):
+        at = p.out.data_ptr()
+        _lib.check(lib.odit_qknorm_rope(at, at + H * 128, at + H * 256, *(t.data_ptr() for t in want), p.wq.data_ptr(), p.wk.data_ptr(), p.cos.data_ptr(),
+                                        p.sin.data_ptr(), B, p.S, H, 64, 64, _lib.i64_array([p.S * N, N]), o, S0 + S1, 1e-6, _lib.ODIT_NORM_HEAD, code, code, 0,
+                                        _stream()), "odit_qknorm_rope")
+    assert torch.equal(want[2], joint[2])
+    for a, b in zip(want[:2], joint[:2]):
+        assert torch.equal(a[..., 0::2], b[..., 0::2])
+        assert (a != b).float().mean().item() < 1e-3 and ((a.double() - b.double()).norm() / a.double().norm()).item() < 1e-4

@@ -28,7 +28,8 @@ NATIVE_SRC = CSRC / "native.cpp"
 NATIVE_PATH = PKG / "_native.so"
 OBJ_DIR = CSRC / "build"
 HEADERS = [CSRC / "odit_common.h", CSRC / "attn_common.h", CSRC / "attn_tail.h", CSRC / "gemm_bf16.h",
-           CSRC / "gemm_epilogue.h", CSRC / "gemm_tile.h", PKG.parent / "include" / "omni_dit.h"]
+           CSRC / "gemm_epilogue.h", CSRC / "gemm_tile.h",
+           CSRC / "gemm_heads.h", CSRC / "gemm_small.h", PKG.parent / "include" / "omni_dit.h"]
 
 # (source file, extra defines, object stem)
 UNITS: list[tuple[str, list[str], str]] = [
@@ -48,6 +49,7 @@ UNITS: list[tuple[str, list[str], str]] = [
     ("gemm_bf16_tile.hip", [], "gemm_bf16_tile"),
     ("gemm_tile_heads.hip", [], "gemm_tile_heads"),
     ("gemm_small.hip", [], "gemm_small"),
+    ("gemm_small_heads.hip", [], "gemm_small_heads"),
 ]
 PROBE_UNITS: list[tuple[str, list[str], str]] = [("probe.hip", [], "probe")]
 

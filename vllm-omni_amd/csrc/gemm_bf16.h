@@ -90,5 +90,7 @@ int launch_gemm_tile_heads(const GemmCall* c, int count, const HeadsOut* heads, 
 // One problem, or two of the same N and K in one launch, which gemm_streamk_takes takes. No scratch.
 bool gemm_small_rule(const GemmCall* c, int count, int cus, int max_k);
 int launch_gemm_small(const GemmCall* c, int count, int dtype, hipStream_t stream);
+// the same with query, key and value heads of 64 features (gemm_small_heads.hip)
+int launch_gemm_small_heads(const GemmCall* c, int count, const HeadsOut* heads, int dtype, hipStream_t stream);
 
 }  // namespace odit

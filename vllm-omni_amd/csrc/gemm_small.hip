@@ -1,168 +1,7 @@
-// 16-bit GEMM y = x W^T for products that are small altogether (models of a few hundred channels), one problem or two of the same
-// N and K in one launch: one 64 x 64 output tile per workgroup of 4 wavefronts, no reduction is divided.
-//
-// What bounds it: latency. A launch of some dozens of workgroups is one chain of arguments, first loads, matrix work, epilogue
-// operands and stores; at these sizes the work itself takes a microsecond. So everything that does not depend on the product is
-// asked for at once: bias, gate and residual go to registers and up to 8 steps of both operands (64 x 64 pieces of x and of W,
-// global memory straight into LDS, 16 KB a step) are in flight before anything is waited for, and the tile is stored from
-// registers. The stream-K kernel, which cuts reductions of four steps over several workgroups, spends most of its time on the
-// hand-over there. us, stream-K / this kernel: M=256+64, K=256: N=768 13.7 / 5.3, N=256 13.0 / 4.5, N=1024 with GELU 14.9 / 5.9;
-// N=256, K=1024 21.5 / 7.8. One problem, the library / this kernel: M=64, N=256, K=256 9.0 / 5.2.
-//
-// A wavefront owns 32 rows x 32 features as 2 x 2 accumulators of v_mfma_f32_16x16x32 with W rows as the A operand; the features
-// of the two accumulators interleave by 4, so that a lane ends up with 8 consecutive ones of a row. Chunks of 16 bytes are
-// XORed with bits of the row as in gemm_bf16_tile.hip. One barrier per step.
-#include "gemm_epilogue.h"
+// The rule and the launches of the kernel for small products (the kernel itself: gemm_small.h).
+#include "gemm_small.h"
 
 namespace odit {
-
-namespace {
-
-constexpr int kSmallTile = 64, kSmallStages = 8, kSmallPiece = kSmallTile * kGemmBK * 2, kSmallStage = 2 * kSmallPiece;
-
-struct SmallProblem {
-  const void *x, *w;
-  int M;
-  uint32_t ldx, ldw;  // bytes
-  uint32_t x_bytes, w_bytes;
-  GemmEpilogue ep;
-};
-
-struct SmallParams {
-  SmallProblem q[2];
-  int N, k_steps, n_tiles;
-  int tiles0;  // of the first problem
-};
-
-typedef __attribute__((address_space(3))) void* lds_void_p;
-
-// S: stages (as many as there are steps where those are fewer than 8: several workgroups to a CU)
-template <typename T, int S>
-__global__ __launch_bounds__(256) void gemm_small_kernel(const SmallParams p) {
-  using M = Mma16<T>;
-  using frag = typename M::frag;
-  __shared__ __attribute__((aligned(1024))) char lds[S * kSmallStage];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave & 1, wn = wave >> 1;
-  const int l16 = lane & 15, lq = lane >> 4;
-  const int which = static_cast<int>(blockIdx.x) >= p.tiles0 ? 1 : 0;
-  const SmallProblem& q = p.q[which];
-  const int t = static_cast<int>(blockIdx.x) - (which ? p.tiles0 : 0);
-  const int mt = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(t) / static_cast<unsigned>(p.n_tiles));
-  const int m0 = mt * kSmallTile, n0 = (t - mt * p.n_tiles) * kSmallTile;
-  const int nk = p.k_steps;
-
-  auto make_rsrc = [](const void* base, uint32_t bytes) {
-    const uint64_t a = reinterpret_cast<uint64_t>(base);
-    u32x4_v r;
-    r.x = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(a));
-    r.y = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(a >> 32) & 0xffffu);
-    r.z = __builtin_amdgcn_readfirstlane(bytes);
-    r.w = 0x00020000u;
-    return r;
-  };
-  const u32x4_v xr = make_rsrc(q.x, q.x_bytes), wr = make_rsrc(q.w, q.w_bytes);
-
-  // instruction j of this wavefront's share of a piece fills rows 16 wave + 8 j .. + 7; rows past the end re-read the last one
-  uint32_t vx[2], vw[2];
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int r = wave * 16 + j * 8 + (lane >> 3), ch = lane & 7;
-    const int rx = m0 + r < q.M ? m0 + r : q.M - 1, rw = n0 + r < p.N ? n0 + r : p.N - 1;
-    vx[j] = static_cast<uint32_t>(rx) * q.ldx + static_cast<uint32_t>((ch ^ ((r >> 1) & 7)) << 4);
-    vw[j] = static_cast<uint32_t>(rw) * q.ldw + static_cast<uint32_t>((ch ^ (((r >> 1) & 1) | (((r >> 3) & 3) << 1))) << 4);
-  }
-  const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void_p)lds)) + wave * 2048;
-  auto load = [&](uint32_t dst, uint32_t off, u32x4_v rs, int soff) {
-    load_lds16(__builtin_amdgcn_readfirstlane(dst), off, rs, __builtin_amdgcn_readfirstlane(soff));
-  };
-  auto issue = [&](int i, int stage) {
-    const uint32_t d = lds0 + stage * kSmallStage;
-    const int k = i * (kGemmBK * 2);
-    load(d, vx[0], xr, k);
-    load(d + 1024, vx[1], xr, k);
-    load(d + kSmallPiece, vw[0], wr, k);
-    load(d + kSmallPiece + 1024, vw[1], wr, k);
-  };
-
-  // operands of the epilogue: rows m, m + 16, features n .. n + 7
-  const GemmEpilogue& e = q.ep;
-  const int m = m0 + wm * 32 + l16, n = n0 + wn * 32 + lq * 8;
-  const bool gated = e.epilogue == ODIT_EPI_GATED_RESIDUAL || e.epilogue == ODIT_EPI_GATED_RESIDUAL_PRE;
-  const bool gelu = e.epilogue == ODIT_EPI_GELU_TANH || e.epilogue == ODIT_EPI_BIAS_GELU_TANH;
-  float gt[2][8], bs[2][8];
-  u32x4 res[2] = {};
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int row = m + 16 * i < q.M ? m + 16 * i : q.M - 1, col = n < p.N ? n : 0;
-    gemm_epilogue_vectors8<T>(e, row, col, gt[i], bs[i]);
-    if (gated) res[i] = load_raw(static_cast<const T*>(e.residual) + row * e.ldr + col);
-  }
-#pragma unroll
-  for (int d = 0; d < S; ++d)
-    if (d < nk) issue(d, d);
-
-  const int xrow = wm * 32 + l16;
-  const int xa = xrow * 128 + ((lq ^ ((xrow >> 1) & 7)) << 4);
-  const int wrow = wn * 32 + ((l16 >> 2) << 3) + (l16 & 3);
-  const int wa = kSmallPiece + wrow * 128 + ((lq ^ (((wrow >> 1) & 1) | (((wrow >> 3) & 3) << 1))) << 4);
-  f32x4_v acc[2][2];
-#pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int b = 0; b < 2; ++b) acc[a][b] = f32x4_v{0.f, 0.f, 0.f, 0.f};
-  for (int i = 0; i < nk; ++i) {
-    // this wavefront's loads of step i have landed and its reads of step i - 1 are in registers; behind the barrier that holds for
-    // every wavefront, and the stage of step i - 1 is free
-    if (S == kSmallStages && i + S - 2 < nk) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((kSmallStages - 2) * 4) : "memory");
-    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    if (S == kSmallStages && i > 0 && i - 1 + S < nk) issue(i - 1 + S, (i - 1) % S);
-    const char* st = lds + (i % S) * kSmallStage;
-    frag xf[2][2], wf[2][2];
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-      for (int a = 0; a < 2; ++a) {
-        xf[ks][a] = __builtin_bit_cast(frag, *reinterpret_cast<const u32x4_v*>(st + (xa ^ (ks * 64)) + a * 2048));
-        wf[ks][a] = __builtin_bit_cast(frag, *reinterpret_cast<const u32x4_v*>(st + (wa ^ (ks * 64)) + a * 512));
-      }
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-      for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b) acc[a][b] = M::run(wf[ks][b], xf[ks][a], acc[a][b]);
-  }
-
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    if (m + 16 * i >= q.M || n >= p.N) continue;
-    float y[8];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      y[u] = acc[i][0][u];
-      y[4 + u] = acc[i][1][u];
-    }
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      if (gated) {
-        y[u] = fmaf(gt[i][u], y[u], bs[i][u]) + Raw<T>::get(res[i], u);
-      } else {
-        y[u] += bs[i][u];
-        if (gelu) y[u] = gemm_gelu_tanh(y[u]);
-      }
-    }
-    u32x4 o;
-#pragma unroll
-    for (int u = 0; u < 4; ++u) Raw<T>::set2(o, u, y[2 * u], y[2 * u + 1]);
-    store_raw(static_cast<T*>(e.out) + (m + 16 * i) * e.ldo + n, o);
-  }
-}
-
-}  // namespace
 
 // Where the kernel is the one to run: every tile has a place at once (as many workgroups to a CU as its LDS holds; a second
 // round begins behind the whole latency of the first) and the reduction is short (a step takes 0.25 us). us with the host's part,
@@ -179,29 +18,16 @@ bool gemm_small_rule(const GemmCall* c, int count, int cus, int max_k) {
 }
 
 int launch_gemm_small(const GemmCall* c, int count, int dtype, hipStream_t stream) {
-  SmallParams p;
+  SmallArgs<false> p;
   int tiles[2] = {0, 0};
-  p.N = c[0].N;
-  p.n_tiles = (p.N + kSmallTile - 1) / kSmallTile;
-  p.k_steps = c[0].K / kGemmBK;
-  for (int i = 0; i < 2; ++i) {
-    const GemmCall& g = c[i < count ? i : 0];
-    SmallProblem& q = p.q[i];
-    q.x = g.x; q.w = g.w; q.M = g.M;
-    q.ldx = static_cast<uint32_t>(g.ldx * 2); q.ldw = static_cast<uint32_t>(g.ldw * 2);
-    q.x_bytes = static_cast<uint32_t>((static_cast<uint64_t>(g.M - 1) * g.ldx + g.K) * 2);
-    q.w_bytes = static_cast<uint32_t>((static_cast<uint64_t>(g.N - 1) * g.ldw + g.K) * 2);
-    q.ep = gemm_epilogue_of(g);
-    if (i < count) tiles[i] = (g.M + kSmallTile - 1) / kSmallTile * p.n_tiles;
-  }
-  p.tiles0 = tiles[0];
+  fill_small_params(p, c, count, tiles);
   const dim3 grid(tiles[0] + tiles[1]), block(256);
 #define ODIT_SMALL(T)                                                                                                    \
   do {                                                                                                                   \
-    if (p.k_steps == 1) hipLaunchKernelGGL((gemm_small_kernel<T, 1>), grid, block, 0, stream, p);                         \
-    else if (p.k_steps == 2) hipLaunchKernelGGL((gemm_small_kernel<T, 2>), grid, block, 0, stream, p);                    \
-    else if (p.k_steps <= 4) hipLaunchKernelGGL((gemm_small_kernel<T, 4>), grid, block, 0, stream, p);                    \
-    else hipLaunchKernelGGL((gemm_small_kernel<T, kSmallStages>), grid, block, 0, stream, p);                             \
+    if (p.k_steps == 1) hipLaunchKernelGGL((gemm_small_kernel<T, 1, false>), grid, block, 0, stream, p);                         \
+    else if (p.k_steps == 2) hipLaunchKernelGGL((gemm_small_kernel<T, 2, false>), grid, block, 0, stream, p);                    \
+    else if (p.k_steps <= 4) hipLaunchKernelGGL((gemm_small_kernel<T, 4, false>), grid, block, 0, stream, p);                    \
+    else hipLaunchKernelGGL((gemm_small_kernel<T, kSmallStages, false>), grid, block, 0, stream, p);                             \
   } while (0)
   if (dtype == ODIT_BF16) ODIT_SMALL(bf16_t);
   else ODIT_SMALL(f16_t);

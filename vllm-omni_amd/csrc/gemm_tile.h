@@ -47,6 +47,7 @@
 #include <type_traits>
 
 #include "gemm_epilogue.h"
+#include "gemm_heads.h"
 
 namespace odit {
 
@@ -168,9 +169,6 @@ __device__ __forceinline__ void finish_quadrant(int kind, const GemmEpilogue& e,
 }
 
 // ---- query, key and value heads (HeadsOut): the end of a quadrant in two passes with a barrier between them ----
-// s of this lane and of the one 16 (32) further or before: the swap of two copies of s leaves one's lanes in each half's pairs
-template <typename Pair> __device__ __forceinline__ float add_swapped(float, Pair p) { return __uint_as_float(p[0]) + __uint_as_float(p[1]); }
-
 // The projection's values as they would be stored, which take the registers of the sums, and what this wavefront's 32 features add to
 // the squares of their head's row: squares[row][wavefront along the features]. r: the lane's first row in the tile. (Row by row: what
 // the compiler would form of all rows at once does not fit beside the sums.)
@@ -192,28 +190,8 @@ __device__ __forceinline__ void square_heads(const f32x4_v (&v)[MH][2], u32x4 bi
   }
 }
 
-// Where this lane's rows r, r + 16, ... of a tile go, and their rotary factors of in-head features d .. d + 7
-template <int MH>
-struct HeadRows {
-  int at[MH];  // row of the outputs, -1: none
-  f32x4_v cos[MH], sin[MH];
-  __device__ __forceinline__ void ask(const HeadsOut& h, int M, int m0, int r, int d) {
-#pragma unroll
-    for (int i = 0; i < MH; ++i) {
-      const int row = m0 + r + i * 16, m = row < M ? row : M - 1;
-      const int b = h.div_mul == 0 ? m : static_cast<int>(__umulhi(m, h.div_mul) >> h.div_shift), s = m - b * h.S;
-      at[i] = row < M ? b * h.S_total + h.offset + s : -1;
-      const int64_t t = static_cast<int64_t>(s) * (h.D / 2) + d / 2;
-      cos[i] = *reinterpret_cast<const f32x4_v*>(h.cos + t);
-      sin[i] = *reinterpret_cast<const f32x4_v*>(h.sin + t);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  }
-};
-
-// The second pass, features f .. f + 7: norm over the head, weight, rotation (queries and keys), and the store. The operations are
-// those of qknorm_flat_kernel and the sums of squares are added in its order: its bits, but for which of an odd feature's two products
-// the compiler rounds (f16: 6 elements in 100000 differ, by a step).
+// The second pass, features f .. f + 7: norm over the head, weight, rotation (queries and keys), and the store. The sums of squares are
+// added in the order of qknorm_flat_kernel.
 template <typename T, int MH>
 __device__ __forceinline__ void store_heads(const HeadsOut& h, const u32x4 (&v)[MH], const HeadRows<MH>& rows, const float* squares, int r, int wn, int third,
                                             int f, u32x4 weight) {
@@ -226,11 +204,7 @@ __device__ __forceinline__ void store_heads(const HeadsOut& h, const u32x4 (&v)[
       const float lo = s[0] + s[1], hi = s[2] + s[3];
       const float sum = h.D == 128 ? lo + hi : (wn & 2 ? hi : lo);
       const float rstd = rsqrtf(sum * (h.D == 128 ? 1.f / 128 : 1.f / 64) + h.eps);
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const float x0 = Raw<T>::get(v[i], 2 * u) * rstd * Raw<T>::get(weight, 2 * u), x1 = Raw<T>::get(v[i], 2 * u + 1) * rstd * Raw<T>::get(weight, 2 * u + 1);
-        Raw<T>::set2(o, u, x0 * rows.cos[i][u] - x1 * rows.sin[i][u], x1 * rows.cos[i][u] + x0 * rows.sin[i][u]);
-      }
+      o = turn_head<T>(v[i], rstd, weight, rows.cos[i], rows.sin[i]);
     }
     if (rows.at[i] >= 0) store_raw(out + static_cast<int64_t>(rows.at[i]) * h.HD, o);
     __builtin_amdgcn_sched_barrier(0);

@@ -20,13 +20,7 @@ int launch_gemm_tile_heads(const GemmCall* c, int count, const HeadsOut* heads, 
   for (int i = 0; i < 2; ++i) {
     HeadsOut& h = p.heads[i];
     h = heads[i < count ? i : 0];
-    h.div_mul = h.div_shift = 0;
-    if (h.q == nullptr || h.S <= 1) continue;  // (one row per batch entry: the row number is the entry's)
-    // m / S as a multiply-high and a shift, exact for m < 2^31: l = ceil(log2 S), mul = ceil(2^(31 + l) / S)
-    uint32_t l = 1;
-    while ((1ull << l) < static_cast<uint64_t>(h.S)) ++l;
-    h.div_mul = static_cast<uint32_t>(((1ull << (31 + l)) + h.S - 1) / h.S);
-    h.div_shift = l - 1;
+    fill_heads_division(h);
   }
   const dim3 grid(plan.grid), block(512);
 #define ODIT_TILE(T)                                                                                \

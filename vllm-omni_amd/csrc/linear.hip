@@ -794,7 +794,10 @@ extern "C" int odit_linear_heads(const odit_linear_problem* q, const int* N, int
   if (engine == 2) return launch == 0 ? ODIT_OK : launch_gemm_tile_heads(g, 2, h, dtype, sk, static_cast<hipStream_t>(stream));
   const int cus = device_cus();
   const bool pair = both && N[0] == N[1], streamk_takes = pair && gemm_streamk_takes(g[0], dtype) && gemm_streamk_takes(g[1], dtype);
-  if (streamk_takes && gemm_small_rule(g, 2, cus, kSmallPairK)) return ODIT_ENOTSUP;
+  if (streamk_takes && gemm_small_rule(g, 2, cus, kSmallPairK)) {
+    if (h[0].D != 64 || h[1].D != 64) return ODIT_ENOTSUP;  // (a tile of the small kernel is a head of 64 features)
+    return launch == 0 ? ODIT_OK : launch_gemm_small_heads(g, 2, h, dtype, static_cast<hipStream_t>(stream));
+  }
   for (int i = 0; i < 2; ++i) apart += lin_call_us(dev, calls[i], g[i], sk);
   const TilePlan plan = plan_gemm_tile(g, 2, cus, sk != nullptr);
   if (plan.bm == 0) return ODIT_ENOTSUP;
