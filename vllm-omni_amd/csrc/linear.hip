@@ -750,7 +750,8 @@ extern "C" int odit_linear_fork(const odit_linear_problem* q, const int* N, int 
 // model, us, projections + pass / one launch: 2048 + 342 rows, N=9216, K=3072 119 + 17 / 130; 1024 + 512 rows 73 + 11 / 79; 8192 + 512
 // rows 340 + 45 / 365; 1536 rows, N=12288 with GELU beside N=9216 153 + 10 / 157; 4608 rows 435 + 25 / 438. Few rows, where the
 // stream-K kernel takes the pair, stay there unless the tile kernel wins with its time of cold weights (kColdTile times the
-// expected one, which is of a round in which others fetch the same): 512 + 80 rows 48 + 6 / 56, in the model 0.5 % slower.
+// expected one, which is of a round in which others fetch the same): 512 + 80 rows 48 + 6 / 56, in the model 0.5 % slower. The same
+// holds for rows that would take two calls otherwise: 772 rows, N=9216 beside N=12288 with GELU 52 + 64 + 7 / 129.
 constexpr float kColdTile = 1.18f;
 
 extern "C" int odit_linear_heads(const odit_linear_problem* q, const int* N, int K, const int* epilogue, const odit_head_output* const* heads, int dtype,
@@ -810,6 +811,7 @@ extern "C" int odit_linear_heads(const odit_linear_problem* q, const int* N, int
     if (streamk > 0.f && !(plan.us < apart && plan.us < streamk)) apart = streamk - (kColdTile - 1.f) * plan.us;
   } else {
     apart *= kOneLaunchGain;
+    if (plan.us >= apart) apart -= (kColdTile - 1.f) * plan.us;
   }
   if (plan.us + end >= (plan.us < apart ? plan.us : apart) + pass) return ODIT_ENOTSUP;
   if (launch == 0) return ODIT_OK;
