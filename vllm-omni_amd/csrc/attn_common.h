@@ -39,7 +39,6 @@ typedef __attribute__((__vector_size__(2 * sizeof(_Float16)))) _Float16 f16x2_v;
 template <typename T> struct Mma;
 template <> struct Mma<bf16_t> {
   using frag = bf16x8_v;
-  using acc = f32x16_v;
   static __device__ __forceinline__ f32x16_v run(frag a, frag b, f32x16_v c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
   }
@@ -50,7 +49,6 @@ template <> struct Mma<bf16_t> {
 };
 template <> struct Mma<f16_t> {
   using frag = f16x8_v;
-  using acc = f32x16_v;
   static __device__ __forceinline__ f32x16_v run(frag a, frag b, f32x16_v c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
   }
@@ -58,24 +56,6 @@ template <> struct Mma<f16_t> {
     const f32x2_v f = {lo, hi};
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, f16x2_v));
   }
-};
-// the same with 16 x 16 results of 32 products each
-template <typename T> struct Mma16;
-template <> struct Mma16<bf16_t> {
-  using frag = bf16x8_v;
-  using acc = f32x4_v;
-  static __device__ __forceinline__ f32x4_v run(frag a, frag b, f32x4_v c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ uint32_t pack2(float lo, float hi) { return Mma<bf16_t>::pack2(lo, hi); }
-};
-template <> struct Mma16<f16_t> {
-  using frag = f16x8_v;
-  using acc = f32x4_v;
-  static __device__ __forceinline__ f32x4_v run(frag a, frag b, f32x4_v c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ uint32_t pack2(float lo, float hi) { return Mma<f16_t>::pack2(lo, hi); }
 };
 
 struct AttnParams {

@@ -11,28 +11,27 @@
 // key row, so rows past Sk read as zeros without any clamping.
 //   K:  f(r) = r % 16       a quarter-wave (16 key rows, one chunk column) of a ds_read_b128 covers
 //                           all 64 banks
-//   V:  f(r) = 4 * (r % 4)  (D = 64: 2 * (r / 2 % 4)) the 4 (8) keys x 4 eight-byte words of two
-//                           ds_read_b64_tr_b16 groups cover all 64 banks
+//   V:  f(r) = 4 * (r % 4)  the 4 keys x 4 eight-byte words of two ds_read_b64_tr_b16 groups cover
+//                           all 64 banks
 // Fragment addresses then are (per-lane base) XOR (a compile-time constant) plus an immediate.
 //
-// Matrix instructions and vector work. A wavefront's 32 queries are one group for v_mfma_f32_32x32x16 or two for 16x16x32;
-// a lane holds 4 keys of every 8 (of every 16) for one query of each group, and those of two runs of 4, which it packs itself, are its
-// operand of O^T = V^T P^T (V's transpose reads fetch the same keys). Launches are bound by the vector work of the softmax,
-// which shares its issue with the MFMAs, and by the part's power, of which 32x32x16 takes more for the same products (a loop of
-// nothing else: 1784 TFLOP/s on random operands against 2054, 2440 and 2415 on zeros), while 16x16x32 is twice as many
-// instructions. So the vector work is kept to what a tile cannot do without: the maximum over the lanes of a query is formed only where
-// a lane sees the running one left behind (settle_max), its exponent is kept, and the next scores' maxima are formed an
-// instruction or two behind each MFMA of stage B. us, before all this / 32x32x16 / 16x16x32, bf16:
-//   D=128  B=1 S=16384 H=40  4645 / 4572 / 4424 (on zeros 3548 / 3436 / 3869)   B=2 S=4352 H=24  439 / 432 / 421
-//          B=1 S=4608 H=24  248 / 244 / 245    B=1 S=1536 H=24  42.7 / 41.2 / 42.8
-//   D=64   B=2 S=4352 H=24  278 / - / 267      B=1 S=9000 H=8  203 / - / 195      B=2 S=1357 H=32  48.6 / - / 47.3, padded row 42.1 / - / 39.7
-// At head size 64 16x16x32 wins everywhere. At 128 it wins by the operands' power alone, where they are standard normal: in the models,
-// whose probabilities are nearly even, it gives less (a video step of 32760 keys: 1.003 times as fast as before, 1.008 with
-// 32x32x16), so it stays with the form that needs fewer instructions. With 16x16x32 and the maxima of every tile reduced over the lanes the first launch took 4665, an
-// exp2 pair behind every second MFMA 4804; sums of the probabilities in stage B, more fragments ahead, the first V fragments ahead of the
-// stages' barrier and other priorities were all slower.
+// Vector work. The softmax's vector instructions bound the launches beside the part's power, so a tile has only those that it cannot do
+// without (32 exp2, 32 multiply-adds, 32 adds, 16 packs, 16 maxima): the row maximum is formed over the lane halves only where a lane
+// sees the running one left behind, its exponent is kept from there (settle_max), the next scores' maximum is formed an
+// instruction or two behind each MFMA of stage B instead of in one piece behind the second, and there is one path of selects for
+// excluded keys (mask_and_max). us, before / now, the same bits:
+//   D=128  B=1 S=16384 H=40  4645 / 4572 (on zeros, without the power limit, 3548 / 3430)    B=2 S=4352 H=24  439 / 432
+//          B=1 S=4608 H=24  248 / 243      B=1 S=1536 H=24  42.7 / 41.2
+//   D=64   B=2 S=4178 H=4  67.6 / 65.1     B=1 S=4096 H=8  55.5 / 52.1     B=1 S=8192 H=8  155 / 152     B=2 S=4352 H=24  278 / 268
+//          B=2 S=1357 H=32  48.6 / 46.6, padded row 42.1 / 39.0
+// v_mfma_f32_16x16x32 (two groups of 16 queries a wavefront) draws less power for the same products (a loop of nothing else: 2054
+// TFLOP/s on random operands, 32x32x16 1784; on zeros 2415 and 2440) and is twice as many instructions to issue. It took the first
+// launch to 4424 and zeros to 3869, but a video step of 32760 keys, whose probabilities are nearly even, to 0.997 of the time before
+// where this form takes it to 0.99, and wavefronts alone on their SIMD 8 % longer (B=2 S=4178 H=4 73.0): not kept. Sums of the
+// probabilities in stage B, packing pinned in stage A, the first V fragments ahead of the stages' barrier, other priorities and
+// more fragments ahead: all slower.
 //
-// Everything else (transposed S^T = K Q^T / O^T = V^T P^T formulation, lazy
+// Everything else (transposed S^T = K Q^T / O^T = V^T P^T formulation, one query per lane, lazy
 // rescale, stage A = next-tile QK^T MFMAs interleaved with this tile's exp2 work, stage B = PV, one
 // barrier per tile - two in the anti-phase form of 8 wavefronts, see NW below -, XCD-aware workgroup order)
 // is as in attn_fwd_pipe_kernel.
@@ -84,7 +83,6 @@
 #include <stddef.h>
 
 #include <cstdlib>
-#include <type_traits>
 
 #include "attn_common.h"
 #include "attn_tail.h"
@@ -127,24 +125,17 @@ typedef __attribute__((address_space(3))) void* lds_void_p;
 // words in the launches without a mask: 452 -> 460 us at B=2 S=4352 H=24 D=128, 252 -> 262 at B=1 S=4608).
 constexpr int kMaskWords = 1024;  // 8 KB of LDS: two workgroups of D = 128 still fit a compute unit (144 of 160 KB)
 
-// results of a matrix instruction are this many keys by as many queries (see the head of the file)
-constexpr int mma_edge(int D) { return D == 64 ? 16 : 32; }
-
 template <typename T, int D, int NW, int MODE>
 __global__ __launch_bounds__(NW * 64, MODE >= 6 ? 3 : 8 / NW) void attn_fwd_dma_kernel(const AttnParams p) {
   constexpr bool TAIL = MODE == 1 || MODE == 4;
   constexpr bool PERSIST = MODE == 2;
   constexpr bool WORDS = MODE >= 3 && MODE != 6;
   constexpr bool THREE = MODE >= 6, SPREAD = MODE == 5 || MODE == 8;
-  // matrix instructions with N x N results: U groups of N queries, a lane's element e of a tile of N keys is key e / 4 * 8 + e % 4 + 4 lg
-  constexpr int N = mma_edge(D), U = 32 / N, NK = 64 / N, E = N * N / 64, KD = 512 / N;
-  static_assert(N == 32 ? D == 128 : D == 64, "the V tile's swizzle");
-  using M = std::conditional_t<N == 16, Mma16<T>, Mma<T>>;
+  using M = Mma<T>;
   using frag = typename M::frag;
-  using acc = typename M::acc;
   constexpr int BN = 64;
-  constexpr int KS = D / KD;  // reduction steps of the scores
-  constexpr int DT = D / N;   // tiles of output features
+  constexpr int KS = D / 16;
+  constexpr int DT = D / 32;
   constexpr int ROWB = D * 2;                 // bytes per tile row
   constexpr int CPR = ROWB / 16;              // 16-byte chunks per row (16 for D=128, 8 for D=64)
   constexpr int RPI = 64 / CPR;               // tile rows filled by one wave instruction (4 or 8)
@@ -193,7 +184,7 @@ __global__ __launch_bounds__(NW * 64, MODE >= 6 ? 3 : 8 / NW) void attn_fwd_dma_
     if (pid >= x_hi) return;  // fewer units than workgroups on this XCD (before any barrier: the whole workgroup leaves)
   }
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int lq = lane % N, lg = lane / N;
+  const int l32 = lane & 31, hh = lane >> 5;
   const int wl = PP ? (wave & 3) : wave;     // this wavefront's share of a tile load
   const bool grp1 = PP && wave >= 4;          // second group of the anti-phase form (wave-uniform)
 
@@ -275,12 +266,11 @@ __global__ __launch_bounds__(NW * 64, MODE >= 6 ? 3 : 8 / NW) void attn_fwd_dma_
   // relative to the tile's first row; instruction i moves the rows RPI * i further down, which is a scalar
   // term (it goes into the load's scalar offset), and its swizzle differs from the first one's by a constant:
   // for K, row % 16 = (row0 % 16) + (RPI * i) % 16 without a carry (row0 % 16 < RPI), so the chunk index is that
-  // of instruction 0 XOR ((RPI * i) % 16 % CPR), and likewise for V. The
+  // of instruction 0 XOR ((RPI * i) % 16 % CPR) - for V (4 * (row % 4), RPI a multiple of 4) it is the same. The
   // XOR is done on the byte offset, which needs row strides that are multiples of the row's own 2 D bytes.
-  auto v_swizzle = [](int r) { return N == 32 ? 4 * (r % 4) : 2 * (r / 2 % 4); };
   const int r0 = wl * IPW * RPI + lane / CPR, pc0 = lane % CPR;
   const uint32_t kvoff0 = static_cast<uint32_t>(r0 * p.ks_s * 2) + static_cast<uint32_t>(((pc0 ^ (r0 % 16)) % CPR) * 16);
-  const uint32_t vvoff0 = static_cast<uint32_t>(r0 * p.vs_s * 2) + static_cast<uint32_t>(((pc0 ^ v_swizzle(r0)) % CPR) * 16);
+  const uint32_t vvoff0 = static_cast<uint32_t>(r0 * p.vs_s * 2) + static_cast<uint32_t>(((pc0 ^ (4 * (r0 % 4))) % CPR) * 16);
   const uint32_t k_inst_step = static_cast<uint32_t>(RPI * p.ks_s * 2);
   const uint32_t v_inst_step = static_cast<uint32_t>(RPI * p.vs_s * 2);
   const uint32_t k_tile_step = static_cast<uint32_t>(BN * p.ks_s * 2);
@@ -304,7 +294,7 @@ __global__ __launch_bounds__(NW * 64, MODE >= 6 ? 3 : 8 / NW) void attn_fwd_dma_
 #pragma unroll
     for (int i = 0; i < IPW; ++i) {
       const uint32_t m0v = __builtin_amdgcn_readfirstlane(lds0 + i * 1024);
-      const uint32_t voff_i = voff0 ^ static_cast<uint32_t>(is_k ? ((RPI * i) % 16) % CPR * 16 : 0);
+      const uint32_t voff_i = is_k ? (voff0 ^ static_cast<uint32_t>((((RPI * i) % 16) % CPR) * 16)) : voff0;
       const uint32_t soff_i = soff + static_cast<uint32_t>(i) * (is_k ? k_inst_step : v_inst_step);
       load_lds16<true>(m0v, voff_i, rsrc, soff_i);
     }
@@ -327,196 +317,155 @@ __global__ __launch_bounds__(NW * 64, MODE >= 6 ? 3 : 8 / NW) void attn_fwd_dma_
   };
 
   // ---- Q fragments stay in registers ----
-  frag qf[KS * U];  // (step, group of queries)
+  frag qf[KS];
   // (the persistent form calls these two inside the tile loop: they take the lane's position from the thread
   // index again, so that nothing of theirs is carried through the loop)
-  auto lane_again = [&](int& lq_, int& lg_) {
+  auto lane_again = [&](int& l32_, int& hh_) {
     int t = tid;
     if constexpr (PERSIST) asm volatile("" : "+v"(t));
-    lq_ = t % N;
-    lg_ = (t & 63) / N;
+    l32_ = t & 31;
+    hh_ = (t >> 5) & 1;
   };
   auto load_q = [&](int b_, int h_, int q0_) {
-    int lq, lg;
-    lane_again(lq, lg);
+    int l32, hh;
+    lane_again(l32, hh);
+    int row = q0_ + l32;
+    const int rows = ODIT_ARG(Sq);
+    row = row < rows ? row : rows - 1;
+    const T* qp = static_cast<const T*>(ODIT_ARG(q)) + b_ * ODIT_ARG(qs_b) + h_ * ODIT_ARG(qs_h) + row * ODIT_ARG(qs_s) + hh * 8;
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      int row = q0_ + u * N + lq;
-      const int rows = ODIT_ARG(Sq);
-      row = row < rows ? row : rows - 1;
-      const T* qp = static_cast<const T*>(ODIT_ARG(q)) + b_ * ODIT_ARG(qs_b) + h_ * ODIT_ARG(qs_h) + row * ODIT_ARG(qs_s) + lg * 8;
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) qf[ks * U + u] = __builtin_bit_cast(frag, *reinterpret_cast<const u32x4_v*>(qp + ks * KD));
-    }
+    for (int ks = 0; ks < KS; ++ks)
+      qf[ks] = __builtin_bit_cast(frag, *reinterpret_cast<const u32x4_v*>(qp + ks * 16));
   };
   load_q(b, h, q0);
-  auto q_kept = [&](int f) { return __builtin_bit_cast(frag, q_lds[(wave * QL + f - (KS * U - QL)) * 64 + lane]); };  // (each lane its own)
+  auto q_kept = [&](int ks) { return __builtin_bit_cast(frag, q_lds[(wave * QL + ks - (KS - QL)) * 64 + lane]); };  // (each lane its own)
 #pragma unroll
-  for (int i = 0; i < QL; ++i) q_lds[(wave * QL + i) * 64 + lane] = __builtin_bit_cast(u32x4_v, qf[KS * U - QL + i]);
+  for (int i = 0; i < QL; ++i) q_lds[(wave * QL + i) * 64 + lane] = __builtin_bit_cast(u32x4_v, qf[KS - QL + i]);
 
-  acc o[DT][U];
+  f32x16_v o[DT];
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-    for (int u = 0; u < U; ++u)
-#pragma unroll
-      for (int e = 0; e < E; ++e) o[dt][u][e] = 0.f;
-  float m_run[U], l_run[U], mc[U];  // mc: m_run as an exponent, 0 before the first score
-#pragma unroll
-  for (int u = 0; u < U; ++u) {
-    m_run[u] = -INFINITY;
-    l_run[u] = mc[u] = 0.f;
-  }
+    for (int e = 0; e < 16; ++e) o[dt][e] = 0.f;
+  float m_run = -INFINITY, l_run = 0.f, mc = 0.f;  // mc: m_run as an exponent, 0 before the first score
 
   const float c = p.scale_log2, c_rescale = fmaxf(c, 0.f);
 
-  // K fragment (kt, ks): row kt*N + lq, logical chunk (64/N)*ks + lg  ->  chunk ((64/N)*ks) ^ (lg ^ lq % 16)
-  const int k_lane = lq * ROWB + (((lg ^ (lq % 16)) % CPR) << 4);
-  // V transpose read, 16-lane group lane/16, lane s = lane%16: key 4*lg + s/4 (+ tile offsets), features of half dh of the tile
-  // (N = 32: lane/16 % 2), logical chunk (N/8)*dt + 2*dh + (s%4)/2, 8-byte half (s%4)%2, physical chunk = logical ^ f(key)
-  // ->  XOR of the dt field only
-  const int sq = (lane & 15) >> 2, dh = N == 32 ? (lane >> 4) & 1 : 0;
-  const int v_lane = (4 * lg + sq) * ROWB + (((v_swizzle(4 * lg + sq) % CPR) ^ (2 * dh + ((lane & 3) >> 1))) << 4) + ((lane & 1) << 3);
+  // K fragment (kt, ks): row kt*32 + l32, logical chunk 2*ks + hh  ->  chunk (2*ks) ^ (hh ^ l32 % 16)
+  const int k_lane = l32 * ROWB + ((((hh ^ (l32 % 16)) % CPR)) << 4);
+  // V transpose read, 16-lane group g = lane/16 (d half dh = g&1, key half = hh), lane s = lane%16:
+  // key 4*hh + s/4 (+ tile offsets), logical chunk 4*dt + 2*dh + (s%4)/2, 8-byte half (s%4)%2,
+  // physical chunk = logical ^ 4*(s/4)  ->  XOR of the dt field only
+  const int sq = (lane & 15) >> 2;
+  const int dh = (lane >> 4) & 1;
+  const int v_lane = (4 * hh + sq) * ROWB + ((((4 * sq) % CPR) ^ (2 * dh + ((lane & 3) >> 1))) << 4) + ((lane & 1) << 3);
 
-  auto qk_plain = [&](const char* kt_base, acc(&s)[NK][U]) {
+  auto qk_plain = [&](const char* kt_base, f32x16_v(&s)[2]) {
 #pragma unroll
-    for (int kt = 0; kt < NK; ++kt)
+    for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-      for (int u = 0; u < U; ++u)
-#pragma unroll
-        for (int e = 0; e < E; ++e) s[kt][u][e] = 0.f;
+      for (int e = 0; e < 16; ++e) s[kt][e] = 0.f;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-      for (int kt = 0; kt < NK; ++kt) {
-        const frag a = __builtin_bit_cast(frag, *reinterpret_cast<const u32x4_v*>(kt_base + kt * N * ROWB + (k_lane ^ (ks * KD * 2))));
-#pragma unroll
-        for (int u = 0; u < U; ++u) s[kt][u] = M::run(a, ks * U + u < KS * U - QL ? qf[ks * U + u] : q_kept(ks * U + u), s[kt][u]);
+      for (int kt = 0; kt < 2; ++kt) {
+        const frag a = __builtin_bit_cast(
+            frag, *reinterpret_cast<const u32x4_v*>(kt_base + kt * 32 * ROWB + (k_lane ^ (ks * 32))));
+        s[kt] = M::run(a, ks < KS - QL ? qf[ks] : q_kept(ks), s[kt]);
       }
   };
 
-  // (inline assembly: the compiler puts a quieting maximum with itself in front of values that it has not computed)
-  auto max2 = [&](float a, float b) __attribute__((always_inline)) {
+  // The lane's maximum of its 32 scores, in 16 instructions. (Inline assembly: the compiler puts a maximum with itself, which quiets a
+  // NaN, in front of values that it has not computed.)
+  constexpr int NMAX = 16;
+  auto max_step = [&](const f32x16_v(&s)[2], float mx, int n) __attribute__((always_inline)) -> float {
     float r;
-    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    if (n == 0) asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(s[0][0]), "v"(s[0][1]), "v"(s[0][2]));
+    else if (n == NMAX - 1) asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(mx), "v"(s[1][15]));
+    else asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(mx), "v"(s[(2 * n + 1) >> 4][(2 * n + 1) & 15]), "v"(s[(2 * n + 2) >> 4][(2 * n + 2) & 15]));
     return r;
   };
-  auto max3 = [&](float a, float b, float c) __attribute__((always_inline)) {
-    float r;
-    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-    return r;
-  };
-  // the n-th of the 16 / U instructions that form the maximum of the lane's scores of a query
-  constexpr int NMAX = 16 / U;
-  auto max_step = [&](const acc(&s)[NK][U], float(&mx)[U], int n) __attribute__((always_inline)) {
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      auto at = [&](int e) __attribute__((always_inline)) { return s[e / E][u][e % E]; };
-      mx[u] = n == 0 ? max3(at(0), at(1), at(2)) : n == NMAX - 1 ? max2(mx[u], at(2 * NMAX - 1)) : max3(mx[u], at(2 * n + 1), at(2 * n + 2));
-    }
-  };
-  auto lane_max = [&](const acc(&s)[NK][U], float(&mx)[U]) __attribute__((always_inline)) {
-#pragma unroll
-    for (int n = 0; n < NMAX; ++n) max_step(s, mx, n);
-  };
-  // over the lanes that share a query
-  auto over_query = [&](float x, auto op) __attribute__((always_inline)) {
-    if constexpr (N == 16) {
-      auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-      x = op(__uint_as_float(a[0]), __uint_as_float(a[1]));
-    }
-    auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    return op(__uint_as_float(b[0]), __uint_as_float(b[1]));
-  };
-  auto query_sum = [&](float x) __attribute__((always_inline)) { return over_query(x, [](float a, float b) { return a + b; }); };
 
-  // excluded scores of tile j become -inf (branch-free selects: every lane rewrites all its scores).
-  // w: the tile's mask word (WORDS)
-  auto mask_scores = [&](int j, const uint8_t* mrow, uint64_t w, acc(&s)[NK][U]) {
-    auto keep = [&](auto live) __attribute__((always_inline)) {  // live(position in the tile, but for 4 lg)
+  // excluded scores of tile j become -inf (branch-free selects: every lane rewrites all its scores); returns the lane's maximum.
+  // w: the tile's mask word (WORDS; formed here otherwise: one path of selects for what is excluded by a mask and by the sequence's
+  // end, as with two of them the tiles without either paid 16 to 32 register copies each, 4 % of a launch)
+  auto mask_and_max = [&](int j, const uint8_t* mrow, uint64_t w, f32x16_v(&s)[2]) -> float {
+    if constexpr (!WORDS) {
+      const int keys = p.Sk - j * BN;  // from here to the end (one at least)
+      w = keys < BN ? (1ull << keys) - 1 : ~0ull;
+      if (mrow != nullptr) w &= __ballot(mrow[lane < keys ? j * BN + lane : p.Sk - 1] != 0);
+    }
+    // (this lane's keys are 8 g + 4 hh + t of each half of the tile)
+    const uint32_t half[2] = {static_cast<uint32_t>(w) >> (4 * hh), static_cast<uint32_t>(w >> 32) >> (4 * hh)};
 #pragma unroll
-      for (int kt = 0; kt < NK; ++kt)
+    for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-        for (int e = 0; e < E; ++e) {
-          const bool on = live(kt * N + e / 4 * 8 + e % 4);
+      for (int g = 0; g < 4; ++g)
 #pragma unroll
-          for (int u = 0; u < U; ++u) {
-            const float x = s[kt][u][e];
-            s[kt][u][e] = on ? x : -INFINITY;
-          }
+        for (int t = 0; t < 4; ++t) {
+          const float x = s[kt][g * 4 + t];
+          s[kt][g * 4 + t] = (half[kt] & (1u << (g * 8 + t))) ? x : -INFINITY;
         }
-    };
-    if constexpr (WORDS) {
-      const uint32_t half[2] = {static_cast<uint32_t>(w) >> (4 * lg), static_cast<uint32_t>(w >> 32) >> (4 * lg)};
-      keep([&](int at) __attribute__((always_inline)) { return (half[at / 32] & (1u << (at % 32))) != 0; });
-    } else if (mrow != nullptr) {
-      keep([&](int at) __attribute__((always_inline)) {
-        const int key = j * BN + at + lg * 4, kc = key < p.Sk ? key : p.Sk - 1;
-        return (key < p.Sk) & (mrow[kc] != 0);
-      });
-    } else if ((j + 1) * BN > p.Sk) {
-      keep([&](int at) __attribute__((always_inline)) { return j * BN + at + lg * 4 < p.Sk; });
-    }
+    float mx = 0.f;
+#pragma unroll
+    for (int n = 0; n < NMAX; ++n) mx = max_step(s, mx, n);
+    return mx;
   };
 
-  // mx: the lane's maxima of its queries. The maximum over the lanes that share a query is formed only where the running one is left
-  // behind by a factor of 2^8 in any lane.
-  auto settle_max = [&](const float(&mx)[U]) __attribute__((always_inline)) {
-    float ahead = mx[0] - m_run[0];
-    if constexpr (U == 2) ahead = fmaxf(ahead, mx[1] - m_run[1]);
-    if (__any(ahead * c_rescale > 8.f)) {
+  // x of the lane 32 further or before
+  auto swapped = [&](float x) __attribute__((always_inline)) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return __uint_as_float(hh ? r[0] : r[1]);
+  };
+  // mx: the lane's maximum. The row's, over both lane halves, is formed only where the running one is left behind by a factor of 2^8.
+  auto settle_max = [&](float mx) __attribute__((always_inline)) {
+    if (__any((mx - m_run) * c_rescale > 8.f)) {
+      const float m_new = fmaxf(m_run, fmaxf(mx, swapped(mx)));
+      const float m_safe = (m_new == -INFINITY) ? 0.f : m_new;
+      const float alpha = __builtin_amdgcn_exp2f((m_run - m_safe) * c);
+      l_run *= alpha;
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const float m_new = fmaxf(m_run[u], over_query(mx[u], [](float a, float b) { return fmaxf(a, b); }));
-        const float m_safe = m_new == -INFINITY ? 0.f : m_new;
-        const float alpha = __builtin_amdgcn_exp2f((m_run[u] - m_safe) * c);
-        l_run[u] *= alpha;
+      for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-          for (int e = 0; e < E; ++e) o[dt][u][e] *= alpha;
-        m_run[u] = m_new;
-        mc[u] = m_safe * c;
-      }
+        for (int e = 0; e < 16; ++e) o[dt][e] *= alpha;
+      m_run = m_new;
+      mc = m_safe * c;
     }
   };
 
   // normalises and stores the finished unit (b, h, q0): the tail of MODE 0 and of every unit of the persistent form
   auto finish_unit = [&]() {
-    int lq, lg;
-    lane_again(lq, lg);
+    int l32, hh;
+    lane_again(l32, hh);
+    const float l_tot = l_run + swapped(l_run);
+    const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+    const int row = q0 + l32;
+    if (row < ODIT_ARG(Sq)) {
+      // head of the joint sequence in `o`, tail in `o_tail` (out_row_ptr, with the arguments fetched here)
+      T* op;
+      void* const o_tail = ODIT_ARG(o_tail);
+      const int q_split = ODIT_ARG(q_split);
+      if (o_tail != nullptr && row >= q_split) {
+        op = static_cast<T*>(o_tail) + b * ODIT_ARG(ts_b) + h * ODIT_ARG(ts_h) + static_cast<int64_t>(row - q_split) * ODIT_ARG(ts_s);
+      } else {
+        op = static_cast<T*>(ODIT_ARG(o)) + b * ODIT_ARG(os_b) + h * ODIT_ARG(os_h) + static_cast<int64_t>(row) * ODIT_ARG(os_s);
+      }
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const float l_tot = query_sum(l_run[u]);
-      const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-      const int row = q0 + u * N + lq;
-      if (row < ODIT_ARG(Sq)) {
-        // head of the joint sequence in `o`, tail in `o_tail` (out_row_ptr, with the arguments fetched here)
-        T* op;
-        void* const o_tail = ODIT_ARG(o_tail);
-        const int q_split = ODIT_ARG(q_split);
-        if (o_tail != nullptr && row >= q_split) {
-          op = static_cast<T*>(o_tail) + b * ODIT_ARG(ts_b) + h * ODIT_ARG(ts_h) + static_cast<int64_t>(row - q_split) * ODIT_ARG(ts_s);
-        } else {
-          op = static_cast<T*>(ODIT_ARG(o)) + b * ODIT_ARG(os_b) + h * ODIT_ARG(os_h) + static_cast<int64_t>(row) * ODIT_ARG(os_s);
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          u32x2_v w;
+          w.x = M::pack2(o[dt][g * 4 + 0] * inv, o[dt][g * 4 + 1] * inv);
+          w.y = M::pack2(o[dt][g * 4 + 2] * inv, o[dt][g * 4 + 3] * inv);
+          *reinterpret_cast<u32x2_v*>(op + dt * 32 + g * 8 + hh * 4) = w;
+          // (in the persistent form this runs inside the tile loop, with the next unit's queries and first scores
+          // live: the values go out one store at a time instead of being formed all at once)
+          if constexpr (PERSIST) __builtin_amdgcn_sched_barrier(0);
         }
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-          for (int g = 0; g < E / 4; ++g) {
-            u32x2_v w;
-            w.x = M::pack2(o[dt][u][g * 4 + 0] * inv, o[dt][u][g * 4 + 1] * inv);
-            w.y = M::pack2(o[dt][u][g * 4 + 2] * inv, o[dt][u][g * 4 + 3] * inv);
-            *reinterpret_cast<u32x2_v*>(op + dt * N + g * 8 + lg * 4) = w;
-            // (in the persistent form this runs inside the tile loop, with the next unit's queries and first scores
-            // live: the values go out one store at a time instead of being formed all at once)
-            if constexpr (PERSIST) __builtin_amdgcn_sched_barrier(0);
-          }
-        float* const lse_out = ODIT_ARG(lse);
-        if (lse_out != nullptr && lg == 0) {
-          const float lse = l_tot > 0.f ? m_run[u] * ODIT_ARG(scale) + __logf(l_tot) : -INFINITY;
-          lse_out[(static_cast<int64_t>(b) * ODIT_ARG(H) + h) * ODIT_ARG(Sq) + row] = lse;
-        }
+      float* const lse_out = ODIT_ARG(lse);
+      if (lse_out != nullptr && hh == 0) {
+        const float lse = l_tot > 0.f ? m_run * ODIT_ARG(scale) + __logf(l_tot) : -INFINITY;
+        lse_out[(static_cast<int64_t>(b) * ODIT_ARG(H) + h) * ODIT_ARG(Sq) + row] = lse;
       }
     }
   };
@@ -525,7 +474,7 @@ __global__ __launch_bounds__(NW * 64, MODE >= 6 ? 3 : 8 / NW) void attn_fwd_dma_
   // workgroup's next unit (`cross`), and the tile after that its tile 1.
   // `buf` (the LDS buffer pair of this tile: the parity of its running index) is a literal at every call, so the
   // LDS addresses below are compile-time offsets.
-  auto tile = [&](int j, const int buf, acc(&s_cur)[NK][U], acc(&s_next)[NK][U]) {
+  auto tile = [&](int j, const int buf, f32x16_v(&s_cur)[2], f32x16_v(&s_next)[2]) {
     const bool last = j + 1 == n_tiles;
     const bool cross = PERSIST && last && next_pid >= 0;
     const bool has_next = !last || cross;
@@ -555,21 +504,8 @@ __global__ __launch_bounds__(NW * 64, MODE >= 6 ? 3 : 8 / NW) void attn_fwd_dma_
 
     // (Row sums in fp32 from the unrounded probabilities. Summing the packed pairs with v_dot2c_f32_bf16, one
     // instruction per pair instead of two adds, measured 4 % slower at D = 128, with one chain or four.)
-    // fragments of probabilities, (KD keys, group of queries); their element i
-    uint32_t pf[4][4];
-    auto score = [&](int f, int i) __attribute__((always_inline)) -> float { return N == 32 ? s_cur[f >> 1][0][(f & 1) * 8 + i] : s_cur[2 * (f >> 1) + (i >> 2)][f % U][i % E]; };
-    float psum[U] = {};
-    float p0;
-    auto probability = [&](int e, const float(&mc)[U]) __attribute__((always_inline)) {
-      const int f = e >> 3, u = f % U;
-      const float p = __builtin_amdgcn_exp2f(fmaf(score(f, e & 7), c, -mc[u]));
-      if ((e & 1) == 0) {
-        p0 = p;
-      } else {
-        psum[u] += p0 + p;
-        pf[f][(e & 7) >> 1] = M::pack2(p0, p);
-      }
-    };
+    uint32_t pf[2][2][4];
+    float psum = 0.f;
     // Stage A mixes this wave's MFMAs with its exp2 work; giving it issue priority over the SIMD's other
     // wave (which is then mostly in its MFMA + LDS-read stage B) measured +5 % at 32760 keys, +9 % at
     // batch 1 / 4608 keys and nothing lost at the 4352-token, batch-2 shape.
@@ -582,54 +518,54 @@ __global__ __launch_bounds__(NW * 64, MODE >= 6 ? 3 : 8 / NW) void attn_fwd_dma_
       int k_lane_t = k_lane;
       if constexpr (PERSIST) asm volatile("" : "+v"(k_lane_t));
 #pragma unroll
-      for (int kt = 0; kt < NK; ++kt)
+      for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-        for (int u = 0; u < U; ++u)
-#pragma unroll
-          for (int e = 0; e < E; ++e) s_next[kt][u][e] = 0.f;
-      constexpr int KPF = THREE ? 1 : ODIT_ATTN_KPF;  // K fragments in flight ahead of the MFMAs that consume them
-      constexpr int NF = NK * KS;
+        for (int e = 0; e < 16; ++e) s_next[kt][e] = 0.f;
+      constexpr int KPF = THREE ? (WORDS ? 1 : 2) : ODIT_ATTN_KPF;  // K fragments in flight ahead of the MFMA that consumes them
       u32x4_v kfr[KPF + 1];
       auto k_fetch = [&](int i) {
-        const int ks = i / NK, kt = i % NK;
-        kfr[i % (KPF + 1)] = *reinterpret_cast<const u32x4_v*>(kt_base + kt * N * ROWB + (k_lane_t ^ (ks * KD * 2)));
+        const int ks = i >> 1, kt = i & 1;
+        kfr[i % (KPF + 1)] = *reinterpret_cast<const u32x4_v*>(kt_base + kt * 32 * ROWB + (k_lane_t ^ (ks * 32)));
       };
-      frag qt[U];
+      frag qt[2];
+      if constexpr (QL == KS) qt[0] = q_kept(0);
 #pragma unroll
       for (int i = 0; i < KPF; ++i) k_fetch(i);
 #pragma unroll
-      for (int i = 0; i < NF; ++i) {
-        if (i + KPF < NF) k_fetch(i + KPF);
-        const int ks = i / NK, kt = i % NK;
-        if constexpr (QL > 0) {
+      for (int i = 0; i < 2 * KS; ++i) {
+        if (i + KPF < 2 * KS) k_fetch(i + KPF);
+        const int ks = i >> 1, kt = i & 1;
+        if (kt == 0 && ks + 1 < KS && ks + 1 >= KS - QL) qt[(ks + 1) & 1] = q_kept(ks + 1);
+        s_next[kt] = M::run(__builtin_bit_cast(frag, kfr[i % (KPF + 1)]), ks < KS - QL ? qf[ks] : qt[ks & 1], s_next[kt]);
+        constexpr int PAIRS = 16 / (2 * KS) > 0 ? 16 / (2 * KS) : 1;
 #pragma unroll
-          for (int u = 0; u < U; ++u)
-            if (kt == 0 && ks * U + u >= KS * U - QL) qt[u] = q_kept(ks * U + u);
+        for (int q = 0; q < PAIRS; ++q) {
+          const int pi = i * PAIRS + q;
+          if (pi < 16) {
+            const int pkt = pi >> 3, e0 = (pi & 7) * 2;
+            const float p0 = __builtin_amdgcn_exp2f(fmaf(s_cur[pkt][e0], c, -mc));
+            const float p1 = __builtin_amdgcn_exp2f(fmaf(s_cur[pkt][e0 + 1], c, -mc));
+            psum += p0 + p1;
+            pf[pkt][(pi & 7) >> 2][pi & 3] = M::pack2(p0, p1);
+          }
         }
-#pragma unroll
-        for (int n = 0; n < U; ++n) {
-          const int u = i & 1 ? U - 1 - n : n;  // (one operand stays from each MFMA to the next)
-          s_next[kt][u] = M::run(__builtin_bit_cast(frag, kfr[i % (KPF + 1)]), ks * U + u < KS * U - QL ? qf[ks * U + u] : qt[u], s_next[kt][u]);
-          constexpr int EACH = 32 / (NF * U);
-#pragma unroll
-          for (int q = 0; q < EACH; ++q) probability((i * U + n) * EACH + q, mc);
-          __builtin_amdgcn_sched_barrier(0);  // pin: fetch(i+KPF), MFMA, its share of the exp2 work
-        }
+        __builtin_amdgcn_sched_barrier(0);  // pin: fetch(i+KPF), MFMA(i), this step's exp2 work
       }
     } else {
       // (an opaque copy of the offset: were the two branches' exponent arguments the same expressions, the
       // compiler would form all 32 ahead of the branch, out of the MFMAs' shadow and in 32 more registers)
-      float mc_t[U];
+      float mc_t = mc;
+      asm volatile("" : "+v"(mc_t));
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        mc_t[u] = mc[u];
-        asm volatile("" : "+v"(mc_t[u]));
+      for (int pi = 0; pi < 16; ++pi) {
+        const int pkt = pi >> 3, e0 = (pi & 7) * 2;
+        const float p0 = __builtin_amdgcn_exp2f(fmaf(s_cur[pkt][e0], c, -mc_t));
+        const float p1 = __builtin_amdgcn_exp2f(fmaf(s_cur[pkt][e0 + 1], c, -mc_t));
+        psum += p0 + p1;
+        pf[pkt][(pi & 7) >> 2][pi & 3] = M::pack2(p0, p1);
       }
-#pragma unroll
-      for (int e = 0; e < 32; ++e) probability(e, mc_t);
     }
-#pragma unroll
-    for (int u = 0; u < U; ++u) l_run[u] += psum[u];
+    l_run += psum;
     if constexpr (PERSIST) {
       // The next unit's queries replace this unit's once its last scores have been formed, a tile before they are
       // used: they land behind this tile's closing wait. (Loaded at the top of the tile that uses them, the
@@ -648,42 +584,38 @@ __global__ __launch_bounds__(NW * 64, MODE >= 6 ? 3 : 8 / NW) void attn_fwd_dma_
       __builtin_amdgcn_sched_barrier(0);
     }
     // ---- stage B: O^T += V(j)^T P(j)^T ----
-    // 2*DT steps of two MFMAs, head-dim tile innermost so that consecutive ones hit different accumulators and a
-    // pair of P fragments serves DT steps; the two transpose reads of step n + PF are issued before the MFMAs
-    // of step n, so LDS latency is covered by 2 PF matrix instructions. The lane's maxima of
-    // S(j+1) — vector work with nothing to wait for — are placed in the shadow of these MFMAs.
+    // 4*DT steps, head-dim tile innermost so that consecutive MFMAs hit different accumulators and one
+    // P fragment serves DT of them; the two transpose reads of step n + PF are issued before the MFMA
+    // of step n, so LDS latency is covered by PF matrix instructions. The in-lane row maximum of
+    // S(j+1) — vector work with nothing to wait for — is placed in the shadow of these MFMAs.
     const char* vt_base = Vb + buf * TILEB;
     int v_lane_t = v_lane;  // (opaque copy, as for the key fragments)
     if constexpr (PERSIST) asm volatile("" : "+v"(v_lane_t));
-    constexpr int NSTEP = 64 / KD * DT;
+    constexpr int NSTEP = 4 * DT;
     constexpr int PF = THREE ? 2 : ODIT_ATTN_VPF;
     s16x4_d vlo[PF + 1], vhi[PF + 1];
     auto v_fetch = [&](int step) {
-      const int dt = step % DT, part = step / DT;
-      const char* vp = vt_base + part * KD * ROWB + (v_lane_t ^ (dt * N * 2));
+      const int dt = step % DT, kt = (step / DT) >> 1, g2 = (step / DT) & 1;
+      const char* vp = vt_base + (kt * 32 + g2 * 16) * ROWB + (v_lane_t ^ ((dt * 64) % ROWB));
       vlo[step % (PF + 1)] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_p)(vp));
-      vhi[step % (PF + 1)] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_p)(vp + KD / 2 * ROWB));
+      vhi[step % (PF + 1)] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_p)(vp + 8 * ROWB));
     };
     bool plain_next = has_next && mrow_n == nullptr && (jn + 1) * BN <= p.Sk;  // no exclusions in the next scores
     uint64_t word = 0;  // (the same in every lane)
     if constexpr (WORDS) {
       if (has_next) word = mask_words[jn - jt0];
     }
-    float mx[U];
+    float mx = 0.f;
 #pragma unroll
     for (int st = 0; st < PF; ++st) v_fetch(st);
 #pragma unroll
     for (int st = 0; st < NSTEP; ++st) {
       if (st + PF < NSTEP) v_fetch(st + PF);
-      const int dt = st % DT, part = st / DT;
+      const int dt = st % DT, kt = (st / DT) >> 1, g2 = (st / DT) & 1;
       const s16x8_d av = __builtin_shufflevector(vlo[st % (PF + 1)], vhi[st % (PF + 1)], 0, 1, 2, 3, 4, 5, 6, 7);
-#pragma unroll
-      for (int n = 0; n < U; ++n) {
-        const int u = st & 1 ? U - 1 - n : n, f = part * U + u;
-        u32x4_v pb;
-        pb.x = pf[f][0]; pb.y = pf[f][1]; pb.z = pf[f][2]; pb.w = pf[f][3];
-        o[dt][u] = M::run(__builtin_bit_cast(frag, av), __builtin_bit_cast(frag, pb), o[dt][u]);
-      }
+      u32x4_v pb;
+      pb.x = pf[kt][g2][0]; pb.y = pf[kt][g2][1]; pb.z = pf[kt][g2][2]; pb.w = pf[kt][g2][3];
+      o[dt] = M::run(__builtin_bit_cast(frag, av), __builtin_bit_cast(frag, pb), o[dt]);
       if constexpr (WORDS) {
         if (st == 1) {
           const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(word));
@@ -691,18 +623,16 @@ __global__ __launch_bounds__(NW * 64, MODE >= 6 ? 3 : 8 / NW) void attn_fwd_dma_
           plain_next = has_next && (lo & hi) == ~0u;
         }
       }
-      // (the next scores' maxima in the shadow of the MFMAs, a pair of instructions at a time; formed again where keys are excluded)
+      // (the next scores' maximum, an instruction or two behind each MFMA; formed again where keys are excluded)
       constexpr int EACH = (NMAX + NSTEP - 2) / (NSTEP - 1);
       if (st > 0) {
 #pragma unroll
-        for (int q = 0; q < EACH; ++q)
-          if ((st - 1) * EACH + q < NMAX) max_step(s_next, mx, (st - 1) * EACH + q);
+        for (int n = (st - 1) * EACH; n < st * EACH && n < NMAX; ++n) mx = max_step(s_next, mx, n);
       }
-      __builtin_amdgcn_sched_barrier(0);  // keep the reads of step st+PF ahead of these MFMAs
+      __builtin_amdgcn_sched_barrier(0);  // keep the reads of step st+PF ahead of this MFMA
     }
     if (has_next && !plain_next) {
-      mask_scores(jn, mrow_n, word, s_next);
-      lane_max(s_next, mx);
+      mx = mask_and_max(jn, mrow_n, word, s_next);
     }
     __builtin_amdgcn_s_waitcnt(0);  // this wave's tile loads have landed in LDS
     __syncthreads();
@@ -722,14 +652,9 @@ __global__ __launch_bounds__(NW * 64, MODE >= 6 ? 3 : 8 / NW) void attn_fwd_dma_
 #pragma unroll
           for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-            for (int u = 0; u < U; ++u)
-#pragma unroll
-              for (int e = 0; e < E; ++e) o[dt][u][e] = 0.f;
-#pragma unroll
-          for (int u = 0; u < U; ++u) {
-            m_run[u] = -INFINITY;
-            l_run[u] = mc[u] = 0.f;
-          }
+            for (int e = 0; e < 16; ++e) o[dt][e] = 0.f;
+          m_run = -INFINITY;
+          l_run = mc = 0.f;
         }
       }
     }
@@ -761,17 +686,14 @@ __global__ __launch_bounds__(NW * 64, MODE >= 6 ? 3 : 8 / NW) void attn_fwd_dma_
   }
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
-  acc sa[NK][U], sb[NK][U];
+  f32x16_v sa[2], sb[2];
   uint64_t w = 0;
   if constexpr (WORDS) w = jt0 + lane < n_tiles ? mask_words[lane] : 0;
   qk_plain(Kb, sa);
   {
     uint64_t word = 0;
     if constexpr (WORDS) word = mask_words[0];
-    float mx[U];
-    mask_scores(jt0, mrow, word, sa);
-    lane_max(sa, mx);
-    settle_max(mx);
+    settle_max(mask_and_max(jt0, mrow, word, sa));
   }
   if (WORDS && n_tiles - jt0 > 1) {
     // the unit ends with its last tile that has a live key (the same in every wavefront); where none has, with the first
@@ -820,25 +742,22 @@ __global__ __launch_bounds__(NW * 64, MODE >= 6 ? 3 : 8 / NW) void attn_fwd_dma_
 
   // ---- epilogue ----
   if constexpr (TAIL) {
+    const float l_tot = l_run + swapped(l_run);
     // partial result of a key range: unnormalised O (fp32, [BM][D] per part) and the row's (m, l)
+    float* wo = p.ws + (static_cast<int64_t>(part) * BM + wave * 32 + l32) * D;
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const float l_tot = query_sum(l_run[u]);
-      const int64_t row = static_cast<int64_t>(part) * BM + wave * 32 + u * N + lq;
-      float* wo = p.ws + row * D;
+    for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-        for (int g = 0; g < E / 4; ++g) {
-          f32x4_v w4;
-          w4.x = o[dt][u][g * 4 + 0]; w4.y = o[dt][u][g * 4 + 1]; w4.z = o[dt][u][g * 4 + 2]; w4.w = o[dt][u][g * 4 + 3];
-          *reinterpret_cast<f32x4_v*>(wo + dt * N + g * 8 + lg * 4) = w4;
-        }
-      if (lg == 0) {
-        float* ml = p.ws + static_cast<int64_t>(gridDim.x) * BM * D + row * 2;
-        ml[0] = m_run[u];
-        ml[1] = l_tot;
+      for (int g = 0; g < 4; ++g) {
+        f32x4_v w4;
+        w4.x = o[dt][g * 4 + 0]; w4.y = o[dt][g * 4 + 1]; w4.z = o[dt][g * 4 + 2]; w4.w = o[dt][g * 4 + 3];
+        *reinterpret_cast<f32x4_v*>(wo + dt * 32 + g * 8 + hh * 4) = w4;
       }
+    if (hh == 0) {
+      float* ml = p.ws + static_cast<int64_t>(gridDim.x) * BM * D +
+                  (static_cast<int64_t>(part) * BM + wave * 32 + l32) * 2;
+      ml[0] = m_run;
+      ml[1] = l_tot;
     }
     return;
   }
@@ -881,7 +800,7 @@ static bool spread_batch(const AttnParams& p, int slots) {
 // second one that the key split does not take. Three wavefronts on a SIMD multiply no faster than two (the vector work of the
 // softmax fills either: B=2 S=4352 H=24 283 us, three everywhere 297; 1024 units of 128 key tiles 315 and 380), so it is a
 // matter of the rounds alone: up to 1.5 rounds of two are one round of three, in which a unit takes 1.5 times as long, and a second
-// round of two takes 0.6 of a first one, its workgroups having a compute unit each. us, two / three (both with 32x32x16), 688 to 752 units:
+// round of two takes 0.6 of a first one, its workgroups having a compute unit each. us, two / three, 688 to 752 units:
 //   B=2 S=1357 H=32 f16 54.8 / 48.6, with a padded row 44.5 / 40.7    B=1 S=5500 H=16 174.5 / 151.4, 500 keys 24.2 / 20.8,
 //   64 keys 11.2 / 10.3    B=1 S=12000 H=8 397 / 336    B=3 S=700 H=40 30.8 / 27.1
 // 544 units whose keys are too few to be split (B=1 S=2060, 300 keys, H=32): 18.4 / 14.8.

@@ -8,6 +8,20 @@
 
 namespace odit {
 
+template <typename T> struct Mma16;
+template <> struct Mma16<bf16_t> {
+  using frag = bf16x8_v;
+  static __device__ __forceinline__ f32x4_v run(frag a, frag b, f32x4_v c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+  }
+};
+template <> struct Mma16<f16_t> {
+  using frag = f16x8_v;
+  static __device__ __forceinline__ f32x4_v run(frag a, frag b, f32x4_v c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+  }
+};
+
 struct GemmEpilogue {
   const void *bias, *residual, *gate;
   void* out;
