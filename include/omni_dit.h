@@ -419,7 +419,7 @@ int odit_linear_pair(const odit_linear_problem problems[2], int N, int K, int ep
 int odit_linear_fork(const odit_linear_problem problems[2], const int N[2], int K, const int epilogue[2], int dtype, unsigned flags,
                      void* workspace, size_t workspace_bytes, void* stream);
 
-/* Two projections of the same K in one launch of the tile kernel, of which one or both are projections to query, key and value heads
+/* Two projections of the same K in one launch of the tile kernel (or, for two of heads of 64 features, the small one), of which one or both are projections to query, key and value heads
  * (heads[i] not NULL): N[i] = 3 H D features (bias or none), S rows of each batch entry (M = B S), whose queries and keys are normed
  * over each head (mean of squares + eps), weighted and rotated in pairs (2 i, 2 i + 1) at the tile's end and stored with the values in
  * rows offset .. offset + S - 1 of joint tensors [B, S_total, H D]: to_qkv and add_kv_proj with norm_q, norm_k, norm_added_q,

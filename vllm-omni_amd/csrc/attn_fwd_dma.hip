@@ -44,7 +44,7 @@
 //   B=2 S=4352 H=24 D=128  439 / 737 / 451      B=1 S=4608 H=24 D=128  249 / 469 / 258
 //   B=2 S=592 H=24 D=128   18.4 / 26.8 / 18.8   B=2 S=4352 H=24 D=64   279 / 505 / 289
 // (and 490 / 290 / 20.6 / 333 with a random mask, where every tile is mixed).
-// Past kMaskWords tiles, and in the persistent form, whose units change the batch row, the mask is read as bytes.
+// Past kMaskWords tiles, and in the persistent form, whose units change the batch row, the word is formed at each tile, from one byte a lane.
 // With the words a unit ends with the last tile that has a live key: the tiles behind it would add zero probabilities (and are not
 // read: a NaN among their values does not reach the rows). Together with spread_batch below, one batch row padded to 40 % of
 // the other's keys, us, f16, before / now, and the same with an all-true mask (what a launch gains depends on the padding: with

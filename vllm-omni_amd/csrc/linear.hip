@@ -5,7 +5,8 @@
 // Which kernel runs is decided here per call. Few rows: the hand-written stream-K kernel (gemm_bf16.hip) where the reduction is
 // long, and a kernel for products that are small altogether (gemm_small.hip). Many rows: the hand-written tile kernel
 // (gemm_bf16_tile.hip) or hipBLASLt's MFMA kernels, by expected time. The two streams of a dual-stream block: one launch of a
-// hand-written kernel, or two calls, by expected time (odit_linear_pair). For the library this file sets the problem up so that
+// hand-written kernel, or two calls, by expected time (odit_linear_pair), with what follows a projection to heads at its end where
+// that is expected to be faster (odit_linear_heads). For the library this file sets the problem up so that
 // its epilogue does the elementwise work (bias vector, activation, a per-output-feature alpha vector for the gate, beta = 1 on the
 // residual), keeps problem descriptors per thread, chooses among the library's candidates for long reductions by expected time, and
 // has an explicit tuning call that times the library's kernels and the hand-written ones for one problem and remembers the fastest.
