@@ -123,29 +123,54 @@ __device__ __forceinline__ void loads_arrived() { __builtin_amdgcn_s_waitcnt(0x0
 template <typename T, int MH, int K>
 __device__ __forceinline__ void finish_quadrant(const GemmEpilogue& e, int m0, int m, int n, const f32x4_v (&v)[MH][2]) {
   const bool in = n < e.N;
-  float gt[8], bs[8];
-  if constexpr (K != 3) gemm_epilogue_vectors8<T>(e, m0, in ? n : 0, gt, bs);
-  u32x4 res[MH];
-  if constexpr (K == 2) {
+  if constexpr (K == 3) {
+    // Two rows a round trip to memory, each with its gate vector. (Row by row a quadrant is four trips one after the other, and where a launch
+    // is one round its end waits for such a tile: 2048 + 342 rows, two gate vectors each, N=3072, K=3072 59.9 us, now 56.6. More rows at
+    // once do not fit beside the sums.)
+#pragma unroll
+    for (int i0 = 0; i0 < MH; i0 += 2) {
+      float gt[2][8], bs[2][8];
+      u32x4 res[2];
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int row = m + (i0 + j) * 16 < e.M ? m + (i0 + j) * 16 : e.M - 1;
+        gemm_epilogue_vectors8<T>(e, row, in ? n : 0, gt[j], bs[j]);
+        res[j] = load_raw(static_cast<const T*>(e.residual) + row * e.ldr + (in ? n : 0));
+      }
+      loads_arrived();
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        u32x4 o;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const f32x4_v a = v[i0 + j][u >> 1];
+          Raw<T>::set2(o, u, fmaf(gt[j][2 * u], a[2 * (u & 1)], bs[j][2 * u]) + Raw<T>::get(res[j], 2 * u),
+                       fmaf(gt[j][2 * u + 1], a[2 * (u & 1) + 1], bs[j][2 * u + 1]) + Raw<T>::get(res[j], 2 * u + 1));
+        }
+        if (in && m + (i0 + j) * 16 < e.M) store_raw(static_cast<T*>(e.out) + (m + (i0 + j) * 16) * e.ldo + n, o);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  } else {
+    float gt[8], bs[8];
+    gemm_epilogue_vectors8<T>(e, m0, in ? n : 0, gt, bs);
+    u32x4 res[MH];
+    if constexpr (K == 2) {
+#pragma unroll
+      for (int i = 0; i < MH; ++i) {
+        const int row = m + i * 16 < e.M ? m + i * 16 : e.M - 1;
+        res[i] = load_raw(static_cast<const T*>(e.residual) + row * e.ldr + (in ? n : 0));
+      }
+    }
+    loads_arrived();
 #pragma unroll
     for (int i = 0; i < MH; ++i) {
-      const int row = m + i * 16 < e.M ? m + i * 16 : e.M - 1;
-      res[i] = load_raw(static_cast<const T*>(e.residual) + row * e.ldr + (in ? n : 0));
-    }
-  }
-  loads_arrived();
+      float y[8];
 #pragma unroll
-  for (int i = 0; i < MH; ++i) {
-    float y[8];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      y[u] = v[i][0][u];
-      y[4 + u] = v[i][1][u];
-    }
-    const bool store = in && m + i * 16 < e.M;
-    if constexpr (K == 3) {
-      if (store) gemm_epilogue_store8<T>(e, m + i * 16, n, y);
-    } else {
+      for (int u = 0; u < 4; ++u) {
+        y[u] = v[i][0][u];
+        y[4 + u] = v[i][1][u];
+      }
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
         if constexpr (K == 2) y[u] = fmaf(gt[u], y[u], bs[u]) + Raw<T>::get(res[i], u);
@@ -155,10 +180,9 @@ __device__ __forceinline__ void finish_quadrant(const GemmEpilogue& e, int m0, i
       u32x4 o;
 #pragma unroll
       for (int u = 0; u < 4; ++u) Raw<T>::set2(o, u, y[2 * u], y[2 * u + 1]);
-      if (store) store_raw(static_cast<T*>(e.out) + (m + i * 16) * e.ldo + n, o);
+      if (in && m + i * 16 < e.M) store_raw(static_cast<T*>(e.out) + (m + i * 16) * e.ldo + n, o);
     }
   }
-  if constexpr (K == 3) loads_arrived();
 }
 template <typename T, int MH, bool UNGATED>
 __device__ __forceinline__ void finish_quadrant(int kind, const GemmEpilogue& e, int m0, int m, int n, const f32x4_v (&v)[MH][2]) {
