@@ -1,4 +1,4 @@
-"""Attention whose running maximum is left behind by one key at a time: a lane holds 4 keys of every 16 for a query, and the maximum over
+"""Attention whose running maximum is left behind by one key at a time: a lane holds 4 keys of every 8 for a query, and the maximum over
 the lanes of a query is formed only when one of them sees its keys exceed the running one by 2^8. Against a float64 product."""
 import pytest
 import torch
