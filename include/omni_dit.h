@@ -419,6 +419,13 @@ int odit_linear_pair(const odit_linear_problem problems[2], int N, int K, int ep
 int odit_linear_fork(const odit_linear_problem problems[2], const int N[2], int K, const int epilogue[2], int dtype, unsigned flags,
                      void* workspace, size_t workspace_bytes, void* stream);
 
+/* Three projections of the same K, of rows and widths of their own, as odit_linear_fork takes two: to_qkv of a block's self-attention with
+ * to_k and to_v of its cross-attention, whose rows are there from the start (wan2_2_transformer.py:520-530). launch = 0: nothing is
+ * launched, only the answer given. ODIT_ENOTSUP, with nothing launched, where the first one's own call and the others, in one launch
+ * or two, are expected to be faster (ODIT_LINEAR_HANDWRITTEN: in one launch whatever is expected). */
+int odit_linear_three(const odit_linear_problem problems[3], const int N[3], int K, const int epilogue[3], int dtype, unsigned flags,
+                      int launch, void* workspace, size_t workspace_bytes, void* stream);
+
 /* Two projections of the same K in one launch of the tile kernel (or, for two of heads of 64 features, the small one), of which one or both are projections to query, key and value heads
  * (heads[i] not NULL): N[i] = 3 H D features (bias or none), S rows of each batch entry (M = B S), whose queries and keys are normed
  * over each head (mean of squares + eps), weighted and rotated in pairs (2 i, 2 i + 1) at the tile's end and stored with the values in

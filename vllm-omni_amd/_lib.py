@@ -107,6 +107,8 @@ _SIGNATURES = {
         C.c_int, [C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_uint, C.c_void_p, C.c_size_t, C.c_void_p]),
     "odit_linear_fork": (
         C.c_int, [C.c_void_p, C.POINTER(C.c_int), C.c_int, C.POINTER(C.c_int), C.c_int, C.c_uint, C.c_void_p, C.c_size_t, C.c_void_p]),
+    "odit_linear_three": (
+        C.c_int, [C.c_void_p, C.POINTER(C.c_int), C.c_int, C.POINTER(C.c_int), C.c_int, C.c_uint, C.c_int, C.c_void_p, C.c_size_t, C.c_void_p]),
     "odit_linear_heads": (
         C.c_int, [C.c_void_p, C.POINTER(C.c_int), C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_void_p), C.c_int, C.c_uint, C.c_int, C.c_void_p,
                   C.c_size_t, C.c_void_p]),

@@ -58,15 +58,15 @@ struct TileX2 {
 
 struct TilePlan {
   int bm = 0;             // rows per tile (0: no plan)
-  int tiles0, tiles;      // tiles of the first problem, of all
+  int tiles0, tiles1, tiles;  // tiles of the first problem, of the first two, of all
   int whole, parts;       // tiles that are not cut along the reduction; parts of each of the others
   int grid;
   float us;               // expected time
 };
-// One problem or two of the same K; `scratch`: whether tiles may be cut.
+// One problem, or two or three of the same K; `scratch`: whether tiles may be cut.
 TilePlan plan_gemm_tile(const GemmCall* c, int count, int cus, bool scratch);
 
-// One problem, or two of the same K in one launch. `scratch` as for launch_gemm_streamk, or null (no tile is cut). `x2`: with
+// One problem, or two or three of the same K in one launch. `scratch` as for launch_gemm_streamk, or null (no tile is cut). `x2`: with
 // one problem only.
 int launch_gemm_tile(const GemmCall* c, int count, const TileX2* x2, int dtype, void* scratch, hipStream_t stream);
 

@@ -37,7 +37,8 @@ TilePlan plan_gemm_tile(const GemmCall* c, int count, int cus, bool scratch) {
     TilePlan p;
     p.bm = bm;
     p.tiles0 = row_tiles(c[0].M, bm) * row_tiles(c[0].N, kTileN);
-    p.tiles = p.tiles0 + (count > 1 ? row_tiles(c[1].M, bm) * row_tiles(c[1].N, kTileN) : 0);
+    p.tiles1 = p.tiles0 + (count > 1 ? row_tiles(c[1].M, bm) * row_tiles(c[1].N, kTileN) : 0);
+    p.tiles = p.tiles1 + (count > 2 ? row_tiles(c[2].M, bm) * row_tiles(c[2].N, kTileN) : 0);
     const int rounds = p.tiles / most, rest = p.tiles - rounds * most;
     float end = 5.7f;
     for (int i = 0; i < count; ++i)

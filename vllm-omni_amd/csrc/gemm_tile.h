@@ -1,4 +1,4 @@
-// 16-bit GEMM y = x W^T for projections with many rows, for one problem or two of the same reduction length in one launch.
+// 16-bit GEMM y = x W^T for projections with many rows, for one problem or up to three of the same reduction length in one launch.
 //
 // Workgroup: 8 wavefronts, two per SIMD, on an output tile of BM x BN = 256 x 256 (or 128 x 256). The tile's rows are two
 // halves X0, X1 and its features two halves W0, W1; a wavefront (2 along the rows x 4 along the features) owns a quarter of
@@ -70,8 +70,8 @@ struct TileProblem {
 };
 
 struct TileParams {
-  TileProblem q[2];
-  int tiles0, tiles;  // tiles of the first problem, of both
+  TileProblem q[3];
+  int tiles0, tiles1, tiles;  // tiles of the first problem, of the first two, of all
   int whole;          // tiles that are not cut; the others are cut into `parts` along the reduction
   int parts;
   int k_steps;
@@ -82,7 +82,7 @@ struct TileParams {
 
 template <bool HEADS> struct TileArgs : TileParams {};
 template <> struct TileArgs<true> : TileParams {
-  HeadsOut heads[2];  // of the two problems; q null: an ordinary output
+  HeadsOut heads[2];  // of the two problems (there are no three with heads); q null: an ordinary output
 };
 
 typedef __attribute__((address_space(3))) void* lds_void_p;
@@ -270,8 +270,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // problem, first row and first feature of a tile: groups of 8 row tiles, feature tiles outer inside a group, so that the 32
   // tiles an XCD runs at a time share 8 pieces of x and 4 of W
   auto locate = [&](int tile, int& which, int& m0, int& n0) __attribute__((always_inline)) {
-    which = tile >= p.tiles0 ? 1 : 0;
-    const int t = which ? tile - p.tiles0 : tile;
+    which = tile >= p.tiles1 ? 2 : tile >= p.tiles0 ? 1 : 0;
+    const int t = tile - (which == 2 ? p.tiles1 : which == 1 ? p.tiles0 : 0);
     const int mt = p.q[which].m_tiles, per = 8 * p.q[which].n_tiles;
     const int g = quotient(t, per), first = g * 8, gm = mt - first < 8 ? mt - first : 8;
     const int r = t - g * per, nt = quotient(r, gm);
@@ -739,7 +739,7 @@ int row_tiles(int M, int bm) { return (M + bm - 1) / bm; }
 
 // What a launch of `plan` takes beside its heads
 inline void fill_tile_params(TileParams& p, const TilePlan& plan, const GemmCall* c, int count, const TileX2* x2, void* scratch) {
-  for (int i = 0; i < 2; ++i) {
+  for (int i = 0; i < 3; ++i) {
     const GemmCall& g = c[i < count ? i : 0];
     TileProblem& q = p.q[i];
     q.x = g.x; q.w = g.w; q.M = g.M; q.N = g.N;
@@ -755,7 +755,7 @@ inline void fill_tile_params(TileParams& p, const TilePlan& plan, const GemmCall
     q.n_tiles = (g.N + kTileN - 1) / kTileN;
     q.ep = gemm_epilogue_of(g);
   }
-  p.tiles0 = plan.tiles0; p.tiles = plan.tiles; p.whole = plan.whole; p.parts = plan.parts;
+  p.tiles0 = plan.tiles0; p.tiles1 = plan.tiles1; p.tiles = plan.tiles; p.whole = plan.whole; p.parts = plan.parts;
   p.k_steps = c[0].K / kTileK;
   p.counters = static_cast<unsigned long long*>(scratch);
   p.epoch = plan.parts > 1 ? next_ticket_epoch() : 0;

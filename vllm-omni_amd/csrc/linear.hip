@@ -717,31 +717,56 @@ extern "C" int odit_linear_pair(const odit_linear_problem* q, int N, int K, int 
 // rows' pieces in L2 for both.
 constexpr float kOneLaunchGain = .98f;
 
-extern "C" int odit_linear_fork(const odit_linear_problem* q, const int* N, int K, const int* epilogue, int dtype, unsigned flags, void* workspace,
-                                size_t workspace_bytes, void* stream) {
+// The same for a third one, of other rows (what it is compared with: the first one's call and the others in one launch or two calls).
+// Wan's QKV with the cross-attention's keys and values, whose rows are there from the start, us, apart / one launch: 2706 rows and 512 353 +
+// 60 / 364; 5000 and 512 584 + 60 / 601; 2048 and 512 238 + 60 / 287; 1500 and 512 188 + 60 / 244.
+static int lin_beside(const char* name, const odit_linear_problem* q, int count, const int* N, int K, const int* epilogue, int dtype, unsigned flags,
+                      int launch, bool force, void* workspace, size_t workspace_bytes, void* stream) {
   using namespace odit;
-  ODIT_CHECK_ARG(q != nullptr && N != nullptr && epilogue != nullptr, "odit_linear_fork: null arguments");
   void *sk, *lib;
   size_t lib_bytes;
   lin_split_ws(workspace, workspace_bytes, &sk, &lib, &lib_bytes);
   int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) { set_error("odit_linear_fork: hipGetDevice failed"); return ODIT_ELAUNCH; }
-  GemmCall g[2];
-  bool tile = lin_engine_of(flags) == 0 && (flags & (ODIT_LINEAR_FIRST | ODIT_LINEAR_NO_TILE)) == 0;
-  float two = 0;
-  for (int i = 0; i < 2; ++i) {
+  if (hipGetDevice(&dev) != hipSuccess) { set_error("%s: hipGetDevice failed", name); return ODIT_ELAUNCH; }
+  GemmCall g[3];
+  const bool tile = (lin_engine_of(flags) == 0 || force) && (flags & (ODIT_LINEAR_FIRST | ODIT_LINEAR_NO_TILE)) == 0;
+  float us[3] = {0.f, 0.f, 0.f};
+  for (int i = 0; i < count; ++i) {
     const LinCall c{q[i].x, q[i].w, q[i].bias, nullptr, nullptr, q[i].out, q[i].M, N[i], K, q[i].ldx, q[i].ldw, q[i].ldo, 0,
                     epilogue[i], dtype, dtype, lib, lib_bytes, static_cast<hipStream_t>(stream)};
     const int rc = lin_check(c);
     if (rc != ODIT_OK) return rc;
-    ODIT_CHECK_ARG(!lin_is_residual(c), "odit_linear_fork: no residual");
+    if (lin_is_residual(c)) { set_error("%s: no residual", name); return ODIT_EINVAL; }
     g[i] = lin_gemm_call(c, 0, 0);
-    if (!tile || q[i].M < kTileMinAuto || !gemm_tile_takes(g[i], dtype)) return ODIT_ENOTSUP;
-    two += lin_call_us(dev, c, g[i], sk);
+    if (!tile || (!force && q[i].M < kTileMinAuto) || !gemm_tile_takes(g[i], dtype)) return ODIT_ENOTSUP;
+    if (!force) us[i] = lin_call_us(dev, c, g[i], sk);
   }
-  const TilePlan plan = plan_gemm_tile(g, 2, device_cus(), sk != nullptr);
-  if (plan.bm == 0 || plan.us >= kOneLaunchGain * two) return ODIT_ENOTSUP;
-  return launch_gemm_tile(g, 2, nullptr, dtype, sk, static_cast<hipStream_t>(stream));
+  const int cus = device_cus();
+  const TilePlan plan = plan_gemm_tile(g, count, cus, sk != nullptr);
+  if (plan.bm == 0) return ODIT_ENOTSUP;
+  if (!force) {
+    float others = us[1] + us[2];
+    if (count == 3) {
+      const TilePlan two = plan_gemm_tile(g + 1, 2, cus, sk != nullptr);
+      if (two.bm > 0 && two.us < others) others = two.us;
+    }
+    if (plan.us >= kOneLaunchGain * (us[0] + others)) return ODIT_ENOTSUP;
+  }
+  return launch == 0 ? ODIT_OK : launch_gemm_tile(g, count, nullptr, dtype, sk, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int odit_linear_fork(const odit_linear_problem* q, const int* N, int K, const int* epilogue, int dtype, unsigned flags, void* workspace,
+                                size_t workspace_bytes, void* stream) {
+  using namespace odit;
+  ODIT_CHECK_ARG(q != nullptr && N != nullptr && epilogue != nullptr, "odit_linear_fork: null arguments");
+  return lin_beside("odit_linear_fork", q, 2, N, K, epilogue, dtype, flags, 1, false, workspace, workspace_bytes, stream);
+}
+
+extern "C" int odit_linear_three(const odit_linear_problem* q, const int* N, int K, const int* epilogue, int dtype, unsigned flags, int launch,
+                                 void* workspace, size_t workspace_bytes, void* stream) {
+  using namespace odit;
+  ODIT_CHECK_ARG(q != nullptr && N != nullptr && epilogue != nullptr, "odit_linear_three: null arguments");
+  return lin_beside("odit_linear_three", q, 3, N, K, epilogue, dtype, flags, launch, lin_engine_of(flags) == 2, workspace, workspace_bytes, stream);
 }
 
 // Projections to query, key and value heads with the heads' norm and rotation at the tile's end, or the projections and a pass over

@@ -1048,6 +1048,24 @@ void project_fork(BlockCall& c, const void* x, const Lin l[2], void* const y[2],
   for (int i = 0; i < 2; ++i) c.project(x, l[i], y[i], M, gelu && i == 0);
 }
 
+// Three projections, of rows of their own, in one launch; launch false: whether they would. False, with nothing launched, where calls of
+// their own are the better way.
+bool project_three(BlockCall& c, const void* const x[3], const Lin l[3], void* const y[3], const int64_t M[3], bool launch) {
+  if (c.rc != 0) return true;
+  if (l[0].k != l[1].k || l[0].k != l[2].k || (c.engine & ODIT_LINEAR_HANDWRITTEN)) return false;
+  odit_linear_problem q[3];
+  int n[3], epi[3];
+  for (int i = 0; i < 3; ++i) {
+    q[i] = {x[i], l[i].w, l[i].b, nullptr, nullptr, y[i], static_cast<int>(M[i]), 0, l[i].k, l[i].ldw, l[i].n, 0, 0};
+    n[i] = static_cast<int>(l[i].n);
+    epi[i] = l[i].b ? ODIT_EPI_BIAS : ODIT_EPI_NONE;
+  }
+  const int rc = odit_linear_three(q, n, static_cast<int>(l[0].k), epi, c.dtype, c.engine, launch, c.lin_ws.p, c.lin_ws.bytes, c.where.stream);
+  if (rc == ODIT_ENOTSUP && !launch) return false;
+  c.check(rc);
+  return true;
+}
+
 // Two projections of which one or both go to query, key and value heads, in one launch: heads[i].q null is an ordinary output y[i]
 // (GELU where `gelu`). launch false: whether they would. False, with nothing launched, where the projections and the pass behind
 // them are the better way.
@@ -1568,17 +1586,34 @@ PyObject* py_wan_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
   std::optional<Unlocked> others_run(std::in_place);
   const int esz = 2;
   void *nx, *q3, *q, *k, *o, *u, *kc, *kn, *vc, *y;
+  // the text's keys and values with the self-attention's projection where that is expected to be faster (asked with addresses that stand
+  // in for the ones to come)
+  const Lin three[3] = {qkv, k2, v2};
+  const int64_t three_rows[3] = {B * S, B * T, B * T};
+  const void* const any[3] = {ctx->data_ptr(), ctx->data_ptr(), ctx->data_ptr()};
+  void* const any_out[3] = {ctx->data_ptr(), ctx->data_ptr(), ctx->data_ptr()};
+  const bool early = project_three(c, any, three, any_out, three_rows, false);
+  if (c.rc != 0) {
+    others_run.reset();
+    return block_failed(c.rc);
+  }
   Slab slab(esz);
   slab.want(&nx, B * S * C);
   slab.want(&q, B * S * HD);
   slab.want(&k, B * S * HD);
   slab.want(&o, B * S * HD);
+  if (early) {
+    slab.want(&kc, B * T * HD);
+    slab.want(&vc, B * T * HD);
+  }
   slab.mark();
   slab.want(&q3, B * S * 3 * HD);  // self-attention
   slab.rewind();
-  slab.want(&kc, B * T * HD);  // cross-attention
-  slab.want(&kn, B * T * HD);
-  slab.want(&vc, B * T * HD);
+  slab.want(&kn, B * T * HD);  // cross-attention
+  if (!early) {
+    slab.want(&kc, B * T * HD);
+    slab.want(&vc, B * T * HD);
+  }
   slab.rewind();
   slab.want(&u, B * S * F);  // feed-forward
   slab.allocate(x->options());
@@ -1623,7 +1658,13 @@ PyObject* py_wan_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
     project_gated(c, src, l, residual, out.data_ptr(), B, S, g, min_rows, y, plain);
   };
   modulate(x->data_ptr(), 0);
-  c.project(nx, qkv, q3, B * S, false);
+  if (early) {
+    const void* const rows[3] = {nx, ctx->data_ptr(), ctx->data_ptr()};
+    void* const into[3] = {q3, kc, vc};
+    project_three(c, rows, three, into, three_rows, true);
+  } else {
+    c.project(nx, qkv, q3, B * S, false);
+  }
   char* qp = static_cast<char*>(q3);
   const int64_t st3[2] = {S * 3 * HD, 3 * HD}, st1[2] = {S * HD, HD}, stc[2] = {T * HD, HD};
   if (c.rc == 0)
@@ -1644,9 +1685,11 @@ PyObject* py_wan_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
     n2 = nx;
   }
   c.project(n2, q2, k, B * S, false);
-  const Lin kv[2] = {k2, v2};
-  void* const kv_out[2] = {kc, vc};
-  project_fork(c, ctx->data_ptr(), kv, kv_out, B * T, false);
+  if (!early) {
+    const Lin kv[2] = {k2, v2};
+    void* const kv_out[2] = {kc, vc};
+    project_fork(c, ctx->data_ptr(), kv, kv_out, B * T, false);
+  }
   if (c.rc == 0)
     c.check(odit_qknorm_rope(k, nullptr, nullptr, q, nullptr, nullptr, nw[2], nullptr, nullptr, nullptr, B, S, H, D, 0, st1, 0, S,
                              static_cast<float>(eps_n[2]), ODIT_NORM_ROW, w_dtype, c.dtype, 0u, c.where.stream));
