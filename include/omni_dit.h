@@ -119,7 +119,8 @@ size_t odit_attn_fwd_workspace_bytes(int B, int Sq, int Sk, int H, int D);
 /* Which kernels odit_attn_fwd_ex launches for a problem, as text: "<kernel> units=<workgroups>" per
  * launch, joined by "; " (the kernel names are the ones a profiler reports). k_seq_stride / v_seq_stride
  * are the sequence strides of k and v in elements; with_workspace says whether scratch will be given. (With a key mask of
- * up to 65536 keys the last template argument of attn_fwd_dma_kernel is 3 where it says 0 and 4 where it says 1.)
+ * up to 65536 keys the last template argument of attn_fwd_dma_kernel is 3 or 5 where it says 0, 4 where it says 1 and 7 or 8 where
+ * it says 6.)
  * Returns the number of launches, or a negative status. Host-only: enqueues nothing. No counterpart in the
  * reference; for tests and for benchmarks that must name the kernel they time.
  */

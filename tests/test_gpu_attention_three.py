@@ -1,5 +1,5 @@
-"""Head size 64 with three workgroups per compute unit (csrc/attn_fwd_dma.hip, fills_three): the bits of the same attention in
-launches of fewer units, which run two of them, and the oracle's result."""
+"""Head size 64 with three workgroups per compute unit and, where those need as many rounds, with two (csrc/attn_fwd_dma.hip,
+fills_two): the bits of the same attention in launches of fewer units, and the result in 64 bits."""
 
 import pytest
 import torch
@@ -9,16 +9,20 @@ from vllm_omni_amd import kernels
 pytestmark = pytest.mark.gpu
 
 
-# units of 128 query rows: from 513 to 768 a launch takes the form (from 641 on where the keys are enough to be split)
+# units of 128 query rows: from 769 to 1024 a launch runs two workgroups per compute unit
 @pytest.mark.parametrize("B,Sq,Sk,H,Hkv,masked", [
     (1, 5500, 1, 16, 16, False),    # one key
     (1, 5500, 65, 16, 4, False),    # 688 units, a tile and one key
     (1, 2049, 300, 31, 31, False),  # 527 units, one row in the last block, keys too few to be split
     (1, 1300, 64, 48, 48, False),   # 528 units, one tile
     (2, 1536, 130, 32, 32, False),  # 768 units: all there is room for
-    (1, 6145, 1100, 16, 16, False), # 784 units: two workgroups per compute unit again
+    (1, 6145, 1100, 16, 16, False), # 784 units: two workgroups per compute unit
+    (1, 8192, 64, 16, 4, False),    # 1024 units: the last launch of two
     (3, 700, 700, 40, 8, True),     # batch rows spread over the XCDs
     (2, 1357, 129, 31, 31, True),   # heads that do not divide over them
+    (2, 2049, 300, 24, 24, True),   # 816 units: two with mask words, batch rows spread over the XCDs
+    (2, 2049, 65, 25, 25, True),    # 850 units, heads that do not divide over them
+    (3, 1200, 193, 40, 8, True),    # 1200 units: three again
 ])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_three_workgroups_per_compute_unit(gpu, B, Sq, Sk, H, Hkv, masked, dtype):

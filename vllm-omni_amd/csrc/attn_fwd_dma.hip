@@ -120,17 +120,22 @@ typedef __attribute__((address_space(3))) void* lds_void_p;
 //         result in scratch for attn_merge_kernel.
 // MODE 2: persistent, see above.
 // MODE 3, 4: 0 and 1 for a key mask held as words. MODE 5: 3 with the batch rows spread over the XCDs (spread_batch).
-// MODE 6, 7, 8: 0, 3 and 5 of head size 64 with three workgroups per compute unit (fills_three).
+// MODE 6, 7, 8: 0, 3 and 5 of head size 64 with two workgroups per compute unit in the place of three (fills_two).
 // Separate instantiations, so the extra bookkeeping of one cannot disturb the register allocation of another (that of the
 // words in the launches without a mask: 452 -> 460 us at B=2 S=4352 H=24 D=128, 252 -> 262 at B=1 S=4608).
 constexpr int kMaskWords = 1024;  // 8 KB of LDS: two workgroups of D = 128 still fit a compute unit (144 of 160 KB)
 
+// Wavefronts on a SIMD, which is workgroups of 4 wavefronts on a compute unit: stated, both ways, because at head size 64 the registers
+// that a form happens to take (162 to 174, three wavefronts up to 168) would settle it otherwise.
+constexpr int kWavesPerSimd(int D, int NW, int MODE) { return D == 64 && NW == 4 && (MODE == 0 || MODE == 3 || MODE == 5) ? 3 : 2; }
+
 template <typename T, int D, int NW, int MODE>
-__global__ __launch_bounds__(NW * 64, MODE >= 6 ? 3 : 8 / NW) void attn_fwd_dma_kernel(const AttnParams p) {
+__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(kWavesPerSimd(D, NW, MODE), kWavesPerSimd(D, NW, MODE))))
+void attn_fwd_dma_kernel(const AttnParams p) {
   constexpr bool TAIL = MODE == 1 || MODE == 4;
   constexpr bool PERSIST = MODE == 2;
   constexpr bool WORDS = MODE >= 3 && MODE != 6;
-  constexpr bool THREE = MODE >= 6, SPREAD = MODE == 5 || MODE == 8;
+  constexpr bool SPREAD = MODE == 5 || MODE == 8;
   using M = Mma<T>;
   using frag = typename M::frag;
   constexpr int BN = 64;
@@ -162,10 +167,7 @@ __global__ __launch_bounds__(NW * 64, MODE >= 6 ? 3 : 8 / NW) void attn_fwd_dma_
   const int part = blockIdx.x;
   // persistent form: the unit after the current one (-1: none, or not drawn yet)
   int next_pid = -1;
-  // three wavefronts per SIMD: 168 registers, so most of the query fragments stay in LDS and fewer reads run ahead
-  static_assert(!THREE || (D == 64 && NW == 4), "three workgroups per compute unit: head size 64");
-  constexpr int QL = THREE ? (WORDS ? 3 : 4) : 0;
-  __shared__ u32x4_v q_lds[QL > 0 ? NW * QL * 64 : 1];
+  static_assert(MODE < 6 || (D == 64 && NW == 4), "two workgroups per compute unit in the place of three: head size 64");
   __shared__ int next_unit_box;  // thread 0's draw, handed to the workgroup across a tile's barrier
   __shared__ uint64_t mask_words[WORDS ? kMaskWords : 1];  // of key tiles jt0, jt0 + 1, ...
   if constexpr (!TAIL && !PERSIST) {
@@ -183,7 +185,9 @@ __global__ __launch_bounds__(NW * 64, MODE >= 6 ? 3 : 8 / NW) void attn_fwd_dma_
     pid = x_lo + part / kNumXcd;
     if (pid >= x_hi) return;  // fewer units than workgroups on this XCD (before any barrier: the whole workgroup leaves)
   }
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  // (a scalar only where three workgroups with mask words leave no vector register for it: two went to memory)
+  const int wave = WORDS && kWavesPerSimd(D, NW, MODE) == 3 ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6;
   const int l32 = lane & 31, hh = lane >> 5;
   const int wl = PP ? (wave & 3) : wave;     // this wavefront's share of a tile load
   const bool grp1 = PP && wave >= 4;          // second group of the anti-phase form (wave-uniform)
@@ -338,9 +342,6 @@ __global__ __launch_bounds__(NW * 64, MODE >= 6 ? 3 : 8 / NW) void attn_fwd_dma_
       qf[ks] = __builtin_bit_cast(frag, *reinterpret_cast<const u32x4_v*>(qp + ks * 16));
   };
   load_q(b, h, q0);
-  auto q_kept = [&](int ks) { return __builtin_bit_cast(frag, q_lds[(wave * QL + ks - (KS - QL)) * 64 + lane]); };  // (each lane its own)
-#pragma unroll
-  for (int i = 0; i < QL; ++i) q_lds[(wave * QL + i) * 64 + lane] = __builtin_bit_cast(u32x4_v, qf[KS - QL + i]);
 
   f32x16_v o[DT];
 #pragma unroll
@@ -371,7 +372,7 @@ __global__ __launch_bounds__(NW * 64, MODE >= 6 ? 3 : 8 / NW) void attn_fwd_dma_
       for (int kt = 0; kt < 2; ++kt) {
         const frag a = __builtin_bit_cast(
             frag, *reinterpret_cast<const u32x4_v*>(kt_base + kt * 32 * ROWB + (k_lane ^ (ks * 32))));
-        s[kt] = M::run(a, ks < KS - QL ? qf[ks] : q_kept(ks), s[kt]);
+        s[kt] = M::run(a, qf[ks], s[kt]);
       }
   };
 
@@ -521,22 +522,19 @@ __global__ __launch_bounds__(NW * 64, MODE >= 6 ? 3 : 8 / NW) void attn_fwd_dma_
       for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
         for (int e = 0; e < 16; ++e) s_next[kt][e] = 0.f;
-      constexpr int KPF = THREE ? (WORDS ? 1 : 2) : ODIT_ATTN_KPF;  // K fragments in flight ahead of the MFMA that consumes them
+      constexpr int KPF = ODIT_ATTN_KPF;  // K fragments in flight ahead of the MFMA that consumes them
       u32x4_v kfr[KPF + 1];
       auto k_fetch = [&](int i) {
         const int ks = i >> 1, kt = i & 1;
         kfr[i % (KPF + 1)] = *reinterpret_cast<const u32x4_v*>(kt_base + kt * 32 * ROWB + (k_lane_t ^ (ks * 32)));
       };
-      frag qt[2];
-      if constexpr (QL == KS) qt[0] = q_kept(0);
 #pragma unroll
       for (int i = 0; i < KPF; ++i) k_fetch(i);
 #pragma unroll
       for (int i = 0; i < 2 * KS; ++i) {
         if (i + KPF < 2 * KS) k_fetch(i + KPF);
         const int ks = i >> 1, kt = i & 1;
-        if (kt == 0 && ks + 1 < KS && ks + 1 >= KS - QL) qt[(ks + 1) & 1] = q_kept(ks + 1);
-        s_next[kt] = M::run(__builtin_bit_cast(frag, kfr[i % (KPF + 1)]), ks < KS - QL ? qf[ks] : qt[ks & 1], s_next[kt]);
+        s_next[kt] = M::run(__builtin_bit_cast(frag, kfr[i % (KPF + 1)]), qf[ks], s_next[kt]);
         constexpr int PAIRS = 16 / (2 * KS) > 0 ? 16 / (2 * KS) : 1;
 #pragma unroll
         for (int q = 0; q < PAIRS; ++q) {
@@ -592,7 +590,7 @@ __global__ __launch_bounds__(NW * 64, MODE >= 6 ? 3 : 8 / NW) void attn_fwd_dma_
     int v_lane_t = v_lane;  // (opaque copy, as for the key fragments)
     if constexpr (PERSIST) asm volatile("" : "+v"(v_lane_t));
     constexpr int NSTEP = 4 * DT;
-    constexpr int PF = THREE ? 2 : ODIT_ATTN_VPF;
+    constexpr int PF = ODIT_ATTN_VPF;
     s16x4_d vlo[PF + 1], vhi[PF + 1];
     auto v_fetch = [&](int step) {
       const int dt = step % DT, kt = (step / DT) >> 1, g2 = (step / DT) & 1;
@@ -791,20 +789,27 @@ static int persistent_workgroups(int units, int n_tiles, int slots, int nw) {
 // the longest row finish last (B=2, one row of 22 tiles and one of 9, 704 units: the XCDs 0 to 3 had 88 units of 22 tiles each).
 // Where the heads divide evenly every XCD gets its share of each row's heads instead, as many in all (keys and values are shared
 // in its L2 as before), by a grid whose linear index runs over the XCDs first.
-// (With units for less than half the slots each has a compute unit, or nearly, to itself either way.)
+// (With no more units than compute units each has one, or nearly, to itself either way.)
 static bool spread_batch(const AttnParams& p, int slots) {
   return p.B > 1 && p.B < 65536 && p.H % kNumXcd == 0 && p.n_full == p.total_blocks && 2 * p.total_blocks > slots;
 }
 
-// Head size 64 in three workgroups per compute unit instead of two, where they take all units in one round and two would need a
-// second one that the key split does not take. Three wavefronts on a SIMD multiply no faster than two (the vector work of the
-// softmax fills either: B=2 S=4352 H=24 283 us, three everywhere 297; 1024 units of 128 key tiles 315 and 380), so it is a
-// matter of the rounds alone: up to 1.5 rounds of two are one round of three, in which a unit takes 1.5 times as long, and a second
-// round of two takes 0.6 of a first one, its workgroups having a compute unit each. us, two / three, 688 to 752 units:
-//   B=2 S=1357 H=32 f16 54.8 / 48.6, with a padded row 44.5 / 40.7    B=1 S=5500 H=16 174.5 / 151.4, 500 keys 24.2 / 20.8,
-//   64 keys 11.2 / 10.3    B=1 S=12000 H=8 397 / 336    B=3 S=700 H=40 30.8 / 27.1
-// 544 units whose keys are too few to be split (B=1 S=2060, 300 keys, H=32): 18.4 / 14.8.
-static bool fills_three(const TailPlan& t, int units, int slots) { return t.rem == 0 && units > slots && 2 * units <= 3 * slots; }
+// Head size 64 runs three workgroups on a compute unit (kWavesPerSimd): a round of three takes 768 units instead of 512 and, its
+// wavefronts covering each other's softmax, less than 1.5 times as long. Where two workgroups need no more rounds than three, two of
+// them are faster: units in (768, 1024], two rounds either way, the second one of three partly empty. (Up to 512 units nothing differs.)
+// us, two / three, the same bits, bf16:
+//   512 units, 8 key tiles 15.4 / 15.2, 64 tiles 76.1 / 76.0     528, 1 tile 10.7 / 8.3     688, 8 tiles 24.3 / 20.4, 86 tiles 170 / 138
+//   752, 188 tiles 387 / 307     768, 24 tiles 55.0 / 47.1     776, 16 tiles 41.7 / 43.3, 64 tiles 139 / 148     832, 104 tiles 223 / 238
+//   896, 16 tiles 43.0 / 44.4     1024, 16 tiles 45.0 / 45.4, 128 tiles 292 / 300     1200, 32 tiles 106 / 93     1280, 64 tiles 218 / 181
+//   1536, 64 tiles 225 / 215     1632, 68 tiles 272 / 261     2048, 8 tiles 53.9 / 48.9     2512, 64 tiles 371 / 353     6144, 8 tiles 162 / 140
+// with a mask, f16, every key live: 704, 22 tiles 52.5 / 42.3     800, 20 tiles 53.6 / 56.8     816, 47 tiles 113 / 124     1024, 16 tiles
+//   46.8 / 48.2, 64 tiles 162 / 171     1632, 8 tiles 50 / 44.5, 68 tiles 293 / 273     2944, 64 tiles 475 / 436     3072, 16 tiles 143 / 127;
+//   one of two rows padded to 40 %, which the launch does not know: 800 units 40.3 / 33.9, 1024 117 / 109, 1632 289 / 271.
+// (A unit's first 4 query fragments in LDS and fewer reads ahead, 164 registers: as fast at one round, 1 to 7 % slower beyond.)
+// `main_units`: without those that the key split takes. It counts rounds of two (device_slots) in either form, so that what a unit's
+// keys are cut into does not depend on the form: us, bf16, split / whole, 520 units of 64 tiles 90 / 97, 640 of 64 113 / 102, of 16
+// tiles 47 / 31, 1088 of 64 177 / 169, 1544 of 64 230 / 248, of 16 76 / 71.
+static bool fills_two(int64_t main_units, int slots) { return 2 * main_units > 3 * static_cast<int64_t>(slots) && main_units <= 2 * static_cast<int64_t>(slots); }
 
 template <typename T, int D, int NW>
 static int launch_dma(AttnParams& p, hipStream_t stream, void* ws, size_t ws_bytes) {
@@ -849,14 +854,14 @@ static int launch_dma(AttnParams& p, hipStream_t stream, void* ws, size_t ws_byt
         hipLaunchKernelGGL((attn_fwd_dma_kernel<T, D, NW, 2>), dim3(W), dim3(NW * 64), 0, stream, p);
       }
     }
-    const bool three = D == 64 && NW == 4 && W == 0 && fills_three(t, p.total_blocks, slots);
+    const bool two = D == 64 && NW == 4 && W == 0 && fills_two(p.n_full, slots);
     if constexpr (D == 64 && NW == 4) {
-      if (three && words && spread_batch(p, slots))
+      if (two && words && spread_batch(p, slots))
         hipLaunchKernelGGL((attn_fwd_dma_kernel<T, D, NW, 8>), dim3(p.n_qblocks * kNumXcd, p.H / kNumXcd, p.B), dim3(NW * 64), 0, stream, p);
-      else if (three && words) hipLaunchKernelGGL((attn_fwd_dma_kernel<T, D, NW, 7>), dim3(p.n_full), dim3(NW * 64), 0, stream, p);
-      else if (three) hipLaunchKernelGGL((attn_fwd_dma_kernel<T, D, NW, 6>), dim3(p.n_full), dim3(NW * 64), 0, stream, p);
+      else if (two && words) hipLaunchKernelGGL((attn_fwd_dma_kernel<T, D, NW, 7>), dim3(p.n_full), dim3(NW * 64), 0, stream, p);
+      else if (two) hipLaunchKernelGGL((attn_fwd_dma_kernel<T, D, NW, 6>), dim3(p.n_full), dim3(NW * 64), 0, stream, p);
     }
-    if (W == 0 && !three) {
+    if (W == 0 && !two) {
       if (words && spread_batch(p, slots))
         hipLaunchKernelGGL((attn_fwd_dma_kernel<T, D, NW, 5>), dim3(p.n_qblocks * kNumXcd, p.H / kNumXcd, p.B), dim3(NW * 64), 0, stream, p);
       else if (words) hipLaunchKernelGGL((attn_fwd_dma_kernel<T, D, NW, 3>), dim3(p.n_full), dim3(NW * 64), 0, stream, p);
@@ -937,8 +942,8 @@ int attn_dma_plan(int B, int Sq, int Sk, int H, int D, bool with_workspace, char
     snprintf(main_text, sizeof(main_text), "attn_fwd_dma_kernel<T, %d, %d, 2> units=%lld on %d persistent workgroups", D,
              nw, static_cast<long long>(main_units), W);
   } else {
-    const bool three = D == 64 && nw == 4 && main_units <= 0x3fffffff && fills_three(t, static_cast<int>(main_units), slots);
-    snprintf(main_text, sizeof(main_text), "attn_fwd_dma_kernel<T, %d, %d, %d> units=%lld", D, nw, three ? 6 : 0,
+    const bool two = D == 64 && nw == 4 && fills_two(main_units, slots);
+    snprintf(main_text, sizeof(main_text), "attn_fwd_dma_kernel<T, %d, %d, %d> units=%lld", D, nw, two ? 6 : 0,
              static_cast<long long>(main_units));
   }
   if (t.rem == 0) {

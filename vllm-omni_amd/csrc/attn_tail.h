@@ -79,8 +79,9 @@ struct TailPlan { int rem, key_chunks, tiles_per_chunk; };
 constexpr int kMinTilesPerChunk = 8;
 constexpr int kMaxKeyChunks = kMergeMaxChunks;
 
-// workgroups resident at once: compute units x workgroups per unit (8 / nw for the nw-wave kernels that run
-// two wavefronts per SIMD; pass nw = 8 for one workgroup per unit)
+// workgroups of a round: compute units x workgroups per unit, with two wavefronts per SIMD (8 / nw for the nw-wave kernels; pass nw = 8
+// for one workgroup per unit). Head size 64 runs three wavefronts per SIMD mostly; its plans count rounds of two all the same
+// (attn_fwd_dma.hip, fills_two).
 inline int device_slots(int nw) {
   static int cus[64] = {0};
   int dev = 0;
