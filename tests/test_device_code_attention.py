@@ -3,7 +3,9 @@ attn_fwd_dma.hip. CPU only."""
 
 import re
 
-from test_device_code import _assembly
+import pytest
+
+from test_device_code import _CSRC, _assembly
 
 
 def _kernels():
@@ -33,3 +35,13 @@ def test_as_many_workgroups_on_a_compute_unit_as_the_launch_rules_count_on():
         want = 3 if (d, waves) == (64, 4) and form in (0, 3, 5) else 8 // waves
         assert by_registers == want and by_lds >= want, (dtype, d, waves, form, k["next_free_vgpr"], k["group_segment_fixed_size"])
         assert int(k["private_segment_fixed_size"]) == 0, ("registers in memory", dtype, d, waves, form)
+
+
+@pytest.mark.parametrize("source", sorted(p.name for p in _CSRC.iterdir() if p.suffix in (".hip", ".h")))
+def test_no_vector_instruction_in_inline_assembly(source):
+    """A vector instruction may read what a matrix instruction wrote some wait states later only. The compiler counts them, but does not
+    look into inline assembly."""
+    text = (_CSRC / source).read_text()
+    for m in re.finditer(r"\basm\b(?:\s+volatile)?\s*\(", text):
+        code = "".join(re.findall(r'"((?:[^"\\]|\\.)*)"', text[m.end():text.index(";", text.index(")", m.end()))].split(":")[0]))
+        assert not re.search(r"(^|[\s;]|\\[nt])v_", code), code

@@ -34,3 +34,30 @@ def test_single_keys_take_the_maximum(head_size, keys, queries, dtype):
     eps = torch.finfo(dtype).eps / 2
     bound = 2 * eps * ((p @ vd.abs()).transpose(1, 2).reshape(out.shape) + want.abs()) + 1e-6
     assert bool(((out - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("head_size, keys", [(128, 640), (128, 2112), (64, 193)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_nan_scores_stay_with_their_query(head_size, keys, dtype):
+    """A NaN among the queries spoils its own row, one among the keys its head, and one among keys that are excluded nothing."""
+    from vllm_omni_amd import kernels
+
+    g = torch.Generator(device="cuda").manual_seed(keys)
+    q, k, v = (torch.randn(1, s, 4, head_size, device="cuda", generator=g).to(dtype) for s in (130, keys, keys))
+    mask = torch.ones(1, keys, dtype=torch.bool, device="cuda")
+    mask[0, 70] = False
+    for m in (None, mask):
+        clean = kernels.attn_fwd(q, k, v, head_size ** -0.5, key_mask=m)
+        spoiled = q.clone()
+        spoiled[0, 33, 1, 5] = float("nan")
+        out = kernels.attn_fwd(spoiled, k, v, head_size ** -0.5, key_mask=m)
+        assert bool(out[0, 33, 1].isnan().all())
+        out[0, 33, 1] = clean[0, 33, 1]
+        assert torch.equal(out, clean)
+        at_key = k.clone()
+        at_key[0, 70, 2, 0] = float("nan")
+        out = kernels.attn_fwd(q, at_key, v, head_size ** -0.5, key_mask=m)
+        if m is None:
+            assert bool(out[0, :, 2].isnan().all())
+            out[0, :, 2] = clean[0, :, 2]
+        assert torch.equal(out, clean)

@@ -376,15 +376,16 @@ void attn_fwd_dma_kernel(const AttnParams p) {
       }
   };
 
-  // The lane's maximum of its 32 scores, in 16 instructions. (Inline assembly: the compiler puts a maximum with itself, which quiets a
-  // NaN, in front of values that it has not computed.)
+  // The lane's maximum of its 32 scores, in 16 instructions (v_maximum3_f32; fmaxf would first put a maximum with itself, which quiets
+  // a NaN, in front of every score). A NaN score takes the lane's maximum, which then is not looked at: the query's result is NaN
+  // anyway. Not inline assembly, although the scores are matrix results: the vector unit may read those some wait states later
+  // only, and it is the compiler that sees to them.
   constexpr int NMAX = 16;
   auto max_step = [&](const f32x16_v(&s)[2], float mx, int n) __attribute__((always_inline)) -> float {
-    float r;
-    if (n == 0) asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(s[0][0]), "v"(s[0][1]), "v"(s[0][2]));
-    else if (n == NMAX - 1) asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(mx), "v"(s[1][15]));
-    else asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(mx), "v"(s[(2 * n + 1) >> 4][(2 * n + 1) & 15]), "v"(s[(2 * n + 2) >> 4][(2 * n + 2) & 15]));
-    return r;
+    auto e = [&](int i) __attribute__((always_inline)) { return s[i >> 4][i & 15]; };
+    if (n == 0) return __builtin_elementwise_maximum(__builtin_elementwise_maximum(e(0), e(1)), e(2));
+    if (n == NMAX - 1) return __builtin_elementwise_maximum(mx, e(31));
+    return __builtin_elementwise_maximum(__builtin_elementwise_maximum(mx, e(2 * n + 1)), e(2 * n + 2));
   };
 
   // excluded scores of tile j become -inf (branch-free selects: every lane rewrites all its scores); returns the lane's maximum.
@@ -621,11 +622,13 @@ void attn_fwd_dma_kernel(const AttnParams p) {
           plain_next = has_next && (lo & hi) == ~0u;
         }
       }
-      // (the next scores' maximum, an instruction or two behind each MFMA; formed again where keys are excluded)
+      // (the next scores' maximum, an instruction or two behind each MFMA, where the empty asm holds it: it would sink below the test of
+      // plain_next otherwise, 264 units of head size 64 65 -> 68 us; formed again where keys are excluded)
       constexpr int EACH = (NMAX + NSTEP - 2) / (NSTEP - 1);
       if (st > 0) {
 #pragma unroll
         for (int n = (st - 1) * EACH; n < st * EACH && n < NMAX; ++n) mx = max_step(s_next, mx, n);
+        asm volatile("" : "+v"(mx));
       }
       __builtin_amdgcn_sched_barrier(0);  // keep the reads of step st+PF ahead of this MFMA
     }
