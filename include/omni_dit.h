@@ -420,9 +420,17 @@ int odit_linear_pair(const odit_linear_problem problems[2], int N, int K, int ep
 int odit_linear_fork(const odit_linear_problem problems[2], const int N[2], int K, const int epilogue[2], int dtype, unsigned flags,
                      void* workspace, size_t workspace_bytes, void* stream);
 
+/* What the next two functions do: launch where one launch is expected to be the faster way (ODIT_LAUNCH_CHOOSE), answer whether it is
+ * and launch nothing (ODIT_LAUNCH_ASK), or launch because an earlier answer for problems of these sizes was ODIT_OK
+ * (ODIT_LAUNCH_ANSWERED: the operands are checked, what is expected is not looked at again, and a tuning call in between
+ * changes nothing). */
+#define ODIT_LAUNCH_ASK 0
+#define ODIT_LAUNCH_CHOOSE 1
+#define ODIT_LAUNCH_ANSWERED 2
+
 /* Three projections of the same K, of rows and widths of their own, as odit_linear_fork takes two: to_qkv of a block's self-attention with
- * to_k and to_v of its cross-attention, whose rows are there from the start (wan2_2_transformer.py:520-530). launch = 0: nothing is
- * launched, only the answer given. ODIT_ENOTSUP, with nothing launched, where the first one's own call and the others, in one launch
+ * to_k and to_v of its cross-attention, whose rows are there from the start (wan2_2_transformer.py:520-530). launch: ODIT_LAUNCH_.
+ * ODIT_ENOTSUP, with nothing launched, where the first one's own call and the others, in one launch
  * or two, are expected to be faster (ODIT_LINEAR_HANDWRITTEN: in one launch whatever is expected). */
 int odit_linear_three(const odit_linear_problem problems[3], const int N[3], int K, const int epilogue[3], int dtype, unsigned flags,
                       int launch, void* workspace, size_t workspace_bytes, void* stream);
@@ -435,7 +443,7 @@ int odit_linear_three(const odit_linear_problem problems[3], const int N[3], int
  * single-stream block (flux_transformer.py:288-309). What odit_qknorm_rope makes of the projection's output (the same operations in the same
  * order; of the two products of an odd feature's rotation the compiler may round the other one) without that output
  * (problems[i].out is not used). The other problem as for odit_linear_fork. wq, wk [D] of `dtype`; cos, sin float32
- * [S, D / 2]; D = 64 or 128; everything 16-byte aligned. launch = 0: nothing is launched, only the answer given. ODIT_ENOTSUP,
+ * [S, D / 2]; D = 64 or 128; everything 16-byte aligned. launch: ODIT_LAUNCH_. ODIT_ENOTSUP,
  * with nothing launched, where the projections and the pass behind them are expected to be faster apart (ODIT_LINEAR_HANDWRITTEN: in
  * one launch whatever is expected). */
 typedef struct odit_head_output {

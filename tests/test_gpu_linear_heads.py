@@ -157,6 +157,18 @@ def test_heads_in_one_launch_where_that_is_expected_to_be_faster(scratch, gpu):
         assert _run(ps, (S1, 0), joint, 3072, torch.bfloat16, scratch, launch=0) == want
 
 
+def test_what_was_answered_is_launched(scratch, gpu):
+    """A caller that has laid its memory out by an answer gets the launch, whatever is expected by then; operands are checked as ever."""
+    ps = [_Problem(gpu, torch.bfloat16, 2, S, 3072, 24, 128, seed=S) for S in (256, 40)]
+    joint = [torch.full((2, 296, 24, 128), float("nan"), dtype=torch.bfloat16, device=gpu) for _ in range(3)]
+    assert _run(ps, (40, 0), joint, 3072, torch.bfloat16, scratch, launch=_lib.ODIT_LAUNCH_CHOOSE) == -2  # ODIT_ENOTSUP
+    assert all(bool(t.isnan().all()) for t in joint)
+    assert _run(ps, (40, 0), joint, 3072, torch.bfloat16, scratch, launch=_lib.ODIT_LAUNCH_ANSWERED) == 0
+    _check(ps, (40, 0), joint, torch.bfloat16)
+    assert _run(ps, (41, 0), joint, 3072, torch.bfloat16, scratch, launch=_lib.ODIT_LAUNCH_ANSWERED) == -1  # ODIT_EINVAL: rows past the joint tensors
+    assert _run(ps, (40, 0), joint, 3072, torch.bfloat16, scratch, launch=_lib.ODIT_LAUNCH_ANSWERED, flags=_lib.ODIT_LINEAR_LIBRARY) == -2
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("B,S0,S1,H,K", [
     (1, 256, 64, 4, 256),   # whole tiles

@@ -730,6 +730,7 @@ static int lin_beside(const char* name, const odit_linear_problem* q, int count,
   if (hipGetDevice(&dev) != hipSuccess) { set_error("%s: hipGetDevice failed", name); return ODIT_ELAUNCH; }
   GemmCall g[3];
   const bool tile = (lin_engine_of(flags) == 0 || force) && (flags & (ODIT_LINEAR_FIRST | ODIT_LINEAR_NO_TILE)) == 0;
+  const bool choose = !force && launch != ODIT_LAUNCH_ANSWERED;
   float us[3] = {0.f, 0.f, 0.f};
   for (int i = 0; i < count; ++i) {
     const LinCall c{q[i].x, q[i].w, q[i].bias, nullptr, nullptr, q[i].out, q[i].M, N[i], K, q[i].ldx, q[i].ldw, q[i].ldo, 0,
@@ -739,12 +740,12 @@ static int lin_beside(const char* name, const odit_linear_problem* q, int count,
     if (lin_is_residual(c)) { set_error("%s: no residual", name); return ODIT_EINVAL; }
     g[i] = lin_gemm_call(c, 0, 0);
     if (!tile || (!force && q[i].M < kTileMinAuto) || !gemm_tile_takes(g[i], dtype)) return ODIT_ENOTSUP;
-    if (!force) us[i] = lin_call_us(dev, c, g[i], sk);
+    if (choose) us[i] = lin_call_us(dev, c, g[i], sk);
   }
   const int cus = device_cus();
   const TilePlan plan = plan_gemm_tile(g, count, cus, sk != nullptr);
   if (plan.bm == 0) return ODIT_ENOTSUP;
-  if (!force) {
+  if (choose) {
     float others = us[1] + us[2];
     if (count == 3) {
       const TilePlan two = plan_gemm_tile(g + 1, 2, cus, sk != nullptr);
@@ -752,14 +753,14 @@ static int lin_beside(const char* name, const odit_linear_problem* q, int count,
     }
     if (plan.us >= kOneLaunchGain * (us[0] + others)) return ODIT_ENOTSUP;
   }
-  return launch == 0 ? ODIT_OK : launch_gemm_tile(g, count, nullptr, dtype, sk, static_cast<hipStream_t>(stream));
+  return launch == ODIT_LAUNCH_ASK ? ODIT_OK : launch_gemm_tile(g, count, nullptr, dtype, sk, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int odit_linear_fork(const odit_linear_problem* q, const int* N, int K, const int* epilogue, int dtype, unsigned flags, void* workspace,
                                 size_t workspace_bytes, void* stream) {
   using namespace odit;
   ODIT_CHECK_ARG(q != nullptr && N != nullptr && epilogue != nullptr, "odit_linear_fork: null arguments");
-  return lin_beside("odit_linear_fork", q, 2, N, K, epilogue, dtype, flags, 1, false, workspace, workspace_bytes, stream);
+  return lin_beside("odit_linear_fork", q, 2, N, K, epilogue, dtype, flags, ODIT_LAUNCH_CHOOSE, false, workspace, workspace_bytes, stream);
 }
 
 extern "C" int odit_linear_three(const odit_linear_problem* q, const int* N, int K, const int* epilogue, int dtype, unsigned flags, int launch,
@@ -818,13 +819,15 @@ extern "C" int odit_linear_heads(const odit_linear_problem* q, const int* N, int
     g[i] = lin_gemm_call(c, 0, 0);
     if (!gemm_tile_takes(g[i], dtype) || (heads[i] != nullptr && !gemm_tile_heads_takes(g[i], h[i]))) return ODIT_ENOTSUP;
   }
-  if (engine == 2) return launch == 0 ? ODIT_OK : launch_gemm_tile_heads(g, 2, h, dtype, sk, static_cast<hipStream_t>(stream));
+  auto tile = [&] { return launch == ODIT_LAUNCH_ASK ? ODIT_OK : launch_gemm_tile_heads(g, 2, h, dtype, sk, static_cast<hipStream_t>(stream)); };
+  if (engine == 2) return tile();
   const int cus = device_cus();
   const bool pair = both && N[0] == N[1], streamk_takes = pair && gemm_streamk_takes(g[0], dtype) && gemm_streamk_takes(g[1], dtype);
   if (streamk_takes && gemm_small_rule(g, 2, cus, kSmallPairK)) {
     if (h[0].D != 64 || h[1].D != 64) return ODIT_ENOTSUP;  // (a tile of the small kernel is a head of 64 features)
-    return launch == 0 ? ODIT_OK : launch_gemm_small_heads(g, 2, h, dtype, static_cast<hipStream_t>(stream));
+    return launch == ODIT_LAUNCH_ASK ? ODIT_OK : launch_gemm_small_heads(g, 2, h, dtype, static_cast<hipStream_t>(stream));
   }
+  if (launch == ODIT_LAUNCH_ANSWERED) return tile();
   for (int i = 0; i < 2; ++i) apart += lin_call_us(dev, calls[i], g[i], sk);
   const TilePlan plan = plan_gemm_tile(g, 2, cus, sk != nullptr);
   if (plan.bm == 0) return ODIT_ENOTSUP;
@@ -840,8 +843,7 @@ extern "C" int odit_linear_heads(const odit_linear_problem* q, const int* N, int
     if (plan.us >= apart) apart -= (kColdTile - 1.f) * plan.us;
   }
   if (plan.us + end >= (plan.us < apart ? plan.us : apart) + pass) return ODIT_ENOTSUP;
-  if (launch == 0) return ODIT_OK;
-  return launch_gemm_tile_heads(g, 2, h, dtype, sk, static_cast<hipStream_t>(stream));
+  return tile();
 }
 
 // One projection of rows that lie in two tensors, in one reduction or as two products that add up, by expected time. One

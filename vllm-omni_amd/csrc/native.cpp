@@ -1048,8 +1048,8 @@ void project_fork(BlockCall& c, const void* x, const Lin l[2], void* const y[2],
   for (int i = 0; i < 2; ++i) c.project(x, l[i], y[i], M, gelu && i == 0);
 }
 
-// Three projections, of rows of their own, in one launch; launch false: whether they would. False, with nothing launched, where calls of
-// their own are the better way.
+// Three projections, of rows of their own, in one launch. launch false: whether that is expected to be the faster way (false: calls of
+// their own are); true: what has been answered so, and is not asked again: the block's memory is laid out by the answer.
 bool project_three(BlockCall& c, const void* const x[3], const Lin l[3], void* const y[3], const int64_t M[3], bool launch) {
   if (c.rc != 0) return true;
   if (l[0].k != l[1].k || l[0].k != l[2].k || (c.engine & ODIT_LINEAR_HANDWRITTEN)) return false;
@@ -1060,15 +1060,14 @@ bool project_three(BlockCall& c, const void* const x[3], const Lin l[3], void* c
     n[i] = static_cast<int>(l[i].n);
     epi[i] = l[i].b ? ODIT_EPI_BIAS : ODIT_EPI_NONE;
   }
-  const int rc = odit_linear_three(q, n, static_cast<int>(l[0].k), epi, c.dtype, c.engine, launch, c.lin_ws.p, c.lin_ws.bytes, c.where.stream);
+  const int rc = odit_linear_three(q, n, static_cast<int>(l[0].k), epi, c.dtype, c.engine, launch ? ODIT_LAUNCH_ANSWERED : ODIT_LAUNCH_ASK, c.lin_ws.p, c.lin_ws.bytes, c.where.stream);
   if (rc == ODIT_ENOTSUP && !launch) return false;
   c.check(rc);
   return true;
 }
 
 // Two projections of which one or both go to query, key and value heads, in one launch: heads[i].q null is an ordinary output y[i]
-// (GELU where `gelu`). launch false: whether they would. False, with nothing launched, where the projections and the pass behind
-// them are the better way.
+// (GELU where `gelu`). launch as above; false: the projections and the pass behind them are the better way.
 bool project_heads(BlockCall& c, const void* const x[2], const Lin l[2], void* const y[2], const int64_t M[2], const odit_head_output heads[2],
                    bool gelu, bool launch) {
   if (c.rc != 0) return true;
@@ -1082,7 +1081,7 @@ bool project_heads(BlockCall& c, const void* const x[2], const Lin l[2], void* c
     n[i] = static_cast<int>(l[i].n);
     epi[i] = !h[i] && gelu ? (l[i].b ? ODIT_EPI_BIAS_GELU_TANH : ODIT_EPI_GELU_TANH) : (l[i].b ? ODIT_EPI_BIAS : ODIT_EPI_NONE);
   }
-  const int rc = odit_linear_heads(q, n, static_cast<int>(l[0].k), epi, h, c.dtype, c.engine, launch, c.lin_ws.p, c.lin_ws.bytes, c.where.stream);
+  const int rc = odit_linear_heads(q, n, static_cast<int>(l[0].k), epi, h, c.dtype, c.engine, launch ? ODIT_LAUNCH_ANSWERED : ODIT_LAUNCH_ASK, c.lin_ws.p, c.lin_ws.bytes, c.where.stream);
   if (rc == ODIT_ENOTSUP && !launch) return false;
   c.check(rc);
   return true;
