@@ -26,8 +26,8 @@ if ROOT not in sys.path:
 PEAK_MFMA_BF16_TFLOPS = 2500.0   # MI355X dense bf16 MFMA, vendor figure
 PEAK_HBM_GBS = 8000.0            # MI355X HBM3E, vendor figure
 # HBM traffic, MFMA-busy share and in-kernel clock of the attention call come from the committed counter
-# summaries under profiles/ (vllm_omni_amd.profiling.attention_figures), which name the launches they were
-# measured on: a build that dispatches other launches for the headline shape makes bench.py stop.
+# summaries under profiles/ (vllm_omni_amd.profiling.attention_figures), which name the launches and the kernel
+# source they were measured on: for other launches or another source bench.py quotes none and says why ("stale").
 
 # Qwen-Image shape at 1024x1024, the headline workload
 LAYERS, HEADS, HEAD_DIM, MLP_RATIO = 60, 24, 128, 4
@@ -588,6 +588,7 @@ def kernel_rooflines(torch):
 def counter_probe(torch, kernels, dev):
     """Three launches of each kernel of the path at the headline shapes on N(0,1) data, nothing else: short
     enough for a hardware-counter pass (counters serialise the dispatches)."""
+    from vllm_omni_amd import profiling
     from vllm_omni_amd._lib import ODIT_NORM_HEAD
 
     bf = torch.bfloat16
@@ -626,7 +627,7 @@ def counter_probe(torch, kernels, dev):
     torch.cuda.synchronize()
     print(json.dumps({"probe": "attention, qknorm+rope, adaLN, gated residual, rel-L1, MLP-up GEMM (GELU epilogue), "
                                "QKV GEMM, text MLP-down GEMM (stream-K, gated residual) at the Qwen-Image shape, 3 launches each",
-                      "attention_plan": kernels.attn_plan(B, S, S, HEADS, HEAD_DIM),
+                      "attention_plan": kernels.attn_plan(B, S, S, HEADS, HEAD_DIM), "attention_source": profiling.attention_source(),
                       "text_mlp_down_flop": 2.0 * B * S_TXT * C * MLP_RATIO * C,
                       "attention_flop": 4.0 * B * HEADS * S * S * HEAD_DIM,
                       "mlp_up_flop": 2.0 * B * S_IMG * C * MLP_RATIO * C, "qkv_flop": 2.0 * B * S_IMG * C * 3 * C}))
@@ -750,7 +751,7 @@ def main():
     _lib.load()
     if not torch.cuda.is_available():
         sys.exit("bench.py needs a GPU")
-    from vllm_omni_amd import gemm_tuning
+    from vllm_omni_amd import gemm_tuning, profiling
 
     tuned = gemm_tuning.enable()  # hipBLASLt solution ids picked offline for this model's GEMM shapes
     kernels.set_linear_engine(args.linear_engine)
@@ -767,7 +768,7 @@ def main():
             dst.copy_(src)
         torch.cuda.synchronize()
         print(json.dumps({"probe": "attention B=2 S=4352 24x128 bf16 x4, copy 512 MiB x4",
-                          "attention_plan": kernels.attn_plan(B, S, S, HEADS, HEAD_DIM),
+                          "attention_plan": kernels.attn_plan(B, S, S, HEADS, HEAD_DIM), "attention_source": profiling.attention_source(),
                           "attention_min_bytes": 4 * q.numel() * 2, "copy_bytes_each_way": src.numel()}))
         return
     if args.counter_probe:
@@ -823,11 +824,9 @@ def main():
     S = S_IMG + S_TXT
     attn_flop = 4.0 * B * HEADS * S * S * HEAD_DIM
     attn_tflops = attn_flop / attn_ms / 1e9
-    from vllm_omni_amd import profiling
-
     plan = kernels.attn_plan(B, S, S, HEADS, HEAD_DIM)
     try:
-        prof = profiling.attention_figures(plan)
+        prof = profiling.attention_figures(plan, profiling.attention_source())
     except (RuntimeError, ValueError, OSError) as e:
         # the committed counter summaries were measured on other launches than this build makes: quote none
         prof = {"traffic_bytes": None, "mfma_busy_frac": None, "clock_MHz": None, "profiled_kernel": None,
@@ -864,7 +863,7 @@ def main():
                                   "kernel": prof["profiled_kernel"], "stale": prof.get("stale"),
                                   "source": "profiles/" + profiling.COUNTERS_FILE + " and profiles/" + profiling.TRAFFIC_FILE +
                                             " (rocprofv3 --pmc passes over bench.py --counter-probe / --traffic-probe, not live; "
-                                            "launch plan checked against this build)"},
+                                            "launch plan and kernel source checked against this build)"},
                      "launches_timed": n_attn, "avg_ms": attn_ms, "flop_per_launch": attn_flop},
         "step_flop": None,
     }

@@ -322,7 +322,7 @@ int odit_silu(const void* x, void* out, int64_t n, int dtype, void* stream);
  * Engines. hipBLASLt's MFMA kernels (a plain dense GEMM), set up so that bias, activation, gate and
  * residual ride in that kernel's epilogue, and three hand-written MFMA kernels, bf16 or fp16 (K a multiple of 64, N a
  * multiple of 8, 16-byte aligned rows): a stream-K kernel for few rows (csrc/gemm_bf16.hip) and a tile kernel for many
- * (csrc/gemm_bf16_tile.hip: 256 x 256 or 128 x 256 output tiles, the last round's cut along the reduction where they are
+ * (csrc/gemm_tile.h: 256 x 256 or 128 x 256 output tiles, the last round's cut along the reduction where they are
  * few), and one for products that are small altogether (csrc/gemm_small.hip: 64 x 64 tiles). All take one gate vector per
  * group of rows in a single launch (odit_linear_rows). Which runs: what a tuning call found, else for 48 to 1024 rows and K >= 2 N
  * (and N K >= 2^22) the stream-K kernel or, from 256 rows on, the tile kernel, by expected time, else the small kernel where

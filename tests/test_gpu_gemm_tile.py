@@ -1,4 +1,4 @@
-"""The tile kernel (csrc/gemm_bf16_tile.hip) where it can go wrong: whole tiles, tiles cut along the reduction into 2, 3 and 4
+"""The tile kernel (csrc/gemm_tile.h) where it can go wrong: whole tiles, tiles cut along the reduction into 2, 3 and 4
 parts, alone and behind whole rounds, ragged edges, two problems in one launch, ticket words left behind, graph replays.
 
 The reference is a float64 product. A result is one rounding of an fp32 sum: its relative error in the 2-norm is that of the

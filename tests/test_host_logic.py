@@ -1,6 +1,7 @@
 """Host-side logic of the product package against the oracle and against closed forms (CPU only)."""
 
 import math
+import re
 
 import numpy as np
 import pytest
@@ -681,6 +682,12 @@ def test_profile_records_name_the_launches_they_were_measured_on():
     assert "attn_fwd_dma_kernel" in fig["profiled_kernel"]
     with pytest.raises(RuntimeError, match="re-run the counter passes"):
         profiling.attention_figures(plan.replace("units=768", "units=769"))
+    # ... and on the kernel source they were measured on
+    source = traffic["attention_source"]
+    assert source == counters["attention_source"] and re.fullmatch("[0-9a-f]{16}", source) and re.fullmatch("[0-9a-f]{16}", profiling.attention_source())
+    assert profiling.attention_figures(plan, source) == fig
+    with pytest.raises(RuntimeError, match="another version of the attention kernels"):
+        profiling.attention_figures(plan, "0" * 16)
     assert profiling._plan_kernels(plan) == ["attn_fwd_dma_kernel<T, 128, 8, 0>", "attn_fwd_dma_kernel<T, 128, 8, 1>",
                                              "attn_merge_kernel<T, 128, 256>"]
     assert profiling._is_kernel("attn_merge_kernel<T, 128, 256>", "void odit::attn_merge_kernel<odit::bf16_t, 128, 256>(odit::AttnParams, int)")

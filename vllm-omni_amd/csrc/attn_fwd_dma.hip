@@ -22,8 +22,8 @@
 // excluded keys (mask_and_max). us, before / now, the same bits:
 //   D=128  B=1 S=16384 H=40  4645 / 4572 (on zeros, without the power limit, 3548 / 3430)    B=2 S=4352 H=24  439 / 432
 //          B=1 S=4608 H=24  248 / 243      B=1 S=1536 H=24  42.7 / 41.2
-//   D=64   B=2 S=4178 H=4  67.6 / 65.1     B=1 S=4096 H=8  55.5 / 52.1     B=1 S=8192 H=8  155 / 152     B=2 S=4352 H=24  278 / 268
-//          B=2 S=1357 H=32  48.6 / 46.6, padded row 42.1 / 39.0
+//   D=64 (with fills_two's rule)  B=2 S=4178 H=4  67.6 / 64.0     B=1 S=4096 H=8  55.6 / 51.2     B=1 S=8192 H=16  298 / 293
+//          B=2 S=4352 H=24  276 / 260     B=2 S=1357 H=32 f16 with a mask 53.8 / 42.4, padded row 42.0 / 34.2
 // v_mfma_f32_16x16x32 (two groups of 16 queries a wavefront) draws less power for the same products (a loop of nothing else: 2054
 // TFLOP/s on random operands, 32x32x16 1784; on zeros 2415 and 2440) and is twice as many instructions to issue. It took the first
 // launch to 4424 and zeros to 3869, but a video step of 32760 keys, whose probabilities are nearly even, to 0.997 of the time before
@@ -43,7 +43,7 @@
 // no mask / all-true mask, bytes / all-true mask, words:
 //   B=2 S=4352 H=24 D=128  439 / 737 / 451      B=1 S=4608 H=24 D=128  249 / 469 / 258
 //   B=2 S=592 H=24 D=128   18.4 / 26.8 / 18.8   B=2 S=4352 H=24 D=64   279 / 505 / 289
-// (and 490 / 290 / 20.6 / 333 with a random mask, where every tile is mixed).
+// (and 490 / 290 / 20.6 / 333 with a random mask, where every tile is mixed; at D=64 now 260 / - / 272).
 // Past kMaskWords tiles, and in the persistent form, whose units change the batch row, the word is formed at each tile, from one byte a lane.
 // With the words a unit ends with the last tile that has a live key: the tiles behind it would add zero probabilities (and are not
 // read: a NaN among their values does not reach the rows). Together with spread_batch below, one batch row padded to 40 % of
@@ -51,6 +51,7 @@
 // three drawn lengths of the second row the first shape takes 46 to 53):
 //   B=2 S=1357 H=32 (8 of keys) D=64  60.1 / 43.0, 56.0 / 56.2    B=2 S=1195 H=24 D=128  45.8 / 36.4, 46.1 / 45.4
 //   B=2 S=4352 H=24 D=64              320 / 296, 298 / 299        B=2 S=4352 H=24 D=128  485 / 468, 473 / 474
+// (at D=64 since then, three workgroups to a compute unit: 34, 42 and 270, 272)
 // Passing over the dead tiles between live ones too, by a list of the live ones, cost 1 to 2 % of every masked launch in the tile
 // loop, and skipping those ahead of the first live one 0.3 us of a second copy of the first scores.
 //
@@ -72,8 +73,8 @@
 // i.e. 3 to 5 % slower everywhere, also at 40 units per workgroup where the boundaries no longer matter: the
 // steady-state tile loop itself is slower. It carries the next unit's state and the boundary's branches in 97 of
 // 102 scalar registers, so the tile loads' LDS destinations and the fragment addresses are formed again in every
-// tile instead of being held: the hardware counters show 5.77 vector instructions per MFMA against 4.82 and the
-// matrix pipe busy 50.8 % of the cycles against 57.0 %. And what it saves is little: at 8 key tiles per unit, where
+// tile instead of being held: the hardware counters show 5.07 vector instructions per MFMA against 4.54 and the
+// matrix pipe busy 54.0 % of the cycles against 60.1 %. And what it saves is little: at 8 key tiles per unit, where
 // a unit's fixed cost (8 us: dispatch, cold first tiles, first scores, store) is a third of the unit, it runs in
 // the time of one workgroup per unit (899 / 901 us at 32760 queries x 512 keys x 40 heads), so its boundary costs
 // what a dispatch and a cold start cost. With a fixed assignment of units (w, w + W, ...) instead of the ticket

@@ -44,7 +44,7 @@ int device_cus();
 // expected time of the launch (us), 0 where the kernel has no plan for it
 float gemm_streamk_us(int M0, int M1, int N, int K, int cus);
 
-// ---- gemm_bf16_tile.hip: output tiles of 256 x 256 or 128 x 256, for many rows -------
+// ---- gemm_tile.h, gemm_bf16_tile.hip: output tiles of 256 x 256 or 128 x 256, for many rows -------
 // whether the kernel takes this problem (bf16 or fp16, K a multiple of 64, N of 8, 8 rows or more, 16-byte aligned rows,
 // operands addressable with 32-bit byte offsets)
 bool gemm_tile_takes(const GemmCall& c, int dtype);

@@ -1,6 +1,6 @@
 // The elementwise tail of the hand-written GEMM kernels: what happens to 8 consecutive output features of
 // one row on their way from the fp32 accumulators to memory (bias, GELU(tanh), gate, residual, rounding).
-// Shared by the stream-K kernel for few rows (gemm_bf16.hip) and the tile kernel for many (gemm_bf16_tile.hip).
+// Shared by the stream-K kernel for few rows (gemm_bf16.hip) and the tile kernel for many (gemm_tile.h).
 #pragma once
 
 #include "attn_common.h"

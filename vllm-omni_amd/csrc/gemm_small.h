@@ -11,7 +11,7 @@
 //
 // A wavefront owns 32 rows x 32 features as 2 x 2 accumulators of v_mfma_f32_16x16x32 with W rows as the A operand; the features
 // of the two accumulators interleave by 4, so that a lane ends up with 8 consecutive ones of a row. Chunks of 16 bytes are
-// XORed with bits of the row as in gemm_bf16_tile.hip. One barrier per step.
+// XORed with bits of the row as in gemm_tile.h. One barrier per step.
 #pragma once
 
 #include "gemm_epilogue.h"

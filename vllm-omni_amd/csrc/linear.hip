@@ -4,7 +4,7 @@
 //                                              gated-residual pass)
 // Which kernel runs is decided here per call. Few rows: the hand-written stream-K kernel (gemm_bf16.hip) where the reduction is
 // long, and a kernel for products that are small altogether (gemm_small.hip). Many rows: the hand-written tile kernel
-// (gemm_bf16_tile.hip) or hipBLASLt's MFMA kernels, by expected time. The two streams of a dual-stream block: one launch of a
+// (gemm_tile.h) or hipBLASLt's MFMA kernels, by expected time. The two streams of a dual-stream block: one launch of a
 // hand-written kernel, or two calls, by expected time (odit_linear_pair), with what follows a projection to heads at its end where
 // that is expected to be faster (odit_linear_heads). For the library this file sets the problem up so that
 // its epilogue does the elementwise work (bias vector, activation, a per-output-feature alpha vector for the gate, beta = 1 on the
@@ -772,8 +772,11 @@ extern "C" int odit_linear_three(const odit_linear_problem* q, const int* N, int
 
 // Projections to query, key and value heads with the heads' norm and rotation at the tile's end, or the projections and a pass over
 // their output, by expected time. The pass takes 6 us and 8 bytes for every feature of q at 5 TB/s; the tile's end 4.5 us more a round
-// on 256-row tiles and 1.3 on 128-row ones (its arithmetic has no matrix work to hide behind; beside GELU tiles, whose end is
-// as long, nothing): what would be one launch of the tile kernel anyway nearly always takes the pass with it. Kernel time in a
+// on 256-row tiles and 1.3 on 128-row ones (its arithmetic has no matrix work to hide behind). Beside a projection without heads nothing is
+// counted for it: a GELU tile's end is as long, and where the other has no GELU, as much is gained that is not counted either (charged for
+// the rounds of the heads' tiles, 19 of 2160 answers change, every one to the slower way. us with cold weights, apart / one launch: K=512, 2500
+// rows, N=6144 beside 4 heads of 64 53.0 / 48.2, 1800 rows, N=6144 beside 8 of 128 50.9 / 48.0; K=1024, 3000 rows, N=9216 beside 24 of 128
+// 155 / 138). What would be one launch of the tile kernel anyway nearly always takes the pass with it. Kernel time in a
 // model, us, projections + pass / one launch: 2048 + 342 rows, N=9216, K=3072 119 + 17 / 130; 1024 + 512 rows 73 + 11 / 79; 8192 + 512
 // rows 340 + 45 / 365; 1536 rows, N=12288 with GELU beside N=9216 153 + 10 / 157; 4608 rows 435 + 25 / 438. Few rows, where the
 // stream-K kernel takes the pair, stay there unless the tile kernel wins with its time of cold weights (kColdTile times the

@@ -1537,7 +1537,10 @@ PyObject* py_wan_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
   // summation is neither better nor worse: against a float32 model the guided noise of 16 batches is 2.03e-2 to 2.8e-2 off (bf16;
   // fp16 2.6e-3 to 3.5e-3) whichever kernels ran. But guidance (scale 5) multiplies the difference of the two rows, so two orders
   // are as far from each other, and results of earlier versions are reproduced. It costs 12 % at B=2 S=3536 and 0 to 7 %
-  // elsewhere; at S=3220 it gains 7 %.
+  // elsewhere; at S=3220 it gains 7 %. One video takes whatever is expected to be the fastest: its text's keys and values, in one
+  // launch with the queries' projection or in one of their own (project_three, by the number of rows of both), are summed as whole tiles or in up
+  // to four parts, so that their last bit can depend on the video's size. Whole tiles give the library's bits; against float64, 512 rows, both
+  // are 1.6537107e-3 off (bf16), 2.070324e-4 and 2.070321e-4 (fp16): the one rounding of the result.
   if (B > 1) c.engine |= ODIT_LINEAR_FIRST;
   if (B * S >= (1ll << 31) || S == 0 || T == 0 || (D != 64 && D != 128) || !c.operand(*ctx) || !ctx->is_contiguous() || ctx->size(0) != B || ctx->size(2) != C || HD != C) return none();
   const bool per_token = temb != nullptr;

@@ -2,8 +2,8 @@
 
 Every summary ends with one line ``bench.py reads: {...}`` (JSON): the figures ``bench.py`` quotes in its
 ``roofline`` object together with the attention launch plan (kernel names and unit counts, as
-``kernels.attn_plan`` reports them) that was profiled. ``bench.py`` compares that plan with the one the
-library dispatches now and refuses to quote figures measured on other kernels.
+``kernels.attn_plan`` reports them) that was profiled and a digest of the kernel's source. ``bench.py`` compares
+both with the library's and the tree's own and refuses to quote figures measured on other kernels.
 
     python -m vllm_omni_amd.profiling counters <dir of pass a> <dir of pass b> <probe stdout>
     python -m vllm_omni_amd.profiling traffic  <dir of FETCH_SIZE pass> <dir of WRITE_SIZE pass> <probe stdout>
@@ -17,8 +17,10 @@ from __future__ import annotations
 import collections
 import csv
 import glob
+import hashlib
 import json
 import os
+import re
 import sys
 from pathlib import Path
 
@@ -45,16 +47,29 @@ def read_record(name: str) -> dict:
     raise ValueError(f"{path} has no '{MARK.strip()}' line: re-create it with python -m vllm_omni_amd.profiling")
 
 
-def attention_figures(current_plan: str) -> dict:
+def attention_source() -> str:
+    """A digest of the attention kernels' source without its comments: two builds whose launch plans are the same text may
+    still run other code."""
+    csrc, h = Path(__file__).resolve().parent / "csrc", hashlib.sha256()
+    for name in ("attn_fwd_dma.hip", "attn_tail.h", "attn_common.h", "odit_common.h"):
+        for line in (csrc / name).read_text().splitlines():
+            h.update("".join(re.sub(r"//.*", "", line).split()).encode())
+    return h.hexdigest()[:16]
+
+
+def attention_figures(current_plan: str, source: str | None = None) -> dict:
     """HBM traffic, MFMA-busy share and in-kernel clock of the attention call at the headline shape from the
     committed counter summaries, after checking that they were measured on the launches ``current_plan``
-    names (``kernels.attn_plan`` of the headline shape)."""
+    names (``kernels.attn_plan`` of the headline shape) and, where given, on the code with this ``attention_source``."""
     traffic, counters = read_record(TRAFFIC_FILE), read_record(COUNTERS_FILE)
     for name, rec in ((TRAFFIC_FILE, traffic), (COUNTERS_FILE, counters)):
         if rec["attention_plan"] != current_plan:
             raise RuntimeError(
                 f"profiles/{name} was measured on the attention launches\n    {rec['attention_plan']}\n"
                 f"but this build dispatches\n    {current_plan}\nre-run the counter passes named at the top of that file")
+        if source is not None and rec.get("attention_source") != source:
+            raise RuntimeError(f"profiles/{name} was measured on another version of the attention kernels (source {rec.get('attention_source')}, "
+                               f"here {source}): re-run the counter passes named at the top of that file")
     return {"traffic_bytes": traffic["traffic_bytes"], "mfma_busy_frac": counters["mfma_busy_frac"],
             "clock_MHz": counters["clock_MHz"], "profiled_kernel": counters["main_kernel"]}
 
@@ -178,7 +193,7 @@ def summarise_counters(dir_a: str, dir_b: str, probe_stdout: str) -> str:
           "the 2.5 PFLOP/s peak assumes",
           f"#   ({100 * busy:.1f} % x {mhz:.0f}/2400 = {100 * busy * mhz / 2400:.1f} % of nominal peak for this launch). The library GEMMs run at the "
           "same reduced clock.",
-          MARK + json.dumps({"attention_plan": plan, "main_kernel": at, "mfma_busy_frac": round(busy, 4), "clock_MHz": round(mhz, 1)})]
+          MARK + json.dumps({"attention_plan": plan, "attention_source": probe["attention_source"], "main_kernel": at, "mfma_busy_frac": round(busy, 4), "clock_MHz": round(mhz, 1)})]
     text = "\n".join(L) + "\n"
     (PROFILES / COUNTERS_FILE).write_text(text)
     return text
@@ -208,7 +223,7 @@ def summarise_traffic(dir_fetch: str, dir_write: str, probe_stdout: str) -> str:
          f"bench.py --traffic-probe makes the attention call 4 times and a plain {copy_kib / 1024:.0f} MiB device-to-device copy 4 times",
          f"(known traffic: {copy_kib:.0f} KiB read, {copy_kib:.0f} KiB written), nothing else. Launch plan of one call at this shape:",
          f"  {plan}",
-         "(the units that fill whole rounds of the 512 workgroup slots, the left-over units cut into key ranges that write",
+         "(the units that fill whole rounds of workgroups, the left-over units cut into key ranges that write",
          "fp32 partial results, and the merge of those partials).",
          "",
          f"{'counter':12s} {'kernel':60s} per-dispatch readings (KiB as reported)"]
@@ -233,7 +248,7 @@ def summarise_traffic(dir_fetch: str, dir_write: str, probe_stdout: str) -> str:
           "that miss L2 (K and V of a head are re-read by the 34 query blocks of that head; the XCD-contiguous workgroup order",
           "keeps most of them in L2) and the key split (partials written and read back, K/V ranges read again). The call is",
           f"MFMA-bound: {both / 1e6:.0f} MB in about 0.455 ms is {both / 0.455e-3 / 1e12:.1f} TB/s, {100 * both / 0.455e-3 / 8e12:.0f} % of HBM peak.",
-          MARK + json.dumps({"attention_plan": plan, "traffic_bytes": round(both), "fetched_bytes": round(total["FETCH_SIZE"]),
+          MARK + json.dumps({"attention_plan": plan, "attention_source": probe["attention_source"], "traffic_bytes": round(both), "fetched_bytes": round(total["FETCH_SIZE"]),
                              "written_bytes": round(total["WRITE_SIZE"]), "scale_fetch": round(scale["FETCH_SIZE"], 4),
                              "scale_write": round(scale["WRITE_SIZE"], 4)})]
     text = "\n".join(L) + "\n"
