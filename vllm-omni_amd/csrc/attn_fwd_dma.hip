@@ -885,8 +885,9 @@ static int launch_dma(AttnParams& p, hipStream_t stream, void* ws, size_t ws_byt
   return check_launch("odit_attn_fwd (merge)");
 }
 
-// Wavefronts per workgroup: 4 (two workgroups per compute unit, each on its own) or 8 (one workgroup per compute unit
-// whose two halves run in anti-phase). Side by side in one process (bf16, us, 4 / 8 wavefronts; two boxes):
+// Wavefronts per workgroup: 4 (two workgroups per compute unit or, at head size 64, mostly three, each on its own) or 8 (one
+// workgroup per compute unit whose two halves run in anti-phase). Side by side in one process when the line was drawn (bf16, us, 4 / 8
+// wavefronts, two workgroups of 4 at either head size; two boxes):
 //   D=128  B=2 S=4352 H=24  514 / 491, 492 / 473     B=2 S=4096 H=24  429 / 420, 407 / 402
 //          B=1 S=4608 H=24  302 / 297, 289 / 288     B=2 S=32760 H=40  38910 / 38616, 37053 / 36483
 //   D=64   B=2 S=4352 H=24  326 / 334, 316 / 328
@@ -898,6 +899,10 @@ static int launch_dma(AttnParams& p, hipStream_t stream, void* ws, size_t ws_byt
 // 32760 queries x 512 keys x 40 heads, 901 / 947). (With the two halves' roles paired wrongly, wavefronts w and
 // w + 1 or w and w + 2 in anti-phase instead of w and w + 4, the same kernel is 10 to 18 % slower: two wavefronts of a
 // SIMD in the same stage is what costs, and independent workgroups already avoid it most of the time by themselves.)
+// Since the softmax's vector work was cut the two are closer, 4 wavefronts ahead in the middle and 8 at many keys (D=128, us, 4 / 8, the
+// same bits): B=1 S=2048 H=24 56.6 / 56.2, B=2 S=2390 H=24 138.6 / 144.5, B=2 S=3276 H=40 417 / 427, B=1 S=4608 H=24 242.7 / 241.2, B=2 S=4352
+// H=24 423 / 427, with a mask 460 / 458, B=2 S=6032 H=24 797 / 818, B=1 S=8192 H=24 696 / 692, B=1 S=16384 H=40 4565 / 4500, B=2 S=32760 H=40
+// 36223 / 35657; 16384 queries x 2048 keys x 40 heads 620 / 638. The line stays where it was drawn.
 // ODIT_ATTN_WAVES in the environment, read at the first attention launch, overrides the choice (for measurements).
 static int dma_waves(int D, int Sk) {
   static const int forced = [] {
