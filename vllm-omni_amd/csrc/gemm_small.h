@@ -1,5 +1,5 @@
 // 16-bit GEMM y = x W^T for products that are small altogether (models of a few hundred channels), one problem or two of the same
-// N and K in one launch: one 64 x 64 output tile per workgroup of 4 wavefronts, no reduction is divided.
+// N and K in one launch: one 64 x 64 output tile per workgroup of 8 wavefronts, no reduction is divided.
 //
 // What bounds it: latency. A launch of some dozens of workgroups is one chain of arguments, first loads, matrix work, epilogue
 // operands and stores; at these sizes the work itself takes a microsecond. So everything that does not depend on the product is
@@ -9,7 +9,12 @@
 // hand-over there. us, stream-K / this kernel: M=256+64, K=256: N=768 13.7 / 5.3, N=256 13.0 / 4.5, N=1024 with GELU 14.9 / 5.9;
 // N=256, K=1024 21.5 / 7.8. One problem, the library / this kernel: M=64, N=256, K=256 9.0 / 5.2.
 //
-// A wavefront owns 32 rows x 32 features as 2 x 2 accumulators of v_mfma_f32_16x16x32 with W rows as the A operand; the features
+// Two wavefronts to a SIMD, which issue while the other one waits: a wavefront alone issues a vector instruction every 7 to 8 cycles, and
+// addresses, first fragments and the epilogue's arithmetic are in the chain. us a launch in a row, 4 wavefronts (32 x 32 outputs each) / 8, the
+// same bits: M=64 N=64 K=256 4.06 / 3.41; M=128 N=768 K=256 4.31 / 3.64; M=320 N=1024 K=256 with GELU 4.95 / 3.92; M=1024 N=1024 K=1024 with
+// GELU 8.35 / 7.26; 1024 tiles of K=64 5.81 / 5.69, of K=128 with GELU 7.44 / 6.66; 512 of K=256 5.50 / 5.02.
+//
+// A wavefront owns 16 rows x 32 features as two accumulators of v_mfma_f32_16x16x32 with W rows as the A operand; the features
 // of the two accumulators interleave by 4, so that a lane ends up with 8 consecutive ones of a row. Chunks of 16 bytes are
 // XORed with bits of the row as in gemm_tile.h. One barrier per step.
 #pragma once
@@ -21,7 +26,7 @@ namespace odit {
 
 namespace {
 
-constexpr int kSmallTile = 64, kSmallStages = 8, kSmallPiece = kSmallTile * kGemmBK * 2, kSmallStage = 2 * kSmallPiece;
+constexpr int kSmallWaves = 8, kSmallTile = 64, kSmallStages = 8, kSmallPiece = kSmallTile * kGemmBK * 2, kSmallStage = 2 * kSmallPiece;
 
 struct SmallProblem {
   const void *x, *w;
@@ -47,14 +52,14 @@ typedef __attribute__((address_space(3))) void* lds_void_p;
 // S: stages (as many as there are steps where those are fewer than 8: several workgroups to a CU)
 // HEADS: query, key and value heads of 64 features (gemm_heads.h), a tile each
 template <typename T, int S, bool HEADS>
-__global__ __launch_bounds__(256) void gemm_small_kernel(const SmallArgs<HEADS> p) {
+__global__ __launch_bounds__(64 * kSmallWaves) void gemm_small_kernel(const SmallArgs<HEADS> p) {
   using M = Mma16<T>;
   using frag = typename M::frag;
   __shared__ __attribute__((aligned(1024))) char lds[S * kSmallStage];
   __shared__ float squares[HEADS ? kSmallTile * 2 : 1];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave & 1, wn = wave >> 1;
+  const int wm = wave & 3, wn = wave >> 2;
   const int l16 = lane & 15, lq = lane >> 4;
   const int which = static_cast<int>(blockIdx.x) >= p.tiles0 ? 1 : 0;
   const SmallProblem& q = p.q[which];
@@ -74,36 +79,30 @@ __global__ __launch_bounds__(256) void gemm_small_kernel(const SmallArgs<HEADS> 
   };
   const u32x4_v xr = make_rsrc(q.x, q.x_bytes), wr = make_rsrc(q.w, q.w_bytes);
 
-  // instruction j of this wavefront's share of a piece fills rows 16 wave + 8 j .. + 7; rows past the end re-read the last one
-  uint32_t vx[2], vw[2];
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int r = wave * 16 + j * 8 + (lane >> 3), ch = lane & 7;
-    const int rx = m0 + r < q.M ? m0 + r : q.M - 1, rw = n0 + r < p.N ? n0 + r : p.N - 1;
-    vx[j] = static_cast<uint32_t>(rx) * q.ldx + static_cast<uint32_t>((ch ^ ((r >> 1) & 7)) << 4);
-    vw[j] = static_cast<uint32_t>(rw) * q.ldw + static_cast<uint32_t>((ch ^ (((r >> 1) & 1) | (((r >> 3) & 3) << 1))) << 4);
-  }
-  const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void_p)lds)) + wave * 2048;
+  // this wavefront's share of a piece is rows 8 wave .. + 7, one instruction; rows past the end re-read the last one
+  const int r = wave * 8 + (lane >> 3), ch = lane & 7;
+  const int rx = m0 + r < q.M ? m0 + r : q.M - 1, rw = n0 + r < p.N ? n0 + r : p.N - 1;
+  const uint32_t vx = static_cast<uint32_t>(rx) * q.ldx + static_cast<uint32_t>((ch ^ ((r >> 1) & 7)) << 4);
+  const uint32_t vw = static_cast<uint32_t>(rw) * q.ldw + static_cast<uint32_t>((ch ^ (((r >> 1) & 1) | (((r >> 3) & 3) << 1))) << 4);
+  const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void_p)lds)) + wave * 1024;
   auto load = [&](uint32_t dst, uint32_t off, u32x4_v rs, int soff) {
     load_lds16(__builtin_amdgcn_readfirstlane(dst), off, rs, __builtin_amdgcn_readfirstlane(soff));
   };
   auto issue = [&](int i, int stage) {
     const uint32_t d = lds0 + stage * kSmallStage;
     const int k = i * (kGemmBK * 2);
-    load(d, vx[0], xr, k);
-    load(d + 1024, vx[1], xr, k);
-    load(d + kSmallPiece, vw[0], wr, k);
-    load(d + kSmallPiece + 1024, vw[1], wr, k);
+    load(d, vx, xr, k);
+    load(d + kSmallPiece, vw, wr, k);
   };
 
-  // operands of the epilogue: rows m, m + 16, features n .. n + 7
+  // operands of the epilogue: row m, features n .. n + 7
   const GemmEpilogue& e = q.ep;
-  const int m = m0 + wm * 32 + l16, n = n0 + wn * 32 + lq * 8;
+  const int m = m0 + wm * 16 + l16, n = n0 + wn * 32 + lq * 8;
   const bool gated = e.epilogue == ODIT_EPI_GATED_RESIDUAL || e.epilogue == ODIT_EPI_GATED_RESIDUAL_PRE;
   const bool gelu = e.epilogue == ODIT_EPI_GELU_TANH || e.epilogue == ODIT_EPI_BIAS_GELU_TANH;
-  float gt[2][8], bs[2][8];
-  u32x4 res[2] = {};
-  HeadRows<2> rows;
+  float gt[8], bs[8];
+  u32x4 res = {};
+  HeadRows<1> rows;
   u32x4 bias = {0u, 0u, 0u, 0u}, weight = bias;
   int third = 0;
   if constexpr (HEADS) {
@@ -111,68 +110,56 @@ __global__ __launch_bounds__(256) void gemm_small_kernel(const SmallArgs<HEADS> 
     third = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(n0) / static_cast<unsigned>(h.HD));
     if (e.bias != nullptr) bias = load_raw(static_cast<const T*>(e.bias) + n);
     if (third < 2) weight = load_raw(static_cast<const T*>(third == 0 ? h.wq : h.wk) + (n - n0));
-    rows.ask(h, q.M, m0, wm * 32 + l16, n - n0);
+    rows.ask(h, q.M, m0, wm * 16 + l16, n - n0);
   } else {
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int row = m + 16 * i < q.M ? m + 16 * i : q.M - 1, col = n < p.N ? n : 0;
-      gemm_epilogue_vectors8<T>(e, row, col, gt[i], bs[i]);
-      if (gated) res[i] = load_raw(static_cast<const T*>(e.residual) + row * e.ldr + col);
-    }
+    const int row = m < q.M ? m : q.M - 1, col = n < p.N ? n : 0;
+    gemm_epilogue_vectors8<T>(e, row, col, gt, bs);
+    if (gated) res = load_raw(static_cast<const T*>(e.residual) + row * e.ldr + col);
   }
 #pragma unroll
   for (int d = 0; d < S; ++d)
     if (d < nk) issue(d, d);
 
-  const int xrow = wm * 32 + l16;
+  const int xrow = wm * 16 + l16;
   const int xa = xrow * 128 + ((lq ^ ((xrow >> 1) & 7)) << 4);
   const int wrow = wn * 32 + ((l16 >> 2) << 3) + (l16 & 3);
   const int wa = kSmallPiece + wrow * 128 + ((lq ^ (((wrow >> 1) & 1) | (((wrow >> 3) & 3) << 1))) << 4);
-  f32x4_v acc[2][2];
-#pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int b = 0; b < 2; ++b) acc[a][b] = f32x4_v{0.f, 0.f, 0.f, 0.f};
+  f32x4_v acc[2] = {f32x4_v{0.f, 0.f, 0.f, 0.f}, f32x4_v{0.f, 0.f, 0.f, 0.f}};
   for (int i = 0; i < nk; ++i) {
     // this wavefront's loads of step i have landed and its reads of step i - 1 are in registers; behind the barrier that holds for
     // every wavefront, and the stage of step i - 1 is free
-    if (S == kSmallStages && i + S - 2 < nk) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((kSmallStages - 2) * 4) : "memory");
+    if (S == kSmallStages && i + S - 2 < nk) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((kSmallStages - 2) * 2) : "memory");
     else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     if (S == kSmallStages && i > 0 && i - 1 + S < nk) issue(i - 1 + S, (i - 1) % S);
     const char* st = lds + (i % S) * kSmallStage;
-    frag xf[2][2], wf[2][2];
+    frag xf[2], wf[2][2];
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      xf[ks] = __builtin_bit_cast(frag, *reinterpret_cast<const u32x4_v*>(st + (xa ^ (ks * 64))));
+#pragma unroll
+      for (int b = 0; b < 2; ++b) wf[ks][b] = __builtin_bit_cast(frag, *reinterpret_cast<const u32x4_v*>(st + (wa ^ (ks * 64)) + b * 512));
+    }
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-      for (int a = 0; a < 2; ++a) {
-        xf[ks][a] = __builtin_bit_cast(frag, *reinterpret_cast<const u32x4_v*>(st + (xa ^ (ks * 64)) + a * 2048));
-        wf[ks][a] = __builtin_bit_cast(frag, *reinterpret_cast<const u32x4_v*>(st + (wa ^ (ks * 64)) + a * 512));
-      }
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-      for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b) acc[a][b] = M::run(wf[ks][b], xf[ks][a], acc[a][b]);
+      for (int b = 0; b < 2; ++b) acc[b] = M::run(wf[ks][b], xf[ks], acc[b]);
   }
 
   if constexpr (HEADS) {
     const HeadsOut& h = p.heads[which];
-    u32x4 x[2];
+    const int r = wm * 16 + l16;
+    u32x4 x;
+    float s = 0.f;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      float s = 0.f;
+    for (int u = 0; u < 4; ++u)
+      Raw<T>::set2(x, u, acc[u / 2][2 * (u % 2)] + Raw<T>::get(bias, 2 * u), acc[u / 2][2 * (u % 2) + 1] + Raw<T>::get(bias, 2 * u + 1));
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
-        Raw<T>::set2(x[i], u, acc[i][u / 2][2 * (u % 2)] + Raw<T>::get(bias, 2 * u), acc[i][u / 2][2 * (u % 2) + 1] + Raw<T>::get(bias, 2 * u + 1));
-#pragma unroll
-      for (int u = 0; u < 8; ++u) s = fmaf(Raw<T>::get(x[i], u), Raw<T>::get(x[i], u), s);
-      s = add_swapped(s, __builtin_amdgcn_permlane16_swap(__float_as_uint(s), __float_as_uint(s), false, false));
-      s = add_swapped(s, __builtin_amdgcn_permlane32_swap(__float_as_uint(s), __float_as_uint(s), false, false));
-      squares[(wm * 32 + l16 + 16 * i) * 2 + wn] = s;  // (the same from four lanes)
-    }
+    for (int u = 0; u < 8; ++u) s = fmaf(Raw<T>::get(x, u), Raw<T>::get(x, u), s);
+    s = add_swapped(s, __builtin_amdgcn_permlane16_swap(__float_as_uint(s), __float_as_uint(s), false, false));
+    s = add_swapped(s, __builtin_amdgcn_permlane32_swap(__float_as_uint(s), __float_as_uint(s), false, false));
+    squares[r * 2 + wn] = s;  // (the same from four lanes)
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
@@ -181,40 +168,28 @@ __global__ __launch_bounds__(256) void gemm_small_kernel(const SmallArgs<HEADS> 
     asm("" : "+s"(qo), "+s"(ko), "+s"(vo));  // (values of their own: the choice by `third` would be an index into a copy of them in memory)
 #endif
     T* const out = static_cast<T*>(third == 0 ? qo : third == 1 ? ko : vo) + (n - third * h.HD);
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int r = wm * 32 + l16 + 16 * i;
-      if (third < 2) {
-        const float rstd = rsqrtf((squares[r * 2] + squares[r * 2 + 1]) * (1.f / 64) + h.eps);
-        x[i] = turn_head<T>(x[i], rstd, weight, rows.cos[i], rows.sin[i]);
-      }
-      if (rows.at[i] >= 0) store_raw(out + static_cast<int64_t>(rows.at[i]) * h.HD, x[i]);
+    if (third < 2) {
+      const float rstd = rsqrtf((squares[r * 2] + squares[r * 2 + 1]) * (1.f / 64) + h.eps);
+      x = turn_head<T>(x, rstd, weight, rows.cos[0], rows.sin[0]);
     }
+    if (rows.at[0] >= 0) store_raw(out + static_cast<int64_t>(rows.at[0]) * h.HD, x);
     return;
   }
+  if (m >= q.M || n >= p.N) return;
+  u32x4 o;
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    if (m + 16 * i >= q.M || n >= p.N) continue;
-    float y[8];
+  for (int u = 0; u < 4; ++u) {
+    float y[2];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      y[u] = acc[i][0][u];
-      y[4 + u] = acc[i][1][u];
+    for (int t = 0; t < 2; ++t) {
+      const int f = 2 * u + t;
+      const float a = acc[f / 4][f % 4];
+      y[t] = gated ? fmaf(gt[f], a, bs[f]) + Raw<T>::get(res, f) : a + bs[f];
+      if (!gated && gelu) y[t] = gemm_gelu_tanh(y[t]);
     }
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      if (gated) {
-        y[u] = fmaf(gt[i][u], y[u], bs[i][u]) + Raw<T>::get(res[i], u);
-      } else {
-        y[u] += bs[i][u];
-        if (gelu) y[u] = gemm_gelu_tanh(y[u]);
-      }
-    }
-    u32x4 o;
-#pragma unroll
-    for (int u = 0; u < 4; ++u) Raw<T>::set2(o, u, y[2 * u], y[2 * u + 1]);
-    store_raw(static_cast<T*>(e.out) + (m + 16 * i) * e.ldo + n, o);
+    Raw<T>::set2(o, u, y[0], y[1]);
   }
+  store_raw(static_cast<T*>(e.out) + m * e.ldo + n, o);
 }
 
 inline void fill_small_params(SmallParams& p, const GemmCall* c, int count, int (&tiles)[2]) {

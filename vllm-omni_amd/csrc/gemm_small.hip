@@ -13,7 +13,7 @@ bool gemm_small_rule(const GemmCall* c, int count, int cus, int max_k) {
   int64_t tiles = 0;
   for (int i = 0; i < count; ++i)
     tiles += static_cast<int64_t>((c[i].M + kSmallTile - 1) / kSmallTile) * ((c[i].N + kSmallTile - 1) / kSmallTile);
-  const int per_cu = nk > 4 ? 1 : (nk > 2 ? 2 : 4);  // 160 KB of LDS, and no more than 16 wavefronts
+  const int per_cu = nk > 4 ? 1 : (nk > 2 ? 2 : 4);  // 160 KB of LDS, and 32 wavefronts
   return tiles <= static_cast<int64_t>(cus) * per_cu;
 }
 
@@ -21,7 +21,7 @@ int launch_gemm_small(const GemmCall* c, int count, int dtype, hipStream_t strea
   SmallArgs<false> p;
   int tiles[2] = {0, 0};
   fill_small_params(p, c, count, tiles);
-  const dim3 grid(tiles[0] + tiles[1]), block(256);
+  const dim3 grid(tiles[0] + tiles[1]), block(64 * kSmallWaves);
 #define ODIT_SMALL(T)                                                                                                    \
   do {                                                                                                                   \
     if (p.k_steps == 1) hipLaunchKernelGGL((gemm_small_kernel<T, 1, false>), grid, block, 0, stream, p);                         \

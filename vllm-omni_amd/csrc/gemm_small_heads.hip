@@ -11,7 +11,7 @@ int launch_gemm_small_heads(const GemmCall* c, int count, const HeadsOut* heads,
     p.heads[i] = heads[i < count ? i : 0];
     fill_heads_division(p.heads[i]);
   }
-  const dim3 grid(tiles[0] + tiles[1]), block(256);
+  const dim3 grid(tiles[0] + tiles[1]), block(64 * kSmallWaves);
 #define ODIT_SMALL(T)                                                                                                     \
   do {                                                                                                                    \
     if (p.k_steps == 1) hipLaunchKernelGGL((gemm_small_kernel<T, 1, true>), grid, block, 0, stream, p);                    \
