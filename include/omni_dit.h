@@ -458,6 +458,22 @@ int odit_linear_heads(const odit_linear_problem problems[2], const int N[2], int
                       const odit_head_output* const heads[2], int dtype, unsigned flags, int launch, void* workspace,
                       size_t workspace_bytes, void* stream);
 
+/* odit_linear_pair, or with `heads` odit_linear_heads of two, of rows that are normed and modulated on the way: x' = LayerNorm(x) (1 + scale) +
+ * shift as odit_adaln_modulate makes it of x [M, K] (the same bits), without that launch and its output. norm[i]: shift and scale rows of `dtype`
+ * (16-byte aligned, K elements), `stride` elements apart, one for S consecutive rows of x: img_norm1 / txt_norm1 with to_qkv / add_kv_proj, img_norm2 /
+ * txt_norm2 with the up projections (qwen_image_transformer.py:764-812) of a small model. ODIT_ENOTSUP, with nothing launched, where the kernel
+ * for small products is not the one for the pair, K is more than 256 or an operand is not of that form; the caller then makes the calls one by one.
+ * launch: ODIT_LAUNCH_. Needs no workspace. */
+typedef struct odit_row_norm {
+  const void *shift, *scale;
+  int64_t stride;
+  int S;
+  float eps;
+} odit_row_norm;
+
+int odit_linear_pair_norm(const odit_linear_problem problems[2], const odit_row_norm norm[2], int N, int K, int epilogue,
+                          const odit_head_output* const heads[2], int dtype, unsigned flags, int launch, void* stream);
+
 /* odit_linear_rows of rows that lie in two tensors, x [M,K] beside x2 [M,K2] (W is [N, K + K2]), as one reduction in one launch
  * of the tile kernel: proj_out of a single-stream block without the concatenation (flux_transformer.py:303-309).
  * ODIT_ENOTSUP, with nothing launched, where two calls that add up are the better way. */

@@ -113,6 +113,8 @@ _SIGNATURES = {
     "odit_linear_heads": (
         C.c_int, [C.c_void_p, C.POINTER(C.c_int), C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_void_p), C.c_int, C.c_uint, C.c_int, C.c_void_p,
                   C.c_size_t, C.c_void_p]),
+    "odit_linear_pair_norm": (
+        C.c_int, [C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_int, C.POINTER(C.c_void_p), C.c_int, C.c_uint, C.c_int, C.c_void_p]),
     "odit_linear_join": (
         C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_int,
                   C.c_int64, C.c_int64, C.c_int64, C.c_int64, C.c_int64, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int64, C.c_uint,
@@ -166,6 +168,12 @@ class HeadOutput(C.Structure):
 
     _fields_ = [(n, C.c_void_p) for n in ("q", "k", "v", "wq", "wk", "cos", "sin")] + [
         (n, C.c_int) for n in ("S", "offset", "S_total", "H", "D")] + [("eps", C.c_float)]
+
+
+class RowNorm(C.Structure):
+    """``odit_row_norm``"""
+
+    _fields_ = [("shift", C.c_void_p), ("scale", C.c_void_p), ("stride", C.c_int64), ("S", C.c_int), ("eps", C.c_float)]
 
 
 class OmniDitLibraryError(RuntimeError):

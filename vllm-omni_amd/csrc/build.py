@@ -50,6 +50,7 @@ UNITS: list[tuple[str, list[str], str]] = [
     ("gemm_tile_heads.hip", [], "gemm_tile_heads"),
     ("gemm_small.hip", [], "gemm_small"),
     ("gemm_small_heads.hip", [], "gemm_small_heads"),
+    ("gemm_small_norm.hip", [], "gemm_small_norm"),
 ]
 PROBE_UNITS: list[tuple[str, list[str], str]] = [("probe.hip", [], "probe")]
 

@@ -90,6 +90,16 @@ int launch_gemm_tile_heads(const GemmCall* c, int count, const HeadsOut* heads, 
 // One problem, or two of the same N and K in one launch, which gemm_streamk_takes takes. No scratch.
 bool gemm_small_rule(const GemmCall* c, int count, int cus, int max_k);
 int launch_gemm_small(const GemmCall* c, int count, int dtype, hipStream_t stream);
+// LayerNorm without affine and modulation of a problem's rows, x' = norm(x) (1 + scale) + shift, in front of the product: shift and scale of
+// the tensors' type, one row for S rows of x, `stride` elements apart. For two problems of K <= kSmallNormK.
+struct RowNorm {
+  const void *shift, *scale;
+  int64_t stride;
+  int S;
+  float eps;
+};
+constexpr int kSmallNormK = 256;
+int launch_gemm_small_norm(const GemmCall* c, const RowNorm* norm, const HeadsOut* heads, int dtype, hipStream_t stream);
 // the same with query, key and value heads of 64 features (gemm_small_heads.hip)
 int launch_gemm_small_heads(const GemmCall* c, int count, const HeadsOut* heads, int dtype, hipStream_t stream);
 

@@ -17,6 +17,11 @@
 // A wavefront owns 16 rows x 32 features as two accumulators of v_mfma_f32_16x16x32 with W rows as the A operand; the features
 // of the two accumulators interleave by 4, so that a lane ends up with 8 consecutive ones of a row. Chunks of 16 bytes are
 // XORed with bits of the row as in gemm_tile.h. One barrier per step.
+//
+// NORM: the rows are normed and modulated on the way (adaln_rows_kernel's operations, its bits), for reductions whose steps are all in LDS
+// at once. A launch of that kernel in front is 2.3 to 2.5 us one after the other, for a microsecond of work that every workgroup can do for
+// the 64 rows it reads anyway (1.7 us more of a launch): each wavefront norms the 8 rows that it has fetched itself, eight lanes to a
+// row, so nothing is waited for that was not before.
 #pragma once
 
 #include "gemm_epilogue.h"
@@ -42,17 +47,79 @@ struct SmallParams {
   int tiles0;  // of the first problem
 };
 
-template <bool HEADS> struct SmallArgs : SmallParams {};
-template <> struct SmallArgs<true> : SmallParams {
+template <bool HEADS> struct SmallHeads : SmallParams {};
+template <> struct SmallHeads<true> : SmallParams {
   HeadsOut heads[2];  // of 64 features: a tile is one head
+};
+template <bool HEADS, bool NORM> struct SmallArgs : SmallHeads<HEADS> {};
+template <bool HEADS> struct SmallArgs<HEADS, true> : SmallHeads<HEADS> {
+  RowNorm norm[2];
 };
 
 typedef __attribute__((address_space(3))) void* lds_void_p;
 
+// The wavefront's 8 rows of the tile, whose pieces it has asked for: LayerNorm and modulation in place. `ask` asks for what comes behind
+// them. Lane l works on row l / 8, chunk l % 8 of every step: the sums over a row go chunk by chunk, over the 8 lanes, by twos of steps, and up
+// from there: the order of adaln_rows_kernel's wavefront with a chunk to a lane.
+template <typename T, int S, typename Ask>
+__device__ __forceinline__ void norm_rows(const RowNorm& nm, char* lds, int m0, int M, int nk, int wave, int lane, Ask&& ask) {
+  const int r = wave * 8 + (lane >> 3), j = lane & 7, C = nk * kGemmBK;
+  const int m = m0 + r < M ? m0 + r : M - 1;
+  const int64_t at = static_cast<int64_t>(static_cast<unsigned>(m) / static_cast<unsigned>(nm.S)) * nm.stride + j * 8;
+  u32x4 scale[S], shift[S], raw[S];
+#pragma unroll
+  for (int i = 0; i < S; ++i)
+    if (i < nk) {
+      scale[i] = load_raw(static_cast<const T*>(nm.scale) + at + i * kGemmBK);
+      shift[i] = load_raw(static_cast<const T*>(nm.shift) + at + i * kGemmBK);
+    }
+  ask();
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  const int turn = (r >> 1) & 7;
+  auto chunk = [&](int i) { return lds + i * kSmallStage + r * 128 + ((j ^ turn) << 4); };
+  const float k0 = to_float(*reinterpret_cast<const T*>(lds + r * 128 + (turn << 4)));
+  float s1[S], s2[S];
+#pragma unroll
+  for (int i = 0; i < S; ++i) {
+    s1[i] = s2[i] = 0.f;
+    if (i < nk) {
+      raw[i] = *reinterpret_cast<const u32x4*>(chunk(i));
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const float d = Raw<T>::get(raw[i], u) - k0;
+        s1[i] += d;
+        s2[i] = fmaf(d, d, s2[i]);
+      }
+      s1[i] = row_group_sum<8>(s1[i]);
+      s2[i] = row_group_sum<8>(s2[i]);
+    }
+  }
+  float a1 = 0.f, a2 = 0.f;
+#pragma unroll
+  for (int i = 0; i < S; i += 2) {
+    a1 += s1[i] + (i + 1 < S ? s1[i + 1 < S ? i + 1 : i] : 0.f);
+    a2 += s2[i] + (i + 1 < S ? s2[i + 1 < S ? i + 1 : i] : 0.f);
+  }
+  const float inv_c = 1.f / static_cast<float>(C);
+  const float m1 = a1 * inv_c;
+  const float mean = k0 + m1;
+  const float rstd = rsqrtf(fmaxf(a2 * inv_c - m1 * m1, 0.f) + nm.eps);
+#pragma unroll
+  for (int i = 0; i < S; ++i)
+    if (i < nk) {
+      u32x4 o;
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        Raw<T>::set2(o, u, fmaf((Raw<T>::get(raw[i], 2 * u) - mean) * rstd, 1.f + Raw<T>::get(scale[i], 2 * u), Raw<T>::get(shift[i], 2 * u)),
+                     fmaf((Raw<T>::get(raw[i], 2 * u + 1) - mean) * rstd, 1.f + Raw<T>::get(scale[i], 2 * u + 1), Raw<T>::get(shift[i], 2 * u + 1)));
+      *reinterpret_cast<u32x4*>(chunk(i)) = o;
+    }
+}
+
 // S: stages (as many as there are steps where those are fewer than 8: several workgroups to a CU)
 // HEADS: query, key and value heads of 64 features (gemm_heads.h), a tile each
-template <typename T, int S, bool HEADS>
-__global__ __launch_bounds__(64 * kSmallWaves) void gemm_small_kernel(const SmallArgs<HEADS> p) {
+template <typename T, int S, bool HEADS, bool NORM>
+__global__ __launch_bounds__(64 * kSmallWaves) void gemm_small_kernel(const SmallArgs<HEADS, NORM> p) {
   using M = Mma16<T>;
   using frag = typename M::frag;
   __shared__ __attribute__((aligned(1024))) char lds[S * kSmallStage];
@@ -88,11 +155,11 @@ __global__ __launch_bounds__(64 * kSmallWaves) void gemm_small_kernel(const Smal
   auto load = [&](uint32_t dst, uint32_t off, u32x4_v rs, int soff) {
     load_lds16(__builtin_amdgcn_readfirstlane(dst), off, rs, __builtin_amdgcn_readfirstlane(soff));
   };
+  auto issue_x = [&](int i, int stage) { load(lds0 + stage * kSmallStage, vx, xr, i * (kGemmBK * 2)); };
+  auto issue_w = [&](int i, int stage) { load(lds0 + stage * kSmallStage + kSmallPiece, vw, wr, i * (kGemmBK * 2)); };
   auto issue = [&](int i, int stage) {
-    const uint32_t d = lds0 + stage * kSmallStage;
-    const int k = i * (kGemmBK * 2);
-    load(d, vx, xr, k);
-    load(d + kSmallPiece, vw, wr, k);
+    issue_x(i, stage);
+    issue_w(i, stage);
   };
 
   // operands of the epilogue: row m, features n .. n + 7
@@ -116,9 +183,20 @@ __global__ __launch_bounds__(64 * kSmallWaves) void gemm_small_kernel(const Smal
     gemm_epilogue_vectors8<T>(e, row, col, gt, bs);
     if (gated) res = load_raw(static_cast<const T*>(e.residual) + row * e.ldr + col);
   }
+  if constexpr (NORM) {
 #pragma unroll
-  for (int d = 0; d < S; ++d)
-    if (d < nk) issue(d, d);
+    for (int d = 0; d < S; ++d)
+      if (d < nk) issue_x(d, d);
+    norm_rows<T, S>(p.norm[which], lds, m0, q.M, nk, wave, lane, [&] {
+#pragma unroll
+      for (int d = 0; d < S; ++d)
+        if (d < nk) issue_w(d, d);
+    });
+  } else {
+#pragma unroll
+    for (int d = 0; d < S; ++d)
+      if (d < nk) issue(d, d);
+  }
 
   const int xrow = wm * 16 + l16;
   const int xa = xrow * 128 + ((lq ^ ((xrow >> 1) & 7)) << 4);

@@ -784,6 +784,17 @@ extern "C" int odit_linear_three(const odit_linear_problem* q, const int* N, int
 // holds for rows that would take two calls otherwise: 772 rows, N=9216 beside N=12288 with GELU 52 + 64 + 7 / 129.
 constexpr float kColdTile = 1.18f;
 
+// (rows or features that do not fit the heads: false, with the message set)
+static bool lin_heads_out(const char* name, const odit_linear_problem& q, int N, const odit_head_output& o, odit::HeadsOut* h) {
+  if (!(o.S > 0 && o.H > 0 && o.D > 0 && o.offset >= 0 && o.offset + static_cast<int64_t>(o.S) <= o.S_total && q.M % o.S == 0 &&
+        static_cast<int64_t>(o.H) * o.D * 3 == N && static_cast<int64_t>(q.M / o.S) * o.S_total < (1ll << 31))) {
+    odit::set_error("%s: rows or features do not fit the heads", name);
+    return false;
+  }
+  *h = odit::HeadsOut{o.q, o.k, o.v, o.wq, o.wk, o.cos, o.sin, o.S, o.offset, o.S_total, o.H * o.D, o.D, 0, 0, o.eps};
+  return true;
+}
+
 extern "C" int odit_linear_heads(const odit_linear_problem* q, const int* N, int K, const int* epilogue, const odit_head_output* const* heads, int dtype,
                                  unsigned flags, int launch, void* workspace, size_t workspace_bytes, void* stream) {
   using namespace odit;
@@ -806,12 +817,8 @@ extern "C" int odit_linear_heads(const odit_linear_problem* q, const int* N, int
     LinCall& c = calls[i] = LinCall{q[i].x, q[i].w, q[i].bias, nullptr, nullptr, q[i].out, q[i].M, N[i], K, q[i].ldx, q[i].ldw, q[i].ldo, 0,
                                     epilogue[i], dtype, dtype, lib, lib_bytes, static_cast<hipStream_t>(stream)};
     if (heads[i] != nullptr) {
-      const odit_head_output& o = *heads[i];
-      ODIT_CHECK_ARG(o.S > 0 && o.H > 0 && o.D > 0 && o.offset >= 0 && o.offset + static_cast<int64_t>(o.S) <= o.S_total && q[i].M % o.S == 0 &&
-                         static_cast<int64_t>(o.H) * o.D * 3 == N[i] && static_cast<int64_t>(q[i].M / o.S) * o.S_total < (1ll << 31),
-                     "odit_linear_heads: rows or features do not fit the heads");
-      h[i] = HeadsOut{o.q, o.k, o.v, o.wq, o.wk, o.cos, o.sin, o.S, o.offset, o.S_total, o.H * o.D, o.D, 0, 0, o.eps};
-      c.out = o.q;
+      if (!lin_heads_out("odit_linear_heads", q[i], N[i], *heads[i], &h[i])) return ODIT_EINVAL;
+      c.out = heads[i]->q;
       c.ldo = N[i];
       pass += 8.f / 15e6f * q[i].M * N[i];
     }
@@ -847,6 +854,41 @@ extern "C" int odit_linear_heads(const odit_linear_problem* q, const int* N, int
   }
   if (plan.us + end >= (plan.us < apart ? plan.us : apart) + pass) return ODIT_ENOTSUP;
   return tile();
+}
+
+// LayerNorm and modulation in front of a pair that the small kernel takes, up to 4 steps of the reduction. us, the norm's launch and the pair's /
+// one launch, one after the other without the host: M=256+64, K=256, heads of N=768 6.48 / 5.67, N=1024 with GELU 6.45 / 5.61; M=64+64, K=128,
+// N=512 5.76 / 4.35; with 8 steps, M=512+64, K=512, heads of N=1536 8.40 / 9.02 (every workgroup norms its rows again). The host, which such a
+// model mostly waits for, is asked for a launch less: 3.6 us.
+extern "C" int odit_linear_pair_norm(const odit_linear_problem* q, const odit_row_norm* norm, int N, int K, int epilogue,
+                                     const odit_head_output* const* heads, int dtype, unsigned flags, int launch, void* stream) {
+  using namespace odit;
+  ODIT_CHECK_ARG(q != nullptr && norm != nullptr && (heads == nullptr || (heads[0] != nullptr && heads[1] != nullptr)), "odit_linear_pair_norm: null arguments");
+  if (lin_engine_of(flags) != 0 || (flags & (ODIT_LINEAR_FIRST | ODIT_LINEAR_NO_TILE)) != 0) return ODIT_ENOTSUP;
+  GemmCall g[2];
+  HeadsOut h[2];
+  RowNorm r[2];
+  for (int i = 0; i < 2; ++i) {
+    LinCall c{q[i].x, q[i].w, q[i].bias, nullptr, nullptr, q[i].out, q[i].M, N, K, q[i].ldx, q[i].ldw, q[i].ldo, 0, epilogue, dtype, dtype, nullptr, 0,
+              static_cast<hipStream_t>(stream)};
+    if (heads != nullptr) {
+      if (!lin_heads_out("odit_linear_pair_norm", q[i], N, *heads[i], &h[i])) return ODIT_EINVAL;
+      c.out = heads[i]->q;
+      c.ldo = N;
+    }
+    const int rc = lin_check(c);
+    if (rc != ODIT_OK) return rc;
+    ODIT_CHECK_ARG(!lin_is_residual(c), "odit_linear_pair_norm: no residual");
+    const odit_row_norm& n = norm[i];
+    ODIT_CHECK_ARG(n.shift != nullptr && n.scale != nullptr && n.S > 0 && n.stride >= 0, "odit_linear_pair_norm: bad modulation rows");
+    g[i] = lin_gemm_call(c, 0, 0);
+    r[i] = RowNorm{n.shift, n.scale, n.stride, n.S, n.eps};
+    if (!aligned16(n.shift) || !aligned16(n.scale) || n.stride % 8 != 0 || K > kSmallNormK || !gemm_streamk_takes(g[i], dtype) ||
+        (heads != nullptr && (h[i].D != 64 || !gemm_tile_takes(g[i], dtype) || !gemm_tile_heads_takes(g[i], h[i]))))
+      return ODIT_ENOTSUP;
+  }
+  if (static_cast<int64_t>(N) * K < (1 << 14) || !gemm_small_rule(g, 2, device_cus(), kSmallNormK)) return ODIT_ENOTSUP;
+  return launch == ODIT_LAUNCH_ASK ? ODIT_OK : launch_gemm_small_norm(g, r, heads != nullptr ? h : nullptr, dtype, static_cast<hipStream_t>(stream));
 }
 
 // One projection of rows that lie in two tensors, in one reduction or as two products that add up, by expected time. One

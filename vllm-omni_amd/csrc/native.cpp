@@ -1087,6 +1087,24 @@ bool project_heads(BlockCall& c, const void* const x[2], const Lin l[2], void* c
   return true;
 }
 
+// project_pair or, with heads, project_heads of two, of rows x[i] [B S[i], K] that are normed and modulated on the way: one launch in the place of
+// two, or false. launch as above.
+bool project_normed(BlockCall& c, const void* const x[2], const Lin l[2], void* const y[2], int64_t B, const int64_t S[2], const odit_row_norm norm[2],
+                    const odit_head_output heads[2], bool gelu, bool launch) {
+  if (c.rc != 0) return true;
+  if (l[0].n != l[1].n || l[0].k != l[1].k || (l[0].b == nullptr) != (l[1].b == nullptr) || (c.engine & ODIT_LINEAR_HANDWRITTEN)) return false;
+  odit_linear_problem q[2];
+  const odit_head_output* h[2] = {heads, heads + 1};
+  for (int i = 0; i < 2; ++i)
+    q[i] = {x[i], l[i].w, l[i].b, nullptr, nullptr, y[i], static_cast<int>(B * S[i]), 0, l[i].k, l[i].ldw, l[i].n, 0, 0};
+  const int epi = gelu ? (l[0].b ? ODIT_EPI_BIAS_GELU_TANH : ODIT_EPI_GELU_TANH) : (l[0].b ? ODIT_EPI_BIAS : ODIT_EPI_NONE);
+  const int rc = odit_linear_pair_norm(q, norm, static_cast<int>(l[0].n), static_cast<int>(l[0].k), epi, heads ? h : nullptr, c.dtype, c.engine,
+                                       launch ? ODIT_LAUNCH_ANSWERED : ODIT_LAUNCH_ASK, c.where.stream);
+  if (rc == ODIT_ENOTSUP && !launch) return false;
+  c.check(rc);
+  return true;
+}
+
 // One allocation for a block's intermediate tensors. What is dead before another part begins shares its memory: after
 // `mark`, every `rewind` starts laying out from there again, over what came since (all launches are on one stream). A Wan
 // block of 2 x 32760 rows and width 5120 takes 4.7 GB this way; with every part apart it took 7.2.
@@ -1189,6 +1207,19 @@ bool run_dual(BlockCall& c, const DualBlock& k, const Tensor& img, const Tensor&
   const void* const any[2] = {at, at};
   const bool fused = k.w_dtype == c.dtype && 2 * cos[0]->size(1) == D && project_heads(c, any, k.qkv, qkv, M, heads, false, false);
   if (c.rc != 0) return true;
+  // the norms in the projections' launches (those of a small model)
+  auto mod_at = [&](int stream, int col) { return mod[stream].p + col * C * esz; };
+  auto row_norms = [&](int which, odit_row_norm r[2]) {
+    for (int i = 0; i < 2; ++i)
+      r[i] = {mod_at(i, 3 * which), mod_at(i, 3 * which + 1), mod[i].stride, static_cast<int>(S[i]), static_cast<float>(k.eps[which])};
+  };
+  odit_row_norm rn[2];
+  void* const anywhere[2] = {at, at};
+  row_norms(0, rn);
+  const bool normed_qkv = !idx && project_normed(c, any, k.qkv, anywhere, B, S, rn, fused ? heads : nullptr, false, false);
+  row_norms(1, rn);
+  const bool normed_up = !idx && project_normed(c, any, k.up, anywhere, B, S, rn, nullptr, true, false);
+  if (c.rc != 0) return true;
   // values are read where the projections left them when the text rows are whole key tiles and 32-bit offsets reach them
   const bool v_in_place = !fused && S[1] % 64 == 0 && (Sj + 64) * 3 * HD * esz < (1ll << 31);
   Slab slab(esz);
@@ -1208,7 +1239,6 @@ bool run_dual(BlockCall& c, const DualBlock& k, const Tensor& img, const Tensor&
   for (int i = 0; i < 2; ++i) result[i] = at::empty({B, S[i], C}, img.options());
 
   const int64_t rows[2][2] = {{S[0] * C, C}, {S[1] * C, C}};
-  auto mod_at = [&](int stream, int col) { return mod[stream].p + col * C * esz; };
   auto norm = [&](int stream, const void* src, int which) {
     if (c.rc != 0) return;
     c.check(odit_adaln_modulate(src, n[stream], mod_at(stream, 3 * which), mod_at(stream, 3 * which + 1), stream == 0 ? idx : nullptr, nullptr, nullptr,
@@ -1251,11 +1281,14 @@ bool run_dual(BlockCall& c, const DualBlock& k, const Tensor& img, const Tensor&
   if (idx) {
     norm(0, src[0], 0);
     norm(1, src[1], 0);
-  } else {
+  } else if (!normed_qkv) {
     norms(src, 0);
   }
-  if (fused) {
-    heads_at(jq, jk, jv);
+  heads_at(jq, jk, jv);
+  row_norms(0, rn);
+  if (normed_qkv) {
+    project_normed(c, src, k.qkv, qkv, B, S, rn, fused ? heads : nullptr, false, true);
+  } else if (fused) {
     project_heads(c, n, k.qkv, qkv, M, heads, false, true);
   } else {
     project_pair(c, n, k.qkv, qkv, M, false);
@@ -1296,8 +1329,10 @@ bool run_dual(BlockCall& c, const DualBlock& k, const Tensor& img, const Tensor&
   gated(o, k.out, src, 0);
   const void* mid[2] = {res[0], res[1]};
   if (idx) norm(1, mid[1], 1);
-  else if (c.rc == 0) norms(mid, 1);
-  project_pair(c, n, k.up, u, M, true);
+  else if (c.rc == 0 && !normed_up) norms(mid, 1);
+  row_norms(1, rn);
+  if (normed_up) project_normed(c, mid, k.up, u, B, S, rn, nullptr, true, true);
+  else project_pair(c, n, k.up, u, M, true);
   gated(u, k.down, mid, 1);
   return true;
 }
