@@ -247,6 +247,82 @@ __global__ __launch_bounds__(256) void qknorm_flat_kernel(
   }
 }
 
+// ---- one dense tensor, per-head norm or rotation alone: the layers that are called by themselves ----
+// Less of everything that qknorm_flat_kernel needs for two problems, three tensors and strides, and addresses that follow from the lane's number by
+// a shift. What bounds them is the copy rate on long sequences and the launch on short ones. The norm takes two vectors of a lane, 8 KB of a
+// tensor to a workgroup, which is about what the rotation's workgroup of the same number takes (256 lanes, both halves of the heads): so it runs
+// on the XCD whose L2 the norm's results went through. us on the GPU, one after the other, qknorm_flat_kernel / these (bf16):
+//   norm, then rotation  S=77 H=24 D=128 5.4 / 4.9    S=500 7.2 / 5.7    S=1600 11.3 / 7.7    S=3000 H=40 D=64 18.1 / 12.0 (one vector
+//   of a lane in the norm, another assignment: 17.3)    B=2 S=6032 H=24 D=128 54.2 / 48.9    S=20000 83.9 / 79.4    B=2 S=16384 139 / 134
+//   norm alone           S=77 2.66 / 2.62    S=1600 4.3 / 3.7    S=4096 8.6 / 7.2    B=2 S=6032 25.9 / 24.3    B=2 S=16384 61.6 / 57.2
+//   rotation alone       S=77 2.64 / 2.41    B=2 S=6032 27.5 / 26.3
+// KEEP: the norm's results go to the caches like any other store instead of past them (qk_dense).
+// Rows of D elements, D / EPV lanes each (a power of two up to 64).
+template <typename T, bool KEEP>
+__global__ __launch_bounds__(256) void head_norm_kernel(const T* __restrict__ x, T* __restrict__ out, const T* __restrict__ weight, unsigned total_vec,
+                                                        int D, float inv_d, float eps) {
+  constexpr int EPV = Vec16<T>::N;
+  const unsigned first = blockIdx.x * 512u + threadIdx.x;
+  u32x4 raw[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const unsigned v = first + i * 256u;
+    raw[i] = load_raw(x + static_cast<int64_t>(v < total_vec ? v : total_vec - 1) * EPV);
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const unsigned v = first + i * 256u;
+    float xf[EPV], sq = 0.f;
+#pragma unroll
+    for (int j = 0; j < EPV; ++j) {
+      xf[j] = Raw<T>::get(raw[i], j);
+      sq = fmaf(xf[j], xf[j], sq);
+    }
+    switch (D / EPV) {  // lanes per row: launch-uniform
+      case 64: sq = group_sum<64>(sq); break;
+      case 32: sq = group_sum<32>(sq); break;
+      case 16: sq = group_sum<16>(sq); break;
+      case 8: sq = group_sum<8>(sq); break;
+      case 4: sq = group_sum<4>(sq); break;
+      case 2: sq = group_sum<2>(sq); break;
+      default: break;
+    }
+    const int d0 = static_cast<int>(v * EPV) & (D - 1);
+    transform_vec<T, T, true, true, false>(xf, rsqrtf(sq * inv_d + eps), weight + d0, nullptr, nullptr, d0, 0, true, 0, false, false);
+    u32x4* const o = reinterpret_cast<u32x4*>(out + static_cast<int64_t>(v) * EPV);
+    if (v < total_vec) {
+      if constexpr (KEEP) *o = pack_vec<T>(xf);
+      else __builtin_nontemporal_store(pack_vec<T>(xf), o);
+    }
+  }
+}
+
+// [B, S, H, D], tables [S, rot / 2], pairs (2 i, 2 i + 1). A lane takes the same vector of both halves of the heads (qk_flat), H even.
+template <typename T>
+__global__ __launch_bounds__(256) void rotary_kernel(const T* __restrict__ x, T* __restrict__ out, const float* __restrict__ cos_t,
+                                                     const float* __restrict__ sin_t, unsigned lanes, FastDiv by_half, FastDiv by_s, int half, int S, uint16_t D,
+                                                     uint16_t rot) {
+  constexpr int EPV = Vec16<T>::N;
+  const unsigned i_raw = blockIdx.x * 256u + threadIdx.x, i = i_raw < lanes ? i_raw : lanes - 1;
+  const unsigned tok = by_half.div(i), s = tok - by_s.div(tok) * static_cast<unsigned>(S);
+  const int e0 = static_cast<int>(i - tok * static_cast<unsigned>(half)) * EPV, d0 = e0 & (D - 1), width = half * EPV;
+  const int64_t at = static_cast<int64_t>(tok) * (2 * width) + e0;
+  const u32x4 lo = load_raw(x + at), hi = load_raw(x + at + width);
+  float a[EPV], b[EPV];
+#pragma unroll
+  for (int j = 0; j < EPV; ++j) {
+    a[j] = Raw<T>::get(lo, j);
+    b[j] = Raw<T>::get(hi, j);
+  }
+  const int64_t row = static_cast<int64_t>(s) * (rot >> 1);
+  transform_vec<T, T, false, true, false>(a, 1.f, nullptr, cos_t + row, sin_t + row, d0, rot, true, 0, false, false);
+  transform_vec<T, T, false, true, false>(b, 1.f, nullptr, cos_t + row, sin_t + row, d0, rot, true, 0, false, false);
+  if (i_raw < lanes) {
+    __builtin_nontemporal_store(pack_vec<T>(a), reinterpret_cast<u32x4*>(out + at));
+    __builtin_nontemporal_store(pack_vec<T>(b), reinterpret_cast<u32x4*>(out + at + width));
+  }
+}
+
 // ---- whole-row statistics: one wavefront per (token, part), row held in registers ---------------
 template <typename T, typename TW, int NV, bool GENERAL>
 __global__ __launch_bounds__(256) void qknorm_row_kernel(
@@ -386,6 +462,38 @@ template <typename T, typename TW, int NORM_MODE, bool GENERAL> static int qk_fl
   return check_launch("odit_qknorm_rope");
 }
 
+// One dense tensor with per-head norm or interleaved rotation alone, 32-bit vector numbers. False: not such a call.
+template <typename T> static bool qk_dense(const QkArgs& a) {
+  constexpr int EPV = Vec16<T>::N;
+  if (a.k_in != nullptr || a.v_in != nullptr || a.pair || a.neox || a.ref_round || (a.D & (a.D - 1)) != 0) return false;
+  if (a.is_s != a.HD || (a.B > 1 && a.is_b != static_cast<int64_t>(a.S) * a.HD) || a.out_seq_offset != 0 || a.S_total != a.S) return false;
+  const int64_t vec = static_cast<int64_t>(a.B) * a.S * (a.HD / EPV);
+  if (vec >= (1ll << 31)) return false;
+  if (a.norm_mode == ODIT_NORM_HEAD && a.cos == nullptr && a.wq != nullptr && (a.w_is_f32 == std::is_same<T, float>::value)) {
+    // Results of 32 to 128 MB go to the caches: what comes next, the rotation mostly, finds them in the last-level cache (256 MB). Smaller ones
+    // come back from the L2s' way to memory anyway and are flushed from there at the launch's end, larger ones are displaced before they
+    // are read. us, norm and rotation, past the caches / to them: 10 MB 7.7 / 8.2, 25 MB 21.0 / 21.0 (the norm alone 7.2 / 11.2), 37 MB 28.8 /
+    // 27.6, 61 MB 44.4 / 41.7, 104 MB 69.3 / 66.1, 123 MB 80.1 / 79.4, 168 MB 110 / 112 (alone 48 / 58).
+    const bool keep = vec >= (2 << 20) && vec <= (8 << 20);
+    const dim3 grid(static_cast<unsigned>((vec + 511) / 512));
+    auto go = [&](auto k) {
+      hipLaunchKernelGGL((head_norm_kernel<T, decltype(k)::value>), grid, dim3(256), 0, a.stream, static_cast<const T*>(a.q_in), static_cast<T*>(a.q_out),
+                         static_cast<const T*>(a.wq), static_cast<unsigned>(vec), a.D, 1.f / static_cast<float>(a.D), a.eps);
+    };
+    if (keep) go(std::true_type{});
+    else go(std::false_type{});
+    return true;
+  }
+  if (a.norm_mode == ODIT_NORM_NONE && a.cos != nullptr && a.HD / a.D % 2 == 0) {
+    const unsigned half = static_cast<unsigned>(a.HD / EPV / 2), lanes = static_cast<unsigned>(vec / 2);
+    hipLaunchKernelGGL((rotary_kernel<T>), dim3((lanes + 255) / 256), dim3(256), 0, a.stream, static_cast<const T*>(a.q_in), static_cast<T*>(a.q_out), a.cos,
+                       a.sin, lanes, FastDiv::make(half), FastDiv::make(static_cast<uint32_t>(a.S)), static_cast<int>(half), a.S,
+                       static_cast<uint16_t>(a.D), static_cast<uint16_t>(a.rot));
+    return true;
+  }
+  return false;
+}
+
 template <typename T, typename TW, int NV, bool GENERAL> static int qk_row(const QkArgs& a) {
   const int64_t toks = static_cast<int64_t>(a.B) * a.S;
   const int nparts = 1 + (a.k_in != nullptr) + (a.v_in != nullptr);
@@ -400,6 +508,7 @@ template <typename T, typename TW, int NV, bool GENERAL> static int qk_row(const
 }
 
 template <typename T, typename TW> static int qk_go(const QkArgs& a) {
+  if (qk_dense<T>(a)) return check_launch("odit_qknorm_rope");
   const bool general = a.neox || a.ref_round;
   switch (a.norm_mode) {
     case ODIT_NORM_NONE:
