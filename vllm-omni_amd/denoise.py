@@ -260,6 +260,14 @@ class CFGParallelMixin:
         return self.scheduler_step(noise_pred, t, latents)
 
 
+def _model_timesteps(timesteps, latents: torch.Tensor) -> list[torch.Tensor] | None:
+    """``timestep.to(latents) / 1000`` of every step as [1] tensors: two launches for all steps in the place of two for each, the same
+    roundings. None where the steps are not one tensor."""
+    if not torch.is_tensor(timesteps) or timesteps.dim() != 1 or timesteps.numel() == 0:
+        return None
+    return list((timesteps.to(device=latents.device, dtype=latents.dtype) / 1000).split(1))
+
+
 class QwenImageCFGParallelMixin(CFGParallelMixin):
     """The Qwen-Image step loop with the reference's signature
     (vllm_omni/diffusion/models/qwen_image/cfg_parallel.py:27-125)."""
@@ -275,15 +283,19 @@ class QwenImageCFGParallelMixin(CFGParallelMixin):
         self.scheduler.set_begin_index(0)
         self.transformer.do_true_cfg = do_true_cfg
         extra = additional_transformer_kwargs or {}
-        for t in timesteps:
+        scaled, scaled_for = _model_timesteps(timesteps, latents), latents.dtype
+        for i, t in enumerate(timesteps):
             if self.interrupt:
                 continue
             self._current_timestep = t
-            timestep = t.expand(latents.shape[0]).to(device=latents.device, dtype=latents.dtype)
+            if scaled is not None and latents.shape[0] == 1 and latents.dtype == scaled_for:
+                timestep = scaled[i]
+            else:
+                timestep = t.expand(latents.shape[0]).to(device=latents.device, dtype=latents.dtype) / 1000
             model_input = latents if image_latents is None else torch.cat([latents, image_latents], dim=1)
 
             def branch(embeds, mask, lens):
-                return {"hidden_states": model_input, "timestep": timestep / 1000, "guidance": guidance,
+                return {"hidden_states": model_input, "timestep": timestep, "guidance": guidance,
                         "encoder_hidden_states_mask": mask, "encoder_hidden_states": embeds,
                         "img_shapes": img_shapes, "txt_seq_lens": lens, **extra}
 
