@@ -413,6 +413,10 @@ typedef struct odit_linear_problem {
 int odit_linear_pair(const odit_linear_problem problems[2], int N, int K, int epilogue, int gate_dtype, int dtype,
                      unsigned flags, void* workspace, size_t workspace_bytes, void* stream);
 
+/* 1 where odit_linear_pair (flags 0) runs the kernel for small products on 16-bit problems of M0 and M1 rows with 16-byte aligned operands,
+ * else 0: what gate and bias are wanted as (that kernel needs no gate * bias rows) without the operands in hand. */
+int odit_linear_pair_is_small(int M0, int M1, int N, int K);
+
 /* Two projections that read the same rows, of widths N[0], N[1] and epilogues of their own (no residual), in one launch of the
  * tile kernel: to_qkv beside proj_mlp of a single-stream block (flux_transformer.py:288-309), to_k beside to_v of a
  * cross-attention (wan2_2_transformer.py:520-530). Fields as for odit_linear_pair; problems[0].x and problems[1].x may also

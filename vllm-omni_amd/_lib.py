@@ -113,6 +113,7 @@ _SIGNATURES = {
     "odit_linear_heads": (
         C.c_int, [C.c_void_p, C.POINTER(C.c_int), C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_void_p), C.c_int, C.c_uint, C.c_int, C.c_void_p,
                   C.c_size_t, C.c_void_p]),
+    "odit_linear_pair_is_small": (C.c_int, [C.c_int, C.c_int, C.c_int, C.c_int]),
     "odit_linear_pair_norm": (
         C.c_int, [C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_int, C.POINTER(C.c_void_p), C.c_int, C.c_uint, C.c_int, C.c_void_p]),
     "odit_linear_join": (

@@ -536,6 +536,7 @@ class QwenImageTransformer2DModel(nn.Module):
                                       zero_cond_t=zero_cond_t)
             for _ in range(num_layers)])
         self.norm_out = AdaLayerNormContinuous(self.inner_dim, self.inner_dim, eps=1e-6)
+        self._mlp_dim = mlp_ratio * self.inner_dim
         self.proj_out = nn.Linear(self.inner_dim, patch_size * patch_size * self.out_channels, bias=True)
         self.zero_cond_t = zero_cond_t
         self.parallel_config = getattr(od_config, "parallel_config", None)
@@ -600,12 +601,16 @@ class QwenImageTransformer2DModel(nn.Module):
                 for path in (("attn", "to_out", "bias"), ("img_mlp", "net", "2", "bias"), ("attn", "to_add_out", "bias"),
                              ("txt_mlp", "net", "2", "bias"))]
 
-    def all_gate_rows(self, mods: torch.Tensor | None):
+    def all_gate_rows(self, mods: torch.Tensor | None, rows: tuple[int, int] | None = None):
         """float32 (gates, gates * biases) [B, L, 2, 2, C] of the four gated projections of every block,
-        from the stacked modulation parameters: one launch per step, or four small ops."""
+        from the stacked modulation parameters: one launch per step, or four small ops. None where the kernels that take the
+        projections of ``rows`` (image, text) need no such rows: in a small model the launch and the host's look at all the biases are
+        a tenth of a step."""
         if mods is None or mods.dtype == torch.float32 or self.zero_cond_t:
             return None  # per-token gates of the editing variant do not fit one row per batch entry
         B, L, C = mods.shape[0], mods.shape[1], self.inner_dim
+        if rows is not None and kernels.small_pairs(rows, (C, C), (C, self._mlp_dim)):
+            return None
         biases = self._gated_biases()
         rows = kernels.gate_rows(mods, biases)
         if rows is not None:
@@ -631,7 +636,7 @@ class QwenImageTransformer2DModel(nn.Module):
         mask = encoder_hidden_states_mask
         joint = joint_key_mask(mask, None, img.shape[0], txt.shape[1], img.shape[1], img.device)
         mods = self.all_modulations(temb)
-        rows = self.all_gate_rows(mods)
+        rows = self.all_gate_rows(mods, (img.shape[0] * img.shape[1], txt.shape[0] * txt.shape[1]))
         for i, block in enumerate(self.transformer_blocks):
             mp = (mods[:, i, 0], mods[:txt.shape[0], i, 1]) if mods is not None else None
             gr = (rows[0][:, i], rows[1][:, i]) if rows is not None else None

@@ -711,6 +711,15 @@ extern "C" int odit_linear_pair(const odit_linear_problem* q, int N, int K, int 
   return launch_gemm_tile(g, 2, nullptr, dtype, sk, static_cast<hipStream_t>(stream));
 }
 
+extern "C" int odit_linear_pair_is_small(int M0, int M1, int N, int K) {
+  using namespace odit;
+  if (M0 <= 0 || M1 <= 0 || N <= 0 || K <= 0 || K % kGemmBK != 0 || N % 8 != 0 || static_cast<int64_t>(N) * K < (1 << 14)) return 0;
+  GemmCall g[2] = {};
+  for (int i = 0; i < 2; ++i) { g[i].M = i == 0 ? M0 : M1; g[i].N = N; g[i].K = K; }
+  const int cus = device_cus();
+  return cus > 0 && gemm_small_rule(g, 2, cus, kSmallPairK) ? 1 : 0;
+}
+
 // Two projections that read the same rows, in one launch of the tile kernel or two calls, by expected time (2 % have to be
 // promised: where two calls would run this kernel too, its estimate is off by the same for both). What one launch
 // gains is full rounds (M=1536, N=9216 and 12288, K=3072: 504 tiles, 1.97 rounds, 150 us; 216 and 288 in two calls 194) and the

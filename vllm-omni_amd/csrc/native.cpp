@@ -694,6 +694,18 @@ PyObject* py_gate_rows(PyObject*, PyObject* const* a, Py_ssize_t n) {
   NATIVE_END
 }
 
+// (rows, rows of the second problem, N, K): whether odit_linear_pair runs the kernel for small products
+PyObject* py_pair_is_small(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  long v[4];
+  if (n != 4) return none();
+  for (int i = 0; i < 4; ++i) {
+    v[i] = PyLong_AsLong(a[i]);
+    if (PyErr_Occurred()) return nullptr;
+    if (v[i] <= 0 || v[i] >= (1l << 31)) Py_RETURN_FALSE;
+  }
+  return PyBool_FromLong(odit_linear_pair_is_small(static_cast<int>(v[0]), static_cast<int>(v[1]), static_cast<int>(v[2]), static_cast<int>(v[3])));
+}
+
 // (x, weight, bias or None, silu of x first)
 PyObject* py_linear_few(PyObject*, PyObject* const* a, Py_ssize_t n) {
   NATIVE_BEGIN
@@ -1801,6 +1813,7 @@ PyMethodDef kMethods[] = {
     NATIVE_FN("rotary", &py_rotary),
     NATIVE_FN("attn", &py_attn),
     NATIVE_FN("linear", &py_linear),
+    NATIVE_FN("pair_is_small", &py_pair_is_small),
     NATIVE_FN("linear_few", &py_linear_few),
     NATIVE_FN("project", &py_project),
     NATIVE_FN("time_sinusoid", &py_time_sinusoid),

@@ -783,6 +783,12 @@ def euler_step(x: torch.Tensor, v: torch.Tensor, dt: float) -> torch.Tensor | No
     return (_nat or _load_native()).euler_step(x, v, dt)
 
 
+def small_pairs(rows: tuple[int, int], *products: tuple[int, int]) -> bool:
+    """Whether a dual-stream block in inference runs each of these (N, K) products of its two streams on the kernel for small products,
+    which takes gates and biases as they are."""
+    return native_blocks() and _LINEAR_ENGINE_FLAGS == 0 and all((_nat or _load_native()).pair_is_small(*rows, n, k) for n, k in products)
+
+
 def gate_rows(mods: torch.Tensor, biases: list):
     """float32 (gates, gates * biases) [B, n, C] of n gated projections, ``mods`` [B, ...] holding 3 C parameters for each with its
     gate last; None for what the kernel does not take."""
