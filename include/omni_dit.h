@@ -493,6 +493,17 @@ int odit_linear_join(const void* x, const void* x2, const void* w, const void* b
 int odit_linear_few(const void* x, const void* w, const void* bias, void* out, int M, int N, int K, int64_t ldx, int64_t ldw,
                     int64_t ldo, int dtype, int silu_input, void* stream);
 
+/* odit_linear_few of the same rows with two weights, in one launch: the modulation parameters of all blocks and the head's norm
+ * (qwen_image_transformer.py:760-767, 1065). The bits of two calls. */
+int odit_linear_few_pair(const void* x, const void* const w[2], const void* const bias[2], void* const out[2], int M, const int N[2], int K,
+                         int64_t ldx, const int64_t ldw[2], const int64_t ldo[2], int dtype, int silu_input, void* stream);
+
+/* odit_linear_few of the rows that odit_time_sinusoid makes of t [M] (t_dtype; neg_log_period, scale, pre as there, the rows rounded to `dtype`),
+ * without that launch: the first projection of a timestep embedding. The bits of the two calls; ODIT_ENOTSUP also where odit_linear_few would
+ * run K as a stream (a multiple of 512 and few rows). */
+int odit_time_linear(const void* t, const void* w, const void* bias, void* out, int M, int N, int K, int64_t ldw, int64_t ldo,
+                     float neg_log_period, float scale, float pre, int t_dtype, int dtype, void* stream);
+
 /* The small work of a denoise step, one launch each, rounded where the torch expressions of the reference round:
  * odit_time_sinusoid: t [n] (t_dtype) -> out [n, dim] (out_dtype) = cos | sin of scale * (t * exp(neg_log_period j / (dim / 2)))
  *   (diffusers Timesteps with flip_sin_to_cos, qwen_image_transformer.py:165); `pre` other than 1: t is first rounded to

@@ -123,6 +123,12 @@ _SIGNATURES = {
     "odit_linear_few": (
         C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_int64, C.c_int64, C.c_int64,
                   C.c_int, C.c_int, C.c_void_p]),
+    "odit_linear_few_pair": (
+        C.c_int, [C.c_void_p, C.POINTER(C.c_void_p), C.POINTER(C.c_void_p), C.POINTER(C.c_void_p), C.c_int, C.POINTER(C.c_int), C.c_int,
+                  C.c_int64, C.POINTER(C.c_int64), C.POINTER(C.c_int64), C.c_int, C.c_int, C.c_void_p]),
+    "odit_time_linear": (
+        C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_int64, C.c_int64, C.c_float, C.c_float,
+                  C.c_float, C.c_int, C.c_int, C.c_void_p]),
     "odit_time_sinusoid": (
         C.c_int, [C.c_void_p, C.c_void_p, C.c_int64, C.c_int, C.c_float, C.c_float, C.c_float, C.c_int, C.c_int, C.c_void_p]),
     "odit_rope_tables": (

@@ -373,10 +373,10 @@ class CombinedTimestepGuidanceTextProjEmbeddings(nn.Module):
 
     def forward(self, timestep: torch.Tensor, guidance: torch.Tensor | None, pooled_projection: torch.Tensor,
                 pre: float = 1.0):
-        proj = QwenTimestepProjEmbeddings.time_proj
-        emb = self.timestep_embedder(proj(timestep, scale=1.0, dtype=pooled_projection.dtype, pre=pre))
+        embed, dtype = QwenTimestepProjEmbeddings.embed, pooled_projection.dtype
+        emb = embed(self.timestep_embedder, timestep, dtype, scale=1.0, pre=pre)
         if guidance is not None:
-            emb = emb + self.guidance_embedder(proj(guidance, scale=1.0, dtype=pooled_projection.dtype, pre=pre))
+            emb = emb + embed(self.guidance_embedder, guidance, dtype, scale=1.0, pre=pre)
         return emb + self.text_embedder(pooled_projection)
 
 
@@ -500,13 +500,27 @@ class FluxTransformer2DModel(nn.Module):
         w = getattr(self, "_mod_weight", None)
         if w is None:
             return None
-        C, L, Ls = self.inner_dim, len(self.transformer_blocks), len(self.single_transformer_blocks)
-        out = kernels.linear_few(temb, w, self._mod_bias, silu_input=True)
-        B = temb.shape[0]
+        return self._block_parts(kernels.linear_few(temb, w, self._mod_bias, silu_input=True))
+
+    def _block_parts(self, out: torch.Tensor):
+        B, C, L, Ls = out.shape[0], self.inner_dim, len(self.transformer_blocks), len(self.single_transformer_blocks)
         return out[:, :L * 12 * C].view(B, L, 2, 6 * C), out[:, L * 12 * C:].view(B, Ls, 3 * C)
 
-    def run_blocks(self, img, txt, temb, rotary, joint_attention_kwargs=None):
-        mods = self.all_modulations(temb)
+    def step_rows(self, img, temb):
+        """(``all_modulations``, the projection of the head's norm) of ``temb`` from one launch, or two Nones: not fused, or a head or a
+        stage of this model that is not the one of its class."""
+        w = getattr(self, "_mod_weight", None)
+        if (w is None or temb.dtype != img.dtype or type(self) is not FluxTransformer2DModel
+                or not kernels.plain_module(self.norm_out, AdaLayerNormContinuous)
+                or not self.__dict__.keys().isdisjoint(("all_modulations", "run_blocks", "finish"))):
+            return None, None
+        both = kernels.linear_few_pair(temb, w, self._mod_bias, self.norm_out.linear)
+        return (None, None) if both is None else (self._block_parts(both[0]), both[1])
+
+    def run_blocks(self, img, txt, temb, rotary, joint_attention_kwargs=None, mods=None):
+        """``mods``: ``all_modulations(temb)`` where the caller has it."""
+        if mods is None:
+            mods = self.all_modulations(temb)
         dual_rows, single_rows = self.all_gate_rows(mods)
         for i, block in enumerate(self.transformer_blocks):
             mp = (mods[0][:, i, 0], mods[0][:, i, 1]) if mods is not None else None
@@ -523,8 +537,9 @@ class FluxTransformer2DModel(nn.Module):
                                     gate_rows=gr)
         return x[:, n_txt:], x[:, :n_txt]
 
-    def finish(self, img, temb, return_dict: bool = True):
-        out = kernels.project(self.proj_out, self.norm_out(img, temb))
+    def finish(self, img, temb, return_dict: bool = True, head=None):
+        """``head``: the projection of the head's norm where the caller has it."""
+        out = kernels.project(self.proj_out, self.norm_out(img, temb) if head is None else self.norm_out.modulate(img, head))
         return Transformer2DModelOutput(sample=out) if return_dict else (out,)
 
     def forward(self, hidden_states: torch.Tensor, encoder_hidden_states: torch.Tensor = None,
@@ -533,8 +548,12 @@ class FluxTransformer2DModel(nn.Module):
                 joint_attention_kwargs: dict[str, Any] | None = None, return_dict: bool = True):
         img, txt, temb, rotary = self.prepare(hidden_states, encoder_hidden_states, pooled_projections, timestep,
                                               img_ids, txt_ids, guidance)
-        img, txt = self.run_blocks(img, txt, temb, rotary, joint_attention_kwargs)
-        return self.finish(img, temb, return_dict=return_dict)
+        mods, head = self.step_rows(img, temb)
+        if mods is None:
+            img, txt = self.run_blocks(img, txt, temb, rotary, joint_attention_kwargs)
+            return self.finish(img, temb, return_dict=return_dict)
+        img, txt = self.run_blocks(img, txt, temb, rotary, joint_attention_kwargs, mods=mods)
+        return self.finish(img, temb, return_dict=return_dict, head=head)
 
     # -- weights --------------------------------------------------------------------------------
     def load_weights(self, weights) -> set[str]:

@@ -465,8 +465,14 @@ class QwenTimestepProjEmbeddings(nn.Module):
         arg = scale * (t[:, None].float() * freqs[None, :])
         return torch.cat((torch.cos(arg), torch.sin(arg)), dim=-1).to(dtype)
 
+    @classmethod
+    def embed(cls, embedder: nn.Module, t: torch.Tensor, dtype: torch.dtype, scale: float = 1000.0, pre: float = 1.0):
+        """``embedder`` of ``time_proj`` of ``t``."""
+        done = kernels.time_embedding(embedder, t, 256, 10000, scale, dtype, pre)
+        return embedder(cls.time_proj(t, scale=scale, dtype=dtype, pre=pre)) if done is None else done
+
     def forward(self, timestep: torch.Tensor, hidden_states: torch.Tensor, addition_t_cond=None):
-        emb = self.timestep_embedder(self.time_proj(timestep, dtype=hidden_states.dtype))
+        emb = self.embed(self.timestep_embedder, timestep, hidden_states.dtype)
         if self.use_additional_t_cond:
             if addition_t_cond is None:
                 raise ValueError("When additional_t_cond is True, addition_t_cond must be provided.")
@@ -487,6 +493,10 @@ class AdaLayerNormContinuous(nn.Module):
             emb = kernels.project(self.linear, cond, silu_input=True)
         else:
             emb = self.linear(kernels.silu(cond).to(x.dtype))
+        return self.modulate(x, emb)
+
+    def modulate(self, x: torch.Tensor, emb: torch.Tensor) -> torch.Tensor:
+        """``forward`` with the projection of the condition at hand."""
         scale, shift = emb.chunk(2, dim=1)
         return kernels.adaln_modulate(x, shift, scale, eps=self.eps)
 
@@ -629,13 +639,27 @@ class QwenImageTransformer2DModel(nn.Module):
         out = kernels.linear_few(temb, w.view(L * 2 * 6 * C, C), self._mod_bias.view(-1), silu_input=True)
         return out.view(temb.shape[0], L, 2, 6 * C)
 
+    def step_rows(self, img, temb):
+        """(``all_modulations``, the projection of the head's norm) of ``temb`` from one launch, or two Nones: not fused, a head or a
+        stage of this model that is not the one of its class, or (editing variant) a head that follows from fewer rows."""
+        w = getattr(self, "_mod_weight", None)
+        if (w is None or self.zero_cond_t or temb.dtype != img.dtype or type(self) is not QwenImageTransformer2DModel
+                or not kernels.plain_module(self.norm_out, AdaLayerNormContinuous)
+                or not self.__dict__.keys().isdisjoint(("all_modulations", "run_blocks", "finish"))):
+            return None, None
+        L, C = w.shape[0], self.inner_dim
+        both = kernels.linear_few_pair(temb, w.view(L * 2 * 6 * C, C), self._mod_bias.view(-1), self.norm_out.linear)
+        return (None, None) if both is None else (both[0].view(temb.shape[0], L, 2, 6 * C), both[1])
+
     def run_blocks(self, img, txt, temb, rotary, encoder_hidden_states_mask=None, attention_kwargs=None,
-                   modulate_index=None):
+                   modulate_index=None, mods=None):
+        """``mods``: ``all_modulations(temb)`` where the caller has it."""
         # the reference drops an all-true mask (qit.py:1044-1048), which takes a synchronisation; the masked kernel gives
         # the same values for one at 1 to 4 % of its time, as a tile without an excluded key runs without selects
         mask = encoder_hidden_states_mask
         joint = joint_key_mask(mask, None, img.shape[0], txt.shape[1], img.shape[1], img.device)
-        mods = self.all_modulations(temb)
+        if mods is None:
+            mods = self.all_modulations(temb)
         rows = self.all_gate_rows(mods, (img.shape[0] * img.shape[1], txt.shape[0] * txt.shape[1]))
         for i, block in enumerate(self.transformer_blocks):
             mp = (mods[:, i, 0], mods[:txt.shape[0], i, 1]) if mods is not None else None
@@ -645,10 +669,11 @@ class QwenImageTransformer2DModel(nn.Module):
                              modulate_index=modulate_index, mod_params=mp, gate_rows=gr, joint_mask=joint)
         return img, txt
 
-    def finish(self, img, temb, return_dict: bool = True):
+    def finish(self, img, temb, return_dict: bool = True, head=None):
+        """``head``: the projection of the head's norm where the caller has it."""
         if self.zero_cond_t:
             temb = temb.chunk(2, dim=0)[0]  # the head is conditioned on the real timestep (qit.py:1062-1063)
-        out = kernels.project(self.proj_out, self.norm_out(img, temb))
+        out = kernels.project(self.proj_out, self.norm_out(img, temb) if head is None else self.norm_out.modulate(img, head))
         return Transformer2DModelOutput(sample=out) if return_dict else (out,)
 
     def forward(self, hidden_states: torch.Tensor, encoder_hidden_states: torch.Tensor = None,
@@ -662,9 +687,12 @@ class QwenImageTransformer2DModel(nn.Module):
         img, txt, temb, rotary = self.prepare(hidden_states, encoder_hidden_states, timestep, img_shapes, txt_seq_lens,
                                               additional_t_cond)
         index = self.modulate_index(img_shapes, img.device)
-        img, txt = self.run_blocks(img, txt, temb, rotary, encoder_hidden_states_mask, attention_kwargs,
-                                   modulate_index=index)
-        return self.finish(img, temb, return_dict=return_dict)
+        mods, head = self.step_rows(img, temb)
+        if mods is None:
+            img, txt = self.run_blocks(img, txt, temb, rotary, encoder_hidden_states_mask, attention_kwargs, modulate_index=index)
+            return self.finish(img, temb, return_dict=return_dict)
+        img, txt = self.run_blocks(img, txt, temb, rotary, encoder_hidden_states_mask, attention_kwargs, mods=mods)
+        return self.finish(img, temb, return_dict=return_dict, head=head)
 
     # -- weights --------------------------------------------------------------------------------
     def load_weights(self, weights) -> set[str]:
@@ -686,6 +714,6 @@ class QwenImageTransformer2DModel(nn.Module):
                 p.copy_(weights[k].to(device=p.device, dtype=p.dtype))
 
 
-kernels.native_classes(Linear=nn.Linear, RMSNorm=RMSNorm, AdaLayerNorm=AdaLayerNorm, Attention=Attention,
+kernels.native_classes(Linear=nn.Linear, TimestepEmbedding=TimestepEmbedding, RMSNorm=RMSNorm, AdaLayerNorm=AdaLayerNorm, Attention=Attention,
                        AttentionImpl=HipFlashAttentionImpl, FeedForward=FeedForward, ApproxGELU=ApproxGELU,
                        QwenImageCrossAttention=QwenImageCrossAttention)

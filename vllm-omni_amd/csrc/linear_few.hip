@@ -21,6 +21,12 @@
 // length: conflict-free), is the B operand (column = row of x; columns past M repeat the last row and are not stored), and is
 // activated once while it is staged. The 8 partial sums of a tile meet in LDS (two buffers by turns, so one barrier per
 // tile), in the order of the waves: results do not depend on timing.
+//
+// Both take two weights in one launch, the second one's features behind the first one's: the modulation parameters of all blocks and the
+// head's norm follow from the same rows. us, two launches / one, cold weights, two rows: K=3072, 442368 + 6144 features 429.7 / 427.2,
+// 73728 + 6144 81.3 / 78.2, 18432 + 6144 30.7 / 26.5; K=256, 24576 + 512 14.3 / 11.2, 6144 + 512 9.4 / 5.6.
+// linear_few_sinusoid_kernel: the rows of x are a timestep's cosines and sines, formed where they are staged (time_sinusoid_kernel's
+// operations): 3072 features, K=256 5.8 / 4.3, the launch less.
 #include "odit_common.h"
 #include "gemm_bf16.h"
 
@@ -59,16 +65,43 @@ __device__ __forceinline__ void stage_rows(const T* __restrict__ x, u32x4* xs, i
   }
 }
 
-template <typename T, bool SILU>
-__global__ __launch_bounds__(kWaves * 64, 6) void linear_few_kernel(const T* __restrict__ x, const T* __restrict__ w,
-                                                                    const T* __restrict__ bias, T* __restrict__ out, int M,
-                                                                    int N, int K, int64_t ldx, int64_t ldw, int64_t ldo,
-                                                                    int tiles) {
+// A weight and where its products go
+template <typename T> struct FewOut {
+  const T *w, *bias;
+  T* out;
+  int64_t ldw, ldo;
+  int N;
+};
+
+// The timesteps' cosines and sines [M, K] to LDS, as time_sinusoid_kernel forms them
+template <typename TT> struct Sinusoid {
+  const TT* t;
+  float neg_log_period, scale, pre;
+};
+template <typename T, typename TT>
+__device__ __forceinline__ void stage_sinusoid(const Sinusoid<TT>& a, u32x4* xs, int rows, int K, int pitch) {
+#pragma clang fp contract(off)
+  const int half = K / 2;
+  T* const to = reinterpret_cast<T*>(xs);
+  for (int i = threadIdx.x; i < rows * half; i += kWaves * 64) {
+    const int m = i / half, j = i - m * half;
+    const float freq = expf(a.neg_log_period * static_cast<float>(j) / static_cast<float>(half));
+    float tv = to_float(a.t[m]);
+    if (a.pre != 1.f) tv = round_to<T>(round_to<T>(tv) * a.pre);
+    const float arg = a.scale * (tv * freq);
+    to[m * pitch * 8 + j] = from_float<T>(cosf(arg));
+    to[m * pitch * 8 + half + j] = from_float<T>(sinf(arg));
+  }
+}
+
+// tiles0: of the first weight. PAIR: of two (a template, so that one costs no selects: 442368 features, two rows 418 us, with them 421)
+template <typename T, bool PAIR, typename Stage>
+__device__ __forceinline__ void few_rows(Stage&& stage, const FewOut<T>& o0, const FewOut<T>& o1, int M, int K, int tiles0, int tiles) {
   extern __shared__ u32x4 lds[];
   f32x4* red = reinterpret_cast<f32x4*>(lds);
   u32x4* xs = lds + kRedBytes / 16;
   const int vecs = K / 8, pitch = vecs + 1;  // 16-byte vectors of a row of x
-  stage_rows<T, SILU>(x, xs, M, vecs, pitch, ldx);
+  stage(xs, vecs, pitch);
   __syncthreads();
 
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -80,7 +113,9 @@ __global__ __launch_bounds__(kWaves * 64, 6) void linear_few_kernel(const T* __r
 
   // loads past the wave's share repeat its last step (an L1 hit); a wave without a share reads the row's last step
   auto fetch = [&](u32x4 (&r)[kSteps], int tile, int chunk) {
-    const T* p = w + static_cast<int64_t>(min(tile * kTile + col, N - 1)) * ldw + quad * 8;
+    const bool second = PAIR && tile >= tiles0;  // (uniform; past the last tile too)
+    const int row = min((second ? tile - tiles0 : tile) * kTile + col, (second ? o1.N : o0.N) - 1);
+    const T* p = (second ? o1.w : o0.w) + row * (second ? o1.ldw : o0.ldw) + quad * 8;
     const int last = max(first + count - 1, 0);
 #pragma unroll
     for (int s = 0; s < kSteps; ++s) {
@@ -105,11 +140,14 @@ __global__ __launch_bounds__(kWaves * 64, 6) void linear_few_kernel(const T* __r
       f32x4 sum = buf[lane];
 #pragma unroll
       for (int q = 1; q < kWaves; ++q) sum += buf[q * 64 + lane];
-      const int n = tile * kTile + quad * 4;
+      const bool second = PAIR && tile >= tiles0;
+      const int n = (second ? tile - tiles0 : tile) * kTile + quad * 4, N = second ? o1.N : o0.N;
+      const T* const bias = second ? o1.bias : o0.bias;
+      T* const out = (second ? o1.out : o0.out) + col * (second ? o1.ldo : o0.ldo);
       if (col < M) {
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-          if (n + j < N) out[col * ldo + n + j] = from_float<T>(sum[j] + (bias != nullptr ? to_float(bias[n + j]) : 0.f));
+          if (n + j < N) out[n + j] = from_float<T>(sum[j] + (bias != nullptr ? to_float(bias[n + j]) : 0.f));
       }
     }
     ++turn;
@@ -137,21 +175,34 @@ __global__ __launch_bounds__(kWaves * 64, 6) void linear_few_kernel(const T* __r
   }
 }
 
-template <typename T, bool SILU, int M, int R>
-__global__ __launch_bounds__(kWaves * 64, 6) void linear_stream_kernel(const T* __restrict__ x, const T* __restrict__ w,
-                                                                       const T* __restrict__ bias, T* __restrict__ out, int rows,
-                                                                       int N, int K, int64_t ldx, int64_t ldw, int64_t ldo) {
+template <typename T, bool SILU, bool PAIR>
+__global__ __launch_bounds__(kWaves * 64, 6) void linear_few_kernel(const T* __restrict__ x, const FewOut<T> o0, const FewOut<T> o1, int M, int K,
+                                                                    int64_t ldx, int tiles0, int tiles) {
+  few_rows<T, PAIR>([&](u32x4* xs, int vecs, int pitch) { stage_rows<T, SILU>(x, xs, M, vecs, pitch, ldx); }, o0, o1, M, K, tiles0, tiles);
+}
+template <typename T, typename TT>
+__global__ __launch_bounds__(kWaves * 64, 6) void linear_few_sinusoid_kernel(const Sinusoid<TT> a, const FewOut<T> o, int M, int K, int tiles) {
+  few_rows<T, false>([&](u32x4* xs, int, int pitch) { stage_sinusoid<T, TT>(a, xs, M, K, pitch); }, o, o, M, K, tiles, tiles);
+}
+
+// (groups of R features; those of the first weight come first)
+template <typename T, bool SILU, int M, int R, bool PAIR>
+__global__ __launch_bounds__(kWaves * 64, 6) void linear_stream_kernel(const T* __restrict__ x, const FewOut<T> o0, const FewOut<T> o1, int rows, int K,
+                                                                       int64_t ldx) {
   extern __shared__ u32x4 lds[];
   const int vecs = K / 8;
   stage_rows<T, SILU>(x, lds, rows, vecs, vecs, ldx);
   __syncthreads();
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int chunks = K / 512, groups = (N + R - 1) / R, stride = gridDim.x * kWaves;
-  const T* const mine = w + lane * 8;
+  const int groups0 = (o0.N + R - 1) / R, groups = groups0 + (PAIR ? (o1.N + R - 1) / R : 0);
+  const int chunks = K / 512, stride = gridDim.x * kWaves;
   auto fetch = [&](u32x4 (&r)[R], int g, int c) {
+    const bool second = PAIR && g >= groups0;  // (uniform; past the last group too)
+    const T* const mine = (second ? o1.w : o0.w) + lane * 8 + c * 512;
+    const int64_t ldw = second ? o1.ldw : o0.ldw;
+    const int n0 = (second ? g - groups0 : g) * R, last = (second ? o1.N : o0.N) - 1;
 #pragma unroll
-    for (int i = 0; i < R; ++i)
-      r[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(mine + static_cast<int64_t>(min(g * R + i, N - 1)) * ldw + c * 512));
+    for (int i = 0; i < R; ++i) r[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(mine + min(n0 + i, last) * ldw));
   };
   float acc[R][M];
 #pragma unroll
@@ -184,8 +235,12 @@ __global__ __launch_bounds__(kWaves * 64, 6) void linear_stream_kernel(const T* 
         if (lane == i * M + m) mine_sum = s;
         acc[i][m] = 0.f;
       }
-    const int n = g * R + lane / M, m = lane % M;
-    if (lane < R * M && n < N && m < rows) out[m * ldo + n] = from_float<T>(mine_sum + (bias != nullptr ? to_float(bias[n]) : 0.f));
+    const bool second = PAIR && g >= groups0;
+    const int n = (second ? g - groups0 : g) * R + lane / M, m = lane % M;
+    const T* const bias = second ? o1.bias : o0.bias;
+    T* const out = second ? o1.out : o0.out;
+    if (lane < R * M && n < (second ? o1.N : o0.N) && m < rows)
+      out[m * (second ? o1.ldo : o0.ldo) + n] = from_float<T>(mine_sum + (bias != nullptr ? to_float(bias[n]) : 0.f));
   };
   u32x4 a[R], b[R];
   auto next = [&](int& g, int& c) {
@@ -208,29 +263,19 @@ __global__ __launch_bounds__(kWaves * 64, 6) void linear_stream_kernel(const T* 
   }
 }
 
-template <typename T, bool SILU>
-int launch_few(const void* x, const void* w, const void* bias, void* out, int M, int N, int K, int64_t ldx, int64_t ldw,
-               int64_t ldo, int grid, int tiles, size_t lds, hipStream_t stream) {
-  linear_few_kernel<T, SILU><<<grid, kWaves * 64, lds, stream>>>(static_cast<const T*>(x), static_cast<const T*>(w),
-                                                                 static_cast<const T*>(bias), static_cast<T*>(out), M, N, K,
-                                                                 ldx, ldw, ldo, tiles);
-  return check_launch("odit_linear_few");
-}
-
 // Rows of W a wavefront takes at a time: two; four (twice the loads in flight, half the steps) where every wavefront of the grid
 // has three or more such groups and one or two rows of x leave the registers for it: N=442368, two rows of x 414 / 405 us,
 // 73728 69.5 / 68.1, but 36864 36.5 / 37.3, 9216 13.2 / 15.0; with four rows of x 440 / 566.
 constexpr int kStreamWide = 1 << 16;
 
-template <typename T, bool SILU>
-int launch_stream(const void* x, const void* w, const void* bias, void* out, int M, int N, int K, int64_t ldx, int64_t ldw, int64_t ldo, int slots,
-                  hipStream_t stream) {
+template <typename T, bool SILU, bool PAIR>
+int launch_stream(const T* x, const FewOut<T>& o0, const FewOut<T>& o1, int M, int K, int64_t ldx, int slots, hipStream_t stream) {
   const size_t lds = static_cast<size_t>(M) * K * 2;
+  const int N = o0.N + (PAIR ? o1.N : 0);
 #define ODIT_STREAM(ROWS, R)                                                                                                             \
   do {                                                                                                                                   \
-    const int wanted = (N + R * kWaves - 1) / (R * kWaves);                                                                              \
-    linear_stream_kernel<T, SILU, ROWS, R><<<wanted < slots ? wanted : slots, kWaves * 64, lds, stream>>>(                                 \
-        static_cast<const T*>(x), static_cast<const T*>(w), static_cast<const T*>(bias), static_cast<T*>(out), M, N, K, ldx, ldw, ldo);     \
+    const int groups = (o0.N + R - 1) / R + (PAIR ? (o1.N + R - 1) / R : 0), wanted = (groups + kWaves - 1) / kWaves;                      \
+    linear_stream_kernel<T, SILU, ROWS, R, PAIR><<<wanted < slots ? wanted : slots, kWaves * 64, lds, stream>>>(x, o0, o1, M, K, ldx);     \
   } while (0)
   if (M > 2) ODIT_STREAM(4, 2);
   else if (N >= kStreamWide && M == 2) ODIT_STREAM(2, 4);
@@ -241,45 +286,118 @@ int launch_stream(const void* x, const void* w, const void* bias, void* out, int
   return check_launch("odit_linear_few (stream)");
 }
 
-}  // namespace
-}  // namespace odit
-
 // Taken: up to 16 rows of x (the columns of one MFMA operand) that fit a CU's LDS; three workgroups per CU while they fit,
 // one still has 64 KB of loads in flight.
 constexpr int kFewMaxRows = 16, kFewMaxGroups = 3, kStreamMaxRows = 4;
 constexpr size_t kFewMaxLds = 160 * 1024;
 
+size_t few_lds(int M, int K) { return kRedBytes + static_cast<size_t>(M) * (K / 8 + 1) * 16; }
+int few_grid(int tiles, size_t lds, int cus) {
+  const int fit = static_cast<int>(kFewMaxLds / lds), slots = cus * (fit < kFewMaxGroups ? fit : kFewMaxGroups);
+  return tiles < slots ? tiles : slots;
+}
+
+struct FewArgs { const void *w, *bias; void* out; int N; int64_t ldw, ldo; };
+
+// How many rows a wavefront takes at a time follows from the features
+// of both; the bits do not (a feature's sum is one wavefront's).
+template <typename T, bool SILU, bool PAIR>
+int run_few(const void* x, const FewArgs* a, int M, int K, int64_t ldx, int cus, hipStream_t stream) {
+  FewOut<T> o[2];
+  for (int i = 0; i < 2; ++i)  // (without a second weight nothing reads the second)
+    o[i] = FewOut<T>{static_cast<const T*>(a[i].w), static_cast<const T*>(a[i].bias), static_cast<T*>(a[i].out), a[i].ldw, a[i].ldo, a[i].N};
+  if (M <= kStreamMaxRows && K % 512 == 0 && static_cast<size_t>(M) * K * 2 <= kFewMaxLds / kFewMaxGroups)
+    return launch_stream<T, SILU, PAIR>(static_cast<const T*>(x), o[0], o[1], M, K, ldx, cus * kFewMaxGroups, stream);
+  const int tiles0 = (a[0].N + kTile - 1) / kTile, tiles = tiles0 + (PAIR ? (a[1].N + kTile - 1) / kTile : 0);
+  const size_t lds = few_lds(M, K);
+  linear_few_kernel<T, SILU, PAIR><<<few_grid(tiles, lds, cus), kWaves * 64, lds, stream>>>(static_cast<const T*>(x), o[0], o[1], M, K, ldx, tiles0, tiles);
+  return check_launch("odit_linear_few");
+}
+
+template <typename T, typename TT>
+int run_sinusoid(const void* t, float neg_log_period, float scale, float pre, const FewArgs& a, int M, int K, int cus, hipStream_t stream) {
+  const FewOut<T> o{static_cast<const T*>(a.w), static_cast<const T*>(a.bias), static_cast<T*>(a.out), a.ldw, a.ldo, a.N};
+  const int tiles = (a.N + kTile - 1) / kTile;
+  const size_t lds = few_lds(M, K);
+  linear_few_sinusoid_kernel<T, TT><<<few_grid(tiles, lds, cus), kWaves * 64, lds, stream>>>(
+      Sinusoid<TT>{static_cast<const TT*>(t), neg_log_period, scale, pre}, o, M, K, tiles);
+  return check_launch("odit_time_linear");
+}
+
+}  // namespace
+}  // namespace odit
+
+static int few_check(const char* name, const odit::FewArgs* a, int count, int M, int K, int dtype) {
+  using namespace odit;
+  ODIT_CHECK_ARG(M >= 0 && K > 0, "%s: bad shape M=%d K=%d", name, M, K);
+  const size_t lds = few_lds(M, K);
+  bool takes = (dtype == ODIT_BF16 || dtype == ODIT_F16) && M <= kFewMaxRows && K % kStepK == 0 && lds <= kFewMaxLds;
+  for (int i = 0; i < count; ++i) {
+    ODIT_CHECK_ARG(a[i].w && a[i].out, "%s: w/out must not be null", name);
+    ODIT_CHECK_ARG(a[i].N > 0, "%s: bad shape N=%d", name, a[i].N);
+    ODIT_CHECK_ARG(a[i].ldw >= K && a[i].ldo >= a[i].N, "%s: leading dimensions too small", name);
+    takes = takes && a[i].ldw % 8 == 0 && aligned16(a[i].w);
+  }
+  if (!takes) {
+    set_error("%s: takes 16-bit types, M <= %d, K a multiple of %d, 16-byte aligned rows and M (K + 8) 2 bytes of LDS (M=%d N=%d K=%d)", name, kFewMaxRows,
+              kStepK, M, a[0].N, K);
+    return ODIT_ENOTSUP;
+  }
+  return ODIT_OK;
+}
+
+static int few_go(const char* name, const void* x, odit::FewArgs (&a)[2], int count, int M, int K, int64_t ldx, int dtype, int silu_input, void* stream) {
+  using namespace odit;
+  ODIT_CHECK_ARG(x != nullptr, "%s: x must not be null", name);
+  ODIT_CHECK_ARG(ldx >= K, "%s: leading dimensions too small", name);
+  const int rc = few_check(name, a, count, M, K, dtype);
+  if (rc != ODIT_OK) return rc;
+  if (ldx % 8 != 0 || !aligned16(x)) { set_error("%s: rows of x must be 16-byte aligned", name); return ODIT_ENOTSUP; }
+  if (M == 0) return ODIT_OK;
+  const int cus = device_cus();
+  if (cus <= 0) { set_error("%s: cannot read the device's compute-unit count", name); return ODIT_ELAUNCH; }
+  const hipStream_t s = static_cast<hipStream_t>(stream);
+#define ODIT_FEW(T, SILU) (count == 2 ? run_few<T, SILU, true>(x, a, M, K, ldx, cus, s) : run_few<T, SILU, false>(x, a, M, K, ldx, cus, s))
+  if (dtype == ODIT_BF16) return silu_input ? ODIT_FEW(bf16_t, true) : ODIT_FEW(bf16_t, false);
+  return silu_input ? ODIT_FEW(f16_t, true) : ODIT_FEW(f16_t, false);
+#undef ODIT_FEW
+}
+
 extern "C" int odit_linear_few(const void* x, const void* w, const void* bias, void* out, int M, int N, int K, int64_t ldx,
                                int64_t ldw, int64_t ldo, int dtype, int silu_input, void* stream) {
+  odit::FewArgs a[2] = {{w, bias, out, N, ldw, ldo}, {}};
+  return few_go("odit_linear_few", x, a, 1, M, K, ldx, dtype, silu_input, stream);
+}
+
+extern "C" int odit_linear_few_pair(const void* x, const void* const w[2], const void* const bias[2], void* const out[2], int M, const int N[2], int K,
+                                    int64_t ldx, const int64_t ldw[2], const int64_t ldo[2], int dtype, int silu_input, void* stream) {
   using namespace odit;
-  ODIT_CHECK_ARG(x && w && out, "odit_linear_few: x/w/out must not be null");
-  ODIT_CHECK_ARG(M >= 0 && N > 0 && K > 0, "odit_linear_few: bad shape M=%d N=%d K=%d", M, N, K);
-  ODIT_CHECK_ARG(ldx >= K && ldw >= K && ldo >= N, "odit_linear_few: leading dimensions too small");
-  const size_t lds = kRedBytes + static_cast<size_t>(M) * (K / 8 + 1) * 16;
-  if ((dtype != ODIT_BF16 && dtype != ODIT_F16) || M > kFewMaxRows || K % kStepK != 0 || ldx % 8 != 0 || ldw % 8 != 0 ||
-      !aligned16(x) || !aligned16(w) || lds > kFewMaxLds) {
-    set_error("odit_linear_few: takes 16-bit types, M <= %d, K a multiple of %d, 16-byte aligned rows and M (K + 8) 2 bytes of LDS (M=%d N=%d K=%d)",
-              kFewMaxRows, kStepK, M, N, K);
+  ODIT_CHECK_ARG(w && bias && out && N && ldw && ldo, "odit_linear_few_pair: null arguments");
+  FewArgs a[2];
+  for (int i = 0; i < 2; ++i) a[i] = FewArgs{w[i], bias[i], out[i], N[i], ldw[i], ldo[i]};
+  ODIT_CHECK_ARG(static_cast<int64_t>(N[0]) + N[1] < (1ll << 31) - 64, "odit_linear_few_pair: too many features");
+  return few_go("odit_linear_few_pair", x, a, 2, M, K, ldx, dtype, silu_input, stream);
+}
+
+extern "C" int odit_time_linear(const void* t, const void* w, const void* bias, void* out, int M, int N, int K, int64_t ldw, int64_t ldo,
+                                float neg_log_period, float scale, float pre, int t_dtype, int dtype, void* stream) {
+  using namespace odit;
+  ODIT_CHECK_ARG(t != nullptr, "odit_time_linear: t must not be null");
+  const FewArgs a{w, bias, out, N, ldw, ldo};
+  const int rc = few_check("odit_time_linear", &a, 1, M, K, dtype);
+  if (rc != ODIT_OK) return rc;
+  // (a reduction that the stream kernel would take has another order of summation)
+  if (M <= kStreamMaxRows && K % 512 == 0 && static_cast<size_t>(M) * K * 2 <= kFewMaxLds / kFewMaxGroups) {
+    set_error("odit_time_linear: K=%d is the stream kernel's", K);
     return ODIT_ENOTSUP;
   }
   if (M == 0) return ODIT_OK;
   const int cus = device_cus();
-  if (cus <= 0) { set_error("odit_linear_few: cannot read the device's compute-unit count"); return ODIT_ELAUNCH; }
-  const int tiles = (N + kTile - 1) / kTile, fit = static_cast<int>(kFewMaxLds / lds);
-  const int slots = cus * (fit < kFewMaxGroups ? fit : kFewMaxGroups), grid = tiles < slots ? tiles : slots;
+  if (cus <= 0) { set_error("odit_time_linear: cannot read the device's compute-unit count"); return ODIT_ELAUNCH; }
   const hipStream_t s = static_cast<hipStream_t>(stream);
-  const size_t stream_lds = static_cast<size_t>(M) * K * 2;
-  if (M <= kStreamMaxRows && K % 512 == 0 && stream_lds <= kFewMaxLds / kFewMaxGroups) {
-    const int all = cus * kFewMaxGroups;
-    if (dtype == ODIT_BF16)
-      return silu_input ? launch_stream<bf16_t, true>(x, w, bias, out, M, N, K, ldx, ldw, ldo, all, s)
-                        : launch_stream<bf16_t, false>(x, w, bias, out, M, N, K, ldx, ldw, ldo, all, s);
-    return silu_input ? launch_stream<f16_t, true>(x, w, bias, out, M, N, K, ldx, ldw, ldo, all, s)
-                      : launch_stream<f16_t, false>(x, w, bias, out, M, N, K, ldx, ldw, ldo, all, s);
-  }
-  if (dtype == ODIT_BF16)
-    return silu_input ? launch_few<bf16_t, true>(x, w, bias, out, M, N, K, ldx, ldw, ldo, grid, tiles, lds, s)
-                      : launch_few<bf16_t, false>(x, w, bias, out, M, N, K, ldx, ldw, ldo, grid, tiles, lds, s);
-  return silu_input ? launch_few<f16_t, true>(x, w, bias, out, M, N, K, ldx, ldw, ldo, grid, tiles, lds, s)
-                    : launch_few<f16_t, false>(x, w, bias, out, M, N, K, ldx, ldw, ldo, grid, tiles, lds, s);
+  ODIT_DISPATCH_DTYPE(t_dtype, TT, {
+    return dtype == ODIT_BF16 ? run_sinusoid<bf16_t, TT>(t, neg_log_period, scale, pre, a, M, K, cus, s)
+                              : run_sinusoid<f16_t, TT>(t, neg_log_period, scale, pre, a, M, K, cus, s);
+  });
+  return ODIT_OK;
 }

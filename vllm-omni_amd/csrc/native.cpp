@@ -826,7 +826,7 @@ struct Names {
 Names g_name;
 PyTypeObject *g_linear_type, *g_rmsnorm_type, *g_rownorm_type, *g_adaln_type, *g_attention_type, *g_attention_impl_type,
     *g_feed_forward_type, *g_gelu_type, *g_wan_ffn_type, *g_qwen_attention_type, *g_flux_attention_type, *g_flux_single_norm_type,
-    *g_wan_self_type, *g_wan_cross_type;
+    *g_wan_self_type, *g_wan_cross_type, *g_time_embedding_type;
 
 PyObject* instance_dict(PyObject* m) {
   PyObject** d = m ? _PyObject_GetDictPtr(m) : nullptr;
@@ -970,6 +970,67 @@ PyObject* py_project(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return odit_linear_rows(x->data_ptr(), l.w, l.b, out.data_ptr(), nullptr, nullptr, static_cast<int>(M), static_cast<int>(l.n),
                             static_cast<int>(l.k), ldx, l.ldw, l.n, 0, epi, c.dtype, c.dtype, 0, 0, static_cast<unsigned>(flags),
                             c.lin_ws.p, c.lin_ws.bytes, c.where.stream);
+  });
+  if (rc != 0) return none();
+  return wrap(std::move(out));
+  NATIVE_END
+}
+
+// (x, weight, bias or None, plain Linear): silu(x) W^T + bias of the weight and of the module's, each [rows of x, features], in one launch
+PyObject* py_linear_few_pair(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  NATIVE_BEGIN
+  const Tensor *x, *wt, *b;
+  if (n != 4 || g_linear_type == nullptr || !(x = tensor_of(a[0])) || !(wt = tensor_of(a[1])) || !optional_tensor(a[2], &b)) return none();
+  BlockCall c;
+  c.dtype = code_of(*x);
+  c.st = x->scalar_type();
+  Lin l;
+  int64_t M, ldx;
+  if (c.dtype < 0 || !c.operand(*x) || !c.operand(*wt) || wt->dim() != 2 || wt->stride(1) != 1 || x->dim() != 2 || !c.linear(a[3], &l, false) ||
+      x->size(1) != l.k || wt->size(1) != l.k || !rows_of(*x, &M, &ldx) || M < 1 || M > 16)
+    return none();
+  const int64_t N = wt->size(0), K = l.k;
+  if (N < 1 || l.n < 1 || K < 1 || N >= (1ll << 30) || l.n >= (1ll << 30)) return none();
+  if (b && (!c.operand(*b) || b->numel() != N || !b->is_contiguous())) return none();
+  Tensor out = fresh({M, N}, x->options()), out2 = fresh({M, l.n}, x->options());
+  const void *const w[2] = {wt->data_ptr(), l.w}, *const bias[2] = {ptr(b), l.b};
+  void* const to[2] = {out.data_ptr(), out2.data_ptr()};
+  const int features[2] = {static_cast<int>(N), static_cast<int>(l.n)};
+  const int64_t ldw[2] = {N > 1 ? wt->stride(0) : K, l.ldw}, ldo[2] = {N, l.n};
+  if (unlocked([&] { return odit_linear_few_pair(x->data_ptr(), w, bias, to, static_cast<int>(M), features, static_cast<int>(K), ldx, ldw, ldo, c.dtype, 1,
+                                                 c.where.stream); }) != 0)
+    return none();
+  return Py_BuildValue("(NN)", wrap(std::move(out)), wrap(std::move(out2)));
+  NATIVE_END
+}
+
+// (TimestepEmbedding, t [n], cosines and sines, - ln of the longest period, scale, type code of the rows, pre): linear_2(silu(linear_1(sinusoid of t))) in two launches
+PyObject* py_time_embedding(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  NATIVE_BEGIN
+  const Tensor* t;
+  PyObject* const d = n == 7 && g_linear_type != nullptr && g_time_embedding_type != nullptr ? plain_module(a[0], g_time_embedding_type) : nullptr;
+  if (d == nullptr || !(t = tensor_of(a[1]))) return none();
+  const double period = PyFloat_AsDouble(a[3]), scale = PyFloat_AsDouble(a[4]), pre = PyFloat_AsDouble(a[6]);
+  const long dim = PyLong_AsLong(a[2]), code = PyLong_AsLong(a[5]);
+  if (PyErr_Occurred()) return nullptr;
+  if (code != ODIT_BF16 && code != ODIT_F16) return none();
+  BlockCall c;
+  c.dtype = static_cast<int>(code);
+  c.st = code == ODIT_BF16 ? at::kBFloat16 : at::kHalf;
+  const int dt = code_of(*t);
+  Lin l1, l2;
+  if (dt < 0 || !c.where.holds(t) || t->dim() != 1 || !t->is_contiguous() || t->size(0) < 1 || t->size(0) > 16 ||
+      !c.linear(child(d, "linear_1"), &l1, false) || !c.linear(child(d, "linear_2"), &l2, false) || l2.k != l1.n || l1.k != dim || dim < 2 || l1.n < 1 || l2.n < 1 ||
+      l1.n >= (1ll << 30) || l2.n >= (1ll << 30))
+    return none();
+  const int M = static_cast<int>(t->size(0));
+  const auto options = t->options().dtype(c.st);
+  Tensor hidden = fresh({M, l1.n}, options), out = fresh({M, l2.n}, options);
+  const int rc = unlocked([&] {
+    const int first = odit_time_linear(t->data_ptr(), l1.w, l1.b, hidden.data_ptr(), M, static_cast<int>(l1.n), static_cast<int>(l1.k), l1.ldw, l1.n,
+                                       static_cast<float>(period), static_cast<float>(scale), static_cast<float>(pre), dt, c.dtype, c.where.stream);
+    return first != 0 ? first : odit_linear_few(hidden.data_ptr(), l2.w, l2.b, out.data_ptr(), M, static_cast<int>(l2.n), static_cast<int>(l2.k), l2.k, l2.ldw,
+                                                l2.n, c.dtype, 1, c.where.stream);
   });
   if (rc != 0) return none();
   return wrap(std::move(out));
@@ -1776,7 +1837,8 @@ PyObject* py_classes(PyObject*, PyObject* const* a, Py_ssize_t n) {
       {"Attention", &g_attention_type}, {"AttentionImpl", &g_attention_impl_type}, {"FeedForward", &g_feed_forward_type},
       {"ApproxGELU", &g_gelu_type}, {"WanFeedForward", &g_wan_ffn_type}, {"QwenImageCrossAttention", &g_qwen_attention_type},
       {"FluxAttention", &g_flux_attention_type},
-      {"AdaLayerNormZeroSingle", &g_flux_single_norm_type}, {"WanSelfAttention", &g_wan_self_type}, {"WanCrossAttention", &g_wan_cross_type}};
+      {"AdaLayerNormZeroSingle", &g_flux_single_norm_type}, {"WanSelfAttention", &g_wan_self_type}, {"WanCrossAttention", &g_wan_cross_type},
+      {"TimestepEmbedding", &g_time_embedding_type}};
   for (const auto& w : want) {
     PyObject* t = PyDict_GetItemString(a[0], w.name);
     if (t == nullptr) continue;
@@ -1815,6 +1877,8 @@ PyMethodDef kMethods[] = {
     NATIVE_FN("linear", &py_linear),
     NATIVE_FN("pair_is_small", &py_pair_is_small),
     NATIVE_FN("linear_few", &py_linear_few),
+    NATIVE_FN("linear_few_pair", &py_linear_few_pair),
+    NATIVE_FN("time_embedding", &py_time_embedding),
     NATIVE_FN("project", &py_project),
     NATIVE_FN("time_sinusoid", &py_time_sinusoid),
     NATIVE_FN("rope_tables", &py_rope_tables),

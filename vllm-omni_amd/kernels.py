@@ -739,6 +739,14 @@ def linear_few(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None 
     return torch.nn.functional.linear(silu(x) if silu_input else x, weight, bias) if done is None else done
 
 
+def linear_few_pair(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, lin: torch.nn.Module):
+    """``linear_few(x, weight, bias, silu_input=True)`` and ``project(lin, x, silu_input=True)`` in one launch; None for what the kernel
+    does not take and for a ``lin`` that is not a plain Linear module."""
+    if not x.is_cuda or not native_blocks():
+        return None
+    return (_nat or _load_native()).linear_few_pair(x, weight, bias, lin)
+
+
 def project(lin: torch.nn.Module, x: torch.Tensor, silu_input: bool = False) -> torch.Tensor:
     """lin(x) or lin(silu(x)) for a Linear module of a model's stem, conditioning or head. A plain ``nn.Linear`` in inference
     goes down as one native call; a module with hooks or of another class, and everything the kernels do not take, is called
@@ -758,6 +766,16 @@ def time_sinusoid(t: torch.Tensor, dim: int, max_period: float, scale: float, dt
     if code is None or not t.is_cuda or torch.is_grad_enabled():
         return None
     return (_nat or _load_native()).time_sinusoid(t, dim, -math.log(max_period), float(scale), code, float(pre))
+
+
+def time_embedding(embedder: torch.nn.Module, t: torch.Tensor, dim: int, max_period: float, scale: float, dtype: torch.dtype,
+                   pre: float = 1.0) -> torch.Tensor | None:
+    """``embedder`` (two Linear modules with a SiLU between) of ``time_sinusoid``'s rows, in two launches; None for what the kernels
+    do not take."""
+    code = _DTYPE_CODE.get(dtype)
+    if code is None or not t.is_cuda or not native_blocks():
+        return None
+    return (_nat or _load_native()).time_embedding(embedder, t, dim, -math.log(max_period), float(scale), code, float(pre))
 
 
 def rope_tables(txt_ids: torch.Tensor, img_ids: torch.Tensor, axes_dim: tuple[int, ...], theta: float):
