@@ -515,7 +515,10 @@ int odit_time_linear(const void* t, const void* w, const void* bias, void* out, 
  * odit_euler_step: out = x + dt * v in float32 (pipeline schedulers' step);
  * odit_gate_rows: for the n gated output projections of a model's blocks, from stacked modulation parameters mods [B, n, 3C]
  *   (dtype, 16-bit; rows dense, batch rows mods_batch_stride apart) and the projections' biases (n pointers on the host, [C] each):
- *   float32 gates [B, n, C] = the last third of every triple and gated = gates * bias. */
+ *   float32 gates [B, n, C] = the last third of every triple and gated = gates * bias;
+ * odit_pad_rows: n pieces (at most ODIT_PAD_PIECES) of dense destinations that do not overlap the sources or each other. Row r of a piece's
+ *   `rows`: `copy` bytes of src + r * src_pitch (of the byte `head` where src is null), then bytes `tail` up to `pitch`. The two branches of
+ *   classifier-free guidance stacked, the shorter prompt padded, with its key mask, are such pieces (cfg_parallel.py:28-140). */
 int odit_time_sinusoid(const void* t, void* out, int64_t n, int dim, float neg_log_period, float scale, float pre, int t_dtype,
                        int out_dtype, void* stream);
 int odit_rope_tables(const void* txt_ids, int64_t n_txt, const void* img_ids, int64_t n_img, float* cos_out, float* sin_out,
@@ -523,6 +526,14 @@ int odit_rope_tables(const void* txt_ids, int64_t n_txt, const void* img_ids, in
 int odit_cfg_combine(const void* pos, const void* neg, void* out, int64_t rows, int C, float scale, int normalize, int dtype,
                      void* stream);
 int odit_euler_step(const void* x, const void* v, void* out, int64_t n, float dt, int dtype, void* stream);
+#define ODIT_PAD_PIECES 16
+typedef struct {
+  const void* src;
+  void* dst;
+  int64_t rows, copy, src_pitch, pitch; /* bytes */
+  unsigned char head, tail;
+} odit_pad_piece;
+int odit_pad_rows(const odit_pad_piece* pieces, int n, void* stream);
 int odit_gate_rows(const void* const* bias, int n, const void* mods, int64_t mods_batch_stride, int B, int C, float* gates,
                    float* gated, int dtype, void* stream);
 

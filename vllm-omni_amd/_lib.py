@@ -137,6 +137,7 @@ _SIGNATURES = {
     "odit_cfg_combine": (
         C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_int64, C.c_int, C.c_float, C.c_int, C.c_int, C.c_void_p]),
     "odit_euler_step": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_int64, C.c_float, C.c_int, C.c_void_p]),
+    "odit_pad_rows": (C.c_int, [C.c_void_p, C.c_int, C.c_void_p]),
     "odit_gate_rows": (
         C.c_int, [C.POINTER(C.c_void_p), C.c_int, C.c_void_p, C.c_int64, C.c_int, C.c_int, C.c_void_p, C.c_void_p, C.c_int, C.c_void_p]),
     "odit_linear_rows_plan": (
@@ -169,6 +170,14 @@ class LinearProblem(C.Structure):
 
     _fields_ = [(n, C.c_void_p) for n in ("x", "w", "bias", "residual", "gate", "out")] + [("M", C.c_int), ("rows_per_gate", C.c_int)] + [
         (n, C.c_int64) for n in ("ldx", "ldw", "ldo", "ldr", "gate_stride")]
+
+
+class PadPiece(C.Structure):
+    """``odit_pad_piece``."""
+
+    _fields_ = [("src", C.c_void_p), ("dst", C.c_void_p)] + [(n, C.c_int64) for n in ("rows", "copy", "src_pitch", "pitch")] + [
+        ("head", C.c_ubyte), ("tail", C.c_ubyte)]
+
 
 class HeadOutput(C.Structure):
     """``odit_head_output``."""

@@ -250,6 +250,10 @@ def joint_key_mask(txt_mask, img_mask, B: int, S_txt: int, S_img: int, device) -
     """[B, S_txt + S_img] boolean key mask of the joint sequence from the two streams' masks (None = all true)."""
     if txt_mask is None and img_mask is None:
         return None
+    if img_mask is None and txt_mask.shape == (B, S_txt) and txt_mask.device == device:
+        out = kernels.extend_mask(txt_mask, S_img)
+        if out is not None:
+            return out
     out = torch.ones((B, S_txt + S_img), dtype=torch.bool, device=device)
     if txt_mask is not None:
         out[:, :S_txt] = txt_mask

@@ -24,6 +24,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <algorithm>
 #include <map>
 #include <optional>
 #include <utility>
@@ -591,6 +592,81 @@ PyObject* py_time_sinusoid(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (unlocked([&] { return odit_time_sinusoid(t->data_ptr(), out.data_ptr(), t->size(0), static_cast<int>(dim), static_cast<float>(period),
                          static_cast<float>(scale), static_cast<float>(pre), dt, static_cast<int>(code), w.stream); }) != 0)
     return none();
+  return wrap(std::move(out));
+  NATIVE_END
+}
+
+// Key masks and pairs of tensors stacked on the first axis, one launch. A list of (p, n): [B, S, ...] alike but for the second axis -> [2B, longer S,
+// ...], rows past a shorter S zero; or (p, n, mask of p, mask of n): masks [B, S] or None (all true) -> [2B, longer S], false past the shorter. None
+// where one is not taken.
+PyObject* py_stack_pairs(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  NATIVE_BEGIN
+  if (n != 1 || !PyList_Check(a[0]) || PyList_GET_SIZE(a[0]) < 1 || 2 * PyList_GET_SIZE(a[0]) > ODIT_PAD_PIECES) return none();
+  const Where w;
+  const Py_ssize_t count = PyList_GET_SIZE(a[0]);
+  odit_pad_piece pieces[ODIT_PAD_PIECES];
+  std::vector<Tensor> made;
+  made.reserve(count);
+  for (Py_ssize_t i = 0; i < count; ++i) {
+    PyObject* item = PyList_GET_ITEM(a[0], i);
+    if (!PyTuple_Check(item)) return none();
+    const Py_ssize_t size = PyTuple_GET_SIZE(item);
+    if (size != 2 && size != 4) return none();
+    const Tensor* half[4] = {};
+    for (Py_ssize_t j = 0; j < size; ++j) {
+      PyObject* o = PyTuple_GET_ITEM(item, j);
+      if (!optional_tensor(o, &half[j]) || (j < 2 && half[j] == nullptr)) return none();
+      if (half[j] && (!THPVariable_CheckExact(o) || !w.holds(*half[j]) || !half[j]->is_contiguous() || half[j]->numel() == 0)) return none();
+    }
+    const Tensor &p = *half[0], &q = *half[1];
+    if (code_of(p) < 0 || p.scalar_type() != q.scalar_type() || p.dim() != q.dim() || p.dim() < 1 || p.size(0) != q.size(0)) return none();
+    const bool flat = p.dim() == 1;
+    const int64_t B = flat ? 1 : p.size(0), S[2] = {flat ? p.size(0) : p.size(1), flat ? q.size(0) : q.size(1)}, longer = std::max(S[0], S[1]);
+    int64_t inner = p.element_size();
+    for (int64_t d = 2; d < p.dim(); ++d) {
+      if (p.size(d) != q.size(d)) return none();
+      inner *= p.size(d);
+    }
+    const Tensor* from[2] = {half[0], half[1]};
+    if (size == 4) {
+      if (flat) return none();
+      inner = 1;
+      for (int j = 0; j < 2; ++j) {
+        from[j] = half[2 + j];
+        if (from[j] && (from[j]->scalar_type() != at::kBool || from[j]->dim() != 2 || from[j]->size(0) != B || from[j]->size(1) != S[j])) return none();
+      }
+      made.push_back(fresh({2 * B, longer}, p.options().dtype(at::kBool)));
+    } else {
+      std::vector<int64_t> shape = p.sizes().vec();
+      shape[0] *= 2;
+      if (!flat) shape[1] = longer;
+      made.push_back(fresh(shape, p.options()));
+    }
+    const int64_t pitch = longer * inner;
+    for (int j = 0; j < 2; ++j)
+      pieces[2 * i + j] = {ptr(from[j]), static_cast<char*>(made.back().data_ptr()) + j * B * pitch, B, S[j] * inner, S[j] * inner, pitch, 1, 0};
+  }
+  if (unlocked([&] { return odit_pad_rows(pieces, 2 * static_cast<int>(count), w.stream); }) != 0) return none();
+  PyObject* r = PyTuple_New(count);
+  if (r == nullptr) return nullptr;
+  for (Py_ssize_t i = 0; i < count; ++i) PyTuple_SET_ITEM(r, i, wrap(std::move(made[i])));
+  return r;
+  NATIVE_END
+}
+
+// (bool mask [B, S], rows more) -> [B, S + more], true past S
+PyObject* py_extend_mask(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  NATIVE_BEGIN
+  const Tensor* m;
+  if (n != 2 || !(m = tensor_of(a[0]))) return none();
+  const int64_t more = PyLong_AsLong(a[1]);
+  if (PyErr_Occurred()) return nullptr;
+  const Where w;
+  if (!w.holds(m) || m->scalar_type() != at::kBool || m->dim() != 2 || m->numel() == 0 || !m->is_contiguous() || more < 0) return none();
+  const int64_t B = m->size(0), S = m->size(1);
+  Tensor out = fresh({B, S + more}, m->options());
+  const odit_pad_piece piece = {m->data_ptr(), out.data_ptr(), B, S, S, S + more, 1, 1};
+  if (unlocked([&] { return odit_pad_rows(&piece, 1, w.stream); }) != 0) return none();
   return wrap(std::move(out));
   NATIVE_END
 }
@@ -1882,6 +1958,8 @@ PyMethodDef kMethods[] = {
     NATIVE_FN("project", &py_project),
     NATIVE_FN("time_sinusoid", &py_time_sinusoid),
     NATIVE_FN("rope_tables", &py_rope_tables),
+    NATIVE_FN("stack_pairs", &py_stack_pairs),
+    NATIVE_FN("extend_mask", &py_extend_mask),
     NATIVE_FN("cfg_combine", &py_cfg_combine),
     NATIVE_FN("euler_step", &py_euler_step),
     NATIVE_FN("gate_rows", &py_gate_rows),

@@ -1,5 +1,5 @@
 // The small work around the transformer in a denoise step: the timestep sinusoid, the rotary tables of the position ids, the gate
-// rows of the blocks, the CFG combination and the Euler update.
+// rows of the blocks, the stacked branches of CFG, their combination and the Euler update.
 // Every tensor here is a few KB to a few MB, so what bounds it is the number of launches and the host time of each: as torch
 // operations the first and the last two were 10, 7 and 5 launches (about 2 us each on the GPU and 4 to 8 us on the host); here
 // each is one.
@@ -28,6 +28,50 @@ __global__ __launch_bounds__(kBlock) void time_sinusoid_kernel(const TT* __restr
     const float arg = scale * (tv * freq);
     out[row * 2 * half + j] = from_float<T>(cosf(arg));
     out[row * 2 * half + half + j] = from_float<T>(sinf(arg));
+  }
+}
+
+// Rows copied and padded, up to 16 tensors in a launch. As torch operations the branches of a CFG pair were three concatenations, with prompts of
+// unequal length ten launches, one after the other in front of a step's first projection: 19 and 58 us a step, the host's, here 10 and 11
+// (1024 latent tokens and 171 + 171, 171 + 23 text tokens of width 3584). A workgroup has kPadEach granules of one piece for each lane: the widest power of two up to 16 bytes that divides the piece's addresses and lengths.
+constexpr int kPadEach = 4;
+struct PadPiece {
+  const char* src;
+  char* dst;
+  int64_t src_pitch;
+  uint32_t granules, copy, pitch, first;  // granules in all, of a row that are copied, of a row; first workgroup
+  uint8_t log2, head, tail;
+};
+struct PadPieces {
+  PadPiece p[ODIT_PAD_PIECES];
+  int n;
+};
+template <typename V> __device__ __forceinline__ V filled(uint32_t byte) { return static_cast<V>(static_cast<uint64_t>(byte) * 0x0101010101010101ull); }
+template <> __device__ __forceinline__ u32x4 filled<u32x4>(uint32_t byte) { const uint32_t w = byte * 0x01010101u; return u32x4{w, w, w, w}; }
+template <typename V> __device__ __forceinline__ void pad_granules(const PadPiece& p, uint32_t g0) {
+  V v[kPadEach];
+#pragma unroll
+  for (int i = 0; i < kPadEach; ++i) {
+    const uint32_t g = g0 + i * kBlock, row = g / p.pitch, at = g - row * p.pitch;
+    if (g >= p.granules || at >= p.copy) v[i] = filled<V>(p.tail);
+    else if (p.src == nullptr) v[i] = filled<V>(p.head);
+    else v[i] = *reinterpret_cast<const V*>(p.src + row * p.src_pitch + static_cast<int64_t>(at) * sizeof(V));
+  }
+#pragma unroll
+  for (int i = 0; i < kPadEach; ++i)
+    if (g0 + i * kBlock < p.granules) reinterpret_cast<V*>(p.dst)[g0 + i * kBlock] = v[i];
+}
+__global__ __launch_bounds__(kBlock) void pad_rows_kernel(const PadPieces a) {
+  int i = 0;
+  while (i + 1 < a.n && blockIdx.x >= a.p[i + 1].first) ++i;  // (launch-uniform per workgroup)
+  const PadPiece& p = a.p[i];
+  const uint32_t g0 = (blockIdx.x - p.first) * (kBlock * kPadEach) + threadIdx.x;
+  switch (p.log2) {
+    case 4: pad_granules<u32x4>(p, g0); break;
+    case 3: pad_granules<uint64_t>(p, g0); break;
+    case 2: pad_granules<uint32_t>(p, g0); break;
+    case 1: pad_granules<uint16_t>(p, g0); break;
+    default: pad_granules<uint8_t>(p, g0); break;
   }
 }
 
@@ -229,6 +273,35 @@ extern "C" int odit_euler_step(const void* x, const void* v, void* out, int64_t 
     euler_step_kernel<T><<<blocks_for(n), kBlock, 0, s>>>(static_cast<const T*>(x), static_cast<const T*>(v), static_cast<T*>(out), n, dt);
   });
   return check_launch("odit_euler_step");
+}
+
+extern "C" int odit_pad_rows(const odit_pad_piece* pieces, int n, void* stream) {
+  using namespace odit;
+  ODIT_CHECK_ARG(n >= 0 && n <= ODIT_PAD_PIECES && (pieces != nullptr || n == 0), "odit_pad_rows: %d pieces, at most %d", n, ODIT_PAD_PIECES);
+  PadPieces a;
+  a.n = 0;
+  uint64_t blocks = 0;
+  for (int i = 0; i < n; ++i) {
+    const odit_pad_piece& s = pieces[i];
+    ODIT_CHECK_ARG(s.dst != nullptr && s.rows >= 0 && s.copy >= 0 && s.pitch >= s.copy && s.src_pitch >= 0, "odit_pad_rows: piece %d is bad", i);
+    if (s.rows == 0 || s.pitch == 0) continue;
+    uint64_t all = reinterpret_cast<uintptr_t>(s.dst) | static_cast<uint64_t>(s.copy) | static_cast<uint64_t>(s.pitch) | 16u;
+    if (s.src != nullptr) all |= reinterpret_cast<uintptr_t>(s.src) | static_cast<uint64_t>(s.rows > 1 ? s.src_pitch : 0);
+    const int log2 = __builtin_ctzll(all);
+    const int64_t pitch = s.pitch >> log2;
+    if (pitch >= (1ll << 31) || s.rows >= (1ll << 31) || s.rows * pitch >= (1ll << 31)) {
+      set_error("odit_pad_rows: piece %d has more than 2^31 granules", i);
+      return ODIT_ENOTSUP;
+    }
+    PadPiece& p = a.p[a.n++];
+    p = PadPiece{static_cast<const char*>(s.src), static_cast<char*>(s.dst), s.src_pitch, static_cast<uint32_t>(s.rows * pitch),
+                 static_cast<uint32_t>(s.copy >> log2), static_cast<uint32_t>(pitch), static_cast<uint32_t>(blocks), static_cast<uint8_t>(log2), s.head,
+                 s.tail};
+    blocks += (p.granules + kBlock * kPadEach - 1) / (kBlock * kPadEach);
+  }
+  if (a.n == 0) return ODIT_OK;
+  pad_rows_kernel<<<static_cast<unsigned>(blocks), kBlock, 0, static_cast<hipStream_t>(stream)>>>(a);
+  return check_launch("odit_pad_rows");
 }
 
 extern "C" int odit_gate_rows(const void* const* bias, int n, const void* mods, int64_t mods_batch_stride, int B, int C, float* gates,

@@ -159,13 +159,28 @@ def _pad_rows(t: torch.Tensor, n: int) -> torch.Tensor:
     return torch.cat([t, pad], dim=1)
 
 
+def _stacked(pair: tuple) -> torch.Tensor:
+    """One of ``kernels.stack_pairs``."""
+    if len(pair) == 2:
+        p, n = pair
+        if p.shape[1:2] != n.shape[1:2]:
+            p, n = (_pad_rows(t, max(p.shape[1], n.shape[1])) for t in pair)
+        return torch.cat([p, n], dim=0)
+    length = max(pair[0].shape[1], pair[1].shape[1])
+
+    def mask_of(m, e):
+        m = torch.ones(e.shape[:2], dtype=torch.bool, device=e.device) if m is None else m.bool()
+        return _pad_rows(m, length)   # padding rows are False
+    return torch.cat([mask_of(pair[2], pair[0]), mask_of(pair[3], pair[1])], dim=0)
+
+
 def batch_cfg_kwargs(positive: dict, negative: dict) -> dict | None:
     """One set of transformer arguments for both branches, stacked on the batch axis (positive rows first),
     or None when they cannot be stacked. Prompts of different lengths are padded to the longer one and masked
     out as keys (``encoder_hidden_states_mask``); arguments that are equal in both branches are passed once."""
     if positive.keys() != negative.keys():
         return None
-    out = {}
+    out, pairs = {}, {}  # pairs: tensors to stack
     for k, p in positive.items():
         n = negative[k]
         if k in ("encoder_hidden_states", "encoder_hidden_states_mask", "txt_seq_lens"):
@@ -173,7 +188,7 @@ def batch_cfg_kwargs(positive: dict, negative: dict) -> dict | None:
         if torch.is_tensor(p) and torch.is_tensor(n):
             if p.shape != n.shape or p.dtype != n.dtype:
                 return None
-            out[k] = torch.cat([p, n], dim=0)
+            pairs[k] = (p, n)
         elif p is None and n is None:
             out[k] = None
         elif k == "img_shapes" and isinstance(p, list) and isinstance(n, list):
@@ -189,17 +204,15 @@ def batch_cfg_kwargs(positive: dict, negative: dict) -> dict | None:
         if pe.shape[0] != ne.shape[0] or pe.shape[2:] != ne.shape[2:] or pe.dtype != ne.dtype:
             return None
         length = max(pe.shape[1], ne.shape[1])
-        out["encoder_hidden_states"] = torch.cat([_pad_rows(pe, length), _pad_rows(ne, length)], dim=0)
+        pairs["encoder_hidden_states"] = (pe, ne)
         pm, nm = positive.get("encoder_hidden_states_mask"), negative.get("encoder_hidden_states_mask")
         if pm is None and nm is None and pe.shape[1] == ne.shape[1]:
             out["encoder_hidden_states_mask"] = None
         else:
-            def mask_of(m, e):
-                m = torch.ones(e.shape[:2], dtype=torch.bool, device=e.device) if m is None else m.bool()
-                return _pad_rows(m, length)   # padding rows are False
-            out["encoder_hidden_states_mask"] = torch.cat([mask_of(pm, pe), mask_of(nm, ne)], dim=0)
+            pairs["encoder_hidden_states_mask"] = (pe, ne, pm, nm)
         if "txt_seq_lens" in positive:
-            out["txt_seq_lens"] = [length] * out["encoder_hidden_states"].shape[0]
+            out["txt_seq_lens"] = [length] * (2 * pe.shape[0])
+    out.update(zip(pairs, kernels.stack_pairs(list(pairs.values())) or map(_stacked, pairs.values())))
     return out
 
 

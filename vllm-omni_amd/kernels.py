@@ -778,6 +778,18 @@ def time_embedding(embedder: torch.nn.Module, t: torch.Tensor, dim: int, max_per
     return (_nat or _load_native()).time_embedding(embedder, t, dim, -math.log(max_period), float(scale), code, float(pre))
 
 
+def stack_pairs(pairs: list[tuple]) -> tuple[torch.Tensor, ...] | None:
+    """Each (p, n) of [B, S, ...] tensors stacked on the first axis, rows past the shorter S zero, and each (p, n, mask of p or
+    None, mask of n or None) as a key mask [2B, longer S], false past the shorter; all in one launch. None for what the kernel does
+    not take."""
+    return (_nat or _load_native()).stack_pairs(pairs) if native_blocks() else None
+
+
+def extend_mask(mask: torch.Tensor, more: int) -> torch.Tensor | None:
+    """[B, S + more] boolean mask, true past S, in one launch; None for what the kernel does not take."""
+    return (_nat or _load_native()).extend_mask(mask, more) if mask.is_cuda and native_blocks() else None
+
+
 def rope_tables(txt_ids: torch.Tensor, img_ids: torch.Tensor, axes_dim: tuple[int, ...], theta: float):
     """float32 (cos, sin) rotary tables of text ids followed by image ids, evaluated in float64, in one launch; None for what
     the kernel does not take."""
