@@ -899,24 +899,40 @@ static int launch_dma(AttnParams& p, hipStream_t stream, void* ws, size_t ws_byt
 // 32760 queries x 512 keys x 40 heads, 901 / 947). (With the two halves' roles paired wrongly, wavefronts w and
 // w + 1 or w and w + 2 in anti-phase instead of w and w + 4, the same kernel is 10 to 18 % slower: two wavefronts of a
 // SIMD in the same stage is what costs, and independent workgroups already avoid it most of the time by themselves.)
-// Since the softmax's vector work was cut the two are closer, 4 wavefronts ahead in the middle and 8 at many keys (D=128, us, 4 / 8, the
-// same bits): B=1 S=2048 H=24 56.6 / 56.2, B=2 S=2390 H=24 138.6 / 144.5, B=2 S=3276 H=40 417 / 427, B=1 S=4608 H=24 242.7 / 241.2, B=2 S=4352
-// H=24 423 / 427, with a mask 460 / 458, B=2 S=6032 H=24 797 / 818, B=1 S=8192 H=24 696 / 692, B=1 S=16384 H=40 4565 / 4500, B=2 S=32760 H=40
-// 36223 / 35657; 16384 queries x 2048 keys x 40 heads 620 / 638. The line stays where it was drawn.
+// Since the softmax's vector work was cut the two are closer, and at head size 128 (us, 4 / 8, one box, the same bits)
+//   from 128 key tiles on 8 are ahead wherever there is a round of units:  B=1 S=8192 H=24 736 / 728, B=2 1475 / 1449, S=16384 H=40 4814 / 4754,
+//     B=2 S=32760 H=40 36223 / 35657;
+//   below, 4 are, whose units are half as large: of few units every compute unit has one (B=1 S=2100 H=8, 136 units, 41.6 / 54.8, S=4096
+//     77.1 / 93.0, 700 queries x 4096 keys H=24 68.6 / 91.3), and a last round is filled better (B=1 H=40 S=2100 105 / 120, B=4 H=16 S=2500
+//     210 / 224, B=1 S=3600 H=24 174 / 195, S=6000 H=16 286 / 310, B=2 S=2390 H=24 146 / 151, 16384 queries x 2048 keys H=40 651 / 660);
+//   but with more than two rounds of 64 tiles and more it is a draw (B=2 S=4352 H=24 447 / 447, S=4808 552 / 550, S=6032 845 / 858, S=7000 H=40
+//     1845 / 1840), in whole steps too: 8. With two rounds or less whole steps are in favour of 4, B=1 S=4608 H=24 alone 256 / 253, in a Flux
+//     step 259 / 271, step 0.993; B=1 S=2706 H=40 in a step 0.995;
+//   and where 4 put two units of half the size on some compute units in the place of one whole, the anti-phase is 2 to 4 % ahead (units of 4
+//     wavefronts above one for each compute unit: B=1 S=5000 H=8, 320 units, 119.6 / 116.2, 1536 queries x 4096 keys H=24, 288, 96.3 / 93.0;
+//     cut by keys: 512 x 4096 H=24, 96, 50.0 / 46.4, 256 x 7000 H=40, 80, 59.5 / 54.9). The queries must be whole units of 8 for that: 300 x 4096
+//     H=40, 120 units, 50 / 91, 2100 x 2100 H=16, 272, 56.0 / 59.7.
 // ODIT_ATTN_WAVES in the environment, read at the first attention launch, overrides the choice (for measurements).
-static int dma_waves(int D, int Sk) {
+static int dma_waves(int B, int Sq, int Sk, int H, int D) {
   static const int forced = [] {
     const char* e = getenv("ODIT_ATTN_WAVES");
     const int v = e != nullptr ? atoi(e) : 0;
     return (v == 4 || v == 8) ? v : 0;
   }();
   if (forced != 0) return forced;
-  return (D == 128 && Sk >= 32 * 64) ? 8 : 4;
+  const int tiles = (Sk + 63) / 64;
+  if (D != 128 || tiles < 32) return 4;
+  if (tiles >= 128) return 8;
+  const int64_t heads = static_cast<int64_t>(B) * H, units = (Sq + 127) / 128 * heads;
+  const int cus = device_slots(8);
+  if (tiles >= 64 && units > 4 * cus) return 8;
+  const bool whole = 2 * ((Sq + 255) / 256 * heads) == units;
+  return whole && ((units > cus && 2 * units <= 3 * cus) || (4 * units > cus && 2 * units <= cus)) ? 8 : 4;
 }
 
 size_t attn_dma_workspace_bytes(int B, int Sq, int Sk, int H, int D) {
   if (B <= 0 || Sq <= 0 || Sk <= 0 || H <= 0) return 0;
-  const int nw = dma_waves(D, Sk);
+  const int nw = dma_waves(B, Sq, Sk, H, D);
   const int bm = nw * 32;
   const int64_t units = static_cast<int64_t>((Sq + bm - 1) / bm) * H * B;
   const int n_tiles = (Sk + 63) / 64, slots = device_slots(nw);
@@ -938,7 +954,7 @@ bool attn_dma_addressable(int Sk, int D, int64_t k_seq_stride, int64_t v_seq_str
 }
 
 int attn_dma_plan(int B, int Sq, int Sk, int H, int D, bool with_workspace, char* text, size_t text_bytes) {
-  const int nw = dma_waves(D, Sk), bm = nw * 32;
+  const int nw = dma_waves(B, Sq, Sk, H, D), bm = nw * 32;
   const int64_t units = static_cast<int64_t>((Sq + bm - 1) / bm) * H * B;
   const int n_tiles = (Sk + 63) / 64, slots = device_slots(nw);
   TailPlan t{0, 1, 0};
@@ -968,7 +984,7 @@ int attn_dma_plan(int B, int Sq, int Sk, int H, int D, bool with_workspace, char
 int launch_attn_dma(AttnParams& p, int dtype, int D, hipStream_t stream, void* ws, size_t ws_bytes) {
   if (!attn_dma_addressable(p.Sk, D, p.ks_s, p.vs_s)) return ODIT_ENOTSUP;
 #define ODIT_DMA_GO(T)                                                                     \
-  if (dma_waves(D, p.Sk) == 8) {                                                                  \
+  if (dma_waves(p.B, p.Sq, p.Sk, p.H, D) == 8) {                                           \
     if (D == 128) return launch_dma<T, 128, 8>(p, stream, ws, ws_bytes);                   \
     return launch_dma<T, 64, 8>(p, stream, ws, ws_bytes);                                  \
   }                                                                                        \
