@@ -504,6 +504,24 @@ int odit_linear_few_pair(const void* x, const void* const w[2], const void* cons
 int odit_time_linear(const void* t, const void* w, const void* bias, void* out, int M, int N, int K, int64_t ldw, int64_t ldo,
                      float neg_log_period, float scale, float pre, int t_dtype, int dtype, void* stream);
 
+/* A timestep for each of n tokens, t [n] (t_dtype): temb [n, C] = w[1] silu(w[0] rows + bias[0]) + bias[1] and proj [n, P] = w[2] silu(temb) +
+ * bias[2], where rows [n, K] are odit_time_sinusoid's (pre 1) and everything is rounded to `dtype` (wan2_2_transformer.py:282-296). Where the
+ * timesteps are at most four different ones, found on the device without a synchronisation, the products are formed once for each of them.
+ * Both outputs dense and 16-byte aligned. `scratch`: odit_time_tokens_bytes, 256-byte aligned; `workspace` as for odit_linear_rows.
+ * ODIT_ENOTSUP (nothing launched) where the second and the third product of all tokens are not for the tile kernel, or those of four rows not
+ * odit_linear_few's. */
+typedef struct {
+  const void* t;
+  const void *w[3], *bias[3];
+  int64_t ldw[3];
+  void *temb, *proj;
+  int n, K, C, P;
+  float neg_log_period, scale;
+} odit_time_tokens_args;
+size_t odit_time_tokens_bytes(int n, int K, int C, int P);
+int odit_time_tokens(const odit_time_tokens_args* args, void* scratch, size_t scratch_bytes, int t_dtype, int dtype, void* workspace,
+                     size_t workspace_bytes, void* stream);
+
 /* The small work of a denoise step, one launch each, rounded where the torch expressions of the reference round:
  * odit_time_sinusoid: t [n] (t_dtype) -> out [n, dim] (out_dtype) = cos | sin of scale * (t * exp(neg_log_period j / (dim / 2)))
  *   (diffusers Timesteps with flip_sin_to_cos, qwen_image_transformer.py:165); `pre` other than 1: t is first rounded to

@@ -1,0 +1,107 @@
+"""A timestep per token (``odit_time_tokens``): rows of distinct timesteps formed once where there are at most four, all of them otherwise."""
+
+import pytest
+import torch
+
+from vllm_omni_amd import _lib, kernels
+from vllm_omni_amd.blocks.qwen_image import QwenTimestepProjEmbeddings, TimestepEmbedding
+
+pytestmark = pytest.mark.gpu
+BF16, F16, F32 = torch.bfloat16, torch.float16, torch.float32
+
+
+def _modules(gpu, dtype, C, P, bias=True):
+    emb, proj = TimestepEmbedding(256, C).to(device=gpu, dtype=dtype), torch.nn.Linear(C, P, bias=bias, device=gpu, dtype=dtype)
+    with torch.no_grad():
+        for lin in (emb.linear_1, emb.linear_2, proj):
+            lin.weight.normal_(0, lin.in_features ** -0.5)
+    return emb, proj
+
+
+def _as_before(emb, proj, t, dtype):
+    temb = emb(QwenTimestepProjEmbeddings.time_proj(t, scale=1.0, dtype=dtype))
+    return temb, kernels.project(proj, temb, silu_input=True)
+
+
+def _in_double(emb, proj, t, dtype):
+    """With the roundings to the type that every step has."""
+    def lin(m, x):
+        return (x.double() @ m.weight.double().t() + (m.bias.double() if m.bias is not None else 0)).to(dtype)
+
+    def silu(x):
+        return torch.nn.functional.silu(x.double()).to(dtype)
+    temb = lin(emb.linear_2, silu(lin(emb.linear_1, QwenTimestepProjEmbeddings.time_proj(t, scale=1.0, dtype=dtype))))
+    return temb, lin(proj, silu(temb))
+
+
+# C a multiple of 512: the stream kernel's rows; others the matrix kernel's. 8192 and more tokens: more than one trip of the search
+@pytest.mark.parametrize("n,C,P", [(2706, 1536, 9216), (1100, 1024, 6144), (8193, 1088, 2176), (20000, 512, 3072)])
+@pytest.mark.parametrize("dtype,t_dtype,bias", [(BF16, F32, True), (F16, BF16, False)])
+@pytest.mark.parametrize("distinct", [1, 2, 3, 4, 5, 9])
+def test_distinct_timesteps(gpu, n, C, P, dtype, t_dtype, bias, distinct):
+    print(f"timesteps of {n} tokens, {distinct} distinct, {C} {P} {dtype}", flush=True)
+    torch.manual_seed(n + distinct)
+    emb, proj = _modules(gpu, dtype, C, P, bias)
+    values = (torch.randperm(900, device=gpu)[:distinct].to(t_dtype) if t_dtype == F32 else torch.arange(distinct, device=gpu).to(t_dtype) * 8)
+    t = values[torch.randint(distinct, (n,), device=gpu)]
+    t[:distinct] = values.flip(0)
+    t[n - 1] = values[0]  # (the last one alone may be the one of its kind)
+    with torch.inference_mode():
+        got = kernels.time_tokens(emb, proj, t, 256, 10000, 1.0, dtype)
+        before = _as_before(emb, proj, t, dtype)
+        for a, b in zip(got, before, strict=True):
+            # (of more distinct ones the same rows in tiles that are cut along the reduction and in whole ones differ by their order)
+            assert a.shape == b.shape and all(distinct > 4 or int(torch.unique(a[t == v], dim=0).shape[0]) == 1 for v in values)
+        # beside 64-bit sums only the elements differ whose float32 sum rounds to the type the other way, a step apart, and what follows from
+        # them: less in all than a row of which every element is a step off
+        tol = 2.0 ** -8 if dtype == BF16 else 2.0 ** -11
+        for a, b, w in zip(got, before, _in_double(emb, proj, values, dtype), strict=True):
+            for v, row in zip(values, w.double()):
+                i = int((t == v).nonzero()[0])
+                for x in (a, b):
+                    assert float((x[i].double() - row).norm() / row.norm()) < tol
+
+
+def test_bit_patterns(gpu):
+    """Infinities and NaN are timesteps like others; zeros of both signs give the same rows."""
+    emb, proj = _modules(gpu, BF16, 1536, 9216)
+    t = torch.tensor([0.0, -0.0, 700.0, 0.0], device=gpu).repeat(700)
+    with torch.inference_mode():
+        temb, rows = kernels.time_tokens(emb, proj, t, 256, 10000, 1.0, BF16)
+        assert torch.equal(temb[0], temb[1]) and torch.equal(rows[0], rows[1]) and not torch.equal(temb[0], temb[2])
+        t[5] = float("nan")
+        temb, rows = kernels.time_tokens(emb, proj, t, 256, 10000, 1.0, BF16)
+        assert bool(temb[5].isnan().all()) and bool(rows[5].isnan().all()) and int(temb.isnan().any(1).sum()) == 1 and int(rows.isnan().any(1).sum()) == 1
+
+
+def test_refused(gpu):
+    emb, proj = _modules(gpu, BF16, 1536, 9216)
+    t = torch.zeros(2706, device=gpu)
+    assert kernels.time_tokens(emb, proj, t, 256, 10000, 1.0, BF16) is None  # with gradients
+    with torch.inference_mode():
+        assert kernels.time_tokens(emb, proj, t, 256, 10000, 1.0, BF16) is not None
+        assert kernels.time_tokens(emb, proj, t[:40], 256, 10000, 1.0, BF16) is None  # not for the tile kernel
+        assert kernels.time_tokens(emb, proj, t, 256, 10000, 1.0, F16) is None
+        assert kernels.time_tokens(emb, proj, t, 128, 10000, 1.0, BF16) is None
+        proj.register_forward_hook(lambda *a: None)
+        assert kernels.time_tokens(emb, proj, t, 256, 10000, 1.0, BF16) is None
+    lib, a = _lib.load(), _lib.TimeTokens()
+    assert lib.odit_time_tokens(_lib.C.addressof(a), None, 0, _lib.ODIT_F32, _lib.ODIT_BF16, None, 0, None) == -1
+    assert lib.odit_time_tokens_bytes(0, 256, 1536, 9216) == 0
+
+
+def test_captured(gpu):
+    """Which way the rows come is found when the graph runs."""
+    emb, proj = _modules(gpu, BF16, 1536, 9216)
+    t = torch.zeros(2706, device=gpu)
+    with torch.inference_mode():
+        kernels.time_tokens(emb, proj, t, 256, 10000, 1.0, BF16)
+        graph, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+        with torch.cuda.graph(graph, stream=stream):
+            temb, rows = kernels.time_tokens(emb, proj, t, 256, 10000, 1.0, BF16)
+        for distinct in (1, 3, 700, 2, 5):
+            t.copy_(torch.arange(2706, device=gpu) % distinct)
+            graph.replay()
+            want = kernels.time_tokens(emb, proj, t, 256, 10000, 1.0, BF16)
+            torch.cuda.synchronize()
+            assert torch.equal(temb, want[0]) and torch.equal(rows, want[1])

@@ -129,6 +129,9 @@ _SIGNATURES = {
     "odit_time_linear": (
         C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_int64, C.c_int64, C.c_float, C.c_float,
                   C.c_float, C.c_int, C.c_int, C.c_void_p]),
+    "odit_time_tokens_bytes": (C.c_size_t, [C.c_int] * 4),
+    "odit_time_tokens": (
+        C.c_int, [C.c_void_p, C.c_void_p, C.c_size_t, C.c_int, C.c_int, C.c_void_p, C.c_size_t, C.c_void_p]),
     "odit_time_sinusoid": (
         C.c_int, [C.c_void_p, C.c_void_p, C.c_int64, C.c_int, C.c_float, C.c_float, C.c_float, C.c_int, C.c_int, C.c_void_p]),
     "odit_rope_tables": (
@@ -170,6 +173,13 @@ class LinearProblem(C.Structure):
 
     _fields_ = [(n, C.c_void_p) for n in ("x", "w", "bias", "residual", "gate", "out")] + [("M", C.c_int), ("rows_per_gate", C.c_int)] + [
         (n, C.c_int64) for n in ("ldx", "ldw", "ldo", "ldr", "gate_stride")]
+
+
+class TimeTokens(C.Structure):
+    """``odit_time_tokens_args``."""
+
+    _fields_ = [("t", C.c_void_p), ("w", C.c_void_p * 3), ("bias", C.c_void_p * 3), ("ldw", C.c_int64 * 3), ("temb", C.c_void_p), ("proj", C.c_void_p)] + [
+        (n, C.c_int) for n in ("n", "K", "C", "P")] + [("neg_log_period", C.c_float), ("scale", C.c_float)]
 
 
 class PadPiece(C.Structure):

@@ -425,12 +425,16 @@ class WanTimeTextImageEmbedding(nn.Module):
                 encoder_hidden_states_image: torch.Tensor | None = None, timestep_seq_len: int | None = None):
         """timestep [B] -> temb [B,C], timestep_proj [B,6C]; flattened per-token timesteps [B*S] with
         ``timestep_seq_len`` = S -> temb [B,S,C], timestep_proj [B,S,6C] (wan.py:282-296)."""
-        t = QwenTimestepProjEmbeddings.time_proj(timestep, dim=self.time_freq_dim, scale=1.0,
-                                                 dtype=self.time_embedder.linear_1.weight.dtype)
-        if timestep_seq_len is not None:
-            t = t.unflatten(0, (-1, timestep_seq_len))
-        mlp = self.time_embedder
-        if encoder_hidden_states.shape[0] == 1:
+        mlp, dtype, done = self.time_embedder, self.time_embedder.linear_1.weight.dtype, None
+        if timestep_seq_len is not None and encoder_hidden_states.shape[0] == 1 and encoder_hidden_states.dtype == dtype:
+            done = kernels.time_tokens(mlp, self.time_proj, timestep, self.time_freq_dim, 10000, 1.0, dtype)
+        if done is None:
+            t = QwenTimestepProjEmbeddings.time_proj(timestep, dim=self.time_freq_dim, scale=1.0, dtype=dtype)
+            if timestep_seq_len is not None:
+                t = t.unflatten(0, (-1, timestep_seq_len))
+        if done is not None:
+            temb, timestep_proj = (x.unflatten(0, (-1, timestep_seq_len)) for x in done)
+        elif encoder_hidden_states.shape[0] == 1:
             temb = mlp(t).type_as(encoder_hidden_states)
             timestep_proj = kernels.project(self.time_proj, temb, silu_input=True)
         else:  # a batch keeps the library's order of summation, as its blocks do (csrc/native.cpp, the Wan block)

@@ -29,7 +29,7 @@ NATIVE_PATH = PKG / "_native.so"
 OBJ_DIR = CSRC / "build"
 HEADERS = [CSRC / "odit_common.h", CSRC / "attn_common.h", CSRC / "attn_tail.h", CSRC / "gemm_bf16.h",
            CSRC / "gemm_epilogue.h", CSRC / "gemm_tile.h",
-           CSRC / "gemm_heads.h", CSRC / "gemm_small.h", PKG.parent / "include" / "omni_dit.h"]
+           CSRC / "gemm_heads.h", CSRC / "gemm_small.h", CSRC / "time_sinusoid.h", CSRC / "time_tokens.h", PKG.parent / "include" / "omni_dit.h"]
 
 # (source file, extra defines, object stem)
 UNITS: list[tuple[str, list[str], str]] = [
@@ -45,9 +45,11 @@ UNITS: list[tuple[str, list[str], str]] = [
     ("linear.hip", [], "linear"),
     ("linear_few.hip", [], "linear_few"),
     ("step.hip", [], "step"),
+    ("time_tokens.hip", [], "time_tokens"),
     ("gemm_bf16.hip", [], "gemm_bf16"),
     ("gemm_bf16_tile.hip", [], "gemm_bf16_tile"),
     ("gemm_tile_heads.hip", [], "gemm_tile_heads"),
+    ("gemm_tile_unless.hip", [], "gemm_tile_unless"),
     ("gemm_small.hip", [], "gemm_small"),
     ("gemm_small_heads.hip", [], "gemm_small_heads"),
     ("gemm_small_norm.hip", [], "gemm_small_norm"),

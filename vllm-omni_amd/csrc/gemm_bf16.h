@@ -69,6 +69,8 @@ TilePlan plan_gemm_tile(const GemmCall* c, int count, int cus, bool scratch);
 // One problem, or two or three of the same K in one launch. `scratch` as for launch_gemm_streamk, or null (no tile is cut). `x2`: with
 // one problem only.
 int launch_gemm_tile(const GemmCall* c, int count, const TileX2* x2, int dtype, void* scratch, hipStream_t stream);
+// gemm_tile_unless.hip: one problem, and nothing where *unless (device memory) is not 0 when the launch begins
+int launch_gemm_tile_unless(const GemmCall& c, const int* unless, int dtype, void* scratch, hipStream_t stream);
 
 // ---- gemm_tile_heads.hip: the tile kernel with query, key and value heads at its end -------
 // Output of a projection to 3 HD features: per batch entry S rows of queries, keys and values of HD / D heads, the first two normed

@@ -65,13 +65,13 @@ int launch_gemm_tile(const GemmCall* c, int count, const TileX2* x2, int dtype, 
   const int cus = device_cus();
   if (cus <= 0) { set_error("odit_linear: cannot read the device's compute-unit count"); return ODIT_ELAUNCH; }
   const TilePlan plan = plan_gemm_tile(c, count, cus, scratch != nullptr);
-  TileArgs<false> p;
+  TileArgs<false, false> p;
   fill_tile_params(p, plan, c, count, x2, scratch);
   const dim3 grid(plan.grid), block(512);
 #define ODIT_TILE(T)                                                                          \
   do {                                                                                        \
-    if (plan.bm == 256) hipLaunchKernelGGL((gemm_tile_kernel<T, 4, false>), grid, block, 0, stream, p); \
-    else hipLaunchKernelGGL((gemm_tile_kernel<T, 2, false>), grid, block, 0, stream, p);              \
+    if (plan.bm == 256) hipLaunchKernelGGL((gemm_tile_kernel<T, 4, false, false>), grid, block, 0, stream, p); \
+    else hipLaunchKernelGGL((gemm_tile_kernel<T, 2, false, false>), grid, block, 0, stream, p);              \
   } while (0)
   if (dtype == ODIT_BF16) ODIT_TILE(bf16_t);
   else ODIT_TILE(f16_t);

@@ -80,9 +80,12 @@ struct TileParams {
   char* slots;
 };
 
-template <bool HEADS> struct TileArgs : TileParams {};
-template <> struct TileArgs<true> : TileParams {
+template <bool HEADS, bool UNLESS> struct TileArgs : TileParams {};
+template <> struct TileArgs<true, false> : TileParams {
   HeadsOut heads[2];  // of the two problems (there are no three with heads); q null: an ordinary output
+};
+template <> struct TileArgs<false, true> : TileParams {
+  const int* unless;
 };
 
 typedef __attribute__((address_space(3))) void* lds_void_p;
@@ -236,9 +239,10 @@ __device__ __forceinline__ void store_heads(const HeadsOut& h, const u32x4 (&v)[
 }
 
 // MH: 16-row accumulators of a wavefront in each half of the rows (4: 256-row tiles, 2: 128). HEADS: the form for problems whose
-// output is query, key and value heads, beside ordinary ones without a gate.
-template <typename T, int MH, bool HEADS>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_tile_kernel(const TileArgs<HEADS> p) {
+// output is query, key and value heads, beside ordinary ones without a gate. UNLESS: nothing is done where a word of device memory is not 0 (a
+// form of its own, as the test made the others up to 0.6 % slower: M=1536, N=12288, K=3072 109.7 / 110.4 us).
+template <typename T, int MH, bool HEADS, bool UNLESS>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_tile_kernel(const TileArgs<HEADS, UNLESS> p) {
   using M = Mma16<T>;
   using frag = typename M::frag;
   constexpr int BM = 64 * MH, HM = 32 * MH;           // rows of a tile, of a half
@@ -256,6 +260,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int G = gridDim.x;
   const int v = xcd_remap(blockIdx.x, G);
   const int nk = p.k_steps;
+  if constexpr (UNLESS) {
+    if (*p.unless != 0) return;  // (the whole launch: no ticket is drawn)
+  }
 
   auto make_rsrc = [](const void* base, uint32_t bytes) __attribute__((always_inline)) {
     const uint64_t a = reinterpret_cast<uint64_t>(base);

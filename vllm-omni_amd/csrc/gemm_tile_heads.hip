@@ -15,7 +15,7 @@ int launch_gemm_tile_heads(const GemmCall* c, int count, const HeadsOut* heads, 
   const int cus = device_cus();
   if (cus <= 0) { set_error("odit_linear_heads: cannot read the device's compute-unit count"); return ODIT_ELAUNCH; }
   const TilePlan plan = plan_gemm_tile(c, count, cus, scratch != nullptr);
-  TileArgs<true> p;
+  TileArgs<true, false> p;
   fill_tile_params(p, plan, c, count, nullptr, scratch);
   for (int i = 0; i < 2; ++i) {
     HeadsOut& h = p.heads[i];
@@ -25,8 +25,8 @@ int launch_gemm_tile_heads(const GemmCall* c, int count, const HeadsOut* heads, 
   const dim3 grid(plan.grid), block(512);
 #define ODIT_TILE(T)                                                                                \
   do {                                                                                              \
-    if (plan.bm == 256) hipLaunchKernelGGL((gemm_tile_kernel<T, 4, true>), grid, block, 0, stream, p); \
-    else hipLaunchKernelGGL((gemm_tile_kernel<T, 2, true>), grid, block, 0, stream, p);              \
+    if (plan.bm == 256) hipLaunchKernelGGL((gemm_tile_kernel<T, 4, true, false>), grid, block, 0, stream, p); \
+    else hipLaunchKernelGGL((gemm_tile_kernel<T, 2, true, false>), grid, block, 0, stream, p);              \
   } while (0)
   if (dtype == ODIT_BF16) ODIT_TILE(bf16_t);
   else ODIT_TILE(f16_t);

@@ -16,6 +16,7 @@
 // D's rows, i.e. along the N output features, as needed.
 #include "odit_common.h"
 #include "gemm_bf16.h"
+#include "time_tokens.h"
 
 #include <hipblaslt/hipblaslt.h>
 #include <hipblaslt/hipblaslt-ext.hpp>
@@ -582,6 +583,23 @@ static int lin_rule_kind(const odit::LinCall& c, const odit::GemmCall& g, const 
 static int lin_auto_kind(int dev, const odit::LinCall& c, const odit::GemmCall& g, const void* sk) {
   odit::Tuned found;
   return lin_tuned(dev, c, g, sk, &found) ? found.kind : lin_rule_kind(c, g, sk);
+}
+
+int odit::linear_tile_unless(const void* x, const void* w, const void* bias, void* out, int M, int N, int K, int64_t ldw, int dtype, void* workspace,
+                             size_t workspace_bytes, const int* unless, bool ask, hipStream_t stream) {
+  void *sk, *lib;
+  size_t lib_bytes;
+  lin_split_ws(workspace, workspace_bytes, &sk, &lib, &lib_bytes);
+  const LinCall c{x, w, bias, nullptr, nullptr, out, M, N, K, K, ldw, N, 0, bias != nullptr ? ODIT_EPI_BIAS : ODIT_EPI_NONE, dtype, dtype, lib, lib_bytes, stream};
+  const int rc = lin_check(c);
+  if (rc != ODIT_OK) return rc;
+  const GemmCall g = lin_gemm_call(c, 0, 0);
+  int dev = 0;
+  if (M < kTileMinAuto || !gemm_tile_takes(g, dtype) || hipGetDevice(&dev) != hipSuccess) return ODIT_ENOTSUP;
+  // a launch that mostly ends at once may be behind the best one by a little where it does not
+  const TilePlan plan = plan_gemm_tile(&g, 1, device_cus(), sk != nullptr);
+  if (plan.bm == 0 || plan.us > 1.15f * lin_call_us(dev, c, g, sk)) return ODIT_ENOTSUP;
+  return ask ? ODIT_OK : launch_gemm_tile_unless(g, unless, dtype, sk, stream);
 }
 
 extern "C" int odit_linear_prefer(int M, int N, int K, int dtype, int solution) {

@@ -29,6 +29,8 @@
 // operations): 3072 features, K=256 5.8 / 4.3, the launch less.
 #include "odit_common.h"
 #include "gemm_bf16.h"
+#include "time_sinusoid.h"
+#include "time_tokens.h"
 
 namespace odit {
 namespace {
@@ -80,17 +82,11 @@ template <typename TT> struct Sinusoid {
 };
 template <typename T, typename TT>
 __device__ __forceinline__ void stage_sinusoid(const Sinusoid<TT>& a, u32x4* xs, int rows, int K, int pitch) {
-#pragma clang fp contract(off)
   const int half = K / 2;
   T* const to = reinterpret_cast<T*>(xs);
   for (int i = threadIdx.x; i < rows * half; i += kWaves * 64) {
     const int m = i / half, j = i - m * half;
-    const float freq = expf(a.neg_log_period * static_cast<float>(j) / static_cast<float>(half));
-    float tv = to_float(a.t[m]);
-    if (a.pre != 1.f) tv = round_to<T>(round_to<T>(tv) * a.pre);
-    const float arg = a.scale * (tv * freq);
-    to[m * pitch * 8 + j] = from_float<T>(cosf(arg));
-    to[m * pitch * 8 + half + j] = from_float<T>(sinf(arg));
+    time_sinusoid<T>(a.t[m], j, half, a.neg_log_period, a.scale, a.pre, to[m * pitch * 8 + j], to[m * pitch * 8 + half + j]);
   }
 }
 
@@ -177,18 +173,22 @@ __device__ __forceinline__ void few_rows(Stage&& stage, const FewOut<T>& o0, con
 
 template <typename T, bool SILU, bool PAIR>
 __global__ __launch_bounds__(kWaves * 64, 6) void linear_few_kernel(const T* __restrict__ x, const FewOut<T> o0, const FewOut<T> o1, int M, int K,
-                                                                    int64_t ldx, int tiles0, int tiles) {
+                                                                    int64_t ldx, int tiles0, int tiles, const int* only_if) {
+  if (only_if != nullptr && *only_if == 0) return;
   few_rows<T, PAIR>([&](u32x4* xs, int vecs, int pitch) { stage_rows<T, SILU>(x, xs, M, vecs, pitch, ldx); }, o0, o1, M, K, tiles0, tiles);
 }
 template <typename T, typename TT>
-__global__ __launch_bounds__(kWaves * 64, 6) void linear_few_sinusoid_kernel(const Sinusoid<TT> a, const FewOut<T> o, int M, int K, int tiles) {
+__global__ __launch_bounds__(kWaves * 64, 6) void linear_few_sinusoid_kernel(const Sinusoid<TT> a, const FewOut<T> o, int M, int K, int tiles,
+                                                                             const int* only_if) {
+  if (only_if != nullptr && *only_if == 0) return;
   few_rows<T, false>([&](u32x4* xs, int, int pitch) { stage_sinusoid<T, TT>(a, xs, M, K, pitch); }, o, o, M, K, tiles, tiles);
 }
 
 // (groups of R features; those of the first weight come first)
 template <typename T, bool SILU, int M, int R, bool PAIR>
 __global__ __launch_bounds__(kWaves * 64, 6) void linear_stream_kernel(const T* __restrict__ x, const FewOut<T> o0, const FewOut<T> o1, int rows, int K,
-                                                                       int64_t ldx) {
+                                                                       int64_t ldx, const int* only_if) {
+  if (only_if != nullptr && *only_if == 0) return;
   extern __shared__ u32x4 lds[];
   const int vecs = K / 8;
   stage_rows<T, SILU>(x, lds, rows, vecs, vecs, ldx);
@@ -269,13 +269,13 @@ __global__ __launch_bounds__(kWaves * 64, 6) void linear_stream_kernel(const T* 
 constexpr int kStreamWide = 1 << 16;
 
 template <typename T, bool SILU, bool PAIR>
-int launch_stream(const T* x, const FewOut<T>& o0, const FewOut<T>& o1, int M, int K, int64_t ldx, int slots, hipStream_t stream) {
+int launch_stream(const T* x, const FewOut<T>& o0, const FewOut<T>& o1, int M, int K, int64_t ldx, int slots, const int* only_if, hipStream_t stream) {
   const size_t lds = static_cast<size_t>(M) * K * 2;
   const int N = o0.N + (PAIR ? o1.N : 0);
 #define ODIT_STREAM(ROWS, R)                                                                                                             \
   do {                                                                                                                                   \
     const int groups = (o0.N + R - 1) / R + (PAIR ? (o1.N + R - 1) / R : 0), wanted = (groups + kWaves - 1) / kWaves;                      \
-    linear_stream_kernel<T, SILU, ROWS, R, PAIR><<<wanted < slots ? wanted : slots, kWaves * 64, lds, stream>>>(x, o0, o1, M, K, ldx);     \
+    linear_stream_kernel<T, SILU, ROWS, R, PAIR><<<wanted < slots ? wanted : slots, kWaves * 64, lds, stream>>>(x, o0, o1, M, K, ldx, only_if); \
   } while (0)
   if (M > 2) ODIT_STREAM(4, 2);
   else if (N >= kStreamWide && M == 2) ODIT_STREAM(2, 4);
@@ -291,6 +291,9 @@ int launch_stream(const T* x, const FewOut<T>& o0, const FewOut<T>& o1, int M, i
 constexpr int kFewMaxRows = 16, kFewMaxGroups = 3, kStreamMaxRows = 4;
 constexpr size_t kFewMaxLds = 160 * 1024;
 
+// whether a reduction is the stream kernel's
+bool few_streams(int M, int K) { return M <= kStreamMaxRows && K % 512 == 0 && static_cast<size_t>(M) * K * 2 <= kFewMaxLds / kFewMaxGroups; }
+
 size_t few_lds(int M, int K) { return kRedBytes + static_cast<size_t>(M) * (K / 8 + 1) * 16; }
 int few_grid(int tiles, size_t lds, int cus) {
   const int fit = static_cast<int>(kFewMaxLds / lds), slots = cus * (fit < kFewMaxGroups ? fit : kFewMaxGroups);
@@ -302,25 +305,27 @@ struct FewArgs { const void *w, *bias; void* out; int N; int64_t ldw, ldo; };
 // How many rows a wavefront takes at a time follows from the features
 // of both; the bits do not (a feature's sum is one wavefront's).
 template <typename T, bool SILU, bool PAIR>
-int run_few(const void* x, const FewArgs* a, int M, int K, int64_t ldx, int cus, hipStream_t stream) {
+int run_few(const void* x, const FewArgs* a, int M, int K, int64_t ldx, int cus, hipStream_t stream, const int* only_if = nullptr) {
   FewOut<T> o[2];
   for (int i = 0; i < 2; ++i)  // (without a second weight nothing reads the second)
     o[i] = FewOut<T>{static_cast<const T*>(a[i].w), static_cast<const T*>(a[i].bias), static_cast<T*>(a[i].out), a[i].ldw, a[i].ldo, a[i].N};
-  if (M <= kStreamMaxRows && K % 512 == 0 && static_cast<size_t>(M) * K * 2 <= kFewMaxLds / kFewMaxGroups)
-    return launch_stream<T, SILU, PAIR>(static_cast<const T*>(x), o[0], o[1], M, K, ldx, cus * kFewMaxGroups, stream);
+  if (few_streams(M, K))
+    return launch_stream<T, SILU, PAIR>(static_cast<const T*>(x), o[0], o[1], M, K, ldx, cus * kFewMaxGroups, only_if, stream);
   const int tiles0 = (a[0].N + kTile - 1) / kTile, tiles = tiles0 + (PAIR ? (a[1].N + kTile - 1) / kTile : 0);
   const size_t lds = few_lds(M, K);
-  linear_few_kernel<T, SILU, PAIR><<<few_grid(tiles, lds, cus), kWaves * 64, lds, stream>>>(static_cast<const T*>(x), o[0], o[1], M, K, ldx, tiles0, tiles);
+  linear_few_kernel<T, SILU, PAIR><<<few_grid(tiles, lds, cus), kWaves * 64, lds, stream>>>(static_cast<const T*>(x), o[0], o[1], M, K, ldx, tiles0, tiles,
+                                                                                                          only_if);
   return check_launch("odit_linear_few");
 }
 
 template <typename T, typename TT>
-int run_sinusoid(const void* t, float neg_log_period, float scale, float pre, const FewArgs& a, int M, int K, int cus, hipStream_t stream) {
+int run_sinusoid(const void* t, float neg_log_period, float scale, float pre, const FewArgs& a, int M, int K, int cus, hipStream_t stream,
+                 const int* only_if = nullptr) {
   const FewOut<T> o{static_cast<const T*>(a.w), static_cast<const T*>(a.bias), static_cast<T*>(a.out), a.ldw, a.ldo, a.N};
   const int tiles = (a.N + kTile - 1) / kTile;
   const size_t lds = few_lds(M, K);
   linear_few_sinusoid_kernel<T, TT><<<few_grid(tiles, lds, cus), kWaves * 64, lds, stream>>>(
-      Sinusoid<TT>{static_cast<const TT*>(t), neg_log_period, scale, pre}, o, M, K, tiles);
+      Sinusoid<TT>{static_cast<const TT*>(t), neg_log_period, scale, pre}, o, M, K, tiles, only_if);
   return check_launch("odit_time_linear");
 }
 
@@ -363,6 +368,31 @@ static int few_go(const char* name, const void* x, odit::FewArgs (&a)[2], int co
 #undef ODIT_FEW
 }
 
+int odit::linear_few_if(const void* x, const void* w, const void* bias, void* out, int M, int N, int K, int64_t ldw, int dtype, const int* only_if, bool ask,
+                        hipStream_t stream) {
+  const FewArgs a[2] = {{w, bias, out, N, ldw, N}, {}};
+  const int rc = few_check("odit_linear_few", a, 1, M, K, dtype);
+  if (rc != ODIT_OK || ask) return rc;
+  const int cus = device_cus();
+  if (cus <= 0) { set_error("odit_linear_few: cannot read the device's compute-unit count"); return ODIT_ELAUNCH; }
+  return dtype == ODIT_BF16 ? run_few<bf16_t, true, false>(x, a, M, K, K, cus, stream, only_if)
+                            : run_few<f16_t, true, false>(x, a, M, K, K, cus, stream, only_if);
+}
+
+int odit::time_linear_if(const void* t, const void* w, const void* bias, void* out, int M, int N, int K, int64_t ldw, float neg_log_period, float scale,
+                         int t_dtype, int dtype, const int* only_if, bool ask, hipStream_t stream) {
+  const FewArgs a{w, bias, out, N, ldw, N};
+  const int rc = few_check("odit_time_linear", &a, 1, M, K, dtype);
+  if (rc != ODIT_OK || ask) return rc;
+  const int cus = device_cus();
+  if (cus <= 0) { set_error("odit_time_linear: cannot read the device's compute-unit count"); return ODIT_ELAUNCH; }
+  ODIT_DISPATCH_DTYPE(t_dtype, TT, {
+    return dtype == ODIT_BF16 ? run_sinusoid<bf16_t, TT>(t, neg_log_period, scale, 1.f, a, M, K, cus, stream, only_if)
+                              : run_sinusoid<f16_t, TT>(t, neg_log_period, scale, 1.f, a, M, K, cus, stream, only_if);
+  });
+  return ODIT_OK;
+}
+
 extern "C" int odit_linear_few(const void* x, const void* w, const void* bias, void* out, int M, int N, int K, int64_t ldx,
                                int64_t ldw, int64_t ldo, int dtype, int silu_input, void* stream) {
   odit::FewArgs a[2] = {{w, bias, out, N, ldw, ldo}, {}};
@@ -387,7 +417,7 @@ extern "C" int odit_time_linear(const void* t, const void* w, const void* bias, 
   const int rc = few_check("odit_time_linear", &a, 1, M, K, dtype);
   if (rc != ODIT_OK) return rc;
   // (a reduction that the stream kernel would take has another order of summation)
-  if (M <= kStreamMaxRows && K % 512 == 0 && static_cast<size_t>(M) * K * 2 <= kFewMaxLds / kFewMaxGroups) {
+  if (few_streams(M, K)) {
     set_error("odit_time_linear: K=%d is the stream kernel's", K);
     return ODIT_ENOTSUP;
   }

@@ -1113,6 +1113,47 @@ PyObject* py_time_embedding(PyObject*, PyObject* const* a, Py_ssize_t n) {
   NATIVE_END
 }
 
+// (TimestepEmbedding, plain Linear time_proj, t [n], cosines and sines, - ln of the longest period, scale, type code of the rows) ->
+// (linear_2(silu(linear_1(sinusoid of t))) [n, C], time_proj(silu of that) [n, P])
+PyObject* py_time_tokens(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  NATIVE_BEGIN
+  const Tensor* t;
+  PyObject* const d = n == 7 && g_linear_type != nullptr && g_time_embedding_type != nullptr ? plain_module(a[0], g_time_embedding_type) : nullptr;
+  if (d == nullptr || !(t = tensor_of(a[2]))) return none();
+  const long dim = PyLong_AsLong(a[3]), code = PyLong_AsLong(a[6]);
+  const double period = PyFloat_AsDouble(a[4]), scale = PyFloat_AsDouble(a[5]);
+  if (PyErr_Occurred()) return nullptr;
+  if (code != ODIT_BF16 && code != ODIT_F16) return none();
+  BlockCall c;
+  c.dtype = static_cast<int>(code);
+  c.st = code == ODIT_BF16 ? at::kBFloat16 : at::kHalf;
+  const int dt = code_of(*t);
+  Lin l[3];
+  if (dt < 0 || !c.where.holds(t) || t->dim() != 1 || !t->is_contiguous() || t->size(0) < 1 || t->size(0) >= (1 << 30) ||
+      !c.linear(child(d, "linear_1"), &l[0], false) || !c.linear(child(d, "linear_2"), &l[1], false) || !c.linear(a[1], &l[2], false) || l[0].k != dim ||
+      dim < 2 || l[1].k != l[0].n || l[1].n != l[0].n || l[2].k != l[1].n || l[0].n < 1 || l[2].n < 1 || l[0].n >= (1 << 30) || l[2].n >= (1 << 30))
+    return none();
+  if (!linear_scratch(c.where, &c.lin_ws)) return nullptr;
+  const int N = static_cast<int>(t->size(0)), C = static_cast<int>(l[1].n), P = static_cast<int>(l[2].n);
+  const auto options = t->options().dtype(c.st);
+  const size_t bytes = odit_time_tokens_bytes(N, static_cast<int>(dim), C, P);
+  Tensor temb = fresh({N, C}, options), proj = fresh({N, P}, options), scratch = fresh({static_cast<int64_t>(bytes)}, t->options().dtype(at::kByte));
+  odit_time_tokens_args args = {};
+  args.t = t->data_ptr();
+  for (int i = 0; i < 3; ++i) { args.w[i] = l[i].w; args.bias[i] = l[i].b; args.ldw[i] = l[i].ldw; }
+  args.temb = temb.data_ptr();
+  args.proj = proj.data_ptr();
+  args.n = N;
+  args.K = static_cast<int>(dim);
+  args.C = C;
+  args.P = P;
+  args.neg_log_period = static_cast<float>(period);
+  args.scale = static_cast<float>(scale);
+  if (unlocked([&] { return odit_time_tokens(&args, scratch.data_ptr(), bytes, dt, c.dtype, c.lin_ws.p, c.lin_ws.bytes, c.where.stream); }) != 0) return none();
+  return wrap2(std::move(temb), std::move(proj));
+  NATIVE_END
+}
+
 // a gate row per batch entry (and, in the pre-scaled form, the gate times the projection's bias), or no gate at all
 struct Gate {
   const void* gate = nullptr;   // element type `dtype`, or float32 when pre
@@ -1955,6 +1996,7 @@ PyMethodDef kMethods[] = {
     NATIVE_FN("linear_few", &py_linear_few),
     NATIVE_FN("linear_few_pair", &py_linear_few_pair),
     NATIVE_FN("time_embedding", &py_time_embedding),
+    NATIVE_FN("time_tokens", &py_time_tokens),
     NATIVE_FN("project", &py_project),
     NATIVE_FN("time_sinusoid", &py_time_sinusoid),
     NATIVE_FN("rope_tables", &py_rope_tables),

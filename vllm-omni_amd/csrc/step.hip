@@ -5,6 +5,7 @@
 // each is one.
 // Every intermediate is rounded where the torch expression rounds it, with no contraction of multiply and add.
 #include "odit_common.h"
+#include "time_sinusoid.h"
 
 #pragma clang fp contract(off)
 
@@ -14,20 +15,14 @@ namespace {
 constexpr int kBlock = 256;
 constexpr int kMaxBlocks = 4096;
 
-// out[i, :] = cos | sin of scale * (t[i] * exp(-log(max_period) j / half)); the accurate exp, cos and sin, which torch calls.
-// `pre` other than 1 is a factor that the caller's expression applies in T before it (Flux: timestep.to(T) * 1000).
+// out[i, :] = cos | sin (time_sinusoid.h) of every frequency
 template <typename TT, typename T>
 __global__ __launch_bounds__(kBlock) void time_sinusoid_kernel(const TT* __restrict__ t, T* __restrict__ out, int64_t n, int half,
                                                                float neg_log_period, float scale, float pre) {
   for (int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x; i < n * half; i += static_cast<int64_t>(gridDim.x) * kBlock) {
     const int64_t row = i / half;
     const int j = static_cast<int>(i - row * half);
-    const float freq = expf(neg_log_period * static_cast<float>(j) / static_cast<float>(half));
-    float tv = to_float(t[row]);
-    if (pre != 1.f) tv = round_to<T>(round_to<T>(tv) * pre);
-    const float arg = scale * (tv * freq);
-    out[row * 2 * half + j] = from_float<T>(cosf(arg));
-    out[row * 2 * half + half + j] = from_float<T>(sinf(arg));
+    time_sinusoid<T>(t[row], j, half, neg_log_period, scale, pre, out[row * 2 * half + j], out[row * 2 * half + half + j]);
   }
 }
 

@@ -1,0 +1,252 @@
+// Timestep embedding and modulation parameters of a timestep per token: temb = linear_2(silu(linear_1(sinusoid of t))), proj =
+// time_proj(silu(temb)) for n tokens. Where an image or a first frame is given, its tokens have one timestep and the others
+// another, and n rows of these projections are two rows over and over (width 5120, 2706 tokens: 1 TFLOP, 770 us, an eighth of a
+// step of three blocks). So the distinct timesteps are found on the device (up to kRows, no synchronisation), those rows go
+// through the kernels for few rows, which stream the weights once, and are spread out over the tokens: 80 us for the products and
+// 31 for the 190 MB that are written. The launches for all tokens follow as ever, and end at once where the first ones have done
+// the work. us, before / two timesteps / all different: n=1000, width 5120 350 / 117 / 348; 2706, 5120 770 / 134 / 799; 9000, 3072
+// 918 / 134 / 953; 32760, 5120 8488 / 667 / 8507: where tokens have more timesteps the search and six launches that end at once
+// are 20 to 35 us.
+#include "gemm_bf16.h"
+#include "time_sinusoid.h"
+#include "time_tokens.h"
+
+namespace odit {
+namespace {
+
+constexpr int kRows = 4;  // what linear_stream_kernel takes at a time
+constexpr int kThreads = 1024, kEach = 8;
+
+// What the device knows of the timesteps: `few` distinct ones, or 0 of them where there are more than kRows. `value`: they, padded with the first.
+struct TimeGroups {
+  int few;
+  int pad[3];
+  float value[kRows];  // (of the timesteps' type, from the first byte)
+};
+constexpr size_t kHeadBytes = 256;  // (every part on whole cache lines: rows 64 bytes off made the products 16 % slower)
+static_assert(sizeof(TimeGroups) <= kHeadBytes, "");
+
+// One workgroup: the first timestep that is none of those found so far, until there is none. `index`: each token's number among them.
+template <typename TT, typename Bits>
+__global__ __launch_bounds__(kThreads) void time_groups_kernel(const Bits* __restrict__ t, int n, TimeGroups* __restrict__ g, int* __restrict__ index) {
+  __shared__ int first[kRows + 1];
+  __shared__ Bits found;
+  const int tid = threadIdx.x;
+  if (tid <= kRows) first[tid] = n;
+  __syncthreads();
+  // (the first trip's timesteps stay in registers)
+  Bits v[kRows], held[kEach];
+#pragma unroll
+  for (int e = 0; e < kEach; ++e) held[e] = t[min(tid + e * kThreads, n - 1)];
+  int count = 0;
+  for (int k = 0; k <= kRows; ++k) {
+    int mine = n;
+    Bits its = 0;
+    for (int i0 = tid; i0 < n && mine == n; i0 += kThreads * kEach) {
+      Bits b[kEach];
+#pragma unroll
+      for (int e = 0; e < kEach; ++e) b[e] = i0 == tid ? held[e] : t[min(i0 + e * kThreads, n - 1)];
+#pragma unroll
+      for (int e = kEach - 1; e >= 0; --e) {
+        bool known = false;
+#pragma unroll
+        for (int j = 0; j < kRows; ++j) known |= j < k && b[e] == v[j];
+        if (!known) {
+          mine = min(i0 + e * kThreads, n - 1);
+          its = b[e];
+        }
+      }
+    }
+    if (mine < n) atomicMin(&first[k], mine);
+    __syncthreads();
+    if (first[k] == n) break;
+    ++count;
+    if (mine == first[k]) found = its;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kRows; ++j)
+      if (j == k) v[j] = found;
+  }
+  const int few = count <= kRows ? count : 0;
+  if (tid == 0) {
+    g->few = few;
+    Bits* const out = reinterpret_cast<Bits*>(g->value);
+#pragma unroll
+    for (int j = 0; j < kRows; ++j) out[j] = j < count ? v[j] : v[0];
+  }
+  if (few == 0) return;
+  for (int i0 = tid; i0 < n; i0 += kThreads * kEach) {
+#pragma unroll
+    for (int e = 0; e < kEach; ++e) {
+      const int i = i0 + e * kThreads;
+      if (i >= n) break;
+      const Bits b = i0 == tid ? held[e] : t[i];
+      int at = 0;
+#pragma unroll
+      for (int j = 1; j < kRows; ++j) at = j < few && b == v[j] ? j : at;
+      index[i] = at;
+    }
+  }
+}
+
+// row i of out[k] = row index[i] of table[k]; a workgroup to a token
+struct SpreadRows {
+  const u32x4* table[2];
+  u32x4* out[2];
+  int vecs[2];
+};
+__global__ __launch_bounds__(256) void spread_rows_kernel(const SpreadRows a, const TimeGroups* g, const int* __restrict__ index) {
+  if (g->few == 0) return;
+  const int row = blockIdx.x, from = index[row];
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const u32x4* const src = a.table[k] + static_cast<int64_t>(from) * a.vecs[k];
+    u32x4* const dst = a.out[k] + static_cast<int64_t>(row) * a.vecs[k];
+    for (int i = threadIdx.x; i < a.vecs[k]; i += 256) dst[i] = src[i];
+  }
+}
+
+template <typename T, typename TT>
+__global__ __launch_bounds__(256) void token_sinusoid_kernel(const TT* __restrict__ t, T* __restrict__ out, int64_t n, int half, float neg_log_period, float scale,
+                                                             const TimeGroups* g) {
+  if (g != nullptr && g->few != 0) return;
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i < n * half; i += static_cast<int64_t>(gridDim.x) * 256) {
+    const int64_t row = i / half;
+    const int j = static_cast<int>(i - row * half);
+    time_sinusoid<T>(t[row], j, half, neg_log_period, scale, 1.f, out[row * 2 * half + j], out[row * 2 * half + half + j]);
+  }
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void token_silu_kernel(const T* __restrict__ x, T* __restrict__ out, int64_t vecs, const TimeGroups* g) {
+  if (g->few != 0) return;
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i < vecs; i += static_cast<int64_t>(gridDim.x) * 256) {
+    u32x4 r = load_raw(x + i * 8);
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const float a = Raw<T>::get(r, 2 * p), b = Raw<T>::get(r, 2 * p + 1);
+      Raw<T>::set2(r, p, a / (1.f + __expf(-a)), b / (1.f + __expf(-b)));
+    }
+    store_raw(out + i * 8, r);
+  }
+}
+
+struct TokenScratch {
+  size_t index, few[3], all[3], bytes;
+};
+TokenScratch token_scratch(int64_t n, int K, int C, int P) {
+  TokenScratch s;
+  size_t at = kHeadBytes;
+  auto take = [&](size_t bytes) {
+    const size_t was = at;
+    at += (bytes + 255) / 256 * 256;
+    return was;
+  };
+  s.index = take(static_cast<size_t>(n) * 4);
+  s.few[0] = take(static_cast<size_t>(kRows) * C * 2);
+  s.few[1] = take(static_cast<size_t>(kRows) * C * 2);
+  s.few[2] = take(static_cast<size_t>(kRows) * P * 2);
+  s.all[0] = take(static_cast<size_t>(n) * K * 2);
+  s.all[1] = take(static_cast<size_t>(n) * C * 2);
+  s.all[2] = take(static_cast<size_t>(n) * C * 2);
+  s.bytes = at;
+  return s;
+}
+unsigned blocks(int64_t items) { return static_cast<unsigned>(items < 4096 * 256 ? (items + 255) / 256 : 4096); }
+
+template <typename T, typename TT>
+int run(const odit_time_tokens_args& a, const TokenScratch& at, char* s, void* workspace, size_t workspace_bytes, int t_dtype, int dtype, hipStream_t stream) {
+  const int n = a.n;
+  TimeGroups* const g = reinterpret_cast<TimeGroups*>(s);
+  int* const index = reinterpret_cast<int*>(s + at.index);
+  const int* const few = &g->few;
+  void *const h4 = s + at.few[0], *const t4 = s + at.few[1], *const p4 = s + at.few[2], *const rows = s + at.all[0], *const hidden = s + at.all[1],
+              *const act = s + at.all[2];
+  using Bits = std::conditional_t<sizeof(TT) == 4, uint32_t, uint16_t>;
+  // nothing is launched unless all of it can be
+  auto tile = [&](const void* x, int i, void* out, int N, int K, bool ask) {
+    return linear_tile_unless(x, a.w[i], a.bias[i], out, n, N, K, a.ldw[i], dtype, workspace, workspace_bytes, few, ask, stream);
+  };
+  auto some = [&](const void* x, int i, void* out, int N, int K, bool ask) {
+    return linear_few_if(x, a.w[i], a.bias[i], out, kRows, N, K, a.ldw[i], dtype, few, ask, stream);
+  };
+  auto first = [&](bool ask) {
+    return time_linear_if(g->value, a.w[0], a.bias[0], h4, kRows, a.C, a.K, a.ldw[0], a.neg_log_period, a.scale, t_dtype, dtype, few, ask, stream);
+  };
+  // (the first product, K of 256, is a fiftieth of the work: by any kernel, then for all tokens in either case)
+  const bool first_tile = tile(rows, 0, hidden, a.C, a.K, true) == ODIT_OK;
+  for (const bool ask : {true, false}) {
+    int rc = ODIT_OK;
+    auto go = [&](auto&& f) { if (rc == ODIT_OK) rc = f(); };
+    if (!ask) {
+      time_groups_kernel<TT, Bits><<<1, kThreads, 0, stream>>>(static_cast<const Bits*>(a.t), n, g, index);
+      rc = check_launch("odit_time_tokens (distinct timesteps)");
+    }
+    go([&] { return first(ask); });
+    go([&] { return some(h4, 1, t4, a.C, a.C, ask); });
+    go([&] { return some(t4, 2, p4, a.P, a.C, ask); });
+    if (!ask && rc == ODIT_OK) {
+      const SpreadRows spread{{static_cast<const u32x4*>(t4), static_cast<const u32x4*>(p4)}, {static_cast<u32x4*>(a.temb), static_cast<u32x4*>(a.proj)},
+                              {a.C / 8, a.P / 8}};
+      spread_rows_kernel<<<n, 256, 0, stream>>>(spread, g, index);
+      token_sinusoid_kernel<T, TT><<<blocks(static_cast<int64_t>(n) * (a.K / 2)), 256, 0, stream>>>(
+          static_cast<const TT*>(a.t), static_cast<T*>(rows), n, a.K / 2, a.neg_log_period, a.scale, first_tile ? g : nullptr);
+      rc = check_launch("odit_time_tokens (rows)");
+    }
+    auto silu = [&](const void* x) {
+      if (ask) return static_cast<int>(ODIT_OK);
+      const int64_t vecs = static_cast<int64_t>(n) * (a.C / 8);
+      token_silu_kernel<T><<<blocks(vecs), 256, 0, stream>>>(static_cast<const T*>(x), static_cast<T*>(act), vecs, g);
+      return check_launch("odit_time_tokens (silu)");
+    };
+    if (first_tile) go([&] { return tile(rows, 0, hidden, a.C, a.K, ask); });
+    else if (!ask)
+      go([&] { return odit_linear_rows(rows, a.w[0], a.bias[0], hidden, nullptr, nullptr, n, a.C, a.K, a.K, a.ldw[0], a.C, 0, a.bias[0] != nullptr ? ODIT_EPI_BIAS : ODIT_EPI_NONE, dtype,
+                                       dtype, 0, 0, 0, workspace, workspace_bytes, stream); });
+    go([&] { return silu(hidden); });
+    go([&] { return tile(act, 1, a.temb, a.C, a.C, ask); });
+    go([&] { return silu(a.temb); });
+    go([&] { return tile(act, 2, a.proj, a.P, a.C, ask); });
+    if (rc != ODIT_OK) return rc;
+  }
+  return ODIT_OK;
+}
+
+}  // namespace
+}  // namespace odit
+
+extern "C" size_t odit_time_tokens_bytes(int n, int K, int C, int P) {
+  return n > 0 && K > 0 && C > 0 && P > 0 ? odit::token_scratch(n, K, C, P).bytes : 0;
+}
+
+extern "C" int odit_time_tokens(const odit_time_tokens_args* args, void* scratch, size_t scratch_bytes, int t_dtype, int dtype, void* workspace,
+                                size_t workspace_bytes, void* stream) {
+  using namespace odit;
+  ODIT_CHECK_ARG(args != nullptr, "odit_time_tokens: null arguments");
+  const odit_time_tokens_args& a = *args;
+  ODIT_CHECK_ARG(a.t && a.temb && a.proj && a.n > 0 && a.n < (1 << 30) && a.K > 0 && a.K % 2 == 0 && a.C > 0 && a.P > 0, "odit_time_tokens: bad arguments (n=%d K=%d C=%d P=%d)", a.n,
+                 a.K, a.C, a.P);
+  for (int i = 0; i < 3; ++i) ODIT_CHECK_ARG(a.w[i] != nullptr && a.ldw[i] >= (i == 0 ? a.K : a.C), "odit_time_tokens: weight %d", i);
+  ODIT_CHECK_ARG(t_dtype >= ODIT_BF16 && t_dtype <= ODIT_F32, "odit_time_tokens: dtype code %d", t_dtype);
+  if ((dtype != ODIT_BF16 && dtype != ODIT_F16) || a.C % 8 != 0 || a.P % 8 != 0 || !aligned16(a.temb) || !aligned16(a.proj)) {
+    set_error("odit_time_tokens: takes 16-bit types and 16-byte aligned rows (C=%d P=%d)", a.C, a.P);
+    return ODIT_ENOTSUP;
+  }
+  const TokenScratch at = token_scratch(a.n, a.K, a.C, a.P);
+  if (scratch == nullptr || scratch_bytes < at.bytes || (reinterpret_cast<uintptr_t>(scratch) & 255) != 0) {
+    set_error("odit_time_tokens: %zu bytes of 256-byte aligned scratch needed, %zu given", at.bytes, scratch_bytes);
+    return ODIT_EWORKSPACE;
+  }
+  const hipStream_t s = static_cast<hipStream_t>(stream);
+  char* const p = static_cast<char*>(scratch);
+#define ODIT_TOKENS(T, TT) return run<T, TT>(a, at, p, workspace, workspace_bytes, t_dtype, dtype, s)
+  if (dtype == ODIT_BF16) {
+    if (t_dtype == ODIT_BF16) ODIT_TOKENS(bf16_t, bf16_t);
+    if (t_dtype == ODIT_F16) ODIT_TOKENS(bf16_t, f16_t);
+    ODIT_TOKENS(bf16_t, float);
+  }
+  if (t_dtype == ODIT_BF16) ODIT_TOKENS(f16_t, bf16_t);
+  if (t_dtype == ODIT_F16) ODIT_TOKENS(f16_t, f16_t);
+  ODIT_TOKENS(f16_t, float);
+#undef ODIT_TOKENS
+}

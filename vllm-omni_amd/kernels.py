@@ -778,6 +778,15 @@ def time_embedding(embedder: torch.nn.Module, t: torch.Tensor, dim: int, max_per
     return (_nat or _load_native()).time_embedding(embedder, t, dim, -math.log(max_period), float(scale), code, float(pre))
 
 
+def time_tokens(embedder: torch.nn.Module, time_proj: torch.nn.Module, t: torch.Tensor, dim: int, max_period: float, scale: float, dtype: torch.dtype):
+    """(``embedder`` of ``time_sinusoid``'s rows of a timestep per token, t [n], ``time_proj`` of its SiLU), each distinct timestep's rows
+    formed once where there are at most four; None for what the kernels do not take."""
+    code = _DTYPE_CODE.get(dtype)
+    if code is None or not t.is_cuda or not native_blocks() or _LINEAR_ENGINE_FLAGS:
+        return None
+    return (_nat or _load_native()).time_tokens(embedder, time_proj, t, dim, -math.log(max_period), float(scale), code)
+
+
 def stack_pairs(pairs: list[tuple]) -> tuple[torch.Tensor, ...] | None:
     """Each (p, n) of [B, S, ...] tensors stacked on the first axis, rows past the shorter S zero, and each (p, n, mask of p or
     None, mask of n or None) as a key mask [2B, longer S], false past the shorter; all in one launch. None for what the kernel does
