@@ -504,10 +504,20 @@ int odit_linear_few_pair(const void* x, const void* const w[2], const void* cons
 int odit_time_linear(const void* t, const void* w, const void* bias, void* out, int M, int N, int K, int64_t ldw, int64_t ldo,
                      float neg_log_period, float scale, float pre, int t_dtype, int dtype, void* stream);
 
-/* A timestep for each of n tokens, t [n] (t_dtype): temb [n, C] = w[1] silu(w[0] rows + bias[0]) + bias[1] and proj [n, P] = w[2] silu(temb) +
- * bias[2], where rows [n, K] are odit_time_sinusoid's (pre 1) and everything is rounded to `dtype` (wan2_2_transformer.py:282-296). Where the
- * timesteps are at most four different ones, found on the device without a synchronisation, the products are formed once for each of them.
- * Both outputs dense and 16-byte aligned. `scratch`: odit_time_tokens_bytes, 256-byte aligned; `workspace` as for odit_linear_rows.
+/* odit_adaln_modulate and odit_gated_residual_adaln (its norm with ln_weight and ln_bias alone; out null: none) for S tokens that have row
+ * index[s] (int32, on the device; every one a row of the table) of shift, scale and gate, `mod_stride` or `gate_stride` elements apart. Rows of x,
+ * out, h and y as there, h, y, x and out of the second dense; the float32 [C] tables are added to the rows. */
+int odit_adaln_modulate_rows(const void* x, void* out, const void* shift, const void* scale, const int32_t* index, const float* shift_bias,
+                             const float* scale_bias, int S, int C, int64_t x_stride, int64_t out_stride, int64_t mod_stride, float eps, int mod_dtype,
+                             int dtype, void* stream);
+int odit_gated_residual_adaln_rows(const void* h, const void* y, const void* gate, const float* gate_bias, void* x, const float* ln_weight,
+                                   const float* ln_bias, void* out, const int32_t* index, int S, int C, int64_t gate_stride, float eps, int dtype,
+                                   void* stream);
+
+/* A timestep for each of n tokens, t [n] (t_dtype): token i has row index[i] of temb [n, C] = w[1] silu(w[0] rows + bias[0]) + bias[1] and of
+ * proj [n, P] = w[2] silu(temb) + bias[2], where rows [n, K] are odit_time_sinusoid's (pre 1) and everything is rounded to `dtype`
+ * (wan2_2_transformer.py:282-296). index[i] is i, or, where the timesteps are at most four different ones (found on the device without a
+ * synchronisation), one of 0 to 3: then the first four rows alone are written. n >= 4, index int32 [n], both outputs dense and 16-byte aligned. `scratch`: odit_time_tokens_bytes, 256-byte aligned; `workspace` as for odit_linear_rows.
  * ODIT_ENOTSUP (nothing launched) where the second and the third product of all tokens are not for the tile kernel, or those of four rows not
  * odit_linear_few's. */
 typedef struct {
@@ -515,10 +525,11 @@ typedef struct {
   const void *w[3], *bias[3];
   int64_t ldw[3];
   void *temb, *proj;
+  int32_t* index;
   int n, K, C, P;
   float neg_log_period, scale;
 } odit_time_tokens_args;
-size_t odit_time_tokens_bytes(int n, int K, int C, int P);
+size_t odit_time_tokens_bytes(int n, int K, int C);
 int odit_time_tokens(const odit_time_tokens_args* args, void* scratch, size_t scratch_bytes, int t_dtype, int dtype, void* workspace,
                      size_t workspace_bytes, void* stream);
 

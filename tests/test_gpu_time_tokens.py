@@ -18,6 +18,10 @@ def _modules(gpu, dtype, C, P, bias=True):
     return emb, proj
 
 
+def _spread(done):
+    return done if done is None else tuple(x[done[2].long()] for x in done[:2])
+
+
 def _as_before(emb, proj, t, dtype):
     temb = emb(QwenTimestepProjEmbeddings.time_proj(t, scale=1.0, dtype=dtype))
     return temb, kernels.project(proj, temb, silu_input=True)
@@ -47,7 +51,10 @@ def test_distinct_timesteps(gpu, n, C, P, dtype, t_dtype, bias, distinct):
     t[:distinct] = values.flip(0)
     t[n - 1] = values[0]  # (the last one alone may be the one of its kind)
     with torch.inference_mode():
-        got = kernels.time_tokens(emb, proj, t, 256, 10000, 1.0, dtype)
+        done = kernels.time_tokens(emb, proj, t, 256, 10000, 1.0, dtype)
+        got = _spread(done)
+        assert done[2].dtype == torch.int32 and (torch.equal(done[2].long(), torch.arange(n, device=gpu)) if distinct > 4 else
+                                                 int(done[2].min()) == 0 and int(done[2].max()) == distinct - 1)
         before = _as_before(emb, proj, t, dtype)
         for a, b in zip(got, before, strict=True):
             # (of more distinct ones the same rows in tiles that are cut along the reduction and in whole ones differ by their order)
@@ -67,10 +74,10 @@ def test_bit_patterns(gpu):
     emb, proj = _modules(gpu, BF16, 1536, 9216)
     t = torch.tensor([0.0, -0.0, 700.0, 0.0], device=gpu).repeat(700)
     with torch.inference_mode():
-        temb, rows = kernels.time_tokens(emb, proj, t, 256, 10000, 1.0, BF16)
+        temb, rows = _spread(kernels.time_tokens(emb, proj, t, 256, 10000, 1.0, BF16))
         assert torch.equal(temb[0], temb[1]) and torch.equal(rows[0], rows[1]) and not torch.equal(temb[0], temb[2])
         t[5] = float("nan")
-        temb, rows = kernels.time_tokens(emb, proj, t, 256, 10000, 1.0, BF16)
+        temb, rows = _spread(kernels.time_tokens(emb, proj, t, 256, 10000, 1.0, BF16))
         assert bool(temb[5].isnan().all()) and bool(rows[5].isnan().all()) and int(temb.isnan().any(1).sum()) == 1 and int(rows.isnan().any(1).sum()) == 1
 
 
@@ -87,7 +94,7 @@ def test_refused(gpu):
         assert kernels.time_tokens(emb, proj, t, 256, 10000, 1.0, BF16) is None
     lib, a = _lib.load(), _lib.TimeTokens()
     assert lib.odit_time_tokens(_lib.C.addressof(a), None, 0, _lib.ODIT_F32, _lib.ODIT_BF16, None, 0, None) == -1
-    assert lib.odit_time_tokens_bytes(0, 256, 1536, 9216) == 0
+    assert lib.odit_time_tokens_bytes(0, 256, 1536) == 0
 
 
 def test_captured(gpu):
@@ -98,10 +105,67 @@ def test_captured(gpu):
         kernels.time_tokens(emb, proj, t, 256, 10000, 1.0, BF16)
         graph, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
         with torch.cuda.graph(graph, stream=stream):
-            temb, rows = kernels.time_tokens(emb, proj, t, 256, 10000, 1.0, BF16)
+            out = kernels.time_tokens(emb, proj, t, 256, 10000, 1.0, BF16)
         for distinct in (1, 3, 700, 2, 5):
             t.copy_(torch.arange(2706, device=gpu) % distinct)
             graph.replay()
-            want = kernels.time_tokens(emb, proj, t, 256, 10000, 1.0, BF16)
-            torch.cuda.synchronize()
-            assert torch.equal(temb, want[0]) and torch.equal(rows, want[1])
+            want = _spread(kernels.time_tokens(emb, proj, t, 256, 10000, 1.0, BF16))
+            assert all(torch.equal(a, b) for a, b in zip(_spread(out), want, strict=True))
+
+
+# widths of every number of wavefronts to a row, and one that takes the general kernel
+@pytest.mark.parametrize("S,C", [(1, 512), (77, 1024), (300, 1536), (5, 3072), (129, 4096), (33, 5120), (64, 6152), (9, 8192)])
+@pytest.mark.parametrize("dtype", [BF16, F16])
+def test_rows_by_number(gpu, S, C, dtype):
+    """A table's rows by number give the bits of the same rows written out for every token."""
+    print(f"rows by number {S} x {C} {dtype}", flush=True)
+    g = torch.Generator(device=gpu).manual_seed(S)
+    rand = lambda *s: torch.randn(*s, device=gpu, generator=g)  # noqa: E731
+    x, y, table, rows = rand(1, S, C).to(dtype), rand(1, S, C).to(dtype), rand(6, C), rand(7, 6, C).to(dtype)
+    rows[5] = float("nan")  # (of no token)
+    index = torch.randint(5, (S,), device=gpu, generator=g, dtype=torch.int32)
+    full = rows.index_select(0, index).unsqueeze(0)
+    with torch.inference_mode():
+        got = kernels.adaln_rows(x, rows[:, 0], rows[:, 1], index, table[0], table[1], 1e-6)
+        assert torch.equal(got, kernels.adaln_modulate(x, full[:, :, 0], full[:, :, 1], eps=1e-6, shift_bias=table[0], scale_bias=table[1]))
+        lib, ptr = _lib.load(), lambda t: None if t is None else t.data_ptr()  # noqa: E731
+        for norm in (True, False):
+            out, n = torch.full_like(x, -1), torch.full_like(x, -1) if norm else None
+            lw, lb = (rand(C), rand(C)) if norm else (None, None)
+            gate = rows[:, 2]
+            rc = lib.odit_gated_residual_adaln_rows(ptr(x), ptr(y), ptr(gate), ptr(table[2]), ptr(out), ptr(lw), ptr(lb), ptr(n), ptr(index), S, C, 6 * C, 1e-6,
+                                                    _lib.ODIT_BF16 if dtype == BF16 else _lib.ODIT_F16, torch.cuda.current_stream().cuda_stream)
+            assert rc == 0 and torch.equal(out, kernels.gated_residual(x, y, full[:, :, 2], gate_bias=table[2]))
+            if norm:  # a LayerNorm of the rounded row: one rounding of the result, the kernels' float32 sums
+                want = torch.nn.functional.layer_norm(out.double(), (C,), lw.double(), lb.double(), 1e-6)
+                assert float(((n.double() - want).abs() / (1 + want.abs())).max()) < (2.0 ** -8 if dtype == BF16 else 2.0 ** -10)
+
+
+def test_model(gpu, monkeypatch):
+    """A model with a timestep per token: rows by number where blocks and head are the plain ones, written out where a hook looks on."""
+    from vllm_omni_amd.blocks.wan import TokenRows, WanTransformer3DModel
+
+    g = torch.Generator(device=gpu).manual_seed(3)
+    model = WanTransformer3DModel(num_attention_heads=12, attention_head_dim=128, ffn_dim=2048, num_layers=2, text_dim=256, cross_attn_norm=True).to(device=gpu, dtype=BF16)
+    with torch.no_grad():
+        for p in model.parameters():
+            p.normal_(0.0, 0.03, generator=g)
+    x, text = torch.randn(1, 16, 5, 40, 48, device=gpu, generator=g).to(BF16), torch.randn(1, 20, 256, device=gpu, generator=g).to(BF16)
+    t = torch.full((1, 5, 480), 700.0, device=gpu)
+    t[:, 0] = 0
+    made = []
+    full = TokenRows.full
+    monkeypatch.setattr(TokenRows, "full", lambda self: made.append(1) or full(self))
+    with torch.inference_mode():
+        got = model(x, t.flatten(1), text, return_dict=False)[0]
+        assert not made
+        seen = []
+        handle = model.blocks[1].register_forward_pre_hook(lambda m, a: seen.append(a[2].shape))
+        again = model(x, t.flatten(1), text, return_dict=False)[0]
+        handle.remove()
+        assert seen == [(1, 2400, 6, 1536)] and len(made) == 1 and bool(torch.isfinite(got).all())
+        monkeypatch.setattr(kernels, "time_tokens", lambda *a: None)
+        before = model(x, t.flatten(1), text, return_dict=False)[0]
+    scale = float(before.float().norm())
+    # the same rows but for last bits of float32 sums: far less than the type's own rounding, half a step in every element
+    assert float((got.float() - again.float()).norm()) < 2.0 ** -8 * scale and float((got.float() - before.float()).norm()) < 2.0 ** -8 * scale

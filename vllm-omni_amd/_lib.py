@@ -129,7 +129,11 @@ _SIGNATURES = {
     "odit_time_linear": (
         C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_int64, C.c_int64, C.c_float, C.c_float,
                   C.c_float, C.c_int, C.c_int, C.c_void_p]),
-    "odit_time_tokens_bytes": (C.c_size_t, [C.c_int] * 4),
+    "odit_adaln_modulate_rows": (
+        C.c_int, [C.c_void_p] * 7 + [C.c_int, C.c_int, C.c_int64, C.c_int64, C.c_int64, C.c_float, C.c_int, C.c_int, C.c_void_p]),
+    "odit_gated_residual_adaln_rows": (
+        C.c_int, [C.c_void_p] * 9 + [C.c_int, C.c_int, C.c_int64, C.c_float, C.c_int, C.c_void_p]),
+    "odit_time_tokens_bytes": (C.c_size_t, [C.c_int] * 3),
     "odit_time_tokens": (
         C.c_int, [C.c_void_p, C.c_void_p, C.c_size_t, C.c_int, C.c_int, C.c_void_p, C.c_size_t, C.c_void_p]),
     "odit_time_sinusoid": (
@@ -178,7 +182,7 @@ class LinearProblem(C.Structure):
 class TimeTokens(C.Structure):
     """``odit_time_tokens_args``."""
 
-    _fields_ = [("t", C.c_void_p), ("w", C.c_void_p * 3), ("bias", C.c_void_p * 3), ("ldw", C.c_int64 * 3), ("temb", C.c_void_p), ("proj", C.c_void_p)] + [
+    _fields_ = [("t", C.c_void_p), ("w", C.c_void_p * 3), ("bias", C.c_void_p * 3), ("ldw", C.c_int64 * 3), ("temb", C.c_void_p), ("proj", C.c_void_p), ("index", C.c_void_p)] + [
         (n, C.c_int) for n in ("n", "K", "C", "P")] + [("neg_log_period", C.c_float), ("scale", C.c_float)]
 
 

@@ -288,15 +288,19 @@ class WanTransformerBlock(nn.Module):
         """``mod`` = float32 [B, 6, C] = scale_shift_table + temb when the caller formed it for all
         blocks at once; otherwise it is formed here as in the reference. ``gate_bias`` = float32 [B, 2, C]:
         the two gates times the biases of the projections they scale (attn1.to_out, ffn.net_2). ``table`` = float32 [6, C],
-        ``norm2_affine`` = float32 weight and bias [C], likewise formed by the caller for all blocks."""
+        ``norm2_affine`` = float32 weight and bias [C], likewise formed by the caller for all blocks. A ``temb`` of one row a token may be
+        ``TokenRows``."""
         if norm2_affine is None and not isinstance(self.norm2, nn.Identity):
             norm2_affine = self._norm2_affine()
-        if mod is None and temb.ndim == 4 and table is None:
+        rows, temb = (temb, None) if isinstance(temb, TokenRows) else (None, temb)
+        if mod is None and (rows is not None or temb.ndim == 4) and table is None:
             table = self._table()
         if kernels.native_blocks() and hidden_states.dtype != torch.float32:
-            done = self._forward_native(hidden_states, encoder_hidden_states, temb, rotary_emb, mod, gate_bias, table, norm2_affine)
+            done = self._forward_native(hidden_states, encoder_hidden_states, temb, rotary_emb, mod, gate_bias, table, norm2_affine, rows)
             if done is not None:
                 return done
+        if rows is not None:
+            temb = rows.full()
         if mod is None and temb.ndim == 4:
             return self._forward_per_token(hidden_states, encoder_hidden_states, temb, rotary_emb, table, norm2_affine)
         if mod is None:
@@ -316,9 +320,11 @@ class WanTransformerBlock(nn.Module):
         n = kernels.adaln_modulate(x, c_shift, c_scale, eps=self.eps, out=n if n is not x else None)
         return project_residual(self.ffn.net_2, _feed_up(self.ffn.net_0, n), x, c_gate, out=x, pre=pre2, engine=_batch_engine(n))
 
-    def _forward_native(self, x, ctx, temb, rotary_emb, mod, gate_bias, table, norm2_affine):
+    def _forward_native(self, x, ctx, temb, rotary_emb, mod, gate_bias, table, norm2_affine, rows=None):
         """The whole block as one native call, or None where the call or a submodule is not of the plain form."""
         rot = _rotary(rotary_emb)
+        if rows is not None and mod is None:
+            temb = rows.rows.unsqueeze(0)
         per_token = mod is None and temb.ndim == 4
         if rot is None:
             return None
@@ -331,7 +337,7 @@ class WanTransformerBlock(nn.Module):
         return kernels.native().wan_block(self, a.num_heads, a.head_dim, x, ctx, None if per_token else mod,
                                           None if per_token else gate_bias, temb if per_token else None,
                                           table if per_token else None, lw, lb, rot.cos32, rot.sin32,
-                                          qwen_image.FUSE_MIN_ROWS, kernels.linear_engine_flags())
+                                          qwen_image.FUSE_MIN_ROWS, kernels.linear_engine_flags(), None if rows is None else rows.index)
 
     def _forward_per_token(self, x: torch.Tensor, ctx: torch.Tensor, temb: torch.Tensor, rotary_emb, tab: torch.Tensor,
                            norm2_affine: tuple[torch.Tensor, torch.Tensor] | None) -> torch.Tensor:
@@ -408,6 +414,21 @@ class WanImageEmbedding(nn.Module):
         return self._norm(self.norm2, self.ff(self._norm(self.norm1, x.contiguous())))
 
 
+class TokenRows:
+    """Rows for the tokens of one video: token i has row ``index[i]`` (int32 [S]) of ``rows`` [n, ...], of which only those may hold
+    anything."""
+
+    def __init__(self, rows: torch.Tensor, index: torch.Tensor):
+        self.rows, self.index = rows, index
+
+    def full(self) -> torch.Tensor:
+        """[1, S, ...]"""
+        return self.rows.index_select(0, self.index).unsqueeze(0)
+
+    def unflatten(self, sizes: tuple[int, int]) -> "TokenRows":
+        return TokenRows(self.rows.unflatten(-1, sizes), self.index)
+
+
 class WanTimeTextImageEmbedding(nn.Module):
     """wan.py:251-296."""
 
@@ -422,18 +443,23 @@ class WanTimeTextImageEmbedding(nn.Module):
                                if image_embed_dim is not None else None)
 
     def forward(self, timestep: torch.Tensor, encoder_hidden_states: torch.Tensor,
-                encoder_hidden_states_image: torch.Tensor | None = None, timestep_seq_len: int | None = None):
+                encoder_hidden_states_image: torch.Tensor | None = None, timestep_seq_len: int | None = None,
+                token_rows: bool = False):
         """timestep [B] -> temb [B,C], timestep_proj [B,6C]; flattened per-token timesteps [B*S] with
-        ``timestep_seq_len`` = S -> temb [B,S,C], timestep_proj [B,S,6C] (wan.py:282-296)."""
+        ``timestep_seq_len`` = S -> temb [B,S,C], timestep_proj [B,S,6C] (wan.py:282-296), with ``token_rows`` both as ``TokenRows``
+        where one video's can be formed so."""
         mlp, dtype, done = self.time_embedder, self.time_embedder.linear_1.weight.dtype, None
-        if timestep_seq_len is not None and encoder_hidden_states.shape[0] == 1 and encoder_hidden_states.dtype == dtype:
+        if (timestep_seq_len is not None and timestep.shape[0] == timestep_seq_len and encoder_hidden_states.shape[0] == 1
+                and encoder_hidden_states.dtype == dtype):
             done = kernels.time_tokens(mlp, self.time_proj, timestep, self.time_freq_dim, 10000, 1.0, dtype)
         if done is None:
             t = QwenTimestepProjEmbeddings.time_proj(timestep, dim=self.time_freq_dim, scale=1.0, dtype=dtype)
             if timestep_seq_len is not None:
                 t = t.unflatten(0, (-1, timestep_seq_len))
         if done is not None:
-            temb, timestep_proj = (x.unflatten(0, (-1, timestep_seq_len)) for x in done)
+            temb, timestep_proj = TokenRows(done[0], done[2]), TokenRows(done[1], done[2])
+            if not token_rows:
+                temb, timestep_proj = temb.full(), timestep_proj.full()
         elif encoder_hidden_states.shape[0] == 1:
             temb = mlp(t).type_as(encoder_hidden_states)
             timestep_proj = kernels.project(self.time_proj, temb, silu_input=True)
@@ -521,9 +547,9 @@ class WanTransformer3DModel(nn.Module):
         return F.linear(x, weight, bias)
 
     def prepare(self, hidden_states: torch.Tensor, timestep: torch.Tensor, encoder_hidden_states: torch.Tensor,
-                encoder_hidden_states_image: torch.Tensor | None = None):
-        """-> tokens, context, temb, timestep_proj ([B,6,C], or [B,S,6,C] for per-token timesteps [B,S]),
-        rotary. Image tokens, when given, are embedded and put in front of the text tokens (wan.py:878-879)."""
+                encoder_hidden_states_image: torch.Tensor | None = None, token_rows: bool = False):
+        """-> tokens, context, temb, timestep_proj ([B,6,C], or [B,S,6,C] for per-token timesteps [B,S]; with ``token_rows`` those of one
+        video, and their temb, may come as ``TokenRows``), rotary. Image tokens, when given, are embedded and put in front of the text tokens (wan.py:878-879)."""
         rotary = self.rope(hidden_states)
         x = self.patchify(hidden_states)
         ts_len = None
@@ -531,11 +557,13 @@ class WanTransformer3DModel(nn.Module):
             if timestep.shape[1] != x.shape[1]:
                 raise ValueError(f"per-token timesteps need one value per token: {timestep.shape[1]} vs {x.shape[1]}")
             ts_len, timestep = timestep.shape[1], timestep.flatten()
+        rows = dict(token_rows=True) if token_rows and kernels.plain_module(self.condition_embedder, WanTimeTextImageEmbedding) else {}
         temb, tproj, ctx, image = self.condition_embedder(timestep, encoder_hidden_states,
-                                                          encoder_hidden_states_image, timestep_seq_len=ts_len)
+                                                          encoder_hidden_states_image, timestep_seq_len=ts_len, **rows)
         if image is not None:
             ctx = torch.cat([image, ctx], dim=1)
-        return x, ctx, temb, tproj.unflatten(tproj.ndim - 1, (6, -1)), rotary
+        tproj = tproj.unflatten((6, -1)) if isinstance(tproj, TokenRows) else tproj.unflatten(tproj.ndim - 1, (6, -1))
+        return x, ctx, temb, tproj, rotary
 
     def all_modulations(self, timestep_proj: torch.Tensor) -> torch.Tensor:
         """float32 [L, B, 6, C]: every block's scale_shift_table + temb in one op."""
@@ -556,7 +584,8 @@ class WanTransformer3DModel(nn.Module):
         return [(rows[2 * i], rows[2 * i + 1]) for i in range(len(norms))]
 
     def run_blocks(self, x, ctx, timestep_proj, rotary):
-        per_token = timestep_proj.ndim == 4  # the blocks read the rows of timestep_proj directly
+        rows = timestep_proj if isinstance(timestep_proj, TokenRows) else None
+        per_token = rows is not None or timestep_proj.ndim == 4  # the blocks read the rows of timestep_proj directly
         mods = gb = tables = None
         if per_token:
             tables = torch.cat([blk.scale_shift_table for blk in self.blocks], dim=0).detach().float() if len(self.blocks) else None
@@ -570,11 +599,23 @@ class WanTransformer3DModel(nn.Module):
                 kw["norm2_affine"] = affines[i]
                 if per_token:
                     kw["table"] = tables[i]
-            x = block(x, ctx, timestep_proj if per_token else None, rotary, **kw)
+            mine = timestep_proj if per_token else None
+            if rows is not None and kernels.plain_module(block, WanTransformerBlock):
+                mine = rows
+            elif rows is not None and mine is rows:
+                mine = timestep_proj = rows.full()
+            x = block(x, ctx, mine, rotary, **kw)
         return x
 
     def finish(self, x: torch.Tensor, temb: torch.Tensor, grid: tuple[int, int, int], return_dict: bool = True):
         prep = self.output_scale_shift_prepare
+        if isinstance(temb, TokenRows):
+            if kernels.plain_module(prep, OutputScaleShiftPrepare) and temb.rows.dtype == x.dtype:
+                table = prep.scale_shift_table.detach().float()[0]
+                done = kernels.adaln_rows(x, temb.rows, temb.rows, temb.index, table[0], table[1], self.eps)
+                if done is not None:
+                    return self._unpatchify(self.proj_out(done), grid, return_dict)
+            temb = temb.full()
         if (temb.shape == x.shape and temb.dtype == x.dtype and x.shape[0] == 1 and not torch.is_grad_enabled()
                 and kernels.plain_module(prep, OutputScaleShiftPrepare)):
             # a timestep per token: the norm adds the table's rows to the token's own in float32, where the module writes and
@@ -586,7 +627,9 @@ class WanTransformer3DModel(nn.Module):
             if shift.ndim == 2:
                 shift, scale = shift.contiguous(), scale.contiguous()
             x = kernels.adaln_modulate(x, shift, scale, eps=self.eps)
-        x = self.proj_out(x)
+        return self._unpatchify(self.proj_out(x), grid, return_dict)
+
+    def _unpatchify(self, x: torch.Tensor, grid: tuple[int, int, int], return_dict: bool):
         p_t, p_h, p_w = self.patch_size
         x = x.reshape(x.shape[0], *grid, p_t, p_h, p_w, -1).permute(0, 7, 1, 4, 2, 5, 3, 6)
         out = x.flatten(6, 7).flatten(4, 5).flatten(2, 3)
@@ -597,8 +640,9 @@ class WanTransformer3DModel(nn.Module):
                 attention_kwargs: dict[str, Any] | None = None):
         _, _, nf, hh, ww = hidden_states.shape
         p_t, p_h, p_w = self.patch_size
-        x, ctx, temb, tproj, rotary = self.prepare(hidden_states, timestep, encoder_hidden_states,
-                                                   encoder_hidden_states_image)
+        own = type(self) is WanTransformer3DModel and self.__dict__.keys().isdisjoint(("prepare", "run_blocks", "finish"))
+        x, ctx, temb, tproj, rotary = self.prepare(hidden_states, timestep, encoder_hidden_states, encoder_hidden_states_image,
+                                                   **(dict(token_rows=True) if own else {}))
         x = self.run_blocks(x, ctx, tproj, rotary)
         return self.finish(x, temb, (nf // p_t, hh // p_h, ww // p_w), return_dict=return_dict)
 

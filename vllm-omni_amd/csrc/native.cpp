@@ -654,6 +654,35 @@ PyObject* py_stack_pairs(PyObject*, PyObject* const* a, Py_ssize_t n) {
   NATIVE_END
 }
 
+// (x [1, S, C], shift and scale [n, C], index int32 [S], shift table, scale table float32 [C], eps): token s normed, with row index[s] of shift and scale
+PyObject* py_adaln_rows(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  NATIVE_BEGIN
+  const Tensor *x, *sh, *sc, *ix, *shb, *scb;
+  if (n != 7 || !(x = tensor_of(a[0])) || !(sh = tensor_of(a[1])) || !(sc = tensor_of(a[2])) || !(ix = tensor_of(a[3])) || !(shb = tensor_of(a[4])) ||
+      !(scb = tensor_of(a[5])))
+    return none();
+  const double eps = PyFloat_AsDouble(a[6]);
+  if (PyErr_Occurred()) return nullptr;
+  const Where w;
+  const int dt = code_of(*x);
+  for (const Tensor* t : {x, sh, sc, ix, shb, scb})
+    if (!w.holds(t)) return none();
+  if (dt < 0 || x->dim() != 3 || x->size(0) != 1 || !x->is_contiguous() || x->numel() == 0 || ix->scalar_type() != at::kInt || !ix->is_contiguous() ||
+      ix->numel() != x->size(1) || x->size(1) >= (1ll << 31) || x->size(2) >= (1ll << 31))
+    return none();
+  const int64_t S = x->size(1), C = x->size(2);
+  for (const Tensor* t : {sh, sc})
+    if (t->scalar_type() != x->scalar_type() || t->dim() != 2 || t->size(1) != C || t->stride(1) != 1 || t->stride(0) != sh->stride(0) || t->stride(0) < C) return none();
+  if (!f32_row(shb, C) || !f32_row(scb, C)) return none();
+  Tensor out = fresh(x->sizes(), x->options());
+  if (unlocked([&] { return odit_adaln_modulate_rows(x->data_ptr(), out.data_ptr(), sh->data_ptr(), sc->data_ptr(), ix->data_ptr<int32_t>(), shb->data_ptr<float>(),
+                                                     scb->data_ptr<float>(), static_cast<int>(S), static_cast<int>(C), C, C, sh->stride(0), static_cast<float>(eps), dt,
+                                                     dt, w.stream); }) != 0)
+    return none();
+  return wrap(std::move(out));
+  NATIVE_END
+}
+
 // (bool mask [B, S], rows more) -> [B, S + more], true past S
 PyObject* py_extend_mask(PyObject*, PyObject* const* a, Py_ssize_t n) {
   NATIVE_BEGIN
@@ -1114,7 +1143,7 @@ PyObject* py_time_embedding(PyObject*, PyObject* const* a, Py_ssize_t n) {
 }
 
 // (TimestepEmbedding, plain Linear time_proj, t [n], cosines and sines, - ln of the longest period, scale, type code of the rows) ->
-// (linear_2(silu(linear_1(sinusoid of t))) [n, C], time_proj(silu of that) [n, P])
+// (linear_2(silu(linear_1(sinusoid of t))) [n, C], time_proj(silu of that) [n, P], the row int32 [n] of both that is a token's)
 PyObject* py_time_tokens(PyObject*, PyObject* const* a, Py_ssize_t n) {
   NATIVE_BEGIN
   const Tensor* t;
@@ -1136,13 +1165,14 @@ PyObject* py_time_tokens(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (!linear_scratch(c.where, &c.lin_ws)) return nullptr;
   const int N = static_cast<int>(t->size(0)), C = static_cast<int>(l[1].n), P = static_cast<int>(l[2].n);
   const auto options = t->options().dtype(c.st);
-  const size_t bytes = odit_time_tokens_bytes(N, static_cast<int>(dim), C, P);
-  Tensor temb = fresh({N, C}, options), proj = fresh({N, P}, options), scratch = fresh({static_cast<int64_t>(bytes)}, t->options().dtype(at::kByte));
+  const size_t bytes = odit_time_tokens_bytes(N, static_cast<int>(dim), C);
+  Tensor temb = fresh({N, C}, options), proj = fresh({N, P}, options), index = fresh({N}, t->options().dtype(at::kInt)), scratch = fresh({static_cast<int64_t>(bytes)}, t->options().dtype(at::kByte));
   odit_time_tokens_args args = {};
   args.t = t->data_ptr();
   for (int i = 0; i < 3; ++i) { args.w[i] = l[i].w; args.bias[i] = l[i].b; args.ldw[i] = l[i].ldw; }
   args.temb = temb.data_ptr();
   args.proj = proj.data_ptr();
+  args.index = index.data_ptr<int32_t>();
   args.n = N;
   args.K = static_cast<int>(dim);
   args.C = C;
@@ -1150,7 +1180,7 @@ PyObject* py_time_tokens(PyObject*, PyObject* const* a, Py_ssize_t n) {
   args.neg_log_period = static_cast<float>(period);
   args.scale = static_cast<float>(scale);
   if (unlocked([&] { return odit_time_tokens(&args, scratch.data_ptr(), bytes, dt, c.dtype, c.lin_ws.p, c.lin_ws.bytes, c.where.stream); }) != 0) return none();
-  return wrap2(std::move(temb), std::move(proj));
+  return Py_BuildValue("(NNN)", wrap(std::move(temb)), wrap(std::move(proj)), wrap(std::move(index)));
   NATIVE_END
 }
 
@@ -1742,12 +1772,15 @@ PyObject* py_flux_single_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
 
 // ---- Wan block: self-attention, cross-attention to the text, feed-forward ------------------------------------------
 // (block, heads, head_dim, x [B,S,C], context [B,T,C], mod float32 [B,6,C] or None, gate * bias float32 [B,2,C] or None, temb [B,S,6,C] or None,
-//  table float32 [6,C] or None, norm2 weight, norm2 bias (float32 [C] or None), cos, sin, min rows, engine flags) -> x or None
+//  table float32 [6,C] or None, norm2 weight, norm2 bias (float32 [C] or None), cos, sin, min rows, engine flags, index int32 [S] or None: with one
+//  video, token s has row index[s] of temb [1,rows,6,C]) -> x or None
 // (gate * bias rows lie as far apart from batch entry to batch entry as the mod rows)
 PyObject* py_wan_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
   NATIVE_BEGIN
-  if (n != 15) return none();
+  if (n != 16) return none();
   BlockCall c;
+  const Tensor* index;
+  if (!optional_tensor(a[15], &index)) return none();
   const Tensor *x = tensor_of(a[3]), *ctx = tensor_of(a[4]), *mod, *gb, *temb, *table, *lw, *lb, *cos = tensor_of(a[11]), *sin = tensor_of(a[12]);
   const int64_t H = PyLong_AsLong(a[1]), D = PyLong_AsLong(a[2]);
   const int64_t min_rows = PyLong_AsLong(a[13]);
@@ -1770,15 +1803,19 @@ PyObject* py_wan_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (B * S >= (1ll << 31) || S == 0 || T == 0 || (D != 64 && D != 128) || !c.operand(*ctx) || !ctx->is_contiguous() || ctx->size(0) != B || ctx->size(2) != C || HD != C) return none();
   const bool per_token = temb != nullptr;
   if (per_token) {
-    if (!table || !c.operand(*temb) || temb->dim() != 4 || temb->size(0) != B || temb->size(1) != S || temb->size(2) != 6 || temb->size(3) != C ||
+    if (!table || !c.operand(*temb) || temb->dim() != 4 || temb->size(0) != B || (!index && temb->size(1) != S) || temb->size(2) != 6 || temb->size(3) != C ||
         temb->stride(3) != 1 || !c.where.holds(*table) || table->scalar_type() != at::kFloat || !table->is_contiguous() || table->numel() != 6 * C)
       return none();
   } else {
-    if (!mod || !gb || !c.where.holds(*mod) || !c.where.holds(*gb) || mod->scalar_type() != at::kFloat || gb->scalar_type() != at::kFloat ||
+    if (index || !mod || !gb || !c.where.holds(*mod) || !c.where.holds(*gb) || mod->scalar_type() != at::kFloat || gb->scalar_type() != at::kFloat ||
         mod->dim() != 3 || mod->size(0) != B || mod->size(1) != 6 || mod->size(2) != C || mod->stride(2) != 1 || gb->dim() != 3 || gb->size(0) != B ||
         gb->size(1) != 2 || gb->size(2) != C || gb->stride(2) != 1 || (B > 1 && gb->stride(0) != mod->stride(0)))
       return none();
   }
+  if (index && (B != 1 || !c.where.holds(*index) || index->scalar_type() != at::kInt || index->dim() != 1 || index->size(0) != S || !index->is_contiguous() ||
+                temb->stride(1) < C || C % 8 != 0 || C > 8192 || temb->stride(1) % 8 != 0 || temb->stride(2) % 8 != 0 || !aligned16(temb->data_ptr()) ||
+                !aligned16(table->data_ptr())))
+    return none();
   if ((lw == nullptr) != (lb == nullptr) || !f32_row(lw, C) || !f32_row(lb, C) || !c.where.holds(lw) || !c.where.holds(lb)) return none();
   if (!f32_table(c, cos, S, cos->size(1)) || !f32_table(c, sin, S, cos->size(1))) return none();
   PyObject* d = instance_dict(a[0]);
@@ -1849,7 +1886,12 @@ PyObject* py_wan_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const int64_t rs[2] = {S * C, C};
   const char* tp = per_token ? static_cast<const char*>(temb->data_ptr()) : nullptr;
   auto modulate = [&](const void* src, int row) {  // rows `row` (shift) and row + 1 (scale)
-    if (per_token) {
+    if (index) {
+      const float* tab = table->data_ptr<float>();
+      c.check(odit_adaln_modulate_rows(src, nx, tp + row * temb->stride(2) * esz, tp + (row + 1) * temb->stride(2) * esz, index->data_ptr<int32_t>(), tab + row * C,
+                                       tab + (row + 1) * C, static_cast<int>(S), static_cast<int>(C), C, C, temb->stride(1), static_cast<float>(eps), c.dtype,
+                                       c.dtype, c.where.stream));
+    } else if (per_token) {
       const float* tab = table->data_ptr<float>();
       c.check(odit_adaln_modulate(src, nx, tp + row * temb->stride(2) * esz, tp + (row + 1) * temb->stride(2) * esz, nullptr, nullptr, nullptr,
                                   tab + row * C, tab + (row + 1) * C, B, S, C, rs, rs, B > 1 ? temb->stride(0) : 0, S > 1 ? temb->stride(1) : C,
@@ -1867,6 +1909,14 @@ PyObject* py_wan_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (per_token) {
       c.project(src, l, y, B * S, false);
       const int64_t gs[2] = {B > 1 ? temb->stride(0) : 0, S > 1 ? temb->stride(1) : 0}, none[2] = {0, 0};
+      if (c.rc == 0 && index) {
+        const bool norm = which == 0 && norm2_fused;
+        c.check(odit_gated_residual_adaln_rows(residual, y, tp + row * temb->stride(2) * esz, table->data_ptr<float>() + row * C, out.data_ptr(),
+                                               norm ? lw->data_ptr<float>() : nullptr, norm ? lb->data_ptr<float>() : nullptr, norm ? nx : nullptr,
+                                               index->data_ptr<int32_t>(), static_cast<int>(S), static_cast<int>(C), temb->stride(1), static_cast<float>(eps), c.dtype,
+                                               c.where.stream));
+        return;
+      }
       if (c.rc == 0 && which == 0 && norm2_fused)
         c.check(odit_gated_residual_adaln(residual, y, tp + row * temb->stride(2) * esz, table->data_ptr<float>() + row * C, out.data_ptr(), nullptr,
                                           nullptr, nullptr, nullptr, lw->data_ptr<float>(), lb->data_ptr<float>(), nx, nullptr, B, S, C, gs, none,
@@ -2002,6 +2052,7 @@ PyMethodDef kMethods[] = {
     NATIVE_FN("rope_tables", &py_rope_tables),
     NATIVE_FN("stack_pairs", &py_stack_pairs),
     NATIVE_FN("extend_mask", &py_extend_mask),
+    NATIVE_FN("adaln_rows", &py_adaln_rows),
     NATIVE_FN("cfg_combine", &py_cfg_combine),
     NATIVE_FN("euler_step", &py_euler_step),
     NATIVE_FN("gate_rows", &py_gate_rows),

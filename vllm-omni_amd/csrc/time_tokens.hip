@@ -2,8 +2,7 @@
 // time_proj(silu(temb)) for n tokens. Where an image or a first frame is given, its tokens have one timestep and the others
 // another, and n rows of these projections are two rows over and over (width 5120, 2706 tokens: 1 TFLOP, 770 us, an eighth of a
 // step of three blocks). So the distinct timesteps are found on the device (up to kRows, no synchronisation), those rows go
-// through the kernels for few rows, which stream the weights once, and are spread out over the tokens: 80 us for the products and
-// 31 for the 190 MB that are written. The launches for all tokens follow as ever, and end at once where the first ones have done
+// through the kernels for few rows, which stream the weights once (80 us), and every token is told which are its own. The launches for all tokens follow as ever, and end at once where the first ones have done
 // the work. us, before / two timesteps / all different: n=1000, width 5120 350 / 117 / 348; 2706, 5120 770 / 134 / 799; 9000, 3072
 // 918 / 134 / 953; 32760, 5120 8488 / 667 / 8507: where tokens have more timesteps the search and six launches that end at once
 // are 20 to 35 us.
@@ -26,7 +25,8 @@ struct TimeGroups {
 constexpr size_t kHeadBytes = 256;  // (every part on whole cache lines: rows 64 bytes off made the products 16 % slower)
 static_assert(sizeof(TimeGroups) <= kHeadBytes, "");
 
-// One workgroup: the first timestep that is none of those found so far, until there is none. `index`: each token's number among them.
+// One workgroup: the first timestep that is none of those found so far, until there is none. `index`: each token's number
+// among them, its own where they are too many.
 template <typename TT, typename Bits>
 __global__ __launch_bounds__(kThreads) void time_groups_kernel(const Bits* __restrict__ t, int n, TimeGroups* __restrict__ g, int* __restrict__ index) {
   __shared__ int first[kRows + 1];
@@ -74,7 +74,6 @@ __global__ __launch_bounds__(kThreads) void time_groups_kernel(const Bits* __res
 #pragma unroll
     for (int j = 0; j < kRows; ++j) out[j] = j < count ? v[j] : v[0];
   }
-  if (few == 0) return;
   for (int i0 = tid; i0 < n; i0 += kThreads * kEach) {
 #pragma unroll
     for (int e = 0; e < kEach; ++e) {
@@ -84,25 +83,8 @@ __global__ __launch_bounds__(kThreads) void time_groups_kernel(const Bits* __res
       int at = 0;
 #pragma unroll
       for (int j = 1; j < kRows; ++j) at = j < few && b == v[j] ? j : at;
-      index[i] = at;
+      index[i] = few == 0 ? i : at;
     }
-  }
-}
-
-// row i of out[k] = row index[i] of table[k]; a workgroup to a token
-struct SpreadRows {
-  const u32x4* table[2];
-  u32x4* out[2];
-  int vecs[2];
-};
-__global__ __launch_bounds__(256) void spread_rows_kernel(const SpreadRows a, const TimeGroups* g, const int* __restrict__ index) {
-  if (g->few == 0) return;
-  const int row = blockIdx.x, from = index[row];
-#pragma unroll
-  for (int k = 0; k < 2; ++k) {
-    const u32x4* const src = a.table[k] + static_cast<int64_t>(from) * a.vecs[k];
-    u32x4* const dst = a.out[k] + static_cast<int64_t>(row) * a.vecs[k];
-    for (int i = threadIdx.x; i < a.vecs[k]; i += 256) dst[i] = src[i];
   }
 }
 
@@ -132,9 +114,9 @@ __global__ __launch_bounds__(256) void token_silu_kernel(const T* __restrict__ x
 }
 
 struct TokenScratch {
-  size_t index, few[3], all[3], bytes;
+  size_t few, all[3], bytes;
 };
-TokenScratch token_scratch(int64_t n, int K, int C, int P) {
+TokenScratch token_scratch(int64_t n, int K, int C) {
   TokenScratch s;
   size_t at = kHeadBytes;
   auto take = [&](size_t bytes) {
@@ -142,10 +124,7 @@ TokenScratch token_scratch(int64_t n, int K, int C, int P) {
     at += (bytes + 255) / 256 * 256;
     return was;
   };
-  s.index = take(static_cast<size_t>(n) * 4);
-  s.few[0] = take(static_cast<size_t>(kRows) * C * 2);
-  s.few[1] = take(static_cast<size_t>(kRows) * C * 2);
-  s.few[2] = take(static_cast<size_t>(kRows) * P * 2);
+  s.few = take(static_cast<size_t>(kRows) * C * 2);
   s.all[0] = take(static_cast<size_t>(n) * K * 2);
   s.all[1] = take(static_cast<size_t>(n) * C * 2);
   s.all[2] = take(static_cast<size_t>(n) * C * 2);
@@ -158,10 +137,8 @@ template <typename T, typename TT>
 int run(const odit_time_tokens_args& a, const TokenScratch& at, char* s, void* workspace, size_t workspace_bytes, int t_dtype, int dtype, hipStream_t stream) {
   const int n = a.n;
   TimeGroups* const g = reinterpret_cast<TimeGroups*>(s);
-  int* const index = reinterpret_cast<int*>(s + at.index);
   const int* const few = &g->few;
-  void *const h4 = s + at.few[0], *const t4 = s + at.few[1], *const p4 = s + at.few[2], *const rows = s + at.all[0], *const hidden = s + at.all[1],
-              *const act = s + at.all[2];
+  void *const h4 = s + at.few, *const rows = s + at.all[0], *const hidden = s + at.all[1], *const act = s + at.all[2];
   using Bits = std::conditional_t<sizeof(TT) == 4, uint32_t, uint16_t>;
   // nothing is launched unless all of it can be
   auto tile = [&](const void* x, int i, void* out, int N, int K, bool ask) {
@@ -179,16 +156,13 @@ int run(const odit_time_tokens_args& a, const TokenScratch& at, char* s, void* w
     int rc = ODIT_OK;
     auto go = [&](auto&& f) { if (rc == ODIT_OK) rc = f(); };
     if (!ask) {
-      time_groups_kernel<TT, Bits><<<1, kThreads, 0, stream>>>(static_cast<const Bits*>(a.t), n, g, index);
+      time_groups_kernel<TT, Bits><<<1, kThreads, 0, stream>>>(static_cast<const Bits*>(a.t), n, g, a.index);
       rc = check_launch("odit_time_tokens (distinct timesteps)");
     }
     go([&] { return first(ask); });
-    go([&] { return some(h4, 1, t4, a.C, a.C, ask); });
-    go([&] { return some(t4, 2, p4, a.P, a.C, ask); });
+    go([&] { return some(h4, 1, a.temb, a.C, a.C, ask); });
+    go([&] { return some(a.temb, 2, a.proj, a.P, a.C, ask); });
     if (!ask && rc == ODIT_OK) {
-      const SpreadRows spread{{static_cast<const u32x4*>(t4), static_cast<const u32x4*>(p4)}, {static_cast<u32x4*>(a.temb), static_cast<u32x4*>(a.proj)},
-                              {a.C / 8, a.P / 8}};
-      spread_rows_kernel<<<n, 256, 0, stream>>>(spread, g, index);
       token_sinusoid_kernel<T, TT><<<blocks(static_cast<int64_t>(n) * (a.K / 2)), 256, 0, stream>>>(
           static_cast<const TT*>(a.t), static_cast<T*>(rows), n, a.K / 2, a.neg_log_period, a.scale, first_tile ? g : nullptr);
       rc = check_launch("odit_time_tokens (rows)");
@@ -215,8 +189,8 @@ int run(const odit_time_tokens_args& a, const TokenScratch& at, char* s, void* w
 }  // namespace
 }  // namespace odit
 
-extern "C" size_t odit_time_tokens_bytes(int n, int K, int C, int P) {
-  return n > 0 && K > 0 && C > 0 && P > 0 ? odit::token_scratch(n, K, C, P).bytes : 0;
+extern "C" size_t odit_time_tokens_bytes(int n, int K, int C) {
+  return n > 0 && K > 0 && C > 0 ? odit::token_scratch(n, K, C).bytes : 0;
 }
 
 extern "C" int odit_time_tokens(const odit_time_tokens_args* args, void* scratch, size_t scratch_bytes, int t_dtype, int dtype, void* workspace,
@@ -224,7 +198,7 @@ extern "C" int odit_time_tokens(const odit_time_tokens_args* args, void* scratch
   using namespace odit;
   ODIT_CHECK_ARG(args != nullptr, "odit_time_tokens: null arguments");
   const odit_time_tokens_args& a = *args;
-  ODIT_CHECK_ARG(a.t && a.temb && a.proj && a.n > 0 && a.n < (1 << 30) && a.K > 0 && a.K % 2 == 0 && a.C > 0 && a.P > 0, "odit_time_tokens: bad arguments (n=%d K=%d C=%d P=%d)", a.n,
+  ODIT_CHECK_ARG(a.t && a.temb && a.proj && a.index && a.n >= kRows && a.n < (1 << 30) && a.K > 0 && a.K % 2 == 0 && a.C > 0 && a.P > 0, "odit_time_tokens: bad arguments (n=%d K=%d C=%d P=%d)", a.n,
                  a.K, a.C, a.P);
   for (int i = 0; i < 3; ++i) ODIT_CHECK_ARG(a.w[i] != nullptr && a.ldw[i] >= (i == 0 ? a.K : a.C), "odit_time_tokens: weight %d", i);
   ODIT_CHECK_ARG(t_dtype >= ODIT_BF16 && t_dtype <= ODIT_F32, "odit_time_tokens: dtype code %d", t_dtype);
@@ -232,7 +206,7 @@ extern "C" int odit_time_tokens(const odit_time_tokens_args* args, void* scratch
     set_error("odit_time_tokens: takes 16-bit types and 16-byte aligned rows (C=%d P=%d)", a.C, a.P);
     return ODIT_ENOTSUP;
   }
-  const TokenScratch at = token_scratch(a.n, a.K, a.C, a.P);
+  const TokenScratch at = token_scratch(a.n, a.K, a.C);
   if (scratch == nullptr || scratch_bytes < at.bytes || (reinterpret_cast<uintptr_t>(scratch) & 255) != 0) {
     set_error("odit_time_tokens: %zu bytes of 256-byte aligned scratch needed, %zu given", at.bytes, scratch_bytes);
     return ODIT_EWORKSPACE;

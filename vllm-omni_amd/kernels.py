@@ -779,12 +779,19 @@ def time_embedding(embedder: torch.nn.Module, t: torch.Tensor, dim: int, max_per
 
 
 def time_tokens(embedder: torch.nn.Module, time_proj: torch.nn.Module, t: torch.Tensor, dim: int, max_period: float, scale: float, dtype: torch.dtype):
-    """(``embedder`` of ``time_sinusoid``'s rows of a timestep per token, t [n], ``time_proj`` of its SiLU), each distinct timestep's rows
-    formed once where there are at most four; None for what the kernels do not take."""
+    """(``embedder`` of ``time_sinusoid``'s rows of a timestep per token, t [n], ``time_proj`` of its SiLU, int32 [n] whose entry i says
+    which row of both is token i's): each distinct timestep's rows are formed once where there are at most four. None for what the kernels do
+    not take."""
     code = _DTYPE_CODE.get(dtype)
     if code is None or not t.is_cuda or not native_blocks() or _LINEAR_ENGINE_FLAGS:
         return None
     return (_nat or _load_native()).time_tokens(embedder, time_proj, t, dim, -math.log(max_period), float(scale), code)
+
+
+def adaln_rows(x: torch.Tensor, shift: torch.Tensor, scale: torch.Tensor, index: torch.Tensor, shift_bias: torch.Tensor, scale_bias: torch.Tensor,
+               eps: float) -> torch.Tensor | None:
+    """``adaln_modulate`` of x [1, S, C] where token s has row index[s] of shift and scale [rows, C]; None for what the kernel does not take."""
+    return (_nat or _load_native()).adaln_rows(x, shift, scale, index, shift_bias, scale_bias, float(eps)) if native_blocks() else None
 
 
 def stack_pairs(pairs: list[tuple]) -> tuple[torch.Tensor, ...] | None:
