@@ -478,6 +478,16 @@ typedef struct odit_row_norm {
 int odit_linear_pair_norm(const odit_linear_problem problems[2], const odit_row_norm norm[2], int N, int K, int epilogue,
                           const odit_head_output* const heads[2], int dtype, unsigned flags, int launch, void* stream);
 
+/* odit_linear_pair_norm of one problem: the head's norm and projection (qwen_image_transformer.py:1065-1066) of a small model. */
+int odit_linear_norm(const odit_linear_problem* problem, const odit_row_norm* norm, int N, int K, int epilogue, int dtype, unsigned flags,
+                     void* stream);
+
+/* Two projections to N features in one launch, of K[0] and K[1] elements, the second one's rows RMS-normed over their K[1] elements (a power of
+ * two) with `weight` [K[1]] of `dtype`, as odit_qknorm_rope makes them (the same bits): img_in beside txt_norm and txt_in
+ * (qwen_image_transformer.py:1008-1012) of a small model. ODIT_ENOTSUP, with nothing launched, as for odit_linear_pair_norm. */
+int odit_linear_stem(const odit_linear_problem problems[2], int N, const int K[2], const void* weight, float eps, int dtype, unsigned flags,
+                     void* stream);
+
 /* odit_linear_rows of rows that lie in two tensors, x [M,K] beside x2 [M,K2] (W is [N, K + K2]), as one reduction in one launch
  * of the tile kernel: proj_out of a single-stream block without the concatenation (flux_transformer.py:303-309).
  * ODIT_ENOTSUP, with nothing launched, where two calls that add up are the better way. */

@@ -116,6 +116,9 @@ _SIGNATURES = {
     "odit_linear_pair_is_small": (C.c_int, [C.c_int, C.c_int, C.c_int, C.c_int]),
     "odit_linear_pair_norm": (
         C.c_int, [C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_int, C.POINTER(C.c_void_p), C.c_int, C.c_uint, C.c_int, C.c_void_p]),
+    "odit_linear_norm": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_int, C.c_uint, C.c_void_p]),
+    "odit_linear_stem": (
+        C.c_int, [C.c_void_p, C.c_int, C.POINTER(C.c_int), C.c_void_p, C.c_float, C.c_int, C.c_uint, C.c_void_p]),
     "odit_linear_join": (
         C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_int,
                   C.c_int64, C.c_int64, C.c_int64, C.c_int64, C.c_int64, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int64, C.c_uint,

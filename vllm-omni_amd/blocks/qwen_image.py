@@ -565,11 +565,14 @@ class QwenImageTransformer2DModel(nn.Module):
                 additional_t_cond=None):
         """Stem. With ``zero_cond_t`` (editing checkpoints) the timestep is doubled to [t, 0 * t], so temb
         has 2B rows: real-timestep conditioning, then timestep-zero conditioning (qit.py:141-145)."""
-        img = kernels.project(self.img_in, hidden_states)
+        both = None
+        if encoder_hidden_states.shape[-1] <= 256 and kernels.plain_module(self.txt_norm, RMSNorm):  # (a small model: one launch)
+            both = kernels.project_stem(self.img_in, hidden_states, self.txt_norm, self.txt_in, encoder_hidden_states)
+        img = kernels.project(self.img_in, hidden_states) if both is None else both[0]
         timestep = timestep.to(device=img.device, dtype=img.dtype)
         if self.zero_cond_t:
             timestep = torch.cat([timestep, timestep * 0], dim=0)
-        txt = kernels.project(self.txt_in, self.txt_norm(encoder_hidden_states))
+        txt = kernels.project(self.txt_in, self.txt_norm(encoder_hidden_states)) if both is None else both[1]
         if additional_t_cond is not None and self.zero_cond_t:
             additional_t_cond = torch.cat([additional_t_cond, additional_t_cond], dim=0)
         temb = self.time_text_embed(timestep, img, additional_t_cond)
@@ -677,7 +680,12 @@ class QwenImageTransformer2DModel(nn.Module):
         """``head``: the projection of the head's norm where the caller has it."""
         if self.zero_cond_t:
             temb = temb.chunk(2, dim=0)[0]  # the head is conditioned on the real timestep (qit.py:1062-1063)
-        out = kernels.project(self.proj_out, self.norm_out(img, temb) if head is None else self.norm_out.modulate(img, head))
+        out = None
+        if head is not None and self.inner_dim <= 256:  # (a small model: one launch)
+            scale, shift = head.chunk(2, dim=1)
+            out = kernels.project_normed(self.proj_out, img, shift, scale, self.norm_out.eps)
+        if out is None:
+            out = kernels.project(self.proj_out, self.norm_out(img, temb) if head is None else self.norm_out.modulate(img, head))
         return Transformer2DModelOutput(sample=out) if return_dict else (out,)
 
     def forward(self, hidden_states: torch.Tensor, encoder_hidden_states: torch.Tensor = None,

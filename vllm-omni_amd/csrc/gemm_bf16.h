@@ -101,7 +101,10 @@ struct RowNorm {
   float eps;
 };
 constexpr int kSmallNormK = 256;
-int launch_gemm_small_norm(const GemmCall* c, const RowNorm* norm, const HeadsOut* heads, int dtype, hipStream_t stream);
+// (`heads` with two problems only)
+int launch_gemm_small_norm(const GemmCall* c, int count, const RowNorm* norm, const HeadsOut* heads, int dtype, hipStream_t stream);
+// two problems of the same N, the second one's rows RMS-normed and weighted (K of it 64, 128 or 256)
+int launch_gemm_small_stem(const GemmCall* c, const void* weight, float eps, int dtype, hipStream_t stream);
 // the same with query, key and value heads of 64 features (gemm_small_heads.hip)
 int launch_gemm_small_heads(const GemmCall* c, int count, const HeadsOut* heads, int dtype, hipStream_t stream);
 

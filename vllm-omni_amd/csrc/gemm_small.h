@@ -18,7 +18,7 @@
 // of the two accumulators interleave by 4, so that a lane ends up with 8 consecutive ones of a row. Chunks of 16 bytes are
 // XORed with bits of the row as in gemm_tile.h. One barrier per step.
 //
-// NORM: the rows are normed and modulated on the way (adaln_rows_kernel's operations, its bits), for reductions whose steps are all in LDS
+// NORM: the rows are normed (and modulated) on the way (adaln_rows_kernel's operations, its bits), for reductions whose steps are all in LDS
 // at once. A launch of that kernel in front is 2.3 to 2.5 us one after the other, for a microsecond of work that every workgroup can do for
 // the 64 rows it reads anyway (1.7 us more of a launch): each wavefront norms the 8 rows that it has fetched itself, eight lanes to a
 // row, so nothing is waited for that was not before.
@@ -32,6 +32,10 @@ namespace odit {
 namespace {
 
 constexpr int kSmallWaves = 8, kSmallTile = 64, kSmallStages = 8, kSmallPiece = kSmallTile * kGemmBK * 2, kSmallStage = 2 * kSmallPiece;
+
+// kNormAll: LayerNorm and modulation of the rows of every problem. kNormStem: of two problems with reductions of their own the second one's rows
+// are RMS-normed and weighted (head_norm_kernel's operations, its bits), the first one's as they are.
+constexpr int kNormAll = 1, kNormStem = 2;
 
 struct SmallProblem {
   const void *x, *w;
@@ -51,9 +55,14 @@ template <bool HEADS> struct SmallHeads : SmallParams {};
 template <> struct SmallHeads<true> : SmallParams {
   HeadsOut heads[2];  // of 64 features: a tile is one head
 };
-template <bool HEADS, bool NORM> struct SmallArgs : SmallHeads<HEADS> {};
-template <bool HEADS> struct SmallArgs<HEADS, true> : SmallHeads<HEADS> {
+template <bool HEADS, int NORM> struct SmallArgs : SmallHeads<HEADS> {};
+template <bool HEADS> struct SmallArgs<HEADS, kNormAll> : SmallHeads<HEADS> {
   RowNorm norm[2];
+};
+template <> struct SmallArgs<false, kNormStem> : SmallParams {
+  const void* weight;  // of the second problem's norm
+  float eps;
+  int k_steps1;  // the second problem's
 };
 
 typedef __attribute__((address_space(3))) void* lds_void_p;
@@ -116,9 +125,46 @@ __device__ __forceinline__ void norm_rows(const RowNorm& nm, char* lds, int m0, 
     }
 }
 
+// RMSNorm and weight of the same rows, a power of two of steps: the sums go over the lanes of a row in head_norm_kernel's order
+template <typename T, int S, typename Ask>
+__device__ __forceinline__ void rms_rows(const void* weight, float eps, char* lds, int nk, int wave, int lane, Ask&& ask) {
+  const int r = wave * 8 + (lane >> 3), j = lane & 7, turn = (r >> 1) & 7;
+  u32x4 w[S], raw[S];
+#pragma unroll
+  for (int i = 0; i < S; ++i)
+    if (i < nk) w[i] = load_raw(static_cast<const T*>(weight) + j * 8 + i * kGemmBK);
+  ask();
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  auto chunk = [&](int i) { return lds + i * kSmallStage + r * 128 + ((j ^ turn) << 4); };
+  float sq[S];
+#pragma unroll
+  for (int i = 0; i < S; ++i) {
+    sq[i] = 0.f;
+    if (i < nk) {
+      raw[i] = *reinterpret_cast<const u32x4*>(chunk(i));
+#pragma unroll
+      for (int u = 0; u < 8; ++u) sq[i] = fmaf(Raw<T>::get(raw[i], u), Raw<T>::get(raw[i], u), sq[i]);
+      sq[i] = row_group_sum<8>(sq[i]);
+    }
+  }
+  float sum = 0.f;
+#pragma unroll
+  for (int i = 0; i < S; i += 2) sum += sq[i] + (i + 1 < S ? sq[i + 1 < S ? i + 1 : i] : 0.f);
+  const float rstd = rsqrtf(sum * (1.f / static_cast<float>(nk * kGemmBK)) + eps);
+#pragma unroll
+  for (int i = 0; i < S; ++i)
+    if (i < nk) {
+      u32x4 o;
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        Raw<T>::set2(o, u, Raw<T>::get(raw[i], 2 * u) * rstd * Raw<T>::get(w[i], 2 * u), Raw<T>::get(raw[i], 2 * u + 1) * rstd * Raw<T>::get(w[i], 2 * u + 1));
+      *reinterpret_cast<u32x4*>(chunk(i)) = o;
+    }
+}
+
 // S: stages (as many as there are steps where those are fewer than 8: several workgroups to a CU)
 // HEADS: query, key and value heads of 64 features (gemm_heads.h), a tile each
-template <typename T, int S, bool HEADS, bool NORM>
+template <typename T, int S, bool HEADS, int NORM>
 __global__ __launch_bounds__(64 * kSmallWaves) void gemm_small_kernel(const SmallArgs<HEADS, NORM> p) {
   using M = Mma16<T>;
   using frag = typename M::frag;
@@ -133,7 +179,8 @@ __global__ __launch_bounds__(64 * kSmallWaves) void gemm_small_kernel(const Smal
   const int t = static_cast<int>(blockIdx.x) - (which ? p.tiles0 : 0);
   const int mt = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(t) / static_cast<unsigned>(p.n_tiles));
   const int m0 = mt * kSmallTile, n0 = (t - mt * p.n_tiles) * kSmallTile;
-  const int nk = p.k_steps;
+  int nk = p.k_steps;
+  if constexpr (NORM == kNormStem) nk = which ? p.k_steps1 : nk;
 
   auto make_rsrc = [](const void* base, uint32_t bytes) {
     const uint64_t a = reinterpret_cast<uint64_t>(base);
@@ -183,19 +230,20 @@ __global__ __launch_bounds__(64 * kSmallWaves) void gemm_small_kernel(const Smal
     gemm_epilogue_vectors8<T>(e, row, col, gt, bs);
     if (gated) res = load_raw(static_cast<const T*>(e.residual) + row * e.ldr + col);
   }
-  if constexpr (NORM) {
+  auto issue_first = [&](auto&& one) {
 #pragma unroll
     for (int d = 0; d < S; ++d)
-      if (d < nk) issue_x(d, d);
-    norm_rows<T, S>(p.norm[which], lds, m0, q.M, nk, wave, lane, [&] {
-#pragma unroll
-      for (int d = 0; d < S; ++d)
-        if (d < nk) issue_w(d, d);
-    });
+      if (d < nk) one(d, d);
+  };
+  if constexpr (NORM == kNormAll) {
+    issue_first(issue_x);
+    norm_rows<T, S>(p.norm[which], lds, m0, q.M, nk, wave, lane, [&] { issue_first(issue_w); });
+  } else if constexpr (NORM == kNormStem) {
+    issue_first(issue_x);
+    if (which) rms_rows<T, S>(p.weight, p.eps, lds, nk, wave, lane, [&] { issue_first(issue_w); });
+    else issue_first(issue_w);
   } else {
-#pragma unroll
-    for (int d = 0; d < S; ++d)
-      if (d < nk) issue(d, d);
+    issue_first(issue);
   }
 
   const int xrow = wm * 16 + l16;

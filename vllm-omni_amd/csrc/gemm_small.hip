@@ -18,16 +18,16 @@ bool gemm_small_rule(const GemmCall* c, int count, int cus, int max_k) {
 }
 
 int launch_gemm_small(const GemmCall* c, int count, int dtype, hipStream_t stream) {
-  SmallArgs<false, false> p;
+  SmallArgs<false, 0> p;
   int tiles[2] = {0, 0};
   fill_small_params(p, c, count, tiles);
   const dim3 grid(tiles[0] + tiles[1]), block(64 * kSmallWaves);
 #define ODIT_SMALL(T)                                                                                                    \
   do {                                                                                                                   \
-    if (p.k_steps == 1) hipLaunchKernelGGL((gemm_small_kernel<T, 1, false, false>), grid, block, 0, stream, p);                         \
-    else if (p.k_steps == 2) hipLaunchKernelGGL((gemm_small_kernel<T, 2, false, false>), grid, block, 0, stream, p);                    \
-    else if (p.k_steps <= 4) hipLaunchKernelGGL((gemm_small_kernel<T, 4, false, false>), grid, block, 0, stream, p);                    \
-    else hipLaunchKernelGGL((gemm_small_kernel<T, kSmallStages, false, false>), grid, block, 0, stream, p);                             \
+    if (p.k_steps == 1) hipLaunchKernelGGL((gemm_small_kernel<T, 1, false, 0>), grid, block, 0, stream, p);                         \
+    else if (p.k_steps == 2) hipLaunchKernelGGL((gemm_small_kernel<T, 2, false, 0>), grid, block, 0, stream, p);                    \
+    else if (p.k_steps <= 4) hipLaunchKernelGGL((gemm_small_kernel<T, 4, false, 0>), grid, block, 0, stream, p);                    \
+    else hipLaunchKernelGGL((gemm_small_kernel<T, kSmallStages, false, 0>), grid, block, 0, stream, p);                             \
   } while (0)
   if (dtype == ODIT_BF16) ODIT_SMALL(bf16_t);
   else ODIT_SMALL(f16_t);

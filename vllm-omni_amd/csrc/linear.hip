@@ -887,35 +887,67 @@ extern "C" int odit_linear_heads(const odit_linear_problem* q, const int* N, int
 // one launch, one after the other without the host: M=256+64, K=256, heads of N=768 6.48 / 5.67, N=1024 with GELU 6.45 / 5.61; M=64+64, K=128,
 // N=512 5.76 / 4.35; with 8 steps, M=512+64, K=512, heads of N=1536 8.40 / 9.02 (every workgroup norms its rows again). The host, which such a
 // model mostly waits for, is asked for a launch less: 3.6 us.
-extern "C" int odit_linear_pair_norm(const odit_linear_problem* q, const odit_row_norm* norm, int N, int K, int epilogue,
-                                     const odit_head_output* const* heads, int dtype, unsigned flags, int launch, void* stream) {
+static int lin_normed(const char* name, const odit_linear_problem* q, const odit_row_norm* norm, int count, int N, int K, int epilogue,
+                      const odit_head_output* const* heads, int dtype, unsigned flags, int launch, void* stream) {
   using namespace odit;
-  ODIT_CHECK_ARG(q != nullptr && norm != nullptr && (heads == nullptr || (heads[0] != nullptr && heads[1] != nullptr)), "odit_linear_pair_norm: null arguments");
+  ODIT_CHECK_ARG(q != nullptr && norm != nullptr && (heads == nullptr || (heads[0] != nullptr && heads[1] != nullptr)), "%s: null arguments", name);
   if (lin_engine_of(flags) != 0 || (flags & (ODIT_LINEAR_FIRST | ODIT_LINEAR_NO_TILE)) != 0) return ODIT_ENOTSUP;
   GemmCall g[2];
   HeadsOut h[2];
   RowNorm r[2];
-  for (int i = 0; i < 2; ++i) {
+  for (int i = 0; i < count; ++i) {
     LinCall c{q[i].x, q[i].w, q[i].bias, nullptr, nullptr, q[i].out, q[i].M, N, K, q[i].ldx, q[i].ldw, q[i].ldo, 0, epilogue, dtype, dtype, nullptr, 0,
               static_cast<hipStream_t>(stream)};
     if (heads != nullptr) {
-      if (!lin_heads_out("odit_linear_pair_norm", q[i], N, *heads[i], &h[i])) return ODIT_EINVAL;
+      if (!lin_heads_out(name, q[i], N, *heads[i], &h[i])) return ODIT_EINVAL;
       c.out = heads[i]->q;
       c.ldo = N;
     }
     const int rc = lin_check(c);
     if (rc != ODIT_OK) return rc;
-    ODIT_CHECK_ARG(!lin_is_residual(c), "odit_linear_pair_norm: no residual");
+    ODIT_CHECK_ARG(!lin_is_residual(c), "%s: no residual", name);
     const odit_row_norm& n = norm[i];
-    ODIT_CHECK_ARG(n.shift != nullptr && n.scale != nullptr && n.S > 0 && n.stride >= 0, "odit_linear_pair_norm: bad modulation rows");
+    ODIT_CHECK_ARG(n.shift != nullptr && n.scale != nullptr && n.S > 0 && n.stride >= 0, "%s: bad modulation rows", name);
     g[i] = lin_gemm_call(c, 0, 0);
     r[i] = RowNorm{n.shift, n.scale, n.stride, n.S, n.eps};
     if (!aligned16(n.shift) || !aligned16(n.scale) || n.stride % 8 != 0 || K > kSmallNormK || !gemm_streamk_takes(g[i], dtype) ||
         (heads != nullptr && (h[i].D != 64 || !gemm_tile_takes(g[i], dtype) || !gemm_tile_heads_takes(g[i], h[i]))))
       return ODIT_ENOTSUP;
   }
-  if (static_cast<int64_t>(N) * K < (1 << 14) || !gemm_small_rule(g, 2, device_cus(), kSmallNormK)) return ODIT_ENOTSUP;
-  return launch == ODIT_LAUNCH_ASK ? ODIT_OK : launch_gemm_small_norm(g, r, heads != nullptr ? h : nullptr, dtype, static_cast<hipStream_t>(stream));
+  if (static_cast<int64_t>(N) * K < (1 << 14) || !gemm_small_rule(g, count, device_cus(), kSmallNormK)) return ODIT_ENOTSUP;
+  return launch == ODIT_LAUNCH_ASK ? ODIT_OK : launch_gemm_small_norm(g, count, r, heads != nullptr ? h : nullptr, dtype, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int odit_linear_pair_norm(const odit_linear_problem* q, const odit_row_norm* norm, int N, int K, int epilogue,
+                                     const odit_head_output* const* heads, int dtype, unsigned flags, int launch, void* stream) {
+  return lin_normed("odit_linear_pair_norm", q, norm, 2, N, K, epilogue, heads, dtype, flags, launch, stream);
+}
+
+extern "C" int odit_linear_norm(const odit_linear_problem* q, const odit_row_norm* norm, int N, int K, int epilogue, int dtype, unsigned flags, void* stream) {
+  return lin_normed("odit_linear_norm", q, norm, 1, N, K, epilogue, nullptr, dtype, flags, ODIT_LAUNCH_ANSWERED, stream);
+}
+
+// What a small model's step begins with: two projections that hang on nothing but the inputs, with the norm of one of them. us, three
+// launches one after the other / one: 256 rows of 64 and 64 rows of 256 to 256 features 9.7 / 4.75, 1024 and 128 rows 9.9 / 4.8, 64 rows of 64 and 20 of 128
+// to 128 8.3 / 3.6. And what it ends with (odit_linear_norm), norm and projection: 256 rows of 256 to 64 features 7.4 / 5.3, 2 x 512 7.5 / 5.3.
+extern "C" int odit_linear_stem(const odit_linear_problem* q, int N, const int K[2], const void* weight, float eps, int dtype, unsigned flags, void* stream) {
+  using namespace odit;
+  ODIT_CHECK_ARG(q != nullptr && K != nullptr && weight != nullptr, "odit_linear_stem: null arguments");
+  if (lin_engine_of(flags) != 0 || (flags & (ODIT_LINEAR_FIRST | ODIT_LINEAR_NO_TILE)) != 0) return ODIT_ENOTSUP;
+  GemmCall g[2];
+  for (int i = 0; i < 2; ++i) {
+    const LinCall c{q[i].x, q[i].w, q[i].bias, nullptr, nullptr, q[i].out, q[i].M, N, K[i], q[i].ldx, q[i].ldw, q[i].ldo, 0,
+                    q[i].bias != nullptr ? ODIT_EPI_BIAS : ODIT_EPI_NONE, dtype, dtype, nullptr, 0, static_cast<hipStream_t>(stream)};
+    const int rc = lin_check(c);
+    if (rc != ODIT_OK) return rc;
+    g[i] = lin_gemm_call(c, 0, 0);
+    if (!gemm_streamk_takes(g[i], dtype) || K[i] > kSmallNormK) return ODIT_ENOTSUP;
+  }
+  const int most = K[0] > K[1] ? 0 : 1;  // (as many workgroups to a CU as the longer reduction's LDS leaves room for)
+  GemmCall both[2] = {g[most], g[1 - most]};
+  if ((K[1] & (K[1] - 1)) != 0 || !aligned16(weight) || (g[0].bias == nullptr) != (g[1].bias == nullptr) || !gemm_small_rule(both, 2, device_cus(), kSmallNormK))
+    return ODIT_ENOTSUP;
+  return launch_gemm_small_stem(g, weight, eps, dtype, static_cast<hipStream_t>(stream));
 }
 
 // One projection of rows that lie in two tensors, in one reduction or as two products that add up, by expected time. One

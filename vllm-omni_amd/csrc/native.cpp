@@ -1081,6 +1081,71 @@ PyObject* py_project(PyObject*, PyObject* const* a, Py_ssize_t n) {
   NATIVE_END
 }
 
+// (plain Linear, x [B, S, C], shift, scale [B, C] with rows equally far apart, eps, engine flags): the module's projection of the rows of x normed and
+// modulated, in one launch; None where the kernel for small products is not the one
+PyObject* py_project_normed(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  NATIVE_BEGIN
+  const Tensor *x, *sh, *sc;
+  if (n != 6 || g_linear_type == nullptr || !(x = tensor_of(a[1])) || !(sh = tensor_of(a[2])) || !(sc = tensor_of(a[3]))) return none();
+  const double eps = PyFloat_AsDouble(a[4]);
+  const long flags = PyLong_AsLong(a[5]);
+  if (PyErr_Occurred()) return nullptr;
+  BlockCall c;
+  c.dtype = code_of(*x);
+  c.st = x->scalar_type();
+  Lin l;
+  if ((c.dtype != ODIT_BF16 && c.dtype != ODIT_F16) || !c.operand(*x) || x->dim() != 3 || !x->is_contiguous() || x->numel() == 0 || !aligned16(x->data_ptr()) ||
+      !c.linear(a[0], &l, false) || x->size(2) != l.k || l.n == 0 || l.n >= (1ll << 31) || l.k >= (1ll << 31) || x->size(0) * x->size(1) >= (1ll << 31))
+    return none();
+  for (const Tensor* t : {sh, sc})
+    if (!c.operand(*t) || t->dim() != 2 || t->size(0) != x->size(0) || t->size(1) != l.k || t->stride(1) != 1 || t->stride(0) != sh->stride(0)) return none();
+  Tensor out = fresh({x->size(0), x->size(1), l.n}, x->options());
+  odit_linear_problem q = {x->data_ptr(), l.w, l.b, nullptr, nullptr, out.data_ptr(), static_cast<int>(x->size(0) * x->size(1)), 0, l.k, l.ldw, l.n, 0, 0};
+  odit_row_norm r = {sh->data_ptr(), sc->data_ptr(), x->size(0) > 1 ? sh->stride(0) : 0, static_cast<int>(x->size(1)), static_cast<float>(eps)};
+  if (unlocked([&] { return odit_linear_norm(&q, &r, static_cast<int>(l.n), static_cast<int>(l.k), l.b ? ODIT_EPI_BIAS : ODIT_EPI_NONE, c.dtype,
+                                             static_cast<unsigned>(flags), c.where.stream); }) != 0)
+    return none();
+  return wrap(std::move(out));
+  NATIVE_END
+}
+
+// (plain Linear, x, plain RMSNorm, its eps, plain Linear, y, engine flags): the first module's projection of x and the last one's of the normed y, in one
+// launch; None where the kernel for small products is not the one
+PyObject* py_project_stem(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  NATIVE_BEGIN
+  const Tensor* x[2];
+  if (n != 7 || g_linear_type == nullptr || g_rmsnorm_type == nullptr || !(x[0] = tensor_of(a[1])) || !(x[1] = tensor_of(a[5]))) return none();
+  const double eps = PyFloat_AsDouble(a[3]);
+  const long flags = PyLong_AsLong(a[6]);
+  if (PyErr_Occurred()) return nullptr;
+  BlockCall c;
+  c.dtype = code_of(*x[0]);
+  c.st = x[0]->scalar_type();
+  Lin l[2];
+  const void* weight = nullptr;
+  int w_dtype = c.dtype;
+  if ((c.dtype != ODIT_BF16 && c.dtype != ODIT_F16) || !c.linear(a[0], &l[0], false) || !c.linear(a[4], &l[1], false) || l[0].n != l[1].n || l[0].n == 0 ||
+      l[0].n >= (1ll << 31) || !c.norm_weight(a[2], g_rmsnorm_type, l[1].k, &weight, &w_dtype))
+    return none();
+  odit_linear_problem q[2];
+  Tensor out[2];
+  for (int i = 0; i < 2; ++i) {
+    if (!c.operand(*x[i]) || x[i]->dim() < 1 || !x[i]->is_contiguous() || x[i]->numel() == 0 || x[i]->size(-1) != l[i].k || l[i].k >= (1ll << 31) ||
+        x[i]->numel() / l[i].k >= (1ll << 31) || !aligned16(x[i]->data_ptr()))
+      return none();
+    auto sizes = x[i]->sizes().vec();
+    sizes.back() = l[i].n;
+    out[i] = fresh(sizes, x[i]->options());
+    q[i] = {x[i]->data_ptr(), l[i].w, l[i].b, nullptr, nullptr, out[i].data_ptr(), static_cast<int>(x[i]->numel() / l[i].k), 0, l[i].k, l[i].ldw, l[i].n, 0, 0};
+  }
+  const int K[2] = {static_cast<int>(l[0].k), static_cast<int>(l[1].k)};
+  if (unlocked([&] { return odit_linear_stem(q, static_cast<int>(l[0].n), K, weight, static_cast<float>(eps), c.dtype, static_cast<unsigned>(flags),
+                                             c.where.stream); }) != 0)
+    return none();
+  return wrap2(std::move(out[0]), std::move(out[1]));
+  NATIVE_END
+}
+
 // (x, weight, bias or None, plain Linear): silu(x) W^T + bias of the weight and of the module's, each [rows of x, features], in one launch
 PyObject* py_linear_few_pair(PyObject*, PyObject* const* a, Py_ssize_t n) {
   NATIVE_BEGIN
@@ -2047,6 +2112,8 @@ PyMethodDef kMethods[] = {
     NATIVE_FN("linear_few_pair", &py_linear_few_pair),
     NATIVE_FN("time_embedding", &py_time_embedding),
     NATIVE_FN("time_tokens", &py_time_tokens),
+    NATIVE_FN("project_normed", &py_project_normed),
+    NATIVE_FN("project_stem", &py_project_stem),
     NATIVE_FN("project", &py_project),
     NATIVE_FN("time_sinusoid", &py_time_sinusoid),
     NATIVE_FN("rope_tables", &py_rope_tables),

@@ -758,6 +758,20 @@ def project(lin: torch.nn.Module, x: torch.Tensor, silu_input: bool = False) -> 
     return project(lin, silu(x)) if silu_input else lin(x)
 
 
+def project_normed(lin: torch.nn.Module, x: torch.Tensor, shift: torch.Tensor, scale: torch.Tensor, eps: float) -> torch.Tensor | None:
+    """``lin`` of ``adaln_modulate(x, shift, scale)`` in one launch, where the kernel for small products takes it; None elsewhere."""
+    if not x.is_cuda or x.shape[-1] > 256 or not native_blocks():
+        return None
+    return (_nat or _load_native()).project_normed(lin, x, shift, scale, float(eps), _LINEAR_ENGINE_FLAGS)
+
+
+def project_stem(lin: torch.nn.Module, x: torch.Tensor, norm: torch.nn.Module, lin2: torch.nn.Module, y: torch.Tensor):
+    """(``lin`` of x, ``lin2`` of the RMS norm of y) in one launch, where the kernel for small products takes both; None elsewhere."""
+    if not x.is_cuda or y.shape[-1] > 256 or not native_blocks():
+        return None
+    return (_nat or _load_native()).project_stem(lin, x, norm, norm.variance_epsilon, lin2, y, _LINEAR_ENGINE_FLAGS)
+
+
 def time_sinusoid(t: torch.Tensor, dim: int, max_period: float, scale: float, dtype: torch.dtype,
                   pre: float = 1.0) -> torch.Tensor | None:
     """[n, dim] cosines and sines of the timesteps ``t`` [n], or of ``t.to(dtype) * pre``, in one launch; None for what the
