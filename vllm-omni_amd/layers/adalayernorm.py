@@ -38,6 +38,13 @@ class AdaLayerNorm(CustomOp):
 
         return pick(shift), pick(scale), pick(gate)
 
+    def forward(self, x: torch.Tensor, mod_params: torch.Tensor, index: torch.Tensor | None = None):
+        if index is not None:
+            return self._forward_method(x, mod_params, index)
+        nat = kernels._nat
+        out = None if nat is None else nat.adaln_of(self, x, mod_params)  # (None also for a layer that was given another method)
+        return self._forward_method(x, mod_params) if out is None else out
+
     def forward_hip(self, x: torch.Tensor, mod_params: torch.Tensor, index: torch.Tensor | None = None):
         if x.shape[-1] != self.hidden_size:
             raise ValueError(f"expected last dim {self.hidden_size}, got {x.shape[-1]}")
@@ -60,6 +67,9 @@ class AdaLayerNorm(CustomOp):
             nb = gate.size(0) // 2
             gate_result = torch.where(index.unsqueeze(-1) == 0, gate[:nb].unsqueeze(1), gate[nb:].unsqueeze(1))
         return (out.squeeze(0) if squeeze else out), gate_result
+
+
+kernels.native_classes(AdaLayerNorm=AdaLayerNorm, **{"AdaLayerNorm.forward_hip": AdaLayerNorm.forward_hip})
 
 
 def adaln_pair(norm_a: AdaLayerNorm, x_a: torch.Tensor, mod_a: torch.Tensor,

@@ -19,6 +19,11 @@ class RMSNorm(CustomOp):
         self.variance_epsilon = eps
         self.weight = nn.Parameter(torch.ones(hidden_size))
 
+    def forward(self, x: torch.Tensor) -> torch.Tensor:
+        nat = kernels._nat
+        out = None if nat is None else nat.rmsnorm_of(self, x)  # (None also for a layer that was given another method)
+        return self._forward_method(x) if out is None else out
+
     def forward_hip(self, x: torch.Tensor) -> torch.Tensor:
         n = self.hidden_size
         if x.shape[-1] == n:
@@ -47,3 +52,6 @@ class RMSNorm(CustomOp):
         kernels.qknorm_rope(x2, None, None, out, None, None, w, None, None, None,
                             eps=self.variance_epsilon, norm_mode=mode)
         return out.reshape(x.shape)
+
+
+kernels.native_classes(RMSNorm=RMSNorm, **{"RMSNorm.forward_hip": RMSNorm.forward_hip})

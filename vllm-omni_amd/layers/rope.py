@@ -19,6 +19,11 @@ class RotaryEmbedding(CustomOp):
         self.interleaved = not is_neox_style
         self.ref_rounding = ref_rounding
 
+    def forward(self, x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.Tensor:
+        nat = kernels._nat
+        out = None if nat is None else nat.rotary_of(self, x, cos, sin)  # (None also for a layer that was given another method)
+        return self._forward_method(x, cos, sin) if out is None else out
+
     def forward_hip(self, x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.Tensor:
         if cos.dim() == 3:  # (B,S,rot/2) -> first batch row, as rope.py:117-120
             cos, sin = cos[0], sin[0]
@@ -36,3 +41,6 @@ class RotaryEmbedding(CustomOp):
                             norm_mode=ODIT_NORM_NONE, neox=self.is_neox_style,
                             ref_rounding=self.ref_rounding)
         return out
+
+
+kernels.native_classes(RotaryEmbedding=RotaryEmbedding, **{"RotaryEmbedding.forward_hip": RotaryEmbedding.forward_hip})
