@@ -273,12 +273,12 @@ class CFGParallelMixin:
         return self.scheduler_step(noise_pred, t, latents)
 
 
-def _model_timesteps(timesteps, latents: torch.Tensor) -> list[torch.Tensor] | None:
-    """``timestep.to(latents) / 1000`` of every step as [1] tensors: two launches for all steps in the place of two for each, the same
-    roundings. None where the steps are not one tensor."""
+def _model_timesteps(timesteps, latents: torch.Tensor) -> torch.Tensor | None:
+    """``timestep.to(latents) / 1000`` of every step [n]: two launches for all steps in the place of two for each, the same roundings. None
+    where the steps are not one tensor."""
     if not torch.is_tensor(timesteps) or timesteps.dim() != 1 or timesteps.numel() == 0:
         return None
-    return list((timesteps.to(device=latents.device, dtype=latents.dtype) / 1000).split(1))
+    return timesteps.to(device=latents.device, dtype=latents.dtype) / 1000
 
 
 class QwenImageCFGParallelMixin(CFGParallelMixin):
@@ -286,6 +286,14 @@ class QwenImageCFGParallelMixin(CFGParallelMixin):
     (vllm_omni/diffusion/models/qwen_image/cfg_parallel.py:27-125)."""
 
     interrupt = False
+
+    def _steps_rows(self):
+        """The transformer's own way to form what hangs on the timestep alone for several steps at once, where the calls of this loop reach
+        it as they are made."""
+        own = ("predict_noise", "predict_noise_maybe_with_cfg")
+        if any(getattr(type(self), name) is not getattr(CFGParallelMixin, name) for name in own) or not vars(self).keys().isdisjoint(own):
+            return None
+        return getattr(type(self.transformer), "steps_rows", None) and self.transformer.steps_rows
 
     def diffuse(self, prompt_embeds: torch.Tensor, prompt_embeds_mask: torch.Tensor | None,
                 negative_prompt_embeds: torch.Tensor | None, negative_prompt_embeds_mask: torch.Tensor | None,
@@ -296,13 +304,24 @@ class QwenImageCFGParallelMixin(CFGParallelMixin):
         self.scheduler.set_begin_index(0)
         self.transformer.do_true_cfg = do_true_cfg
         extra = additional_transformer_kwargs or {}
-        scaled, scaled_for = _model_timesteps(timesteps, latents), latents.dtype
+        every, scaled_for = _model_timesteps(timesteps, latents), latents.dtype
+        scaled = None if every is None else every.split(1)
+        steps_rows = self._steps_rows() if scaled is not None and guidance is None and extra.get("additional_t_cond") is None else None
+        rows, rows_at = None, 0  # of up to 16 steps from rows_at
         for i, t in enumerate(timesteps):
             if self.interrupt:
                 continue
             self._current_timestep = t
+            step = {}
             if scaled is not None and latents.shape[0] == 1 and latents.dtype == scaled_for:
                 timestep = scaled[i]
+                if steps_rows is not None:
+                    if rows is None or i >= rows_at + len(rows):
+                        rows, rows_at = steps_rows(every[i:i + 16]), i
+                    if rows is None:
+                        steps_rows = None
+                    else:
+                        step = {"step": rows[i - rows_at]}
             else:
                 timestep = t.expand(latents.shape[0]).to(device=latents.device, dtype=latents.dtype) / 1000
             model_input = latents if image_latents is None else torch.cat([latents, image_latents], dim=1)
@@ -310,7 +329,7 @@ class QwenImageCFGParallelMixin(CFGParallelMixin):
             def branch(embeds, mask, lens):
                 return {"hidden_states": model_input, "timestep": timestep, "guidance": guidance,
                         "encoder_hidden_states_mask": mask, "encoder_hidden_states": embeds,
-                        "img_shapes": img_shapes, "txt_seq_lens": lens, **extra}
+                        "img_shapes": img_shapes, "txt_seq_lens": lens, **extra, **step}
 
             positive = branch(prompt_embeds, prompt_embeds_mask, txt_seq_lens)
             negative = branch(negative_prompt_embeds, negative_prompt_embeds_mask, negative_txt_seq_lens) if do_true_cfg else None
