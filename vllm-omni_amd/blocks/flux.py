@@ -380,6 +380,26 @@ class CombinedTimestepGuidanceTextProjEmbeddings(nn.Module):
         return emb + self.text_embedder(pooled_projection)
 
 
+class FluxSteps:
+    """What of a loop's calls of ``FluxTransformer2DModel`` does not hang on the latents: text tokens, rotary tables and each step's embedding,
+    and where ``fused`` each step's modulation parameters and head rows, formed for four steps at a time (the rows that the kernel which streams
+    the weights takes, and the bits of one). ``at(i)`` is the ``step`` of a call."""
+
+    def __init__(self, model: "FluxTransformer2DModel", txt: torch.Tensor, rotary: FluxRotary, temb: torch.Tensor, fused: bool):
+        self.model, self.txt, self.rotary, self.temb, self.fused = model, txt, rotary, temb, fused
+        self._first, self._rows = 0, None
+
+    def at(self, i: int):
+        mods = head = None
+        if self.fused:
+            if self._rows is None or not 0 <= i - self._first < 4:
+                self._first, self._rows = i, self.model.step_rows(self.txt, self.temb[i:i + 4])
+            if self._rows[0] is not None:
+                j = slice(i - self._first, i - self._first + 1)
+                mods, head = tuple(m[j] for m in self._rows[0]), self._rows[1][j]
+        return self.txt, self.rotary, self.temb[i:i + 1], mods, head
+
+
 class FluxTransformer2DModel(nn.Module):
     """Stem, dual blocks, single blocks, head (flux.py:399-586). ``prepare`` / ``run_blocks`` /
     ``finish`` are the stages TeaCache calls separately."""
@@ -425,9 +445,37 @@ class FluxTransformer2DModel(nn.Module):
     def dtype(self) -> torch.dtype:
         return next(self.parameters()).dtype
 
+    def loop_steps(self, timesteps: torch.Tensor, guidance, pooled_projections, encoder_hidden_states, img_ids, txt_ids) -> FluxSteps | None:
+        """``FluxSteps`` of a loop over one image with these timesteps [n]; None where somebody else than the cache of whole steps stands between
+        the loop and the model, or a part of it is not the one of its class."""
+        from ..cache.teacache.hook import is_only_hook
+
+        embed, plain = self.time_text_embed, kernels.plain_module(self, FluxTransformer2DModel)
+        if (not (plain or type(self) is FluxTransformer2DModel and is_only_hook(self)) or not kernels.native_blocks()
+                or not kernels.plain_module(embed, CombinedTimestepGuidanceTextProjEmbeddings) or not kernels.plain_module(embed.text_embedder, PixArtAlphaTextProjection)
+                or not self.__dict__.keys().isdisjoint(("all_modulations", "prepare", "run_blocks", "finish")) or pooled_projections.shape[0] != 1
+                or encoder_hidden_states.shape[0] != 1 or pooled_projections.dtype != encoder_hidden_states.dtype or not timesteps.is_cuda):
+            return None
+        dtype = pooled_projections.dtype
+        rows = [kernels.time_embedding(embed.timestep_embedder, t, 256, 10000, 1.0, dtype, 1000.0) for t in timesteps.split(4)]
+        if any(r is None for r in rows):
+            return None
+        temb = rows[0] if len(rows) == 1 else torch.cat(rows)
+        if guidance is not None:
+            temb = temb + QwenTimestepProjEmbeddings.embed(embed.guidance_embedder, guidance.to(device=temb.device), dtype, scale=1.0, pre=1000.0)
+        temb = temb + embed.text_embedder(pooled_projections)
+        txt = kernels.project(self.context_embedder, encoder_hidden_states)
+        if txt.dtype != temb.dtype:
+            return None
+        ids = [i[0] if i.ndim == 3 else i for i in (txt_ids, img_ids)]
+        return FluxSteps(self, txt, FluxRotary.of_ids(self.pos_embed, *ids), temb, fused=plain)
+
     def prepare(self, hidden_states, encoder_hidden_states, pooled_projections, timestep, img_ids, txt_ids,
-                guidance=None):
+                guidance=None, step=None):
         img = kernels.project(self.x_embedder, hidden_states)
+        if step is not None:
+            txt, rotary, temb = step[:3]
+            return img, txt, temb, rotary
         if kernels.plain_module(self.time_text_embed, CombinedTimestepGuidanceTextProjEmbeddings) and pooled_projections.dtype == img.dtype:
             if guidance is not None:
                 guidance = guidance.to(device=img.device)
@@ -545,10 +593,15 @@ class FluxTransformer2DModel(nn.Module):
     def forward(self, hidden_states: torch.Tensor, encoder_hidden_states: torch.Tensor = None,
                 pooled_projections: torch.Tensor = None, timestep: torch.Tensor = None,
                 img_ids: torch.Tensor = None, txt_ids: torch.Tensor = None, guidance: torch.Tensor | None = None,
-                joint_attention_kwargs: dict[str, Any] | None = None, return_dict: bool = True):
-        img, txt, temb, rotary = self.prepare(hidden_states, encoder_hidden_states, pooled_projections, timestep,
-                                              img_ids, txt_ids, guidance)
-        mods, head = self.step_rows(img, temb)
+                joint_attention_kwargs: dict[str, Any] | None = None, return_dict: bool = True, step=None):
+        """``step``: of ``FluxSteps`` (then nothing but ``hidden_states`` of the inputs is read)."""
+        if step is not None:
+            img, txt, temb, rotary = self.prepare(hidden_states, None, None, None, None, None, step=step)
+            mods, head = step[3:] if step[3] is not None else self.step_rows(img, temb)
+        else:
+            img, txt, temb, rotary = self.prepare(hidden_states, encoder_hidden_states, pooled_projections, timestep,
+                                                  img_ids, txt_ids, guidance)
+            mods, head = self.step_rows(img, temb)
         if mods is None:
             img, txt = self.run_blocks(img, txt, temb, rotary, joint_attention_kwargs)
             return self.finish(img, temb, return_dict=return_dict)

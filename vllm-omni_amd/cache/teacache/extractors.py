@@ -124,8 +124,9 @@ def extract_flux_context(module: nn.Module, hidden_states: torch.Tensor,
     if not hasattr(module, "prepare"):
         raise TypeError("extract_flux_context drives this package's FluxTransformer2DModel (prepare / run_blocks / "
                         f"finish stages); got {type(module).__module__}.{type(module).__name__}")
+    step = {"step": kwargs["step"]} if kwargs.get("step") is not None else {}
     img, txt, temb, rotary = module.prepare(hidden_states, encoder_hidden_states, pooled_projections, timestep,
-                                            img_ids, txt_ids, guidance)
+                                            img_ids, txt_ids, guidance, **step)
     norm1 = module.transformer_blocks[0].norm1
     n = 2 * img.shape[-1]
     rows = _first_rows(norm1.linear, temb, n)

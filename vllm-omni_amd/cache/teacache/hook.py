@@ -21,7 +21,7 @@ import torch
 from ... import kernels
 from ...hooks.base import HookRegistry, ModelHook, StateManager
 from .config import TeaCacheConfig
-from .extractors import get_extractor
+from .extractors import extract_flux_context, get_extractor
 from .state import TeaCacheState
 
 
@@ -31,6 +31,15 @@ def rel_l1_from_sums(sum_diff: float, sum_prev: float, n: int, dtype: torch.dtyp
     md = torch.tensor(sum_diff / n, dtype=torch.float64).to(torch.float32).to(dtype)
     mp = torch.tensor(sum_prev / n, dtype=torch.float64).to(torch.float32).to(dtype)
     return (md / (mp + 1e-8)).item()
+
+
+def is_only_hook(module: torch.nn.Module) -> bool:
+    """Whether a call of ``module`` is its class's own forward behind this hook, driving a Flux model, and nothing else."""
+    registry = module.__dict__.get("_hook_registry")
+    hooks = list(registry._hooks.values()) if registry is not None else []
+    return (len(hooks) == 1 and type(hooks[0]) is TeaCacheHook and hooks[0].extractor_fn is extract_flux_context
+            and module.__dict__.get("forward") == registry._trampoline and getattr(module._original_forward, "__func__", None) is type(module).forward
+            and not module._forward_hooks and not module._forward_pre_hooks)
 
 
 class TeaCacheHook(ModelHook):

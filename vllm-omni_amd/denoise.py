@@ -108,11 +108,19 @@ def diffuse_flux(transformer, latents: torch.Tensor, prompt_embeds: torch.Tensor
     guidance = None
     if guidance_scale is not None and getattr(transformer, "guidance_embeds", True):
         guidance = torch.full((nb,), float(guidance_scale), device=latents.device, dtype=torch.float32)
+    def timestep(i):
+        return torch.full((nb,), float(sig[i]) * 1000.0, device=latents.device, dtype=latents.dtype) / 1000
+
+    every = steps = None
+    if nb == 1 and num_inference_steps > 1 and hasattr(type(transformer), "loop_steps"):
+        # what hangs on prompt and timesteps alone, once for the loop
+        every = torch.cat([timestep(i) for i in range(num_inference_steps)])
+        steps = transformer.loop_steps(every, guidance, pooled_prompt_embeds, prompt_embeds, img_ids, txt_ids)
     for i in range(num_inference_steps):
-        t = (torch.full((nb,), float(sig[i]) * 1000.0, device=latents.device, dtype=latents.dtype) / 1000)
+        t = timestep(i) if every is None else every[i:i + 1]
         noise = transformer(hidden_states=latents, encoder_hidden_states=prompt_embeds,
                             pooled_projections=pooled_prompt_embeds, timestep=t, img_ids=img_ids, txt_ids=txt_ids,
-                            guidance=guidance, return_dict=False)[0]
+                            guidance=guidance, return_dict=False, **({} if steps is None else {"step": steps.at(i)}))[0]
         latents = euler_step(latents, noise, float(sig[i]), float(sig[i + 1]))
         if on_step is not None:
             on_step(i, latents)
