@@ -446,15 +446,20 @@ class FluxTransformer2DModel(nn.Module):
         return next(self.parameters()).dtype
 
     def loop_steps(self, timesteps: torch.Tensor, guidance, pooled_projections, encoder_hidden_states, img_ids, txt_ids) -> FluxSteps | None:
-        """``FluxSteps`` of a loop over one image with these timesteps [n]; None where somebody else than the cache of whole steps stands between
-        the loop and the model, or a part of it is not the one of its class."""
+        """``FluxSteps`` of a loop over one image with these timesteps [n]; None where anything but this package's code, the cache of whole steps
+        included, runs in a call of the model: a hook or a module of somebody else's may do another thing in every step, or change what is kept
+        here."""
         from ..cache.teacache.hook import is_only_hook
 
         embed, plain = self.time_text_embed, kernels.plain_module(self, FluxTransformer2DModel)
-        if (not (plain or type(self) is FluxTransformer2DModel and is_only_hook(self)) or not kernels.native_blocks()
-                or not kernels.plain_module(embed, CombinedTimestepGuidanceTextProjEmbeddings) or not kernels.plain_module(embed.text_embedder, PixArtAlphaTextProjection)
+        if (not (plain or type(self) is FluxTransformer2DModel and is_only_hook(self)) or not kernels.own_tree(*self.children())
+                or type(embed) is not CombinedTimestepGuidanceTextProjEmbeddings or type(embed.text_embedder) is not PixArtAlphaTextProjection
+                or type(self.pos_embed) is not FluxPosEmbed
+                or any(type(m) is not nn.Linear for m in (self.context_embedder, *embed.text_embedder.children()))
+                or guidance is not None and (type(embed.guidance_embedder) is not TimestepEmbedding
+                                             or any(type(m) is not nn.Linear for m in embed.guidance_embedder.children()))
                 or not self.__dict__.keys().isdisjoint(("all_modulations", "prepare", "run_blocks", "finish")) or pooled_projections.shape[0] != 1
-                or encoder_hidden_states.shape[0] != 1 or pooled_projections.dtype != encoder_hidden_states.dtype or not timesteps.is_cuda):
+                or encoder_hidden_states.shape[0] != 1 or pooled_projections.dtype != encoder_hidden_states.dtype):
             return None
         dtype = pooled_projections.dtype
         rows = [kernels.time_embedding(embed.timestep_embedder, t, 256, 10000, 1.0, dtype, 1000.0) for t in timesteps.split(4)]

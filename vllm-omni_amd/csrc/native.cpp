@@ -26,6 +26,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <algorithm>
+#include <cstring>
 #include <map>
 #include <optional>
 #include <utility>
@@ -937,7 +938,8 @@ PyObject* py_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
 // Reading a module tree. Everything below works on borrowed references.
 struct Names {
   PyObject *modules, *parameters, *fwd_hooks, *pre_hooks, *forward, *weight, *bias, *eps, *elementwise_affine, *ref_rounding, *attention,
-      *softmax_scale, *fused, *forward_hip, *kernel_takes_layer, *forward_method, *hidden_size, *variance_epsilon, *is_neox_style;
+      *softmax_scale, *fused, *forward_hip, *kernel_takes_layer, *forward_method, *hidden_size, *variance_epsilon, *is_neox_style,
+      *module;
 };
 Names g_name;
 PyTypeObject *g_linear_type, *g_rmsnorm_type, *g_rownorm_type, *g_adaln_type, *g_attention_type, *g_attention_impl_type,
@@ -977,6 +979,31 @@ bool float_attr(PyObject* d, PyObject* name, double* v) {
 const Tensor* parameter(PyObject* d, PyObject* name) {
   PyObject* p = item(item(d, g_name.parameters), name);
   return p && p != Py_None ? tensor_of(p) : nullptr;
+}
+
+// Whether a call of module `m` runs this package's code and torch's alone: no class of somebody else's in the tree, no hook, no forward and no layer's
+// method put on a module.
+bool own_tree(PyObject* m, const char* package, size_t length, int depth) {
+  if (depth > 64) return false;  // (a module that holds itself)
+  PyObject* d = plain_module(m, nullptr);
+  PyObject* from = d ? item(Py_TYPE(m)->tp_dict, g_name.module) : nullptr;
+  const char* name = from && PyUnicode_Check(from) ? PyUnicode_AsUTF8(from) : nullptr;
+  if (name == nullptr) { PyErr_Clear(); return false; }
+  if (strncmp(name, "torch.nn.modules.", 17) != 0 && (strncmp(name, package, length) != 0 || name[length] != '.')) return false;
+  if (PyObject* f = item(d, g_name.forward_method))
+    if (!PyMethod_Check(f) || PyMethod_GET_SELF(f) != m || PyMethod_GET_FUNCTION(f) != _PyType_Lookup(Py_TYPE(m), g_name.forward_hip)) return false;
+  PyObject *children = item(d, g_name.modules), *child = nullptr;
+  if (children == nullptr || !PyDict_Check(children)) return false;
+  for (Py_ssize_t at = 0; PyDict_Next(children, &at, nullptr, &child);)
+    if (child != Py_None && !own_tree(child, package, length, depth + 1)) return false;
+  return true;
+}
+// (module, name of this package)
+PyObject* py_own_tree(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  Py_ssize_t length = 0;
+  const char* package = n == 2 && PyUnicode_Check(a[1]) ? PyUnicode_AsUTF8AndSize(a[1], &length) : nullptr;
+  if (package == nullptr) { PyErr_Clear(); Py_RETURN_FALSE; }
+  return PyBool_FromLong(own_tree(a[0], package, static_cast<size_t>(length), 0));
 }
 
 // ---- a layer's own call: what it holds is looked up here, where its class and the method that it was made with are this package's ----
@@ -2160,7 +2187,8 @@ bool intern_names() {
       {"eps", &g_name.eps}, {"elementwise_affine", &g_name.elementwise_affine}, {"ref_rounding", &g_name.ref_rounding},
       {"attention", &g_name.attention}, {"softmax_scale", &g_name.softmax_scale}, {"fused", &g_name.fused},
       {"forward_hip", &g_name.forward_hip}, {"kernel_takes_layer", &g_name.kernel_takes_layer}, {"_forward_method", &g_name.forward_method},
-      {"hidden_size", &g_name.hidden_size}, {"variance_epsilon", &g_name.variance_epsilon}, {"is_neox_style", &g_name.is_neox_style}};
+      {"hidden_size", &g_name.hidden_size}, {"variance_epsilon", &g_name.variance_epsilon}, {"is_neox_style", &g_name.is_neox_style},
+      {"__module__", &g_name.module}};
   for (const auto& w : want)
     if ((*w.slot = PyUnicode_InternFromString(w.s)) == nullptr) return false;
   return true;
@@ -2180,6 +2208,7 @@ PyMethodDef kMethods[] = {
     NATIVE_FN("rmsnorm_of", &py_rmsnorm_of),
     NATIVE_FN("adaln_of", &py_adaln_of),
     NATIVE_FN("rotary_of", &py_rotary_of),
+    NATIVE_FN("own_tree", &py_own_tree),
     NATIVE_FN("rotary", &py_rotary),
     NATIVE_FN("attn", &py_attn),
     NATIVE_FN("linear", &py_linear),

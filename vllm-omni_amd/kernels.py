@@ -75,11 +75,18 @@ def plain_module(m: torch.nn.Module, *classes: type) -> bool:
             and not _global_hooks._global_forward_hooks and not _global_hooks._global_forward_pre_hooks)
 
 
+def own_tree(*modules: torch.nn.Module) -> bool:
+    """Whether calls of these modules run this package's code and torch's alone: all classes in the trees are theirs, with no hook and no
+    method put on any module. Then what they make of inputs and weights is the same at the next call, unless the caller changes those."""
+    return native_blocks() and all((_nat or _load_native()).own_tree(m, _PACKAGE) for m in modules)
+
+
 def linear_engine_flags() -> int:
     """The engine bits that ``set_linear_engine`` chose, for the native block functions."""
     return _LINEAR_ENGINE_FLAGS
 
 
+_PACKAGE = __name__.partition(".")[0]
 _NATIVE_CLASSES: dict[str, type] = {}
 
 
