@@ -77,6 +77,50 @@ def test_flux_with_a_part_of_another_class(monkeypatch):
     assert _flux_steps(model) is None
 
 
+class _Ahead:
+    """What a loop forms ahead: a step's own number."""
+
+    def at(self, i):
+        return i
+
+
+class _Recorder(nn.Module):
+    """A transformer that adds the prompt's first value to the latents and notes what it is called with."""
+
+    def __init__(self):
+        super().__init__()
+        self.seen, self.made = [], 0
+
+    def loop_steps(self, timesteps, *rest):
+        self.made += 1
+        return _Ahead()
+
+    def forward(self, hidden_states, encoder_hidden_states, timestep, step=None, **kw):
+        self.seen.append((step, float(encoder_hidden_states.flatten()[0]), timestep.clone()))
+        return (torch.zeros_like(hidden_states),)
+
+
+def _flux_loop(model, prompt, n=5, on_step=None):
+    denoise.diffuse_flux(model, torch.zeros(1, 4, 2), prompt, torch.zeros(1, 3), torch.zeros(4, 3), torch.zeros(2, 3), n, on_step=on_step)
+    return model.seen
+
+
+def test_flux_with_a_callback_between_the_steps():
+    model, prompt, hooked = _Recorder(), torch.zeros(1, 2, 3), []
+
+    def on_step(i, latents):
+        prompt.fill_(i + 1)
+        if i == 2:
+            model.register_forward_pre_hook(lambda m, a, kw: hooked.append(sorted(kw)), with_kwargs=True)
+    seen = _flux_loop(model, prompt, on_step=on_step)
+    assert model.made == 0 and [s[:2] for s in seen] == [(None, float(i)) for i in range(5)]
+    assert len(hooked) == 2 and all("step" not in k for k in hooked)
+    other = _Recorder()
+    plain = _flux_loop(other, torch.zeros(1, 2, 3))
+    assert other.made == 1 and [s[0] for s in plain] == list(range(5))
+    assert all(torch.equal(a[2], b[2]) for a, b in zip(seen, plain))
+
+
 def test_own_tree():
     norm = FluxTransformer2DModel(num_layers=1, num_single_layers=0, attention_head_dim=64, num_attention_heads=1, joint_attention_dim=32,
                                   pooled_projection_dim=8, axes_dims_rope=(8, 28, 28))

@@ -100,7 +100,8 @@ def diffuse_flux(transformer, latents: torch.Tensor, prompt_embeds: torch.Tensor
                  guidance_scale: float | None = 3.5, on_step=None) -> torch.Tensor:
     """Guidance-distilled Flux loop: one transformer call per step, no CFG pair
     (vllm_omni/diffusion/models/flux/pipeline_flux.py denoising loop: timestep / 1000, embedded
-    guidance scale, flow-match Euler step)."""
+    guidance scale, flow-match Euler step). What ``on_step`` changes, of the prompt, the weights or the
+    transformer's hooks, counts from the next step on."""
     transformer.do_true_cfg = False
     transformer.cfg_batched_branches = None
     nb = latents.shape[0]
@@ -112,12 +113,13 @@ def diffuse_flux(transformer, latents: torch.Tensor, prompt_embeds: torch.Tensor
         return torch.full((nb,), float(sig[i]) * 1000.0, device=latents.device, dtype=latents.dtype) / 1000
 
     every = steps = None
-    if nb == 1 and num_inference_steps > 1 and hasattr(type(transformer), "loop_steps"):
-        # what hangs on prompt and timesteps alone, once for the loop
+    if on_step is None and nb == 1 and num_inference_steps > 1 and hasattr(type(transformer), "loop_steps"):
+        # what hangs on prompt and timesteps alone, once for the loop; loop_steps sees to it that nobody's code runs inside the steps,
+        # and without on_step none runs in between
         every = torch.cat([timestep(i) for i in range(num_inference_steps)])
         steps = transformer.loop_steps(every, guidance, pooled_prompt_embeds, prompt_embeds, img_ids, txt_ids)
     for i in range(num_inference_steps):
-        t = timestep(i) if every is None else every[i:i + 1]
+        t = timestep(i) if steps is None else every[i:i + 1]
         noise = transformer(hidden_states=latents, encoder_hidden_states=prompt_embeds,
                             pooled_projections=pooled_prompt_embeds, timestep=t, img_ids=img_ids, txt_ids=txt_ids,
                             guidance=guidance, return_dict=False, **({} if steps is None else {"step": steps.at(i)}))[0]
