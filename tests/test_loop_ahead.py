@@ -121,6 +121,97 @@ def test_flux_with_a_callback_between_the_steps():
     assert all(torch.equal(a[2], b[2]) for a, b in zip(seen, plain))
 
 
+class _Qwen(nn.Module):
+    def __init__(self, number):
+        super().__init__()
+        self.number, self.seen = number, []
+
+    def steps_rows(self, timesteps):
+        return [(self.number, float(t)) for t in timesteps]
+
+    def forward(self, hidden_states, timestep, step=None, **kw):
+        self.seen.append((step, timestep.clone()))
+        return (torch.zeros_like(hidden_states),)
+
+
+class _Pipe(denoise.QwenImageCFGParallelMixin):
+    def __init__(self, scheduler=None):
+        self.transformer, self.scheduler = _Qwen(0), scheduler or denoise.FlowMatchEulerScheduler()
+
+
+def _qwen_loop(pipe, n=5):
+    pipe.scheduler.set_timesteps(n)
+    steps = pipe.scheduler.timesteps
+    pipe.diffuse(torch.zeros(1, 3, 2), None, None, None, torch.zeros(1, 4, 2), [], [3], None, steps, False, None, 1.0)
+    return [float(t) for t in steps]
+
+
+def test_qwen_ahead(monkeypatch):
+    monkeypatch.setattr(kernels, "own_tree", lambda m: True)
+    pipe = _Pipe()
+    steps = _qwen_loop(pipe, 18)
+    # (up to 16 at once)
+    assert [s for s, _ in pipe.transformer.seen] == [(0, pytest.approx(t / 1000)) for t in steps]
+    assert all(torch.equal(t, torch.tensor([s]) / 1000) for (_, t), s in zip(pipe.transformer.seen, steps))
+
+
+class _OwnScheduler(denoise.FlowMatchEulerScheduler):
+    def step(self, *a, **kw):
+        self.between()
+        return super().step(*a, **kw)
+
+
+class _OwnStep(_Pipe):
+    def scheduler_step(self, *a):
+        self.between()
+        return super().scheduler_step(*a)
+
+
+class _OwnCombination(_Pipe):
+    def combine_cfg_noise(self, *a):
+        return super().combine_cfg_noise(*a)
+
+
+class _OwnSwitch(_Pipe):
+    interrupt = property(lambda self: self.between())
+
+
+@pytest.mark.parametrize("how", ["scheduler", "scheduler's method", "step", "own step", "switch"])
+def test_qwen_with_somebody_elses_code_between_the_steps(monkeypatch, how):
+    """It exchanges the transformer, writes to the timesteps and registers a hook on the second one."""
+    monkeypatch.setattr(kernels, "own_tree", lambda m: True)
+    kind = {"own step": _OwnStep, "switch": _OwnSwitch}.get(how, _Pipe)
+    pipe = kind(_OwnScheduler() if how == "scheduler" else None)
+    first, second, hooked, calls = pipe.transformer, _Qwen(1), [], []
+
+    def between():
+        calls.append(1)
+        if len(calls) == 3:
+            pipe.transformer = second
+            pipe.scheduler.timesteps[-1] = 7.0
+            second.register_forward_pre_hook(lambda m, a, kw: hooked.append(sorted(kw)), with_kwargs=True)
+    if how == "scheduler's method":
+        real = pipe.scheduler.step
+        pipe.scheduler.step = lambda *a, **kw: between() or real(*a, **kw)
+    elif how == "step":
+        real = pipe.scheduler_step
+        pipe.scheduler_step = lambda *a: between() or real(*a)
+    pipe.between = pipe.scheduler.between = between
+    _qwen_loop(pipe)
+    seen = first.seen + second.seen
+    assert len(seen) == 5 and len(second.seen) >= 2 and all(s is None for s, _ in seen)
+    assert torch.equal(seen[-1][1], torch.tensor([7.0]) / 1000) and len(hooked) == len(second.seen) and all("step" not in k for k in hooked)
+
+
+def test_qwen_own_steps():
+    assert _Pipe()._own_steps() and not _OwnCombination()._own_steps() and not _OwnSwitch()._own_steps()
+    pipe = _Pipe()
+    pipe.interrupt = True
+    assert pipe._own_steps()
+    with torch.inference_mode():
+        assert not kernels.own_tree(pipe.transformer)  # (a class of this file)
+
+
 def test_own_tree():
     norm = FluxTransformer2DModel(num_layers=1, num_single_layers=0, attention_head_dim=64, num_attention_heads=1, joint_attention_dim=32,
                                   pooled_projection_dim=8, axes_dims_rope=(8, 28, 28))

@@ -297,13 +297,17 @@ class QwenImageCFGParallelMixin(CFGParallelMixin):
 
     interrupt = False
 
-    def _steps_rows(self):
-        """The transformer's own way to form what hangs on the timestep alone for several steps at once, where the calls of this loop reach
-        it as they are made."""
-        own = ("predict_noise", "predict_noise_maybe_with_cfg")
-        if any(getattr(type(self), name) is not getattr(CFGParallelMixin, name) for name in own) or not vars(self).keys().isdisjoint(own):
-            return None
-        return getattr(type(self.transformer), "steps_rows", None) and self.transformer.steps_rows
+    def _own_steps(self) -> bool:
+        """Whether nothing but this package's code runs between the calls of the transformer in ``diffuse``: only then is what hangs on the
+        timesteps the same before the first step as in the step itself. A scheduler or a method of somebody else's may write to the
+        timesteps or the weights, or exchange the transformer (two experts by noise level do)."""
+        kind, ours = type(self), ("predict_noise", "predict_noise_maybe_with_cfg", "combine_cfg_noise", "cfg_normalize_function", "scheduler_step",
+                                  "scheduler_step_maybe_with_cfg")
+        return (all(getattr(kind, name) is getattr(CFGParallelMixin, name) for name in ours) and vars(self).keys().isdisjoint(ours)
+                and isinstance(kind.interrupt, bool) and isinstance(kind.batch_cfg_branches, bool)  # (no properties)
+                and all(getattr(kind, name, None) is None for name in ("transformer", "scheduler", "_current_timestep"))
+                and kind.__setattr__ in (object.__setattr__, torch.nn.Module.__setattr__)
+                and type(self.scheduler) is FlowMatchEulerScheduler and "step" not in vars(self.scheduler))
 
     def diffuse(self, prompt_embeds: torch.Tensor, prompt_embeds_mask: torch.Tensor | None,
                 negative_prompt_embeds: torch.Tensor | None, negative_prompt_embeds_mask: torch.Tensor | None,
@@ -314,26 +318,28 @@ class QwenImageCFGParallelMixin(CFGParallelMixin):
         self.scheduler.set_begin_index(0)
         self.transformer.do_true_cfg = do_true_cfg
         extra = additional_transformer_kwargs or {}
-        every, scaled_for = _model_timesteps(timesteps, latents), latents.dtype
+        model = self.transformer
+        ahead = latents.shape[0] == 1 and self._own_steps() and kernels.own_tree(model)
+        every = _model_timesteps(timesteps, latents) if ahead else None
         scaled = None if every is None else every.split(1)
-        steps_rows = self._steps_rows() if scaled is not None and guidance is None and extra.get("additional_t_cond") is None else None
+        steps_rows = getattr(model, "steps_rows", None) if scaled is not None and guidance is None and extra.get("additional_t_cond") is None else None
         rows, rows_at = None, 0  # of up to 16 steps from rows_at
         for i, t in enumerate(timesteps):
             if self.interrupt:
                 continue
             self._current_timestep = t
             step = {}
-            if scaled is not None and latents.shape[0] == 1 and latents.dtype == scaled_for:
-                timestep = scaled[i]
-                if steps_rows is not None:
-                    if rows is None or i >= rows_at + len(rows):
-                        rows, rows_at = steps_rows(every[i:i + 16]), i
-                    if rows is None:
-                        steps_rows = None
-                    else:
-                        step = {"step": rows[i - rows_at]}
-            else:
+            if scaled is None:
                 timestep = t.expand(latents.shape[0]).to(device=latents.device, dtype=latents.dtype) / 1000
+            else:
+                timestep = scaled[i]
+            if steps_rows is not None and self.transformer is model:
+                if rows is None or i >= rows_at + len(rows):
+                    rows, rows_at = steps_rows(every[i:i + 16]), i
+                if rows is None:
+                    steps_rows = None
+                else:
+                    step = {"step": rows[i - rows_at]}
             model_input = latents if image_latents is None else torch.cat([latents, image_latents], dim=1)
 
             def branch(embeds, mask, lens):
