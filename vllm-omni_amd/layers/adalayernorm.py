@@ -38,12 +38,10 @@ class AdaLayerNorm(CustomOp):
 
         return pick(shift), pick(scale), pick(gate)
 
-    def forward(self, x: torch.Tensor, mod_params: torch.Tensor, index: torch.Tensor | None = None):
-        if index is not None:
-            return self._forward_method(x, mod_params, index)
+    def forward(self, *args, **kwargs):
         nat = kernels._nat
-        out = None if nat is None else nat.adaln_of(self, x, mod_params)  # (None also for a layer that was given another method)
-        return self._forward_method(x, mod_params) if out is None else out
+        out = None if nat is None or kwargs else nat.adaln_of(self, *args)  # (None also for other arguments, another class or method)
+        return self._forward_method(*args, **kwargs) if out is None else out
 
     def forward_hip(self, x: torch.Tensor, mod_params: torch.Tensor, index: torch.Tensor | None = None):
         if x.shape[-1] != self.hidden_size:

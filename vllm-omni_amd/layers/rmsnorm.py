@@ -19,10 +19,10 @@ class RMSNorm(CustomOp):
         self.variance_epsilon = eps
         self.weight = nn.Parameter(torch.ones(hidden_size))
 
-    def forward(self, x: torch.Tensor) -> torch.Tensor:
+    def forward(self, *args, **kwargs):
         nat = kernels._nat
-        out = None if nat is None else nat.rmsnorm_of(self, x)  # (None also for a layer that was given another method)
-        return self._forward_method(x) if out is None else out
+        out = None if nat is None or kwargs else nat.rmsnorm_of(self, *args)  # (None also for other arguments, another class or method)
+        return self._forward_method(*args, **kwargs) if out is None else out
 
     def forward_hip(self, x: torch.Tensor) -> torch.Tensor:
         n = self.hidden_size

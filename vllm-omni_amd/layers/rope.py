@@ -19,10 +19,10 @@ class RotaryEmbedding(CustomOp):
         self.interleaved = not is_neox_style
         self.ref_rounding = ref_rounding
 
-    def forward(self, x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.Tensor:
+    def forward(self, *args, **kwargs):
         nat = kernels._nat
-        out = None if nat is None else nat.rotary_of(self, x, cos, sin)  # (None also for a layer that was given another method)
-        return self._forward_method(x, cos, sin) if out is None else out
+        out = None if nat is None or kwargs else nat.rotary_of(self, *args)  # (None also for other arguments, another class or method)
+        return self._forward_method(*args, **kwargs) if out is None else out
 
     def forward_hip(self, x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.Tensor:
         if cos.dim() == 3:  # (B,S,rot/2) -> first batch row, as rope.py:117-120
