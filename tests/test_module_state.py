@@ -205,3 +205,29 @@ def test_a_replaced_wan_block_gets_the_arguments_it_knows(monkeypatch):
     assert torch.equal(model.run_blocks(x, ctx, torch.zeros(1, 6, 64), None), x + 2)
     assert torch.equal(model.run_blocks(x, ctx, torch.zeros(1, 3, 6, 64), None), x + 2)
     assert got == [(True, False, True)] * 2 + [(False, True, True)] * 2
+
+
+@pytest.mark.parametrize("small", [False, True])
+def test_qwen_gate_rows_of_somebody_elses(monkeypatch, small):
+    """An override with the signature that the method has always had is called in every step, also where this package's would be left out."""
+    from vllm_omni_amd import kernels
+    from vllm_omni_amd.blocks.qwen_image import QwenImageTransformer2DModel
+
+    seen = []
+
+    class Own(QwenImageTransformer2DModel):
+        def all_gate_rows(self, mods):
+            seen.append(mods)
+
+    monkeypatch.setattr(kernels, "small_pairs", lambda *a: small)
+    monkeypatch.setattr(kernels, "gate_rows", lambda *a: seen.append(a[0]))
+    size = dict(num_layers=1, attention_head_dim=64, num_attention_heads=1, joint_attention_dim=64, axes_dims_rope=(8, 28, 28))
+    models = [QwenImageTransformer2DModel(**size), Own(**size), QwenImageTransformer2DModel(**size)]
+    models[2].all_gate_rows = lambda mods: seen.append(mods)
+    mods = torch.zeros(1, 1, 2, 6 * 64, dtype=torch.bfloat16)
+    for model, calls in zip(models, (not small, True, True)):
+        monkeypatch.setattr(model, "_gated_biases", lambda: [torch.zeros(64)] * 4)
+        model.transformer_blocks = torch.nn.ModuleList()
+        model.run_blocks(torch.zeros(1, 4, 64), torch.zeros(1, 3, 64), None, None, mods=mods)
+        assert len(seen) == calls and all(torch.equal(m, mods) for m in seen)
+        seen.clear()

@@ -639,22 +639,26 @@ class QwenImageTransformer2DModel(nn.Module):
                 for path in (("attn", "to_out", "bias"), ("img_mlp", "net", "2", "bias"), ("attn", "to_add_out", "bias"),
                              ("txt_mlp", "net", "2", "bias"))]
 
-    def all_gate_rows(self, mods: torch.Tensor | None, rows: tuple[int, int] | None = None):
+    def all_gate_rows(self, mods: torch.Tensor | None):
         """float32 (gates, gates * biases) [B, L, 2, 2, C] of the four gated projections of every block,
-        from the stacked modulation parameters: one launch per step, or four small ops. None where the kernels that take the
-        projections of ``rows`` (image, text) need no such rows: in a small model the launch and the host's look at all the biases are
-        a tenth of a step."""
+        from the stacked modulation parameters: one launch per step, or four small ops."""
         if mods is None or mods.dtype == torch.float32 or self.zero_cond_t:
             return None  # per-token gates of the editing variant do not fit one row per batch entry
         B, L, C = mods.shape[0], mods.shape[1], self.inner_dim
-        if rows is not None and kernels.small_pairs(rows, (C, C), (C, self._mlp_dim)):
-            return None
         biases = self._gated_biases()
         rows = kernels.gate_rows(mods if mods.stride(0) else mods[:1], biases)
         if rows is not None:
             return tuple(t.view(-1, L, 2, 2, C).expand(B, -1, -1, -1, -1) for t in rows)
         gates = mods.view(B, L, 2, 2, 3 * C)[..., 2 * C:].float()
         return gates, gates * torch.stack(biases).detach().float().view(L, 2, 2, C)
+
+    def _takes_gates_as_they_are(self, mods: torch.Tensor | None, img: torch.Tensor, txt: torch.Tensor) -> bool:
+        """Whether the kernels that take the gated projections need no rows of ``all_gate_rows``: in a small model the launch and the host's
+        look at all the biases are a tenth of a step."""
+        if mods is None or type(self).all_gate_rows is not QwenImageTransformer2DModel.all_gate_rows or "all_gate_rows" in self.__dict__:
+            return False
+        C = self.inner_dim
+        return kernels.small_pairs((img.shape[0] * img.shape[1], txt.shape[0] * txt.shape[1]), (C, C), (C, self._mlp_dim))
 
     def all_modulations(self, temb: torch.Tensor) -> torch.Tensor | None:
         """[B, L, 2, 6C] modulation parameters of every block, or None when not fused. For the editing
@@ -688,7 +692,7 @@ class QwenImageTransformer2DModel(nn.Module):
         joint = joint_key_mask(mask, None, img.shape[0], txt.shape[1], img.shape[1], img.device)
         if mods is None:
             mods = self.all_modulations(temb)
-        rows = self.all_gate_rows(mods, (img.shape[0] * img.shape[1], txt.shape[0] * txt.shape[1]))
+        rows = None if self._takes_gates_as_they_are(mods, img, txt) else self.all_gate_rows(mods)
         for i, block in enumerate(self.transformer_blocks):
             mp = (mods[:, i, 0], mods[:txt.shape[0], i, 1]) if mods is not None else None
             gr = (rows[0][:, i], rows[1][:, i]) if rows is not None else None
