@@ -231,3 +231,19 @@ def test_qwen_gate_rows_of_somebody_elses(monkeypatch, small):
         model.run_blocks(torch.zeros(1, 4, 64), torch.zeros(1, 3, 64), None, None, mods=mods)
         assert len(seen) == calls and all(torch.equal(m, mods) for m in seen)
         seen.clear()
+
+
+def test_a_qwen_model_saved_whole_earlier(monkeypatch):
+    import pickle
+
+    from vllm_omni_amd import kernels
+    from vllm_omni_amd.blocks.qwen_image import QwenImageTransformer2DModel
+
+    model = QwenImageTransformer2DModel(num_layers=1, attention_head_dim=64, num_attention_heads=1, joint_attention_dim=64, axes_dims_rope=(8, 28, 28))
+    del model._mlp_dim
+    model, called = pickle.loads(pickle.dumps(model)), []
+    monkeypatch.setattr(kernels, "small_pairs", lambda *a: True)
+    monkeypatch.setattr(type(model), "all_gate_rows", lambda self, mods: called.append(mods))
+    model.transformer_blocks = torch.nn.ModuleList()
+    model.run_blocks(torch.zeros(1, 4, 64), torch.zeros(1, 3, 64), None, None, mods=torch.zeros(1, 1, 2, 6 * 64, dtype=torch.bfloat16))
+    assert len(called) == 1

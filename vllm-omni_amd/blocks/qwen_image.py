@@ -519,6 +519,7 @@ class QwenImageTransformer2DModel(nn.Module):
 
     _repeated_blocks = ["QwenImageTransformerBlock"]
     enable_separate_cfg = True   # class attribute of the reference's CachedTransformer base (cache/base.py:105-112)
+    _mlp_dim: int | None = None  # (a model that was saved whole may be without one of its own)
 
     def __init__(self, od_config: Any | None = None, patch_size: int = 2, in_channels: int = 64,
                  out_channels: int | None = 16, num_layers: int = 60, attention_head_dim: int = 128,
@@ -655,7 +656,7 @@ class QwenImageTransformer2DModel(nn.Module):
     def _takes_gates_as_they_are(self, mods: torch.Tensor | None, img: torch.Tensor, txt: torch.Tensor) -> bool:
         """Whether the kernels that take the gated projections need no rows of ``all_gate_rows``: in a small model the launch and the host's
         look at all the biases are a tenth of a step."""
-        if mods is None or type(self).all_gate_rows is not QwenImageTransformer2DModel.all_gate_rows or "all_gate_rows" in self.__dict__:
+        if mods is None or self._mlp_dim is None or type(self).all_gate_rows is not QwenImageTransformer2DModel.all_gate_rows or "all_gate_rows" in self.__dict__:
             return False
         C = self.inner_dim
         return kernels.small_pairs((img.shape[0] * img.shape[1], txt.shape[0] * txt.shape[1]), (C, C), (C, self._mlp_dim))
