@@ -469,14 +469,20 @@ class QwenTimestepProjEmbeddings(nn.Module):
         arg = scale * (t[:, None].float() * freqs[None, :])
         return torch.cat((torch.cos(arg), torch.sin(arg)), dim=-1).to(dtype)
 
-    @classmethod
-    def embed(cls, embedder: nn.Module, t: torch.Tensor, dtype: torch.dtype, scale: float = 1000.0, pre: float = 1.0):
-        """``embedder`` of ``time_proj`` of ``t``."""
+    @staticmethod
+    def embed(embedder: nn.Module, t: torch.Tensor, dtype: torch.dtype, scale: float = 1000.0, pre: float = 1.0):
+        """``embedder`` of this class's ``time_proj`` of ``t``."""
         done = kernels.time_embedding(embedder, t, 256, 10000, scale, dtype, pre)
-        return embedder(cls.time_proj(t, scale=scale, dtype=dtype, pre=pre)) if done is None else done
+        return embedder(QwenTimestepProjEmbeddings.time_proj(t, scale=scale, dtype=dtype, pre=pre)) if done is None else done
+
+    def own_time_proj(self) -> bool:
+        return self.time_proj is QwenTimestepProjEmbeddings.time_proj
 
     def forward(self, timestep: torch.Tensor, hidden_states: torch.Tensor, addition_t_cond=None):
-        emb = self.embed(self.timestep_embedder, timestep, hidden_states.dtype)
+        if self.own_time_proj():
+            emb = self.embed(self.timestep_embedder, timestep, hidden_states.dtype)
+        else:
+            emb = self.timestep_embedder(self.time_proj(timestep, dtype=hidden_states.dtype))
         if self.use_additional_t_cond:
             if addition_t_cond is None:
                 raise ValueError("When additional_t_cond is True, addition_t_cond must be provided.")
@@ -569,7 +575,7 @@ class QwenImageTransformer2DModel(nn.Module):
         w, embed = getattr(self, "_mod_weight", None), self.time_text_embed
         if (w is None or self.zero_cond_t or timesteps.dtype != self.img_in.weight.dtype or timesteps.shape[0] > 16
                 or not kernels.plain_module(self, QwenImageTransformer2DModel) or not kernels.plain_module(embed, QwenTimestepProjEmbeddings)
-                or embed.use_additional_t_cond or not kernels.plain_module(self.norm_out, AdaLayerNormContinuous)
+                or not embed.own_time_proj() or embed.use_additional_t_cond or not kernels.plain_module(self.norm_out, AdaLayerNormContinuous)
                 or not self.__dict__.keys().isdisjoint(("all_modulations", "prepare", "run_blocks", "finish"))):
             return None
         temb = kernels.time_embedding(embed.timestep_embedder, timesteps, 256, 10000, 1000.0, timesteps.dtype)
