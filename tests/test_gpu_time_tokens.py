@@ -169,3 +169,24 @@ def test_model(gpu, monkeypatch):
     scale = float(before.float().norm())
     # the same rows but for last bits of float32 sums: far less than the type's own rounding, half a step in every element
     assert float((got.float() - again.float()).norm()) < 2.0 ** -8 * scale and float((got.float() - before.float()).norm()) < 2.0 ** -8 * scale
+
+
+@pytest.mark.parametrize("n", [1025, 8192, 8193, 20000])
+@pytest.mark.parametrize("places", [(0, 63), (64, 1023), (1024, 65), (8191, 8192), (8192, 16384, 19998), (1, 2, 1025, 9000), (1, 2, 3, 1024), (5, 700, 1000, 1024, 8200)])
+def test_where_a_timestep_stands_first(gpu, n, places):
+    """One token of its kind at the borders of the search's wavefronts and trips: numbers by timestep, whichever comes first."""
+    print(f"timesteps of {n} tokens, alone at {places}", flush=True)
+    emb, proj = _modules(gpu, BF16, 512, 3072)
+    t = torch.full((n,), 500.0, device=gpu)
+    t[n - 1] = 1.0
+    for j, at in enumerate(places):
+        if at < n:
+            t[at] = 600.0 + j
+    with torch.inference_mode():
+        index = kernels.time_tokens(emb, proj, t, 256, 10000, 1.0, BF16)[2].long()
+    values = t.unique()
+    if len(values) > 4:
+        assert torch.equal(index, torch.arange(n, device=gpu))
+    else:
+        numbers = [index[t == v].unique() for v in values]
+        assert all(len(i) == 1 for i in numbers) and sorted(int(i) for i in numbers) == list(range(len(values)))

@@ -27,6 +27,8 @@
 // 73728 + 6144 81.3 / 78.2, 18432 + 6144 30.7 / 26.5; K=256, 24576 + 512 14.3 / 11.2, 6144 + 512 9.4 / 5.6.
 // linear_few_sinusoid_kernel: the rows of x are a timestep's cosines and sines, formed where they are staged (time_sinusoid_kernel's
 // operations): 3072 features, K=256 5.8 / 4.3, the launch less.
+#include <type_traits>
+
 #include "odit_common.h"
 #include "gemm_bf16.h"
 #include "time_sinusoid.h"
@@ -50,20 +52,22 @@ template <> __device__ __forceinline__ f32x4 mfma16<f16_t>(u32x4 a, u32x4 b, f32
 constexpr int kWaves = 8, kTile = 16, kStepK = 32, kSteps = 4;
 constexpr int kRedBytes = 2 * kWaves * 64 * 16;
 
+template <typename T> __device__ __forceinline__ u32x4 silu8(u32x4 r) {
+#pragma unroll
+  for (int p = 0; p < 4; ++p) {
+    const float a = Raw<T>::get(r, 2 * p), b = Raw<T>::get(r, 2 * p + 1);
+    Raw<T>::set2(r, p, a / (1.f + __expf(-a)), b / (1.f + __expf(-b)));
+  }
+  return r;
+}
+
 // x, activated, to LDS: `rows` rows of `vecs` 16-byte vectors, `pitch` apart
 template <typename T, bool SILU>
 __device__ __forceinline__ void stage_rows(const T* __restrict__ x, u32x4* xs, int rows, int vecs, int pitch, int64_t ldx) {
   for (int i = threadIdx.x; i < rows * vecs; i += kWaves * 64) {
     const int m = i / vecs, v = i - m * vecs;
-    u32x4 r = load_raw(x + m * ldx + v * 8);
-    if (SILU) {
-#pragma unroll
-      for (int p = 0; p < 4; ++p) {
-        const float a = Raw<T>::get(r, 2 * p), b = Raw<T>::get(r, 2 * p + 1);
-        Raw<T>::set2(r, p, a / (1.f + __expf(-a)), b / (1.f + __expf(-b)));
-      }
-    }
-    xs[m * pitch + v] = r;
+    const u32x4 r = load_raw(x + m * ldx + v * 8);
+    xs[m * pitch + v] = SILU ? silu8<T>(r) : r;
   }
 }
 
@@ -171,24 +175,68 @@ __device__ __forceinline__ void few_rows(Stage&& stage, const FewOut<T>& o0, con
   }
 }
 
-template <typename T, bool SILU, bool PAIR>
+// What a launch does where *few, on the device, is 0 (time_tokens.hip): nothing of the kind; the next product's operand for all tokens, of `vecs` 16-byte
+// vectors; all tokens' rows for the first product (`out` null: nothing).
+struct Always {
+  __device__ __forceinline__ bool instead() const { return false; }
+};
+template <typename T> struct OrSilu {
+  const int* few;
+  const T* x;
+  T* out;
+  int64_t vecs;
+  __device__ __forceinline__ bool instead() const {
+    if (*few != 0) return false;
+    const int64_t stride = static_cast<int64_t>(gridDim.x) * (kWaves * 64);
+    for (int64_t i = static_cast<int64_t>(blockIdx.x) * (kWaves * 64) + threadIdx.x; i < vecs; i += 4 * stride) {
+      u32x4 r[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (i + j * stride < vecs) r[j] = load_raw(x + (i + j * stride) * 8);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (i + j * stride < vecs) store_raw(out + (i + j * stride) * 8, silu8<T>(r[j]));
+    }
+    return true;
+  }
+};
+template <typename T, typename TT> struct OrSinusoid {
+  const int* few;
+  const TT* t;
+  T* out;
+  int64_t items;  // tokens times `half`
+  int half;
+  float neg_log_period, scale;
+  __device__ __forceinline__ bool instead() const {
+    if (*few != 0) return false;
+    if (out == nullptr) return true;
+    for (int64_t i = static_cast<int64_t>(blockIdx.x) * (kWaves * 64) + threadIdx.x; i < items; i += static_cast<int64_t>(gridDim.x) * (kWaves * 64)) {
+      const int64_t row = i / half;
+      const int j = static_cast<int>(i - row * half);
+      time_sinusoid<T>(t[row], j, half, neg_log_period, scale, 1.f, out[row * 2 * half + j], out[row * 2 * half + half + j]);
+    }
+    return true;
+  }
+};
+
+template <typename T, bool SILU, bool PAIR, typename Or>
 __global__ __launch_bounds__(kWaves * 64, 6) void linear_few_kernel(const T* __restrict__ x, const FewOut<T> o0, const FewOut<T> o1, int M, int K,
-                                                                    int64_t ldx, int tiles0, int tiles, const int* only_if) {
-  if (only_if != nullptr && *only_if == 0) return;
+                                                                    int64_t ldx, int tiles0, int tiles, const Or other) {
+  if (other.instead()) return;
   few_rows<T, PAIR>([&](u32x4* xs, int vecs, int pitch) { stage_rows<T, SILU>(x, xs, M, vecs, pitch, ldx); }, o0, o1, M, K, tiles0, tiles);
 }
-template <typename T, typename TT>
+template <typename T, typename TT, typename Or>
 __global__ __launch_bounds__(kWaves * 64, 6) void linear_few_sinusoid_kernel(const Sinusoid<TT> a, const FewOut<T> o, int M, int K, int tiles,
-                                                                             const int* only_if) {
-  if (only_if != nullptr && *only_if == 0) return;
+                                                                             const Or other) {
+  if (other.instead()) return;
   few_rows<T, false>([&](u32x4* xs, int, int pitch) { stage_sinusoid<T, TT>(a, xs, M, K, pitch); }, o, o, M, K, tiles, tiles);
 }
 
 // (groups of R features; those of the first weight come first)
-template <typename T, bool SILU, int M, int R, bool PAIR>
+template <typename T, bool SILU, int M, int R, bool PAIR, typename Or>
 __global__ __launch_bounds__(kWaves * 64, 6) void linear_stream_kernel(const T* __restrict__ x, const FewOut<T> o0, const FewOut<T> o1, int rows, int K,
-                                                                       int64_t ldx, const int* only_if) {
-  if (only_if != nullptr && *only_if == 0) return;
+                                                                       int64_t ldx, const Or other) {
+  if (other.instead()) return;
   extern __shared__ u32x4 lds[];
   const int vecs = K / 8;
   stage_rows<T, SILU>(x, lds, rows, vecs, vecs, ldx);
@@ -268,15 +316,20 @@ __global__ __launch_bounds__(kWaves * 64, 6) void linear_stream_kernel(const T* 
 // 73728 69.5 / 68.1, but 36864 36.5 / 37.3, 9216 13.2 / 15.0; with four rows of x 440 / 566.
 constexpr int kStreamWide = 1 << 16;
 
-template <typename T, bool SILU, bool PAIR>
-int launch_stream(const T* x, const FewOut<T>& o0, const FewOut<T>& o1, int M, int K, int64_t ldx, int slots, const int* only_if, hipStream_t stream) {
+template <typename T, bool SILU, bool PAIR, typename Or>
+int launch_stream(const T* x, const FewOut<T>& o0, const FewOut<T>& o1, int M, int K, int64_t ldx, int slots, const Or& other, hipStream_t stream) {
   const size_t lds = static_cast<size_t>(M) * K * 2;
   const int N = o0.N + (PAIR ? o1.N : 0);
 #define ODIT_STREAM(ROWS, R)                                                                                                             \
   do {                                                                                                                                   \
     const int groups = (o0.N + R - 1) / R + (PAIR ? (o1.N + R - 1) / R : 0), wanted = (groups + kWaves - 1) / kWaves;                      \
-    linear_stream_kernel<T, SILU, ROWS, R, PAIR><<<wanted < slots ? wanted : slots, kWaves * 64, lds, stream>>>(x, o0, o1, M, K, ldx, only_if); \
+    linear_stream_kernel<T, SILU, ROWS, R, PAIR, Or><<<wanted < slots ? wanted : slots, kWaves * 64, lds, stream>>>(x, o0, o1, M, K, ldx, other); \
   } while (0)
+  if constexpr (!std::is_same<Or, Always>::value) {
+    // four rows; every place on the chip, for what the launch may do instead (5120 features alone would be 320 workgroups, two on some compute units)
+    linear_stream_kernel<T, SILU, 4, 2, PAIR, Or><<<slots, kWaves * 64, lds, stream>>>(x, o0, o1, M, K, ldx, other);
+    return check_launch("odit_linear_few (stream)");
+  }
   if (M > 2) ODIT_STREAM(4, 2);
   else if (N >= kStreamWide && M == 2) ODIT_STREAM(2, 4);
   else if (N >= kStreamWide) ODIT_STREAM(1, 4);
@@ -304,28 +357,28 @@ struct FewArgs { const void *w, *bias; void* out; int N; int64_t ldw, ldo; };
 
 // How many rows a wavefront takes at a time follows from the features
 // of both; the bits do not (a feature's sum is one wavefront's).
-template <typename T, bool SILU, bool PAIR>
-int run_few(const void* x, const FewArgs* a, int M, int K, int64_t ldx, int cus, hipStream_t stream, const int* only_if = nullptr) {
+template <typename T, bool SILU, bool PAIR, typename Or = Always>
+int run_few(const void* x, const FewArgs* a, int M, int K, int64_t ldx, int cus, hipStream_t stream, const Or& other = Or{}) {
   FewOut<T> o[2];
   for (int i = 0; i < 2; ++i)  // (without a second weight nothing reads the second)
     o[i] = FewOut<T>{static_cast<const T*>(a[i].w), static_cast<const T*>(a[i].bias), static_cast<T*>(a[i].out), a[i].ldw, a[i].ldo, a[i].N};
   if (few_streams(M, K))
-    return launch_stream<T, SILU, PAIR>(static_cast<const T*>(x), o[0], o[1], M, K, ldx, cus * kFewMaxGroups, only_if, stream);
+    return launch_stream<T, SILU, PAIR>(static_cast<const T*>(x), o[0], o[1], M, K, ldx, cus * kFewMaxGroups, other, stream);
   const int tiles0 = (a[0].N + kTile - 1) / kTile, tiles = tiles0 + (PAIR ? (a[1].N + kTile - 1) / kTile : 0);
   const size_t lds = few_lds(M, K);
-  linear_few_kernel<T, SILU, PAIR><<<few_grid(tiles, lds, cus), kWaves * 64, lds, stream>>>(static_cast<const T*>(x), o[0], o[1], M, K, ldx, tiles0, tiles,
-                                                                                                          only_if);
+  linear_few_kernel<T, SILU, PAIR, Or><<<few_grid(tiles, lds, cus), kWaves * 64, lds, stream>>>(static_cast<const T*>(x), o[0], o[1], M, K, ldx, tiles0, tiles,
+                                                                                                other);
   return check_launch("odit_linear_few");
 }
 
-template <typename T, typename TT>
+template <typename T, typename TT, typename Or = Always>
 int run_sinusoid(const void* t, float neg_log_period, float scale, float pre, const FewArgs& a, int M, int K, int cus, hipStream_t stream,
-                 const int* only_if = nullptr) {
+                 const Or& other = Or{}) {
   const FewOut<T> o{static_cast<const T*>(a.w), static_cast<const T*>(a.bias), static_cast<T*>(a.out), a.ldw, a.ldo, a.N};
   const int tiles = (a.N + kTile - 1) / kTile;
   const size_t lds = few_lds(M, K);
-  linear_few_sinusoid_kernel<T, TT><<<few_grid(tiles, lds, cus), kWaves * 64, lds, stream>>>(
-      Sinusoid<TT>{static_cast<const TT*>(t), neg_log_period, scale, pre}, o, M, K, tiles, only_if);
+  linear_few_sinusoid_kernel<T, TT, Or><<<few_grid(tiles, lds, cus), kWaves * 64, lds, stream>>>(
+      Sinusoid<TT>{static_cast<const TT*>(t), neg_log_period, scale, pre}, o, M, K, tiles, other);
   return check_launch("odit_time_linear");
 }
 
@@ -368,28 +421,32 @@ static int few_go(const char* name, const void* x, odit::FewArgs (&a)[2], int co
 #undef ODIT_FEW
 }
 
-int odit::linear_few_if(const void* x, const void* w, const void* bias, void* out, int M, int N, int K, int64_t ldw, int dtype, const int* only_if, bool ask,
+int odit::linear_few_or(const void* x, const void* w, const void* bias, void* out, int M, int N, int K, int64_t ldw, int dtype, const FewOr& other, bool ask,
                         hipStream_t stream) {
   const FewArgs a[2] = {{w, bias, out, N, ldw, N}, {}};
   const int rc = few_check("odit_linear_few", a, 1, M, K, dtype);
   if (rc != ODIT_OK || ask) return rc;
   const int cus = device_cus();
   if (cus <= 0) { set_error("odit_linear_few: cannot read the device's compute-unit count"); return ODIT_ELAUNCH; }
-  return dtype == ODIT_BF16 ? run_few<bf16_t, true, false>(x, a, M, K, K, cus, stream, only_if)
-                            : run_few<f16_t, true, false>(x, a, M, K, K, cus, stream, only_if);
+#define ODIT_OR(T) \
+  run_few<T, true, false>(x, a, M, K, K, cus, stream, OrSilu<T>{other.few, static_cast<const T*>(other.x), static_cast<T*>(other.out), other.n})
+  return dtype == ODIT_BF16 ? ODIT_OR(bf16_t) : ODIT_OR(f16_t);
+#undef ODIT_OR
 }
 
-int odit::time_linear_if(const void* t, const void* w, const void* bias, void* out, int M, int N, int K, int64_t ldw, float neg_log_period, float scale,
-                         int t_dtype, int dtype, const int* only_if, bool ask, hipStream_t stream) {
+int odit::time_linear_or(const void* t, const void* w, const void* bias, void* out, int M, int N, int K, int64_t ldw, float neg_log_period, float scale,
+                         int t_dtype, int dtype, const FewOr& other, bool ask, hipStream_t stream) {
   const FewArgs a{w, bias, out, N, ldw, N};
   const int rc = few_check("odit_time_linear", &a, 1, M, K, dtype);
   if (rc != ODIT_OK || ask) return rc;
   const int cus = device_cus();
   if (cus <= 0) { set_error("odit_time_linear: cannot read the device's compute-unit count"); return ODIT_ELAUNCH; }
-  ODIT_DISPATCH_DTYPE(t_dtype, TT, {
-    return dtype == ODIT_BF16 ? run_sinusoid<bf16_t, TT>(t, neg_log_period, scale, 1.f, a, M, K, cus, stream, only_if)
-                              : run_sinusoid<f16_t, TT>(t, neg_log_period, scale, 1.f, a, M, K, cus, stream, only_if);
-  });
+#define ODIT_OR(T)                                                                                                                       \
+  run_sinusoid<T, TT>(t, neg_log_period, scale, 1.f, a, M, K, cus, stream,                                                                \
+                      OrSinusoid<T, TT>{other.few, static_cast<const TT*>(other.x), static_cast<T*>(other.out), other.n * (K / 2), K / 2, \
+                                        neg_log_period, scale})
+  ODIT_DISPATCH_DTYPE(t_dtype, TT, { return dtype == ODIT_BF16 ? ODIT_OR(bf16_t) : ODIT_OR(f16_t); });
+#undef ODIT_OR
   return ODIT_OK;
 }
 

@@ -2,10 +2,12 @@
 // time_proj(silu(temb)) for n tokens. Where an image or a first frame is given, its tokens have one timestep and the others
 // another, and n rows of these projections are two rows over and over (width 5120, 2706 tokens: 1 TFLOP, 770 us, an eighth of a
 // step of three blocks). So the distinct timesteps are found on the device (up to kRows, no synchronisation), those rows go
-// through the kernels for few rows, which stream the weights once (80 us), and every token is told which are its own. The launches for all tokens follow as ever, and end at once where the first ones have done
-// the work. us, before / two timesteps / all different: n=1000, width 5120 350 / 117 / 348; 2706, 5120 770 / 134 / 799; 9000, 3072
-// 918 / 134 / 953; 32760, 5120 8488 / 667 / 8507: where tokens have more timesteps the search and six launches that end at once
-// are 20 to 35 us.
+// through the kernels for few rows, which stream the weights once (80 us), and every token is told which are its own. Launches of the tile kernel for
+// all tokens stand in between and end at once where that went well; where it did not, the launches for few rows make those launches' operands instead
+// (the sinusoids, the SiLU), so that the calls that gain nothing pay for the search and for nothing else: seven launches, six without any of this. us,
+// every token's rows formed / two timesteps / all different: n=1000, width 5120 319 / 89 / 325; 2706, 5120 773 / 89 / 779; 9000, 3072 935 / 51 / 943;
+// 32760, 5120 8650 / 234 / 8615; where the products are small the search and a tile kernel that is not always the best one for them show: 500, 3072 95 /
+// - / 108, 2161, 1536 104 / - / 124, 16 us at most. (With launches of their own for the operands and a search of 26 us, 319 / 99 / 343, 773 / 100 / 790, 931 / 63 / 955.)
 #include "gemm_bf16.h"
 #include "time_sinusoid.h"
 #include "time_tokens.h"
@@ -25,47 +27,57 @@ struct TimeGroups {
 constexpr size_t kHeadBytes = 256;  // (every part on whole cache lines: rows 64 bytes off made the products 16 % slower)
 static_assert(sizeof(TimeGroups) <= kHeadBytes, "");
 
-// One workgroup: the first timestep that is none of those found so far, until there is none. `index`: each token's number
-// among them, its own where they are too many.
+// One workgroup: timesteps that are none of those found so far, until there is none or they are too many. `index`: each token's number among them, its
+// own where they are too many. A round is the compares, one candidate of each wavefront by ballot, one barrier, and every wavefront going through the
+// candidates: the launch is this chain, of one round where all are different. us, 2706 tokens, two timesteps / all different: 6.0 / 5.1; one timestep a
+// round 5.6 / 10.1; one a round by an LDS minimum over all lanes (64 lanes at one address, 4.5 a round) and two barriers 11.2 / 25.7.
 template <typename TT, typename Bits>
 __global__ __launch_bounds__(kThreads) void time_groups_kernel(const Bits* __restrict__ t, int n, TimeGroups* __restrict__ g, int* __restrict__ index) {
-  __shared__ int first[kRows + 1];
-  __shared__ Bits found;
-  const int tid = threadIdx.x;
-  if (tid <= kRows) first[tid] = n;
-  __syncthreads();
+  constexpr int kWaves = kThreads / 64;
+  __shared__ int has[2][kWaves];  // (by turns: a wavefront may be a round ahead of one that still reads)
+  __shared__ Bits found[2][kWaves];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   // (the first trip's timesteps stay in registers)
   Bits v[kRows], held[kEach];
 #pragma unroll
   for (int e = 0; e < kEach; ++e) held[e] = t[min(tid + e * kThreads, n - 1)];
-  int count = 0;
-  for (int k = 0; k <= kRows; ++k) {
-    int mine = n;
+  int count = 0, from = tid;  // what a thread has before `from` is known, and stays so
+  for (int k = 0; count <= kRows; ++k) {  // (a round finds one timestep at least, or ends)
+    bool mine = false;
     Bits its = 0;
-    for (int i0 = tid; i0 < n && mine == n; i0 += kThreads * kEach) {
+    while (from < n) {
       Bits b[kEach];
 #pragma unroll
-      for (int e = 0; e < kEach; ++e) b[e] = i0 == tid ? held[e] : t[min(i0 + e * kThreads, n - 1)];
+      for (int e = 0; e < kEach; ++e) b[e] = from == tid ? held[e] : t[min(from + e * kThreads, n - 1)];
 #pragma unroll
       for (int e = kEach - 1; e >= 0; --e) {
         bool known = false;
 #pragma unroll
-        for (int j = 0; j < kRows; ++j) known |= j < k && b[e] == v[j];
+        for (int j = 0; j < kRows; ++j) known |= j < count && b[e] == v[j];
         if (!known) {
-          mine = min(i0 + e * kThreads, n - 1);
+          mine = true;
           its = b[e];
         }
       }
+      if (mine) break;
+      from += kThreads * kEach;
     }
-    if (mine < n) atomicMin(&first[k], mine);
+    const uint64_t who = __ballot(mine);
+    if (lane == 0) has[k & 1][wave] = who != 0;
+    if (mine && (who & ((1ull << lane) - 1)) == 0) found[k & 1][wave] = its;
     __syncthreads();
-    if (first[k] == n) break;
-    ++count;
-    if (mine == first[k]) found = its;
-    __syncthreads();
+    uint64_t waves = __ballot(lane < kWaves && has[k & 1][lane % kWaves] != 0);
+    if (waves == 0) break;  // (the same for all)
+    const Bits theirs = found[k & 1][lane % kWaves];
+    while (waves != 0 && count <= kRows) {  // (every pass takes one timestep out, its own at least)
+      const int w = __builtin_ctzll(waves);
+      const Bits next = static_cast<Bits>(__builtin_amdgcn_readlane(static_cast<int>(theirs), w));
 #pragma unroll
-    for (int j = 0; j < kRows; ++j)
-      if (j == k) v[j] = found;
+      for (int j = 0; j < kRows; ++j)
+        if (j == count) v[j] = next;
+      ++count;
+      waves &= ~(__ballot(theirs == next));
+    }
   }
   const int few = count <= kRows ? count : 0;
   if (tid == 0) {
@@ -89,27 +101,11 @@ __global__ __launch_bounds__(kThreads) void time_groups_kernel(const Bits* __res
 }
 
 template <typename T, typename TT>
-__global__ __launch_bounds__(256) void token_sinusoid_kernel(const TT* __restrict__ t, T* __restrict__ out, int64_t n, int half, float neg_log_period, float scale,
-                                                             const TimeGroups* g) {
-  if (g != nullptr && g->few != 0) return;
+__global__ __launch_bounds__(256) void token_sinusoid_kernel(const TT* __restrict__ t, T* __restrict__ out, int64_t n, int half, float neg_log_period, float scale) {
   for (int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i < n * half; i += static_cast<int64_t>(gridDim.x) * 256) {
     const int64_t row = i / half;
     const int j = static_cast<int>(i - row * half);
     time_sinusoid<T>(t[row], j, half, neg_log_period, scale, 1.f, out[row * 2 * half + j], out[row * 2 * half + half + j]);
-  }
-}
-
-template <typename T>
-__global__ __launch_bounds__(256) void token_silu_kernel(const T* __restrict__ x, T* __restrict__ out, int64_t vecs, const TimeGroups* g) {
-  if (g->few != 0) return;
-  for (int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i < vecs; i += static_cast<int64_t>(gridDim.x) * 256) {
-    u32x4 r = load_raw(x + i * 8);
-#pragma unroll
-    for (int p = 0; p < 4; ++p) {
-      const float a = Raw<T>::get(r, 2 * p), b = Raw<T>::get(r, 2 * p + 1);
-      Raw<T>::set2(r, p, a / (1.f + __expf(-a)), b / (1.f + __expf(-b)));
-    }
-    store_raw(out + i * 8, r);
   }
 }
 
@@ -144,11 +140,9 @@ int run(const odit_time_tokens_args& a, const TokenScratch& at, char* s, void* w
   auto tile = [&](const void* x, int i, void* out, int N, int K, bool ask) {
     return linear_tile_unless(x, a.w[i], a.bias[i], out, n, N, K, a.ldw[i], dtype, workspace, workspace_bytes, few, ask, stream);
   };
-  auto some = [&](const void* x, int i, void* out, int N, int K, bool ask) {
-    return linear_few_if(x, a.w[i], a.bias[i], out, kRows, N, K, a.ldw[i], dtype, few, ask, stream);
-  };
-  auto first = [&](bool ask) {
-    return time_linear_if(g->value, a.w[0], a.bias[0], h4, kRows, a.C, a.K, a.ldw[0], a.neg_log_period, a.scale, t_dtype, dtype, few, ask, stream);
+  const int64_t vecs = static_cast<int64_t>(n) * (a.C / 8);
+  auto some = [&](const void* x, int i, void* out, int N, const void* of_all, bool ask) {
+    return linear_few_or(x, a.w[i], a.bias[i], out, kRows, N, a.C, a.ldw[i], dtype, FewOr{few, of_all, act, vecs}, ask, stream);
   };
   // (the first product, K of 256, is a fiftieth of the work: by any kernel, then for all tokens in either case)
   const bool first_tile = tile(rows, 0, hidden, a.C, a.K, true) == ODIT_OK;
@@ -159,27 +153,22 @@ int run(const odit_time_tokens_args& a, const TokenScratch& at, char* s, void* w
       time_groups_kernel<TT, Bits><<<1, kThreads, 0, stream>>>(static_cast<const Bits*>(a.t), n, g, a.index);
       rc = check_launch("odit_time_tokens (distinct timesteps)");
     }
-    go([&] { return first(ask); });
-    go([&] { return some(h4, 1, a.temb, a.C, a.C, ask); });
-    go([&] { return some(a.temb, 2, a.proj, a.P, a.C, ask); });
-    if (!ask && rc == ODIT_OK) {
-      token_sinusoid_kernel<T, TT><<<blocks(static_cast<int64_t>(n) * (a.K / 2)), 256, 0, stream>>>(
-          static_cast<const TT*>(a.t), static_cast<T*>(rows), n, a.K / 2, a.neg_log_period, a.scale, first_tile ? g : nullptr);
-      rc = check_launch("odit_time_tokens (rows)");
+    go([&] { return time_linear_or(g->value, a.w[0], a.bias[0], h4, kRows, a.C, a.K, a.ldw[0], a.neg_log_period, a.scale, t_dtype, dtype,
+                                   FewOr{few, a.t, first_tile ? rows : nullptr, n}, ask, stream); });
+    if (first_tile) {
+      go([&] { return tile(rows, 0, hidden, a.C, a.K, ask); });
+    } else if (!ask) {
+      go([&] {
+        token_sinusoid_kernel<T, TT><<<blocks(static_cast<int64_t>(n) * (a.K / 2)), 256, 0, stream>>>(static_cast<const TT*>(a.t), static_cast<T*>(rows), n,
+                                                                                                      a.K / 2, a.neg_log_period, a.scale);
+        return check_launch("odit_time_tokens (rows)");
+      });
+      go([&] { return odit_linear_rows(rows, a.w[0], a.bias[0], hidden, nullptr, nullptr, n, a.C, a.K, a.K, a.ldw[0], a.C, 0,
+                                       a.bias[0] != nullptr ? ODIT_EPI_BIAS : ODIT_EPI_NONE, dtype, dtype, 0, 0, 0, workspace, workspace_bytes, stream); });
     }
-    auto silu = [&](const void* x) {
-      if (ask) return static_cast<int>(ODIT_OK);
-      const int64_t vecs = static_cast<int64_t>(n) * (a.C / 8);
-      token_silu_kernel<T><<<blocks(vecs), 256, 0, stream>>>(static_cast<const T*>(x), static_cast<T*>(act), vecs, g);
-      return check_launch("odit_time_tokens (silu)");
-    };
-    if (first_tile) go([&] { return tile(rows, 0, hidden, a.C, a.K, ask); });
-    else if (!ask)
-      go([&] { return odit_linear_rows(rows, a.w[0], a.bias[0], hidden, nullptr, nullptr, n, a.C, a.K, a.K, a.ldw[0], a.C, 0, a.bias[0] != nullptr ? ODIT_EPI_BIAS : ODIT_EPI_NONE, dtype,
-                                       dtype, 0, 0, 0, workspace, workspace_bytes, stream); });
-    go([&] { return silu(hidden); });
+    go([&] { return some(h4, 1, a.temb, a.C, hidden, ask); });
     go([&] { return tile(act, 1, a.temb, a.C, a.C, ask); });
-    go([&] { return silu(a.temb); });
+    go([&] { return some(a.temb, 2, a.proj, a.P, a.temb, ask); });
     go([&] { return tile(act, 2, a.proj, a.P, a.C, ask); });
     if (rc != ODIT_OK) return rc;
   }
