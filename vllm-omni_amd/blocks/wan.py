@@ -419,11 +419,13 @@ class TokenRows:
     anything."""
 
     def __init__(self, rows: torch.Tensor, index: torch.Tensor):
-        self.rows, self.index = rows, index
+        self.rows, self.index, self._full = rows, index, None
 
     def full(self) -> torch.Tensor:
-        """[1, S, ...]"""
-        return self.rows.index_select(0, self.index).unsqueeze(0)
+        """[1, S, ...], written once for all the blocks that ask"""
+        if self._full is None:
+            self._full = self.rows.index_select(0, self.index).unsqueeze(0)
+        return self._full
 
     def unflatten(self, sizes: tuple[int, int]) -> "TokenRows":
         return TokenRows(self.rows.unflatten(-1, sizes), self.index)
