@@ -451,7 +451,7 @@ class WanTimeTextImageEmbedding(nn.Module):
         ``timestep_seq_len`` = S -> temb [B,S,C], timestep_proj [B,S,6C] (wan.py:282-296), with ``token_rows`` both as ``TokenRows``
         where one video's can be formed so."""
         mlp, dtype, done = self.time_embedder, self.time_embedder.linear_1.weight.dtype, None
-        if (timestep_seq_len is not None and timestep.shape[0] == timestep_seq_len and encoder_hidden_states.shape[0] == 1
+        if (token_rows and timestep_seq_len is not None and timestep.shape[0] == timestep_seq_len and encoder_hidden_states.shape[0] == 1
                 and encoder_hidden_states.dtype == dtype):
             done = kernels.time_tokens(mlp, self.time_proj, timestep, self.time_freq_dim, 10000, 1.0, dtype)
         if done is None:
@@ -460,8 +460,6 @@ class WanTimeTextImageEmbedding(nn.Module):
                 t = t.unflatten(0, (-1, timestep_seq_len))
         if done is not None:
             temb, timestep_proj = TokenRows(done[0], done[2]), TokenRows(done[1], done[2])
-            if not token_rows:
-                temb, timestep_proj = temb.full(), timestep_proj.full()
         elif encoder_hidden_states.shape[0] == 1:
             temb = mlp(t).type_as(encoder_hidden_states)
             timestep_proj = kernels.project(self.time_proj, temb, silu_input=True)
