@@ -17,6 +17,7 @@ def test_a_caller_without_rows_by_number(monkeypatch):
     asked = []
     monkeypatch.setattr(kernels, "time_tokens", lambda *a: asked.append(a) or (torch.zeros(4, 8), torch.zeros(4, 48), torch.zeros(4, dtype=torch.int32)))
     monkeypatch.setattr(kernels, "project", lambda lin, x, **kw: torch.zeros(*x.shape[:-1], lin.out_features))
+    monkeypatch.setattr(kernels, "gelu_tanh", lambda x, out=None: x)
     embed = WanTimeTextImageEmbedding(dim=8, time_freq_dim=16, time_proj_dim=48, text_embed_dim=4)
     args = (torch.rand(4), torch.zeros(1, 3, 4))
     with torch.inference_mode():
