@@ -1,5 +1,5 @@
 """The ends of a small model in two launches: the inputs' projections with the text's norm, and the head's norm with its projection; the bits of
-the launches one by one."""
+the launches one by one, where the kernel for small products takes those too, and a float32 sum of the same products, rounded once, in every element."""
 
 import pytest
 import torch
@@ -19,6 +19,22 @@ def _linear(gpu, k, n, dtype, bias=True):
     return lin
 
 
+def _twice(lin, rows):
+    """``lin`` of the rows [M, K] by the kernel for small products, as both problems of a pair; None where it does not take them."""
+    lib, (M, K), N = _lib.load(), rows.shape, lin.out_features
+    if not lib.odit_linear_pair_is_small(M, M, N, K):
+        return None
+    outs, q = [torch.full((M, N), float("nan"), device=rows.device, dtype=rows.dtype) for _ in range(2)], (_lib.LinearProblem * 2)()
+    for p, out in zip(q, outs):
+        p.x, p.w, p.bias, p.out, p.M = rows.data_ptr(), lin.weight.data_ptr(), None if lin.bias is None else lin.bias.data_ptr(), out.data_ptr(), M
+        p.ldx, p.ldw, p.ldo = K, K, N
+    code, epilogue = 0 if rows.dtype == BF16 else 1, _lib.ODIT_EPI_NONE if lin.bias is None else _lib.ODIT_EPI_BIAS
+    # (without a workspace no other kernel runs)
+    _lib.check(lib.odit_linear_pair(_lib.C.addressof(q), N, K, epilogue, 0, code, 0, None, 0, torch.cuda.current_stream().cuda_stream), "odit_linear_pair")
+    assert torch.equal(*outs)
+    return outs[0]
+
+
 # (rows and K of both; every number of steps on either side, edges of tiles of 64)
 @pytest.mark.parametrize("M0,K0,M1,K1,N", [(256, 64, 64, 256, 256), (1, 64, 1, 64, 64), (63, 192, 65, 128, 72), (128, 256, 7, 64, 520), (300, 128, 200, 256, 8), (64, 64, 64, 128, 256)])
 @pytest.mark.parametrize("dtype,bias", [(BF16, True), (F16, True), (F16, False)])
@@ -34,13 +50,17 @@ def test_stem(gpu, M0, K0, M1, K1, N, dtype, bias):
     with torch.inference_mode():
         got = kernels.project_stem(a, x, norm, b, y)
         normed = norm(y)
+        u = 2.0 ** -8 if dtype == BF16 else 2.0 ** -11
         for out, lin, rows in zip(got, (a, b), (x, normed), strict=True):
-            problem, want = _lib.LinearProblem(), torch.empty_like(out)
-            problem.x, problem.w, problem.bias, problem.out = rows.data_ptr(), lin.weight.data_ptr(), lin.bias.data_ptr() if bias else None, want.data_ptr()
-            # whichever kernel takes it alone: a float32 sum of the same products, rounded once
-            want = kernels.project(lin, rows)
+            exact, size = (torch.nn.functional.linear(f(rows.double()), f(lin.weight.double()), f(lin.bias.double()) if bias else None) for f in (lambda t: t, torch.abs))
+            # the result's rounding and that of K + 1 float32 sums (an element of float16 may be below the normal numbers)
+            assert bool(((out.double() - exact).abs() <= u * exact.abs() + (lin.in_features + 1) * 2.0 ** -23 * size + 2.0 ** -25).all())
+            want = kernels.project(lin, rows)  # (whichever kernel takes it alone)
             assert float((out.double() - want.double()).norm()) <= (2.0 ** -9 if dtype == BF16 else 2.0 ** -12) * float(want.double().norm())
-        if K1 > 64 and N >= 64:  # and by the kernel for small products, a row at a time in any launch, its bits
+            alone = _twice(lin, rows[0])
+            if alone is not None:
+                assert torch.equal(out[0], alone)
+        if K1 > 64 and N >= 64:  # a row at a time, in any launch, the same bits
             assert torch.equal(got[1], kernels.project_stem(a, x[:, :1], norm, b, y)[1]) and torch.equal(got[0], kernels.project_stem(a, x, norm, b, y[:, :1])[0])
 
 

@@ -190,3 +190,23 @@ def test_where_a_timestep_stands_first(gpu, n, places):
     else:
         numbers = [index[t == v].unique() for v in values]
         assert all(len(i) == 1 for i in numbers) and sorted(int(i) for i in numbers) == list(range(len(values)))
+
+
+@pytest.mark.parametrize("distinct", [2, 5])
+def test_two_videos(gpu, distinct):
+    """A batch goes the way it always went, whatever its timesteps: each video's result is that of the video alone but for the order of float32 sums."""
+    from vllm_omni_amd.blocks.wan import WanTransformer3DModel
+
+    g = torch.Generator(device=gpu).manual_seed(7)
+    model = WanTransformer3DModel(num_attention_heads=12, attention_head_dim=128, ffn_dim=2048, num_layers=2, text_dim=256, cross_attn_norm=True).to(device=gpu, dtype=BF16)
+    with torch.no_grad():
+        for p in model.parameters():
+            p.normal_(0.0, 0.03, generator=g)
+    x, text = torch.randn(2, 16, 5, 40, 48, device=gpu, generator=g).to(BF16), torch.randn(2, 20, 256, device=gpu, generator=g).to(BF16)
+    t = (torch.arange(2400, device=gpu) % distinct * 200.0)[None] + torch.tensor([[0.0], [37.0]], device=gpu)
+    with torch.inference_mode():
+        both = model(x, t, text, return_dict=False)[0]
+        for i in range(2):
+            one = model(x[i:i + 1], t[i:i + 1], text[i:i + 1], return_dict=False)[0][0]
+            # (last bits of float32 sums: far less than the type's own rounding, half a step in every element)
+            assert bool(torch.isfinite(one).all()) and float((both[i].float() - one.float()).norm()) < 2.0 ** -8 * float(one.float().norm())
