@@ -907,9 +907,9 @@ static int launch_dma(AttnParams& p, hipStream_t stream, void* ws, size_t ws_byt
 // 32760 queries x 512 keys x 40 heads, 901 / 947). (With the two halves' roles paired wrongly, wavefronts w and
 // w + 1 or w and w + 2 in anti-phase instead of w and w + 4, the same kernel is 10 to 18 % slower: two wavefronts of a
 // SIMD in the same stage is what costs, and independent workgroups already avoid it most of the time by themselves.)
-// Since the softmax's vector work was cut the two are closer, and at head size 128 (us, 4 / 8, one box, the same bits)
+// Since the softmax's vector work was cut the two are closer, and at head size 128 (us, 4 / 8, the same bits; the largest on another box than the others)
 //   from 128 key tiles on 8 are ahead wherever there is a round of units:  B=1 S=8192 H=24 736 / 728, B=2 1475 / 1449, S=16384 H=40 4814 / 4754,
-//     B=2 S=32760 H=40 36223 / 35657;
+//     B=2 S=32760 H=40 37490 / 37000;
 //   below, 4 are, whose units are half as large: of few units every compute unit has one (B=1 S=2100 H=8, 136 units, 41.6 / 54.8, S=4096
 //     77.1 / 93.0, 700 queries x 4096 keys H=24 68.6 / 91.3), and a last round is filled better (B=1 H=40 S=2100 105 / 120, B=4 H=16 S=2500
 //     210 / 224, B=1 S=3600 H=24 174 / 195, S=6000 H=16 286 / 310, B=2 S=2390 H=24 146 / 151, 16384 queries x 2048 keys H=40 651 / 660);

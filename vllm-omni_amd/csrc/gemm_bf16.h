@@ -93,7 +93,7 @@ int launch_gemm_tile_heads(const GemmCall* c, int count, const HeadsOut* heads, 
 bool gemm_small_rule(const GemmCall* c, int count, int cus, int max_k);
 int launch_gemm_small(const GemmCall* c, int count, int dtype, hipStream_t stream);
 // LayerNorm without affine and modulation of a problem's rows, x' = norm(x) (1 + scale) + shift, in front of the product: shift and scale of
-// the tensors' type, one row for S rows of x, `stride` elements apart. For two problems of K <= kSmallNormK.
+// the tensors' type, one row for S rows of x, `stride` elements apart. For one problem or two of K <= kSmallNormK.
 struct RowNorm {
   const void *shift, *scale;
   int64_t stride;

@@ -473,7 +473,10 @@ template <typename T> static bool qk_dense(const QkArgs& a) {
     // Results of 32 to 128 MB go to the caches: what comes next, the rotation mostly, finds them in the last-level cache (256 MB). Smaller ones
     // come back from the L2s' way to memory anyway and are flushed from there at the launch's end, larger ones are displaced before they
     // are read. us, norm and rotation, past the caches / to them: 10 MB 7.7 / 8.2, 25 MB 21.0 / 21.0 (the norm alone 7.2 / 11.2), 37 MB 28.8 /
-    // 27.6, 61 MB 44.4 / 41.7, 104 MB 69.3 / 66.1, 123 MB 80.1 / 79.4, 168 MB 110 / 112 (alone 48 / 58).
+    // 27.6, 61 MB 44.4 / 41.7, 104 MB 69.3 / 66.1, 123 MB 80.1 / 79.4, 168 MB 110 / 112 (alone 48 / 58). Between the lines the norm alone, past the
+    // caches / to them / qknorm_flat_kernel: with its inputs in the last-level cache 41 MB 13.0 / 13.6 / 14.6, 61 MB 18.5 / 19.0 / 20.4, 104 MB 29.9 /
+    // 30.8 / 32.5, from memory 61 MB 22.7 / 21.5 / 23.9, 104 MB 36.1 / 34.3 / 37.7; behind the old kernel only where inputs that just fit that cache
+    // come again and again and the results push them out (four of 61 MB in turn 18.4 / 21.6 / 20.3).
     const bool keep = vec >= (2 << 20) && vec <= (8 << 20);
     const dim3 grid(static_cast<unsigned>((vec + 511) / 512));
     auto go = [&](auto k) {
