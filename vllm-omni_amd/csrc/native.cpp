@@ -443,11 +443,10 @@ PyObject* py_qknorm_rope_pair(PyObject*, PyObject* const* a, Py_ssize_t n) {
 // ----------------------------------------------------------------------------------------------- layers
 // RMSNorm.forward_hip: (x, weight, eps): every row of the last axis on its own
 PyObject* rmsnorm(const Tensor* x, const Tensor* wt, double eps) {
-  const Where w;
   const int dt = code_of(*x);
-  if (dt < 0 || x->dim() < 1 || !w.holds(x) || !w.holds(wt) || !x->is_contiguous() || wt->scalar_type() != x->scalar_type() ||
-      !wt->is_contiguous())
-    return none();
+  if (dt < 0 || x->dim() < 1 || !x->is_contiguous() || wt->scalar_type() != x->scalar_type() || !wt->is_contiguous()) return none();
+  const Where w;
+  if (!w.holds(x) || !w.holds(wt)) return none();
   const int64_t width = x->size(-1);
   if (wt->numel() != width || width == 0) return none();
   const int64_t rows = x->numel() / width;
@@ -483,8 +482,12 @@ PyObject* py_rmsnorm(PyObject*, PyObject* const* a, Py_ssize_t n) {
 
 // RotaryEmbedding.forward_hip: (x [B,S,H,D], cos, sin float32 [S, rot/2], flags)
 PyObject* rotary(const Tensor* x, const Tensor* cs, const Tensor* sn, unsigned flags) {
+  // (what the layer's call and then its method ask for in vain is found out before anything is allocated)
+  if (x->dim() != 4 || code_of(*x) < 0 || x->stride(3) != 1 || x->stride(2) != x->size(3) || cs->dim() != 2 || cs->scalar_type() != at::kFloat ||
+      sn->scalar_type() != at::kFloat)
+    return none();
   const Where w;
-  if (x->dim() != 4 || code_of(*x) < 0 || !w.holds(x)) return none();
+  if (!w.holds(x)) return none();
   Tensor out = fresh(x->sizes(), x->options());
   QkProblem p;
   if (!qk_problem(w, x, nullptr, nullptr, &out, nullptr, nullptr, nullptr, nullptr, cs, sn, ODIT_NORM_NONE, &p)) return none();
