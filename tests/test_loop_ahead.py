@@ -212,6 +212,15 @@ def test_qwen_own_steps():
         assert not kernels.own_tree(pipe.transformer)  # (a class of this file)
 
 
+def test_flux_forms_each_timestep_once(monkeypatch):
+    """Also where the model forms nothing ahead."""
+    model, made, full = _Recorder(), [], torch.full
+    model.loop_steps = lambda *a: None
+    monkeypatch.setattr(denoise.torch, "full", lambda *a, **kw: made.append(a) or full(*a, **kw))
+    _flux_loop(model, torch.zeros(1, 2, 3))
+    assert sum(1 for a in made if a[1] != 3.5) == 5
+
+
 def test_own_tree():
     norm = FluxTransformer2DModel(num_layers=1, num_single_layers=0, attention_head_dim=64, num_attention_heads=1, joint_attention_dim=32,
                                   pooled_projection_dim=8, axes_dims_rope=(8, 28, 28))

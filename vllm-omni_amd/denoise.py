@@ -119,7 +119,7 @@ def diffuse_flux(transformer, latents: torch.Tensor, prompt_embeds: torch.Tensor
         every = torch.cat([timestep(i) for i in range(num_inference_steps)])
         steps = transformer.loop_steps(every, guidance, pooled_prompt_embeds, prompt_embeds, img_ids, txt_ids)
     for i in range(num_inference_steps):
-        t = timestep(i) if steps is None else every[i:i + 1]
+        t = timestep(i) if every is None else every[i:i + 1]
         noise = transformer(hidden_states=latents, encoder_hidden_states=prompt_embeds,
                             pooled_projections=pooled_prompt_embeds, timestep=t, img_ids=img_ids, txt_ids=txt_ids,
                             guidance=guidance, return_dict=False, **({} if steps is None else {"step": steps.at(i)}))[0]
