@@ -210,3 +210,22 @@ def test_two_videos(gpu, distinct):
             one = model(x[i:i + 1], t[i:i + 1], text[i:i + 1], return_dict=False)[0][0]
             # (last bits of float32 sums: far less than the type's own rounding, half a step in every element)
             assert bool(torch.isfinite(one).all()) and float((both[i].float() - one.float()).norm()) < 2.0 ** -8 * float(one.float().norm())
+
+
+@pytest.mark.parametrize("distinct", [2, 5])
+@pytest.mark.parametrize("dtype", [BF16, F16])
+def test_first_product_by_another_kernel(gpu, dtype, distinct):
+    """96 cosines and sines: a reduction that the tile kernel does not take, so the first product of all tokens is made in either case."""
+    print(f"96 sinusoids, {distinct} distinct {dtype}", flush=True)
+    torch.manual_seed(distinct)
+    emb, proj = TimestepEmbedding(96, 1536).to(device=gpu, dtype=dtype), torch.nn.Linear(1536, 9216, device=gpu, dtype=dtype)
+    t = torch.arange(2706, device=gpu) % distinct * 100.0
+    with torch.inference_mode(), torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        got = _spread(kernels.time_tokens(emb, proj, t, 96, 10000, 1.0, dtype))
+        torch.cuda.synchronize()
+    assert any("token_sinusoid_kernel" in e.key for e in prof.key_averages())
+    with torch.inference_mode():
+        temb = emb(QwenTimestepProjEmbeddings.time_proj(t, dim=96, scale=1.0, dtype=dtype))
+        # the same sums in another order and their roundings, three products deep
+        for a, b in zip(got, (temb, kernels.project(proj, temb, silu_input=True)), strict=True):
+            assert bool(torch.isfinite(a).all()) and float((a.double() - b.double()).norm()) < (2.0 ** -7 if dtype == BF16 else 2.0 ** -10) * float(b.double().norm())
