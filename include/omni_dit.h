@@ -514,6 +514,24 @@ int odit_linear_few_pair(const void* x, const void* const w[2], const void* cons
 int odit_time_linear(const void* t, const void* w, const void* bias, void* out, int M, int N, int K, int64_t ldw, int64_t ldo,
                      float neg_log_period, float scale, float pre, int t_dtype, int dtype, void* stream);
 
+/* An embedder: silu(in W1^T + bias1) W2^T + bias2 (biases may be NULL). `in` is the cosines and sines of timesteps x [M], as odit_time_linear
+ * forms them (t_dtype: their type), or rows x [M, K] of the call's type (t_dtype -1). W1 is [N, K], W2 [N, N]. */
+typedef struct odit_embedder {
+  const void* x;
+  int64_t ldx;
+  int K, t_dtype;
+  float neg_log_period, scale, pre;
+  const void *w1, *bias1, *w2, *bias2;
+  int64_t ldw1, ldw2;
+} odit_embedder;
+
+/* out [M, N] = the embedders' results, each rounded to `dtype`, added up from the first to the last with a rounding each: the conditioning of a
+ * step by timestep, guidance and pooled text (flux_transformer.py:462-466, 537-541) in two launches. The bits of odit_time_linear or odit_linear_few
+ * for each first projection, odit_linear_few for each second one and a sum for every further embedder. Up to three; up to 4 rows, N a multiple of
+ * 512, first reductions that are not (with M K up to 27306 elements) a multiple of 512; ODIT_ENOTSUP for anything else, with nothing launched.
+ * `hidden`: scratch for count * M * N elements. */
+int odit_embed_sum(const odit_embedder* embedders, int count, int M, int N, void* hidden, void* out, int dtype, void* stream);
+
 /* odit_adaln_modulate and odit_gated_residual_adaln (its norm with ln_weight and ln_bias alone; out null: none) for S tokens that have row
  * index[s] (int32, on the device; every one a row of the table) of shift, scale and gate, `mod_stride` or `gate_stride` elements apart. Rows of x,
  * out, h and y as there, h, y, x and out of the second dense; the float32 [C] tables are added to the rows. */

@@ -132,6 +132,7 @@ _SIGNATURES = {
     "odit_time_linear": (
         C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_int64, C.c_int64, C.c_float, C.c_float,
                   C.c_float, C.c_int, C.c_int, C.c_void_p]),
+    "odit_embed_sum": (C.c_int, [C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_void_p, C.c_void_p, C.c_int, C.c_void_p]),
     "odit_adaln_modulate_rows": (
         C.c_int, [C.c_void_p] * 7 + [C.c_int, C.c_int, C.c_int64, C.c_int64, C.c_int64, C.c_float, C.c_int, C.c_int, C.c_void_p]),
     "odit_gated_residual_adaln_rows": (
@@ -180,6 +181,13 @@ class LinearProblem(C.Structure):
 
     _fields_ = [(n, C.c_void_p) for n in ("x", "w", "bias", "residual", "gate", "out")] + [("M", C.c_int), ("rows_per_gate", C.c_int)] + [
         (n, C.c_int64) for n in ("ldx", "ldw", "ldo", "ldr", "gate_stride")]
+
+
+class Embedder(C.Structure):
+    """``odit_embedder``."""
+
+    _fields_ = [("x", C.c_void_p), ("ldx", C.c_int64), ("K", C.c_int), ("t_dtype", C.c_int)] + [(n, C.c_float) for n in ("neg_log_period", "scale", "pre")] + [
+        (n, C.c_void_p) for n in ("w1", "bias1", "w2", "bias2")] + [("ldw1", C.c_int64), ("ldw2", C.c_int64)]
 
 
 class TimeTokens(C.Structure):

@@ -373,6 +373,10 @@ class CombinedTimestepGuidanceTextProjEmbeddings(nn.Module):
 
     def forward(self, timestep: torch.Tensor, guidance: torch.Tensor | None, pooled_projection: torch.Tensor,
                 pre: float = 1.0):
+        done = kernels.embed_sum(self.timestep_embedder, timestep, None if guidance is None else self.guidance_embedder, guidance, self.text_embedder,
+                                 pooled_projection, 256, 10000, 1.0, pre)
+        if done is not None:
+            return done
         embed, dtype = QwenTimestepProjEmbeddings.embed, pooled_projection.dtype
         emb = embed(self.timestep_embedder, timestep, dtype, scale=1.0, pre=pre)
         if guidance is not None:
@@ -632,4 +636,4 @@ class FluxTransformer2DModel(nn.Module):
                 p.copy_(weights[k].to(device=p.device, dtype=p.dtype))
 
 
-kernels.native_classes(FluxAttention=FluxAttention, AdaLayerNormZeroSingle=AdaLayerNormZeroSingle)
+kernels.native_classes(FluxAttention=FluxAttention, AdaLayerNormZeroSingle=AdaLayerNormZeroSingle, PixArtAlphaTextProjection=PixArtAlphaTextProjection)

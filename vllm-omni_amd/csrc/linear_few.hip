@@ -94,9 +94,10 @@ __device__ __forceinline__ void stage_sinusoid(const Sinusoid<TT>& a, u32x4* xs,
   }
 }
 
-// tiles0: of the first weight. PAIR: of two (a template, so that one costs no selects: 442368 features, two rows 418 us, with them 421)
+// tiles0: of the first weight. PAIR: of two (a template, so that one costs no selects: 442368 features, two rows 418 us, with them 421). `from`: the
+// workgroup's first tile.
 template <typename T, bool PAIR, typename Stage>
-__device__ __forceinline__ void few_rows(Stage&& stage, const FewOut<T>& o0, const FewOut<T>& o1, int M, int K, int tiles0, int tiles) {
+__device__ __forceinline__ void few_rows(Stage&& stage, const FewOut<T>& o0, const FewOut<T>& o1, int M, int K, int tiles0, int tiles, int from) {
   extern __shared__ u32x4 lds[];
   f32x4* red = reinterpret_cast<f32x4*>(lds);
   u32x4* xs = lds + kRedBytes / 16;
@@ -159,7 +160,7 @@ __device__ __forceinline__ void few_rows(Stage&& stage, const FewOut<T>& o0, con
   auto next = [&](int& tile, int& chunk) {
     if (++chunk == chunks) { chunk = 0; tile += gridDim.x; }
   };
-  int tile = blockIdx.x, chunk = 0;
+  int tile = from, chunk = 0;
   fetch(a, tile, chunk);
   while (true) {
     int tile1 = tile, chunk1 = chunk;
@@ -223,13 +224,13 @@ template <typename T, bool SILU, bool PAIR, typename Or>
 __global__ __launch_bounds__(kWaves * 64, 6) void linear_few_kernel(const T* __restrict__ x, const FewOut<T> o0, const FewOut<T> o1, int M, int K,
                                                                     int64_t ldx, int tiles0, int tiles, const Or other) {
   if (other.instead()) return;
-  few_rows<T, PAIR>([&](u32x4* xs, int vecs, int pitch) { stage_rows<T, SILU>(x, xs, M, vecs, pitch, ldx); }, o0, o1, M, K, tiles0, tiles);
+  few_rows<T, PAIR>([&](u32x4* xs, int vecs, int pitch) { stage_rows<T, SILU>(x, xs, M, vecs, pitch, ldx); }, o0, o1, M, K, tiles0, tiles, blockIdx.x);
 }
 template <typename T, typename TT, typename Or>
 __global__ __launch_bounds__(kWaves * 64, 6) void linear_few_sinusoid_kernel(const Sinusoid<TT> a, const FewOut<T> o, int M, int K, int tiles,
                                                                              const Or other) {
   if (other.instead()) return;
-  few_rows<T, false>([&](u32x4* xs, int, int pitch) { stage_sinusoid<T, TT>(a, xs, M, K, pitch); }, o, o, M, K, tiles, tiles);
+  few_rows<T, false>([&](u32x4* xs, int, int pitch) { stage_sinusoid<T, TT>(a, xs, M, K, pitch); }, o, o, M, K, tiles, tiles, blockIdx.x);
 }
 
 // (groups of R features; those of the first weight come first)
@@ -311,6 +312,109 @@ __global__ __launch_bounds__(kWaves * 64, 6) void linear_stream_kernel(const T* 
   }
 }
 
+// Up to three embedders, two projections each with a SiLU between, and the sum of their results. Each by itself is a chain of two launches that wait
+// more than they read (2 to 5 and 19 MB at width 3072), and none hangs on another: the first projections are one launch, the second ones and the sums
+// another, in which the wavefronts of a workgroup share out the embedders of the features and meet in LDS. Timestep, guidance and 768 values of pooled
+// text at width 3072, one row, us under the profiler: 5.7 + 7.7, 5.8 + 7.4, 5.4 + 7.4 and two sums of 4.8 / 9.3 + 13.5; a step of 1024 + 512 tokens without
+// it 4455 -> 4434.
+constexpr int kEmbedders = 3;
+struct EmbedInput {
+  const void* x;  // timesteps [M], or rows
+  int64_t ldx;
+  int K, t_dtype;  // t_dtype -1: rows
+  float neg_log_period, scale, pre;
+};
+template <typename T> struct EmbedFirst {
+  EmbedInput in[kEmbedders];
+  FewOut<T> out[kEmbedders];
+};
+template <typename T>
+__global__ __launch_bounds__(kWaves * 64, 6) void embed_first_kernel(const EmbedFirst<T> p, int M, int tiles) {
+  const int which = blockIdx.x / tiles;
+  const EmbedInput& in = p.in[which];
+  few_rows<T, false>([&](u32x4* xs, int vecs, int pitch) {
+    auto sinusoid = [&](auto type) {
+      using TT = decltype(type);
+      stage_sinusoid<T, TT>(Sinusoid<TT>{static_cast<const TT*>(in.x), in.neg_log_period, in.scale, in.pre}, xs, M, in.K, pitch);
+    };
+    if (in.t_dtype < 0) stage_rows<T, false>(static_cast<const T*>(in.x), xs, M, vecs, pitch, in.ldx);
+    else if (in.t_dtype == ODIT_F32) sinusoid(0.f);
+    else if (in.t_dtype == ODIT_BF16) sinusoid(bf16_t{});
+    else sinusoid(f16_t{});
+  }, p.out[which], p.out[which], M, in.K, tiles, tiles, static_cast<int>(blockIdx.x) - which * tiles);
+}
+
+template <typename T> struct EmbedSecond {
+  const T* hidden;  // [count, rows, N]
+  const T *w[kEmbedders], *bias[kEmbedders];
+  int64_t ldw[kEmbedders];
+  T* out;
+};
+template <typename T, int M>
+__global__ __launch_bounds__(kWaves * 64, 6) void embed_second_kernel(const EmbedSecond<T> p, int count, int rows, int N) {
+  constexpr int R = 2;  // features of a wavefront
+  extern __shared__ u32x4 lds[];
+  __shared__ float part[kWaves][R * M];
+  const int vecs = N / 8, each = rows * vecs;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int places = kWaves / count, which = wave % count, place = wave / count;
+  const int g = blockIdx.x * places + place, chunks = N / 512;
+  const T* const mine = p.w[which] + lane * 8;
+  auto fetch = [&](u32x4 (&r)[R], int c) {  // (past the last feature and the last chunk the loads repeat it)
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+      r[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(mine + min(g * R + i, N - 1) * p.ldw[which] + min(c, chunks - 1) * 512));
+  };
+  u32x4 a[R], b[R];
+  fetch(a, 0);
+  stage_rows<T, true>(p.hidden, lds, count * rows, vecs, vecs, N);
+  __syncthreads();
+  if (place < places && g * R < N) {
+    const u32x4* const x = lds + which * each + lane;
+    float acc[R][M];
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+#pragma unroll
+      for (int m = 0; m < M; ++m) acc[i][m] = 0.f;
+    auto use = [&](const u32x4 (&r)[R], int c) {  // (linear_stream_kernel's sums)
+#pragma unroll
+      for (int m = 0; m < M; ++m) {
+        const u32x4 v = x[min(m, rows - 1) * vecs + c * 64];
+#pragma unroll
+        for (int i = 0; i < R; ++i)
+#pragma unroll
+          for (int j = 0; j < 8; ++j) acc[i][m] = fmaf(Raw<T>::get(r[i], j), Raw<T>::get(v, j), acc[i][m]);
+      }
+    };
+    for (int c = 0;;) {
+      fetch(b, c + 1);
+      use(a, c);
+      if (++c >= chunks) break;
+      fetch(a, c + 1);
+      use(b, c);
+      if (++c >= chunks) break;
+    }
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+#pragma unroll
+      for (int m = 0; m < M; ++m) {
+        const float s = wave_sum(acc[i][m]);
+        const T* const bias = p.bias[which];
+        if (lane == i * M + m)
+          part[wave][lane] = to_float(from_float<T>(s + (bias != nullptr ? to_float(bias[min(g * R + i, N - 1)]) : 0.f)));
+      }
+  }
+  __syncthreads();
+  if (threadIdx.x < places * R * M) {
+    const int at = threadIdx.x / (R * M), i = threadIdx.x % (R * M) / M, m = threadIdx.x % M, n = (blockIdx.x * places + at) * R + i;
+    if (n < N && m < rows) {
+      float v = part[at * count][i * M + m];
+      for (int e = 1; e < count; ++e) v = to_float(from_float<T>(v + part[at * count + e][i * M + m]));
+      p.out[static_cast<int64_t>(m) * N + n] = from_float<T>(v);
+    }
+  }
+}
+
 // Rows of W a wavefront takes at a time: two; four (twice the loads in flight, half the steps) where every wavefront of the grid
 // has three or more such groups and one or two rows of x leave the registers for it: N=442368, two rows of x 414 / 405 us,
 // 73728 69.5 / 68.1, but 36864 36.5 / 37.3, 9216 13.2 / 15.0; with four rows of x 440 / 566.
@@ -380,6 +484,35 @@ int run_sinusoid(const void* t, float neg_log_period, float scale, float pre, co
   linear_few_sinusoid_kernel<T, TT, Or><<<few_grid(tiles, lds, cus), kWaves * 64, lds, stream>>>(
       Sinusoid<TT>{static_cast<const TT*>(t), neg_log_period, scale, pre}, o, M, K, tiles, other);
   return check_launch("odit_time_linear");
+}
+
+template <typename T>
+int run_embed(const odit_embedder* e, int count, int M, int N, void* hidden, void* out, hipStream_t stream) {
+  EmbedFirst<T> a;
+  EmbedSecond<T> b;
+  int widest = 0;
+  b.hidden = static_cast<const T*>(hidden);
+  b.out = static_cast<T*>(out);
+  for (int i = 0; i < kEmbedders; ++i) {
+    const odit_embedder& m = e[i < count ? i : 0];
+    a.in[i] = EmbedInput{m.x, m.ldx, m.K, m.t_dtype, m.neg_log_period, m.scale, m.pre};
+    a.out[i] = FewOut<T>{static_cast<const T*>(m.w1), static_cast<const T*>(m.bias1), static_cast<T*>(hidden) + static_cast<int64_t>(i) * M * N, m.ldw1, N, N};
+    b.w[i] = static_cast<const T*>(m.w2);
+    b.bias[i] = static_cast<const T*>(m.bias2);
+    b.ldw[i] = m.ldw2;
+    if (m.K > widest) widest = m.K;
+  }
+  const int tiles = (N + kTile - 1) / kTile;
+  embed_first_kernel<T><<<count * tiles, kWaves * 64, few_lds(M, widest), stream>>>(a, M, tiles);
+  const int rc = check_launch("odit_embed_sum");
+  if (rc != ODIT_OK) return rc;
+  const int groups = (N + 1) / 2, places = kWaves / count;
+  const dim3 grid((groups + places - 1) / places);
+  const size_t lds = static_cast<size_t>(count) * M * N * 2;
+  if (M > 2) embed_second_kernel<T, 4><<<grid, kWaves * 64, lds, stream>>>(b, count, M, N);
+  else if (M == 2) embed_second_kernel<T, 2><<<grid, kWaves * 64, lds, stream>>>(b, count, M, N);
+  else embed_second_kernel<T, 1><<<grid, kWaves * 64, lds, stream>>>(b, count, M, N);
+  return check_launch("odit_embed_sum");
 }
 
 }  // namespace
@@ -487,4 +620,30 @@ extern "C" int odit_time_linear(const void* t, const void* w, const void* bias, 
                               : run_sinusoid<f16_t, TT>(t, neg_log_period, scale, pre, a, M, K, cus, s);
   });
   return ODIT_OK;
+}
+
+extern "C" int odit_embed_sum(const odit_embedder* embedders, int count, int M, int N, void* hidden, void* out, int dtype, void* stream) {
+  using namespace odit;
+  ODIT_CHECK_ARG(embedders && hidden && out, "odit_embed_sum: null arguments");
+  ODIT_CHECK_ARG(count >= 1 && count <= kEmbedders && M >= 0 && N > 0, "odit_embed_sum: bad shape count=%d M=%d N=%d", count, M, N);
+  bool takes = N % 8 == 0 && aligned16(hidden) && few_streams(M, N) && static_cast<size_t>(count) * M * N * 2 <= kFewMaxLds - kWaves * 64;
+  for (int i = 0; i < count; ++i) {
+    const odit_embedder& e = embedders[i];
+    ODIT_CHECK_ARG(e.x && e.K > 0, "odit_embed_sum: bad input of embedder %d", i);
+    ODIT_CHECK_ARG(e.t_dtype >= -1 && e.t_dtype <= ODIT_F32, "odit_embed_sum: bad timestep type %d", e.t_dtype);
+    const FewArgs a[2] = {{e.w1, e.bias1, hidden, N, e.ldw1, N}, {e.w2, e.bias2, out, N, e.ldw2, N}};
+    int rc = few_check("odit_embed_sum", a, 1, M, e.K, dtype);
+    if (rc == ODIT_OK) rc = few_check("odit_embed_sum", a + 1, 1, M, N, dtype);
+    if (rc != ODIT_OK) return rc;
+    // (a first projection that the stream kernel would take has another order of summation)
+    takes = takes && !few_streams(M, e.K) && (e.t_dtype < 0 ? e.ldx >= e.K && e.ldx % 8 == 0 && aligned16(e.x) : e.K % 2 == 0);
+  }
+  if (!takes) {
+    set_error("odit_embed_sum: takes up to %d rows, N a multiple of 512, rows of 16-byte alignment and first reductions that odit_linear_few's matrix kernel runs "
+              "(count=%d M=%d N=%d)", kStreamMaxRows, count, M, N);
+    return ODIT_ENOTSUP;
+  }
+  if (M == 0) return ODIT_OK;
+  const hipStream_t s = static_cast<hipStream_t>(stream);
+  return dtype == ODIT_BF16 ? run_embed<bf16_t>(embedders, count, M, N, hidden, out, s) : run_embed<f16_t>(embedders, count, M, N, hidden, out, s);
 }

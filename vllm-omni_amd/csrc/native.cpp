@@ -947,7 +947,7 @@ struct Names {
 Names g_name;
 PyTypeObject *g_linear_type, *g_rmsnorm_type, *g_rownorm_type, *g_adaln_type, *g_attention_type, *g_attention_impl_type,
     *g_feed_forward_type, *g_gelu_type, *g_wan_ffn_type, *g_qwen_attention_type, *g_flux_attention_type, *g_flux_single_norm_type,
-    *g_wan_self_type, *g_wan_cross_type, *g_time_embedding_type, *g_rotary_type;
+    *g_wan_self_type, *g_wan_cross_type, *g_time_embedding_type, *g_rotary_type, *g_text_projection_type;
 
 PyObject* instance_dict(PyObject* m) {
   PyObject** d = m ? _PyObject_GetDictPtr(m) : nullptr;
@@ -1297,6 +1297,47 @@ PyObject* py_time_embedding(PyObject*, PyObject* const* a, Py_ssize_t n) {
                                                 l2.n, c.dtype, 1, c.where.stream);
   });
   if (rc != 0) return none();
+  return wrap(std::move(out));
+  NATIVE_END
+}
+// (timestep embedder, timesteps [M], guidance embedder or None, guidance [M] or None, text projection, pooled text [M, K], dim, neg_log_period, scale, pre): the
+// sum of the embedders' results
+PyObject* py_embed_sum(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  NATIVE_BEGIN
+  const Tensor *t, *guidance, *pooled;
+  if (n != 10 || g_linear_type == nullptr || g_time_embedding_type == nullptr || g_text_projection_type == nullptr || !(t = tensor_of(a[1])) ||
+      !optional_tensor(a[3], &guidance) || (guidance == nullptr) != (a[2] == Py_None) || !(pooled = tensor_of(a[5])))
+    return none();
+  const long dim = PyLong_AsLong(a[6]);
+  const double period = PyFloat_AsDouble(a[7]), scale = PyFloat_AsDouble(a[8]), pre = PyFloat_AsDouble(a[9]);
+  if (PyErr_Occurred()) return nullptr;
+  BlockCall c;
+  c.dtype = code_of(*pooled);
+  c.st = pooled->scalar_type();
+  if ((c.dtype != ODIT_BF16 && c.dtype != ODIT_F16) || !c.where.holds(pooled) || pooled->dim() != 2 || pooled->stride(1) != 1 || pooled->size(0) < 1 ||
+      pooled->size(0) > 4 || pooled->size(1) < 1 || pooled->size(1) >= (1 << 20))
+    return none();
+  const int M = static_cast<int>(pooled->size(0));
+  const struct { PyObject* module; PyTypeObject* type; const Tensor* in; } of[3] = {
+      {a[0], g_time_embedding_type, t}, {a[2], g_time_embedding_type, guidance}, {a[4], g_text_projection_type, pooled}};
+  odit_embedder e[3];
+  int count = 0;
+  int64_t N = 0;
+  for (const auto& m : of) {
+    if (m.in == nullptr) continue;
+    PyObject* const d = plain_module(m.module, m.type);
+    const bool rows = m.in == pooled;
+    Lin l1, l2;
+    if (d == nullptr || !c.linear(child(d, "linear_1"), &l1, false) || !c.linear(child(d, "linear_2"), &l2, false) || l2.k != l1.n || l2.n != l1.n ||
+        l1.k != (rows ? pooled->size(1) : dim) || l1.n < 1 || l1.n >= (1 << 20) || (count > 0 && l1.n != N))
+      return none();
+    if (!rows && (!c.where.holds(m.in) || code_of(*m.in) < 0 || m.in->dim() != 1 || m.in->size(0) != M || !m.in->is_contiguous())) return none();
+    N = l1.n;
+    e[count++] = odit_embedder{m.in->data_ptr(), rows ? (M > 1 ? pooled->stride(0) : l1.k) : 0, static_cast<int>(l1.k), rows ? -1 : code_of(*m.in),
+                               static_cast<float>(period), static_cast<float>(scale), static_cast<float>(pre), l1.w, l1.b, l2.w, l2.b, l1.ldw, l2.ldw};
+  }
+  Tensor hidden = fresh({count, M, N}, pooled->options()), out = fresh({M, N}, pooled->options());
+  if (unlocked([&] { return odit_embed_sum(e, count, M, static_cast<int>(N), hidden.data_ptr(), out.data_ptr(), c.dtype, c.where.stream); }) != 0) return none();
   return wrap(std::move(out));
   NATIVE_END
 }
@@ -2164,7 +2205,8 @@ PyObject* py_classes(PyObject*, PyObject* const* a, Py_ssize_t n) {
       {"ApproxGELU", &g_gelu_type}, {"WanFeedForward", &g_wan_ffn_type}, {"QwenImageCrossAttention", &g_qwen_attention_type},
       {"FluxAttention", &g_flux_attention_type},
       {"AdaLayerNormZeroSingle", &g_flux_single_norm_type}, {"WanSelfAttention", &g_wan_self_type}, {"WanCrossAttention", &g_wan_cross_type},
-      {"TimestepEmbedding", &g_time_embedding_type}, {"RotaryEmbedding", &g_rotary_type}};
+      {"TimestepEmbedding", &g_time_embedding_type}, {"RotaryEmbedding", &g_rotary_type},
+      {"PixArtAlphaTextProjection", &g_text_projection_type}};
   for (const auto& w : want) {
     PyObject* t = PyDict_GetItemString(a[0], w.name);
     if (t == nullptr) continue;
@@ -2219,6 +2261,7 @@ PyMethodDef kMethods[] = {
     NATIVE_FN("linear_few", &py_linear_few),
     NATIVE_FN("linear_few_pair", &py_linear_few_pair),
     NATIVE_FN("time_embedding", &py_time_embedding),
+    NATIVE_FN("embed_sum", &py_embed_sum),
     NATIVE_FN("time_tokens", &py_time_tokens),
     NATIVE_FN("project_normed", &py_project_normed),
     NATIVE_FN("project_stem", &py_project_stem),

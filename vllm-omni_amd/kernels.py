@@ -799,6 +799,16 @@ def time_embedding(embedder: torch.nn.Module, t: torch.Tensor, dim: int, max_per
     return (_nat or _load_native()).time_embedding(embedder, t, dim, -math.log(max_period), float(scale), code, float(pre))
 
 
+def embed_sum(timestep_embedder: torch.nn.Module, t: torch.Tensor, guidance_embedder: torch.nn.Module | None, guidance: torch.Tensor | None,
+              text_embedder: torch.nn.Module, pooled: torch.Tensor, dim: int, max_period: float, scale: float, pre: float = 1.0) -> torch.Tensor | None:
+    """``time_embedding`` of ``t``, of ``guidance`` where given, and ``text_embedder`` of ``pooled``, added up in this order in the type of ``pooled``, in
+    two launches; None for what the kernels do not take."""
+    if not pooled.is_cuda or not native_blocks():
+        return None
+    return (_nat or _load_native()).embed_sum(timestep_embedder, t, guidance_embedder, guidance, text_embedder, pooled, dim, -math.log(max_period),
+                                              float(scale), float(pre))
+
+
 def time_tokens(embedder: torch.nn.Module, time_proj: torch.nn.Module, t: torch.Tensor, dim: int, max_period: float, scale: float, dtype: torch.dtype):
     """(``embedder`` of ``time_sinusoid``'s rows of a timestep per token, t [n], ``time_proj`` of its SiLU, int32 [n] whose entry i says
     which row of both is token i's): each distinct timestep's rows are formed once where there are at most four. None for what the kernels do
