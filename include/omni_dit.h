@@ -384,11 +384,16 @@ int odit_linear_tune(const void* x, const void* w, const void* bias, void* out, 
  * this thread chose a kernel for it, its own first choice (or the one odit_linear_prefer named), not the one expected to be
  * faster, and what ODIT_LINEAR_NO_TILE says; ODIT_LINEAR_NO_TILE = neither the tile nor the small kernel, unless a tuning call
  * found it faster (a caller whose results another order of summation may not move). Per call: no process-wide switch exists.
+ * ODIT_LINEAR_CLIP: of a gated or residual epilogue in ODIT_F16, results are clipped to +-65504, as the blocks' outputs are
+ * (qwen_image_transformer.py:812-815, flux_transformer.py:310-312, 362-364); a NaN stays one. Nothing in other types. Of two problems
+ * the first one's; ODIT_LINEAR_CLIP2 the second one's.
  */
 #define ODIT_LINEAR_LIBRARY 1u
 #define ODIT_LINEAR_HANDWRITTEN 2u
 #define ODIT_LINEAR_FIRST 4u
 #define ODIT_LINEAR_NO_TILE 8u
+#define ODIT_LINEAR_CLIP 16u
+#define ODIT_LINEAR_CLIP2 32u
 
 int odit_linear_rows(const void* x, const void* w, const void* bias, void* out, const void* residual,
                      const void* gate, int M, int N, int K, int64_t ldx, int64_t ldw, int64_t ldo, int64_t ldr,

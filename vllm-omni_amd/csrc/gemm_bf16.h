@@ -16,6 +16,7 @@ struct GemmCall {
   int gate_f32;       // gate (and, in the pre-scaled form, bias) are float32
   int rows_per_gate;  // consecutive rows that share one gate vector (0 = all rows)
   int64_t ldg;        // elements between consecutive gate vectors (and pre-scaled bias vectors)
+  int clip = 0;       // a gated result of f16 is held to the largest finite value (ODIT_LINEAR_CLIP)
 };
 
 constexpr int kGemmBM = 128;  // rows of x per output tile

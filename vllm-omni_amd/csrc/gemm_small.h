@@ -310,7 +310,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void gemm_small_kernel(const Smal
     for (int t = 0; t < 2; ++t) {
       const int f = 2 * u + t;
       const float a = acc[f / 4][f % 4];
-      y[t] = gated ? fmaf(gt[f], a, bs[f]) + Raw<T>::get(res, f) : a + bs[f];
+      y[t] = gated ? gemm_clipped<T>(e, fmaf(gt[f], a, bs[f]) + Raw<T>::get(res, f)) : a + bs[f];
       if (!gated && gelu) y[t] = gemm_gelu_tanh(y[t]);
     }
     Raw<T>::set2(o, u, y[0], y[1]);

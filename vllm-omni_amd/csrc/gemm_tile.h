@@ -147,8 +147,8 @@ __device__ __forceinline__ void finish_quadrant(const GemmEpilogue& e, int m0, i
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
           const f32x4_v a = v[i0 + j][u >> 1];
-          Raw<T>::set2(o, u, fmaf(gt[j][2 * u], a[2 * (u & 1)], bs[j][2 * u]) + Raw<T>::get(res[j], 2 * u),
-                       fmaf(gt[j][2 * u + 1], a[2 * (u & 1) + 1], bs[j][2 * u + 1]) + Raw<T>::get(res[j], 2 * u + 1));
+          Raw<T>::set2(o, u, gemm_clipped<T>(e, fmaf(gt[j][2 * u], a[2 * (u & 1)], bs[j][2 * u]) + Raw<T>::get(res[j], 2 * u)),
+                       gemm_clipped<T>(e, fmaf(gt[j][2 * u + 1], a[2 * (u & 1) + 1], bs[j][2 * u + 1]) + Raw<T>::get(res[j], 2 * u + 1)));
         }
         if (in && m + (i0 + j) * 16 < e.M) store_raw(static_cast<T*>(e.out) + (m + (i0 + j) * 16) * e.ldo + n, o);
       }
@@ -176,7 +176,7 @@ __device__ __forceinline__ void finish_quadrant(const GemmEpilogue& e, int m0, i
       }
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
-        if constexpr (K == 2) y[u] = fmaf(gt[u], y[u], bs[u]) + Raw<T>::get(res[i], u);
+        if constexpr (K == 2) y[u] = gemm_clipped<T>(e, fmaf(gt[u], y[u], bs[u]) + Raw<T>::get(res[i], u));
         else y[u] += bs[u];
         if constexpr (K == 1) y[u] = gemm_gelu_tanh(y[u]);
       }

@@ -187,6 +187,7 @@ struct LinCall {
   hipStream_t stream;
   bool first = false;    // the library's first-ranked kernel, unless one was tuned (ODIT_LINEAR_FIRST)
   bool no_tile = false;  // untuned, neither the tile nor the small kernel (ODIT_LINEAR_NO_TILE)
+  bool clip = false;     // results of f16 clipped (ODIT_LINEAR_CLIP)
 };
 
 static bool lin_is_residual(const LinCall& c) {
@@ -444,6 +445,7 @@ static odit::GemmCall lin_gemm_call(const odit::LinCall& c, int rows_per_gate, i
   g.gate_f32 = c.gate_dtype == ODIT_F32 ? 1 : 0;
   g.rows_per_gate = rows_per_gate;
   g.ldg = ldg;
+  g.clip = c.clip ? 1 : 0;
   return g;
 }
 
@@ -602,6 +604,32 @@ int odit::linear_tile_unless(const void* x, const void* w, const void* bias, voi
   return ask ? ODIT_OK : launch_gemm_tile_unless(g, unless, dtype, sk, stream);
 }
 
+// whether ODIT_LINEAR_CLIP (`bit`) asks anything of a call
+static bool lin_clips(const odit::LinCall& c, unsigned flags, unsigned bit) { return (flags & bit) != 0 && c.dtype == ODIT_F16 && odit::lin_is_residual(c); }
+
+// a clip of what the library has written: eight values to a thread where the rows' starts allow (`wide`)
+__global__ __launch_bounds__(256) void lin_clip_kernel(odit::f16_t* out, int M, int N, int64_t ldo, int wide) {
+  for (int row = blockIdx.x; row < M; row += gridDim.x) {
+    odit::f16_t* const at = out + row * ldo;
+    for (int col = 8 * static_cast<int>(threadIdx.x); col < N; col += 8 * 256) {
+      if (wide) {
+        odit::u32x4* const v = reinterpret_cast<odit::u32x4*>(at + col);
+        odit::u32x4 o = *v;
+#pragma unroll
+        for (int p = 0; p < 4; ++p) odit::Raw<odit::f16_t>::set2(o, p, odit::f16_clipped(odit::Raw<odit::f16_t>::get(o, 2 * p)), odit::f16_clipped(odit::Raw<odit::f16_t>::get(o, 2 * p + 1)));
+        *v = o;
+      } else {
+        for (int u = col; u < N && u < col + 8; ++u) at[u] = odit::from_float<odit::f16_t>(odit::f16_clipped(odit::to_float(at[u])));
+      }
+    }
+  }
+}
+static int lin_clip(const odit::LinCall& c) {
+  const int wide = c.N % 8 == 0 && c.ldo % 8 == 0 && odit::aligned16(c.out) ? 1 : 0;
+  hipLaunchKernelGGL(lin_clip_kernel, dim3(static_cast<unsigned>(c.M)), dim3(256), 0, c.stream, static_cast<odit::f16_t*>(c.out), c.M, c.N, c.ldo, wide);
+  return odit::check_launch("odit_linear (clip)");
+}
+
 extern "C" int odit_linear_prefer(int M, int N, int K, int dtype, int solution) {
   using namespace odit;
   ODIT_CHECK_ARG(M > 0 && N > 0 && K > 0 && solution >= 0, "odit_linear_prefer: bad problem or solution index");
@@ -623,9 +651,9 @@ extern "C" int odit_linear_rows(const void* x, const void* w, const void* bias, 
                                 int64_t gate_stride, unsigned flags, void* workspace, size_t workspace_bytes,
                                 void* stream) {
   using namespace odit;
-  ODIT_CHECK_ARG((flags & ~(ODIT_LINEAR_LIBRARY | ODIT_LINEAR_HANDWRITTEN | ODIT_LINEAR_FIRST | ODIT_LINEAR_NO_TILE)) == 0 &&
+  ODIT_CHECK_ARG((flags & ~(ODIT_LINEAR_LIBRARY | ODIT_LINEAR_HANDWRITTEN | ODIT_LINEAR_FIRST | ODIT_LINEAR_NO_TILE | ODIT_LINEAR_CLIP)) == 0 &&
                      (flags & (ODIT_LINEAR_LIBRARY | ODIT_LINEAR_HANDWRITTEN)) != (ODIT_LINEAR_LIBRARY | ODIT_LINEAR_HANDWRITTEN),
-                 "odit_linear_rows: flags may name one engine (ODIT_LINEAR_LIBRARY or ODIT_LINEAR_HANDWRITTEN), ODIT_LINEAR_FIRST and ODIT_LINEAR_NO_TILE, got %#x", flags);
+                 "odit_linear_rows: flags may name one engine (ODIT_LINEAR_LIBRARY or ODIT_LINEAR_HANDWRITTEN), ODIT_LINEAR_FIRST, ODIT_LINEAR_NO_TILE and ODIT_LINEAR_CLIP, got %#x", flags);
   void *sk, *lib;
   size_t lib_bytes;
   lin_split_ws(workspace, workspace_bytes, &sk, &lib, &lib_bytes);
@@ -635,6 +663,7 @@ extern "C" int odit_linear_rows(const void* x, const void* w, const void* bias, 
   c.no_tile = c.first || (flags & ODIT_LINEAR_NO_TILE) != 0;
   int rc = lin_check(c);
   if (rc != ODIT_OK || M == 0) return rc;
+  c.clip = lin_clips(c, flags, ODIT_LINEAR_CLIP);
   ODIT_CHECK_ARG(rows_per_gate >= 0 && (rows_per_gate == 0 || gate_stride >= 0),
                  "odit_linear_rows: rows_per_gate and gate_stride must not be negative");
   const bool per_rows = lin_is_residual(c) && gate != nullptr && rows_per_gate > 0 && rows_per_gate < M;
@@ -652,7 +681,10 @@ extern "C" int odit_linear_rows(const void* x, const void* w, const void* bias, 
     kind = lin_auto_kind(dev, c, g, sk);
   }
   if (kind != 0) return lin_launch_handwritten(kind, g, dtype, sk, c.stream);
-  if (!per_rows) return lin_run_library(c);
+  if (!per_rows) {
+    rc = lin_run_library(c);
+    return rc == ODIT_OK && c.clip ? lin_clip(c) : rc;
+  }
   // the library's epilogue takes one gate vector per launch: one launch per group of rows
   const size_t esz = dtype == ODIT_F32 ? 4 : 2, gsz = gate_dtype == ODIT_F32 ? 4 : esz;
   for (int r0 = 0; r0 < M; r0 += rows_per_gate) {
@@ -668,7 +700,7 @@ extern "C" int odit_linear_rows(const void* x, const void* w, const void* bias, 
     rc = lin_run_library(cg);
     if (rc != ODIT_OK) return rc;
   }
-  return ODIT_OK;
+  return c.clip ? lin_clip(c) : ODIT_OK;
 }
 
 // Two problems in one launch, or two calls? By expected time, or what was measured for a tuned problem if that is shorter (811
@@ -706,6 +738,7 @@ extern "C" int odit_linear_pair(const odit_linear_problem* q, int N, int K, int 
     if (rc != ODIT_OK) return rc;
     ODIT_CHECK_ARG(q[i].rows_per_gate >= 0 && q[i].gate_stride >= 0, "odit_linear_pair: rows_per_gate and gate_stride must not be negative");
     const bool rows = lin_is_residual(c) && q[i].gate != nullptr && q[i].rows_per_gate > 0 && q[i].rows_per_gate < q[i].M;
+    calls[i].clip = lin_clips(c, flags, i == 0 ? ODIT_LINEAR_CLIP : ODIT_LINEAR_CLIP2);
     g[i] = lin_gemm_call(c, rows ? q[i].rows_per_gate : 0, rows ? q[i].gate_stride : 0);
     per_rows = per_rows || rows;
     takes = takes && q[i].M > 0 && gemm_streamk_takes(g[i], dtype);
@@ -973,6 +1006,7 @@ extern "C" int odit_linear_join(const void* x, const void* x2, const void* w, co
   second.K = K2;
   second.ldx = ldx2;
   whole.K = K + K2;
+  whole.clip = lin_clips(c, flags, ODIT_LINEAR_CLIP);
   const GemmCall g1 = lin_gemm_call(first, rows ? rows_per_gate : 0, rows ? gate_stride : 0), g2 = lin_gemm_call(second, g1.rows_per_gate, g1.ldg);
   GemmCall g = lin_gemm_call(whole, g1.rows_per_gate, g1.ldg);
   if (lin_engine_of(flags) != 0 || (flags & (ODIT_LINEAR_FIRST | ODIT_LINEAR_NO_TILE)) != 0 || M < kTileMinAuto || K % 64 != 0 || K2 % 64 != 0 ||

@@ -1395,10 +1395,11 @@ struct Gate {
 
 // out = residual + gate * (x W^T + b), B batch entries of S rows. The hand-written GEMM takes one gate row per
 // entry in one launch; for short entries the library's one launch per entry is slower than one launch over all rows
-// followed by the gated-residual pass (`min_rows`), which needs the `tmp` rows.
-void project_gated(BlockCall& c, const void* x, const Lin& l, const void* residual, void* out, int64_t B, int64_t S, const Gate& g,
-                   int64_t min_rows, void* tmp, const Gate& plain) {
-  if (c.rc != 0) return;
+// followed by the gated-residual pass (`min_rows`), which needs the `tmp` rows. `clip` has the projection clip its rows of float16;
+// true where it does.
+bool project_gated(BlockCall& c, const void* x, const Lin& l, const void* residual, void* out, int64_t B, int64_t S, const Gate& g,
+                   int64_t min_rows, void* tmp, const Gate& plain, bool clip = false) {
+  if (c.rc != 0) return clip;
   const int M = static_cast<int>(B * S);
   const int epi = g.pre ? ODIT_EPI_GATED_RESIDUAL_PRE : ODIT_EPI_GATED_RESIDUAL;
   const int rows = g.gate && B > 1 ? static_cast<int>(S) : 0;
@@ -1408,17 +1409,18 @@ void project_gated(BlockCall& c, const void* x, const Lin& l, const void* residu
     int own = 0, launches = 0;
     c.check(odit_linear_rows_plan(x, l.w, bias, out, residual, g.gate, M, l.n, l.k, l.k, l.ldw, l.n, l.n, epi, gcode, c.dtype, rows,
                                   g.stride, c.engine, c.lin_ws.p, c.lin_ws.bytes, &own, &launches));
-    if (c.rc != 0) return;
+    if (c.rc != 0) return clip;
     if (!own) {
       c.project(x, l, tmp, M, false);
-      if (c.rc != 0) return;
+      if (c.rc != 0) return clip;
       const int64_t st[2] = {S * l.n, l.n}, gs[2] = {plain.stride, 0};
       c.check(odit_gated_residual(residual, tmp, plain.gate, nullptr, out, B, S, l.n, st, st, st, gs, plain.code, c.dtype, 0u, c.where.stream));
-      return;
+      return false;
     }
   }
   c.check(odit_linear_rows(x, l.w, bias, out, residual, g.gate, M, l.n, l.k, l.k, l.ldw, l.n, l.n, epi, gcode, c.dtype, rows, g.stride,
-                           c.engine, c.lin_ws.p, c.lin_ws.bytes, c.where.stream));
+                           c.engine | (clip ? ODIT_LINEAR_CLIP : 0u), c.lin_ws.p, c.lin_ws.bytes, c.where.stream));
+  return clip;
 }
 
 // y[i] = x[i] W[i]^T + b[i] (GELU) for the two streams: one launch where that is the better way
@@ -1435,17 +1437,18 @@ void project_pair(BlockCall& c, const void* const x[2], const Lin l[2], void* co
   for (int i = 0; i < 2; ++i) c.project(x[i], l[i], y[i], M[i], gelu);
 }
 
-// out[i] = residual[i] + gate[i] * (x[i] W[i]^T + b[i]) for the two streams in one launch; false when two calls are the better way
+// out[i] = residual[i] + gate[i] * (x[i] W[i]^T + b[i]) for the two streams in one launch, clipped where `clip`; false when two calls are the better way
 bool project_gated_pair(BlockCall& c, const void* const x[2], const Lin l[2], const void* const residual[2], void* const out[2], int64_t B,
-                        const int64_t S[2], const Gate g[2]) {
+                        const int64_t S[2], const Gate g[2], const bool clip[2]) {
   if (c.rc != 0) return true;
   if (l[0].n != l[1].n || l[0].k != l[1].k || g[0].pre != g[1].pre || g[0].code != g[1].code) return false;
   odit_linear_problem q[2];
   for (int i = 0; i < 2; ++i)
     q[i] = {x[i], l[i].w, g[i].pre ? g[i].gbias : l[i].b, residual[i], g[i].gate, out[i], static_cast<int>(B * S[i]), B > 1 ? static_cast<int>(S[i]) : 0,
             l[i].k, l[i].ldw, l[i].n, l[i].n, g[i].stride};
+  const unsigned flags = (c.engine & ~static_cast<unsigned>(ODIT_LINEAR_HANDWRITTEN)) | (clip[0] ? ODIT_LINEAR_CLIP : 0u) | (clip[1] ? ODIT_LINEAR_CLIP2 : 0u);
   const int rc = odit_linear_pair(q, l[0].n, l[0].k, g[0].pre ? ODIT_EPI_GATED_RESIDUAL_PRE : ODIT_EPI_GATED_RESIDUAL, g[0].pre ? ODIT_F32 : g[0].code,
-                                  c.dtype, c.engine & ~static_cast<unsigned>(ODIT_LINEAR_HANDWRITTEN), c.lin_ws.p, c.lin_ws.bytes, c.where.stream);
+                                  c.dtype, flags, c.lin_ws.p, c.lin_ws.bytes, c.where.stream);
   if (rc == ODIT_ENOTSUP) return false;
   c.check(rc);
   return true;
@@ -1583,7 +1586,7 @@ bool gate_rows(const BlockCall& c, const Tensor* t, int64_t B, int64_t C) {
 // c.rc carries a C error.
 bool run_dual(BlockCall& c, const DualBlock& k, const Tensor& img, const Tensor& txt, const ModRow mod[2], const Tensor* gates,
               const Tensor* gbias, const Tensor* const cos[2], const Tensor* const sin[2], const Tensor* mask, const Tensor* index,
-              int64_t min_rows, Tensor result[2]) {
+              int64_t min_rows, bool clip[2], Tensor result[2]) {
   const Tensor* x[2] = {&img, &txt};
   const int64_t B = img.size(0), C = img.size(2), H = k.H, D = k.D, HD = H * D;
   const int64_t S[2] = {img.size(1), txt.size(1)}, Sj = S[0] + S[1];
@@ -1737,23 +1740,25 @@ bool run_dual(BlockCall& c, const DualBlock& k, const Tensor& img, const Tensor&
   }
   void* res[2] = {result[0].data_ptr(), result[1].data_ptr()};
   Gate plain;
-  auto gated = [&](const void* const a[2], const Lin l[2], const void* const residual[2], int which) {
+  // (`to`: the streams to clip in float16; false behind it for one that is left to the caller)
+  auto gated = [&](const void* const a[2], const Lin l[2], const void* const residual[2], int which, bool to[2]) {
     const Gate g[2] = {gate_of(0, which, &plain), gate_of(1, which, &plain)};
-    if (!idx && project_gated_pair(c, a, l, residual, res, B, S, g)) return;
+    if (!idx && project_gated_pair(c, a, l, residual, res, B, S, g, to)) return;
     for (int i = 0; i < 2; ++i) {
-      if (i == 0 && idx) { indexed(a[0], l[0], residual[0], res[0], which); continue; }
+      if (i == 0 && idx) { indexed(a[0], l[0], residual[0], res[0], which); to[0] = false; continue; }
       gate_of(i, which, &plain);
-      project_gated(c, a[i], l[i], residual[i], res[i], B, S[i], g[i], min_rows, tmp, plain);
+      to[i] = project_gated(c, a[i], l[i], residual[i], res[i], B, S[i], g[i], min_rows, tmp, plain, to[i]);
     }
   };
-  gated(o, k.out, src, 0);
+  bool unclipped[2] = {false, false};
+  gated(o, k.out, src, 0, unclipped);
   const void* mid[2] = {res[0], res[1]};
   if (idx) norm(1, mid[1], 1);
   else if (c.rc == 0 && !normed_up) norms(mid, 1);
   row_norms(1, rn);
   if (normed_up) project_normed(c, mid, k.up, u, B, S, rn, nullptr, true, true);
   else project_pair(c, n, k.up, u, M, true);
-  gated(u, k.down, mid, 1);
+  gated(u, k.down, mid, 1, clip);
   return true;
 }
 
@@ -1842,12 +1847,15 @@ PyObject* dual_block(PyObject* const* a, Py_ssize_t n, bool flux) {
       return none();
   }
   Tensor out[2];
-  if (!run_dual(c, k, *img, *txt, mod, gates, gbias, cos, sin, mask, index, min_rows, out)) return none();
+  // the reference clips both streams after every Qwen block, the text's after every Flux block; the last projections do it on the way
+  const bool wanted[2] = {c.dtype == ODIT_F16 && !flux, c.dtype == ODIT_F16};
+  bool clipped[2] = {wanted[0], wanted[1]};
+  if (!run_dual(c, k, *img, *txt, mod, gates, gbias, cos, sin, mask, index, min_rows, clipped, out)) return none();
   if (c.rc != 0) return block_failed(c.rc);
-  if (c.dtype == ODIT_F16) {  // the reference clips after every block
+  for (int i = 0; i < 2; ++i) {
+    if (!wanted[i] || clipped[i]) continue;
     const Unlocked others_run;
-    out[1].clamp_(-65504, 65504);
-    if (!flux) out[0].clamp_(-65504, 65504);
+    out[i].clamp_(-65504, 65504);
   }
   return wrap2(std::move(out[1]), std::move(out[0]));
   NATIVE_END
@@ -1953,16 +1961,15 @@ PyObject* py_flux_single_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const int joined = c.rc != 0 ? c.rc : odit_linear_join(o, u, down.w, g.gbias, out.data_ptr(), x->data_ptr(), g.gate, static_cast<int>(B * S),
                                                          static_cast<int>(C), static_cast<int>(C), static_cast<int>(F), C, F, down.ldw, C, C,
                                                          ODIT_EPI_GATED_RESIDUAL_PRE, ODIT_F32, c.dtype, B > 1 ? static_cast<int>(S) : 0, g.stride,
-                                                         c.engine, c.lin_ws.p, c.lin_ws.bytes, c.where.stream);
+                                                         c.engine | ODIT_LINEAR_CLIP, c.lin_ws.p, c.lin_ws.bytes, c.where.stream);
   if (joined != ODIT_ENOTSUP) {
     c.check(joined);
   } else {
     project_gated(c, u, wm, x->data_ptr(), out.data_ptr(), B, S, g, 0, nullptr, Gate());
     written = in_place && c.rc == 0;
     g.gbias = nullptr;
-    project_gated(c, o, wa, out.data_ptr(), out.data_ptr(), B, S, g, 0, nullptr, Gate());
+    project_gated(c, o, wa, out.data_ptr(), out.data_ptr(), B, S, g, 0, nullptr, Gate(), true);  // (no gated-residual pass at min_rows 0)
   }
-  if (c.rc == 0 && c.dtype == ODIT_F16) out.clamp_(-65504, 65504);
   others_run.reset();
   if (c.rc != 0) return block_failed(c.rc, written);
   if (in_place) { Py_INCREF(a[3]); return a[3]; }
