@@ -483,7 +483,8 @@ typedef struct odit_row_norm {
 int odit_linear_pair_norm(const odit_linear_problem problems[2], const odit_row_norm norm[2], int N, int K, int epilogue,
                           const odit_head_output* const heads[2], int dtype, unsigned flags, int launch, void* stream);
 
-/* odit_linear_pair_norm of one problem: the head's norm and projection (qwen_image_transformer.py:1065-1066) of a small model. */
+/* odit_linear_pair_norm of one problem: a model's head, norm and projection (qwen_image_transformer.py:1065-1066, flux_transformer.py:583-584),
+ * small or of 1024, 2048 or 3072 channels and up to 64 features. */
 int odit_linear_norm(const odit_linear_problem* problem, const odit_row_norm* norm, int N, int K, int epilogue, int dtype, unsigned flags,
                      void* stream);
 

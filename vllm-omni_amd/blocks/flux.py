@@ -596,7 +596,7 @@ class FluxTransformer2DModel(nn.Module):
 
     def finish(self, img, temb, return_dict: bool = True, head=None):
         """``head``: the projection of the head's norm where the caller has it."""
-        out = kernels.project(self.proj_out, self.norm_out(img, temb) if head is None else self.norm_out.modulate(img, head))
+        out = AdaLayerNormContinuous.head(self.norm_out, self.proj_out, img, temb, head)
         return Transformer2DModelOutput(sample=out) if return_dict else (out,)
 
     def forward(self, hidden_states: torch.Tensor, encoder_hidden_states: torch.Tensor = None,

@@ -510,6 +510,20 @@ class AdaLayerNormContinuous(nn.Module):
         scale, shift = emb.chunk(2, dim=1)
         return kernels.adaln_modulate(x, shift, scale, eps=self.eps)
 
+    def head(self, lin: nn.Module, x: torch.Tensor, cond: torch.Tensor, emb: torch.Tensor | None = None) -> torch.Tensor:
+        """``lin(self(x, cond))``, in one launch where that is the faster way; ``emb``: the projection of the condition where the caller has it (of a
+        module that is plainly of this class)."""
+        if emb is None:
+            if cond.dtype != x.dtype or not kernels.plain_module(self, AdaLayerNormContinuous):
+                return kernels.project(lin, self(x, cond))
+            emb = kernels.project(self.linear, cond, silu_input=True)
+        if "modulate" not in self.__dict__:
+            scale, shift = emb.chunk(2, dim=1)
+            out = kernels.project_normed(lin, x, shift, scale, self.eps)
+            if out is not None:
+                return out
+        return kernels.project(lin, self.modulate(x, emb))
+
 
 def _build_conditioning_index(samples: tuple, device: str) -> torch.Tensor:
     rows = [[0] * math.prod(s[0]) + [1] * sum(math.prod(x) for x in s[1:]) for s in samples]
@@ -712,12 +726,7 @@ class QwenImageTransformer2DModel(nn.Module):
         """``head``: the projection of the head's norm where the caller has it."""
         if self.zero_cond_t:
             temb = temb.chunk(2, dim=0)[0]  # the head is conditioned on the real timestep (qit.py:1062-1063)
-        out = None
-        if head is not None and self.inner_dim <= 256:  # (a small model: one launch)
-            scale, shift = head.chunk(2, dim=1)
-            out = kernels.project_normed(self.proj_out, img, shift, scale, self.norm_out.eps)
-        if out is None:
-            out = kernels.project(self.proj_out, self.norm_out(img, temb) if head is None else self.norm_out.modulate(img, head))
+        out = AdaLayerNormContinuous.head(self.norm_out, self.proj_out, img, temb, head)
         return Transformer2DModelOutput(sample=out) if return_dict else (out,)
 
     def forward(self, hidden_states: torch.Tensor, encoder_hidden_states: torch.Tensor = None,

@@ -44,6 +44,7 @@ UNITS: list[tuple[str, list[str], str]] = [
     ("attn_fwd_dma.hip", [], "attn_fwd_dma"),
     ("linear.hip", [], "linear"),
     ("linear_few.hip", [], "linear_few"),
+    ("linear_head.hip", [], "linear_head"),
     ("step.hip", [], "step"),
     ("time_tokens.hip", [], "time_tokens"),
     ("gemm_bf16.hip", [], "gemm_bf16"),

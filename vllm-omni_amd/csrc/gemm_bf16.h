@@ -73,6 +73,9 @@ int launch_gemm_tile(const GemmCall* c, int count, const TileX2* x2, int dtype, 
 // gemm_tile_unless.hip: one problem, and nothing where *unless (device memory) is not 0 when the launch begins
 int launch_gemm_tile_unless(const GemmCall& c, const int* unless, int dtype, void* scratch, hipStream_t stream);
 
+// whether 32 bits hold the byte offsets of so many rows
+inline bool gemm_rows_fit(int rows, int64_t ld, int K) { return (static_cast<uint64_t>(rows) * ld + K) * 2 < (1ull << 32); }
+
 // ---- gemm_tile_heads.hip: the tile kernel with query, key and value heads at its end -------
 // Output of a projection to 3 HD features: per batch entry S rows of queries, keys and values of HD / D heads, the first two normed
 // over each head (mean of squares + eps), weighted and rotated in pairs (2 i, 2 i + 1), into rows offset .. of joint tensors [B, S_total, HD].
@@ -108,5 +111,11 @@ int launch_gemm_small_norm(const GemmCall* c, int count, const RowNorm* norm, co
 int launch_gemm_small_stem(const GemmCall* c, const void* weight, float eps, int dtype, hipStream_t stream);
 // the same with query, key and value heads of 64 features (gemm_small_heads.hip)
 int launch_gemm_small_heads(const GemmCall* c, int count, const HeadsOut* heads, int dtype, hipStream_t stream);
+
+
+// ---- linear_head.hip: a norm of the rows and a projection to few features -------
+// features to a tile, 0 where the kernel cannot take the problem or is not the faster way; one problem of K 1024, 2048 or 3072 and N up to 64
+int linear_head_features(const GemmCall& c, const RowNorm& n, int dtype, int cus);
+int launch_linear_head(const GemmCall& c, const RowNorm& n, int features, int dtype, hipStream_t stream);
 
 }  // namespace odit

@@ -316,8 +316,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
   // ---- tile loads ----
   // Instruction j of this wavefront's share of a unit fills rows (wave * J + j) * 8 .. + 7; lane l lands in row + l / 8, chunk
-  // l % 8, and fetches chunk (l % 8) ^ swizzle(row). Rows past the end re-read the last row: their products land in output
-  // rows and features that are never stored.
+  // l % 8, and fetches chunk (l % 8) ^ swizzle(row). The products of rows past the end (fill_tile_params) land in output rows
+  // and features that are never stored.
   // (the lane's number is hidden from the compiler wherever a segment begins or ends: it would form what follows from it once in
   // front of everything and keep it in registers that the main loop needs)
   auto hidden_lane = [&]() __attribute__((always_inline)) {
@@ -746,15 +746,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
 int row_tiles(int M, int bm) { return (M + bm - 1) / bm; }
 
-// What a launch of `plan` takes beside its heads
+// What a launch of `plan` takes beside its heads.
 // Rows of padding are fetched from where they would lie: past the end of the operand, for which its descriptor answers zeros. A tile of 256 rows
 // is bound by power, and a product of zeros takes little; copies of the last row stood in their place. Alone (us, copies / zeros): 8192 + 300
 // rows, N=9216, K=3072, 355.0 / 350.7; 2706 rows, 5120 x 5120, 109.2 / 108.2; 512 + 80 rows, N=9216, tiles of 128 rows, 57.8 / 58.5. In whole
 // models those of 128 rows gain a little too (two prompts of 171 and 23 at 1024 rows, eight blocks, 4693 / 4682, else the same), those of 256
 // more: 950 + 12 rows, five blocks, 2768 / 2732; 6156 + 44, six, 19714 / 19305; 169 + 121 and 269, five, 1811 / 1731.
 // Offsets have 32 bits: an operand whose padding would wrap around keeps the copies.
-inline bool rows_fit(int rows, uint32_t ld, int K) { return static_cast<uint64_t>(rows) * ld + static_cast<uint64_t>(K) * 2 < (1ull << 32); }
-
 inline void fill_tile_params(TileParams& p, const TilePlan& plan, const GemmCall* c, int count, const TileX2* x2, void* scratch) {
   for (int i = 0; i < 3; ++i) {
     const GemmCall& g = c[i < count ? i : 0];
@@ -771,8 +769,8 @@ inline void fill_tile_params(TileParams& p, const TilePlan& plan, const GemmCall
     q.m_tiles = (g.M + plan.bm - 1) / plan.bm;
     q.n_tiles = (g.N + kTileN - 1) / kTileN;
     const int m_end = q.m_tiles * plan.bm, n_end = q.n_tiles * kTileN;
-    q.x_last = rows_fit(m_end, std::max(q.ldx, q.ldx2), g.K) ? m_end : g.M - 1;
-    q.w_last = rows_fit(n_end, q.ldw, g.K) ? n_end : g.N - 1;
+    q.x_last = gemm_rows_fit(m_end, x2 ? std::max(g.ldx, x2->ldx) : g.ldx, g.K) ? m_end : g.M - 1;
+    q.w_last = gemm_rows_fit(n_end, g.ldw, g.K) ? n_end : g.N - 1;
     q.ep = gemm_epilogue_of(g);
   }
   p.tiles0 = plan.tiles0; p.tiles1 = plan.tiles1; p.tiles = plan.tiles; p.whole = plan.whole; p.parts = plan.parts;

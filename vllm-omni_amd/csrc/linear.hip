@@ -943,6 +943,11 @@ static int lin_normed(const char* name, const odit_linear_problem* q, const odit
     ODIT_CHECK_ARG(n.shift != nullptr && n.scale != nullptr && n.S > 0 && n.stride >= 0, "%s: bad modulation rows", name);
     g[i] = lin_gemm_call(c, 0, 0);
     r[i] = RowNorm{n.shift, n.scale, n.stride, n.S, n.eps};
+    if (count == 1 && heads == nullptr && K > kSmallNormK) {
+      const int features = linear_head_features(g[0], r[0], dtype, device_cus());
+      if (features == 0) return ODIT_ENOTSUP;
+      return launch == ODIT_LAUNCH_ASK ? ODIT_OK : launch_linear_head(g[0], r[0], features, dtype, static_cast<hipStream_t>(stream));
+    }
     if (!aligned16(n.shift) || !aligned16(n.scale) || n.stride % 8 != 0 || K > kSmallNormK || !gemm_streamk_takes(g[i], dtype) ||
         (heads != nullptr && (h[i].D != 64 || !gemm_tile_takes(g[i], dtype) || !gemm_tile_heads_takes(g[i], h[i]))))
       return ODIT_ENOTSUP;

@@ -1176,7 +1176,7 @@ PyObject* py_project(PyObject*, PyObject* const* a, Py_ssize_t n) {
 }
 
 // (plain Linear, x [B, S, C], shift, scale [B, C] with rows equally far apart, eps, engine flags): the module's projection of the rows of x normed and
-// modulated, in one launch; None where the kernel for small products is not the one
+// modulated, in one launch; None where two are the way
 PyObject* py_project_normed(PyObject*, PyObject* const* a, Py_ssize_t n) {
   NATIVE_BEGIN
   const Tensor *x, *sh, *sc;

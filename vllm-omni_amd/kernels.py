@@ -766,8 +766,8 @@ def project(lin: torch.nn.Module, x: torch.Tensor, silu_input: bool = False) -> 
 
 
 def project_normed(lin: torch.nn.Module, x: torch.Tensor, shift: torch.Tensor, scale: torch.Tensor, eps: float) -> torch.Tensor | None:
-    """``lin`` of ``adaln_modulate(x, shift, scale)`` in one launch, where the kernel for small products takes it; None elsewhere."""
-    if not x.is_cuda or x.shape[-1] > 256 or not native_blocks():
+    """``lin`` of ``adaln_modulate(x, shift, scale)`` in one launch, where the kernel for heads or small products takes it; None elsewhere."""
+    if not x.is_cuda or not native_blocks():
         return None
     return (_nat or _load_native()).project_normed(lin, x, shift, scale, float(eps), _LINEAR_ENGINE_FLAGS)
 
