@@ -22,9 +22,9 @@
 //
 // The workgroup is persistent and the stream of steps does not stop at a tile's end: the next tile's first units are on their
 // way while this tile's epilogue runs. Tiles are dealt out round by round. The tiles of a last round that would leave half or
-// more of the compute units without work are cut along the reduction instead, into 2 to 4 equal parts, behind the whole tiles.
-// The parts of a tile share its four quadrants out between them: each leaves its fp32 sums for the others' quadrants in scratch
-// (write-through), keeps its own ones' in LDS and takes a ticket; when all have arrived it adds up all sums of its quadrants,
+// more of the compute units without work are cut along the reduction instead, into 2 to 4 equal parts (of tiles of 128 rows up to 8), behind the whole tiles.
+// The parts of a tile share its four quadrants out between them (from the fifth on they have none): each leaves its fp32 sums for the others' quadrants
+// in scratch (write-through), keeps its own ones' in LDS and takes a ticket; when all have arrived it adds up all sums of its quadrants,
 // in the order of the parts (the result does not depend on who arrives when), and runs their epilogue. A part that does not find
 // the others arrived after a bounded number of looks leaves its own sums in scratch too and goes, and the last to arrive takes
 // what is left: nobody waits for anybody without a bound. Ticket words carry the launch's epoch (see gemm_bf16.hip). What the
@@ -108,7 +108,11 @@ constexpr int kThrough = 16;  // sc1 of a buffer access: past the XCD's L2, as a
 // Ticket word of a cut tile: arrivals in bits 0 to 3, quadrants given up 4 to 7, departures 8 to 11, the launch's epoch from 16 on
 constexpr unsigned long long kArrival = 1, kDeparture = 1 << 8;
 constexpr int kLooks = 64;    // looks for the other parts of a tile, about a microsecond each
-constexpr int kMaxParts = 4;
+// Parts of a tile of 128 rows and of 256 at most. Beyond four (the sums of 8 parts of a quadrant fit the registers of the lower tiles only), cold weights,
+// us, stream-K / 4 parts / this many: N=3072, K=12288: M=256 47.1 / 54.8 / 8: 41.3, 300 47.3 / 49.3 / 7: 43.2, 512 55.6 / 56.6 / 5: 52.7, 195 + 256
+// 62.2 / 63.1 / 5: 58.7, 128 + 40 51.5 / 59.4 / 8: 46.5; K=15360: 300 56.4 / 60.0 / 7: 48.8, 451 69.3 / 62.8 / 5: 58.9; N=5120, K=13824: 256
+// 67.0 / 63.5 / 6: 53.9. Short reductions gain nothing: N=3072, K=3072: 256 + 64 22.8 / 24.8 / 5: 24.4.
+constexpr int kMaxParts[2] = {8, 4};
 
 // What the epilogue of a problem is to a tile with rows m0 .. m0 + BM - 1: 0 bias, 1 bias and GELU, 2 gate and residual, 3 the
 // same where gate vectors change inside the tile
@@ -293,7 +297,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // quadrants that this part of a cut tile finishes: its number's, and the one `parts` further
   auto quadrants = [&]() __attribute__((always_inline)) -> int {
     const int part = quotient(v, cut);
-    return scalar(1 << part | (part + p.parts < 4 ? 1 << (part + p.parts) : 0));
+    return scalar((part < 4 ? 1 << part : 0) | (part + p.parts < 4 ? 1 << (part + p.parts) : 0));
   };
   constexpr int kQuad = 2 * MH * 8192;  // bytes of a quadrant's accumulators
   struct Cursor { bool part; int next; };
@@ -648,7 +652,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const auto slots = __builtin_amdgcn_make_buffer_rsrc(p.slots, 0, G * kTileSlot, 0x00020000);
     if (tid == 0) {
       int got = 0;
-      for (int look = 0; look < kLooks && got == 0; ++look) {
+      for (int look = 0; look < kLooks && got == 0 && mine != 0; ++look) {
         const unsigned w = static_cast<unsigned>(__hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
         if ((w & 15u) == all) got = mine;
         else __builtin_amdgcn_s_sleep(8);
@@ -714,7 +718,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       };
       if (parts == 2) add_up(std::integral_constant<int, 2>{});
       else if (parts == 3) add_up(std::integral_constant<int, 3>{});
-      else add_up(std::integral_constant<int, 4>{});
+      else if (MH > 2 || parts == 4) add_up(std::integral_constant<int, 4>{});
+      else if constexpr (MH <= 2) {
+        if (parts == 5) add_up(std::integral_constant<int, 5>{});
+        else if (parts == 6) add_up(std::integral_constant<int, 6>{});
+        else if (parts == 7) add_up(std::integral_constant<int, 7>{});
+        else add_up(std::integral_constant<int, 8>{});
+      }
       const int r = (quad >> 1) * HM + wm * (16 * MH) + (ln & 15), n = n0 + (quad & 1) * 128 + wn * 32 + (ln >> 4) * 8;
       if (has_heads(which)) {  // (the same in all wavefronts)
         if constexpr (HEADS) {
