@@ -26,7 +26,8 @@ bool gemm_tile_takes(const GemmCall& c, int dtype) {
 // launches of 256 to 9500 rows of the projections of widths 3072 and 5120, those within a quarter of a problem's best (6.3 %;
 // choosing by it takes 0.2 % longer than the best of all plans). A step takes 1.22 us on 256-row tiles in a launch's first
 // round, 1.32 in later ones (the clock falls), 1.13 where a round is cut, 0.78 on 128-row tiles; a launch 3.1, a tile's end 5.7,
-// 3 (2) more with GELU; a cut 0.088 for each part (0.057 with 128 rows), 5.7 more behind whole tiles, and 0.2 for every part of a tile beyond four. M=459, N=5120, K=13824: 256
+// 3 (2) more with GELU; a cut 0.088 for each part (0.057 with 128 rows), 5.7 more behind whole tiles, and 0.2 for every part of a tile beyond four, of
+// which there are none behind whole tiles (M=640, N=15360, K=5120: 128 rows in 5 parts 111, 256 rows whole 98; N=13824 8 parts 104, whole 95). M=459, N=5120, K=13824: 256
 // rows in 4 parts 80 us, 3 parts 98, 2 parts 131, whole 238, 128 rows in 3 parts 77, 2 parts 100; M=504, N=9216, K=3072: 256
 // rows in 3 parts 41, whole 64, 128 rows 48; M=2998, N=12288, K=3072 with GELU: 256 rows in 4 parts 184, whole 215.
 TilePlan plan_gemm_tile(const GemmCall* c, int count, int cus, bool scratch) {
@@ -45,7 +46,7 @@ TilePlan plan_gemm_tile(const GemmCall* c, int count, int cus, bool scratch) {
       if (c[i].epilogue == ODIT_EPI_GELU_TANH || c[i].epilogue == ODIT_EPI_BIAS_GELU_TANH) end = tall ? 8.7f : 7.7f;
     auto whole_rounds = [&](int n) { return n == 0 ? 0.f : n * (nk * (tall ? 1.32f : .78f) + end) - nk * (tall ? .1f : 0.f); };
     for (int parts = 1; parts <= kMaxParts[tall]; ++parts) {
-      if (parts > 1 && (!scratch || rest == 0 || rest * parts > most || parts > nk)) break;
+      if (parts > 1 && (!scratch || rest == 0 || rest * parts > most || parts > nk || (rounds > 0 && parts > 4))) break;
       p.parts = parts;
       p.whole = parts > 1 ? p.tiles - rest : p.tiles;
       p.grid = rounds > 0 ? most : rest * parts;
