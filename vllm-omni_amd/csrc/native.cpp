@@ -24,6 +24,7 @@
 #include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 
 #include <algorithm>
 #include <cstring>
@@ -942,7 +943,7 @@ PyObject* py_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
 struct Names {
   PyObject *modules, *parameters, *fwd_hooks, *pre_hooks, *forward, *weight, *bias, *eps, *elementwise_affine, *ref_rounding, *attention,
       *softmax_scale, *fused, *forward_hip, *kernel_takes_layer, *forward_method, *hidden_size, *variance_epsilon, *is_neox_style,
-      *module;
+      *module, *bwd_hooks, *bwd_pre_hooks, *call, *call_impl, *wrapped_call_impl, *compiled_call_impl, *global_hooks[4];
 };
 Names g_name;
 PyTypeObject *g_linear_type, *g_rmsnorm_type, *g_rownorm_type, *g_adaln_type, *g_attention_type, *g_attention_impl_type,
@@ -1060,6 +1061,36 @@ PyObject* py_rotary_of(PyObject*, PyObject* const* a, Py_ssize_t n) {
   }
   return rotary(x, cs, sn, flags);
   NATIVE_END
+}
+
+// Whether a call of `m`, as torch makes it, would do nothing but call its class's own `forward`: no hook of any kind on it or on all modules, nothing compiled, no trace
+// being taken, and neither torch's way of calling modules (which torch.fx exchanges while it traces) nor the layer's forward replaced.
+PyObject *g_module_type, *g_module_globals, *g_module_call[3], *g_rmsnorm_forward, *g_adaln_forward, *g_rotary_forward;
+bool no_hooks(PyObject* dict, PyObject* name) {
+  PyObject* h = item(dict, name);
+  return h != nullptr && PyDict_Check(h) && PyDict_GET_SIZE(h) == 0;
+}
+bool calls_only(PyObject* m, PyObject* forward) {
+  if (forward == nullptr || g_module_type == nullptr || g_module_globals == nullptr || item(Py_TYPE(m)->tp_dict, g_name.forward) != forward) return false;
+  PyObject *d = instance_dict(m), *torch_way = reinterpret_cast<PyTypeObject*>(g_module_type)->tp_dict;
+  for (PyObject* name : {g_name.fwd_hooks, g_name.pre_hooks, g_name.bwd_hooks, g_name.bwd_pre_hooks})
+    if (!no_hooks(d, name)) return false;
+  for (PyObject* name : g_name.global_hooks)
+    if (!no_hooks(g_module_globals, name)) return false;
+  PyObject* const ways[3] = {g_name.call, g_name.call_impl, g_name.wrapped_call_impl};
+  for (int i = 0; i < 3; ++i)
+    if (item(torch_way, ways[i]) != g_module_call[i] || (i > 0 && item(d, ways[i]) != nullptr)) return false;
+  PyObject* compiled = item(d, g_name.compiled_call_impl);
+  return item(d, g_name.forward) == nullptr && (compiled == nullptr || compiled == Py_None) && !torch::jit::tracer::isTracing();
+}
+// (layer, its arguments): the whole call of an RMSNorm, an AdaLayerNorm or a RotaryEmbedding; None where torch has to make it
+PyObject* py_layer_call(PyObject* self, PyObject* const* a, Py_ssize_t n) {
+  if (n < 2) return none();
+  PyTypeObject* const type = Py_TYPE(a[0]);
+  if (type == g_rmsnorm_type) return calls_only(a[0], g_rmsnorm_forward) ? py_rmsnorm_of(self, a, n) : none();
+  if (type == g_adaln_type) return calls_only(a[0], g_adaln_forward) ? py_adaln_of(self, a, n) : none();
+  if (type == g_rotary_type) return calls_only(a[0], g_rotary_forward) ? py_rotary_of(self, a, n) : none();
+  return none();
 }
 
 struct Lin {
@@ -2222,7 +2253,10 @@ PyObject* py_classes(PyObject*, PyObject* const* a, Py_ssize_t n) {
     Py_XSETREF(*w.slot, reinterpret_cast<PyTypeObject*>(t));
   }
   const struct { const char* name; PyObject** slot; } methods[] = {
-      {"RMSNorm.forward_hip", &g_rmsnorm_hip}, {"AdaLayerNorm.forward_hip", &g_adaln_hip}, {"RotaryEmbedding.forward_hip", &g_rotary_hip}};
+      {"RMSNorm.forward_hip", &g_rmsnorm_hip}, {"AdaLayerNorm.forward_hip", &g_adaln_hip}, {"RotaryEmbedding.forward_hip", &g_rotary_hip},
+      {"RMSNorm.forward", &g_rmsnorm_forward}, {"AdaLayerNorm.forward", &g_adaln_forward}, {"RotaryEmbedding.forward", &g_rotary_forward},
+      {"Module", &g_module_type}, {"Module.globals", &g_module_globals}, {"Module.__call__", &g_module_call[0]},
+      {"Module._call_impl", &g_module_call[1]}, {"Module._wrapped_call_impl", &g_module_call[2]}};
   for (const auto& w : methods) {
     PyObject* f = PyDict_GetItemString(a[0], w.name);
     if (f == nullptr) continue;
@@ -2240,7 +2274,10 @@ bool intern_names() {
       {"attention", &g_name.attention}, {"softmax_scale", &g_name.softmax_scale}, {"fused", &g_name.fused},
       {"forward_hip", &g_name.forward_hip}, {"kernel_takes_layer", &g_name.kernel_takes_layer}, {"_forward_method", &g_name.forward_method},
       {"hidden_size", &g_name.hidden_size}, {"variance_epsilon", &g_name.variance_epsilon}, {"is_neox_style", &g_name.is_neox_style},
-      {"__module__", &g_name.module}};
+      {"__module__", &g_name.module}, {"_backward_hooks", &g_name.bwd_hooks}, {"_backward_pre_hooks", &g_name.bwd_pre_hooks}, {"__call__", &g_name.call},
+      {"_call_impl", &g_name.call_impl}, {"_wrapped_call_impl", &g_name.wrapped_call_impl}, {"_compiled_call_impl", &g_name.compiled_call_impl},
+      {"_global_forward_hooks", &g_name.global_hooks[0]}, {"_global_forward_pre_hooks", &g_name.global_hooks[1]},
+      {"_global_backward_hooks", &g_name.global_hooks[2]}, {"_global_backward_pre_hooks", &g_name.global_hooks[3]}};
   for (const auto& w : want)
     if ((*w.slot = PyUnicode_InternFromString(w.s)) == nullptr) return false;
   return true;
@@ -2260,6 +2297,7 @@ PyMethodDef kMethods[] = {
     NATIVE_FN("rmsnorm_of", &py_rmsnorm_of),
     NATIVE_FN("adaln_of", &py_adaln_of),
     NATIVE_FN("rotary_of", &py_rotary_of),
+    NATIVE_FN("layer_call", &py_layer_call),
     NATIVE_FN("own_tree", &py_own_tree),
     NATIVE_FN("rotary", &py_rotary),
     NATIVE_FN("attn", &py_attn),

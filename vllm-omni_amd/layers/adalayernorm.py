@@ -67,7 +67,7 @@ class AdaLayerNorm(CustomOp):
         return (out.squeeze(0) if squeeze else out), gate_result
 
 
-kernels.native_classes(AdaLayerNorm=AdaLayerNorm, **{"AdaLayerNorm.forward_hip": AdaLayerNorm.forward_hip})
+kernels.native_classes(AdaLayerNorm=AdaLayerNorm, **{"AdaLayerNorm.forward": AdaLayerNorm.forward, "AdaLayerNorm.forward_hip": AdaLayerNorm.forward_hip})
 
 
 def adaln_pair(norm_a: AdaLayerNorm, x_a: torch.Tensor, mod_a: torch.Tensor,

@@ -11,6 +11,9 @@ from collections.abc import Callable
 from typing import Any
 
 import torch.nn as nn
+from torch.nn.modules import module as _module
+
+from .. import kernels
 
 
 class CustomOp(nn.Module):
@@ -21,6 +24,16 @@ class CustomOp(nn.Module):
     def dispatch_forward(self) -> Callable:
         return self.forward_hip
 
+    def __call__(self, *args, **kwargs) -> Any:
+        """A module's call; at once the native one where torch's would come to nothing else (two Python functions less: five calls on 77 rows, which wait for the
+        host, 26.0 -> 23.7 us)."""
+        nat = kernels._nat
+        if nat is not None and not kwargs:
+            out = nat.layer_call(self, *args)  # (None where anything is hooked, replaced, compiled or traced, and for other arguments and classes)
+            if out is not None:
+                return out
+        return super().__call__(*args, **kwargs)
+
     def forward(self, *args, **kwargs) -> Any:
         return self._forward_method(*args, **kwargs)
 
@@ -29,3 +42,7 @@ class CustomOp(nn.Module):
 
     def forward_native(self, *args, **kwargs):
         raise NotImplementedError(f"{type(self).__name__} has no torch-native path in this package")
+
+
+kernels.native_classes(**{"Module": nn.Module, "Module.globals": vars(_module)},
+                       **{f"Module.{name}": vars(nn.Module)[name] for name in ("__call__", "_call_impl", "_wrapped_call_impl")})

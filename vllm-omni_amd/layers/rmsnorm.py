@@ -54,4 +54,4 @@ class RMSNorm(CustomOp):
         return out.reshape(x.shape)
 
 
-kernels.native_classes(RMSNorm=RMSNorm, **{"RMSNorm.forward_hip": RMSNorm.forward_hip})
+kernels.native_classes(RMSNorm=RMSNorm, **{"RMSNorm.forward": RMSNorm.forward, "RMSNorm.forward_hip": RMSNorm.forward_hip})

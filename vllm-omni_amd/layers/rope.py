@@ -43,4 +43,4 @@ class RotaryEmbedding(CustomOp):
         return out
 
 
-kernels.native_classes(RotaryEmbedding=RotaryEmbedding, **{"RotaryEmbedding.forward_hip": RotaryEmbedding.forward_hip})
+kernels.native_classes(RotaryEmbedding=RotaryEmbedding, **{"RotaryEmbedding.forward": RotaryEmbedding.forward, "RotaryEmbedding.forward_hip": RotaryEmbedding.forward_hip})
