@@ -9,7 +9,7 @@ from vllm_omni_amd import _lib
 pytestmark = pytest.mark.gpu
 
 C = _lib.C
-LIBRARY, HANDWRITTEN, CLIP, CLIP2 = 1, 2, 16, 32
+LIBRARY, HANDWRITTEN, CLIP, CLIP2 = _lib.ODIT_LINEAR_LIBRARY, _lib.ODIT_LINEAR_HANDWRITTEN, _lib.ODIT_LINEAR_CLIP, _lib.ODIT_LINEAR_CLIP2
 PRE = _lib.ODIT_EPI_GATED_RESIDUAL_PRE
 
 

@@ -20,7 +20,7 @@ ODIT_FLAG_NEOX = 2
 ODIT_NORM_NONE, ODIT_NORM_HEAD, ODIT_NORM_ROW = 0, 1, 2
 ODIT_EPI_NONE, ODIT_EPI_BIAS, ODIT_EPI_GELU_TANH, ODIT_EPI_BIAS_GELU_TANH, ODIT_EPI_GATED_RESIDUAL = 0, 1, 2, 3, 4
 ODIT_EPI_GATED_RESIDUAL_PRE = 5
-ODIT_LINEAR_LIBRARY, ODIT_LINEAR_HANDWRITTEN, ODIT_LINEAR_NO_TILE = 1, 2, 8
+ODIT_LINEAR_LIBRARY, ODIT_LINEAR_HANDWRITTEN, ODIT_LINEAR_NO_TILE, ODIT_LINEAR_CLIP, ODIT_LINEAR_CLIP2 = 1, 2, 8, 16, 32
 ODIT_LAUNCH_ASK, ODIT_LAUNCH_CHOOSE, ODIT_LAUNCH_ANSWERED = 0, 1, 2
 
 # every symbol include/omni_dit.h declares: (name, restype, argtypes)

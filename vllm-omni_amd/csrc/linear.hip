@@ -919,7 +919,7 @@ extern "C" int odit_linear_heads(const odit_linear_problem* q, const int* N, int
 // LayerNorm and modulation in front of a pair that the small kernel takes, up to 4 steps of the reduction. us, the norm's launch and the pair's /
 // one launch, one after the other without the host: M=256+64, K=256, heads of N=768 6.48 / 5.67, N=1024 with GELU 6.45 / 5.61; M=64+64, K=128,
 // N=512 5.76 / 4.35; with 8 steps, M=512+64, K=512, heads of N=1536 8.40 / 9.02 (every workgroup norms its rows again). The host, which such a
-// model mostly waits for, is asked for a launch less: 3.6 us.
+// model mostly waits for, is asked for a launch less: 3.6 us. One problem of a longer reduction and few features, a large model's head: linear_head.hip.
 static int lin_normed(const char* name, const odit_linear_problem* q, const odit_row_norm* norm, int count, int N, int K, int epilogue,
                       const odit_head_output* const* heads, int dtype, unsigned flags, int launch, void* stream) {
   using namespace odit;
