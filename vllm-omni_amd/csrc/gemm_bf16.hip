@@ -530,9 +530,16 @@ static StreamkPlan plan_streamk(int M0, int M1, int N, int K, int cus) {
   return best;
 }
 
+// Two problems whose tiles several workgroups share: each further one costs 3 us more with 192-wide tiles and 5.3 with 256-wide ones than the plan's time has it, as
+// twice the weights arrive from memory meanwhile. us, as planned / so / measured / the tile kernel (N=9216, K=3072): 128 + 40 rows 27.5 / 38 / 38.4 / 35.7, 256 + 64
+// 31.8 / 37 / 45 / 39.8; N=3072, K=3072: 195 + 256 22.9 / 32 / 29.6 / 25.2, 300 + 300 27.5 / 38 / 30.9 / 27.9, 768 + 128 27.5 / 38 / 35.4 / 30.5. Over 79 pairs of 2 to 8
+// row tiles the choice between the two kernels takes 0.45 % longer than the better one each time, by the plan's times 1.5 %; whole models, us:
+// 228 + 34 rows, seven blocks, 1719 and 1664, 210 + 406, five, 1583 and 1552, 2 x (336 + 26), two, 663 and 648.
 float gemm_streamk_us(int M0, int M1, int N, int K, int cus) {
   const StreamkPlan p = plan_streamk(M0, M1, N, K, cus);
-  return p.groups > 0 ? p.us : 0.f;
+  if (p.groups <= 0) return 0.f;
+  const int n_tiles = (N + p.bn - 1) / p.bn, split = p.groups % n_tiles == 0 ? p.groups / n_tiles : 1;
+  return M1 > 0 ? p.us + (split - 1) * (p.bn == 256 ? 5.3f : p.bn == 192 ? 3.f : 0.f) : p.us;
 }
 
 int launch_gemm_streamk(const GemmCall* c, int count, int dtype, void* scratch, hipStream_t stream) {

@@ -713,7 +713,8 @@ extern "C" int odit_linear_rows(const void* x, const void* w, const void* bias, 
 // together, kPairTilesGated where the library would need a call per entry: past them only the tile kernel is compared.
 // Two calls are put 3 % above the sum of their estimates (the second one's rows and weights are cold when it starts). Over 104
 // pairs of 267 to 8759 and 40 to 885 rows, all four products of a dual-stream block (ms): 15.30 by this rule, 15.27 by the better of
-// the three each time, 15.33 with 0 or 6 % in the place of the 3, 15.70 where the tile kernel had to promise 6 %.
+// the three each time, 15.33 with 0 or 6 % in the place of the 3, 15.70 where the tile kernel had to promise 6 %. (Both kernels' times as planned;
+// between the two, gemm_streamk_us counts the weights from memory in.)
 constexpr int kPairTiles = 8, kPairTilesGated = 20;
 constexpr float kPairGain = 1.03f;
 
