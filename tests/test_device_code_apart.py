@@ -1,0 +1,21 @@
+"""The waits of test_device_code.py in the tile kernel's forms that round in the library's order. CPU only."""
+
+import re
+
+from test_device_code import _functions, _registers, _written_in_front
+
+
+def test_waits_that_hold_by_statement():
+    kernels = _functions("gemm_tile_apart.hip", labels=True)
+    assert len(kernels) == 4
+    for name, code in kernels.items():
+        stores = [i for i in code if i.startswith("buffer_store_dwordx4")]
+        assert len(stores) >= 16, name
+        assert [i for i in stores if not re.search(r"\], 0 offen", i)] == [], name
+        loads = [at for at, text in enumerate(code) if text.startswith("buffer_load_dwordx4") and text.endswith("lds")]
+        assert loads, name
+        for at in loads:
+            scalars = {r for o in re.split(r"[,\s]+", code[at]) for r in _registers(o) if r[0] == "s"}
+            assert len(scalars) >= 4, code[at]
+            assert code[at - 2].startswith("s_mov_b32 m0") and code[at - 1] == "s_nop 3", (name, code[at - 2:at + 1])
+            assert _written_in_front(code, at, scalars, 5) is None, (name, code[at - 8:at + 1])

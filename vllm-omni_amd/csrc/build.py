@@ -51,6 +51,7 @@ UNITS: list[tuple[str, list[str], str]] = [
     ("gemm_bf16_tile.hip", [], "gemm_bf16_tile"),
     ("gemm_tile_heads.hip", [], "gemm_tile_heads"),
     ("gemm_tile_unless.hip", [], "gemm_tile_unless"),
+    ("gemm_tile_apart.hip", [], "gemm_tile_apart"),
     ("gemm_small.hip", [], "gemm_small"),
     ("gemm_small_heads.hip", [], "gemm_small_heads"),
     ("gemm_small_norm.hip", [], "gemm_small_norm"),

@@ -73,6 +73,9 @@ int launch_gemm_tile(const GemmCall* c, int count, const TileX2* x2, int dtype, 
 // gemm_tile_unless.hip: one problem, and nothing where *unless (device memory) is not 0 when the launch begins
 int launch_gemm_tile_unless(const GemmCall& c, const int* unless, int dtype, void* scratch, hipStream_t stream);
 
+// gemm_tile_apart.hip: one problem, a gated or residual epilogue in the library's order of operations
+int launch_gemm_tile_apart(const GemmCall& c, int dtype, void* scratch, hipStream_t stream);
+
 // whether 32 bits hold the byte offsets of so many rows
 inline bool gemm_rows_fit(int rows, int64_t ld, int K) { return (static_cast<uint64_t>(rows) * ld + K) * 2 < (1ull << 32); }
 

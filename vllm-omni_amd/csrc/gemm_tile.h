@@ -128,8 +128,14 @@ __device__ __forceinline__ int epilogue_kind(const GemmEpilogue& e, int m0, int 
 // it where the register is written next, inside the main loop, and there for the tile loads in flight too (+25 % on a step).
 __device__ __forceinline__ void loads_arrived() { __builtin_amdgcn_s_waitcnt(0x0f70); }  // vmcnt(0)
 
+// A gated or residual result (APART: in the library's order of operations)
+template <typename T, bool APART>
+__device__ __forceinline__ float gated_result(const GemmEpilogue& e, float a, float gate, float bias, float residual) {
+  return gemm_clipped<T>(e, APART ? gemm_gated_apart(a, gate, residual, bias) : fmaf(gate, a, bias) + residual);
+}
+
 // This lane's part of a quadrant of a tile: 8 features from n on of the rows m, m + 16, ...
-template <typename T, int MH, int K>
+template <typename T, int MH, int K, bool APART>
 __device__ __forceinline__ void finish_quadrant(const GemmEpilogue& e, int m0, int m, int n, const f32x4_v (&v)[MH][2]) {
   const bool in = n < e.N;
   if constexpr (K == 3) {
@@ -153,8 +159,8 @@ __device__ __forceinline__ void finish_quadrant(const GemmEpilogue& e, int m0, i
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
           const f32x4_v a = v[i0 + j][u >> 1];
-          Raw<T>::set2(o, u, gemm_clipped<T>(e, fmaf(gt[j][2 * u], a[2 * (u & 1)], bs[j][2 * u]) + Raw<T>::get(res[j], 2 * u)),
-                       gemm_clipped<T>(e, fmaf(gt[j][2 * u + 1], a[2 * (u & 1) + 1], bs[j][2 * u + 1]) + Raw<T>::get(res[j], 2 * u + 1)));
+          Raw<T>::set2(o, u, gated_result<T, APART>(e, a[2 * (u & 1)], gt[j][2 * u], bs[j][2 * u], Raw<T>::get(res[j], 2 * u)),
+                       gated_result<T, APART>(e, a[2 * (u & 1) + 1], gt[j][2 * u + 1], bs[j][2 * u + 1], Raw<T>::get(res[j], 2 * u + 1)));
         }
         if (in && m + (i0 + j) * 16 < e.M) store_raw(static_cast<T*>(e.out) + (m + (i0 + j) * 16) * e.ldo + n, o);
       }
@@ -182,7 +188,7 @@ __device__ __forceinline__ void finish_quadrant(const GemmEpilogue& e, int m0, i
       }
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
-        if constexpr (K == 2) y[u] = gemm_clipped<T>(e, fmaf(gt[u], y[u], bs[u]) + Raw<T>::get(res[i], u));
+        if constexpr (K == 2) y[u] = gated_result<T, APART>(e, y[u], gt[u], bs[u], Raw<T>::get(res[i], u));
         else y[u] += bs[u];
         if constexpr (K == 1) y[u] = gemm_gelu_tanh(y[u]);
       }
@@ -193,12 +199,12 @@ __device__ __forceinline__ void finish_quadrant(const GemmEpilogue& e, int m0, i
     }
   }
 }
-template <typename T, int MH, bool UNGATED>
+template <typename T, int MH, bool UNGATED, bool APART>
 __device__ __forceinline__ void finish_quadrant(int kind, const GemmEpilogue& e, int m0, int m, int n, const f32x4_v (&v)[MH][2]) {
-  if (kind == 0) finish_quadrant<T, MH, 0>(e, m0, m, n, v);
-  else if (UNGATED || kind == 1) finish_quadrant<T, MH, 1>(e, m0, m, n, v);
-  else if (kind == 2) finish_quadrant<T, MH, 2>(e, m0, m, n, v);
-  else finish_quadrant<T, MH, 3>(e, m0, m, n, v);
+  if (kind == 0) finish_quadrant<T, MH, 0, APART>(e, m0, m, n, v);
+  else if (UNGATED || kind == 1) finish_quadrant<T, MH, 1, APART>(e, m0, m, n, v);
+  else if (kind == 2) finish_quadrant<T, MH, 2, APART>(e, m0, m, n, v);
+  else finish_quadrant<T, MH, 3, APART>(e, m0, m, n, v);
 }
 
 // ---- query, key and value heads (HeadsOut): the end of a quadrant in two passes with a barrier between them ----
@@ -246,8 +252,8 @@ __device__ __forceinline__ void store_heads(const HeadsOut& h, const u32x4 (&v)[
 
 // MH: 16-row accumulators of a wavefront in each half of the rows (4: 256-row tiles, 2: 128). HEADS: the form for problems whose
 // output is query, key and value heads, beside ordinary ones without a gate. UNLESS: nothing is done where a word of device memory is not 0 (a
-// form of its own, as the test made the others up to 0.6 % slower: M=1536, N=12288, K=3072 109.7 / 110.4 us).
-template <typename T, int MH, bool HEADS, bool UNLESS>
+// form of its own, as the test made the others up to 0.6 % slower: M=1536, N=12288, K=3072 109.7 / 110.4 us). APART: gemm_gated_apart (likewise).
+template <typename T, int MH, bool HEADS, bool UNLESS, bool APART = false>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_tile_kernel(const TileArgs<HEADS, UNLESS> p) {
   using M = Mma16<T>;
   using frag = typename M::frag;
@@ -599,7 +605,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
         for (int b = 0; b < 2; ++b)
 #pragma unroll
-          for (int h = 0; h < 2; ++h) finish_quadrant<T, MH, HEADS>(kind, e, m0, m + h * HM, n + b * 128, acc[h][b]);
+          for (int h = 0; h < 2; ++h) finish_quadrant<T, MH, HEADS, APART>(kind, e, m0, m + h * HM, n + b * 128, acc[h][b]);
       }
       // (behind the other, and opaque to it: what comes first keeps the sums in their registers whichever is taken)
       if constexpr (HEADS) {
@@ -744,7 +750,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
           if (third < 3) store_heads<T, MH>(hd, x, rows, sq, r, wn, third, n, weight);
         }
       } else {
-        finish_quadrant<T, MH, HEADS>(kind, e, m0, m0 + r, n, sum);
+        finish_quadrant<T, MH, HEADS, APART>(kind, e, m0, m0 + r, n, sum);
       }
     }
     // the last to leave hands the word back at zero

@@ -67,6 +67,7 @@ struct LinPlan {
   size_t algo_ws = 0;
   bool have_algo = false;
   bool tuned = false;
+  int passed = 0;  // the library's first choice is never run (lin_sound): it would have summed every tile whole (1), or split some (2)
   float us = 0;  // expected time of a kernel that was ranked, 0: not known
 };
 
@@ -272,6 +273,12 @@ static int lin_prepare(const LinCall& c, hipblasLtHandle_t* h, LinPlan** plan, c
   return ODIT_OK;
 }
 
+// The library's hand-scheduled kernel of 256 x 256 x 64 ("Custom_...", its first choice for most problems of many rows) now and then gives other results for
+// the same operands: 8 rows of a tile, those that one of its loads fetches (30 and 31 of each 32 rows of a half), times up to 128 features, off by the size of
+// the values themselves. In passes of a block of width 5120 over 65520 rows, five launches of it each, 1 of 100 and 1 of 300; the tile kernel in its place none of
+// 600, the library's other kernels in the same passes none. It is left out wherever a kernel is chosen, timed or named.
+static bool lin_sound(hipblasLtHandle_t h, hipblasLtMatmulAlgo_t& algo) { return hipblaslt_ext::getKernelNameFromAlgo(h, algo).rfind("Custom", 0) != 0; }
+
 // The solution that odit_linear_prefer named for this problem (a plain projection with bias and dense rows), when the
 // library has it and it accepts the problem and the workspace.
 static bool lin_preferred_algo(hipblasLtHandle_t h, LinPlan& p, const LinCall& c, size_t lib_ws_bytes) {
@@ -285,7 +292,7 @@ static bool lin_preferred_algo(hipblasLtHandle_t h, LinPlan& p, const LinCall& c
   if (solution < 0) return false;
   std::vector<int> index{solution};
   std::vector<hipblasLtMatmulHeuristicResult_t> found;
-  if (hipblaslt_ext::getAlgosFromIndex(h, index, found) != HIPBLAS_STATUS_SUCCESS || found.empty()) return false;
+  if (hipblaslt_ext::getAlgosFromIndex(h, index, found) != HIPBLAS_STATUS_SUCCESS || found.empty() || !lin_sound(h, found[0].algo)) return false;
   const float one = 1.f, zero = 0.f;
   size_t need = 0;
   if (hipblaslt_ext::matmulIsAlgoSupported(h, p.desc, &one, p.a, p.b, &zero, p.c, p.d, found[0].algo, need) != HIPBLAS_STATUS_SUCCESS ||
@@ -298,13 +305,13 @@ static bool lin_preferred_algo(hipblasLtHandle_t h, LinPlan& p, const LinCall& c
 }
 
 // Macro tile of a library kernel, from its name ("..._MT256x192x64_..."): features x rows x reduction step. Only the
-// kernels of the usual wave layout (WG32_8, or a hand-scheduled one) with steps of 64 count: the others of the same
+// kernels of the usual wave layout (WG32_8) with steps of 64 count: the others of the same
 // tile run 10 to 25 % slower, and the time model below was fitted without them.
 static bool lin_macro_tile(const std::string& name, int* features, int* rows, bool* usual) {
   const size_t at = name.find("_MT");
   int step = 0;
   if (at == std::string::npos || sscanf(name.c_str() + at, "_MT%dx%dx%d", features, rows, &step) != 3) return false;
-  *usual = step == 64 && (name.rfind("Custom", 0) == 0 || name.find("_WG32_8_", at) != std::string::npos);
+  *usual = step == 64 && name.find("_WG32_8_", at) != std::string::npos;
   return true;
 }
 
@@ -335,23 +342,45 @@ constexpr int kLinRankMinRows = 1024, kLinRankMinK = 4096;
 constexpr double kLinRankGain = 0.92, kLinTallTile = 1.01;
 constexpr int kLinCandidates = 32;
 
-static int lin_default_algo(hipblasLtHandle_t h, LinPlan& p, const LinCall& c, size_t lib_ws_bytes) {
+// The library's kernels for a problem, in its own order, and LinPlan::passed. (All of them at once: a library that has been asked for one alone, and then for
+// more of the same problem, has the rest in no order of merit. 0.2 ms, once for a problem.)
+static int lin_candidates(hipblasLtHandle_t h, LinPlan& p, size_t lib_ws_bytes, hipblasLtMatmulHeuristicResult_t* res, int* n) {
   hipblasLtMatmulPreference_t pref;
   ODIT_LT(hipblasLtMatmulPreferenceCreate(&pref));
   const uint64_t maxws = lib_ws_bytes;
   hipblasLtMatmulPreferenceSetAttribute(pref, HIPBLASLT_MATMUL_PREF_MAX_WORKSPACE_BYTES, &maxws, sizeof(maxws));
-  const bool rank = c.M >= kLinRankMinRows && c.K >= kLinRankMinK && c.dtype != ODIT_F32 && !c.first;
-  hipblasLtMatmulHeuristicResult_t res[kLinCandidates];
-  int n = 0;
-  const hipblasStatus_t st = hipblasLtMatmulAlgoGetHeuristic(h, p.desc, p.a, p.b, p.c, p.d, pref, rank ? kLinCandidates : 1, res, &n);
+  *n = 0;
+  const hipblasStatus_t st = hipblasLtMatmulAlgoGetHeuristic(h, p.desc, p.a, p.b, p.c, p.d, pref, kLinCandidates, res, n);
   hipblasLtMatmulPreferenceDestroy(pref);
-  if (st != HIPBLAS_STATUS_SUCCESS || n < 1) {
+  if (st != HIPBLAS_STATUS_SUCCESS || *n < 1) {
     set_error("odit_linear: hipBLASLt has no kernel for this problem (status %d)", static_cast<int>(st));
     return ODIT_ENOTSUP;
   }
+  p.passed = lin_sound(h, res[0].algo) ? 0 : res[0].workspaceSize == 0 ? 1 : 2;
+  return ODIT_OK;
+}
+
+static int lin_default_algo(hipblasLtHandle_t h, LinPlan& p, const LinCall& c, size_t lib_ws_bytes) {
+  const bool rank = c.M >= kLinRankMinRows && c.K >= kLinRankMinK && c.dtype != ODIT_F32 && !c.first;
+  hipblasLtMatmulHeuristicResult_t res[kLinCandidates];
+  int n = 0;
+  const int rc = lin_candidates(h, p, lib_ws_bytes, res, &n);
+  if (rc != ODIT_OK) return rc;
+  // What may run; and where the kernel passed over asks for no workspace, as it splits no tile, what asks for none either, if there is any: the
+  // same order of summation, and the same bits.
+  auto keep = [&](auto wanted) {
+    const int m = static_cast<int>(std::stable_partition(res, res + n, wanted) - res);
+    if (m > 0) n = m;
+    return m > 0;
+  };
+  if (!keep([&](hipblasLtMatmulHeuristicResult_t& r) { return lin_sound(h, r.algo); })) {
+    set_error("odit_linear: hipBLASLt has no kernel for this problem that may be run");
+    return ODIT_ENOTSUP;
+  }
+  if (p.passed == 1) keep([](hipblasLtMatmulHeuristicResult_t& r) { return r.workspaceSize == 0; });
   int best = 0;
   double best_us = 0;  // expected time of the choice, times kLinRankGain for the library's first
-  const int cus = rank ? device_cus() : 0;
+  const int cus = rank || p.passed == 1 ? device_cus() : 0;
   for (int i = 0; i < n && cus > 0; ++i) {
     int features, rows;
     bool usual;
@@ -466,6 +495,7 @@ static int lin_handwritten_kind(const odit::GemmCall& g, int dtype, const void* 
 static int lin_launch_handwritten(int kind, const odit::GemmCall& g, int dtype, void* sk, hipStream_t stream) {
   if (kind == 1) return odit::launch_gemm_streamk(&g, 1, dtype, sk, stream);
   if (kind == 3) return odit::launch_gemm_small(&g, 1, dtype, stream);
+  if (kind == 4) return odit::launch_gemm_tile_apart(g, dtype, sk, stream);
   return odit::launch_gemm_tile(&g, 1, nullptr, dtype, sk, stream);
 }
 
@@ -525,6 +555,21 @@ static float lin_library_us(const odit::LinCall& c, const odit::GemmCall& g) {  
   return full * lin_library_us(c, g.rows_per_gate) + (last > 0 ? lin_library_us(c, last) : 0.f);
 }
 
+// Whether the library's first choice for a problem (of launches for groups of rows, the first group's) is one that never runs: LinPlan::passed.
+static int lin_passed(const odit::LinCall& c, const odit::GemmCall& g) {
+  using namespace odit;
+  LinCall one = c;
+  if (g.rows_per_gate > 0) one.M = g.rows_per_gate;
+  hipblasLtHandle_t h;
+  LinPlan* p;
+  const size_t gb = lin_gate_bytes(one), room = one.ws && gb <= one.ws_bytes ? one.ws_bytes - gb : 0;
+  if (lin_find_plan(one, &h, &p) != ODIT_OK || p->tuned) return 0;  // (the call says what is wrong)
+  if (p->passed != 0 || p->have_algo) return p->passed;
+  hipblasLtMatmulHeuristicResult_t res[kLinCandidates];
+  int n = 0;
+  return lin_preferred_algo(h, *p, one, room) || lin_candidates(h, *p, room, res, &n) != ODIT_OK ? 0 : p->passed;
+}
+
 // The stream-K kernel for one problem: where the reduction is long against the number of output features (K >= 2 N: the
 // library's choices split K badly there: M=80, N=3072, K=12288 57 us against 31, M=512 69 against 52, M=1024 110 against 85) and
 // there is work for all CUs; with a small product (kSmallWeights: a few MB of weights) its ranges would be shorter than what
@@ -571,16 +616,26 @@ static float lin_call_us(int dev, const odit::LinCall& c, const odit::GemmCall& 
   return us;
 }
 static int lin_rule_kind(const odit::LinCall& c, const odit::GemmCall& g, const void* sk) {
-  const bool tile = !c.no_tile && g.M >= kTileMinAuto && odit::gemm_tile_takes(g, c.dtype);
+  const bool takes = g.M >= kTileMinAuto && odit::gemm_tile_takes(g, c.dtype), tile = !c.no_tile && takes;
   if (sk != nullptr && lin_streamk_rule(g) && odit::gemm_streamk_takes(g, c.dtype)) {
     const int cus = odit::device_cus();
     const odit::TilePlan plan = tile ? odit::plan_gemm_tile(&g, 1, cus, true) : odit::TilePlan{};
     return plan.bm > 0 && plan.us < odit::gemm_streamk_us(g.M, 0, g.N, g.K, cus) ? 2 : 1;
   }
   if (!c.no_tile && odit::gemm_streamk_takes(g, c.dtype) && odit::gemm_small_rule(&g, 1, odit::device_cus(), kSmallK)) return 3;
-  if (!tile) return 0;
+  if (!takes) return 0;
   const odit::TilePlan plan = odit::plan_gemm_tile(&g, 1, odit::device_cus(), sk != nullptr);
-  return plan.bm > 0 && plan.us < lin_library_us(c, g) ? 2 : 0;
+  if (plan.bm == 0) return 0;
+  if (tile && plan.us < lin_library_us(c, g)) return 2;
+  // In the place of a kernel that never runs the tile kernel does. A call that wants no other order of summation has every tile whole where that kernel would have had it so,
+  // and in gated and residual epilogues the library's order of operations (kind 4): the library's bits, but for GELU, whose own is left to the library's next kernel. (65520
+  // rows of a pair, us, the library's next / this: N=15360, K=5120 7690 / 6930, N=5120 gated 2750 / 2340, K=13824 7200 / 6010.) Where it would have split tiles, no
+  // other kernel's sums are those.
+  const int passed = lin_passed(c, g);
+  if (passed == 0) return 0;
+  if (tile) return 2;
+  const bool gelu = c.epilogue == ODIT_EPI_GELU_TANH || c.epilogue == ODIT_EPI_BIAS_GELU_TANH;
+  return passed == 2 || (plan.parts == 1 && !gelu) ? 4 : 0;
 }
 static int lin_auto_kind(int dev, const odit::LinCall& c, const odit::GemmCall& g, const void* sk) {
   odit::Tuned found;
@@ -1126,7 +1181,7 @@ static int lin_tune_library(const odit::LinCall& c, int iters, void* flush, size
   for (size_t i = 0; i < all.size(); ++i) {
     size_t need = 0;
     if (hipblaslt_ext::matmulIsAlgoSupported(h, p->desc, alpha, p->a, p->b, &beta, p->c, p->d, all[i].algo, need) !=
-            HIPBLAS_STATUS_SUCCESS || need > lws_bytes)
+            HIPBLAS_STATUS_SUCCESS || need > lws_bytes || !lin_sound(h, all[i].algo))
       continue;
     all[i].workspaceSize = need;
     const float us = time_algo(all[i].algo, 2);

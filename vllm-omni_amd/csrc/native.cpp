@@ -2029,7 +2029,7 @@ PyObject* py_wan_block(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return none();
   if (!block_input(c, x)) return PyErr_Occurred() ? nullptr : none();
   const int64_t B = x->size(0), S = x->size(1), C = x->size(2), HD = H * D, T = ctx->dim() == 3 ? ctx->size(1) : 0;
-  // A batch (in the video pipelines a CFG pair) keeps the library's own kernels, or those a tuning call chose. Another order of
+  // A batch (in the video pipelines a CFG pair) keeps the library's own kernels, what stands in for the one of them that is never run, or those a tuning call chose. Another order of
   // summation is neither better nor worse: against a float32 model the guided noise of 16 batches is 2.03e-2 to 2.8e-2 off (bf16;
   // fp16 2.6e-3 to 3.5e-3) whichever kernels ran. But guidance (scale 5) multiplies the difference of the two rows, so two orders
   // are as far from each other, and results of earlier versions are reproduced. It costs 12 % at B=2 S=3536 and 0 to 7 %
