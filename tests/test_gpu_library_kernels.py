@@ -95,3 +95,27 @@ def test_a_tuning_call_does_not_choose_it(gpu):
     kernels.linear(p.x, p.w, p.bias, tune_iters=2, engine="library")
     _, names = p.names(LIBRARY)
     assert names and not any(n.startswith("Custom") for n in names), names
+
+
+@pytest.mark.parametrize("B", [1, 2])
+def test_image_conditioned_video(gpu, B):
+    """A block that runs operation by operation (its cross-attention has image tokens too)."""
+    from vllm_omni_amd.blocks.wan import WanTransformerBlock
+
+    g = torch.Generator(device=gpu).manual_seed(B)
+    with torch.device(gpu):
+        block = WanTransformerBlock(5120, 13824, 40, added_kv_proj_dim=5120, cross_attn_norm=True).bfloat16().eval()
+    with torch.no_grad():
+        for p in block.parameters():
+            p.normal_(0.0, 0.02, generator=g)
+    x, ctx = torch.randn(B, 7072 // B, 5120, device=gpu, generator=g).bfloat16(), torch.randn(B, 257 + 512, 5120, device=gpu, generator=g).bfloat16()
+    temb = torch.randn(B, 6, 5120, device=gpu, generator=g).bfloat16()
+    with torch.inference_mode():
+        out = block(x, ctx, temb)
+        torch.cuda.synchronize()
+        with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as p:
+            again = block(x, ctx, temb)
+            torch.cuda.synchronize()
+    names = [e.name for e in p.events()]
+    assert names and not any(n.startswith("Custom") for n in names), names
+    assert torch.equal(out, again)

@@ -129,6 +129,15 @@ def _batch_engine(x: torch.Tensor) -> str | None:
     return "no_tile" if x.shape[0] > 1 and kernels.linear_engine_flags() == 0 else None
 
 
+def _product(lin: nn.Module, x: torch.Tensor) -> torch.Tensor:
+    """``lin(x)`` on the kernels that the native block's products run on; torch's own call of a Linear may take the one of the library's that
+    ``odit_linear`` never runs."""
+    if (kernels.native_blocks() and kernels.plain_module(lin, nn.Linear) and x.is_cuda and x.dtype in (torch.bfloat16, torch.float16)
+            and lin.weight.dtype == x.dtype):
+        return kernels.linear(x, lin.weight, lin.bias, engine=_batch_engine(x))
+    return lin(x)
+
+
 def _feed_up(net_0: nn.Module, x: torch.Tensor) -> torch.Tensor:
     engine = _batch_engine(x)
     return net_0(x, engine=engine) if engine and kernels.plain_module(net_0, ApproxGELU) else net_0(x)
@@ -168,7 +177,7 @@ class WanSelfAttention(nn.Module):
         rot = _rotary(rotary_emb)
         B, S, _ = hidden_states.shape
         H, D = self.num_heads, self.head_dim
-        qkv = self.to_qkv(hidden_states).view(B, S, 3, H, D)
+        qkv = _product(self.to_qkv, hidden_states).view(B, S, 3, H, D)
         q = torch.empty((B, S, H, D), dtype=qkv.dtype, device=qkv.device)
         k = torch.empty_like(q)
         cos, sin = (rot.cos32, rot.sin32) if rot is not None else (None, None)
@@ -226,7 +235,7 @@ class WanCrossAttention(nn.Module):
                                 eps=norm.eps, norm_mode=ODIT_NORM_ROW)
             return out_
 
-        q = normed(self.to_q(hidden_states).view(B, S, H, D), self.norm_q)
+        q = normed(_product(self.to_q, hidden_states).view(B, S, H, D), self.norm_q)
         k = normed(self.to_k(encoder_hidden_states).view(B, T, H, D), self.norm_k)
         v = self.to_v(encoder_hidden_states).view(B, T, H, D)
         o = self.attn(q, k, v).flatten(2, 3)
