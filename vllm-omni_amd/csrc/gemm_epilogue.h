@@ -33,6 +33,9 @@ struct GemmEpilogue {
   float most;  // largest size of a gated result of f16 (infinite: as it comes)
 };
 
+// Held to a size of at most `most`; a NaN stays one.
+__device__ __forceinline__ float f16_clipped(float y, float most = 65504.f) { return __builtin_elementwise_minimum(__builtin_elementwise_maximum(y, -most), most); }
+
 // A gated result as ODIT_LINEAR_CLIP asks for it. Clipped before it is rounded: what rounds to infinity lies above the largest finite value, so
 // these are the bits of a clip behind the rounding. That was a pass of its own over each stream behind every block; whole models in f16, width
 // 3072, with it and without (us): 1085 + 44 rows, four blocks, 2511 and 2466; 169 + 121 and 269, five, 1852 and 1811; 6156 + 44, six, 19796 and 19714.

@@ -15,7 +15,7 @@
 // K x N (ld = ldw, transposed), B = x stored K x M (ld = ldx): the bias and the alpha vector run along
 // D's rows, i.e. along the N output features, as needed.
 #include "odit_common.h"
-#include "gemm_bf16.h"
+#include "gemm_epilogue.h"
 #include "time_tokens.h"
 
 #include <hipblaslt/hipblaslt.h>

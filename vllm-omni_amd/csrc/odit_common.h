@@ -138,9 +138,6 @@ template <> struct Raw<float> {
   }
 };
 
-// Held to a size of at most `most`; a NaN stays one.
-__device__ __forceinline__ float f16_clipped(float y, float most = 65504.f) { return __builtin_elementwise_minimum(__builtin_elementwise_maximum(y, -most), most); }
-
 // ---- wavefront (64 lanes) reductions ------------------------------------------------------------
 // Cross-lane adds inside a 16-lane DPP row cost one VALU instruction each (no LDS crossbar trip):
 // xor-1 and xor-2 quad permutes, then the half-row and full-row mirrors.
