@@ -692,3 +692,11 @@ def test_profile_records_name_the_launches_they_were_measured_on():
                                              "attn_merge_kernel<T, 128, 256>"]
     assert profiling._is_kernel("attn_merge_kernel<T, 128, 256>", "void odit::attn_merge_kernel<odit::bf16_t, 128, 256>(odit::AttnParams, int)")
     assert not profiling._is_kernel("attn_fwd_dma_kernel<T, 128, 8, 1>", "void odit::attn_fwd_dma_kernel<odit::bf16_t, 128, 8, 0>(odit::AttnParams)")
+
+
+def test_committed_counters_are_of_this_source():
+    """What bench.py prints beside its line holds for the attention kernels that it runs: the digest covers their headers too."""
+    from vllm_omni_amd import profiling
+
+    for name in (profiling.TRAFFIC_FILE, profiling.COUNTERS_FILE):
+        assert profiling.read_record(name)["attention_source"] == profiling.attention_source()
