@@ -513,16 +513,20 @@ class AdaLayerNormContinuous(nn.Module):
     def head(self, lin: nn.Module, x: torch.Tensor, cond: torch.Tensor, emb: torch.Tensor | None = None) -> torch.Tensor:
         """``lin(self(x, cond))``, in one launch where that is the faster way; ``emb``: the projection of the condition where the caller has it (of a
         module that is plainly of this class)."""
+        own = "modulate" not in self.__dict__ and (AdaLayerNormContinuous.forward, AdaLayerNormContinuous.modulate) == _OWN_HEAD
         if emb is None:
-            if cond.dtype != x.dtype or not kernels.plain_module(self, AdaLayerNormContinuous):
+            if not own or cond.dtype != x.dtype or not kernels.plain_module(self, AdaLayerNormContinuous):
                 return kernels.project(lin, self(x, cond))
             emb = kernels.project(self.linear, cond, silu_input=True)
-        if "modulate" not in self.__dict__:
+        if own:
             scale, shift = emb.chunk(2, dim=1)
             out = kernels.project_normed(lin, x, shift, scale, self.eps)
             if out is not None:
                 return out
         return kernels.project(lin, self.modulate(x, emb))
+
+
+_OWN_HEAD = (AdaLayerNormContinuous.forward, AdaLayerNormContinuous.modulate)  # (a program may put others on the class)
 
 
 def _build_conditioning_index(samples: tuple, device: str) -> torch.Tensor:
