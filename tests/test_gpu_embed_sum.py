@@ -61,3 +61,22 @@ def test_what_is_left_to_the_separate_launches(gpu):
         assert _together(m, t, t, pooled, 1.0) is None and torch.equal(m(t, t, pooled), _apart(m, t, t, pooled, 1.0))
     m = _embedders(gpu, 512, 96, BF16)
     assert _together(m, t, t, pooled, 1.0) is None  # with gradients
+
+
+def test_replaced_methods_are_called(gpu, monkeypatch):
+    """What a program has put on a class, as on a module, takes effect."""
+    from vllm_omni_amd.blocks.flux import PixArtAlphaTextProjection
+
+    m, t, pooled = _embedders(gpu, 512, 96, BF16), torch.rand(2, device=gpu), torch.randn(2, 96, device=gpu).to(BF16)
+    with torch.inference_mode():
+        text, times = m.text_embedder(pooled), QwenTimestepProjEmbeddings.embed(m.timestep_embedder, t, BF16, scale=1.0)
+        with monkeypatch.context() as p:
+            p.setattr(PixArtAlphaTextProjection, "forward", lambda self, x: torch.ones_like(text))
+            assert torch.equal(m(t, None, pooled), times + 1)
+        with monkeypatch.context() as p:
+            p.setattr(QwenTimestepProjEmbeddings, "embed", staticmethod(lambda *a, **k: torch.ones_like(text)))
+            assert torch.equal(m(t, None, pooled), 1 + text)
+        with monkeypatch.context() as p:
+            p.setitem(m.text_embedder.__dict__, "forward", lambda x: torch.ones_like(text))
+            assert torch.equal(m(t, None, pooled), times + 1)
+        assert torch.equal(m(t, None, pooled), times + text)

@@ -373,15 +373,19 @@ class CombinedTimestepGuidanceTextProjEmbeddings(nn.Module):
 
     def forward(self, timestep: torch.Tensor, guidance: torch.Tensor | None, pooled_projection: torch.Tensor,
                 pre: float = 1.0):
-        done = kernels.embed_sum(self.timestep_embedder, timestep, None if guidance is None else self.guidance_embedder, guidance, self.text_embedder,
-                                 pooled_projection, 256, 10000, 1.0, pre)
-        if done is not None:
-            return done
+        if (PixArtAlphaTextProjection.forward, QwenTimestepProjEmbeddings.embed) == _OWN_EMBEDDERS:
+            done = kernels.embed_sum(self.timestep_embedder, timestep, None if guidance is None else self.guidance_embedder, guidance, self.text_embedder,
+                                     pooled_projection, 256, 10000, 1.0, pre)
+            if done is not None:
+                return done
         embed, dtype = QwenTimestepProjEmbeddings.embed, pooled_projection.dtype
         emb = embed(self.timestep_embedder, timestep, dtype, scale=1.0, pre=pre)
         if guidance is not None:
             emb = emb + embed(self.guidance_embedder, guidance, dtype, scale=1.0, pre=pre)
         return emb + self.text_embedder(pooled_projection)
+
+
+_OWN_EMBEDDERS = (PixArtAlphaTextProjection.forward, QwenTimestepProjEmbeddings.embed)  # (a program may put others on the classes)
 
 
 class FluxSteps:
