@@ -111,3 +111,21 @@ class _Plain(nn.Module):
 
     def forward(self, x):
         return self.norm(x) * 2
+
+
+@pytest.mark.parametrize("which", [0, 1, 2])
+def test_replaced_on_any_class(gpu, which, monkeypatch):
+    """torch looks for its ways of calling a module in all of the layer's classes."""
+    from vllm_omni_amd.layers.custom_op import CustomOp
+
+    layer, args = _layers(gpu)[which]
+    own = lambda *a, **k: "own"
+    with torch.inference_mode():
+        want = layer.forward(*args)
+        for cls in (type(layer), CustomOp, nn.Module):
+            for name in ("_call_impl", "_compiled_call_impl"):
+                with monkeypatch.context() as m:
+                    m.setattr(cls, name, own, raising=False)
+                    assert not _at_once(layer, args)
+                    assert layer(*args) == "own"
+                assert _at_once(layer, args) and _equal(layer(*args), want)

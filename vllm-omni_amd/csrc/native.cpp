@@ -1077,11 +1077,14 @@ bool calls_only(PyObject* m, PyObject* forward) {
     if (!no_hooks(d, name)) return false;
   for (PyObject* name : g_name.global_hooks)
     if (!no_hooks(g_module_globals, name)) return false;
-  PyObject* const ways[3] = {g_name.call, g_name.call_impl, g_name.wrapped_call_impl};
-  for (int i = 0; i < 3; ++i)
-    if (item(torch_way, ways[i]) != g_module_call[i] || (i > 0 && item(d, ways[i]) != nullptr)) return false;
+  // (torch finds these through the instance and all of its classes)
+  if (item(torch_way, g_name.call) != g_module_call[0]) return false;
+  PyObject* const ways[2] = {g_name.call_impl, g_name.wrapped_call_impl};
+  for (int i = 0; i < 2; ++i)
+    if (item(d, ways[i]) != nullptr || _PyType_Lookup(Py_TYPE(m), ways[i]) != g_module_call[i + 1]) return false;
   PyObject* compiled = item(d, g_name.compiled_call_impl);
-  return item(d, g_name.forward) == nullptr && (compiled == nullptr || compiled == Py_None) && !torch::jit::tracer::isTracing();
+  return item(d, g_name.forward) == nullptr && (compiled == nullptr || compiled == Py_None) && _PyType_Lookup(Py_TYPE(m), g_name.compiled_call_impl) == Py_None &&
+         !torch::jit::tracer::isTracing();
 }
 // (layer, its arguments): the whole call of an RMSNorm, an AdaLayerNorm or a RotaryEmbedding; None where torch has to make it
 PyObject* py_layer_call(PyObject* self, PyObject* const* a, Py_ssize_t n) {
