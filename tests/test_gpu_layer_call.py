@@ -2,6 +2,7 @@
 and classes, compiled modules, traces and a replaced way of calling modules are seen by torch as ever."""
 
 import pickle
+import sys
 
 import pytest
 import torch
@@ -129,3 +130,23 @@ def test_replaced_on_any_class(gpu, which, monkeypatch):
                     assert not _at_once(layer, args)
                     assert layer(*args) == "own"
                 assert _at_once(layer, args) and _equal(layer(*args), want)
+
+
+@pytest.mark.parametrize("which", [0, 1, 2])
+def test_calls_that_are_followed(gpu, which, tmp_path):
+    """A profiler or debugger of the thread sees torch's call of the module and the layer's forward."""
+    layer, args = _layers(gpu)[which]
+    for follow in (sys.setprofile, sys.settrace):
+        calls = []
+        before = sys.gettrace() if follow is sys.settrace else sys.getprofile()
+        with torch.inference_mode():
+            follow(lambda frame, event, arg: calls.append(frame.f_code.co_name) if event == "call" else None)
+            layer(*args)
+            follow(before)
+        assert "_call_impl" in calls and "forward" in calls, calls
+    with torch.inference_mode(), torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU], with_stack=True) as p:
+        layer(*args)
+    p.export_chrome_trace(str(tmp_path / "trace.json"))
+    assert f"nn.Module: {type(layer).__name__}" in (tmp_path / "trace.json").read_text()
+    with torch.inference_mode():
+        assert _at_once(layer, args)

@@ -1064,7 +1064,7 @@ PyObject* py_rotary_of(PyObject*, PyObject* const* a, Py_ssize_t n) {
 }
 
 // Whether a call of `m`, as torch makes it, would do nothing but call its class's own `forward`: no hook of any kind on it or on all modules, nothing compiled, no trace
-// being taken, and neither torch's way of calling modules (which torch.fx exchanges while it traces) nor the layer's forward replaced.
+// being taken, nobody following the thread's calls, and neither torch's way of calling modules (which torch.fx exchanges while it traces) nor the layer's forward replaced.
 PyObject *g_module_type, *g_module_globals, *g_module_call[3], *g_rmsnorm_forward, *g_adaln_forward, *g_rotary_forward;
 bool no_hooks(PyObject* dict, PyObject* name) {
   PyObject* h = item(dict, name);
@@ -1083,8 +1083,9 @@ bool calls_only(PyObject* m, PyObject* forward) {
   for (int i = 0; i < 2; ++i)
     if (item(d, ways[i]) != nullptr || _PyType_Lookup(Py_TYPE(m), ways[i]) != g_module_call[i + 1]) return false;
   PyObject* compiled = item(d, g_name.compiled_call_impl);
+  const PyThreadState* const thread = PyThreadState_Get();  // (a profiler or debugger that follows calls is shown torch's: torch.profiler's module events are those)
   return item(d, g_name.forward) == nullptr && (compiled == nullptr || compiled == Py_None) && _PyType_Lookup(Py_TYPE(m), g_name.compiled_call_impl) == Py_None &&
-         !torch::jit::tracer::isTracing();
+         thread->c_profilefunc == nullptr && thread->c_tracefunc == nullptr && !torch::jit::tracer::isTracing();
 }
 // (layer, its arguments): the whole call of an RMSNorm, an AdaLayerNorm or a RotaryEmbedding; None where torch has to make it
 PyObject* py_layer_call(PyObject* self, PyObject* const* a, Py_ssize_t n) {
