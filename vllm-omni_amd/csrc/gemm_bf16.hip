@@ -495,7 +495,11 @@ bool gemm_streamk_takes(const GemmCall& c, int dtype) {
 // partial tiles per workgroup. The times are fitted to 16 <= M <= 1024 rows of the four projections of width 3072 (us; a
 // step of 64: 128-wide tiles 0.62, 192 0.74, 256 0.88; a launch 8; each further contributor of a tile 1.2, 2.0, 2.7; a
 // second range 4, 10, 16; a further whole tile 6). M=512, N=9216, K=3072: 128-wide 45.7, 192-wide 42.6, 256-wide 47.8;
-// M=80, N=3072, K=12288: 31.1, 41.5, 53.0; M=768, N=9216, K=3072: 65.4, 59.2, 52.3.
+// M=80, N=3072, K=12288: 31.1, 41.5, 53.0; M=768, N=9216, K=3072: 65.4, 59.2, 52.3. Two problems pay more for workgroups that share a tile, as twice
+// the weights arrive from memory meanwhile (pair_*). us, 128 / 192 / 256 wide at their best / the tile kernel: 195 + 256 rows, N=3072, K=3072 25.9 / 25.1 / 29.1 / 24.7;
+// 300 + 300 29.0 / 28.5 / 30.1 / 27.4; 768 + 128 35.2 / 34.8 / 35.6 / 30.4; N=9216: 128 + 40 37.3 / 37.4 / 38.2 / 35.8, 256 + 64 39.8 / 44.2 / 44.6 / 39.4. Choosing among
+// these forms and the tile kernel by the two plans' times takes 0.63 % longer than the best of all over 110 pairs of 2 to 8 row tiles, 0.02 % over 60 of 9 to 20;
+// with one problem's times for two 2.4 and 0.1 %, with what is paid added behind the choice of the form 0.83 %.
 struct StreamkPlan { int bm, bn, mt0, m_tiles, groups; float us; };
 
 static StreamkPlan plan_streamk(int M0, int M1, int N, int K, int cus) {
@@ -507,8 +511,11 @@ static StreamkPlan plan_streamk(int M0, int M1, int N, int K, int cus) {
   p.m_tiles = p.mt0 + (M1 > 0 ? row_tiles(M1, p.bm) : 0);
   if (p.m_tiles > most) return best;
   const int k_steps = K / kGemmBK, room = most / p.m_tiles;
-  static const struct { int bn; float step, share, range; } kinds[3] = {{128, .62f, 1.2f, 4.f}, {192, .74f, 2.f, 10.f}, {256, .88f, 2.7f, 16.f}};
+  // pair_*: what two problems pay beyond that, as twice the weights arrive from memory meanwhile
+  static const struct { int bn; float step, share, range, pair_share, pair_range; } kinds[3] = {
+      {128, .62f, 1.2f, 4.f, 0.f, 2.f}, {192, .74f, 2.f, 10.f, 3.f, 0.f}, {256, .88f, 2.7f, 16.f, 5.3f, 0.f}};
   for (const auto& k : kinds) {
+    const float share = k.share + (M1 > 0 ? k.pair_share : 0.f), range = k.range + (M1 > 0 ? k.pair_range : 0.f);
     if (p.bm == 64 && k.bn != 128) continue;
     const int n_tiles = (N + k.bn - 1) / k.bn;
     if (static_cast<int64_t>(p.m_tiles) * n_tiles * 8 > static_cast<int64_t>(kGemmCounterBytes)) continue;
@@ -520,26 +527,19 @@ static StreamkPlan plan_streamk(int M0, int M1, int N, int K, int cus) {
     };
     if (room >= n_tiles) {
       const int split = room / n_tiles < k_steps ? room / n_tiles : k_steps;
-      offer(n_tiles * split, 8.f + (k_steps + split - 1) / split * k.step + (split - 1) * k.share);
+      offer(n_tiles * split, 8.f + (k_steps + split - 1) / split * k.step + (split - 1) * share);
     }
     const int64_t total = static_cast<int64_t>(n_tiles) * k_steps;
     const int groups = total < room ? static_cast<int>(total) : room;
     const int64_t steps = (total + groups - 1) / groups;
-    offer(groups, 8.f + steps * k.step + k.range + static_cast<float>(steps / k_steps) * 6.f);
+    offer(groups, 8.f + steps * k.step + range + static_cast<float>(steps / k_steps) * 6.f);
   }
   return best;
 }
 
-// Two problems whose tiles several workgroups share: each further one costs 3 us more with 192-wide tiles and 5.3 with 256-wide ones than the plan's time has it, as
-// twice the weights arrive from memory meanwhile. us, as planned / so / measured / the tile kernel (N=9216, K=3072): 128 + 40 rows 27.5 / 38 / 38.4 / 35.7, 256 + 64
-// 31.8 / 37 / 45 / 39.8; N=3072, K=3072: 195 + 256 22.9 / 32 / 29.6 / 25.2, 300 + 300 27.5 / 38 / 30.9 / 27.9, 768 + 128 27.5 / 38 / 35.4 / 30.5. Over 79 pairs of 2 to 8
-// row tiles the choice between the two kernels takes 0.45 % longer than the better one each time, by the plan's times 1.5 %; whole models, us:
-// 228 + 34 rows, seven blocks, 1719 and 1664, 210 + 406, five, 1583 and 1552, 2 x (336 + 26), two, 663 and 648.
 float gemm_streamk_us(int M0, int M1, int N, int K, int cus) {
   const StreamkPlan p = plan_streamk(M0, M1, N, K, cus);
-  if (p.groups <= 0) return 0.f;
-  const int n_tiles = (N + p.bn - 1) / p.bn, split = p.groups % n_tiles == 0 ? p.groups / n_tiles : 1;
-  return M1 > 0 ? p.us + (split - 1) * (p.bn == 256 ? 5.3f : p.bn == 192 ? 3.f : 0.f) : p.us;
+  return p.groups > 0 ? p.us : 0.f;
 }
 
 int launch_gemm_streamk(const GemmCall* c, int count, int dtype, void* scratch, hipStream_t stream) {

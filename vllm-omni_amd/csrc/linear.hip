@@ -767,9 +767,9 @@ extern "C" int odit_linear_rows(const void* x, const void* w, const void* bias, 
 // / 169 / 183, out - / 65 / 83, up - / 219 / 241, down - / 231 / 246. The stream-K kernel's fit ends at kPairTiles tiles of 128 rows
 // together, kPairTilesGated where the library would need a call per entry: past them only the tile kernel is compared.
 // Two calls are put 3 % above the sum of their estimates (the second one's rows and weights are cold when it starts). Over 104
-// pairs of 267 to 8759 and 40 to 885 rows, all four products of a dual-stream block (ms): 15.30 by this rule, 15.27 by the better of
-// the three each time, 15.33 with 0 or 6 % in the place of the 3, 15.70 where the tile kernel had to promise 6 %. (Both kernels' times as planned;
-// between the two, gemm_streamk_us counts the weights from memory in.)
+// pairs of 267 to 8759 and 40 to 885 rows, all four products of a dual-stream block (ms): 15.30 by this margin, 15.27 by the better of
+// the three each time, 15.33 with 0 or 6 % in the place of the 3, 15.70 where the tile kernel had to promise 6 %. (Measured with the times that one
+// problem's form has; plan_streamk says what a pair's cost by now.)
 constexpr int kPairTiles = 8, kPairTilesGated = 20;
 constexpr float kPairGain = 1.03f;
 
