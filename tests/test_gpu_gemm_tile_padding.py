@@ -1,5 +1,5 @@
-"""The tile kernel at the ends of its operands: rows and features of padding (fetched as zeros) in dense and strided operands, in
-one tensor and two, change no row of the result and stay unread, whatever lies behind the operand."""
+"""The tile kernel at the ends of its operands: rows and features of padding in dense and strided operands, in one tensor and two, change no row of the result, and
+none behind the last is written, whatever lies behind the operand. (Where they are fetched from: test_tile_plans.py.)"""
 
 import pytest
 import torch

@@ -22,18 +22,23 @@ def scratch(gpu):
     assert int(ws[:32768].view(torch.int32).abs().max().item()) == 0, "ticket words are handed back at zero"
 
 
-@pytest.mark.parametrize("M, N, K", [
-    (1100, 1280, 12288),  # 45 tiles in 5 parts
-    (1700, 704, 12288),   # 42 in 6
-    (1100, 1000, 12352),  # 36 in 7, of 27 and 28 steps
-    (1025, 520, 8192),    # 27 in 8, one row in the last tile
-    (1100, 8, 704),       # 9 of 11 steps
-])
+# (rows, features, reduction, parts; test_tile_plans.py holds the plan to them)
+PARTS = [
+    (1100, 1280, 12288, 5),  # 45 tiles
+    (1700, 704, 12288, 6),   # 42
+    (1100, 1000, 12352, 7),  # 36, parts of 27 and 28 steps
+    (1025, 520, 8192, 8),    # 27, one row in the last tile
+    (1100, 8, 1408, 6),      # 9, parts of 3 and 4 steps
+]
+HEADS = [(300, 100, 3, 8192, 8), (500, 9, 4, 8192, 8), (640, 9, 4, 8192, 7)]  # (rows of two, heads of 128, reduction, parts)
+
+
+@pytest.mark.parametrize("M, N, K, parts", PARTS)
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-def test_parts(scratch, gpu, M, N, K, dtype):
+def test_parts(scratch, gpu, M, N, K, parts, dtype):
     from vllm_omni_amd import kernels
 
-    print(f"parts {dtype} {M}x{N}x{K}", flush=True)
+    print(f"{parts} parts {dtype} {M}x{N}x{K}", flush=True)
     g = torch.Generator(device=gpu).manual_seed(N)
     x, w, b = torch.randn(M, K, device=gpu, generator=g).to(dtype), (torch.randn(N, K, device=gpu, generator=g) * 0.05).to(dtype), torch.randn(N, device=gpu, generator=g).to(dtype)
     residual = torch.randn(M, N, device=gpu, generator=g).to(dtype)
@@ -46,10 +51,10 @@ def test_parts(scratch, gpu, M, N, K, dtype):
         assert torch.equal(added, kernels.linear(x, w, b, residual=residual, engine="handwritten"))
 
 
-@pytest.mark.parametrize("S0, S1, H, K", [(300, 100, 3, 8192), (500, 9, 8, 8192)])
+@pytest.mark.parametrize("S0, S1, H, K, parts", HEADS)
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-def test_heads(scratch, gpu, S0, S1, H, K, dtype):
-    print(f"heads of parts {dtype} {S0}+{S1} rows, {H} heads, K={K}", flush=True)
+def test_heads(scratch, gpu, S0, S1, H, K, parts, dtype):
+    print(f"heads of {parts} parts {dtype} {S0}+{S1} rows, {H} heads, K={K}", flush=True)
     ps = [_Problem(gpu, dtype, 1, S0, K, H, 128, seed=1), _Problem(gpu, dtype, 1, S1, K, H, 128, seed=2)]
     joint = [torch.full((1, S0 + S1, H, 128), float("nan"), dtype=dtype, device=gpu) for _ in range(3)]
     for _ in range(2):

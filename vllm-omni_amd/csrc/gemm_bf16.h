@@ -78,6 +78,11 @@ int launch_gemm_tile_apart(const GemmCall& c, int dtype, void* scratch, hipStrea
 
 // whether 32 bits hold the byte offsets of so many rows
 inline bool gemm_rows_fit(int rows, int64_t ld, int K) { return (static_cast<uint64_t>(rows) * ld + K) * 2 < (1ull << 32); }
+// the last row that a tile's rows of padding are fetched as: their own place past the operand's end, or where those offsets would wrap around the operand's last row
+inline int tile_padding_row(int rows, int tile, int64_t ld, int K) {
+  const int end = (rows + tile - 1) / tile * tile;
+  return gemm_rows_fit(end, ld, K) ? end : rows - 1;
+}
 
 // ---- gemm_tile_heads.hip: the tile kernel with query, key and value heads at its end -------
 // Output of a projection to 3 HD features: per batch entry S rows of queries, keys and values of HD / D heads, the first two normed

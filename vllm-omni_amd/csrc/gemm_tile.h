@@ -784,9 +784,8 @@ inline void fill_tile_params(TileParams& p, const TilePlan& plan, const GemmCall
     q.w_bytes = static_cast<uint32_t>((static_cast<uint64_t>(g.N - 1) * g.ldw + g.K) * 2);
     q.m_tiles = (g.M + plan.bm - 1) / plan.bm;
     q.n_tiles = (g.N + kTileN - 1) / kTileN;
-    const int m_end = q.m_tiles * plan.bm, n_end = q.n_tiles * kTileN;
-    q.x_last = gemm_rows_fit(m_end, x2 ? std::max(g.ldx, x2->ldx) : g.ldx, g.K) ? m_end : g.M - 1;
-    q.w_last = gemm_rows_fit(n_end, g.ldw, g.K) ? n_end : g.N - 1;
+    q.x_last = tile_padding_row(g.M, plan.bm, x2 ? std::max(g.ldx, x2->ldx) : g.ldx, g.K);
+    q.w_last = tile_padding_row(g.N, kTileN, g.ldw, g.K);
     q.ep = gemm_epilogue_of(g);
   }
   p.tiles0 = plan.tiles0; p.tiles1 = plan.tiles1; p.tiles = plan.tiles; p.whole = plan.whole; p.parts = plan.parts;
