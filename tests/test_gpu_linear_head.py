@@ -4,6 +4,7 @@ batch entries, in each of its three tile widths."""
 import pytest
 import torch
 
+import vllm_omni_amd.blocks.qwen_image  # noqa: F401  (names the module classes that native calls take)
 from vllm_omni_amd import kernels
 
 pytestmark = pytest.mark.gpu
@@ -50,3 +51,15 @@ def test_refused(gpu):
     assert call(3072, 64, 64) is not None
     assert call(3072, 72, 64) is None and call(1536, 64, 64) is None and call(4096, 64, 64) is None  # features and widths that it has no tile for
     assert call(3072, 64, 16384) is None  # more than two rounds
+
+
+@pytest.mark.parametrize("C, N", [(3072, 72), (1536, 64), (4096, 64), (320, 64)])
+def test_refused_widths_cost_no_memory(gpu, C, N):
+    lin = torch.nn.Linear(C, N, device=gpu, dtype=torch.bfloat16).requires_grad_(False)
+    x, head = torch.ones(1, 64, C, device=gpu, dtype=torch.bfloat16), torch.ones(1, 2 * C, device=gpu, dtype=torch.bfloat16)
+    with torch.inference_mode():
+        assert kernels.project_normed(lin, x, head[:, :C], head[:, C:], 1e-6) is None
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        assert kernels.project_normed(lin, x, head[:, :C], head[:, C:], 1e-6) is None
+        assert torch.cuda.max_memory_allocated() == before

@@ -1228,6 +1228,7 @@ PyObject* py_project_normed(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return none();
   for (const Tensor* t : {sh, sc})
     if (!c.operand(*t) || t->dim() != 2 || t->size(0) != x->size(0) || t->size(1) != l.k || t->stride(1) != 1 || t->stride(0) != sh->stride(0)) return none();
+  if (l.k > 256 && (l.n > 64 || l.k > 3072 || l.k % 1024 != 0)) return none();  // (widths that odit_linear_norm takes: nothing is allocated for others)
   Tensor out = fresh({x->size(0), x->size(1), l.n}, x->options());
   odit_linear_problem q = {x->data_ptr(), l.w, l.b, nullptr, nullptr, out.data_ptr(), static_cast<int>(x->size(0) * x->size(1)), 0, l.k, l.ldw, l.n, 0, 0};
   odit_row_norm r = {sh->data_ptr(), sc->data_ptr(), x->size(0) > 1 ? sh->stride(0) : 0, static_cast<int>(x->size(1)), static_cast<float>(eps)};
