@@ -179,6 +179,8 @@ int head_features(int M, int N, int K, int cus) {
 
 }  // namespace
 
+// K: the kernel is made for multiples of 256, a step's fragments of 8 wavefronts, and built for the three that the times above were taken at; heads of other widths keep their
+// two launches. What a tuning call found for the projection alone is not asked: the norm in front of it is a launch of its own there (6 us and more of the 10 to 34).
 int linear_head_features(const GemmCall& c, const RowNorm& n, int dtype, int cus) {
   if ((c.K != 1024 && c.K != 2048 && c.K != 3072) || c.N > 64 || cus <= 0 || !gemm_streamk_takes(c, dtype) || !aligned16(n.shift) || !aligned16(n.scale) ||
       n.stride % 8 != 0 || (c.epilogue != ODIT_EPI_NONE && c.epilogue != ODIT_EPI_BIAS) || !gemm_rows_fit(c.M + 16, c.ldx, c.K) || !gemm_rows_fit(c.N + 64, c.ldw, c.K))
