@@ -1,5 +1,7 @@
 """A native block's intermediate tensors share memory where the per-kernel path frees one before it makes the next."""
 
+import gc
+
 import pytest
 import torch
 
@@ -41,6 +43,7 @@ def test_native_blocks_take_no_more_memory_than_kernel_by_kernel(gpu, monkeypatc
             monkeypatch.setattr(kernels, "NATIVE_BLOCKS", native)
             call()
             torch.cuda.synchronize()
+            gc.collect()  # (modules hold themselves: an earlier test's, collected during the call, would be taken off its peak)
             base = torch.cuda.memory_allocated()
             torch.cuda.reset_peak_memory_stats()
             call()
