@@ -2,12 +2,15 @@
 
 import re
 
+import pytest
+
 from test_device_code import _functions, _registers, _written_in_front
 
 
-def test_waits_that_hold_by_statement():
-    kernels = _functions("gemm_tile_apart.hip", labels=True)
-    assert len(kernels) == 4
+@pytest.mark.parametrize("unit, forms", [("gemm_tile_apart.hip", 4), ("gemm_tile_shared.hip", 2)])
+def test_waits_that_hold_by_statement(unit, forms):
+    kernels = _functions(unit, labels=True)
+    assert len(kernels) == forms
     for name, code in kernels.items():
         stores = [i for i in code if i.startswith("buffer_store_dwordx4")]
         assert len(stores) >= 16, name

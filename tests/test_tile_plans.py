@@ -6,6 +6,7 @@ from pathlib import Path
 import pytest
 
 from test_gpu_gemm_tile_parts import HEADS, PARTS
+from test_gpu_tile_shared import parted
 
 _ROOT = Path(__file__).resolve().parents[1]
 
@@ -43,3 +44,17 @@ def test_where_rows_of_padding_are_fetched_from(ask, rows, tile, K):
     end = -(-rows // tile) * tile
     fits = (2**31 - K - 1) // end  # the longest row
     assert ask(("pad", rows, tile, K, K), ("pad", rows, tile, fits, K), ("pad", rows, tile, fits + 1, K), ("pad", rows, tile, 2**40, K)) == [(end,), (end,), (rows - 1,), (rows - 1,)]
+
+
+def test_shares_of_tiles(ask):
+    """Where the shares of TileShares part a tile is where workers that take one step after the other do; a tile never into three."""
+    problems = [(M, N, K, w) for M in (8192, 8193, 13202, 20011) for N in (3072, 5120, 9216) for K in (64, 448, 5120) for w in (1, 7, 233, 256) if -(-M // 256) * -(-N // 256) >= w]
+    answers = ask(*(("shares", *p) for p in problems))
+    for (M, N, K, w), (known, tiles, first, share, more) in zip(problems, answers):
+        mt, nt, n = -(-M // 256), -(-N // 256), K // 64
+        order = [(r, c) for g in range(0, mt, 16) for c in range(nt) for r in range(g, min(g + 16, mt))]
+        assert known == 1 and tiles == len(order)
+        ends = [i * share + min(i, more) for i in range(1, w + 1)] if share else []
+        assert {order[first + e // n]: e % n for e in ends if e % n} == parted(M, N, K, w)
+        assert not share or (ends[-1] == (tiles - first) * n and n <= share and first % w == 0)
+    assert [a[0] for a in ask(("shares", 256, 2560, 64, 11), ("shares", 256, 2560, 64, 0))] == [0, 0]

@@ -52,6 +52,7 @@ UNITS: list[tuple[str, list[str], str]] = [
     ("gemm_tile_heads.hip", [], "gemm_tile_heads"),
     ("gemm_tile_unless.hip", [], "gemm_tile_unless"),
     ("gemm_tile_apart.hip", [], "gemm_tile_apart"),
+    ("gemm_tile_shared.hip", [], "gemm_tile_shared"),
     ("gemm_small.hip", [], "gemm_small"),
     ("gemm_small_heads.hip", [], "gemm_small_heads"),
     ("gemm_small_norm.hip", [], "gemm_small_norm"),

@@ -82,12 +82,17 @@ struct TileParams {
   char* slots;
 };
 
-template <bool HEADS, bool UNLESS> struct TileArgs : TileParams {};
+template <bool HEADS, bool UNLESS, bool SHARED = false> struct TileArgs : TileParams {};
 template <> struct TileArgs<true, false> : TileParams {
   HeadsOut heads[2];  // of the two problems (there are no three with heads); q null: an ordinary output
 };
 template <> struct TileArgs<false, true> : TileParams {
   const int* unless;
+};
+// The steps of the tiles from `shared` on are shared out one tile after the other, `share` steps to a worker and one more to the first `more` of them. A tile
+// that two of them have a share of is the sum of two sums. (share >= k_steps)
+template <> struct TileArgs<false, false, true> : TileParams {
+  int shared, share, more;
 };
 
 typedef __attribute__((address_space(3))) void* lds_void_p;
@@ -190,7 +195,7 @@ __device__ __forceinline__ void finish_quadrant(const GemmEpilogue& e, int m0, i
       for (int u = 0; u < 8; ++u) {
         if constexpr (K == 2) y[u] = gated_result<T, APART>(e, y[u], gt[u], bs[u], Raw<T>::get(res[i], u));
         else y[u] += bs[u];
-        if constexpr (K == 1) y[u] = gemm_gelu_tanh(y[u]);
+        if constexpr (K == 1) y[u] = APART ? gemm_gelu_apart(y[u]) : gemm_gelu_tanh(y[u]);
       }
       u32x4 o;
 #pragma unroll
@@ -252,9 +257,10 @@ __device__ __forceinline__ void store_heads(const HeadsOut& h, const u32x4 (&v)[
 
 // MH: 16-row accumulators of a wavefront in each half of the rows (4: 256-row tiles, 2: 128). HEADS: the form for problems whose
 // output is query, key and value heads, beside ordinary ones without a gate. UNLESS: nothing is done where a word of device memory is not 0 (a
-// form of its own, as the test made the others up to 0.6 % slower: M=1536, N=12288, K=3072 109.7 / 110.4 us). APART: gemm_gated_apart (likewise).
-template <typename T, int MH, bool HEADS, bool UNLESS, bool APART = false>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_tile_kernel(const TileArgs<HEADS, UNLESS> p) {
+// form of its own, as the test made the others up to 0.6 % slower: M=1536, N=12288, K=3072 109.7 / 110.4 us). APART: gemm_gated_apart and gemm_gelu_apart (likewise).
+// SHARED: TileArgs's shared tiles, each by one workgroup, and no tile in parts.
+template <typename T, int MH, bool HEADS, bool UNLESS, bool APART = false, bool SHARED = false>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_tile_kernel(const TileArgs<HEADS, UNLESS, SHARED> p) {
   using M = Mma16<T>;
   using frag = typename M::frag;
   constexpr int BM = 64 * MH, HM = 32 * MH;           // rows of a tile, of a half
@@ -287,27 +293,45 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   };
 
   // problem, first row and first feature of a tile: groups of 8 row tiles, feature tiles outer inside a group, so that the 32
-  // tiles an XCD runs at a time share 8 pieces of x and 4 of W
+  // tiles an XCD runs at a time share 8 pieces of x and 4 of W (SHARED: of 16, the order in which they are shared out)
+  constexpr int kGroup = SHARED ? 16 : 8;
   auto locate = [&](int tile, int& which, int& m0, int& n0) __attribute__((always_inline)) {
     which = tile >= p.tiles1 ? 2 : tile >= p.tiles0 ? 1 : 0;
     const int t = tile - (which == 2 ? p.tiles1 : which == 1 ? p.tiles0 : 0);
-    const int mt = p.q[which].m_tiles, per = 8 * p.q[which].n_tiles;
-    const int g = quotient(t, per), first = g * 8, gm = mt - first < 8 ? mt - first : 8;
+    const int mt = p.q[which].m_tiles, per = kGroup * p.q[which].n_tiles;
+    const int g = quotient(t, per), first = g * kGroup, gm = mt - first < kGroup ? mt - first : kGroup;
     const int r = t - g * per, nt = quotient(r, gm);
     m0 = (first + r - nt * gm) * BM;
     n0 = nt * kTileN;
   };
   // The segments of this workgroup: whole tiles, then its part of a cut tile. A cursor is (part still to do, next whole tile).
   const int cut = p.tiles - p.whole;
-  const bool has_part = v < cut * p.parts;
+  const bool has_part = !SHARED && v < cut * p.parts;
   // quadrants that this part of a cut tile finishes: its number's, and the one `parts` further
   auto quadrants = [&]() __attribute__((always_inline)) -> int {
     const int part = quotient(v, cut);
     return scalar((part < 4 ? 1 << part : 0) | (part + p.parts < 4 ? 1 << (part + p.parts) : 0));
   };
   constexpr int kQuad = 2 * MH * 8192;  // bytes of a quadrant's accumulators
+  // (SHARED: no tile is cut, and it is whether a tile's second segment is to come.)
   struct Cursor { bool part; int next; };
   auto next_segment = [&](Cursor& c, int& tile, int& k0, int& k1) __attribute__((always_inline)) -> bool {
+    if constexpr (SHARED) {
+      if (c.next >= p.tiles) return false;
+      tile = c.next;
+      k0 = 0;
+      k1 = nk;
+      if (tile >= p.shared) {
+        const int from = (tile - p.shared) * nk, longer = p.more * (p.share + 1);
+        const int to = from < longer ? (quotient(from, p.share + 1) + 1) * (p.share + 1) : longer + (quotient(from - longer, p.share) + 1) * p.share;
+        if (to - from < nk) {
+          c.part = !c.part;
+          (c.part ? k1 : k0) = scalar(to - from);
+        }
+      }
+      if (!c.part) c.next += G;
+      return true;
+    }
     if (c.next < p.whole) {
       tile = c.next;
       c.next += G;
@@ -594,7 +618,41 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
     if (wm == 0) barrier();  // both groups are here
 
-    if (k0 == 0 && k1 == nk) {
+    bool whole = k0 == 0 && k1 == nk;
+    if constexpr (SHARED) {
+      if (!whole) {
+        // The first sum of a shared tile waits in this workgroup's slot for the second, each thread's own accumulators. (no store with a scalar offset: see below)
+        const auto slot = __builtin_amdgcn_make_buffer_rsrc(p.slots + static_cast<int64_t>(v) * kTileSlot, 0, kTileSlot, 0x00020000);
+        const uint32_t own = static_cast<uint32_t>((wave * 64 + hidden_lane()) * 16);
+        whole = k0 != 0;
+#pragma unroll
+        for (int quad = 0; quad < 4; ++quad) {
+          if (!whole) {
+#pragma unroll
+            for (int i = 0; i < 2 * MH; ++i)
+              __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_v, acc[quad >> 1][quad & 1][i / 2][i % 2]), slot,
+                                                     own + (quad * kQuad + i * 8192), 0, kThrough);
+          } else {
+#pragma unroll
+            for (int half = 0; half < 2; ++half) {  // (all at once would not fit the registers)
+              f32x4_v first[MH];
+#pragma unroll
+              for (int i = 0; i < MH; ++i)
+                first[i] = __builtin_bit_cast(f32x4_v, __builtin_amdgcn_raw_buffer_load_b128(slot, own + (quad * kQuad + (half * MH + i) * 8192), 0, kThrough));
+#pragma unroll
+              for (int i = 0; i < MH; ++i) acc[quad >> 1][quad & 1][half * MH / 2 + i / 2][i % 2] += first[i];
+              __builtin_amdgcn_sched_barrier(0);
+            }
+          }
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // they are in memory before they are asked for
+        if (!whole) {
+          more = next_segment(cc, tile, k0, k1);
+          continue;
+        }
+      }
+    }
+    if (whole) {
       int which, m0, n0;
       locate(tile, which, m0, n0);
       const GemmEpilogue& e = p.q[which].ep;
@@ -611,7 +669,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       if constexpr (HEADS) {
         if (scalar(heads) != 0) finish_heads(p.heads[which], e, m0, n0, ln);
       }
-    } else {
+    } else if constexpr (!SHARED) {
       // A part of a cut tile. The parts share the tile's four quadrants out between them: part i adds up and finishes quadrants i,
       // i + parts, ..., which it keeps in LDS (each thread its own accumulators; no tile load is in flight any more), and
       // leaves the others in its slot.
@@ -649,7 +707,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
     more = next_segment(cc, tile, k0, k1);
   }
-  if (has_part) {
+  if (!SHARED && has_part) {
     // A part looks for all parts of its tile to have arrived, a bounded number of times; then it gives its quadrants up (which fails
     // if the last one has arrived by now) and leaves them to the last to arrive.
     const int part = quotient(v, cut), t = v - part * cut, parts = p.parts, mine = quadrants();

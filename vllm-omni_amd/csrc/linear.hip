@@ -67,7 +67,7 @@ struct LinPlan {
   size_t algo_ws = 0;
   bool have_algo = false;
   bool tuned = false;
-  int passed = 0;  // the library's first choice is never run (lin_sound): it would have summed every tile whole (1), or split some (2)
+  int passed = 0;  // the library's first choice is never run (lin_sound): it would have summed every tile whole (1), or split some among passed - 1 workers
   float us = 0;  // expected time of a kernel that was ranked, 0: not known
 };
 
@@ -341,6 +341,7 @@ static double lin_tile_us(int M, int N, int K, int features, int rows, int cus) 
 constexpr int kLinRankMinRows = 1024, kLinRankMinK = 4096;
 constexpr double kLinRankGain = 0.92, kLinTallTile = 1.01;
 constexpr int kLinCandidates = 32;
+constexpr size_t kLinTileSums = 256 * 256 * 4;  // what a worker of the kernel passed over leaves of a tile
 
 // The library's kernels for a problem, in its own order, and LinPlan::passed. (All of them at once: a library that has been asked for one alone, and then for
 // more of the same problem, has the rest in no order of merit. 0.2 ms, once for a problem.)
@@ -356,7 +357,7 @@ static int lin_candidates(hipblasLtHandle_t h, LinPlan& p, size_t lib_ws_bytes, 
     set_error("odit_linear: hipBLASLt has no kernel for this problem (status %d)", static_cast<int>(st));
     return ODIT_ENOTSUP;
   }
-  p.passed = lin_sound(h, res[0].algo) ? 0 : res[0].workspaceSize == 0 ? 1 : 2;
+  p.passed = lin_sound(h, res[0].algo) ? 0 : res[0].workspaceSize == 0 ? 1 : 1 + static_cast<int>((res[0].workspaceSize + kLinTileSums - 1) / kLinTileSums);
   return ODIT_OK;
 }
 
@@ -492,10 +493,13 @@ static int lin_handwritten_kind(const odit::GemmCall& g, int dtype, const void* 
   return sk != nullptr && odit::gemm_streamk_takes(g, dtype) ? 1 : 0;
 }
 
-static int lin_launch_handwritten(int kind, const odit::GemmCall& g, int dtype, void* sk, hipStream_t stream) {
+static int lin_launch_handwritten(int kind, const odit::GemmCall& g, int dtype, void* sk, hipStream_t stream, int workers = 0) {
   if (kind == 1) return odit::launch_gemm_streamk(&g, 1, dtype, sk, stream);
   if (kind == 3) return odit::launch_gemm_small(&g, 1, dtype, stream);
-  if (kind == 4) return odit::launch_gemm_tile_apart(g, dtype, sk, stream);
+  if (kind == 4) {
+    const odit::TileShares shares = odit::tile_shares(g.M, g.N, g.K, workers);
+    return shares.known && sk != nullptr ? odit::launch_gemm_tile_shared(g, dtype, shares, sk, stream) : odit::launch_gemm_tile_apart(g, dtype, sk, stream);
+  }
   return odit::launch_gemm_tile(&g, 1, nullptr, dtype, sk, stream);
 }
 
@@ -629,14 +633,17 @@ static int lin_rule_kind(const odit::LinCall& c, const odit::GemmCall& g, const 
   if (tile && plan.us < lin_library_us(c, g)) return 2;
   // In the place of a kernel that never runs the tile kernel does. A call that wants no other order of summation has every tile whole where that kernel would have had it so,
   // and in gated and residual epilogues the library's order of operations (kind 4): the library's bits, but for GELU, whose own is left to the library's next kernel. (65520
-  // rows of a pair, us, the library's next / this: N=15360, K=5120 7690 / 6930, N=5120 gated 2750 / 2340, K=13824 7200 / 6010.) Where it would have split tiles, no
-  // other kernel's sums are those.
+  // rows of a pair, us, the library's next / this: N=15360, K=5120 7690 / 6930, N=5120 gated 2750 / 2340, K=13824 7200 / 6010.) Where it would have split tiles
+  // this kernel parts the same ones there (gemm_tile_shared.hip; us, bf16, that kernel / this: 13202 rows, N=15360, K=5120 1519 / 1642, N=13824 with GELU 1640 / 1554,
+  // N=5120, K=13824 1513 / 1547; 8192 rows, N=9216, K=3072 449 / 373; 34968 rows, N=15360, K=5120 3911 / 4396).
   const int passed = lin_passed(c, g);
   if (passed == 0) return 0;
   if (tile) return 2;
   const bool gelu = c.epilogue == ODIT_EPI_GELU_TANH || c.epilogue == ODIT_EPI_BIAS_GELU_TANH;
-  return passed == 2 || (plan.parts == 1 && !gelu) ? 4 : 0;
+  return passed > 1 || (plan.parts == 1 && !gelu) ? 4 : 0;
 }
+// for kind 4: how many workers the kernel passed over would have shared tiles out among (0: none is)
+static int lin_workers(const odit::LinCall& c, const odit::GemmCall& g) { return std::max(lin_passed(c, g) - 1, 0); }
 static int lin_auto_kind(int dev, const odit::LinCall& c, const odit::GemmCall& g, const void* sk) {
   odit::Tuned found;
   return lin_tuned(dev, c, g, sk, &found) ? found.kind : lin_rule_kind(c, g, sk);
@@ -735,12 +742,14 @@ extern "C" int odit_linear_rows(const void* x, const void* w, const void* bias, 
   } else if (engine == 0 && hipGetDevice(&dev) == hipSuccess) {
     kind = lin_auto_kind(dev, c, g, sk);
   }
-  if (kind != 0) return lin_launch_handwritten(kind, g, dtype, sk, c.stream);
+  const int workers = kind == 4 ? lin_workers(c, g) : 0;
+  const bool apart = per_rows && workers > 0;
+  if (kind != 0 && !apart) return lin_launch_handwritten(kind, g, dtype, sk, c.stream, workers);
   if (!per_rows) {
     rc = lin_run_library(c);
     return rc == ODIT_OK && c.clip ? lin_clip(c) : rc;
   }
-  // the library's epilogue takes one gate vector per launch: one launch per group of rows
+  // the library's epilogue takes one gate vector per launch: one launch per group of rows (`apart`: and which tiles are split follows from a group's)
   const size_t esz = dtype == ODIT_F32 ? 4 : 2, gsz = gate_dtype == ODIT_F32 ? 4 : esz;
   for (int r0 = 0; r0 < M; r0 += rows_per_gate) {
     LinCall cg = c;
@@ -752,7 +761,9 @@ extern "C" int odit_linear_rows(const void* x, const void* w, const void* bias, 
     cg.gate = static_cast<const char*>(gate) + static_cast<size_t>(grp * gate_stride) * gsz;
     if (epilogue == ODIT_EPI_GATED_RESIDUAL_PRE && bias != nullptr)
       cg.bias = static_cast<const char*>(bias) + static_cast<size_t>(grp * gate_stride) * 4;
-    rc = lin_run_library(cg);
+    const GemmCall gg = lin_gemm_call(cg, 0, 0);
+    if (apart && lin_rule_kind(cg, gg, sk) == 4) rc = lin_launch_handwritten(4, gg, dtype, sk, c.stream, lin_workers(cg, gg));
+    else rc = lin_run_library(cg);
     if (rc != ODIT_OK) return rc;
   }
   return c.clip ? lin_clip(c) : ODIT_OK;
@@ -1100,9 +1111,10 @@ extern "C" int odit_linear_rows_plan(const void* x, const void* w, const void* b
   (void)hipGetDevice(&dev);
   c.first = (flags & ODIT_LINEAR_FIRST) != 0;
   c.no_tile = c.first || (flags & ODIT_LINEAR_NO_TILE) != 0;
-  const bool own = M > 0 && engine != 1 && (engine == 2 ? lin_handwritten_kind(g, dtype, sk) : lin_auto_kind(dev, c, g, sk)) != 0;
+  const int kind = M == 0 || engine == 1 ? 0 : engine == 2 ? lin_handwritten_kind(g, dtype, sk) : lin_auto_kind(dev, c, g, sk);
+  const bool own = kind != 0, grouped = per_rows && (!own || (kind == 4 && lin_workers(c, g) > 0));
   *handwritten = own ? 1 : 0;
-  *launches = M == 0 ? 0 : (own || !per_rows ? 1 : (M + rows_per_gate - 1) / rows_per_gate);
+  *launches = M == 0 ? 0 : (!grouped ? 1 : (M + rows_per_gate - 1) / rows_per_gate);
   if (!own && lin_needs_prep(c)) *launches *= 2;  // plus the [N]-sized gate-vector launch of the library form
   return ODIT_OK;
 }
