@@ -385,8 +385,8 @@ int odit_linear_tune(const void* x, const void* w, const void* bias, void* out, 
  * faster, and what ODIT_LINEAR_NO_TILE says; ODIT_LINEAR_NO_TILE = neither the tile nor the small kernel, unless a tuning call
  * found it faster (a caller whose results another order of summation may not move). Per call: no process-wide switch exists.
  * hipBLASLt's hand-scheduled kernel ("Custom_...") is never run, tuned or preferred, as it now and then gives other results for the same
- * operands. Where it is the first choice the tile kernel takes the call; with ODIT_LINEAR_FIRST or ODIT_LINEAR_NO_TILE, what runs gives the results that it
- * should have given, unless the problem (or, of gates per group of rows, a group) has fewer tiles of 256 x 256 than that kernel would have shared them out among.
+ * operands. Where it is the first choice the tile kernel takes the call; with ODIT_LINEAR_FIRST or ODIT_LINEAR_NO_TILE, what runs has its order of
+ * summation where it would have split tiles.
  * ODIT_LINEAR_CLIP: of a gated or residual epilogue in ODIT_F16, results are clipped to +-65504, as the blocks' outputs are
  * (qwen_image_transformer.py:812-815, flux_transformer.py:310-312, 362-364); a NaN stays one. Nothing in other types. Of two problems
  * the first one's; ODIT_LINEAR_CLIP2 the second one's.

@@ -47,14 +47,14 @@ def test_where_rows_of_padding_are_fetched_from(ask, rows, tile, K):
 
 
 def test_shares_of_tiles(ask):
-    """Where the shares of TileShares part a tile is where workers that take one step after the other do; a tile never into three."""
-    problems = [(M, N, K, w) for M in (8192, 8193, 13202, 20011) for N in (3072, 5120, 9216) for K in (64, 448, 5120) for w in (1, 7, 233, 256) if -(-M // 256) * -(-N // 256) >= w]
+    """Where the shares of TileShares part a tile is where workers that take one step after the other do."""
+    problems = [(M, N, K, w) for M in (8192, 8193, 13202, 20011) for N in (3072, 5120, 9216) for K in (64, 448, 5120) for w in (1, 7, 233, 256)] + [(2400, 5120, 13824, 256), (1500, 5120, 13824, 206)]
     answers = ask(*(("shares", *p) for p in problems))
     for (M, N, K, w), (known, tiles, first, share, more) in zip(problems, answers):
         mt, nt, n = -(-M // 256), -(-N // 256), K // 64
         order = [(r, c) for g in range(0, mt, 16) for c in range(nt) for r in range(g, min(g + 16, mt))]
         assert known == 1 and tiles == len(order)
         ends = [i * share + min(i, more) for i in range(1, w + 1)] if share else []
-        assert {order[first + e // n]: e % n for e in ends if e % n} == parted(M, N, K, w)
-        assert not share or (ends[-1] == (tiles - first) * n and n <= share and first % w == 0)
-    assert [a[0] for a in ask(("shares", 256, 2560, 64, 11), ("shares", 256, 2560, 64, 0))] == [0, 0]
+        assert {(order[first + e // n], e % n) for e in ends if e % n} == {(t, e) for t, es in parted(M, N, K, w).items() for e in es}
+        assert not share or (ends[-1] == (tiles - first) * n and first % w == 0 and (tiles < w or n <= share))
+    assert [a[0] for a in ask(("shares", 256, 2560, 64, 11), ("shares", 256, 2560, 64, 0))] == [0, 0]  # (a worker without a step, no workers)

@@ -76,19 +76,20 @@ int launch_gemm_tile_unless(const GemmCall& c, const int* unless, int dtype, voi
 // gemm_tile_apart.hip: one problem, its epilogue in the library's order of operations
 int launch_gemm_tile_apart(const GemmCall& c, int dtype, void* scratch, hipStream_t stream);
 
-// Which tiles of 256 x 256 the library's kernel that is never run sums in two pieces, and where it parts them, seen from what it gave for sums that lose a term
-// exactly where they are parted (five problems that it parts, 1026 to 8220 tiles and 233 or 256 workers: all 1105 parted tiles as here). Its tiles are numbered in
-// groups of 16 row tiles, features outer; the last workers + tiles % workers of them, from `from` on, are shared out in equal numbers of steps, the first `more`
-// workers one more. share 0: every tile is whole. Fewer tiles than workers: not known (`known` false).
+// Which tiles of 256 x 256 the library's kernel that is never run sums in pieces, and where it parts them, seen from what it gave for sums that lose a term
+// exactly where they are parted (eight problems that it parts, 120 to 8220 tiles and 206 to 256 workers: all 1617 parted tiles as here). Its tiles are numbered in
+// groups of 16 row tiles, features outer; the last workers + tiles % workers of them (of fewer tiles than workers all), from `from` on, are shared out in equal numbers
+// of steps, the first `more` workers one more. A tile's sums are added in the order of their steps. share 0: every tile is whole. `known` false: a worker has no step.
 struct TileShares {
   bool known;
   int tiles, from, share, more;
 };
 inline TileShares tile_shares(int M, int N, int K, int workers) {
   const int tiles = (M + 255) / 256 * ((N + 255) / 256);
-  if (workers <= 0 || tiles < workers) return {false, tiles, tiles, 0, 0};
+  if (workers <= 0) return {false, tiles, tiles, 0, 0};
   if (tiles % workers == 0) return {true, tiles, tiles, 0, 0};
-  const int shared = tiles % workers + workers, steps = shared * (K / 64);
+  const int shared = tiles % workers + (tiles > workers ? workers : 0), steps = shared * (K / 64);
+  if (steps < workers) return {false, tiles, tiles, 0, 0};
   return {true, tiles, tiles - shared, steps / workers, steps % workers};
 }
 // gemm_tile_shared.hip: one problem, the same with these shares (known; with share > 0 it needs `scratch`)

@@ -90,7 +90,7 @@ template <> struct TileArgs<false, true> : TileParams {
   const int* unless;
 };
 // The steps of the tiles from `shared` on are shared out one tile after the other, `share` steps to a worker and one more to the first `more` of them. A tile
-// that two of them have a share of is the sum of two sums. (share >= k_steps)
+// that several of them have a share of is the sum of their sums, in their order. (share 0: all tiles are whole, and shared == tiles)
 template <> struct TileArgs<false, false, true> : TileParams {
   int shared, share, more;
 };
@@ -313,23 +313,21 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     return scalar((part < 4 ? 1 << part : 0) | (part + p.parts < 4 ? 1 << (part + p.parts) : 0));
   };
   constexpr int kQuad = 2 * MH * 8192;  // bytes of a quadrant's accumulators
-  // (SHARED: no tile is cut, and it is whether a tile's second segment is to come.)
-  struct Cursor { bool part; int next; };
+  // SHARED: no tile is cut; the next tile's steps from `at` on are to come, each worker's a segment.
+  struct Cursor { bool part; int next, at = 0; };
   auto next_segment = [&](Cursor& c, int& tile, int& k0, int& k1) __attribute__((always_inline)) -> bool {
     if constexpr (SHARED) {
       if (c.next >= p.tiles) return false;
       tile = c.next;
-      k0 = 0;
+      k0 = c.at;
       k1 = nk;
       if (tile >= p.shared) {
-        const int from = (tile - p.shared) * nk, longer = p.more * (p.share + 1);
+        const int from = (tile - p.shared) * nk + k0, longer = p.more * (p.share + 1);
         const int to = from < longer ? (quotient(from, p.share + 1) + 1) * (p.share + 1) : longer + (quotient(from - longer, p.share) + 1) * p.share;
-        if (to - from < nk) {
-          c.part = !c.part;
-          (c.part ? k1 : k0) = scalar(to - from);
-        }
+        if (to - from < nk - k0) k1 = scalar(k0 + to - from);
       }
-      if (!c.part) c.next += G;
+      c.at = k1 < nk ? k1 : 0;
+      if (c.at == 0) c.next += G;
       return true;
     }
     if (c.next < p.whole) {
@@ -621,28 +619,29 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     bool whole = k0 == 0 && k1 == nk;
     if constexpr (SHARED) {
       if (!whole) {
-        // The first sum of a shared tile waits in this workgroup's slot for the second, each thread's own accumulators. (no store with a scalar offset: see below)
+        // The sum so far of a shared tile waits in this workgroup's slot for the next piece's, each thread's own accumulators. (no store with a scalar offset: see below)
         const auto slot = __builtin_amdgcn_make_buffer_rsrc(p.slots + static_cast<int64_t>(v) * kTileSlot, 0, kTileSlot, 0x00020000);
         const uint32_t own = static_cast<uint32_t>((wave * 64 + hidden_lane()) * 16);
-        whole = k0 != 0;
+        whole = k1 == nk;
 #pragma unroll
         for (int quad = 0; quad < 4; ++quad) {
+          if (k0 != 0) {
+#pragma unroll
+            for (int half = 0; half < 2; ++half) {  // (all at once would not fit the registers)
+              f32x4_v before[MH];
+#pragma unroll
+              for (int i = 0; i < MH; ++i)
+                before[i] = __builtin_bit_cast(f32x4_v, __builtin_amdgcn_raw_buffer_load_b128(slot, own + (quad * kQuad + (half * MH + i) * 8192), 0, kThrough));
+#pragma unroll
+              for (int i = 0; i < MH; ++i) acc[quad >> 1][quad & 1][half * MH / 2 + i / 2][i % 2] += before[i];
+              __builtin_amdgcn_sched_barrier(0);
+            }
+          }
           if (!whole) {
 #pragma unroll
             for (int i = 0; i < 2 * MH; ++i)
               __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_v, acc[quad >> 1][quad & 1][i / 2][i % 2]), slot,
                                                      own + (quad * kQuad + i * 8192), 0, kThrough);
-          } else {
-#pragma unroll
-            for (int half = 0; half < 2; ++half) {  // (all at once would not fit the registers)
-              f32x4_v first[MH];
-#pragma unroll
-              for (int i = 0; i < MH; ++i)
-                first[i] = __builtin_bit_cast(f32x4_v, __builtin_amdgcn_raw_buffer_load_b128(slot, own + (quad * kQuad + (half * MH + i) * 8192), 0, kThrough));
-#pragma unroll
-              for (int i = 0; i < MH; ++i) acc[quad >> 1][quad & 1][half * MH / 2 + i / 2][i % 2] += first[i];
-              __builtin_amdgcn_sched_barrier(0);
-            }
           }
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // they are in memory before they are asked for

@@ -1,5 +1,5 @@
 // The tile kernel with the order of summation that the library's kernel that is never run would have had where it splits tiles (tile_shares), for calls whose results are
-// to be that kernel's. One workgroup sums both pieces of a tile, the first one's sum waiting in its scratch: where the pieces ran on two they would have to wait for
+// to be that kernel's. One workgroup sums all pieces of a tile, the sum so far waiting in its scratch: where the pieces ran on several they would have to wait for
 // each other. A form of its own, as in the kernels of gemm_tile_apart.hip the tests for it put registers into scratch memory.
 #include "gemm_tile.h"
 

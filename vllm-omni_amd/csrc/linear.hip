@@ -635,7 +635,8 @@ static int lin_rule_kind(const odit::LinCall& c, const odit::GemmCall& g, const 
   // and in gated and residual epilogues the library's order of operations (kind 4): the library's bits, but for GELU, whose own is left to the library's next kernel. (65520
   // rows of a pair, us, the library's next / this: N=15360, K=5120 7690 / 6930, N=5120 gated 2750 / 2340, K=13824 7200 / 6010.) Where it would have split tiles
   // this kernel parts the same ones there (gemm_tile_shared.hip; us, bf16, that kernel / this: 13202 rows, N=15360, K=5120 1519 / 1642, N=13824 with GELU 1640 / 1554,
-  // N=5120, K=13824 1513 / 1547; 8192 rows, N=9216, K=3072 449 / 373; 34968 rows, N=15360, K=5120 3911 / 4396).
+  // N=5120, K=13824 1513 / 1547; 8192 rows, N=9216, K=3072 449 / 373; 34968 rows, N=15360, K=5120 3911 / 4396; 2400 rows, N=5120, K=13824, fewer tiles than
+  // workers, 436 / 278).
   const int passed = lin_passed(c, g);
   if (passed == 0) return 0;
   if (tile) return 2;
