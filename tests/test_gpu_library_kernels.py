@@ -69,13 +69,24 @@ def test_hand_scheduled_kernel_never_runs(gpu, M, N, K, epilogue, groups, flags,
 
 @pytest.mark.parametrize("M", [2048, 7072])
 def test_in_its_place_the_tile_kernel_with_the_library_s_bits(gpu, M):
-    """A call that keeps the library's order of summation: the tile kernel, with the bits of the library's kernels that split no tile, but for GELU."""
+    """A call that keeps the library's order of summation: the tile kernel, with the bits of the library's kernels that split no tile."""
     p = _Problem(gpu, M, 15360, 5120, BIAS, torch.bfloat16)
     out, names = p.names(FIRST)
     assert len(names) == 1 and "gemm_tile_kernel" in names[0], names
     assert torch.equal(out, p.run(LIBRARY | FIRST))
-    out, names = _Problem(gpu, M, 13824, 5120, GELU, torch.bfloat16).names(FIRST)
-    assert len(names) == 1 and "Cijk" in names[0], names
+
+
+@pytest.mark.parametrize("M, N", [(3261, 13824), (7072, 13824), (2875, 15360)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_gelu_in_its_place(gpu, M, N, dtype):
+    """The sums of whole tiles, and GELU as the library computes it: x = a power of two times one row of W, so that it is exact."""
+    p = _Problem(gpu, M, N, 5120, GELU, dtype)
+    out, names = p.names(FIRST)
+    assert len(names) == 1 and "gemm_tile_kernel" in names[0], names
+    assert len(p.names(LIBRARY | FIRST)[1]) == 1
+    p.x.zero_()
+    p.x[torch.arange(M, device=gpu), torch.randint(0, 5120, (M,), device=gpu)] = 64.0
+    assert torch.equal(p.run(FIRST), p.run(LIBRARY | FIRST))  # (the library's next kernel may sum in another order, but one term is one term)
 
 
 @pytest.mark.parametrize("epilogue", [GATED, RESIDUAL])

@@ -498,7 +498,8 @@ static int lin_launch_handwritten(int kind, const odit::GemmCall& g, int dtype, 
   if (kind == 3) return odit::launch_gemm_small(&g, 1, dtype, stream);
   if (kind == 4) {
     const odit::TileShares shares = odit::tile_shares(g.M, g.N, g.K, workers);
-    return shares.known && sk != nullptr ? odit::launch_gemm_tile_shared(g, dtype, shares, sk, stream) : odit::launch_gemm_tile_apart(g, dtype, sk, stream);
+    if (shares.known && sk != nullptr) return odit::launch_gemm_tile_shared(g, dtype, shares, sk, stream);
+    return odit::launch_gemm_tile_apart(g, dtype, nullptr, stream);  // (without scratch no tile is cut)
   }
   return odit::launch_gemm_tile(&g, 1, nullptr, dtype, sk, stream);
 }
@@ -632,16 +633,13 @@ static int lin_rule_kind(const odit::LinCall& c, const odit::GemmCall& g, const 
   if (plan.bm == 0) return 0;
   if (tile && plan.us < lin_library_us(c, g)) return 2;
   // In the place of a kernel that never runs the tile kernel does. A call that wants no other order of summation has every tile whole where that kernel would have had it so,
-  // and in gated and residual epilogues the library's order of operations (kind 4): the library's bits, but for GELU, whose own is left to the library's next kernel. (65520
-  // rows of a pair, us, the library's next / this: N=15360, K=5120 7690 / 6930, N=5120 gated 2750 / 2340, K=13824 7200 / 6010.) Where it would have split tiles
+  // and the library's order of operations in the epilogue (kind 4): the library's bits. (65520 rows of a pair, us, the library's next / this: N=15360, K=5120 7690 / 6930,
+  // N=5120 gated 2750 / 2340, K=13824 7200 / 6010. The library's next kernel without a workspace, of another tile, can differ: N=15360 with GELU, 2875 rows.) Where it would have split tiles
   // this kernel parts the same ones there (gemm_tile_shared.hip; us, bf16, that kernel / this: 13202 rows, N=15360, K=5120 1519 / 1642, N=13824 with GELU 1640 / 1554,
   // N=5120, K=13824 1513 / 1547; 8192 rows, N=9216, K=3072 449 / 373; 34968 rows, N=15360, K=5120 3911 / 4396; 2400 rows, N=5120, K=13824, fewer tiles than
   // workers, 436 / 278).
   const int passed = lin_passed(c, g);
-  if (passed == 0) return 0;
-  if (tile) return 2;
-  const bool gelu = c.epilogue == ODIT_EPI_GELU_TANH || c.epilogue == ODIT_EPI_BIAS_GELU_TANH;
-  return passed > 1 || (plan.parts == 1 && !gelu) ? 4 : 0;
+  return passed == 0 ? 0 : tile ? 2 : 4;
 }
 // for kind 4: how many workers the kernel passed over would have shared tiles out among (0: none is)
 static int lin_workers(const odit::LinCall& c, const odit::GemmCall& g) { return std::max(lin_passed(c, g) - 1, 0); }
