@@ -73,8 +73,8 @@ int launch_gemm_tile(const GemmCall* c, int count, const TileX2* x2, int dtype, 
 // gemm_tile_unless.hip: one problem, and nothing where *unless (device memory) is not 0 when the launch begins
 int launch_gemm_tile_unless(const GemmCall& c, const int* unless, int dtype, void* scratch, hipStream_t stream);
 
-// gemm_tile_apart.hip: one problem, its epilogue in the library's order of operations
-int launch_gemm_tile_apart(const GemmCall& c, int dtype, void* scratch, hipStream_t stream);
+// gemm_tile_apart.hip: one problem, every tile whole, its epilogue in the library's order of operations
+int launch_gemm_tile_apart(const GemmCall& c, int dtype, hipStream_t stream);
 
 // Which tiles of 256 x 256 the library's kernel that is never run sums in pieces, and where it parts them, seen from what it gave for sums that lose a term
 // exactly where they are parted (eight problems that it parts, 120 to 8220 tiles and 206 to 256 workers: all 1617 parted tiles as here). Its tiles are numbered in

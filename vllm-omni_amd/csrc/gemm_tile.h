@@ -257,8 +257,8 @@ __device__ __forceinline__ void store_heads(const HeadsOut& h, const u32x4 (&v)[
 
 // MH: 16-row accumulators of a wavefront in each half of the rows (4: 256-row tiles, 2: 128). HEADS: the form for problems whose
 // output is query, key and value heads, beside ordinary ones without a gate. UNLESS: nothing is done where a word of device memory is not 0 (a
-// form of its own, as the test made the others up to 0.6 % slower: M=1536, N=12288, K=3072 109.7 / 110.4 us). APART: gemm_gated_apart and gemm_gelu_apart (likewise).
-// SHARED: TileArgs's shared tiles, each by one workgroup, and no tile in parts.
+// form of its own, as the test made the others up to 0.6 % slower: M=1536, N=12288, K=3072 109.7 / 110.4 us). APART: gemm_gated_apart and gemm_gelu_apart (likewise), and
+// no tile in parts. SHARED: TileArgs's shared tiles, each by one workgroup.
 template <typename T, int MH, bool HEADS, bool UNLESS, bool APART = false, bool SHARED = false>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_tile_kernel(const TileArgs<HEADS, UNLESS, SHARED> p) {
   using M = Mma16<T>;
@@ -293,7 +293,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   };
 
   // problem, first row and first feature of a tile: groups of 8 row tiles, feature tiles outer inside a group, so that the 32
-  // tiles an XCD runs at a time share 8 pieces of x and 4 of W (SHARED: of 16, the order in which they are shared out)
+  // tiles an XCD runs at a time share 8 pieces of x and 4 of W (SHARED: of 16, the order in which they are shared out, which costs 1 to 4 % of a
+  // large launch: all tiles whole, us, groups of 8 / 16: 65520 rows, N=13824, K=5120 with GELU 6136 / 6395, N=15360 6779 / 6939; 7072 rows, N=15360 777 / 790)
   constexpr int kGroup = SHARED ? 16 : 8;
   auto locate = [&](int tile, int& which, int& m0, int& n0) __attribute__((always_inline)) {
     which = tile >= p.tiles1 ? 2 : tile >= p.tiles0 ? 1 : 0;
@@ -306,7 +307,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   };
   // The segments of this workgroup: whole tiles, then its part of a cut tile. A cursor is (part still to do, next whole tile).
   const int cut = p.tiles - p.whole;
-  const bool has_part = !SHARED && v < cut * p.parts;
+  const bool has_part = !APART && v < cut * p.parts;
   // quadrants that this part of a cut tile finishes: its number's, and the one `parts` further
   auto quadrants = [&]() __attribute__((always_inline)) -> int {
     const int part = quotient(v, cut);
@@ -668,7 +669,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       if constexpr (HEADS) {
         if (scalar(heads) != 0) finish_heads(p.heads[which], e, m0, n0, ln);
       }
-    } else if constexpr (!SHARED) {
+    } else if constexpr (!APART) {
       // A part of a cut tile. The parts share the tile's four quadrants out between them: part i adds up and finishes quadrants i,
       // i + parts, ..., which it keeps in LDS (each thread its own accumulators; no tile load is in flight any more), and
       // leaves the others in its slot.
@@ -706,7 +707,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
     more = next_segment(cc, tile, k0, k1);
   }
-  if (!SHARED && has_part) {
+  if (!APART && has_part) {
     // A part looks for all parts of its tile to have arrived, a bounded number of times; then it gives its quadrants up (which fails
     // if the last one has arrived by now) and leaves them to the last to arrive.
     const int part = quotient(v, cut), t = v - part * cut, parts = p.parts, mine = quadrants();

@@ -499,7 +499,7 @@ static int lin_launch_handwritten(int kind, const odit::GemmCall& g, int dtype, 
   if (kind == 4) {
     const odit::TileShares shares = odit::tile_shares(g.M, g.N, g.K, workers);
     if (shares.known && sk != nullptr) return odit::launch_gemm_tile_shared(g, dtype, shares, sk, stream);
-    return odit::launch_gemm_tile_apart(g, dtype, nullptr, stream);  // (without scratch no tile is cut)
+    return odit::launch_gemm_tile_apart(g, dtype, stream);
   }
   return odit::launch_gemm_tile(&g, 1, nullptr, dtype, sk, stream);
 }
