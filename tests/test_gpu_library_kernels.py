@@ -89,6 +89,23 @@ def test_gelu_in_its_place(gpu, M, N, dtype):
     assert torch.equal(p.run(FIRST), p.run(LIBRARY | FIRST))  # (the library's next kernel may sum in another order, but one term is one term)
 
 
+@pytest.mark.parametrize("M", [3261, 4800])  # (whole tiles; some of them parted)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_gelu_of_extremes(gpu, M, dtype):
+    p = _Problem(gpu, M, 13824, 5120, GELU, dtype)
+    top = torch.finfo(dtype).max
+    values = [-float("inf"), float("inf"), float("nan"), -top, top / 4, -100.0, -20.0, -9.0, -6.0, -0.0, 0.0, torch.finfo(dtype).tiny, -torch.finfo(dtype).tiny]
+    p.x.zero_()
+    p.bias.zero_()
+    p.bias[:len(values) + 1] = torch.tensor(values + [top], dtype=dtype, device=gpu)
+    own, library = p.run(FIRST), p.run(LIBRARY | FIRST)
+    n = len(values)
+    assert torch.equal(own[:, n], torch.full_like(own[:, n], top))  # (the library's bf16 overflows there)
+    own[:, n] = library[:, n] = 0
+    assert torch.equal(own.isnan(), library.isnan())
+    assert torch.equal(torch.where(own.isnan(), 0, own.view(torch.int16)), torch.where(library.isnan(), 0, library.view(torch.int16)))
+
+
 @pytest.mark.parametrize("epilogue", [GATED, RESIDUAL])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_gated_and_residual_epilogues_with_the_library_s_bits(gpu, epilogue, dtype):

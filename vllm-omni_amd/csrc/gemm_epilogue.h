@@ -46,6 +46,7 @@ template <typename T> __device__ __forceinline__ float gemm_clipped(const GemmEp
 
 // x sigmoid(2 u) of gemm_gelu_tanh, with the hardware's power and reciprocal as they come and 1 - 1 / (1 + e^(2 u)) for the sigmoid: the operations that
 // give the library's results (bf16, none of 33 million differs; 0.4 % of those are not the nearest to float64's).
+// Minus infinity gives NaN, as there; arguments of more than half the largest number themselves, where the library overflows.
 __device__ __forceinline__ float gemm_gelu_apart(float x) {
 #pragma clang fp contract(off)
   const float e = __builtin_amdgcn_exp2f(x * fmaf(x * 0.044715f, x, 1.f) * static_cast<float>(0.7978845608028654 * 2.885390081777927));
